@@ -13,6 +13,20 @@ def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu on the GPU box)")
 
 
+# the test that asks whether the HIP gradients are at least as close to the float64 oracle as the reference's own functor
+NEEDS_REFERENCE_FUNCTOR = {"test_gradient_error_per_element_beside_the_references_own_functor"}
+
+
+def pytest_collection_modifyitems(config, items):
+    """Without the reference's kernel_cpu.cpp compiled in place (oracle/_ref, built where the reference tree is) that
+    test would compare with the oracle's restatement, whose float64 form is what it measures the distance from."""
+    from oracle import binding
+    if binding.ref_lib() is None:
+        for item in items:
+            if item.name in NEEDS_REFERENCE_FUNCTOR:
+                item.add_marker(pytest.mark.skip(reason="oracle/_ref (the reference's functor) is not built here"))
+
+
 def _ensure_built():
     """Tests load what is already built.  They build what is missing, and they build libkhan_aev.so again when the
     stamp beside it (the digest of the sources and flags it was built from) does not match the sources in the tree:
