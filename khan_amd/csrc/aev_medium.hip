@@ -51,9 +51,10 @@ struct __align__(16) MedShared<T, kJvp, true> {
 
 // With kJvp the kernel computes the Jacobian-vector product instead (featurize_grad_inverse), as the
 // one-wavefront kernel does: list entries also carry (v_i - v_j)/r, the cutoff's derivative and the change of r.
-// With kLarge the kernel takes the molecules of more than 256 atoms: the atoms come type-sorted from `sorted`, and
-// the workgroups of one grid column (blockIdx.y = 0 .. gridDim.y - 1) share a molecule's centres batch by batch.
-template <typename T, bool kJvp, bool kLarge = false>
+// With kShare the workgroups of one grid column (blockIdx.y = 0 .. gridDim.y - 1) share a molecule's centres batch by
+// batch (a form of its own: the grid's sizes in scalar registers cost the plain kernel 6 %).
+// With kLarge the kernel takes the molecules of more than 256 atoms: the atoms come type-sorted from `sorted`.
+template <typename T, bool kJvp, bool kLarge = false, bool kShare = kLarge>
 __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
     const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
     const int32_t* __restrict__ A, const int32_t* __restrict__ MOs,
@@ -164,11 +165,11 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
         };
 
         // ------------------------------------------------------------ batches of kNB centres per wavefront
-        // (a large molecule that has the grid column to itself: shorter batches, so that every wavefront gets centres)
-        const int waves_y = static_cast<int>(gridDim.y) * 4;
-        const int batch = kLarge ? max(1, min(kNB, (n + waves_y - 1) / waves_y)) : kNB;
-        const int first_c0 = (kLarge ? static_cast<int>(blockIdx.y) * 4 + wave : wave) * batch;
-        const int stride_c0 = (kLarge ? waves_y : 4) * batch;
+        // (few centres for many wavefronts: shorter batches, so that every wavefront gets some)
+        const int waves_y = kShare ? static_cast<int>(gridDim.y) * 4 : 4;
+        const int batch = kShare ? max(1, min(kNB, (n + waves_y - 1) / waves_y)) : kNB;
+        const int first_c0 = (kShare ? static_cast<int>(blockIdx.y) * 4 + wave : wave) * batch;
+        const int stride_c0 = waves_y * batch;
         for (c0 = first_c0; c0 < n; c0 += stride_c0) {
             const int nb = min(batch, n - c0);
             unsigned overflow = 0;
@@ -472,8 +473,15 @@ hipError_t launch_fwd_medium(const T* X, const T* Y, const T* Z, const int32_t* 
     // (in float64 the working set lets one workgroup run per CU: a smaller grid costs less when it only skips)
     const int32_t cap = sizeof(T) == 4 ? 4096 : 1024;
     const unsigned blocks = static_cast<unsigned>(n_mols < cap ? n_mols : cap);
-    aev_fwd_medium_kernel<T, false><<<dim3(blocks), dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr,
-                                                                        nullptr, out, min_atoms, order, SortedAtoms<T>{});
+    // workgroups per molecule (dense boxes of 64-256 atoms, float: 216 -> 24 us at 32 molecules, 232 -> 72 at 256,
+    // 236 -> 186 at 1,024, the same at 2,048; double 346 -> 166 us at 256); the rows are the same bits for any number
+    const int parts = molecule_parts(n_mols, 4 * kCUs * (sizeof(T) == 4 ? 4 : 1), 16);
+    auto launch = [&](auto kernel) {
+        kernel<<<dim3(blocks, static_cast<unsigned>(parts)), dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr,
+                                                                                     out, min_atoms, order, SortedAtoms<T>{});
+    };
+    if (parts > 1) launch(aev_fwd_medium_kernel<T, false, false, true>);
+    else launch(aev_fwd_medium_kernel<T, false>);
     return hipGetLastError();
 }
 
@@ -487,8 +495,14 @@ hipError_t launch_jvp_medium(const T* X, const T* Y, const T* Z, const int32_t* 
     // (two workgroups per CU in float32, one in float64: a smaller grid costs less when it only skips)
     const int32_t cap = sizeof(T) == 4 ? 1024 : 512;
     const unsigned blocks = static_cast<unsigned>(n_mols < cap ? n_mols : cap);
-    aev_fwd_medium_kernel<T, true><<<dim3(blocks), dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, VX, VY, VZ,
-                                                                       out, min_atoms, order, SortedAtoms<T>{});
+    // workgroups per molecule (float: 282 -> 30 us at 32 molecules, 303 -> 137 at 256, 476 -> 382 at 512)
+    const int parts = molecule_parts(n_mols, 2 * kCUs * (sizeof(T) == 4 ? 2 : 1), 16);
+    auto launch = [&](auto kernel) {
+        kernel<<<dim3(blocks, static_cast<unsigned>(parts)), dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, VX, VY, VZ, out, min_atoms,
+                                                                                     order, SortedAtoms<T>{});
+    };
+    if (parts > 1) launch(aev_fwd_medium_kernel<T, true, false, true>);
+    else launch(aev_fwd_medium_kernel<T, true>);
     return hipGetLastError();
 }
 

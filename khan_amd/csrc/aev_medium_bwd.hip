@@ -72,10 +72,11 @@ struct __align__(16) MedBwdShared<T, true, false> {
     int next;                              // centres handed out so far by this workgroup
 };
 
-// With kLarge the kernel takes the molecules of more than 256 atoms: the atoms come type-sorted from `sorted`, the
-// workgroups of one grid column (blockIdx.y = 0 .. gridDim.y - 1) share a molecule's centres, and the gradients were
-// zeroed by the kernel that sorted the atoms.
-template <typename T, bool kLarge = false, bool kLocal = false>
+// With kShare the workgroups of one grid column (blockIdx.y = 0 .. gridDim.y - 1) share a molecule's centres, and its
+// gradients were zeroed by a kernel before this one (a form of its own: the grid's sizes in scalar registers cost the
+// plain kernel 6 %).
+// With kLarge the kernel takes the molecules of more than 256 atoms: the atoms come type-sorted from `sorted`.
+template <typename T, bool kLarge = false, bool kLocal = false, bool kShare = kLarge>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (kLocal ? 3 : 4) : (kLocal ? 1 : 2), sizeof(T) == 4 ? (kLocal ? 3 : 4) : (kLocal ? 1 : 2))))
 void aev_bwd_medium_kernel(
@@ -124,7 +125,7 @@ void aev_bwd_medium_kernel(
             z = Z[off + tid];
             type = fold_type(A[off + tid]);
             rowbits = reinterpret_cast<unsigned long long>(gin.p[type] + static_cast<size_t>(SIs[off + tid]) * kFeats);
-            if constexpr (!kLocal) {
+            if constexpr (!kLocal && !kShare) {
                 gX[off + tid] = T(0);
                 gY[off + tid] = T(0);
                 gZ[off + tid] = T(0);
@@ -318,6 +319,8 @@ void aev_bwd_medium_kernel(
             qn = rest;
         };
 
+        // (few centres for many wavefronts: shorter batches, so that every one of them gets some)
+        const int most = kShare && !kLarge ? max(1, min(kMB, (n + static_cast<int>(gridDim.y) * 4 - 1) / (static_cast<int>(gridDim.y) * 4))) : kMB;
         int dealt = 0;             // (forces in LDS) centres this wavefront has taken: it takes every fourth, by position
         int pending = -1;          // a centre that was drawn but did not fit the previous batch
         int scanned = -1;          // (large molecules) the centre whose radial pairs were queued last
@@ -326,7 +329,7 @@ void aev_bwd_medium_kernel(
             int nb = 0, used = 0;
             int pfv = 0, cv = 0;   // lane k: first pool slot and sorted position of centre k of the batch
             P.facc[lane] = Fast<T>::make4(T(0), T(0), T(0), T(0));
-            while (nb < kMB) {
+            while (nb < most) {
                 int c = pending;
                 pending = -1;
                 if (c < 0) {
@@ -336,7 +339,7 @@ void aev_bwd_medium_kernel(
                         int drawn = 0;
                         if (lane == 0) drawn = atomicAdd(&M.next, 1);
                         c = uniform(drawn);
-                        if constexpr (kLarge) c = static_cast<int>(blockIdx.y) + static_cast<int>(gridDim.y) * c;
+                        if constexpr (kShare) c = static_cast<int>(blockIdx.y) + static_cast<int>(gridDim.y) * c;
                     }
                 }
                 if (c >= n) break;
@@ -575,6 +578,19 @@ void aev_bwd_medium_kernel(
     });
 }
 
+// Zeroes the gradients of the molecules of min_atoms to 256 atoms, for launches whose workgroups share molecules.
+template <typename T>
+__global__ __launch_bounds__(256) void bwd_zero_kernel(const int32_t* __restrict__ MOs, const int32_t* __restrict__ MACs, int32_t n_mols,
+                                                       T* __restrict__ gX, T* __restrict__ gY, T* __restrict__ gZ, int min_atoms)
+{
+    const int mol = static_cast<int>(blockIdx.x);
+    const int n = MACs[mol], g = MOs[mol] + static_cast<int>(threadIdx.x);
+    if (n < min_atoms || n > kMediumMaxAtoms || static_cast<int>(threadIdx.x) >= n) return;
+    gX[g] = T(0);
+    gY[g] = T(0);
+    gZ[g] = T(0);
+}
+
 }  // namespace
 
 template <typename T>
@@ -592,9 +608,21 @@ hipError_t launch_bwd_medium(const T* X, const T* Y, const T* Z, const int32_t* 
     if (reproducible)
         aev_bwd_medium_kernel<T, false, true><<<dim3(blocks), dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, g, gX, gY, gZ, min_atoms,
                                                                                    order, walk_in_order, SortedAtoms<T>{});
-    else
-        aev_bwd_medium_kernel<T><<<dim3(blocks), dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, g, gX, gY, gZ, min_atoms,
-                                                                      order, walk_in_order, SortedAtoms<T>{});
+    else {
+        // workgroups per molecule (dense boxes of 64-256 atoms, float: 218 -> 27 us at 32 molecules, 236 -> 88 at 256,
+        // 270 -> 222 at 1,024; double 400 -> 203 us at 256); they add to gradients that are zeroed first
+        const int parts = molecule_parts(n_mols, 2 * kCUs * (sizeof(T) == 4 ? 4 : 2), 16);
+        auto launch = [&](auto kernel) {
+            kernel<<<dim3(blocks, static_cast<unsigned>(parts)), dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, g, gX, gY, gZ, min_atoms,
+                                                                                         order, walk_in_order, SortedAtoms<T>{});
+        };
+        if (parts > 1) {
+            bwd_zero_kernel<T><<<dim3(static_cast<unsigned>(n_mols)), dim3(256), 0, stream>>>(MOs, MACs, n_mols, gX, gY, gZ, min_atoms);
+            launch(aev_bwd_medium_kernel<T, false, false, true>);
+        } else {
+            launch(aev_bwd_medium_kernel<T>);
+        }
+    }
     return hipGetLastError();
 }
 

@@ -1,6 +1,8 @@
 // AEV forward for molecules of up to 64 atoms (float32 and float64): one wavefront per molecule.
 //
 // How one wavefront spends its 64 lanes
+//   (in a batch too small to fill the GPU several wavefronts share a molecule: each sorts it for itself and takes
+//            its own centres)
 //   sort     one atom per lane, lanes reordered by atom type (4-bin counting sort with ballots).  Every
 //            neighbour list built in lane order is then type-sorted, so an unordered type pair (a<=b)
 //            owns a contiguous block of (j,k) pairs of a centre.
@@ -43,7 +45,7 @@ constexpr int kRadSlots = 96;
 // the forward sums is replaced by its derivative along the per-atom vectors (VX, VY, VZ).
 // float: 4 wavefronts per SIMD (LDS 9.8 KB, <= 128 VGPRs; the kernel loses a fifth of its speed at three);
 // float kJvp: 3 (<= 168 VGPRs; its LDS, 13.4 KB, lets twelve wavefronts share a CU); double: 2 (LDS 17 KB); double kJvp: 1.
-template <typename T, bool kJvp, bool kMatrixPhase2 = false>
+template <typename T, bool kJvp, bool kShare = false, bool kMatrixPhase2 = false>
 __global__ __launch_bounds__(64 * kWavesPerBlock)
 __attribute__((amdgpu_waves_per_eu((kJvp && sizeof(T) == 4) ? 3 : (sizeof(T) == 4 ? 4 : 2) / (kJvp ? 2 : 1), (kJvp && sizeof(T) == 4) ? 3 : (sizeof(T) == 4 ? 4 : 2) / (kJvp ? 2 : 1))))
 void aev_fwd_small_kernel(
@@ -51,7 +53,7 @@ void aev_fwd_small_kernel(
     const int32_t* __restrict__ A, const int32_t* __restrict__ MOs,
     const int32_t* __restrict__ MACs, int32_t n_mols, const int32_t* __restrict__ SIs,
     const T* __restrict__ VX, const T* __restrict__ VY, const T* __restrict__ VZ, Buckets<T> out, int max_atoms,
-    const int32_t* __restrict__ order)
+    const int32_t* __restrict__ order, int log_parts)
 {
     typedef typename Fast<T>::vec4 vec4;
     typedef typename Fast<T>::vec2 vec2;
@@ -63,12 +65,17 @@ void aev_fwd_small_kernel(
     __shared__ FwdWaveLds<T, kJvp, kNB, kRadSlots, kCap> lds_all[kWavesPerBlock];
     const int lane = threadIdx.x & 63;
     const int wave = kWavesPerBlock == 1 ? 0 : uniform(threadIdx.x >> 6);    // a constant LDS base with one wavefront per workgroup
-    const int slot = blockIdx.x * kWavesPerBlock + wave;
+    static_assert(!kShare || kWavesPerBlock == 1, "blockIdx = molecule slot and part");
+    const int slot = kShare ? static_cast<int>(blockIdx.x >> log_parts) : static_cast<int>(blockIdx.x) * kWavesPerBlock + wave;
     if (slot >= n_mols) return;
     const int mol = order ? uniform(order[slot]) : slot;      // largest molecules first when an order is given
     const int n = uniform(MACs[mol]);
     const int off = uniform(MOs[mol]);
     if (n <= 0 || n > max_atoms) return;          // larger molecules belong to other kernels (max_atoms <= 64)
+    // kShare: 2^log_parts wavefronts share a molecule's centres, `share` at a time each (log_parts_of below)
+    const int share = kShare ? min(kNB, (n + (1 << log_parts) - 1) >> log_parts) : kNB;
+    const int first = kShare ? static_cast<int>(blockIdx.x & ((1u << log_parts) - 1u)) * share : 0;
+    if (kShare && first >= n) return;
     FwdWaveLds<T, kJvp, kNB, kRadSlots, kCap>& S = lds_all[wave];
     const LaneConsts<T> L = lane_consts<T>(lane);
     const unsigned long long lane_bit = 1ull << lane;
@@ -178,8 +185,8 @@ void aev_fwd_small_kernel(
     fwd_lds_init(S, lane);
     wave_lds_fence();
 
-    for (int c0 = 0; c0 < n; c0 += kNB) {
-        const int nb = min(kNB, n - c0);
+    for (int c0 = first; c0 < n; c0 += kShare ? share << log_parts : kNB) {
+        const int nb = min(share, n - c0);
         unsigned overflow = 0;
 
         // ------------------------------------------------ scan steps: G centres x W partners
@@ -323,6 +330,17 @@ void aev_fwd_small_kernel(
 
 }  // namespace
 
+// Wavefronts per molecule (as a power of two).  organic molecules, 16 / 8 / 12 / 4 wavefronts per CU resident (float,
+// double, and their Jacobian-vector forms); forward float 100 -> 24 us at 1,024 molecules, 106 -> 47 at 4,096,
+// 112 -> 78 at 8,192 (two each), and slower from 16,384 on (137 -> 150 with two); the Jacobian-vector form
+// 131 -> 31 us at 1,024, double forward 162 -> 51 us.  The rows are the same bits for any number.
+template <typename T, bool kJvp>
+static int log_parts_of(int32_t n_mols)
+{
+    constexpr int kResident = kCUs * (sizeof(T) == 4 ? (kJvp ? 12 : 16) : (kJvp ? 4 : 8));
+    return __builtin_ctz(molecule_parts(n_mols, 4 * kResident, 8));
+}
+
 template <typename T>
 hipError_t launch_fwd_small(const T* X, const T* Y, const T* Z, const int32_t* A, const int32_t* MOs,
                             const int32_t* MACs, int32_t n_mols, const int32_t* SIs, Buckets<T> out,
@@ -330,6 +348,7 @@ hipError_t launch_fwd_small(const T* X, const T* Y, const T* Z, const int32_t* A
 {
     if (n_mols <= 0) return hipSuccess;
     const unsigned blocks = (static_cast<unsigned>(n_mols) + kWavesPerBlock - 1u) / kWavesPerBlock;
+    const int log_parts = log_parts_of<T, false>(n_mols);
 #ifdef KHAN_CHECK_BUILD
     if constexpr (sizeof(T) == 4) {
         // check build only: KHAN_AEV_PHASE2=matrix (read once) selects the variant that sums the angular records on the
@@ -339,14 +358,15 @@ hipError_t launch_fwd_small(const T* X, const T* Y, const T* Z, const int32_t* A
             return v != nullptr && std::strcmp(v, "matrix") == 0;
         }();
         if (matrix_phase2) {
-            aev_fwd_small_kernel<T, false, true><<<dim3(blocks), dim3(64 * kWavesPerBlock), 0, stream>>>(
-                X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, out, max_atoms < 64 ? max_atoms : 64, order);
+            aev_fwd_small_kernel<T, false, true, true><<<dim3(blocks << log_parts), dim3(64 * kWavesPerBlock), 0, stream>>>(
+                X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, out, max_atoms < 64 ? max_atoms : 64, order, log_parts);
             return hipGetLastError();
         }
     }
 #endif
-    aev_fwd_small_kernel<T, false><<<dim3(blocks), dim3(64 * kWavesPerBlock), 0, stream>>>(
-        X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, out, max_atoms < 64 ? max_atoms : 64, order);
+    const auto kernel = log_parts ? aev_fwd_small_kernel<T, false, true> : aev_fwd_small_kernel<T, false>;
+    kernel<<<dim3(blocks << log_parts), dim3(64 * kWavesPerBlock), 0, stream>>>(
+        X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, out, max_atoms < 64 ? max_atoms : 64, order, log_parts);
     return hipGetLastError();
 }
 
@@ -357,8 +377,10 @@ hipError_t launch_jvp_small(const T* X, const T* Y, const T* Z, const int32_t* A
 {
     if (n_mols <= 0) return hipSuccess;
     const unsigned blocks = (static_cast<unsigned>(n_mols) + kWavesPerBlock - 1u) / kWavesPerBlock;
-    aev_fwd_small_kernel<T, true><<<dim3(blocks), dim3(64 * kWavesPerBlock), 0, stream>>>(
-        X, Y, Z, A, MOs, MACs, n_mols, SIs, VX, VY, VZ, out, kSmallMaxAtoms, order);
+    const int log_parts = log_parts_of<T, true>(n_mols);
+    const auto kernel = log_parts ? aev_fwd_small_kernel<T, true, true> : aev_fwd_small_kernel<T, true>;
+    kernel<<<dim3(blocks << log_parts), dim3(64 * kWavesPerBlock), 0, stream>>>(
+        X, Y, Z, A, MOs, MACs, n_mols, SIs, VX, VY, VZ, out, kSmallMaxAtoms, order, log_parts);
     return hipGetLastError();
 }
 

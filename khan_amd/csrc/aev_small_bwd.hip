@@ -24,6 +24,8 @@
 // Finally every lane stores the gradient of its own atom: no global atomics, no pre-zeroed output.
 // The derivative is the algebraically reduced form (no acos, no 1/(1+cos) factor); reference:
 // gpu_featurizer/kernel_cpu.cpp:217-366.
+#include <type_traits>
+
 #include "aev_bwd_batch.h"
 
 namespace khan {
@@ -44,8 +46,11 @@ struct __align__(16) BwdLds {
 };
 
 // float: 4 wavefronts per SIMD (LDS 10.2 KB, 127 registers); double: 2 (LDS 20.4 KB, twice the registers)
-template <typename T>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2, sizeof(T) == 4 ? 4 : 2)))
+// kW wavefronts share a molecule (1: as described above).  Each sorts it for itself; they share the steps of the first
+// sweep and take the batches in turn, every one sums forces in an array of its own, and the first adds the arrays up in
+// order: no atomics, and the same bits on every run.
+template <typename T, int kW>
+__global__ __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 4 : 2, sizeof(T) == 4 ? 4 : 2)))
 void aev_bwd_small_kernel(
     const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
     const int32_t* __restrict__ A, const int32_t* __restrict__ MOs,
@@ -54,8 +59,11 @@ void aev_bwd_small_kernel(
     const int32_t* __restrict__ order)
 {
     typedef typename Fast<T>::vec4 vec4;
-    __shared__ BwdLds<T> S;
-    const int lane = threadIdx.x;
+    __shared__ BwdLds<T> lds_all[kW];
+    const int lane = threadIdx.x & 63;
+    const int wave = kW == 1 ? 0 : uniform(threadIdx.x >> 6);
+    __shared__ int counts[kW > 1 ? 64 : 1];
+    BwdLds<T>& S = lds_all[wave];
     if (static_cast<int>(blockIdx.x) >= n_mols) return;
     const int mol = order ? uniform(order[blockIdx.x]) : static_cast<int>(blockIdx.x);   // largest first when ordered
     const int n = uniform(MACs[mol]);
@@ -135,7 +143,7 @@ void aev_bwd_small_kernel(
     int cord, m_at;     // lane p: sorted lane of the centre at position p, and its partner count
     {
         int m_mine = 0;
-        for (int s0 = 0; s0 < n; s0 += G) {
+        for (int s0 = wave * G; s0 < n; s0 += kW * G) {
             const int i = s0 + grp;
             const vec4 ai = S.atom[min(i, 63)];
             const T dx = ai.x - aj.x, dy = ai.y - aj.y, dz = ai.z - aj.z;
@@ -175,6 +183,11 @@ void aev_bwd_small_kernel(
                 S.force[2][i] += cfz;
             }
         }
+        if constexpr (kW > 1) {           // every wavefront counted its own steps' centres
+            if (have && ((lane >> (6 - logW)) & (kW - 1)) == wave) counts[lane] = m_mine;
+            __syncthreads();
+            m_mine = have ? counts[lane] : 0;
+        }
         const int key = have ? ((m_mine << 6) | (63 - lane)) : -1;
         int rank = 0;
         for (int l = 0; l < n; ++l) rank += (lane_read(key, l) > key) ? 1 : 0;
@@ -183,6 +196,8 @@ void aev_bwd_small_kernel(
         m_at = lane_push(rank, m_mine);
     }
 
+    const int most = kW == 1 ? kSmallBwdCentres<T> : min(kSmallBwdCentres<T>, (n + kW - 1) / kW);
+    int turn = 0;                         // batches so far, modulo kW
     for (int c0 = 0, nb = 0; c0 < n; c0 += nb) {
         // centres of this batch: up to kSmallBwdCentres, lists fitting the 64 lanes; pf[b] = first list slot of centre b
         int pf[kB + 1];
@@ -194,7 +209,7 @@ void aev_bwd_small_kernel(
 #pragma unroll
             for (int k = 0; k < kB; ++k) {
                 int m = 0;
-                if (open && k < kSmallBwdCentres<T> && c0 + k < n) {
+                if (open && k < most && c0 + k < n) {
                     m = lane_read(m_at, min(c0 + k, 63));
                     if (k > 0 && tot + m > 64) {
                         open = false;
@@ -208,6 +223,11 @@ void aev_bwd_small_kernel(
                 tot += m;
                 pf[k + 1] = tot;
             }
+        }
+        if constexpr (kW > 1) {           // the wavefronts take the batches in turn
+            const int whose = turn;
+            turn = (turn + 1) & (kW - 1);
+            if (whose != wave) continue;
         }
         const int total = pf[kB];
         unsigned overflow = 0;
@@ -331,11 +351,19 @@ void aev_bwd_small_kernel(
     }
 
     // ------------------------------------------------------------ every lane stores its own atom
-    wave_lds_fence();
-    if (have) {
-        gX[off + orig] = S.force[0][lane];
-        gY[off + orig] = S.force[1][lane];
-        gZ[off + orig] = S.force[2][lane];
+    if constexpr (kW > 1) __syncthreads();
+    else wave_lds_fence();
+    if (have && wave == 0) {
+        T f[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            f[d] = S.force[d][lane];
+#pragma unroll
+            for (int w = 1; w < kW; ++w) f[d] += lds_all[w].force[d][lane];
+        }
+        gX[off + orig] = f[0];
+        gY[off + orig] = f[1];
+        gZ[off + orig] = f[2];
     }
 }
 
@@ -347,7 +375,20 @@ hipError_t launch_bwd_small(const T* X, const T* Y, const T* Z, const int32_t* A
                             T* gX, T* gY, T* gZ, int max_atoms, const int32_t* order, hipStream_t stream)
 {
     if (n_mols <= 0) return hipSuccess;
-    aev_bwd_small_kernel<T><<<dim3(static_cast<unsigned>(n_mols)), dim3(64), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, g, gX, gY, gZ, max_atoms < 64 ? max_atoms : 64, order);
+    // wavefronts per molecule: organic molecules, float 95 -> 28 us at 1,024 molecules (eight each), 100 -> 52 at 3,000
+    // (four), 102 -> 58 at 4,096 (two), double 173 -> 61 us at 1,024; the workgroup's slowest wavefront ends it, so the
+    // line lies lower than for the forward pass (4,096 molecules with four each: 70 us)
+    auto launch = [&](auto waves) {
+        constexpr int kW = decltype(waves)::value;
+        aev_bwd_small_kernel<T, kW><<<dim3(static_cast<unsigned>(n_mols)), dim3(64 * kW), 0, stream>>>(
+            X, Y, Z, A, MOs, MACs, n_mols, SIs, g, gX, gY, gZ, max_atoms < 64 ? max_atoms : 64, order);
+    };
+    constexpr int kMost = sizeof(T) == 4 ? 8 : 4;                                          // (double: eight would take 160 KB of LDS)
+    const int parts = molecule_parts(n_mols, kCUs * (sizeof(T) == 4 ? 3 * 16 : 4 * 8), kMost);
+    if (parts == 8) launch(std::integral_constant<int, kMost>{});
+    else if (parts == 4) launch(std::integral_constant<int, 4>{});
+    else if (parts == 2) launch(std::integral_constant<int, 2>{});
+    else launch(std::integral_constant<int, 1>{});
     return hipGetLastError();
 }
 

@@ -25,6 +25,19 @@ hipError_t launch_jvp_generic(const T* X, const T* Y, const T* Z, const int32_t*
                               const int32_t* SIs, const T* VX, const T* VY, const T* VZ, Buckets<T> out,
                               int min_atoms, const int32_t* order, hipStream_t stream);
 
+// How many wavefronts (workgroups) share each molecule's centres: doubled up to `most` while the launch stays at or
+// below `fill`, a small multiple of what the GPU runs at once.  A molecule that one wavefront works through alone takes
+// as long as its atoms in sequence, whatever the batch: in a batch of a thousand molecules a launch lasted as long as
+// its largest molecule (0.10 ms of 26 atoms) with most of the GPU idle.  Beyond that multiple the work every wavefront
+// repeats (loading and sorting the molecule's atoms) costs more than the shorter tail gives.
+inline int molecule_parts(int32_t n_mols, int64_t fill, int most)
+{
+    int parts = 1;
+    while (parts < most && static_cast<int64_t>(n_mols) * parts * 2 <= fill) parts *= 2;
+    return parts;
+}
+constexpr int kCUs = 256;
+
 // ---- AEV forward for molecules of up to 64 atoms (larger molecules are skipped) ----
 constexpr int kSmallMaxAtoms = 64;      // what one wavefront can hold
 // where a medium-molecule kernel exists, molecules above this size go to it: one wavefront working through a

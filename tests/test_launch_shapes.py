@@ -1,0 +1,61 @@
+"""The launch shapes that depend on the size of the batch, at the sizes where they change: the same molecules in a batch
+that gives each of them more wavefronts or workgroups and in one that does not."""
+import numpy as np
+import pytest
+
+from khan_amd import datagen
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from khan_amd import _lib, ops as _ops
+    _lib.load()
+    return _ops
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+
+
+def passes(ops, b, n_mols, dtype, upstream, vectors):
+    """Rows, gradients and Jacobian-vector rows, in atom order, of the first n_mols molecules of batch b run alone."""
+    n = int(b.MOs[n_mols - 1] + b.MACs[n_mols - 1])
+    X, Y, Z = (dev(v[:n]).to(dtype) for v in (b.X, b.Y, b.Z))
+    macs, mos = ops.mol_offsets(dev(b.mol_idxs[:n]), n_mols)
+    sc, ga, ac = ops.ani_sort(dev(b.A[:n]))
+    acs, order, ga = ac.cpu().tolist(), ops.size_order(macs), ga.long()
+    classes = order[-4:].cpu()
+    args = (X, Y, Z, dev(b.A[:n]), mos, macs, sc, acs)
+    rows = torch.cat(ops.featurize(*args, order=order, size_classes=classes)).view(-1, 384)[ga]
+    buckets = torch.empty((n, 384), dtype=dtype, device=DEV)
+    buckets[ga] = upstream[:n]
+    grads = torch.stack(ops.featurize_grad(*args, *torch.split(buckets.view(-1), [c * 384 for c in acs]), order=order, size_classes=classes), dim=1)
+    jvp = torch.cat(ops.featurize_grad_inverse(*args, *(v[:n].contiguous() for v in vectors), order=order, size_classes=classes)).view(-1, 384)[ga]
+    return rows, grads, jvp
+
+
+# sizes on both sides of the lines at which a molecule gets 2, 4, 8 (16) wavefronts or workgroups
+@pytest.mark.parametrize("kind,dtype,most,sizes", [
+    ("organic", torch.float32, 16500, (1, 1023, 1025, 2049, 4097, 8192)),
+    ("organic", torch.float64, 8300, (1, 511, 1025, 2048, 4096)),
+    ("boxes", torch.float32, 2200, (1, 127, 257, 1024)),
+    ("boxes", torch.float64, 600, (1, 63, 65, 256)),
+])
+def test_molecules_shared_by_several_wavefronts(ops, kind, dtype, most, sizes):
+    b = datagen.make_batch(kind, most)
+    gen = torch.Generator(device=DEV)
+    gen.manual_seed(3)
+    upstream = torch.randn((b.n_atoms, 384), dtype=dtype, device=DEV, generator=gen)
+    vectors = torch.randn((3, b.n_atoms), dtype=dtype, device=DEV, generator=gen)
+    rows, grads, jvp = passes(ops, b, most, dtype, upstream, vectors)
+    tol = 2e-6 if dtype == torch.float32 else 4e-15       # forces are sums in another order
+    for n_mols in sizes:
+        r, g, j = passes(ops, b, n_mols, dtype, upstream, vectors)
+        n = r.shape[0]
+        print("   %s %s, %d molecules" % (kind, dtype, n_mols), flush=True)
+        assert torch.equal(r, rows[:n]) and torch.equal(j, jvp[:n])
+        assert float((g - grads[:n]).abs().max()) <= tol * float(grads[:n].abs().max())
