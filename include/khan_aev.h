@@ -80,6 +80,18 @@ int khan_mol_offsets(const int32_t *mol_idxs, int64_t n_atoms, int32_t n_mols, i
 int khan_ani_sort(const int32_t *atomic_numbers, int64_t n_atoms, int32_t *scatter_idxs,
                   int32_t *gather_idxs, int32_t *atom_counts, khan_stream_t stream);
 
+/* khan_mol_offsets, khan_ani_sort and khan_size_order of one batch together (no counterpart; what a caller runs once per
+ * batch before the passes): macs, mos, scatter_idxs, gather_idxs, atom_counts[4] and order[n_mols + 520] as those give
+ * them, in three launches (one for a batch of up to 4,096 atoms and 2,048 molecules).  Allocates nothing: `workspace` is
+ * khan_prepare_batch_workspace_bytes(n_atoms) bytes of device memory, 16-byte aligned.  counts_pinned (or null): eight
+ * ints of host memory that the GPU can write (hipHostMalloc), which receive the four atom counts and the four size-class
+ * totals (order[-4:]) when the work is done, in place of a copy.  n_mols = 0: nothing is written but atom_counts and the
+ * indices. */
+int64_t khan_prepare_batch_workspace_bytes(int64_t n_atoms);
+int khan_prepare_batch(const int32_t *mol_idxs, const int32_t *atomic_numbers, int64_t n_atoms, int32_t n_mols,
+                       int32_t *macs, int32_t *mos, int32_t *scatter_idxs, int32_t *gather_idxs, int32_t *atom_counts,
+                       int32_t *order, void *workspace, int32_t *counts_pinned, khan_stream_t stream);
+
 /* Featurize (op: gpu_featurizer/ani_op.cpp:95-117; functor: functor_op.h:8-25, functor_op_gpu.cu:57-88;
  * kernel: kernel_cpu.cpp:406-537 / kernel.cu:72-268).
  * in : xs, ys, zs [n_atoms]; as [n_atoms]; mos, macs [n_mols]; sis = scatter_idxs [n_atoms];

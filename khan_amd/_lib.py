@@ -40,6 +40,8 @@ _SIGNATURES = {
     "khan_get_parameters": (None, [ctypes.POINTER(ctypes.c_float)] * 4),
     "khan_mol_offsets": (ctypes.c_int, [_ptr, ctypes.c_int64, ctypes.c_int32, _ptr, _ptr, _ptr]),
     "khan_ani_sort": (ctypes.c_int, [_ptr, ctypes.c_int64, _ptr, _ptr, _ptr, _ptr]),
+    "khan_prepare_batch_workspace_bytes": (ctypes.c_int64, [ctypes.c_int64]),
+    "khan_prepare_batch": (ctypes.c_int, [_ptr, _ptr, ctypes.c_int64, ctypes.c_int32] + [_ptr] * 9),
     "khan_featurize_f32": (ctypes.c_int, _featurize_sig()),
     "khan_featurize_f64": (ctypes.c_int, _featurize_sig()),
     "khan_featurize_f32_noalloc": (ctypes.c_int, _featurize_sig()),

@@ -200,10 +200,10 @@ class DeviceBatch:
 
     def host_counts(self):
         """-> (atoms per type [4], the size order on the device, molecules per size class [4] on the host): what the
-        host has to know before it can launch the passes.  One 32-byte copy, enqueued by the feeder behind the
-        sort; this waits for it."""
+        host has to know before it can launch the passes.  The sort writes them to pinned memory; this waits for it."""
         self.ready.synchronize()
-        return self.counts_pinned[0:4].tolist(), self.size_order, self.counts_pinned[4:8].clone()
+        counts = self.counts_pinned.tolist()
+        return counts[0:4], self.size_order, counts[4:8]
 
     @classmethod
     def from_device_arrays(cls, xs, ys, zs, atom_types, mol_idxs, n_mols):
@@ -221,12 +221,9 @@ class DeviceBatch:
         """Offsets, type sort, size order and the copy of the counts for the arrays already in place; records `ready`."""
         import torch
         from . import ops
-        self.mol_atom_counts, self.mol_offsets = ops.mol_offsets(self.mol_idxs, self.n_mols)
-        self.scatter_idxs, self.gather_idxs, self.atom_counts = ops.ani_sort(self.atom_types)
-        self.size_order = ops.size_order(self.mol_atom_counts)
-        self.counts_pinned = torch.empty(8, dtype=torch.int32, pin_memory=True)     # from the pinned-memory cache
-        self.counts_pinned[0:4].copy_(self.atom_counts, non_blocking=True)
-        self.counts_pinned[4:8].copy_(self.size_order[-4:], non_blocking=True)
+        self.counts_pinned = torch.empty(8, dtype=torch.int32, pin_memory=True)     # from the pinned-memory cache; the sort writes it
+        (self.mol_atom_counts, self.mol_offsets, self.scatter_idxs, self.gather_idxs, self.atom_counts,
+         self.size_order) = ops.prepare_batch(self.mol_idxs, self.atom_types, self.n_mols, self.counts_pinned)
         self.ready = torch.cuda.Event()
         self.ready.record()
 

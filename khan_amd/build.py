@@ -3,6 +3,7 @@
   khan_amd/csrc/libkhan_aev.so      HIP kernels + C ABI, compiled for gfx950 with hipcc
   khan_amd/csrc/libkhan_datagen.so  host-only synthetic batch generator (gcc)
   khan_amd/csrc/libkhan_host.so     host-only batch assembly (gcc, OpenMP)
+  khan_amd/csrc/_khan_ops.so        the tensor side of khan_amd.ops (g++, against the installed torch)
 
 plus csrc/check_build/libkhan_aev.so, the same library with the check switches compiled in (`build_check_variant`),
 which only the tests of those switches load.
@@ -297,8 +298,41 @@ def build_host():
     return out
 
 
+OPS_SOURCES = ("torch_ops.cpp", os.path.join(ROOT, "include", "khan_aev.h"))
+OPS_LIBRARY = os.path.join(CSRC, "_khan_ops.so")
+
+
+def ops_digest():
+    """Digest of the native tensor layer's sources and of the torch it is built against."""
+    import torch
+    h = hashlib.sha256(torch.__version__.encode())
+    for name in OPS_SOURCES:
+        with open(os.path.join(CSRC, name)) as f:
+            h.update(_code_only(f.read()).encode())
+    return h.hexdigest()[:16]
+
+
+def ops_library_is_current():
+    return os.path.exists(OPS_LIBRARY) and library_stamp(OPS_LIBRARY) == ops_digest()
+
+
+def build_torch_ops():
+    """csrc/_khan_ops.so: the tensor side of khan_amd.ops (host code; no GPU code in it), an extension module of Python."""
+    import sysconfig
+    from torch.utils import cpp_extension
+    if os.path.exists(stamp_path(OPS_LIBRARY)):
+        os.remove(stamp_path(OPS_LIBRARY))
+    includes = ["-isystem" + p for p in cpp_extension.include_paths() + [sysconfig.get_paths()["include"], "/opt/rocm/include"]]
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+          "-DTORCH_EXTENSION_NAME=_khan_ops"] + includes + [os.path.join(CSRC, "torch_ops.cpp"), "-o", OPS_LIBRARY] +
+         ["-L" + p for p in cpp_extension.library_paths()] + ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-ldl"])
+    with open(stamp_path(OPS_LIBRARY), "w") as f:
+        f.write(ops_digest() + "\n")
+    return OPS_LIBRARY
+
+
 def build_all():
-    return [build_hip(), build_check_variant(), build_datagen(), build_host()]
+    return [build_hip(), build_check_variant(), build_datagen(), build_host(), build_torch_ops()]
 
 
 if __name__ == "__main__":

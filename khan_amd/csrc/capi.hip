@@ -488,6 +488,22 @@ int khan_ani_sort(const int32_t* atomic_numbers, int64_t n_atoms, int32_t* scatt
                                             as_stream(stream)));
 }
 
+int64_t khan_prepare_batch_workspace_bytes(int64_t n_atoms) { return static_cast<int64_t>(khan::prepare_workspace_bytes(n_atoms)); }
+
+int khan_prepare_batch(const int32_t* mol_idxs, const int32_t* atomic_numbers, int64_t n_atoms, int32_t n_mols, int32_t* macs,
+                       int32_t* mos, int32_t* scatter_idxs, int32_t* gather_idxs, int32_t* atom_counts, int32_t* order,
+                       void* workspace, int32_t* counts_pinned, khan_stream_t stream)
+{
+    if (n_atoms < 0 || n_mols < 0 || !atom_counts) return KHAN_ERR_INVALID_ARG;
+    if (n_atoms > INT32_MAX) return KHAN_ERR_TOO_LARGE;
+    if (n_atoms > 0 && (!mol_idxs || !atomic_numbers || !scatter_idxs || !gather_idxs)) return KHAN_ERR_INVALID_ARG;
+    if (n_mols > 0 && (!macs || !mos || !order || !workspace || (reinterpret_cast<uintptr_t>(workspace) & 15u))) return KHAN_ERR_INVALID_ARG;
+    if (n_mols == 0)        // the sort alone (counts_pinned is left to the caller: there are no passes to launch)
+        return hip_status(khan::launch_ani_sort(atomic_numbers, n_atoms, scatter_idxs, gather_idxs, atom_counts, as_stream(stream)));
+    return hip_status(khan::launch_prepare(mol_idxs, atomic_numbers, n_atoms, n_mols, macs, mos, scatter_idxs, gather_idxs, atom_counts,
+                                           order, static_cast<int32_t*>(workspace), counts_pinned, as_stream(stream)));
+}
+
 int khan_featurize_f32(const float* xs, const float* ys, const float* zs, const int32_t* as,
                        const int32_t* mos, const int32_t* macs, int32_t n_mols, const int32_t* sis,
                        float* h, float* c, float* n, float* o, const int32_t* acs_host,

@@ -123,6 +123,12 @@ __host__ __device__ __forceinline__ int size_bin(int n)
     return kSizeBins - 1 - c;
 }
 hipError_t launch_size_order(const int32_t* MACs, int32_t n_mols, int32_t* order, hipStream_t stream);
+// the three together (n_mols > 0), with a workspace of the caller's; host8 (or null): host memory that the GPU can write,
+// which receives the four atom counts and the four class totals
+size_t prepare_workspace_bytes(int64_t n_atoms);
+hipError_t launch_prepare(const int32_t* mol_idxs, const int32_t* A, int64_t n_atoms, int32_t n_mols, int32_t* MACs, int32_t* MOs,
+                          int32_t* scatter, int32_t* gather, int32_t* counts4, int32_t* order, int32_t* ws, int32_t* host8,
+                          hipStream_t stream);
 
 // zeros to an array of n elements (outputs that no molecule covers)
 template <typename T>

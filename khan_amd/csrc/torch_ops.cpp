@@ -1,0 +1,448 @@
+// The tensor side of khan_amd.ops in native code: argument checks, output allocation and the call into libkhan_aev.so.
+//
+// A call on a small batch is bound by the host: the checks, the allocations and the marshalling of a dozen pointers took
+// 20-35 us per call in Python (ctypes) and take 3-5 us here, which is what the launch itself costs.  The library is opened
+// by path (init), so that a build named by KHAN_AEV_LIBRARY is used here too; nothing is linked against it.
+#include <dlfcn.h>
+
+#include <array>
+#include <string>
+#include <vector>
+
+#include <ATen/hip/CachingHostAllocator.h>
+#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/extension.h>
+
+#include "../../include/khan_aev.h"
+
+namespace py = pybind11;
+using at::Tensor;
+
+namespace {
+
+#define KHAN_API(X)                                                                                                    \
+    X(khan_status_string) X(khan_last_hip_error) X(khan_mol_offsets) X(khan_ani_sort) X(khan_size_order)               \
+    X(khan_prepare_batch_workspace_bytes) X(khan_prepare_batch)                                                        \
+    X(khan_featurize_f32) X(khan_featurize_f64) X(khan_featurize_ordered_f32) X(khan_featurize_ordered_f64)            \
+    X(khan_featurize_grad_f32) X(khan_featurize_grad_f64) X(khan_featurize_grad_ordered_f32)                           \
+    X(khan_featurize_grad_ordered_f64) X(khan_featurize_grad_inverse_f32) X(khan_featurize_grad_inverse_f64)           \
+    X(khan_featurize_grad_inverse_ordered_f32) X(khan_featurize_grad_inverse_ordered_f64)                              \
+    X(khan_ani_charge_f32) X(khan_ani_charge_f64) X(khan_ani_charge_grad_f32) X(khan_ani_charge_grad_f64)              \
+    X(khan_ani_charge_grad_xyz_f32) X(khan_ani_charge_grad_xyz_f64) X(khan_ani_charge_all_f32)                         \
+    X(khan_ani_charge_all_f64) X(khan_mol_energy_f32) X(khan_mol_energy_f64) X(khan_mol_energy_grad_f32)               \
+    X(khan_mol_energy_grad_f64) X(khan_atomic_networks_packed_bytes) X(khan_atomic_networks_f32)
+
+struct Api {
+#define X(name) decltype(&::name) name = nullptr;
+    KHAN_API(X)
+#undef X
+} api;
+
+PyObject* khan_error = nullptr;
+
+void init(const std::string& path, py::object error_type)
+{
+    void* lib = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
+    if (!lib) throw std::runtime_error(dlerror());
+#define X(name)                                                                                  \
+    api.name = reinterpret_cast<decltype(api.name)>(dlsym(lib, #name));                          \
+    if (!api.name) throw std::runtime_error(path + " does not export " #name);
+    KHAN_API(X)
+#undef X
+    khan_error = error_type.release().ptr();
+}
+
+void check(int status)
+{
+    if (status == KHAN_OK) return;
+    const std::string detail = api.khan_last_hip_error();
+    const std::string msg = std::string("libkhan_aev: ") + api.khan_status_string(status) + (detail.empty() ? "" : " (" + detail + ")");
+    PyErr_SetString(khan_error, msg.c_str());
+    throw py::error_already_set();
+}
+
+// the launch, with the interpreter's lock given back as a foreign-function call gives it back
+template <typename Fn, typename... Args>
+void call(Fn fn, Args... args)
+{
+    int status;
+    {
+        py::gil_scoped_release release;
+        status = fn(args...);
+    }
+    check(status);
+}
+
+khan_stream_t stream() { return c10::hip::getCurrentHIPStream().stream(); }
+
+void dev(const Tensor& t, at::ScalarType dtype, const char* name)
+{
+    if (!t.is_cuda()) throw py::type_error(std::string(name) + " must be a CUDA tensor");
+    if (t.scalar_type() != dtype)
+        throw py::type_error(std::string(name) + " must have dtype " + c10::toString(dtype) + ", got " + c10::toString(t.scalar_type()));
+    if (t.dim() != 1) throw py::value_error(std::string(name) + " must be rank 1 (flat), got rank " + std::to_string(t.dim()));
+    if (!t.is_contiguous()) throw py::value_error(std::string(name) + " must be contiguous");
+}
+
+void same_size(bool ok, const char* what)
+{
+    if (!ok) throw py::value_error(what);
+}
+
+template <typename T>
+T* ptr(const Tensor& t)
+{
+    return t.numel() > 0 ? static_cast<T*>(t.data_ptr()) : nullptr;
+}
+
+at::ScalarType float_dtype(const Tensor& x, const char* what)
+{
+    const auto dt = x.scalar_type();
+    if (dt != at::kFloat && dt != at::kDouble) throw py::type_error(std::string(what) + " must be float32 or float64, got " + c10::toString(dt));
+    return dt;
+}
+
+struct Counts {
+    int32_t v[4];
+    int64_t sum() const { return static_cast<int64_t>(v[0]) + v[1] + v[2] + v[3]; }
+};
+
+// four ints from a tensor (a device tensor is copied) or a sequence
+Counts counts4(const py::object& o, const char* what)
+{
+    Counts c{};
+    if (THPVariable_Check(o.ptr())) {
+        const Tensor t = THPVariable_Unpack(o.ptr()).detach().cpu().to(at::kInt).contiguous();
+        same_size(t.numel() == 4, what);
+        std::copy_n(t.data_ptr<int32_t>(), 4, c.v);
+    } else {
+        int k = 0;
+        for (const auto& item : o) {
+            same_size(k < 4, what);
+            c.v[k++] = item.cast<int32_t>();
+        }
+        same_size(k == 4, what);
+    }
+    return c;
+}
+
+constexpr int64_t kFeats = 384;
+constexpr int64_t kOrderExtra = 520;
+
+// ---------------------------------------------------------------------------------------------- preparation
+// -> (macs, mos, scatter_idxs, gather_idxs, atom_counts, order), slices of one allocation
+std::vector<Tensor> prepare_batch(const Tensor& mol_idxs, const Tensor& types, int64_t n_mols, const c10::optional<Tensor>& counts_pinned)
+{
+    dev(mol_idxs, at::kInt, "mol_idxs");
+    dev(types, at::kInt, "atomic_numbers");
+    const int64_t n = types.numel();
+    same_size(mol_idxs.numel() == n, "mol_idxs and atomic_numbers must have the same length");
+    same_size(n_mols >= 0, "n_mols must not be negative");
+    const auto up4 = [](int64_t v) { return (v + 3) & ~int64_t(3); };
+    const int64_t ws = up4(api.khan_prepare_batch_workspace_bytes(n) / 4);
+    const int64_t sizes[6] = {n_mols, n_mols, n, n, 4, n_mols + kOrderExtra};
+    int64_t total = ws;
+    for (const int64_t s : sizes) total += up4(s);
+    const Tensor all = at::empty({total}, types.options());
+    std::vector<Tensor> out;
+    int64_t at = ws;
+    for (const int64_t s : sizes) {
+        out.push_back(all.narrow(0, at, s));
+        at += up4(s);
+    }
+    const khan_stream_t st = stream();
+    int32_t* host = nullptr;
+    if (counts_pinned) {
+        const Tensor& h = *counts_pinned;
+        if (h.scalar_type() != at::kInt || h.numel() != 8 || !h.is_contiguous() || !h.is_pinned())
+            throw py::value_error("counts_pinned must hold 8 int32 in pinned memory");
+        host = h.data_ptr<int32_t>();
+        if (n_mols == 0) std::fill_n(host, 8, 0);
+        // the GPU writes to it: not to be handed out again before this work is done, whoever drops the tensor
+        at::getHostAllocator(at::kCUDA)->record_event(h.data_ptr(), h.storage().data_ptr().get_context(),
+                                                      c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().unwrap());
+    }
+    call(api.khan_prepare_batch, ptr<const int32_t>(mol_idxs), ptr<const int32_t>(types), n, static_cast<int32_t>(n_mols),
+         ptr<int32_t>(out[0]), ptr<int32_t>(out[1]), ptr<int32_t>(out[2]), ptr<int32_t>(out[3]), ptr<int32_t>(out[4]),
+         ptr<int32_t>(out[5]), static_cast<void*>(all.data_ptr()), host, st);
+    return out;
+}
+
+// ---------------------------------------------------------------------------------------------- AEV passes
+struct Atoms {
+    at::ScalarType dt;
+    int64_t n;
+    Counts acs;
+    const int32_t* order = nullptr;
+    bool ordered = false, classes_known = false;
+    Counts classes{};
+    const int32_t* classes_ptr() const { return classes_known ? classes.v : nullptr; }
+};
+
+Atoms check_atoms(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos, const Tensor& macs,
+                  const Tensor& sis, const py::object& acs, const c10::optional<Tensor>& order, const py::object& size_classes)
+{
+    Atoms a;
+    a.dt = float_dtype(xs, "coordinates");
+    dev(xs, a.dt, "xs"); dev(ys, a.dt, "ys"); dev(zs, a.dt, "zs");
+    dev(as, at::kInt, "as"); dev(mos, at::kInt, "mos"); dev(macs, at::kInt, "macs"); dev(sis, at::kInt, "sis");
+    a.n = xs.numel();
+    same_size(ys.numel() == a.n && zs.numel() == a.n && as.numel() == a.n && sis.numel() == a.n, "xs, ys, zs, as, sis must have the same length");
+    same_size(mos.numel() == macs.numel(), "mos and macs must have the same length");
+    a.acs = counts4(acs, "acs must hold 4 atom counts");
+    if (a.acs.sum() != a.n)
+        throw py::value_error("sum(acs)=" + std::to_string(a.acs.sum()) + " does not match the number of atoms " + std::to_string(a.n));
+    if (order) {
+        dev(*order, at::kInt, "order");
+        same_size(order->numel() == macs.numel() + kOrderExtra, "order must come from size_order(macs) of this batch");
+        a.order = ptr<const int32_t>(*order);
+        a.ordered = true;
+        if (!size_classes.is_none()) {
+            a.classes = counts4(size_classes, "size_classes must hold 4 counts");
+            a.classes_known = true;
+        }
+    }
+    return a;
+}
+
+// four consecutive slices of one array, acs[t] * 384 elements each
+std::vector<Tensor> buckets(const Tensor& packed, const Counts& acs, int64_t width = kFeats)
+{
+    std::vector<Tensor> out;
+    int64_t at = 0;
+    for (const int32_t c : acs.v) {
+        out.push_back(packed.narrow(0, at, c * width));
+        at += c * width;
+    }
+    return out;
+}
+
+template <typename T, typename Plain, typename Ordered>
+void run_forward(Plain plain, Ordered ordered, const Atoms& a, const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as,
+                 const Tensor& mos, const Tensor& macs, const Tensor& sis, const std::vector<Tensor>& o)
+{
+    const khan_stream_t st = stream();
+    const int32_t m = static_cast<int32_t>(mos.numel());
+    if (a.ordered)
+        call(ordered, ptr<const T>(xs), ptr<const T>(ys), ptr<const T>(zs), ptr<const int32_t>(as), ptr<const int32_t>(mos), ptr<const int32_t>(macs),
+             m, ptr<const int32_t>(sis), ptr<T>(o[0]), ptr<T>(o[1]), ptr<T>(o[2]), ptr<T>(o[3]), a.acs.v, a.order, a.classes_ptr(), st);
+    else
+        call(plain, ptr<const T>(xs), ptr<const T>(ys), ptr<const T>(zs), ptr<const int32_t>(as), ptr<const int32_t>(mos), ptr<const int32_t>(macs),
+             m, ptr<const int32_t>(sis), ptr<T>(o[0]), ptr<T>(o[1]), ptr<T>(o[2]), ptr<T>(o[3]), a.acs.v, st);
+}
+
+std::vector<Tensor> featurize(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos, const Tensor& macs,
+                              const Tensor& sis, const py::object& acs, const c10::optional<Tensor>& order, const py::object& size_classes)
+{
+    const Atoms a = check_atoms(xs, ys, zs, as, mos, macs, sis, acs, order, size_classes);
+    auto out = buckets(at::empty({a.n * kFeats}, xs.options()), a.acs);
+    if (a.dt == at::kFloat) run_forward<float>(api.khan_featurize_f32, api.khan_featurize_ordered_f32, a, xs, ys, zs, as, mos, macs, sis, out);
+    else run_forward<double>(api.khan_featurize_f64, api.khan_featurize_ordered_f64, a, xs, ys, zs, as, mos, macs, sis, out);
+    return out;
+}
+
+template <typename T, typename Plain, typename Ordered>
+void run_backward(Plain plain, Ordered ordered, const Atoms& a, const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as,
+                  const Tensor& mos, const Tensor& macs, const Tensor& sis, const std::array<Tensor, 4>& g, const std::vector<Tensor>& o)
+{
+    const khan_stream_t st = stream();
+    const int32_t m = static_cast<int32_t>(mos.numel());
+    if (a.ordered)
+        call(ordered, ptr<const T>(xs), ptr<const T>(ys), ptr<const T>(zs), ptr<const int32_t>(as), ptr<const int32_t>(mos), ptr<const int32_t>(macs),
+             m, ptr<const int32_t>(sis), ptr<const T>(g[0]), ptr<const T>(g[1]), ptr<const T>(g[2]), ptr<const T>(g[3]), ptr<T>(o[0]), ptr<T>(o[1]),
+             ptr<T>(o[2]), a.acs.v, a.order, a.classes_ptr(), st);
+    else
+        call(plain, ptr<const T>(xs), ptr<const T>(ys), ptr<const T>(zs), ptr<const int32_t>(as), ptr<const int32_t>(mos), ptr<const int32_t>(macs),
+             m, ptr<const int32_t>(sis), ptr<const T>(g[0]), ptr<const T>(g[1]), ptr<const T>(g[2]), ptr<const T>(g[3]), ptr<T>(o[0]), ptr<T>(o[1]),
+             ptr<T>(o[2]), a.acs.v, st);
+}
+
+std::vector<Tensor> featurize_grad(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos,
+                                   const Tensor& macs, const Tensor& sis, const py::object& acs, const Tensor& h, const Tensor& c,
+                                   const Tensor& nn, const Tensor& oo, const c10::optional<Tensor>& order, const py::object& size_classes)
+{
+    const Atoms a = check_atoms(xs, ys, zs, as, mos, macs, sis, acs, order, size_classes);
+    static const char* const names[4] = {"h_grads", "c_grads", "n_grads", "o_grads"};
+    std::array<Tensor, 4> g = {h.reshape({-1}), c.reshape({-1}), nn.reshape({-1}), oo.reshape({-1})};
+    for (int t = 0; t < 4; ++t) {
+        dev(g[t], a.dt, names[t]);
+        if (g[t].numel() != a.acs.v[t] * kFeats)
+            throw py::value_error(std::string(names[t]) + " has " + std::to_string(g[t].numel()) + " elements, expected " +
+                                  std::to_string(a.acs.v[t] * kFeats));
+    }
+    const std::vector<Tensor> out = {at::empty({a.n}, xs.options()), at::empty({a.n}, xs.options()), at::empty({a.n}, xs.options())};
+    if (a.dt == at::kFloat)
+        run_backward<float>(api.khan_featurize_grad_f32, api.khan_featurize_grad_ordered_f32, a, xs, ys, zs, as, mos, macs, sis, g, out);
+    else
+        run_backward<double>(api.khan_featurize_grad_f64, api.khan_featurize_grad_ordered_f64, a, xs, ys, zs, as, mos, macs, sis, g, out);
+    return out;
+}
+
+template <typename T, typename Plain, typename Ordered>
+void run_inverse(Plain plain, Ordered ordered, const Atoms& a, const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as,
+                 const Tensor& mos, const Tensor& macs, const Tensor& sis, const Tensor& vx, const Tensor& vy, const Tensor& vz,
+                 const std::vector<Tensor>& o)
+{
+    const khan_stream_t st = stream();
+    const int32_t m = static_cast<int32_t>(mos.numel());
+    if (a.ordered)
+        call(ordered, ptr<const T>(xs), ptr<const T>(ys), ptr<const T>(zs), ptr<const int32_t>(as), ptr<const int32_t>(mos), ptr<const int32_t>(macs),
+             m, ptr<const int32_t>(sis), ptr<const T>(vx), ptr<const T>(vy), ptr<const T>(vz), ptr<T>(o[0]), ptr<T>(o[1]), ptr<T>(o[2]), ptr<T>(o[3]),
+             a.acs.v, a.order, a.classes_ptr(), st);
+    else
+        call(plain, ptr<const T>(xs), ptr<const T>(ys), ptr<const T>(zs), ptr<const int32_t>(as), ptr<const int32_t>(mos), ptr<const int32_t>(macs),
+             m, ptr<const int32_t>(sis), ptr<const T>(vx), ptr<const T>(vy), ptr<const T>(vz), ptr<T>(o[0]), ptr<T>(o[1]), ptr<T>(o[2]), ptr<T>(o[3]),
+             a.acs.v, st);
+}
+
+std::vector<Tensor> featurize_grad_inverse(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos,
+                                           const Tensor& macs, const Tensor& sis, const py::object& acs, const Tensor& vx, const Tensor& vy,
+                                           const Tensor& vz, const c10::optional<Tensor>& order, const py::object& size_classes)
+{
+    const Atoms a = check_atoms(xs, ys, zs, as, mos, macs, sis, acs, order, size_classes);
+    dev(vx, a.dt, "x_grads"); dev(vy, a.dt, "y_grads"); dev(vz, a.dt, "z_grads");
+    same_size(vx.numel() == a.n && vy.numel() == a.n && vz.numel() == a.n, "x_grads, y_grads, z_grads must have one element per atom");
+    auto out = buckets(at::empty({a.n * kFeats}, xs.options()), a.acs);
+    if (a.dt == at::kFloat)
+        run_inverse<float>(api.khan_featurize_grad_inverse_f32, api.khan_featurize_grad_inverse_ordered_f32, a, xs, ys, zs, as, mos, macs, sis, vx,
+                           vy, vz, out);
+    else
+        run_inverse<double>(api.khan_featurize_grad_inverse_f64, api.khan_featurize_grad_inverse_ordered_f64, a, xs, ys, zs, as, mos, macs, sis, vx,
+                            vy, vz, out);
+    return out;
+}
+
+// ---------------------------------------------------------------------------------------------- charges
+at::ScalarType check_charge(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& qs, const Tensor& mos, const Tensor& macs)
+{
+    const auto dt = float_dtype(xs, "coordinates");
+    dev(xs, dt, "xs"); dev(ys, dt, "ys"); dev(zs, dt, "zs"); dev(qs, dt, "qs");
+    dev(mos, at::kInt, "mos"); dev(macs, at::kInt, "macs");
+    const int64_t n = xs.numel();
+    same_size(ys.numel() == n && zs.numel() == n && qs.numel() == n, "xs, ys, zs, qs must have the same length");
+    same_size(mos.numel() == macs.numel(), "mos and macs must have the same length");
+    return dt;
+}
+
+Tensor ani_charge(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& qs, const Tensor& mos, const Tensor& macs)
+{
+    const auto dt = check_charge(xs, ys, zs, qs, mos, macs);
+    const Tensor e = at::empty({mos.numel()}, xs.options());
+    const int32_t m = static_cast<int32_t>(mos.numel());
+    const khan_stream_t st = stream();
+    if (dt == at::kFloat)
+        call(api.khan_ani_charge_f32, ptr<const float>(xs), ptr<const float>(ys), ptr<const float>(zs), ptr<const float>(qs), ptr<const int32_t>(mos),
+             ptr<const int32_t>(macs), m, ptr<float>(e), st);
+    else
+        call(api.khan_ani_charge_f64, ptr<const double>(xs), ptr<const double>(ys), ptr<const double>(zs), ptr<const double>(qs),
+             ptr<const int32_t>(mos), ptr<const int32_t>(macs), m, ptr<double>(e), st);
+    return e;
+}
+
+// Gradients (and with `energies` the energies) of the damped charge energy.  One zeroed allocation cut into the outputs:
+// atoms outside every molecule keep zeros.
+std::vector<Tensor> ani_charge_grads(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& qs, const Tensor& mos, const Tensor& macs,
+                                     const Tensor& grads, bool want_xyz, bool energies)
+{
+    const auto dt = check_charge(xs, ys, zs, qs, mos, macs);
+    dev(grads, dt, "grads");
+    same_size(grads.numel() == mos.numel(), "grads must have one element per molecule");
+    const int64_t n = xs.numel(), m64 = mos.numel();
+    const int32_t m = static_cast<int32_t>(m64);
+    const Tensor all = at::zeros({n * (want_xyz ? 4 : 1) + (energies ? m64 : 0)}, xs.options());
+    std::vector<Tensor> out;
+    int64_t at = 0;
+    auto take = [&](int64_t size) {
+        out.push_back(all.narrow(0, at, size));
+        at += size;
+    };
+    if (energies) take(m64);
+    for (int k = 0; k < (want_xyz ? 4 : 1); ++k) take(n);
+    const khan_stream_t st = stream();
+    auto run = [&](auto zero, auto grad, auto xyz, auto every) {
+        using T = decltype(zero);
+        const T *X = ptr<const T>(xs), *Y = ptr<const T>(ys), *Z = ptr<const T>(zs), *Q = ptr<const T>(qs), *G = ptr<const T>(grads);
+        const int32_t *o = ptr<const int32_t>(mos), *c = ptr<const int32_t>(macs);
+        if (energies) call(every, X, Y, Z, Q, o, c, m, G, ptr<T>(out[0]), ptr<T>(out[1]), ptr<T>(out[2]), ptr<T>(out[3]), ptr<T>(out[4]), st);
+        else if (want_xyz) call(xyz, X, Y, Z, Q, o, c, m, G, ptr<T>(out[0]), ptr<T>(out[1]), ptr<T>(out[2]), ptr<T>(out[3]), st);
+        else call(grad, X, Y, Z, Q, o, c, m, G, ptr<T>(out[0]), st);
+    };
+    if (dt == at::kFloat) run(0.0f, api.khan_ani_charge_grad_f32, api.khan_ani_charge_grad_xyz_f32, api.khan_ani_charge_all_f32);
+    else run(0.0, api.khan_ani_charge_grad_f64, api.khan_ani_charge_grad_xyz_f64, api.khan_ani_charge_all_f64);
+    return out;
+}
+
+// ---------------------------------------------------------------------------------------------- networks
+using Four = std::array<Tensor, 4>;
+
+Four four(const std::vector<Tensor>& v, const char* what)
+{
+    same_size(v.size() == 4, what);
+    return {v[0], v[1], v[2], v[3]};
+}
+
+Tensor mol_energy(const std::vector<Tensor>& type_outputs, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs)
+{
+    same_size(type_outputs.size() == 4, "type_outputs must hold the four per-type vectors");
+    const auto dt = float_dtype(type_outputs[0], "type_outputs");
+    Four o;
+    int64_t n = 0;
+    for (int t = 0; t < 4; ++t) {
+        o[t] = type_outputs[t].reshape({-1});
+        dev(o[t], dt, "type_outputs");
+        n += o[t].numel();
+    }
+    dev(types, at::kInt, "atom_types"); dev(sis, at::kInt, "sis"); dev(mos, at::kInt, "mos"); dev(macs, at::kInt, "macs");
+    same_size(n == types.numel() && sis.numel() == n && mos.numel() == macs.numel(),
+              "the four vectors must hold one value per atom, and mos / macs one entry per molecule");
+    const Tensor e = at::empty({macs.numel()}, o[0].options());
+    const int32_t m = static_cast<int32_t>(macs.numel());
+    const khan_stream_t st = stream();
+    auto run = [&](auto zero, auto fn) {
+        using T = decltype(zero);
+        const T* p[4] = {ptr<const T>(o[0]), ptr<const T>(o[1]), ptr<const T>(o[2]), ptr<const T>(o[3])};
+        call(fn, p, ptr<const int32_t>(types), ptr<const int32_t>(sis), ptr<const int32_t>(mos), ptr<const int32_t>(macs), m, ptr<T>(e), st);
+    };
+    if (dt == at::kFloat) run(0.0f, api.khan_mol_energy_f32);
+    else run(0.0, api.khan_mol_energy_f64);
+    return e;
+}
+
+std::vector<Tensor> mol_energy_grad(const Tensor& e_grads, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs,
+                                    const py::object& acs)
+{
+    const auto dt = float_dtype(e_grads, "e_grads");
+    dev(e_grads, dt, "e_grads");
+    dev(types, at::kInt, "atom_types"); dev(sis, at::kInt, "sis"); dev(mos, at::kInt, "mos"); dev(macs, at::kInt, "macs");
+    const Counts c = counts4(acs, "acs must hold 4 atom counts");
+    same_size(c.sum() == types.numel() && sis.numel() == types.numel() && mos.numel() == macs.numel() && e_grads.numel() == macs.numel(),
+              "acs must add up to the number of atoms, and e_grads / mos / macs hold one entry per molecule");
+    // one cleared array cut into the four vectors (atoms outside every molecule keep 0)
+    auto out = buckets(at::zeros({c.sum()}, e_grads.options()), c, 1);
+    const int32_t m = static_cast<int32_t>(macs.numel());
+    const khan_stream_t st = stream();
+    auto run = [&](auto zero, auto fn) {
+        using T = decltype(zero);
+        T* p[4] = {ptr<T>(out[0]), ptr<T>(out[1]), ptr<T>(out[2]), ptr<T>(out[3])};
+        call(fn, ptr<const T>(e_grads), ptr<const int32_t>(types), ptr<const int32_t>(sis), ptr<const int32_t>(mos), ptr<const int32_t>(macs), m, p, st);
+    };
+    if (dt == at::kFloat) run(0.0f, api.khan_mol_energy_grad_f32);
+    else run(0.0, api.khan_mol_energy_grad_f64);
+    return out;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
+{
+    m.def("init", &init);
+    m.def("prepare_batch", &prepare_batch);
+    m.def("featurize", &featurize);
+    m.def("featurize_grad", &featurize_grad);
+    m.def("featurize_grad_inverse", &featurize_grad_inverse);
+    m.def("ani_charge", &ani_charge);
+    m.def("ani_charge_grads", &ani_charge_grads);
+    m.def("mol_energy", &mol_energy);
+    m.def("mol_energy_grad", &mol_energy_grad);
+}

@@ -17,7 +17,7 @@ import ctypes
 
 import torch
 
-from . import _lib
+from . import _lib, _native
 
 FEATURE_SIZE = 384
 
@@ -25,7 +25,7 @@ _SUFFIX = {torch.float32: "f32", torch.float64: "f64"}
 
 
 def _stream():
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _dev(t, dtype, name):
@@ -41,7 +41,7 @@ def _dev(t, dtype, name):
 
 
 def _p(t):
-    return ctypes.c_void_p(t.data_ptr() if t is not None and t.numel() > 0 else None)
+    return t.data_ptr() if t is not None and t.numel() > 0 else None
 
 
 def _float_dtype(x):
@@ -105,34 +105,12 @@ def size_order(macs):
     return order
 
 
-def _order_arg(order, macs):
-    order = _dev(order, torch.int32, "order")
-    if order.numel() != macs.numel() + SIZE_ORDER_EXTRA:
-        raise ValueError("order must come from size_order(macs) of this batch")
-    return order
-
-
-def _classes_arg(size_classes):
-    """host copy of order[-4:] (a CPU tensor or 4 ints), or None"""
-    if size_classes is None:
-        return None
-    vals = [int(v) for v in (size_classes.tolist() if isinstance(size_classes, torch.Tensor) else size_classes)]
-    if len(vals) != 4:
-        raise ValueError("size_classes must hold 4 counts")
-    return (ctypes.c_int32 * 4)(*vals)
-
-
-def _check_common(xs, ys, zs, as_, mos, macs, sis):
-    dt = _float_dtype(xs)
-    _dev(xs, dt, "xs"); _dev(ys, dt, "ys"); _dev(zs, dt, "zs")
-    _dev(as_, torch.int32, "as"); _dev(mos, torch.int32, "mos"); _dev(macs, torch.int32, "macs")
-    _dev(sis, torch.int32, "sis")
-    n = xs.numel()
-    if not (ys.numel() == n and zs.numel() == n and as_.numel() == n and sis.numel() == n):
-        raise ValueError("xs, ys, zs, as, sis must have the same length")
-    if mos.numel() != macs.numel():
-        raise ValueError("mos and macs must have the same length")
-    return dt, n
+def prepare_batch(mol_idxs, atomic_numbers, n_mols, counts_pinned=None):
+    """`mol_offsets`, `ani_sort` and `size_order` of one batch in one call and one to three launches
+    -> (mol_atom_counts, mol_offsets, scatter_idxs, gather_idxs, atom_counts, size order), as those give them.
+    `counts_pinned` (int32[8] in pinned host memory) receives the four atom counts and the four size-class totals once the
+    work is done, without a copy: wait for an event recorded behind this call before reading it."""
+    return _native.load().prepare_batch(mol_idxs, atomic_numbers, n_mols, counts_pinned)
 
 
 def featurize(xs, ys, zs, as_, mos, macs, sis, acs, order=None, size_classes=None):
@@ -141,48 +119,12 @@ def featurize(xs, ys, zs, as_, mos, macs, sis, acs, order=None, size_classes=Non
     The four outputs are consecutive slices of one allocation, so
     ``torch.cat([h, c, n, o]).view(-1, 384)[gather_idxs]`` needs no copy for the concatenation.
     """
-    lib = _lib.load()
-    dt, n = _check_common(xs, ys, zs, as_, mos, macs, sis)
-    acs_c, acs_v = _acs_host(acs)
-    if sum(acs_v) != n:
-        raise ValueError("sum(acs)=%d does not match the number of atoms %d" % (sum(acs_v), n))
-    packed = torch.empty(n * FEATURE_SIZE, dtype=dt, device=xs.device)
-    outs, start = [], 0
-    for c in acs_v:
-        outs.append(packed[start * FEATURE_SIZE:(start + c) * FEATURE_SIZE])
-        start += c
-    args = (_p(xs), _p(ys), _p(zs), _p(as_), _p(mos), _p(macs), mos.numel(), _p(sis),
-            _p(outs[0]), _p(outs[1]), _p(outs[2]), _p(outs[3]), acs_c)
-    if order is None:
-        _lib.check(getattr(lib, "khan_featurize_" + _SUFFIX[dt])(*args, _stream()))
-    else:
-        _lib.check(getattr(lib, "khan_featurize_ordered_" + _SUFFIX[dt])(*args, _p(_order_arg(order, macs)), _classes_arg(size_classes), _stream()))
-    return tuple(outs)
+    return tuple(_native.load().featurize(xs, ys, zs, as_, mos, macs, sis, acs, order, size_classes))
 
 
 def featurize_grad(xs, ys, zs, as_, mos, macs, sis, acs, h_grads, c_grads, n_grads, o_grads, order=None, size_classes=None):
     """-> (x_grads, y_grads, z_grads), each [n_atoms] in original atom order."""
-    lib = _lib.load()
-    dt, n = _check_common(xs, ys, zs, as_, mos, macs, sis)
-    acs_c, acs_v = _acs_host(acs)
-    if sum(acs_v) != n:
-        raise ValueError("sum(acs)=%d does not match the number of atoms %d" % (sum(acs_v), n))
-    grads = []
-    for name, g, c in zip("hcno", (h_grads, c_grads, n_grads, o_grads), acs_v):
-        g = _dev(g.reshape(-1), dt, name + "_grads")
-        if g.numel() != c * FEATURE_SIZE:
-            raise ValueError("%s_grads has %d elements, expected %d" % (name, g.numel(), c * FEATURE_SIZE))
-        grads.append(g)
-    gx = torch.empty(n, dtype=dt, device=xs.device)
-    gy = torch.empty_like(gx)
-    gz = torch.empty_like(gx)
-    args = (_p(xs), _p(ys), _p(zs), _p(as_), _p(mos), _p(macs), mos.numel(), _p(sis),
-            _p(grads[0]), _p(grads[1]), _p(grads[2]), _p(grads[3]), _p(gx), _p(gy), _p(gz), acs_c)
-    if order is None:
-        _lib.check(getattr(lib, "khan_featurize_grad_" + _SUFFIX[dt])(*args, _stream()))
-    else:
-        _lib.check(getattr(lib, "khan_featurize_grad_ordered_" + _SUFFIX[dt])(*args, _p(_order_arg(order, macs)), _classes_arg(size_classes), _stream()))
-    return gx, gy, gz
+    return tuple(_native.load().featurize_grad(xs, ys, zs, as_, mos, macs, sis, acs, h_grads, c_grads, n_grads, o_grads, order, size_classes))
 
 
 def featurize_grad_inverse(xs, ys, zs, as_, mos, macs, sis, acs, x_grads, y_grads, z_grads, order=None, size_classes=None):
@@ -190,29 +132,7 @@ def featurize_grad_inverse(xs, ys, zs, as_, mos, macs, sis, acs, x_grads, y_grad
     features applied to one vector per atom, row_i[f] = sum_a dAEV_i[f]/dxyz_a . (x,y,z)_grads[a].
     It is the gradient of `featurize_grad` with respect to its upstream gradients
     (khan/training/trainer_multi_tower.py:64-91)."""
-    lib = _lib.load()
-    dt, n = _check_common(xs, ys, zs, as_, mos, macs, sis)
-    acs_c, acs_v = _acs_host(acs)
-    if sum(acs_v) != n:
-        raise ValueError("sum(acs)=%d does not match the number of atoms %d" % (sum(acs_v), n))
-    vs = []
-    for name, v in zip("xyz", (x_grads, y_grads, z_grads)):
-        v = _dev(v, dt, name + "_grads")
-        if v.numel() != n:
-            raise ValueError("%s_grads has %d elements, expected %d" % (name, v.numel(), n))
-        vs.append(v)
-    packed = torch.empty(n * FEATURE_SIZE, dtype=dt, device=xs.device)
-    outs, start = [], 0
-    for c in acs_v:
-        outs.append(packed[start * FEATURE_SIZE:(start + c) * FEATURE_SIZE])
-        start += c
-    args = (_p(xs), _p(ys), _p(zs), _p(as_), _p(mos), _p(macs), mos.numel(), _p(sis),
-            _p(vs[0]), _p(vs[1]), _p(vs[2]), _p(outs[0]), _p(outs[1]), _p(outs[2]), _p(outs[3]), acs_c)
-    if order is None:
-        _lib.check(getattr(lib, "khan_featurize_grad_inverse_" + _SUFFIX[dt])(*args, _stream()))
-    else:
-        _lib.check(getattr(lib, "khan_featurize_grad_inverse_ordered_" + _SUFFIX[dt])(*args, _p(_order_arg(order, macs)), _classes_arg(size_classes), _stream()))
-    return tuple(outs)
+    return tuple(_native.load().featurize_grad_inverse(xs, ys, zs, as_, mos, macs, sis, acs, x_grads, y_grads, z_grads, order, size_classes))
 
 
 def _check_charge(xs, ys, zs, qs, mos, macs):
@@ -230,99 +150,35 @@ def _check_charge(xs, ys, zs, qs, mos, macs):
 
 def ani_charge(xs, ys, zs, qs, mos, macs):
     """-> charge_energies[n_mols]"""
-    lib = _lib.load()
-    dt, _ = _check_charge(xs, ys, zs, qs, mos, macs)
-    e = torch.empty(mos.numel(), dtype=dt, device=xs.device)
-    fn = getattr(lib, "khan_ani_charge_" + _SUFFIX[dt])
-    _lib.check(fn(_p(xs), _p(ys), _p(zs), _p(qs), _p(mos), _p(macs), mos.numel(), _p(e), _stream()))
-    return e
+    return _native.load().ani_charge(xs, ys, zs, qs, mos, macs)
 
 
 def ani_charge_grad(xs, ys, zs, qs, mos, macs, grads):
     """-> q_grads[n_atoms]"""
-    lib = _lib.load()
-    dt, n = _check_charge(xs, ys, zs, qs, mos, macs)
-    grads = _dev(grads, dt, "grads")
-    if grads.numel() != mos.numel():
-        raise ValueError("grads must have one element per molecule")
-    qg = torch.zeros(n, dtype=dt, device=xs.device)
-    fn = getattr(lib, "khan_ani_charge_grad_" + _SUFFIX[dt])
-    _lib.check(fn(_p(xs), _p(ys), _p(zs), _p(qs), _p(mos), _p(macs), mos.numel(), _p(grads), _p(qg), _stream()))
-    return qg
+    return _native.load().ani_charge_grads(xs, ys, zs, qs, mos, macs, grads, False, False)[0]
 
 
 def ani_charge_grad_xyz(xs, ys, zs, qs, mos, macs, grads):
     """-> (q_grads, x_grads, y_grads, z_grads); the coordinate gradient is not offered by the reference."""
-    lib = _lib.load()
-    dt, n = _check_charge(xs, ys, zs, qs, mos, macs)
-    grads = _dev(grads, dt, "grads")
-    if grads.numel() != mos.numel():
-        raise ValueError("grads must have one element per molecule")
-    qg = torch.zeros(n, dtype=dt, device=xs.device)
-    gx = torch.zeros(n, dtype=dt, device=xs.device)
-    gy = torch.zeros_like(gx)
-    gz = torch.zeros_like(gx)
-    fn = getattr(lib, "khan_ani_charge_grad_xyz_" + _SUFFIX[dt])
-    _lib.check(fn(_p(xs), _p(ys), _p(zs), _p(qs), _p(mos), _p(macs), mos.numel(), _p(grads), _p(qg),
-                  _p(gx), _p(gy), _p(gz), _stream()))
-    return qg, gx, gy, gz
+    return tuple(_native.load().ani_charge_grads(xs, ys, zs, qs, mos, macs, grads, True, False))
 
 
 def ani_charge_all(xs, ys, zs, qs, mos, macs, grads):
     """`ani_charge` and `ani_charge_grad_xyz` in one pass over the pairs
     -> (charge_energies, q_grads, x_grads, y_grads, z_grads); the energies are not multiplied by `grads`."""
-    lib = _lib.load()
-    dt, n = _check_charge(xs, ys, zs, qs, mos, macs)
-    grads = _dev(grads, dt, "grads")
-    if grads.numel() != mos.numel():
-        raise ValueError("grads must have one element per molecule")
-    e = torch.zeros(mos.numel(), dtype=dt, device=xs.device)
-    qg = torch.zeros(n, dtype=dt, device=xs.device)
-    gx = torch.zeros(n, dtype=dt, device=xs.device)
-    gy = torch.zeros_like(gx)
-    gz = torch.zeros_like(gx)
-    fn = getattr(lib, "khan_ani_charge_all_" + _SUFFIX[dt])
-    _lib.check(fn(_p(xs), _p(ys), _p(zs), _p(qs), _p(mos), _p(macs), mos.numel(), _p(grads), _p(e), _p(qg),
-                  _p(gx), _p(gy), _p(gz), _stream()))
-    return e, qg, gx, gy, gz
+    return tuple(_native.load().ani_charge_grads(xs, ys, zs, qs, mos, macs, grads, True, True))
 
 
 def mol_energy(type_outputs, atom_types, sis, mos, macs):
     """Per-molecule sums of the four per-type output vectors (`type_outputs[t]` is [acs[t]], float32 or float64; atom
     g's value is type_outputs[as[g]][sis[g]]) -> [n_mols]: the reference's gather to atom order + segment_sum by
     molecule (khan/model/nn.py:165-177) in one launch, summed in a fixed order."""
-    lib = _lib.load()
-    dt = type_outputs[0].dtype
-    if dt not in _SUFFIX:
-        raise TypeError("type_outputs must be float32 or float64, got %s" % dt)
-    outs = [_dev(o.reshape(-1), dt, "type_outputs[%d]" % t) for t, o in enumerate(type_outputs)]
-    if len(outs) != 4:
-        raise ValueError("type_outputs must hold the four per-type vectors")
-    a, s_, mo, ma = (_dev(v, torch.int32, n) for v, n in ((atom_types, "atom_types"), (sis, "sis"), (mos, "mos"), (macs, "macs")))
-    if sum(o.numel() for o in outs) != a.numel() or s_.numel() != a.numel() or mo.numel() != ma.numel():
-        raise ValueError("the four vectors must hold one value per atom, and mos / macs one entry per molecule")
-    e = torch.empty(ma.numel(), dtype=dt, device=a.device)
-    fn = getattr(lib, "khan_mol_energy_" + _SUFFIX[dt])
-    _lib.check(fn(_ptr4(outs), _p(a), _p(s_), _p(mo), _p(ma), ma.numel(), _p(e), _stream()))
-    return e
+    return _native.load().mol_energy(list(type_outputs), atom_types, sis, mos, macs)
 
 
 def mol_energy_grad(e_grads, atom_types, sis, mos, macs, acs):
     """The way back through `mol_energy`: -> four vectors [acs[t]] with grad_t[sis[g]] = e_grads[molecule of g]."""
-    lib = _lib.load()
-    dt = e_grads.dtype
-    if dt not in _SUFFIX:
-        raise TypeError("e_grads must be float32 or float64, got %s" % dt)
-    eg = _dev(e_grads, dt, "e_grads")
-    a, s_, mo, ma = (_dev(v, torch.int32, n) for v, n in ((atom_types, "atom_types"), (sis, "sis"), (mos, "mos"), (macs, "macs")))
-    counts = _acs_host(acs)[1]
-    if sum(counts) != a.numel() or s_.numel() != a.numel() or mo.numel() != ma.numel() or eg.numel() != ma.numel():
-        raise ValueError("acs must add up to the number of atoms, and e_grads / mos / macs hold one entry per molecule")
-    # one cleared array cut into the four vectors (atoms outside every molecule keep 0)
-    outs = list(torch.zeros(sum(counts), dtype=dt, device=a.device).split(counts))
-    fn = getattr(lib, "khan_mol_energy_grad_" + _SUFFIX[dt])
-    _lib.check(fn(_p(eg), _p(a), _p(s_), _p(mo), _p(ma), ma.numel(), _ptr4(outs), _stream()))
-    return tuple(outs)
+    return tuple(_native.load().mol_energy_grad(e_grads, atom_types, sis, mos, macs, acs))
 
 
 def coulomb(xs, ys, zs, qs, mos, macs, k=1.0):

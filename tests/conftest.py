@@ -41,6 +41,8 @@ def _ensure_built():
         build.build_datagen()
     if not os.path.exists(host_so):
         build.build_host()
+    if not build.ops_library_is_current():
+        build.build_torch_ops()
     stale = [name for name, lib, defines in (("default", build.LIBRARY, ()), ("check", build.CHECK_LIBRARY, build.CHECK_DEFINES))
              if not build.library_is_current(lib, defines)]
     if stale:

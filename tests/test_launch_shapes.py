@@ -59,3 +59,29 @@ def test_molecules_shared_by_several_wavefronts(ops, kind, dtype, most, sizes):
         print("   %s %s, %d molecules" % (kind, dtype, n_mols), flush=True)
         assert torch.equal(r, rows[:n]) and torch.equal(j, jvp[:n])
         assert float((g - grads[:n]).abs().max()) <= tol * float(grads[:n].abs().max())
+
+@pytest.mark.parametrize("n_atoms,n_mols", [(0, 0), (0, 3), (1, 1), (63, 5), (2047, 100), (2048, 2048), (4096, 2047), (4097, 300), (5000, 1),
+                                            (100003, 9000), (3000, 2049)])
+def test_batch_preparation_in_one_call(ops, n_atoms, n_mols):
+    """prepare_batch against mol_offsets, ani_sort and size_order, around the tile sizes and the line between its two forms."""
+    rng = np.random.default_rng(n_atoms + n_mols)
+    ids = np.sort(rng.integers(0, max(n_mols, 1), n_atoms)).astype(np.int32)
+    types = rng.choice(4, size=n_atoms, p=[0.55, 0.3, 0.1, 0.05]).astype(np.int32)
+    if n_atoms > 4:
+        types[3] = 7                                             # out of range: counted as O
+    pinned = torch.full((8,), -1, dtype=torch.int32, pin_memory=True)
+    macs, mos, sc, ga, ac, order = ops.prepare_batch(dev(ids), dev(types), n_mols, pinned)
+    torch.cuda.synchronize()
+    want_sc, want_ga, want_ac = ops.ani_sort(dev(types))
+    assert torch.equal(sc, want_sc) and torch.equal(ga, want_ga) and torch.equal(ac, want_ac)
+    t = np.where((types < 0) | (types > 3), 3, types)
+    assert np.array_equal(ga.cpu().numpy()[np.argsort(t, kind="stable")], np.arange(n_atoms))
+    if n_mols == 0:
+        return
+    sizes = np.bincount(ids, minlength=n_mols)
+    assert np.array_equal(macs.cpu().numpy(), sizes) and np.array_equal(mos.cpu().numpy(), np.cumsum(sizes) - sizes)
+    want = ops.size_order(macs)
+    assert torch.equal(order[n_mols:n_mols + 258], want[n_mols:n_mols + 258]) and torch.equal(order[-4:], want[-4:])
+    o = order[:n_mols].cpu().numpy()
+    assert np.array_equal(np.sort(o), np.arange(n_mols)) and np.all(np.diff(np.minimum(sizes[o], 257)) <= 0)
+    assert pinned.tolist() == ac.cpu().tolist() + order[-4:].cpu().tolist()
