@@ -384,6 +384,18 @@ int khan_mol_energy_grad_f32(const float *e_grads, const int32_t *as, const int3
 int khan_mol_energy_grad_f64(const double *e_grads, const int32_t *as, const int32_t *sis, const int32_t *mos,
                              const int32_t *macs, int32_t n_mols, double *const *grad_host4, khan_stream_t stream);
 
+/* The charge entry points above with the number of atoms known (which spares the work of looking for molecules of sizes
+ * that so many atoms cannot hold).  grads NULL: the energies only; otherwise the gradients, and the energies too unless e is
+ * NULL; x/y/z_grads all NULL: no coordinate gradients (q_grads must then be given).  outputs_zeroed: e holds zeros already. */
+int khan_ani_charges_f32(const float *xs, const float *ys, const float *zs, const float *qs, const int32_t *mos,
+                         const int32_t *macs, int32_t n_mols, int64_t n_atoms, const float *grads, float *e,
+                         float *q_grads, float *x_grads, float *y_grads, float *z_grads, int32_t outputs_zeroed,
+                         khan_stream_t stream);
+int khan_ani_charges_f64(const double *xs, const double *ys, const double *zs, const double *qs, const int32_t *mos,
+                         const int32_t *macs, int32_t n_mols, int64_t n_atoms, const double *grads, double *e,
+                         double *q_grads, double *x_grads, double *y_grads, double *z_grads, int32_t outputs_zeroed,
+                         khan_stream_t stream);
+
 /* Plain Coulomb sums, E_m = k sum_{i<j in m} q_i q_j / r_ij, and their gradients: the charge kernels with
  * the damping (1 - f_C) switched off and the constant chosen by the caller (k = 1 for charges in e and
  * distances in the unit the energy is wanted in).  No reference counterpart: khan's own op is the damped,

@@ -374,25 +374,25 @@ int featurize_grad_inverse_impl(const T* xs, const T* ys, const T* zs, const int
 
 template <typename T>
 int charge_impl(const T* xs, const T* ys, const T* zs, const T* qs, const int32_t* mos,
-                const int32_t* macs, int32_t n_mols, bool damped, T k, T* e, khan_stream_t stream)
+                const int32_t* macs, int32_t n_mols, bool damped, T k, T* e, khan_stream_t stream, int64_t n_atoms = INT64_MAX)
 {
     if (n_mols < 0) return KHAN_ERR_INVALID_ARG;
     if (n_mols == 0) return KHAN_OK;
     if (!xs || !ys || !zs || !qs || !mos || !macs || !e) return KHAN_ERR_INVALID_ARG;
-    return hip_status(khan::launch_charge_energy<T>(xs, ys, zs, qs, mos, macs, n_mols, damped, k, e, as_stream(stream)));
+    return hip_status(khan::launch_charge_energy<T>(xs, ys, zs, qs, mos, macs, n_mols, n_atoms, damped, k, e, as_stream(stream)));
 }
 
 template <typename T>
 int charge_grad_impl(const T* xs, const T* ys, const T* zs, const T* qs, const int32_t* mos,
                      const int32_t* macs, int32_t n_mols, const T* grads, bool damped, T k, T* qg, T* gx, T* gy, T* gz,
-                     bool want_xyz, khan_stream_t stream, T* energies = nullptr)
+                     bool want_xyz, khan_stream_t stream, T* energies = nullptr, int64_t n_atoms = INT64_MAX, bool zeroed = false)
 {
     if (n_mols < 0) return KHAN_ERR_INVALID_ARG;
     if (n_mols == 0) return KHAN_OK;
     if (!xs || !ys || !zs || !qs || !mos || !macs || !grads) return KHAN_ERR_INVALID_ARG;
     if (want_xyz ? (!gx || !gy || !gz) : !qg) return KHAN_ERR_INVALID_ARG;
-    return hip_status(khan::launch_charge_grad<T>(xs, ys, zs, qs, mos, macs, n_mols, grads, damped, k, qg,
-                                                  want_xyz ? gx : nullptr, gy, gz, energies, as_stream(stream)));
+    return hip_status(khan::launch_charge_grad<T>(xs, ys, zs, qs, mos, macs, n_mols, n_atoms, grads, damped, k, qg,
+                                                  want_xyz ? gx : nullptr, gy, gz, energies, zeroed, as_stream(stream)));
 }
 
 }  // namespace
@@ -422,6 +422,15 @@ static int mol_energy_grad_impl(const T* e_grads, const int32_t* as, const int32
     return hip_status(khan::launch_mol_sum_grad<T>(e_grads, as, sis, mos, macs, n_mols, out, as_stream(stream)));
 }
 
+template <typename T>
+static int ani_charges(const T* xs, const T* ys, const T* zs, const T* qs, const int32_t* mos, const int32_t* macs, int32_t n_mols, int64_t n_atoms,
+                       const T* grads, T k, T* e, T* q_grads, T* gx, T* gy, T* gz, int outputs_zeroed, khan_stream_t stream)
+{
+    if (n_atoms < 0) return KHAN_ERR_INVALID_ARG;
+    if (!grads) return charge_impl<T>(xs, ys, zs, qs, mos, macs, n_mols, true, k, e, stream, n_atoms);
+    return charge_grad_impl<T>(xs, ys, zs, qs, mos, macs, n_mols, grads, true, k, q_grads, gx, gy, gz, gx != nullptr, stream, e, n_atoms,
+                               outputs_zeroed != 0);
+}
 
 extern "C" {
 
@@ -647,6 +656,20 @@ int khan_ani_charge_grad_xyz_f64(const double* xs, const double* ys, const doubl
                                  double* gy, double* gz, khan_stream_t stream)
 {
     return charge_grad_impl<double>(xs, ys, zs, qs, mos, macs, n_mols, grads, true, static_cast<double>(khan::kChargeK_f), q_grads, gx, gy, gz, true, stream);
+}
+
+int khan_ani_charges_f32(const float* xs, const float* ys, const float* zs, const float* qs, const int32_t* mos, const int32_t* macs,
+                         int32_t n_mols, int64_t n_atoms, const float* grads, float* e, float* q_grads, float* gx, float* gy, float* gz,
+                         int32_t outputs_zeroed, khan_stream_t stream)
+{
+    return ani_charges<float>(xs, ys, zs, qs, mos, macs, n_mols, n_atoms, grads, khan::kChargeK_f, e, q_grads, gx, gy, gz, outputs_zeroed, stream);
+}
+int khan_ani_charges_f64(const double* xs, const double* ys, const double* zs, const double* qs, const int32_t* mos, const int32_t* macs,
+                         int32_t n_mols, int64_t n_atoms, const double* grads, double* e, double* q_grads, double* gx, double* gy, double* gz,
+                         int32_t outputs_zeroed, khan_stream_t stream)
+{
+    return ani_charges<double>(xs, ys, zs, qs, mos, macs, n_mols, n_atoms, grads, static_cast<double>(khan::kChargeK_f), e, q_grads, gx, gy, gz,
+                               outputs_zeroed, stream);
 }
 
 int khan_dense_first_f32(const float* const* rows_host4, const int32_t* acs_host, const float* const* wt_host4,

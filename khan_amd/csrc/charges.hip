@@ -12,126 +12,111 @@
 // partners j for molecules of up to 16 atoms, 2 x 32 up to 32, 1 x 64 above -- with the partners' data
 // held in the lanes, and the sums over j are in-wave DPP reductions (a lane per atom i walking all j
 // would leave four fifths of the lanes idle on a 12-atom molecule).  Molecules of 65 to 256 atoms go to a
-// second kernel that tiles the molecule through LDS (charge_tile_kernel below).  Above 256 atoms several
-// workgroups share a molecule: all pairs, the partners tiled through LDS (charge_large_kernel).  Each output
+// workgroup that tiles the molecule through LDS (charge_tile below).  Above 256 atoms several
+// workgroups share a molecule: all pairs, the partners tiled through LDS (charge_large).  Each output
 // element is written once, no atomics and no pre-zeroing -- except the energy of a molecule of more than 256 atoms,
 // which is the sum of its workgroups' shares.
+#include <algorithm>
+
 #include "aev_small_common.h"
 
 namespace khan {
 
 namespace {
 
-// Distance arithmetic per precision.  float: the hardware reciprocal square root with one Newton step, the hardware
-// reciprocal and the minimax cutoff polynomials of the AEV kernels.  double: no library call either (sqrt_and_rcp and
-// the Taylor cutoff of aev_small_common.h) -- the library's sqrt, division, cos and sin come to some 250 instructions
-// per pair, most of them range reduction and special cases that cannot occur here, and made these kernels run at
-// 2.6 % of the double-precision vector peak.
-template <typename T> struct ChargeMath;
-template <> struct ChargeMath<float> {
-    // r = sqrt(d2) and 1/r (0 for d2 = 0)
-    static __device__ __forceinline__ void dist(float d2, float& r, float& inv)
+// What a pair at squared distance d2 contributes: u = (1 - f_C) / r and du = d/dr[(1 - f_C) / r] / r, both zero for
+// coincident atoms.  kDamped = false drops the cutoff function: plain Coulomb pairs (the reference's op is the damped form).
+// f_C is evaluated in every lane and selected: a branch would be taken by nearly every wavefront anyway.
+template <typename T, bool kDamped> struct PairTerms;
+// float: the hardware reciprocal square root with one Newton step and the minimax cutoff polynomials of the AEV kernels
+template <bool kDamped> struct PairTerms<float, kDamped> {
+    static __device__ __forceinline__ void of(float d2, float& u, float& du)
     {
-        r = Fast<float>::sqrt_rn(d2);
-        inv = d2 > 0.0f ? Fast<float>::rcp(r) : 0.0f;
-    }
-    // f_C(r, R_Rc) and its derivative, for r <= R_Rc
-    static __device__ __forceinline__ void cutoff(float r, float& fc, float& dfc)
-    {
-        Fast<float>::cutoff_grad(r, kR_Rc_f, fc, dfc);
-    }
-};
-template <> struct ChargeMath<double> {
-    static __device__ __forceinline__ void dist(double d2, double& r, double& inv) { sqrt_and_rcp(d2, r, inv); }
-    static __device__ __forceinline__ void cutoff(double r, double& fc, double& dfc)
-    {
-        Fast<double>::cutoff_grad(r, static_cast<double>(kR_Rc_f), fc, dfc);
-    }
-};
-
-// kDamped = false drops the cutoff function: plain Coulomb pairs q_i q_j / r (the reference's op is the damped form)
-template <typename T, bool kDamped>
-__device__ __forceinline__ void pair_terms(T dx, T dy, T dz, T& u, T& dudr_over_r)
-{
-    T r, inv;            // coincident atoms (r = 0): inv = 0, so that (1 - f_C)/r -> 0 there and the pair pulls nowhere
-    ChargeMath<T>::dist(dx * dx + dy * dy + dz * dz, r, inv);
-    T fc = T(0), dfc = T(0);
-    if constexpr (kDamped) {
-        // evaluated in every lane and selected: a branch would be taken by nearly every wavefront anyway
-        ChargeMath<T>::cutoff(r, fc, dfc);
-        const bool in = r <= static_cast<T>(kR_Rc_f);
-        fc = in ? fc : T(0);
-        dfc = in ? dfc : T(0);
-    }
-    u = (T(1) - fc) * inv;                            // (1 - f_C) / r
-    dudr_over_r = (-dfc * inv - u * inv) * inv;       // d/dr[(1-f_C)/r] / r
-}
-
-template <typename T, bool kDamped>
-__global__ __launch_bounds__(256) void charge_energy_kernel(
-    const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
-    const T* __restrict__ Q, const int32_t* __restrict__ MOs, const int32_t* __restrict__ MACs,
-    int32_t n_mols, T K, T* __restrict__ E)
-{
-    const int lane = threadIdx.x & 63;
-    const int64_t mol = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    if (mol >= n_mols) return;
-    const int n = MACs[mol], off = MOs[mol];
-    if (n > kSmallMaxAtoms && n <= kMediumMaxAtoms) return;      // the tile kernel's
-    T acc = T(0);
-    if (n <= 64) {
-        const int logW = n <= 16 ? 4 : n <= 32 ? 5 : 6;
-        const int W = 1 << logW, G = 64 >> logW;
-        const int grp = lane >> logW, jl = lane & (W - 1);
-        const bool jok = jl < n;
-        const T xj = jok ? X[off + jl] : T(0), yj = jok ? Y[off + jl] : T(0), zj = jok ? Z[off + jl] : T(0),
-                qj = jok ? Q[off + jl] : T(0);
-        for (int i0 = 0; i0 < n; i0 += G) {
-            const int i = i0 + grp;                      // lane i of the first group holds atom i
-            const T xi = __shfl(xj, i & 63, 64), yi = __shfl(yj, i & 63, 64), zi = __shfl(zj, i & 63, 64),
-                    qi = __shfl(qj, i & 63, 64);
-            const bool valid = (i < n) && jok && (jl > i);
-            T u, du;
-            pair_terms<T, kDamped>(valid ? xi - xj : T(1), valid ? yi - yj : T(0), valid ? zi - zj : T(0), u, du);
-            acc += valid ? K * qi * qj * u : T(0);
+        const float r = Fast<float>::sqrt_rn(d2);
+        const float inv = d2 > 0.0f ? Fast<float>::rcp(r) : 0.0f;
+        float fc = 0.0f, dfc = 0.0f;
+        if constexpr (kDamped) {
+            Fast<float>::cutoff_grad(r, kR_Rc_f, fc, dfc);
+            const bool in = r <= kR_Rc_f;
+            fc = in ? fc : 0.0f;
+            dfc = in ? dfc : 0.0f;
         }
-        acc = wave_sum(acc);
-        if (lane == 0) E[mol] = acc;
-        return;
+        u = (1.0f - fc) * inv;
+        du = (-dfc * inv - u * inv) * inv;
     }
-    // more than 256 atoms: charge_large_kernel adds its workgroups' shares to the energy, which starts from zero here
-    if (lane == 0) E[mol] = T(0);
-}
+};
+// double: no library call, no square root and no angle.  1/r from v_rsq_f64 (5e-8) and one third-order step.  1 - f_C =
+// sin^2(pi r / 2 R_c) = d2 q(d2) and 2 d(1 - f_C)/d(d2) = (d/dr) / r are entire functions of d2: polynomials of degree
+// nine in d2 (Chebyshev interpolation on [0, R_c^2]), exact to 4e-16 of q and 1e-16.  (Before: a square root, a folded half
+// angle, its sine and cosine: 106 vector instructions per pair of the tile kernel, 78 now, with everything around it.)
+template <bool kDamped> struct PairTerms<double, kDamped> {
+    static __device__ __forceinline__ double poly(const double (&c)[10], double x)
+    {
+        double v = c[9];
+#pragma unroll
+        for (int k = 8; k >= 0; --k) v = fma(v, x, c[k]);
+        return v;
+    }
+    static __device__ __forceinline__ void of(double d2, double& u, double& du)
+    {
+        constexpr double kQ[10] = {0.11660686212575191, -0.004532386764938009, 7.046765314658188e-05, -5.869294224571146e-07,
+                                   3.0417776911092683e-09, -1.0748245519813352e-11, 2.7545314816657834e-14,
+                                   -5.3522125411118236e-17, 8.115026416218573e-20, -8.999642674693997e-23};
+        constexpr double kT[10] = {0.23321372425150377, -0.018129547059751505, 0.0004228059188787524, -4.695435379265704e-06,
+                                   3.0417776808067906e-08, -1.2897893108818512e-10, 3.856331055586389e-13,
+                                   -8.562890949169944e-16, 1.4589662776261427e-18, -1.7805957172843363e-21};
+        const double y = __builtin_amdgcn_rsq(d2);
+        const double e = fma(-d2 * y, y, 1.0);
+        double inv = fma(y * e, fma(e, 0.375, 0.5), y);
+        inv = d2 > 0.0 ? inv : 0.0;
+        double s = 1.0, t = 0.0;               // 1 - f_C, and its derivative in r over r
+        if constexpr (kDamped) {
+            constexpr double kRc2 = static_cast<double>(kR_Rc_f) * static_cast<double>(kR_Rc_f);
+            const bool in = d2 <= kRc2;
+            const double sq = d2 * poly(kQ, d2), tq = poly(kT, d2);       // (without meaning outside)
+            s = in ? sq : 1.0;
+            t = in ? tq : 0.0;
+        }
+        u = s * inv;
+        du = fma(t, inv, -u * (inv * inv));
+    }
+};
 
-template <typename T, bool kDamped>
-__global__ __launch_bounds__(256) void charge_grad_kernel(
-    const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
-    const T* __restrict__ Q, const int32_t* __restrict__ MOs, const int32_t* __restrict__ MACs,
-    int32_t n_mols, const T* __restrict__ grads, T K, T* __restrict__ q_grads, T* __restrict__ gX,
-    T* __restrict__ gY, T* __restrict__ gZ, T* __restrict__ E)
+template <typename T>
+struct ChargeArgs {
+    const T *X, *Y, *Z, *Q;
+    const int32_t *MOs, *MACs;
+    int32_t n_mols;
+    const T* grads;          // gradients only
+    T K;
+    T *E, *q_grads, *gX, *gY, *gZ;      // with gradients each of E, q_grads and (gX, gY, gZ) may be null
+};
+
+// A molecule of up to 64 atoms in one wavefront.
+template <typename T, bool kDamped, bool kGrad>
+__device__ __forceinline__ void charge_small(const ChargeArgs<T>& a, int mol, int n)
 {
     const int lane = threadIdx.x & 63;
-    const int64_t mol = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    if (mol >= n_mols) return;
-    const int n = MACs[mol], off = MOs[mol];
-    if (n > kSmallMaxAtoms && n <= kMediumMaxAtoms) return;      // the tile kernel's
-    const T gK = grads[mol] * K;
-    T e_acc = T(0);          // sum over atoms of q_i sum_j q_j u_ij = twice the energy / K
-    if (n <= 64) {
-        const int logW = n <= 16 ? 4 : n <= 32 ? 5 : 6;
-        const int W = 1 << logW, G = 64 >> logW;
-        const int grp = lane >> logW, jl = lane & (W - 1);
-        const bool jok = jl < n;
-        const T xj = jok ? X[off + jl] : T(0), yj = jok ? Y[off + jl] : T(0), zj = jok ? Z[off + jl] : T(0),
-                qj = jok ? Q[off + jl] : T(0);
-        for (int i0 = 0; i0 < n; i0 += G) {
-            const int i = i0 + grp;                      // lane i of the first group holds atom i
-            const T xi = __shfl(xj, i & 63, 64), yi = __shfl(yj, i & 63, 64), zi = __shfl(zj, i & 63, 64),
-                    qi = __shfl(qj, i & 63, 64);
-            const bool valid = (i < n) && jok && (jl != i);
-            const T dx = valid ? xi - xj : T(1), dy = valid ? yi - yj : T(0), dz = valid ? zi - zj : T(0);
-            T u, du;
-            pair_terms<T, kDamped>(dx, dy, dz, u, du);
+    const int off = a.MOs[mol];
+    const int logW = n <= 16 ? 4 : n <= 32 ? 5 : 6;
+    const int W = 1 << logW, G = 64 >> logW;
+    const int grp = lane >> logW, jl = lane & (W - 1);
+    const bool jok = jl < n;
+    const T xj = jok ? a.X[off + jl] : T(0), yj = jok ? a.Y[off + jl] : T(0), zj = jok ? a.Z[off + jl] : T(0),
+            qj = jok ? a.Q[off + jl] : T(0);
+    T gK = T(0);
+    if constexpr (kGrad) gK = a.grads[mol] * a.K;
+    T acc = T(0);                // the energy / K; with gradients twice that: q_i sum_j q_j u_ij over the atoms
+    for (int i0 = 0; i0 < n; i0 += G) {
+        const int i = i0 + grp;                      // lane i of the first group holds atom i
+        const T xi = __shfl(xj, i & 63, 64), yi = __shfl(yj, i & 63, 64), zi = __shfl(zj, i & 63, 64), qi = __shfl(qj, i & 63, 64);
+        const bool valid = (i < n) && jok && (kGrad ? jl != i : jl > i);
+        const T dx = xi - xj, dy = yi - yj, dz = zi - zj;
+        T u, du;
+        PairTerms<T, kDamped>::of(dx * dx + dy * dy + dz * dz, u, du);
+        if constexpr (!kGrad) {
+            acc += valid ? qi * qj * u : T(0);
+        } else {
             const T w = valid ? qj * du : T(0);
             // sums over the W partners of the group end up in its last lane
             const T dq = group_sum_to_last_lane(valid ? qj * u : T(0), logW);
@@ -139,264 +124,318 @@ __global__ __launch_bounds__(256) void charge_grad_kernel(
             const T fy = group_sum_to_last_lane(w * dy, logW);
             const T fz = group_sum_to_last_lane(w * dz, logW);
             if (jl == W - 1 && i < n) {
-                e_acc = fma(qi, dq, e_acc);
-                if (q_grads) q_grads[off + i] = gK * dq;
-                if (gX) {
-                    gX[off + i] = gK * qi * fx;
-                    gY[off + i] = gK * qi * fy;
-                    gZ[off + i] = gK * qi * fz;
+                acc = fma(qi, dq, acc);
+                if (a.q_grads) a.q_grads[off + i] = gK * dq;
+                if (a.gX) {
+                    a.gX[off + i] = gK * qi * fx;
+                    a.gY[off + i] = gK * qi * fy;
+                    a.gZ[off + i] = gK * qi * fz;
                 }
             }
         }
-        if (E) {
-            e_acc = wave_sum(e_acc);
-            if (lane == 0) E[mol] = T(0.5) * K * e_acc;
-        }
-        return;
     }
-    // more than 256 atoms: charge_large_kernel's, which adds its workgroups' shares to an energy that starts from zero
-    if (E && lane == 0) E[mol] = T(0);
+    if (a.E) {
+        acc = wave_sum(acc);
+        if (lane == 0) a.E[mol] = (kGrad ? T(0.5) : T(1)) * a.K * acc;
+    }
 }
 
-// Molecules of 65 to 256 atoms: one workgroup of four wavefronts per molecule, the molecule (x, y, z, q) in LDS, one
-// atom i per thread.  In round d a thread pairs its atom with atom j = (i + d) mod n, read from the tile: after
-// (n-1)/2 rounds (plus half a round when n is even) every unordered pair has been evaluated exactly once -- half the
-// pair evaluations of a walk over all j != i.  In a round the partners j of a wavefront's atoms are distinct, so what a
-// pair contributes to its partner (dE/dq_j and the force on j) is added to the partner's slot in LDS by plain
-// read-add-write, without atomics, while the atom's own side stays in registers.  Every wavefront adds into a copy of
-// its own of the partner slots, so the four never wait for each other inside the rounds (a barrier per round would be
-// the alternative); the copies are summed at the end.  A wavefront whose 64 atoms lie beyond the molecule sits the
-// rounds out.  Every output element is written once.
+// Molecules of 65 to 256 atoms: one workgroup of four wavefronts per molecule, the molecule (x, y, z, q) in LDS.  A
+// wavefront takes a block of 64 atoms, one atom i per lane; in round d a lane pairs its atom with atom j = (i + d) mod n,
+// read from the tile: after (n-1)/2 rounds (plus half a round when n is even) of every block each unordered pair has been
+// evaluated exactly once -- half the pair evaluations of a walk over all j != i.  The blocks' rounds are dealt to the four
+// wavefronts in equal shares (a block per wavefront left a quarter of them without work on average: dense boxes of 64-256
+// atoms).  In a round the partners j of a wavefront's atoms are distinct, so what a pair contributes to its partner
+// (dE/dq_j and the force on j) is added to the partner's slot in LDS by plain read-add-write, without atomics, while the
+// atom's own side stays in registers until the block's share ends.  Every wavefront adds into a copy of its own of the
+// slots, so the four never wait for each other inside the rounds (a barrier per round would be the alternative); the
+// copies are summed at the end.  Every output element is written once.
 template <typename T, bool kGrad> struct ChargeTile;
+// (pairs of values in arrays of their own: 16-byte accesses 32 bytes apart would meet in half of the banks)
 template <typename T> struct __align__(16) ChargeTile<T, false> {
-    typename Fast<T>::vec4 in[kMediumMaxAtoms];     // x, y, z, q
+    typename Fast<T>::vec2 in[2][kMediumMaxAtoms];     // x, y and z, q
     T wpart[4];
 };
 // (in double these are 40,960 bytes, a quarter of a compute unit's LDS to the byte: the wavefronts' partial energies
 // go into the tile's first entry once the rounds are over, not into four words more that would cost the fourth workgroup)
 template <typename T> struct __align__(16) ChargeTile<T, true> {
-    typename Fast<T>::vec4 in[kMediumMaxAtoms];     // x, y, z, q
-    typename Fast<T>::vec4 acc[4][kMediumMaxAtoms]; // partner side, per wavefront: force x, y, z and dE/dq
+    typename Fast<T>::vec2 in[2][kMediumMaxAtoms];     // x, y and z, q
+    typename Fast<T>::vec2 acc[4][2][kMediumMaxAtoms]; // per wavefront: force x, y and force z, dE/dq
 };
 
 template <typename T, bool kDamped, bool kGrad>
-__global__ __launch_bounds__(256) void charge_tile_kernel(
-    const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
-    const T* __restrict__ Q, const int32_t* __restrict__ MOs, const int32_t* __restrict__ MACs,
-    int32_t n_mols, const T* __restrict__ grads, T K, T* __restrict__ E, T* __restrict__ q_grads,
-    T* __restrict__ gX, T* __restrict__ gY, T* __restrict__ gZ)
+__device__ __forceinline__ void charge_tile(const ChargeArgs<T>& a, ChargeTile<T, kGrad>& S, int mol, int n)
 {
-    typedef typename Fast<T>::vec4 vec4;
+    typedef typename Fast<T>::vec2 vec2;
     static_assert(kMediumMaxAtoms == 256, "one atom per thread of a 256-thread workgroup");
-    __shared__ ChargeTile<T, kGrad> S;
-    const int i = threadIdx.x, lane = i & 63, wave = uniform(i >> 6);
-    for (int mol = blockIdx.x; mol < n_mols; mol += gridDim.x) {
-        const int n = uniform(MACs[mol]);
-        if (n <= kSmallMaxAtoms || n > kMediumMaxAtoms) continue;
-        const int off = uniform(MOs[mol]);
-        const bool have = i < n;
-        vec4 own = Fast<T>::make4(T(0), T(0), T(0), T(0));
-        if (have) {
-            own = Fast<T>::make4(X[off + i], Y[off + i], Z[off + i], Q[off + i]);
-            S.in[i] = own;
-        }
-        if constexpr (kGrad) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
+    const int off = uniform(a.MOs[mol]);
+    const bool have = tid < n;
+    if (have) {
+        S.in[0][tid] = Fast<T>::make2(a.X[off + tid], a.Y[off + tid]);
+        S.in[1][tid] = Fast<T>::make2(a.Z[off + tid], a.Q[off + tid]);
+    }
+    if constexpr (kGrad) {
 #pragma unroll
-            for (int w = 0; w < 4; ++w) S.acc[w][i] = Fast<T>::make4(T(0), T(0), T(0), T(0));
-        }
-        __syncthreads();
-        const int half = (n - 1) >> 1;
-        const int rounds = (wave * 64 < n) ? half + (((n & 1) == 0) ? 1 : 0) : 0;
-        T fx = T(0), fy = T(0), fz = T(0), dq = T(0), e_acc = T(0);
-        for (int d = 1; d <= rounds; ++d) {
-            const bool act = have && (d <= half || i < (n >> 1));     // the half round: the lower half only
-            int j = i + d;
-            j -= (j >= n) ? n : 0;
-            const vec4 aj = S.in[act ? j : 0];
-            const T dx = act ? own.x - aj.x : T(1), dy = act ? own.y - aj.y : T(0), dz = act ? own.z - aj.z : T(0);
+        for (int w = 0; w < 4; ++w) S.acc[w][0][tid] = S.acc[w][1][tid] = Fast<T>::make2(T(0), T(0));
+    }
+    __syncthreads();
+    // the rounds of every block of 64 atoms, laid end to end and cut into four equal shares
+    const int half = (n - 1) >> 1, rounds = half + ((n & 1) == 0 ? 1 : 0), blocks = (n + 63) >> 6;
+    const int units = blocks * rounds;
+    int unit = wave * units >> 2;
+    const int last = (wave + 1) * units >> 2;
+    T e_acc = T(0);
+    while (unit < last) {
+        const int block = unit / rounds, d0 = unit - block * rounds;             // rounds d0 + 1 .. d1
+        const int d1 = min(rounds, d0 + (last - unit));
+        unit += d1 - d0;
+        const int i = block * 64 + lane;
+        // a lane without an atom takes part with charge zero: everything it adds is zero, and its partners are, like
+        // everyone's, distinct from those of the other lanes of its wavefront (n > 64)
+        const vec2 own_xy = S.in[0][min(i, n - 1)], own_zq = S.in[1][min(i, n - 1)];
+        const T q_own = i < n ? own_zq.y : T(0);
+        int j = i + d0;                              // (i + d) mod n: i < n + 64, d0 < n / 2
+        j -= j >= n ? n : 0;
+        j -= j >= n ? n : 0;
+        T fx = T(0), fy = T(0), fz = T(0), dq = T(0);
+        auto pair = [&](T q_i, bool act) {
+            j = j + 1 == n ? 0 : j + 1;
+            const vec2 xy = S.in[0][j], zq = S.in[1][j];
+            const T dx = own_xy.x - xy.x, dy = own_xy.y - xy.y, dz = own_zq.x - zq.x;
             T u, du;
-            pair_terms<T, kDamped>(dx, dy, dz, u, du);
-            const T qq = act ? own.w * aj.w : T(0);
-            e_acc = fma(qq, u, e_acc);
-            if constexpr (kGrad) {
-                if (act) {
-                    dq = fma(aj.w, u, dq);
-                    const T wq = qq * du;                    // q_i q_j d/dr[(1-f_C)/r] / r
-                    fx = fma(wq, dx, fx);
-                    fy = fma(wq, dy, fy);
-                    fz = fma(wq, dz, fz);
-                    vec4 pa = S.acc[wave][j];                // distinct j across the lanes of this wavefront
-                    pa.x = fma(-wq, dx, pa.x);
-                    pa.y = fma(-wq, dy, pa.y);
-                    pa.z = fma(-wq, dz, pa.z);
-                    pa.w = fma(own.w, u, pa.w);
-                    S.acc[wave][j] = pa;
-                }
-                wave_lds_fence();                            // the next round may touch slots written here
+            PairTerms<T, kDamped>::of(dx * dx + dy * dy + dz * dz, u, du);
+            const T qq = q_i * zq.y;
+            if constexpr (!kGrad) {
+                e_acc = fma(qq, u, e_acc);
+            } else {
+                dq = fma(act ? zq.y : T(0), u, dq);
+                const T wq = qq * du;                    // q_i q_j d/dr[(1-f_C)/r] / r
+                const T wx = wq * dx, wy = wq * dy, wz = wq * dz;
+                fx += wx;
+                fy += wy;
+                fz += wz;
+                vec2 pa = S.acc[wave][0][j], pb = S.acc[wave][1][j];     // distinct j across the lanes of this wavefront
+                pa.x -= wx;
+                pa.y -= wy;
+                pb.x -= wz;
+                pb.y = fma(q_i, u, pb.y);
+                S.acc[wave][0][j] = pa;
+                S.acc[wave][1][j] = pb;
+                wave_lds_fence();                        // the next round may touch slots written here
+            }
+        };
+        const int full = min(d1, half);
+        for (int d = d0; d < full; ++d) pair(q_own, true);
+        if (d1 > half) pair(i < (n >> 1) ? q_own : T(0), i < (n >> 1));      // the half round of an even n: the lower half only
+        if constexpr (kGrad) {
+            if (i < n) {                                 // the atoms' own side joins this wavefront's copy
+                vec2 pa = S.acc[wave][0][i], pb = S.acc[wave][1][i];
+                pa.x += fx;
+                pa.y += fy;
+                pb.x += fz;
+                pb.y += dq;
+                S.acc[wave][0][i] = pa;
+                S.acc[wave][1][i] = pb;
+            }
+            wave_lds_fence();
+        }
+    }
+    T p[4] = {T(0), T(0), T(0), T(0)};
+    T* wpart;
+    if constexpr (kGrad) {
+        __syncthreads();                             // every wavefront's partner sides are complete, the tile is free
+        if (have) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const vec2 p0 = S.acc[0][h][tid], p1 = S.acc[1][h][tid], p2 = S.acc[2][h][tid], p3 = S.acc[3][h][tid];
+                p[2 * h] = (p0.x + p1.x) + (p2.x + p3.x);
+                p[2 * h + 1] = (p0.y + p1.y) + (p2.y + p3.y);
             }
         }
-        T* wpart;
-        if constexpr (kGrad) {
-            wpart = reinterpret_cast<T*>(&S.in[0]);
-            if (E) __syncthreads();          // every wavefront has finished its rounds: the tile is free
-        } else {
-            wpart = S.wpart;
-        }
-        if (!kGrad || E) {
-            e_acc = wave_sum(e_acc);
-            if (lane == 0) wpart[wave] = e_acc;
-        }
+        // the energy: half of q_i sum_j q_j u_ij over the atoms
+        e_acc = have ? T(0.5) * S.in[1][tid].y * p[3] : T(0);
+        __syncthreads();                             // (the first entry is overwritten below)
+        wpart = reinterpret_cast<T*>(&S.in[0][0]);
+    } else {
+        wpart = S.wpart;
+    }
+    if (a.E) {
+        e_acc = wave_sum(e_acc);
+        if (lane == 0) wpart[wave] = e_acc;
         __syncthreads();
-        if ((!kGrad || E) && i == 0) E[mol] = K * ((wpart[0] + wpart[1]) + (wpart[2] + wpart[3]));
-        if constexpr (kGrad) {
-            if (have) {
-                const T gK = grads[mol] * K;
-                const vec4 p0 = S.acc[0][i], p1 = S.acc[1][i], p2 = S.acc[2][i], p3 = S.acc[3][i];
-                if (q_grads) q_grads[off + i] = gK * (dq + ((p0.w + p1.w) + (p2.w + p3.w)));
-                if (gX) {
-                    // the force sums carry q_i already (wq = q_i q_j ...)
-                    gX[off + i] = gK * (fx + ((p0.x + p1.x) + (p2.x + p3.x)));
-                    gY[off + i] = gK * (fy + ((p0.y + p1.y) + (p2.y + p3.y)));
-                    gZ[off + i] = gK * (fz + ((p0.z + p1.z) + (p2.z + p3.z)));
-                }
+        if (tid == 0) a.E[mol] = a.K * ((wpart[0] + wpart[1]) + (wpart[2] + wpart[3]));
+    }
+    if constexpr (kGrad) {
+        if (have) {
+            const T gK = a.grads[mol] * a.K;
+            if (a.q_grads) a.q_grads[off + tid] = gK * p[3];
+            if (a.gX) {
+                // the force sums carry q_i already (wq = q_i q_j ...)
+                a.gX[off + tid] = gK * p[0];
+                a.gY[off + tid] = gK * p[1];
+                a.gZ[off + tid] = gK * p[2];
             }
         }
-        __syncthreads();         // the next molecule reuses the tile
     }
 }
 
 // Molecules of more than 256 atoms: all pairs, the partners tiled through LDS 256 at a time.  A thread owns one atom i
 // of a block of 256 and sums over every partner j (each pair is evaluated from both ends: no exchange between threads, and
-// every per-atom output is written once, by its owner); the workgroups of a grid column (blockIdx.y) share a molecule's
-// blocks.  The energy is half the sum over atoms of q_i times the atom's sum, added to E[mol] (zeroed by
-// charge_energy_kernel or charge_grad_kernel, which runs before on the same stream) by one floating-point atomic per workgroup and block: its
-// last bits depend on the order of those additions.
+// every per-atom output is written once, by its owner); the `parts` workgroups of a column share a molecule's
+// blocks.  The energy is half the sum over atoms of q_i times the atom's sum, added to E[mol] (zeroed before the launch)
+// by one floating-point atomic per workgroup and block: its last bits depend on the order of those additions.
 template <typename T, bool kDamped, bool kGrad>
-__global__ __launch_bounds__(256) void charge_large_kernel(
-    const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
-    const T* __restrict__ Q, const int32_t* __restrict__ MOs, const int32_t* __restrict__ MACs,
-    int32_t n_mols, const T* __restrict__ grads, T K, T* __restrict__ E, T* __restrict__ q_grads,
-    T* __restrict__ gX, T* __restrict__ gY, T* __restrict__ gZ)
+__device__ __forceinline__ void charge_large(const ChargeArgs<T>& a, typename Fast<T>::vec4* tile, T* wpart, int column, int columns, int part, int parts)
 {
     typedef typename Fast<T>::vec4 vec4;
-    __shared__ vec4 tile[256];
-    __shared__ T wpart[4];
-    __shared__ unsigned long long want[4];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for_each_molecule_in_range(MACs, n_mols, kMediumMaxAtoms + 1, INT32_MAX, want, nullptr, nullptr, [&](int mol) {
-        const int n = uniform(MACs[mol]);
-        const int off = uniform(MOs[mol]);
-        for (int i0 = static_cast<int>(blockIdx.y) * 256; i0 < n; i0 += static_cast<int>(gridDim.y) * 256) {
-            const int i = i0 + tid;
-            const bool have = i < n;
-            const T xi = have ? X[off + i] : T(0), yi = have ? Y[off + i] : T(0), zi = have ? Z[off + i] : T(0),
-                    qi = have ? Q[off + i] : T(0);
-            T su = T(0), fx = T(0), fy = T(0), fz = T(0);      // sums over j of q_j u and of q_j du (x_i - x_j)
-            for (int j0 = 0; j0 < n; j0 += 256) {
-                __syncthreads();                               // the previous tile has been used
-                const int j = j0 + tid;
-                // (places beyond the molecule: charge zero)
-                tile[tid] = j < n ? Fast<T>::make4(X[off + j], Y[off + j], Z[off + j], Q[off + j])
-                                  : Fast<T>::make4(T(0), T(0), T(0), T(0));
-                __syncthreads();
-                const int cnt = min(256, n - j0);
-#pragma unroll 4
-                for (int t = 0; t < cnt; ++t) {
-                    const vec4 aj = tile[t];                   // the same address in every lane
-                    const T dx = xi - aj.x, dy = yi - aj.y, dz = zi - aj.z;
-                    T u, du;
-                    pair_terms<T, kDamped>(dx, dy, dz, u, du);      // zero for the atom itself (r = 0)
-                    su = fma(aj.w, u, su);
-                    if constexpr (kGrad) {
-                        const T w = aj.w * du;
-                        fx = fma(w, dx, fx);
-                        fy = fma(w, dy, fy);
-                        fz = fma(w, dz, fz);
+    for (int64_t base = column; base < a.n_mols; base += static_cast<int64_t>(columns) * 256) {
+        // the next 256 molecules of this column, one per thread: is there a large one?
+        const int64_t mine = base + static_cast<int64_t>(tid) * columns;
+        const bool large = mine < a.n_mols && a.MACs[mine] > kMediumMaxAtoms;
+        const bool some = wave_ballot(large) != 0ull;
+        if (lane == 0) wpart[wave] = some ? T(1) : T(0);
+        __syncthreads();
+        const bool any = wpart[0] + wpart[1] + wpart[2] + wpart[3] > T(0);
+        __syncthreads();
+        if (!any) continue;
+        for (int k = 0; k < 256; ++k) {
+            const int64_t m = base + static_cast<int64_t>(k) * columns;
+            if (m >= a.n_mols) break;
+            const int mol = static_cast<int>(m);
+            const int n = uniform(a.MACs[mol]);
+            if (n <= kMediumMaxAtoms) continue;
+            const int off = uniform(a.MOs[mol]);
+            for (int i0 = part * 256; i0 < n; i0 += parts * 256) {
+                const int i = i0 + tid;
+                const bool have = i < n;
+                const T xi = have ? a.X[off + i] : T(0), yi = have ? a.Y[off + i] : T(0), zi = have ? a.Z[off + i] : T(0),
+                        qi = have ? a.Q[off + i] : T(0);
+                T su = T(0), fx = T(0), fy = T(0), fz = T(0);      // sums over j of q_j u and of q_j du (x_i - x_j)
+                for (int j0 = 0; j0 < n; j0 += 256) {
+                    __syncthreads();                               // the previous tile has been used
+                    const int j = j0 + tid;
+                    // (places beyond the molecule: charge zero)
+                    tile[tid] = j < n ? Fast<T>::make4(a.X[off + j], a.Y[off + j], a.Z[off + j], a.Q[off + j])
+                                      : Fast<T>::make4(T(0), T(0), T(0), T(0));
+                    __syncthreads();
+                    const int cnt = min(256, n - j0);
+#pragma unroll sizeof(T) == 4 ? 4 : 2
+                    for (int t = 0; t < cnt; ++t) {
+                        const vec4 aj = tile[t];                   // the same address in every lane
+                        const T dx = xi - aj.x, dy = yi - aj.y, dz = zi - aj.z;
+                        T u, du;
+                        PairTerms<T, kDamped>::of(dx * dx + dy * dy + dz * dz, u, du);      // zero for the atom itself (r = 0)
+                        su = fma(aj.w, u, su);
+                        if constexpr (kGrad) {
+                            const T w = aj.w * du;
+                            fx = fma(w, dx, fx);
+                            fy = fma(w, dy, fy);
+                            fz = fma(w, dz, fz);
+                        }
+                    }
+                }
+                if (a.E) {                                         // (the same for every thread)
+                    const T share = wave_sum(have ? qi * su : T(0));
+                    __syncthreads();                               // wpart is free
+                    if (lane == 0) wpart[wave] = share;
+                    __syncthreads();
+                    if (tid == 0) atomicAdd(&a.E[mol], T(0.5) * a.K * (wpart[0] + wpart[1] + wpart[2] + wpart[3]));
+                }
+                if (kGrad && have) {
+                    const T gK = a.grads[mol] * a.K;
+                    if (a.q_grads) a.q_grads[off + i] = gK * su;
+                    if (a.gX) {
+                        a.gX[off + i] = gK * qi * fx;
+                        a.gY[off + i] = gK * qi * fy;
+                        a.gZ[off + i] = gK * qi * fz;
                     }
                 }
             }
-            if (E) {                                           // (the same for every thread)
-                const T part = wave_sum(have ? qi * su : T(0));
-                __syncthreads();                               // wpart is free
-                if (lane == 0) wpart[wave] = part;
-                __syncthreads();
-                if (tid == 0) atomicAdd(&E[mol], T(0.5) * K * (wpart[0] + wpart[1] + wpart[2] + wpart[3]));
-            }
-            if (kGrad && have) {
-                const T gK = grads[mol] * K;
-                if (q_grads) q_grads[off + i] = gK * su;
-                if (gX) {
-                    gX[off + i] = gK * qi * fx;
-                    gY[off + i] = gK * qi * fy;
-                    gZ[off + i] = gK * qi * fz;
-                }
-            }
         }
-        __syncthreads();
-    });
+    }
 }
 
-// grid of charge_large_kernel: x = molecules in flight, y = workgroups that share a molecule's blocks of 256 atoms
-static dim3 charge_large_grid(int32_t n_mols)
+// One launch for every size.  Workgroups 0 .. large - 1 (columns x parts of them) share the molecules of more than 256 atoms.
+// The workgroups behind them take `per` molecules each: the wavefronts those of up to 64 atoms (with per = 1 every fourth
+// workgroup the next four), the workgroup those of 65 to 256 one after the other.  (Three launches, one per size, cost
+// 10 us where two of them found nothing to do.)  Four workgroups per compute unit: 128 registers in double.
+template <typename T, bool kDamped, bool kGrad>
+__global__ __launch_bounds__(256, 4) void charge_kernel(ChargeArgs<T> a, int columns, int parts, int per)
 {
-    const unsigned columns = static_cast<unsigned>(n_mols < 256 ? n_mols : 256);
-    const unsigned parts = columns >= 256 ? 4u : (1024u / columns > 256u ? 256u : 1024u / columns);
-    return dim3(columns, parts);
+    __shared__ ChargeTile<T, kGrad> S;
+    const int large = columns * parts;
+    const int b = static_cast<int>(blockIdx.x) - large;
+    if (b < 0) {
+        const int g = static_cast<int>(blockIdx.x);
+        T* wpart;
+        if constexpr (kGrad) wpart = reinterpret_cast<T*>(S.acc[0]);
+        else wpart = S.wpart;
+        charge_large<T, kDamped, kGrad>(a, reinterpret_cast<typename Fast<T>::vec4*>(&S.in[0][0]), wpart, g % columns, columns, g / columns, parts);
+        return;
+    }
+    const int wave = uniform(threadIdx.x >> 6);
+    const int64_t first = static_cast<int64_t>(b) * per;
+    if (per == 4 || (b & 3) == 0) {
+        const int64_t mol = first + wave;
+        if (mol < a.n_mols) {
+            const int n = uniform(a.MACs[mol]);
+            if (n <= kSmallMaxAtoms) charge_small<T, kDamped, kGrad>(a, static_cast<int>(mol), n);
+        }
+    }
+    for (int64_t mol = first; mol < min(first + per, static_cast<int64_t>(a.n_mols)); ++mol) {
+        const int n = uniform(a.MACs[mol]);
+        if (n > kSmallMaxAtoms && n <= kMediumMaxAtoms) {
+            charge_tile<T, kDamped, kGrad>(a, S, static_cast<int>(mol), n);
+            __syncthreads();         // the next molecule reuses the tile
+        }
+    }
+}
+
+template <typename T, bool kGrad>
+hipError_t launch_charges(const ChargeArgs<T>& a, int64_t n_atoms, bool damped, bool zeroed, hipStream_t stream)
+{
+    if (a.n_mols <= 0) return hipSuccess;
+    int columns = 0, parts = 1;
+    if (n_atoms > kMediumMaxAtoms) {          // there may be large ones: at most so many, of at most so many blocks
+        columns = static_cast<int>(std::min<int64_t>({a.n_mols, 256, n_atoms / (kMediumMaxAtoms + 1)}));
+        parts = static_cast<int>(std::min<int64_t>({columns >= 256 ? 4 : 1024 / columns, 256, (n_atoms + 255) / 256}));
+        if (a.E && !zeroed) {
+            const hipError_t e = launch_zero<T>(a.E, a.n_mols, stream);
+            if (e != hipSuccess) return e;
+        }
+    }
+    // a workgroup per four molecules where they are small, per molecule where a workgroup has to work on each: 4,096
+    // boxes on a quarter of the workgroups end when the compute unit with the largest boxes does
+    const int per = n_atoms > 32 * static_cast<int64_t>(a.n_mols) ? 1 : 4;
+    const int64_t blocks = (static_cast<int64_t>(a.n_mols) + per - 1) / per + static_cast<int64_t>(columns) * parts;
+    const auto kernel = damped ? charge_kernel<T, true, kGrad> : charge_kernel<T, false, kGrad>;
+    kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream>>>(a, std::max(columns, 1), columns ? parts : 0, per);
+    return hipGetLastError();
 }
 
 }  // namespace
 
 template <typename T>
-hipError_t launch_charge_energy(const T* X, const T* Y, const T* Z, const T* Q, const int32_t* MOs,
-                                const int32_t* MACs, int32_t n_mols, bool damped, T K, T* E, hipStream_t stream)
+hipError_t launch_charge_energy(const T* X, const T* Y, const T* Z, const T* Q, const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
+                                int64_t n_atoms, bool damped, T K, T* E, hipStream_t stream)
 {
-    if (n_mols <= 0) return hipSuccess;
-    const unsigned blocks = (static_cast<unsigned>(n_mols) + 3u) / 4u;
-    // molecules of 65..256 atoms are the tile kernel's, everything else the first kernel's (each leaves the other's alone)
-    const unsigned tile_blocks = static_cast<unsigned>(n_mols < 8192 ? n_mols : 8192);
-    if (damped) {
-        charge_energy_kernel<T, true><<<dim3(blocks), dim3(256), 0, stream>>>(X, Y, Z, Q, MOs, MACs, n_mols, K, E);
-        charge_tile_kernel<T, true, false><<<dim3(tile_blocks), dim3(256), 0, stream>>>(X, Y, Z, Q, MOs, MACs, n_mols, nullptr, K, E,
-                                                                                   nullptr, nullptr, nullptr, nullptr);
-        charge_large_kernel<T, true, false><<<charge_large_grid(n_mols), dim3(256), 0, stream>>>(X, Y, Z, Q, MOs, MACs, n_mols, nullptr, K,
-                                                                                             E, nullptr, nullptr, nullptr, nullptr);
-    } else {
-        charge_energy_kernel<T, false><<<dim3(blocks), dim3(256), 0, stream>>>(X, Y, Z, Q, MOs, MACs, n_mols, K, E);
-        charge_tile_kernel<T, false, false><<<dim3(tile_blocks), dim3(256), 0, stream>>>(X, Y, Z, Q, MOs, MACs, n_mols, nullptr, K, E,
-                                                                                    nullptr, nullptr, nullptr, nullptr);
-        charge_large_kernel<T, false, false><<<charge_large_grid(n_mols), dim3(256), 0, stream>>>(X, Y, Z, Q, MOs, MACs, n_mols, nullptr, K,
-                                                                                              E, nullptr, nullptr, nullptr, nullptr);
-    }
-    return hipGetLastError();
+    return launch_charges<T, false>(ChargeArgs<T>{X, Y, Z, Q, MOs, MACs, n_mols, nullptr, K, E, nullptr, nullptr, nullptr, nullptr}, n_atoms, damped,
+                                    false, stream);
 }
 
 template <typename T>
-hipError_t launch_charge_grad(const T* X, const T* Y, const T* Z, const T* Q, const int32_t* MOs,
-                              const int32_t* MACs, int32_t n_mols, const T* grads, bool damped, T K, T* q_grads,
-                              T* gX, T* gY, T* gZ, T* E, hipStream_t stream)
+hipError_t launch_charge_grad(const T* X, const T* Y, const T* Z, const T* Q, const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
+                              int64_t n_atoms, const T* grads, bool damped, T K, T* q_grads, T* gX, T* gY, T* gZ, T* E, bool zeroed,
+                              hipStream_t stream)
 {
-    if (n_mols <= 0) return hipSuccess;
-    const unsigned blocks = (static_cast<unsigned>(n_mols) + 3u) / 4u;
-    const unsigned tile_blocks = static_cast<unsigned>(n_mols < 8192 ? n_mols : 8192);
-    if (damped) {
-        charge_grad_kernel<T, true><<<dim3(blocks), dim3(256), 0, stream>>>(X, Y, Z, Q, MOs, MACs, n_mols, grads, K, q_grads, gX, gY, gZ, E);
-        charge_tile_kernel<T, true, true><<<dim3(tile_blocks), dim3(256), 0, stream>>>(X, Y, Z, Q, MOs, MACs, n_mols, grads, K, E,
-                                                                                  q_grads, gX, gY, gZ);
-        charge_large_kernel<T, true, true><<<charge_large_grid(n_mols), dim3(256), 0, stream>>>(X, Y, Z, Q, MOs, MACs, n_mols, grads, K,
-                                                                                            E, q_grads, gX, gY, gZ);
-    } else {
-        charge_grad_kernel<T, false><<<dim3(blocks), dim3(256), 0, stream>>>(X, Y, Z, Q, MOs, MACs, n_mols, grads, K, q_grads, gX, gY, gZ, E);
-        charge_tile_kernel<T, false, true><<<dim3(tile_blocks), dim3(256), 0, stream>>>(X, Y, Z, Q, MOs, MACs, n_mols, grads, K, E,
-                                                                                   q_grads, gX, gY, gZ);
-        charge_large_kernel<T, false, true><<<charge_large_grid(n_mols), dim3(256), 0, stream>>>(X, Y, Z, Q, MOs, MACs, n_mols, grads, K,
-                                                                                             E, q_grads, gX, gY, gZ);
-    }
-    return hipGetLastError();
+    return launch_charges<T, true>(ChargeArgs<T>{X, Y, Z, Q, MOs, MACs, n_mols, grads, K, E, q_grads, gX, gY, gZ}, n_atoms, damped, zeroed, stream);
 }
 
-template hipError_t launch_charge_energy<float>(const float*, const float*, const float*, const float*, const int32_t*, const int32_t*, int32_t, bool, float, float*, hipStream_t);
-template hipError_t launch_charge_energy<double>(const double*, const double*, const double*, const double*, const int32_t*, const int32_t*, int32_t, bool, double, double*, hipStream_t);
-template hipError_t launch_charge_grad<float>(const float*, const float*, const float*, const float*, const int32_t*, const int32_t*, int32_t, const float*, bool, float, float*, float*, float*, float*, float*, hipStream_t);
-template hipError_t launch_charge_grad<double>(const double*, const double*, const double*, const double*, const int32_t*, const int32_t*, int32_t, const double*, bool, double, double*, double*, double*, double*, double*, hipStream_t);
+template hipError_t launch_charge_energy<float>(const float*, const float*, const float*, const float*, const int32_t*, const int32_t*, int32_t, int64_t, bool, float, float*, hipStream_t);
+template hipError_t launch_charge_energy<double>(const double*, const double*, const double*, const double*, const int32_t*, const int32_t*, int32_t, int64_t, bool, double, double*, hipStream_t);
+template hipError_t launch_charge_grad<float>(const float*, const float*, const float*, const float*, const int32_t*, const int32_t*, int32_t, int64_t, const float*, bool, float, float*, float*, float*, float*, float*, bool, hipStream_t);
+template hipError_t launch_charge_grad<double>(const double*, const double*, const double*, const double*, const int32_t*, const int32_t*, int32_t, int64_t, const double*, bool, double, double*, double*, double*, double*, double*, bool, hipStream_t);
 
 }  // namespace khan

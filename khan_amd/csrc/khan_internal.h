@@ -172,14 +172,16 @@ hipError_t launch_dense_first(const float* const rows[4], const int32_t n[4], co
                               const float* const bias[4], bool celu, float alpha, float* const out[4],
                               hipStream_t stream);
 
-// ---- charges: pair energy K q_i q_j (1 - f_C(r)) / r; damped = false drops f_C (plain Coulomb) ----
+// ---- charges: pair energy K q_i q_j (1 - f_C(r)) / r; damped = false drops f_C (plain Coulomb).  n_atoms: of the whole
+// batch, or INT64_MAX where it is not known (which launches for every size) ----
 template <typename T>
-hipError_t launch_charge_energy(const T* X, const T* Y, const T* Z, const T* Q, const int32_t* MOs,
-                                const int32_t* MACs, int32_t n_mols, bool damped, T K, T* E, hipStream_t stream);
+hipError_t launch_charge_energy(const T* X, const T* Y, const T* Z, const T* Q, const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
+                                int64_t n_atoms, bool damped, T K, T* E, hipStream_t stream);
+// E (may be null): the energies as well; zeroed: E holds zeros already
 template <typename T>
-hipError_t launch_charge_grad(const T* X, const T* Y, const T* Z, const T* Q, const int32_t* MOs,
-                              const int32_t* MACs, int32_t n_mols, const T* grads, bool damped, T K, T* q_grads,
-                              T* gX, T* gY, T* gZ, T* E, hipStream_t stream);     // E (may be null): the energies as well
+hipError_t launch_charge_grad(const T* X, const T* Y, const T* Z, const T* Q, const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
+                              int64_t n_atoms, const T* grads, bool damped, T K, T* q_grads, T* gX, T* gY, T* gZ, T* E, bool zeroed,
+                              hipStream_t stream);
 
 // ---- wavefront helpers (64 lanes) ----
 __device__ __forceinline__ unsigned long long wave_ballot(bool p) { return __ballot(p); }

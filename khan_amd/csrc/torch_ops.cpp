@@ -28,9 +28,7 @@ namespace {
     X(khan_featurize_grad_f32) X(khan_featurize_grad_f64) X(khan_featurize_grad_ordered_f32)                           \
     X(khan_featurize_grad_ordered_f64) X(khan_featurize_grad_inverse_f32) X(khan_featurize_grad_inverse_f64)           \
     X(khan_featurize_grad_inverse_ordered_f32) X(khan_featurize_grad_inverse_ordered_f64)                              \
-    X(khan_ani_charge_f32) X(khan_ani_charge_f64) X(khan_ani_charge_grad_f32) X(khan_ani_charge_grad_f64)              \
-    X(khan_ani_charge_grad_xyz_f32) X(khan_ani_charge_grad_xyz_f64) X(khan_ani_charge_all_f32)                         \
-    X(khan_ani_charge_all_f64) X(khan_mol_energy_f32) X(khan_mol_energy_f64) X(khan_mol_energy_grad_f32)               \
+    X(khan_ani_charges_f32) X(khan_ani_charges_f64) X(khan_mol_energy_f32) X(khan_mol_energy_f64) X(khan_mol_energy_grad_f32)               \
     X(khan_mol_energy_grad_f64) X(khan_atomic_networks_packed_bytes) X(khan_atomic_networks_f32)
 
 struct Api {
@@ -325,18 +323,24 @@ at::ScalarType check_charge(const Tensor& xs, const Tensor& ys, const Tensor& zs
     return dt;
 }
 
+template <typename Fn>
+void with_charges(at::ScalarType dt, Fn run)
+{
+    if (dt == at::kFloat) run(0.0f, api.khan_ani_charges_f32);
+    else run(0.0, api.khan_ani_charges_f64);
+}
+
 Tensor ani_charge(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& qs, const Tensor& mos, const Tensor& macs)
 {
     const auto dt = check_charge(xs, ys, zs, qs, mos, macs);
     const Tensor e = at::empty({mos.numel()}, xs.options());
-    const int32_t m = static_cast<int32_t>(mos.numel());
     const khan_stream_t st = stream();
-    if (dt == at::kFloat)
-        call(api.khan_ani_charge_f32, ptr<const float>(xs), ptr<const float>(ys), ptr<const float>(zs), ptr<const float>(qs), ptr<const int32_t>(mos),
-             ptr<const int32_t>(macs), m, ptr<float>(e), st);
-    else
-        call(api.khan_ani_charge_f64, ptr<const double>(xs), ptr<const double>(ys), ptr<const double>(zs), ptr<const double>(qs),
-             ptr<const int32_t>(mos), ptr<const int32_t>(macs), m, ptr<double>(e), st);
+    with_charges(dt, [&](auto zero, auto fn) {
+        using T = decltype(zero);
+        call(fn, ptr<const T>(xs), ptr<const T>(ys), ptr<const T>(zs), ptr<const T>(qs), ptr<const int32_t>(mos), ptr<const int32_t>(macs),
+             static_cast<int32_t>(mos.numel()), xs.numel(), static_cast<const T*>(nullptr), ptr<T>(e), static_cast<T*>(nullptr),
+             static_cast<T*>(nullptr), static_cast<T*>(nullptr), static_cast<T*>(nullptr), 0, st);
+    });
     return e;
 }
 
@@ -348,28 +352,25 @@ std::vector<Tensor> ani_charge_grads(const Tensor& xs, const Tensor& ys, const T
     const auto dt = check_charge(xs, ys, zs, qs, mos, macs);
     dev(grads, dt, "grads");
     same_size(grads.numel() == mos.numel(), "grads must have one element per molecule");
-    const int64_t n = xs.numel(), m64 = mos.numel();
-    const int32_t m = static_cast<int32_t>(m64);
-    const Tensor all = at::zeros({n * (want_xyz ? 4 : 1) + (energies ? m64 : 0)}, xs.options());
+    const int64_t n = xs.numel(), m = mos.numel();
+    const Tensor all = at::zeros({n * (want_xyz ? 4 : 1) + (energies ? m : 0)}, xs.options());
     std::vector<Tensor> out;
     int64_t at = 0;
     auto take = [&](int64_t size) {
         out.push_back(all.narrow(0, at, size));
         at += size;
     };
-    if (energies) take(m64);
+    if (energies) take(m);
     for (int k = 0; k < (want_xyz ? 4 : 1); ++k) take(n);
     const khan_stream_t st = stream();
-    auto run = [&](auto zero, auto grad, auto xyz, auto every) {
+    with_charges(dt, [&](auto zero, auto fn) {
         using T = decltype(zero);
-        const T *X = ptr<const T>(xs), *Y = ptr<const T>(ys), *Z = ptr<const T>(zs), *Q = ptr<const T>(qs), *G = ptr<const T>(grads);
-        const int32_t *o = ptr<const int32_t>(mos), *c = ptr<const int32_t>(macs);
-        if (energies) call(every, X, Y, Z, Q, o, c, m, G, ptr<T>(out[0]), ptr<T>(out[1]), ptr<T>(out[2]), ptr<T>(out[3]), ptr<T>(out[4]), st);
-        else if (want_xyz) call(xyz, X, Y, Z, Q, o, c, m, G, ptr<T>(out[0]), ptr<T>(out[1]), ptr<T>(out[2]), ptr<T>(out[3]), st);
-        else call(grad, X, Y, Z, Q, o, c, m, G, ptr<T>(out[0]), st);
-    };
-    if (dt == at::kFloat) run(0.0f, api.khan_ani_charge_grad_f32, api.khan_ani_charge_grad_xyz_f32, api.khan_ani_charge_all_f32);
-    else run(0.0, api.khan_ani_charge_grad_f64, api.khan_ani_charge_grad_xyz_f64, api.khan_ani_charge_all_f64);
+        const int q = energies ? 1 : 0;
+        T* none = nullptr;
+        call(fn, ptr<const T>(xs), ptr<const T>(ys), ptr<const T>(zs), ptr<const T>(qs), ptr<const int32_t>(mos), ptr<const int32_t>(macs),
+             static_cast<int32_t>(m), n, ptr<const T>(grads), energies ? ptr<T>(out[0]) : none, ptr<T>(out[q]), want_xyz ? ptr<T>(out[q + 1]) : none,
+             want_xyz ? ptr<T>(out[q + 2]) : none, want_xyz ? ptr<T>(out[q + 3]) : none, 1, st);
+    });
     return out;
 }
 

@@ -85,3 +85,38 @@ def test_batch_preparation_in_one_call(ops, n_atoms, n_mols):
     o = order[:n_mols].cpu().numpy()
     assert np.array_equal(np.sort(o), np.arange(n_mols)) and np.all(np.diff(np.minimum(sizes[o], 257)) <= 0)
     assert pinned.tolist() == ac.cpu().tolist() + order[-4:].cpu().tolist()
+
+
+@pytest.mark.parametrize("dtype,rtol", [(torch.float32, 1e-5), (torch.float64, 1e-12)])
+@pytest.mark.parametrize("sizes", [(1,), (64, 65), (2, 63, 64, 65, 66, 127, 128, 129, 255, 256, 257, 513, 700), (12,) * 37 + (200,), (200,) * 9 + (5, 300)])
+def test_charges_of_every_size_in_one_launch(ops, dtype, rtol, sizes):
+    """Energies, dE/dq and dE/dxyz against float64 sums over all pairs: both sides of the limits between the forms, odd and
+    even sizes, and batches of small molecules with a large one and the reverse (a workgroup per four molecules or per one)."""
+    rng = np.random.default_rng(len(sizes))
+    n = sum(sizes)
+    xyz = rng.uniform(0, 1, (n, 3)) * (np.repeat(sizes, sizes)[:, None] / 0.1) ** (1 / 3)
+    q, g = rng.normal(0, 0.3, n), rng.standard_normal(len(sizes))
+    xyz, q, g = (v.astype(np.float32 if dtype == torch.float32 else np.float64).astype(np.float64) for v in (xyz, q, g))
+    macs = np.array(sizes, dtype=np.int32)
+    mos = (np.cumsum(sizes) - sizes).astype(np.int32)
+    out = ops.ani_charge_all(*(dev(v).to(dtype) for v in (xyz[:, 0], xyz[:, 1], xyz[:, 2], q)), dev(mos), dev(macs), dev(g).to(dtype))
+    e_alone = ops.ani_charge(*(dev(v).to(dtype) for v in (xyz[:, 0], xyz[:, 1], xyz[:, 2], q)), dev(mos), dev(macs))
+    e, dq, dx, dy, dz = (v.cpu().numpy().astype(np.float64) for v in out)
+    K, Rc = float(np.float32(0.529176917)), float(np.float32(4.6))
+    for m, (o, k) in enumerate(zip(mos, macs)):
+        s = slice(o, o + k)
+        d = xyz[s][:, None] - xyz[s][None]
+        r = np.sqrt((d ** 2).sum(-1)) + np.eye(k) * 1e9
+        near = r <= Rc
+        damp = np.where(near, 0.5 - 0.5 * np.cos(np.pi * r / Rc), 1.0) * (1 - np.eye(k))
+        ddamp = np.where(near, 0.5 * np.pi / Rc * np.sin(np.pi * r / Rc), 0.0)
+        pot = K * damp / r
+        want_q = pot @ q[s]
+        want_e = 0.5 * q[s] @ want_q
+        fac = K * (ddamp / r - damp / r ** 2) / r * (1 - np.eye(k)) * q[s][:, None] * q[s][None]
+        want_x = (fac[:, :, None] * d).sum(1)
+        mag = 0.5 * np.abs(q[s]) @ (pot @ np.abs(q[s])) + 1e-30
+        assert abs(e[m] - want_e) <= rtol * mag and abs(float(e_alone[m]) - want_e) <= rtol * mag, (m, k)
+        assert np.abs(dq[s] - g[m] * want_q).max() <= rtol * (np.abs(g[m]) * (pot @ np.abs(q[s])).max() + 1e-30), (m, k)
+        got = np.stack([dx[s], dy[s], dz[s]], axis=1)
+        assert np.abs(got - g[m] * want_x).max() <= 2 * rtol * (np.abs(g[m]) * (np.abs(fac)[:, :, None] * np.abs(d)).sum(1).max() + 1e-30), (m, k)
