@@ -368,6 +368,56 @@ int khan_atomic_networks_f32(const float *const *rows_host4, const int32_t *n_ho
                              const float *const *head_b_host4, const float *const *scale_host4, float alpha,
                              float *const *value_host4, float *const *grad_host4, khan_stream_t stream);
 
+/* The per-type networks of any widths with CELU (khan/model/nn.py:38-68), layer by layer, in float32 and float64: forward,
+ * gradient, second order (a loss on the gradient) and the weights' gradients; each call is a launch for the four types.
+ * csrc/net_layers.hip describes the passes these are the steps of.  Arrays are row-major device memory of the precision
+ * in the function's name; an unused pointer is NULL, an empty type's pointers may be NULL. */
+#define KHAN_NET_CELU 0      /* out = celu(in . w + bias) */
+#define KHAN_NET_SLOPE 1     /* y celu'(act), celu' taken from the activations act */
+#define KHAN_NET_ROWS 2      /* scale[row] y (scale NULL: y), added to out where accumulate is set */
+#define KHAN_NET_TANGENT 3   /* y' = scale[row] y: out = y' celu'(act), out2 = y' d / alpha where act < 0, else 0 */
+#define KHAN_NET_SECOND 4    /* y celu'(act) + scale[row] t */
+typedef struct khan_net_layer {
+    const void *in[4], *w[4], *bias[4];                  /* [n, k]; [k, n_out], or [n_out, k] with transposed; [n_out] */
+    const void *act[4], *d[4], *t[4], *scale[4];         /* [n, n_out] and [n] */
+    void *out[4], *out2[4];                              /* [n, n_out] */
+    int32_t n[4], k, n_out, transposed, kind, accumulate;
+    double alpha;
+} khan_net_layer;
+int khan_net_layer_f32(const khan_net_layer *layer, khan_stream_t stream);
+int khan_net_layer_f64(const khan_net_layer *layer, khan_stream_t stream);
+
+/* The output layer (one value per row): value = act . w + bias, and out = w celu'(act) (either may be NULL); with second,
+ * out = scale[row] t instead. */
+typedef struct khan_net_top {
+    const void *act[4], *w[4], *bias[4], *t[4], *scale[4];
+    void *value[4], *out[4];
+    int32_t n[4], k, second;
+    double alpha;
+} khan_net_top;
+int khan_net_top_f32(const khan_net_top *top, khan_stream_t stream);
+int khan_net_top_f64(const khan_net_top *top, khan_stream_t stream);
+
+/* Gradients of all weights and biases: layer l is [widths[l], widths[l + 1]], and out holds for every layer the four types'
+ * weight gradients, then for every layer the four types' bias gradients.  Layer l's are left^T right (bit l of first) +
+ * left2^T right2 (bit l of second), and the column sums of right; left and right are [all rows, width] arrays with type t
+ * from row row0[t] on, except layer 0's left operands, which are x and x2.  A NULL right: ones.  scale_first, scale_second:
+ * the right operands' rows are multiplied by scale.  workspace: khan_net_grads_workspace_bytes_*() bytes, 16-byte aligned. */
+#define KHAN_NET_MAX_LAYERS 12
+typedef struct khan_net_grads {
+    const void *x[4], *x2[4], *scale[4];
+    const void *left[KHAN_NET_MAX_LAYERS], *right[KHAN_NET_MAX_LAYERS], *left2[KHAN_NET_MAX_LAYERS], *right2[KHAN_NET_MAX_LAYERS];
+    int64_t row0[4];
+    int32_t n[4], layers, widths[KHAN_NET_MAX_LAYERS + 1];
+    uint32_t first, second;
+    int32_t scale_first, scale_second;
+    void *out, *workspace;
+} khan_net_grads;
+int64_t khan_net_grads_workspace_bytes_f32(const khan_net_grads *grads);
+int64_t khan_net_grads_workspace_bytes_f64(const khan_net_grads *grads);
+int khan_net_grads_f32(const khan_net_grads *grads, khan_stream_t stream);
+int khan_net_grads_f64(const khan_net_grads *grads, khan_stream_t stream);
+
 /* Per-molecule sums of the atomic networks' outputs: e[m] = sum over the atoms g of molecule m of
  * out_{as[g]}[sis[g]] -- the gather to the batch's atom order and the segment sum by molecule of the reference
  * (khan/model/nn.py:165-177; trainer_multi_tower.py:350) in one launch, without the gathered copy, each molecule's

@@ -83,6 +83,14 @@ _SIGNATURES = {
     "khan_atomic_networks_f32": (ctypes.c_int, [ctypes.POINTER(_ptr), ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(_ptr),
                                                 ctypes.POINTER(_ptr), _ptr] + [ctypes.POINTER(_ptr)] * 4
                                  + [ctypes.c_float, ctypes.POINTER(_ptr), ctypes.POINTER(_ptr), _ptr]),
+    "khan_net_layer_f32": (ctypes.c_int, [_ptr, _ptr]),
+    "khan_net_layer_f64": (ctypes.c_int, [_ptr, _ptr]),
+    "khan_net_top_f32": (ctypes.c_int, [_ptr, _ptr]),
+    "khan_net_top_f64": (ctypes.c_int, [_ptr, _ptr]),
+    "khan_net_grads_workspace_bytes_f32": (ctypes.c_int64, [_ptr]),
+    "khan_net_grads_workspace_bytes_f64": (ctypes.c_int64, [_ptr]),
+    "khan_net_grads_f32": (ctypes.c_int, [_ptr, _ptr]),
+    "khan_net_grads_f64": (ctypes.c_int, [_ptr, _ptr]),
     "khan_mol_energy_f32": (ctypes.c_int, [ctypes.POINTER(_ptr)] + [_ptr] * 4 + [ctypes.c_int32, _ptr, _ptr]),
     "khan_mol_energy_f64": (ctypes.c_int, [ctypes.POINTER(_ptr)] + [_ptr] * 4 + [ctypes.c_int32, _ptr, _ptr]),
     "khan_mol_energy_grad_f32": (ctypes.c_int, [_ptr] * 5 + [ctypes.c_int32, ctypes.POINTER(_ptr), _ptr]),

@@ -15,66 +15,7 @@ Both call the HIP library through `khan_amd.ops`; there is no other implementati
 """
 import torch
 
-from . import ops
-
-
-class _FeaturizeGrad(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, xs, ys, zs, as_, mos, macs, sis, acs_host, order, size_classes, grad_h, grad_c, grad_n, grad_o):
-        ctx.save_for_backward(xs, ys, zs, as_, mos, macs, sis)
-        ctx.acs_host, ctx.order, ctx.size_classes = acs_host, order, size_classes
-        return ops.featurize_grad(xs, ys, zs, as_, mos, macs, sis, acs_host,
-                                  grad_h.contiguous(), grad_c.contiguous(), grad_n.contiguous(), grad_o.contiguous(),
-                                  order=order, size_classes=size_classes)
-
-    @staticmethod
-    def backward(ctx, dx, dy, dz):
-        xs, ys, zs, as_, mos, macs, sis = ctx.saved_tensors
-        zero = lambda: torch.zeros_like(xs)
-        dx, dy, dz = (zero() if d is None else d.contiguous() for d in (dx, dy, dz))
-        dh, dc, dn, do = ops.featurize_grad_inverse(xs, ys, zs, as_, mos, macs, sis, ctx.acs_host, dx, dy, dz,
-                                                    order=ctx.order, size_classes=ctx.size_classes)
-        return (None,) * 10 + (dh, dc, dn, do)
-
-
-class _Featurize(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, xs, ys, zs, as_, mos, macs, sis, acs, order, size_classes):
-        acs_host = [int(v) for v in (acs.detach().cpu().tolist() if isinstance(acs, torch.Tensor) else acs)]
-        ctx.save_for_backward(xs, ys, zs, as_, mos, macs, sis)
-        ctx.acs_host, ctx.order, ctx.size_classes = acs_host, order, size_classes
-        return ops.featurize(xs.detach(), ys.detach(), zs.detach(), as_, mos, macs, sis, acs_host,
-                             order=order, size_classes=size_classes)
-
-    @staticmethod
-    def backward(ctx, grad_h, grad_c, grad_n, grad_o):
-        xs, ys, zs, as_, mos, macs, sis = ctx.saved_tensors
-        grads = []
-        for g, c in zip((grad_h, grad_c, grad_n, grad_o), ctx.acs_host):
-            if g is None:
-                g = torch.zeros(c * ops.FEATURE_SIZE, dtype=xs.dtype, device=xs.device)
-            grads.append(g)
-        gx, gy, gz = _FeaturizeGrad.apply(xs.detach(), ys.detach(), zs.detach(), as_, mos, macs, sis,
-                                          ctx.acs_host, ctx.order, ctx.size_classes, *grads)
-        return gx, gy, gz, None, None, None, None, None, None, None
-
-
-class _AniCharge(torch.autograd.Function):
-    @staticmethod
-    def forward(ctx, xs, ys, zs, qs, mos, macs):
-        ctx.save_for_backward(xs, ys, zs, qs, mos, macs)
-        return ops.ani_charge(xs.detach(), ys.detach(), zs.detach(), qs.detach(), mos, macs)
-
-    @staticmethod
-    def backward(ctx, grads):
-        xs, ys, zs, qs, mos, macs = ctx.saved_tensors
-        need_xyz = any(ctx.needs_input_grad[:3])
-        args = (xs.detach(), ys.detach(), zs.detach(), qs.detach(), mos, macs, grads.contiguous())
-        if need_xyz:
-            qg, gx, gy, gz = ops.ani_charge_grad_xyz(*args)
-            return gx, gy, gz, qg, None, None
-        return None, None, None, ops.ani_charge_grad(*args), None, None
-
+from . import _native, ops
 
 
 def _library_layer_backward(ctx, xs, ws, bs, gouts, celu_act, alpha, head=None):
@@ -222,46 +163,9 @@ def dense_head(inputs, weights, biases, head_weights, head_biases, activation=op
     return _DenseHead.apply(int(activation), float(alpha), weights_t, *inputs, *weights, *biases, *head_weights, *head_biases)
 
 
-class _MolEnergy(torch.autograd.Function):
-    """Per-molecule sums of the four per-type output vectors (`ops.mol_energy`); the way back hands every atom's
-    entry its molecule's gradient (`ops.mol_energy_grad`)."""
-
-    @staticmethod
-    def forward(ctx, atom_types, sis, mos, macs, *outs):
-        ctx.save_for_backward(atom_types, sis, mos, macs)
-        ctx.counts = [int(o.numel()) for o in outs]
-        ctx.shapes = [o.shape for o in outs]
-        return ops.mol_energy([o.detach() for o in outs], atom_types, sis, mos, macs)
-
-    @staticmethod
-    def backward(ctx, ge):
-        atom_types, sis, mos, macs = ctx.saved_tensors
-        gs = _MolEnergyGrad.apply(atom_types, sis, mos, macs, tuple(ctx.counts), ge)
-        return (None, None, None, None) + tuple(g.reshape(sh) for g, sh in zip(gs, ctx.shapes))
-
-
-class _MolEnergyGrad(torch.autograd.Function):
-    """Every atom's entry of the four per-type vectors takes its molecule's value (`ops.mol_energy_grad`), the
-    transpose of the sums by molecule -- whose own way back is therefore those sums again (`ops.mol_energy`).  Both
-    maps are linear, so the pair is differentiable to any order."""
-
-    @staticmethod
-    def forward(ctx, atom_types, sis, mos, macs, counts, ge):
-        ctx.save_for_backward(atom_types, sis, mos, macs)
-        ctx.counts, ctx.dt, ctx.dev = counts, ge.dtype, ge.device
-        return tuple(ops.mol_energy_grad(ge.detach().contiguous(), atom_types, sis, mos, macs, list(counts)))
-
-    @staticmethod
-    def backward(ctx, *dgs):
-        atom_types, sis, mos, macs = ctx.saved_tensors
-        dgs = [torch.zeros(c, dtype=ctx.dt, device=ctx.dev) if d is None else d.contiguous()
-               for d, c in zip(dgs, ctx.counts)]
-        return (None,) * 5 + (_MolEnergy.apply(atom_types, sis, mos, macs, *dgs),)
-
-
 def mol_energy(type_outputs, atom_types, sis, mos, macs):
     """Differentiable per-molecule sums of the four per-type network outputs: -> [n_mols]."""
-    return _MolEnergy.apply(atom_types, sis, mos, macs, *type_outputs)
+    return _native.load().mol_energy_autograd(list(type_outputs), atom_types, sis, mos, macs)
 
 
 def dense_first(atom_type_features, acs_host, weights, biases, activation=ops.ACT_CELU, alpha=0.1, weights_t=None):
@@ -276,9 +180,9 @@ def featurize(xs, ys, zs, as_, mos, macs, sis, acs, order=None, size_classes=Non
     """Differentiable `featurize`: -> (h_feat, c_feat, n_feat, o_feat); gradients flow to xs, ys, zs.
     `order`, `size_classes`: the batch's size order (`ops.size_order`) and its four class totals on the host, shared
     by the forward pass and every derivative of it."""
-    return _Featurize.apply(xs, ys, zs, as_, mos, macs, sis, acs, order, size_classes)
+    return tuple(_native.load().featurize_autograd(xs, ys, zs, as_, mos, macs, sis, acs, order, size_classes))
 
 
 def ani_charge(xs, ys, zs, qs, mos, macs):
     """Differentiable `ani_charge`: -> charge_energies[n_mols]; gradients flow to qs and to xs, ys, zs."""
-    return _AniCharge.apply(xs, ys, zs, qs, mos, macs)
+    return _native.load().ani_charge_autograd(xs, ys, zs, qs, mos, macs)

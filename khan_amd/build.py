@@ -26,8 +26,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 ROOT = os.path.dirname(HERE)
 
-HIP_SOURCES = ["capi.hip", "aev_generic.hip", "aev_small.hip", "aev_small_bwd.hip", "aev_medium.hip", "aev_medium_bwd.hip", "aev_large_sort.hip", "sort_offsets.hip", "charges.hip", "dense_first.hip", "dense_fused.hip", "mol_sum.hip"]
-HIP_HEADERS = ["khan_internal.h", "khan_params.h", "aev_generic_center.h", "aev_small_common.h", "aev_fwd_batch.h", "aev_bwd_batch.h", "aev_large.h", os.path.join(ROOT, "include", "khan_aev.h")]
+HIP_SOURCES = ["capi.hip", "aev_generic.hip", "aev_small.hip", "aev_small_bwd.hip", "aev_medium.hip", "aev_medium_bwd.hip", "aev_large_sort.hip", "sort_offsets.hip", "charges.hip", "dense_first.hip", "dense_fused.hip", "net_layers.hip", "mol_sum.hip"]
+HIP_HEADERS = ["khan_internal.h", "khan_params.h", "aev_generic_center.h", "aev_small_common.h", "aev_fwd_batch.h", "aev_bwd_batch.h", "aev_large.h", "net_layers.h", os.path.join(ROOT, "include", "khan_aev.h")]
 
 # packed-FP32 instruction selection is switched off on purpose (target feature -packed-fp32-ops)
 HIPCC_FLAGS = [
@@ -298,7 +298,7 @@ def build_host():
     return out
 
 
-OPS_SOURCES = ("torch_ops.cpp", os.path.join(ROOT, "include", "khan_aev.h"))
+OPS_SOURCES = ("torch_ops.cpp", "torch_autograd.cpp", "torch_common.h", os.path.join(ROOT, "include", "khan_aev.h"))
 OPS_LIBRARY = os.path.join(CSRC, "_khan_ops.so")
 
 
@@ -323,9 +323,18 @@ def build_torch_ops():
     if os.path.exists(stamp_path(OPS_LIBRARY)):
         os.remove(stamp_path(OPS_LIBRARY))
     includes = ["-isystem" + p for p in cpp_extension.include_paths() + [sysconfig.get_paths()["include"], "/opt/rocm/include"]]
-    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-          "-DTORCH_EXTENSION_NAME=_khan_ops"] + includes + [os.path.join(CSRC, "torch_ops.cpp"), "-o", OPS_LIBRARY] +
-         ["-L" + p for p in cpp_extension.library_paths()] + ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-ldl"])
+    flags = ["-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_EXTENSION_NAME=_khan_ops"]
+    units = [os.path.join(CSRC, name) for name in OPS_SOURCES if name.endswith(".cpp")]
+    objects = [u.replace(".cpp", ".o") for u in units]
+    procs = []
+    for u, o in zip(units, objects):
+        cmd = ["g++"] + flags + includes + ["-c", u, "-o", o]
+        print("+", " ".join(cmd), flush=True)
+        procs.append(subprocess.Popen(cmd))
+    if any([p.wait() != 0 for p in procs]):
+        raise RuntimeError("g++ failed")
+    _run(["g++", "-shared", "-o", OPS_LIBRARY] + objects + ["-L" + p for p in cpp_extension.library_paths()] +
+         ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-lc10", "-lc10_hip", "-ldl"])
     with open(stamp_path(OPS_LIBRARY), "w") as f:
         f.write(ops_digest() + "\n")
     return OPS_LIBRARY

@@ -7,6 +7,7 @@
 #include "../../include/khan_aev.h"
 #include "khan_internal.h"
 #include "khan_params.h"
+#include "net_layers.h"
 
 // Size order of khan_featurize_f32_noalloc: the molecule indices by decreasing atom count, then the class counts
 // and cursors (khan::launch_size_order).  One copy per GPU, held until the process ends.  In host code this name
@@ -432,6 +433,100 @@ static int ani_charges(const T* xs, const T* ys, const T* zs, const T* qs, const
                                outputs_zeroed != 0);
 }
 
+// The per-type networks layer by layer (khan_net_*): the caller's structures, typed.
+template <typename T>
+static int net_layer_impl(const khan_net_layer* l, khan_stream_t stream)
+{
+    if (!l || l->k <= 0 || l->n_out <= 0 || !(l->alpha > 0.0) || l->kind < KHAN_NET_CELU || l->kind > KHAN_NET_SECOND) return KHAN_ERR_INVALID_ARG;
+    khan::NetLayer<T> a = {};
+    int64_t rows = 0;
+    for (int t = 0; t < 4; ++t) {
+        const auto in = [](const void* p) { return static_cast<const T*>(p); };
+        a.n[t] = l->n[t];
+        a.in[t] = in(l->in[t]); a.w[t] = in(l->w[t]); a.bias[t] = in(l->bias[t]); a.act[t] = in(l->act[t]);
+        a.d[t] = in(l->d[t]); a.t[t] = in(l->t[t]); a.scale[t] = in(l->scale[t]);
+        a.out[t] = static_cast<T*>(l->out[t]); a.out2[t] = static_cast<T*>(l->out2[t]);
+        if (l->n[t] < 0) return KHAN_ERR_INVALID_ARG;
+        if (l->n[t] == 0) continue;
+        const bool needs_act = l->kind == KHAN_NET_SLOPE || l->kind == KHAN_NET_TANGENT || l->kind == KHAN_NET_SECOND;
+        if (!a.in[t] || !a.w[t] || !a.out[t] || (needs_act && !a.act[t])) return KHAN_ERR_INVALID_ARG;
+        if (l->kind == KHAN_NET_TANGENT && (!a.d[t] || !a.out2[t])) return KHAN_ERR_INVALID_ARG;
+        if (l->kind == KHAN_NET_SECOND && !a.t[t]) return KHAN_ERR_INVALID_ARG;
+        rows += l->n[t];
+    }
+    if (rows > INT32_MAX) return KHAN_ERR_TOO_LARGE;
+    a.k = l->k; a.n_out = l->n_out; a.kind = l->kind; a.accumulate = l->accumulate;
+    a.alpha = static_cast<T>(l->alpha); a.inv_alpha = static_cast<T>(1.0 / l->alpha);
+    return hip_status(khan::launch_net_layer<T>(a, l->transposed != 0, as_stream(stream)));
+}
+
+template <typename T>
+static int net_top_impl(const khan_net_top* l, khan_stream_t stream)
+{
+    if (!l || l->k <= 0 || !(l->alpha > 0.0)) return KHAN_ERR_INVALID_ARG;
+    khan::NetTop<T> a = {};
+    int64_t rows = 0;
+    for (int t = 0; t < 4; ++t) {
+        const auto in = [](const void* p) { return static_cast<const T*>(p); };
+        a.n[t] = l->n[t];
+        a.act[t] = in(l->act[t]); a.w[t] = in(l->w[t]); a.bias[t] = in(l->bias[t]); a.t[t] = in(l->t[t]); a.scale[t] = in(l->scale[t]);
+        a.value[t] = static_cast<T*>(l->value[t]); a.out[t] = static_cast<T*>(l->out[t]);
+        if (l->n[t] < 0) return KHAN_ERR_INVALID_ARG;
+        if (l->n[t] == 0) continue;
+        if (l->second ? (!a.t[t] || !a.out[t] || a.value[t]) : (!a.act[t] || !a.w[t])) return KHAN_ERR_INVALID_ARG;
+        rows += l->n[t];
+    }
+    if (rows > INT32_MAX) return KHAN_ERR_TOO_LARGE;
+    a.k = l->k; a.second = l->second; a.inv_alpha = static_cast<T>(1.0 / l->alpha);
+    return hip_status(khan::launch_net_top<T>(a, as_stream(stream)));
+}
+
+template <typename T>
+static bool net_grads_args(const khan_net_grads* g, khan::NetGrads<T>& a)
+{
+    if (!g || g->layers < 1 || g->layers > KHAN_NET_MAX_LAYERS) return false;
+    static_assert(KHAN_NET_MAX_LAYERS == khan::kNetMaxLayers, "one limit");
+    a = {};
+    const auto in = [](const void* p) { return static_cast<const T*>(p); };
+    for (int t = 0; t < 4; ++t) {
+        if (g->n[t] < 0 || g->row0[t] < 0) return false;
+        a.n[t] = g->n[t]; a.row0[t] = g->row0[t];
+        a.x[t] = in(g->x[t]); a.x2[t] = in(g->x2[t]); a.scale[t] = in(g->scale[t]);
+    }
+    a.layers = g->layers; a.first = g->first; a.second = g->second;
+    a.scale_first = g->scale_first != 0; a.scale_second = g->scale_second != 0;
+    for (int l = 0; l < g->layers; ++l) {
+        a.left[l] = in(g->left[l]); a.right[l] = in(g->right[l]); a.left2[l] = in(g->left2[l]); a.right2[l] = in(g->right2[l]);
+    }
+    for (int l = 0; l <= g->layers; ++l) {
+        if (g->widths[l] <= 0) return false;
+        a.k[l] = g->widths[l];
+    }
+    a.out = static_cast<T*>(g->out);
+    return true;
+}
+
+template <typename T>
+static int net_grads_impl(const khan_net_grads* g, khan_stream_t stream)
+{
+    khan::NetGrads<T> a;
+    if (!net_grads_args<T>(g, a) || !g->out || !g->workspace) return KHAN_ERR_INVALID_ARG;
+    for (int l = 0; l < a.layers; ++l)
+        for (int t = 0; t < 4; ++t) {
+            if (a.n[t] == 0) continue;
+            if (((a.first >> l) & 1u) && !(l == 0 ? a.x[t] : a.left[l])) return KHAN_ERR_INVALID_ARG;
+            if (((a.second >> l) & 1u) && !(l == 0 ? a.x2[t] : a.left2[l])) return KHAN_ERR_INVALID_ARG;
+        }
+    return hip_status(khan::launch_net_grads<T>(a, g->workspace, as_stream(stream)));
+}
+
+template <typename T>
+static int64_t net_grads_bytes(const khan_net_grads* g)
+{
+    khan::NetGrads<T> a;
+    return net_grads_args<T>(g, a) ? static_cast<int64_t>(khan::net_grads_workspace<T>(a)) : -1;
+}
+
 extern "C" {
 
 int32_t khan_feature_size(void) { return khan::kFeats; }
@@ -823,6 +918,15 @@ int khan_atomic_networks_f32(const float* const* rows_host4, const int32_t* n_ho
         biases_host12, biases_host12 + 4, biases_host12 + 8, head_w_host4, head_b_host4, scale_host4, alpha, value_host4,
         grad_host4, packed, as_stream(stream)));
 }
+
+int khan_net_layer_f32(const khan_net_layer* layer, khan_stream_t stream) { return net_layer_impl<float>(layer, stream); }
+int khan_net_layer_f64(const khan_net_layer* layer, khan_stream_t stream) { return net_layer_impl<double>(layer, stream); }
+int khan_net_top_f32(const khan_net_top* top, khan_stream_t stream) { return net_top_impl<float>(top, stream); }
+int khan_net_top_f64(const khan_net_top* top, khan_stream_t stream) { return net_top_impl<double>(top, stream); }
+int64_t khan_net_grads_workspace_bytes_f32(const khan_net_grads* grads) { return net_grads_bytes<float>(grads); }
+int64_t khan_net_grads_workspace_bytes_f64(const khan_net_grads* grads) { return net_grads_bytes<double>(grads); }
+int khan_net_grads_f32(const khan_net_grads* grads, khan_stream_t stream) { return net_grads_impl<float>(grads, stream); }
+int khan_net_grads_f64(const khan_net_grads* grads, khan_stream_t stream) { return net_grads_impl<double>(grads, stream); }
 
 // Per-molecule sums of the per-type network outputs, and the way back.
 int khan_mol_energy_f32(const float* const* out_host4, const int32_t* as, const int32_t* sis, const int32_t* mos,

@@ -1,0 +1,537 @@
+// The per-type atomic networks of any widths with CELU (khan/model/nn.py:38-68, activations.py:63-65), float32 and float64,
+// layer by layer: the products of the forward pass, of the gradient, of a loss on the gradient (second order), and of the
+// weights' gradients, for the four atom types in one launch each.
+//
+// With z_l = a_{l-1} W_l + b_l, a_l = celu(z_l), value = a_L w + b (L hidden layers, a_0 = the feature row x):
+//     d_l    = d value / d z_l,  d_L = w celu'(z_L),  d_{l-1} = (d_l W_l^T) celu'(z_{l-1}),  d value / d x = d_1 W_1^T
+//     tangent along x' :  z'_l = a'_{l-1} W_l,  a'_l = celu'(z_l) z'_l
+//     q_l    = d phi / d z_l of phi = sum_r s_r (tangent of value_r), whose gradient a loss on d value / d x needs:
+//              q_L = s t_L,  q_{l-1} = (q_l W_l^T) celu'(z_{l-1}) + s t_{l-1},  t_l = celu''(z_l) z'_l (d value / d a_l)
+//     dW_l   = a_{l-1}^T q_l + a'_{l-1}^T (s d_l),   db_l = sum of q_l over the rows
+// and for phi = sum_r s_r value_r, plain training, dW_l = a_{l-1}^T (s d_l).  celu' and celu'' come from the activation: 1
+// and 0 for a >= 0, a / alpha + 1 and that over alpha below; t_l = z'_l d_l / alpha for a_l < 0.  What a product needs of
+// these is formed in its epilogue, so that every operand of the next one is read as it lies in memory.
+//
+// These replace library products (rocBLAS, one per type, with elementwise passes between them) in training, in force
+// training, for networks the one-launch kernel (dense_fused.hip) is not made for, and in float64: a step on 1,024 organic
+// molecules was 95 launches, one with a loss on forces 430, an energy request 330.  Measured with what goes with it (no graph
+// in inference, csrc/torch_autograd.cpp): training on 1,024 organic molecules 1.62 -> 0.57 ms, with a loss on the forces of
+// 3,001 6.95 -> 1.15 ms, a request for an energy and a gradient in float64 3.75 -> 0.65 ms.
+//
+// The products run on the matrix instructions of the operands' own precision, v_mfma_f32_16x16x4_f32 and
+// v_mfma_f64_16x16x4_f64, with nothing staged through LDS: a lane's piece of either operand is 16 contiguous bytes of a
+// row in memory, loaded straight into registers, because the k of a step and the columns of a tile may be dealt to
+// the lanes in any order as long as both operands agree.  A step multiplies 4 kVec k (kVec = values per 16 bytes: 4 or 2),
+// the lanes of group g = lane / 16 holding k = g kVec .. g kVec + kVec - 1, and the columns of a tile are
+// kVec (lane % 16) + j, so that weights as they are stored are read 16 bytes along their columns and outputs are stored 16
+// bytes at a time.  Per step a wavefront of the 32-row form loads six kilobytes for 32 matrix instructions (1,024
+// cycles): the matrix pipe binds, at the float32 rate (52,000 rows of the eleven-layer network: 74 TFLOP/s of 153).
+#include <algorithm>
+
+#include "khan_internal.h"
+#include "net_layers.h"
+
+namespace khan {
+
+namespace {
+
+template <typename T> struct MatrixOp;
+template <> struct MatrixOp<float> {
+    typedef float acc __attribute__((ext_vector_type(4)));
+    static constexpr int kVec = 4;
+    static __device__ __forceinline__ acc mul(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+    static __device__ __forceinline__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }      // of result element v
+    static __device__ __forceinline__ float celu(float z, float alpha, float inv) { return z >= 0.f ? z : alpha * (__expf(z * inv) - 1.0f); }
+};
+template <> struct MatrixOp<double> {
+    typedef double acc __attribute__((ext_vector_type(4)));
+    static constexpr int kVec = 2;
+    static __device__ __forceinline__ acc mul(double a, double b, acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+    static __device__ __forceinline__ int row(int lane, int v) { return (lane >> 4) + 4 * v; }
+    static __device__ __forceinline__ double celu(double z, double alpha, double inv) { return z >= 0. ? z : alpha * expm1(z * inv); }
+};
+template <typename T> using Vec = T __attribute__((ext_vector_type(MatrixOp<T>::kVec)));
+
+template <typename T>
+__device__ __forceinline__ T slope(T a, T inv_alpha) { return a >= T(0) ? T(1) : fma(a, inv_alpha, T(1)); }
+
+// kVec values of a row from column c on; kWhole: 16-byte aligned and inside the row; otherwise one by one, zeros past `end`
+template <bool kWhole, typename T>
+__device__ __forceinline__ Vec<T> load(const T* __restrict__ row, int c, int end)
+{
+    if constexpr (kWhole) {
+        return *reinterpret_cast<const Vec<T>*>(row + c);
+    } else {
+        Vec<T> v;
+#pragma unroll
+        for (int e = 0; e < MatrixOp<T>::kVec; ++e) v[e] = c + e < end ? row[min(c + e, end - 1)] : T(0);
+        return v;
+    }
+}
+
+// One product for the four types, out = epilogue(in . W) with W [k, n_out] as stored, or (kTrans) in . W^T with W [n_out, k]
+// as stored.  A wavefront forms 16 kMI rows x 16 kVec columns.  kSplit: the four wavefronts of a workgroup take every
+// fourth step of one tile and their sums meet in LDS (few rows: the latency of a tile is what the launch lasts);
+// otherwise a tile each, the column tiles of a row tile side by side, so that they share its rows in cache.
+// kWhole: widths are multiples of kVec and every pointer is 16-byte aligned.
+template <typename T, int kMI, bool kTrans, bool kSplit, bool kWhole>
+__global__ __launch_bounds__(256) void layer_kernel(const NetLayer<T> a, int total)
+{
+    typedef MatrixOp<T> Op;
+    typedef typename Op::acc acc_t;
+    constexpr int V = Op::kVec, kStep = 4 * V;
+    __shared__ T part[kSplit ? 3 : 1][kSplit ? kMI * V * 4 : 1][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, grp = lane >> 4;
+    const int tile = kSplit ? static_cast<int>(blockIdx.x) : static_cast<int>(blockIdx.x) * 4 + wave;
+    if (!kSplit && tile >= total) return;
+    const int t = (tile >= a.tile_end[0]) + (tile >= a.tile_end[1]) + (tile >= a.tile_end[2]);
+    const int rel = tile - (t == 0 ? 0 : a.tile_end[t - 1]);
+    const int rt = rel / a.col_tiles, ct = rel - rt * a.col_tiles;
+    const int n = a.n[t], K = a.k, N = a.n_out;
+    const int row0 = rt * 16 * kMI, col0 = ct * 16 * V;
+    const T* __restrict__ in = a.in[t];
+    const T* __restrict__ w = a.w[t];
+
+    const T* rows[kMI];                       // this lane's rows (past the end: the last one again, never stored)
+#pragma unroll
+    for (int i = 0; i < kMI; ++i) rows[i] = in + static_cast<size_t>(min(row0 + i * 16 + l16, n - 1)) * K;
+    const int cols = col0 + V * l16;          // this lane's columns cols .. cols + V - 1
+    const int wcol = kWhole ? min(cols, N - V) : cols;       // (past the end: others again, never stored)
+
+    Vec<T> av[kMI], bv[V];
+    auto fetch = [&](int c) {
+        const int k = c * kStep + grp * V;
+        // k past the end: zeros from the rows are enough, but the loads have to stay inside the arrays
+        const bool live = k < K;
+        const int kk = kWhole ? min(k, K - V) : k;
+#pragma unroll
+        for (int i = 0; i < kMI; ++i) {
+            av[i] = load<kWhole>(rows[i], kk, K);
+            if (kWhole && !live) av[i] = Vec<T>(T(0));
+        }
+        if constexpr (!kTrans) {
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                if constexpr (kWhole) bv[e] = load<true>(w + static_cast<size_t>(kk + e) * N, wcol, N);
+                else bv[e] = load<false>(w + static_cast<size_t>(min(kk + e, K - 1)) * N, wcol, N);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < V; ++j) bv[j] = load<kWhole>(w + static_cast<size_t>(min(wcol + j, N - 1)) * K, kk, K);
+        }
+    };
+    acc_t acc[kMI][V];
+#pragma unroll
+    for (int i = 0; i < kMI; ++i)
+#pragma unroll
+        for (int j = 0; j < V; ++j) acc[i][j] = acc_t(T(0));
+    const int steps = (K + kStep - 1) / kStep;
+    const int first = kSplit ? wave : 0, stride = kSplit ? 4 : 1;
+    if (first < steps) fetch(first);
+#pragma unroll 2
+    for (int c = first; c < steps; c += stride) {
+        Vec<T> x[kMI], y[V];
+#pragma unroll
+        for (int i = 0; i < kMI; ++i) x[i] = av[i];
+#pragma unroll
+        for (int j = 0; j < V; ++j) y[j] = bv[j];
+        if (c + stride < steps) fetch(c + stride);           // in flight while this step is multiplied
+#pragma unroll
+        for (int e = 0; e < V; ++e)
+#pragma unroll
+            for (int i = 0; i < kMI; ++i)
+#pragma unroll
+                for (int j = 0; j < V; ++j) acc[i][j] = Op::mul(x[i][e], kTrans ? y[j][e] : y[e][j], acc[i][j]);
+    }
+    if constexpr (kSplit) {
+        if (wave > 0) {
+#pragma unroll
+            for (int i = 0; i < kMI; ++i)
+#pragma unroll
+                for (int j = 0; j < V; ++j)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) part[wave - 1][(i * V + j) * 4 + v][lane] = acc[i][j][v];
+        }
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int i = 0; i < kMI; ++i)
+#pragma unroll
+            for (int j = 0; j < V; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int q = (i * V + j) * 4 + v;
+                    acc[i][j][v] = (acc[i][j][v] + part[0][q][lane]) + (part[1][q][lane] + part[2][q][lane]);
+                }
+    }
+
+    // ---- epilogue: row row0 + 16 i + row(v), columns cols .. cols + V - 1
+    if (cols >= N) return;
+    Vec<T> bias = Vec<T>(T(0));
+    if (a.bias[t]) bias = load<kWhole>(a.bias[t], cols, N);
+    auto put = [&](T* out, size_t at, Vec<T> y) {
+        if constexpr (kWhole) {
+            *reinterpret_cast<Vec<T>*>(out + at) = y;
+        } else {
+#pragma unroll
+            for (int e = 0; e < V; ++e)
+                if (cols + e < N) out[at + e] = y[e];
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < kMI; ++i) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int r = row0 + i * 16 + Op::row(lane, v);
+            if (r >= n) continue;
+            const size_t at = static_cast<size_t>(r) * N + cols, base = static_cast<size_t>(r) * N;
+            Vec<T> y;
+#pragma unroll
+            for (int j = 0; j < V; ++j) y[j] = acc[i][j][v] + bias[j];
+            switch (a.kind) {
+                case kNetCelu:
+#pragma unroll
+                    for (int j = 0; j < V; ++j) y[j] = Op::celu(y[j], a.alpha, a.inv_alpha);
+                    break;
+                case kNetRows: {
+                    const T s = a.scale[t] ? a.scale[t][r] : T(1);
+#pragma unroll
+                    for (int j = 0; j < V; ++j) y[j] *= s;
+                    if (a.accumulate) y += load<kWhole>(a.out[t] + base, cols, N);
+                    break;
+                }
+                case kNetTangent: {
+                    const T s = a.scale[t] ? a.scale[t][r] : T(1);
+                    const Vec<T> h = load<kWhole>(a.act[t] + base, cols, N), d = load<kWhole>(a.d[t] + base, cols, N);
+                    Vec<T> second;
+#pragma unroll
+                    for (int j = 0; j < V; ++j) {
+                        const T zd = y[j] * s;
+                        second[j] = h[j] >= T(0) ? T(0) : zd * d[j] * a.inv_alpha;
+                        y[j] = zd * slope(h[j], a.inv_alpha);
+                    }
+                    put(a.out2[t], at, second);
+                    break;
+                }
+                default: {          // kNetSlope, kNetSecond
+                    const Vec<T> h = load<kWhole>(a.act[t] + base, cols, N);
+#pragma unroll
+                    for (int j = 0; j < V; ++j) y[j] *= slope(h[j], a.inv_alpha);
+                    if (a.kind == kNetSecond) {
+                        const T s = a.scale[t] ? a.scale[t][r] : T(1);
+                        const Vec<T> second = load<kWhole>(a.t[t] + base, cols, N);
+#pragma unroll
+                        for (int j = 0; j < V; ++j) y[j] = fma(s, second[j], y[j]);
+                    }
+                }
+            }
+            put(a.out[t], at, y);
+        }
+    }
+}
+
+// The output layer, 16 lanes per row: value = a . w + b and d = w celu'(a), whichever is asked for; or (second) q = s t.
+template <typename T>
+__global__ __launch_bounds__(256) void top_kernel(const NetTop<T> a, int total)
+{
+    const int row = static_cast<int>(blockIdx.x) * 16 + static_cast<int>(threadIdx.x >> 4), sub = threadIdx.x & 15;
+    if (row >= total) return;
+    const int t = (row >= a.row_end[0]) + (row >= a.row_end[1]) + (row >= a.row_end[2]);
+    const int r = row - (t == 0 ? 0 : a.row_end[t - 1]);
+    const size_t base = static_cast<size_t>(r) * a.k;
+    T sum = T(0);
+    for (int k = sub; k < a.k; k += 16) {
+        if (a.second) {
+            a.out[t][base + k] = (a.scale[t] ? a.scale[t][r] : T(1)) * a.t[t][base + k];
+        } else {
+            const T h = a.act[t][base + k], w = a.w[t][k];
+            sum = fma(h, w, sum);
+            if (a.out[t]) a.out[t][base + k] = w * slope(h, a.inv_alpha);
+        }
+    }
+    if (a.value[t]) {
+#pragma unroll
+        for (int d = 8; d >= 1; d >>= 1) sum += __shfl_xor(sum, d, 64);
+        if (sub == 0) a.value[t][r] = sum + (a.bias[t] ? *a.bias[t] : T(0));
+    }
+}
+
+// ---- gradients of the weights: dW [k, n_out] = sum over rows of left[r, :]^T right[r, :] (+ left2^T right2), db = sum of right
+// A workgroup forms a tile of 16 kVec x 16 kVec (64 x 64, or 32 x 32 in float64) over `per` rows, its wavefronts four rows in
+// sixteen each; a lane's 16 bytes of a row are kVec of the tile's rows (left) or columns (right), the four groups of lanes
+// hold four rows: one load of each operand per kVec^2 matrix instructions.  The wavefronts' sums meet in LDS, the
+// workgroups' in memory, where grad_sum_kernel adds them up in a fixed order: no atomics, the same bits every time.
+template <typename T>
+struct GradLds {
+    static constexpr int kVec = MatrixOp<T>::kVec;
+    T part[2][kVec * kVec * 4][64];
+    T bias[4][16 * kVec];
+};
+template <typename T, bool kWhole>
+__device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __restrict__ partial, GradLds<T>& S, int job)
+{
+    typedef MatrixOp<T> Op;
+    typedef typename Op::acc acc_t;
+    constexpr int V = Op::kVec, kSide = 16 * V;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, grp = lane >> 4;
+    const int layer = job >> 2, t = job & 3;
+    const int rel = static_cast<int>(blockIdx.x) - (job == 0 ? 0 : a.job_end[job - 1]);
+    const int K = a.k[layer], N = a.k[layer + 1], n = a.n[t];
+    const int tiles_n = (N + kSide - 1) / kSide, tiles = (K + kSide - 1) / kSide * tiles_n;
+    const int split = rel / tiles, tile = rel - split * tiles;
+    const int i0 = tile / tiles_n * kSide, j0 = tile % tiles_n * kSide;
+    const int r0 = split * a.per, r1 = min(n, r0 + a.per);
+    acc_t acc[V][V];
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+#pragma unroll
+        for (int j = 0; j < V; ++j) acc[i][j] = acc_t(T(0));
+    Vec<T> bias = Vec<T>(T(0));
+    const int ci = i0 + V * l16, cj = j0 + V * l16;
+    const int li = kWhole ? min(ci, K - V) : ci, lj = kWhole ? min(cj, N - V) : cj;
+#pragma unroll 1
+    for (int pair = 0; pair < 2; ++pair) {
+        if (!(((pair == 0 ? a.first : a.second) >> layer) & 1u)) continue;
+        const T* left = pair == 0 ? a.left[layer] : a.left2[layer];
+        const T* right = pair == 0 ? a.right[layer] : a.right2[layer];
+        if (layer == 0) left = pair == 0 ? a.x[t] : a.x2[t];
+        else left += static_cast<size_t>(a.row0[t]) * K;
+        const bool ones = right == nullptr;
+        if (!ones) right += static_cast<size_t>(a.row0[t]) * N;
+        const T* scale = (pair == 0 ? a.scale_first : a.scale_second) ? a.scale[t] : nullptr;
+#pragma unroll 4
+        for (int r = r0 + wave * 4 + grp; r < r0 + a.per; r += 16) {
+            const bool live = r < r1;
+            const size_t at = static_cast<size_t>(live ? r : r1 - 1);
+            Vec<T> x = load<kWhole>(left + at * K, li, K);
+            Vec<T> y = ones ? Vec<T>(T(1)) : load<kWhole>(right + at * N, lj, N);
+            const T s = scale ? scale[at] : T(1);
+#pragma unroll
+            for (int e = 0; e < V; ++e) {
+                x[e] = live ? x[e] : T(0);
+                y[e] = live ? y[e] * s : T(0);
+            }
+            if (pair == 0) bias += y;
+#pragma unroll
+            for (int i = 0; i < V; ++i)
+#pragma unroll
+                for (int j = 0; j < V; ++j) acc[i][j] = Op::mul(x[i], y[j], acc[i][j]);
+        }
+    }
+    // the four wavefronts' sums: 2 and 3 into LDS, 0 and 1 take them, 1 into LDS, 0 takes it
+    auto give = [&](int slot) {
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+#pragma unroll
+            for (int j = 0; j < V; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) S.part[slot][(i * V + j) * 4 + v][lane] = acc[i][j][v];
+    };
+    auto take = [&](int slot) {
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+#pragma unroll
+            for (int j = 0; j < V; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[i][j][v] += S.part[slot][(i * V + j) * 4 + v][lane];
+    };
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+        T b = bias[e];
+        b += __shfl_xor(b, 16, 64);
+        b += __shfl_xor(b, 32, 64);
+        if (grp == 0) S.bias[wave][V * l16 + e] = b;
+    }
+    if (wave >= 2) give(wave - 2);
+    __syncthreads();
+    if (wave < 2) take(wave);
+    __syncthreads();
+    if (wave == 1) give(0);
+    __syncthreads();
+    if (wave != 0) return;
+    take(0);
+    // tile element (i, j): row kVec row(v) + i of the tile, column kVec l16 + j
+    T* __restrict__ out = partial + static_cast<size_t>(blockIdx.x) * (kSide * kSide + kSide);
+#pragma unroll
+    for (int i = 0; i < V; ++i)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            Vec<T> y;
+#pragma unroll
+            for (int j = 0; j < V; ++j) y[j] = acc[i][j][v];
+            *reinterpret_cast<Vec<T>*>(out + (V * Op::row(lane, v) + i) * kSide + V * l16) = y;
+        }
+    if (lane < kSide) out[kSide * kSide + lane] = (S.bias[0][lane] + S.bias[1][lane]) + (S.bias[2][lane] + S.bias[3][lane]);
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void weight_grad_kernel(const NetGrads<T> a, T* __restrict__ partial)
+{
+    __shared__ GradLds<T> S;
+    int job = 0;
+    while (static_cast<int>(blockIdx.x) >= a.job_end[job]) ++job;                 // (layer, type)
+    if ((a.whole >> (job >> 2)) & 1u) weight_grad_tile<T, true>(a, partial, S, job);
+    else weight_grad_tile<T, false>(a, partial, S, job);
+}
+
+// the workgroups' partial tiles and bias sums -> the gradients, a thread per element
+template <typename T>
+__global__ __launch_bounds__(256) void grad_sum_kernel(const NetGrads<T> a, const T* __restrict__ partial, int64_t elements)
+{
+    constexpr int V = MatrixOp<T>::kVec, kSide = 16 * V, kStride = kSide * kSide + kSide;
+    const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (e >= elements) return;
+    // all weights first (type by type inside a layer), then all biases
+    int64_t at = e;
+    int layer = 0, t = 0;
+    bool is_bias = false;
+    for (;; ++layer) {
+        if (layer == a.layers) {
+            if (is_bias) return;
+            is_bias = true;
+            layer = 0;
+        }
+        const int64_t size = is_bias ? a.k[layer + 1] : static_cast<int64_t>(a.k[layer]) * a.k[layer + 1];
+        if (at < 4 * size) {
+            t = static_cast<int>(at / size);
+            at -= t * size;
+            break;
+        }
+        at -= 4 * size;
+    }
+    const int K = a.k[layer], N = a.k[layer + 1];
+    const int tiles_n = (N + kSide - 1) / kSide, tiles = (K + kSide - 1) / kSide * tiles_n;
+    const int splits = (a.n[t] + a.per - 1) / a.per, job = layer * 4 + t;
+    int tile;
+    int64_t within;
+    if (is_bias) {
+        tile = static_cast<int>(at) / kSide;                    // the first row of tiles holds the bias sums
+        within = kSide * kSide + at % kSide;
+    } else {
+        const int i = static_cast<int>(at / N), j = static_cast<int>(at % N);
+        tile = i / kSide * tiles_n + j / kSide;
+        within = (i % kSide) * kSide + j % kSide;
+    }
+    const T* p = partial + static_cast<size_t>((job == 0 ? 0 : a.job_end[job - 1]) + tile) * kStride + within;
+    T sum = T(0);
+#pragma unroll 4
+    for (int s = 0; s < splits; ++s) sum += p[static_cast<size_t>(s) * tiles * kStride];
+    a.out[e] = sum;
+}
+
+template <typename T>
+bool aligned(const T* const (&p)[4], const int (&n)[4])
+{
+    for (int t = 0; t < 4; ++t)
+        if (n[t] > 0 && (reinterpret_cast<uintptr_t>(p[t]) & 15u)) return false;
+    return true;
+}
+
+template <typename T, int kMI, bool kSplit>
+void launch_layer_kernel(NetLayer<T>& a, bool trans, bool whole, hipStream_t stream)
+{
+    constexpr int V = MatrixOp<T>::kVec;
+    a.col_tiles = (a.n_out + 16 * V - 1) / (16 * V);
+    int total = 0;
+    for (int t = 0; t < 4; ++t) a.tile_end[t] = total += (a.n[t] + 16 * kMI - 1) / (16 * kMI) * a.col_tiles;
+    const dim3 grid(static_cast<unsigned>(kSplit ? total : (total + 3) / 4));
+    if (trans) {
+        if (whole) layer_kernel<T, kMI, true, kSplit, true><<<grid, dim3(256), 0, stream>>>(a, total);
+        else layer_kernel<T, kMI, true, kSplit, false><<<grid, dim3(256), 0, stream>>>(a, total);
+    } else {
+        if (whole) layer_kernel<T, kMI, false, kSplit, true><<<grid, dim3(256), 0, stream>>>(a, total);
+        else layer_kernel<T, kMI, false, kSplit, false><<<grid, dim3(256), 0, stream>>>(a, total);
+    }
+}
+
+}  // namespace
+
+template <typename T>
+hipError_t launch_net_layer(NetLayer<T> a, bool trans, hipStream_t stream)
+{
+    constexpr int V = MatrixOp<T>::kVec;
+    const int64_t rows = static_cast<int64_t>(a.n[0]) + a.n[1] + a.n[2] + a.n[3];
+    if (rows == 0) return hipSuccess;
+    bool whole = a.k % V == 0 && a.n_out % V == 0 && aligned<T>(a.in, a.n) && aligned<T>(a.w, a.n);
+    for (int t = 0; t < 4 && whole; ++t)
+        if (a.n[t] > 0)
+            whole = ((reinterpret_cast<uintptr_t>(a.bias[t]) | reinterpret_cast<uintptr_t>(a.act[t]) | reinterpret_cast<uintptr_t>(a.d[t]) |
+                      reinterpret_cast<uintptr_t>(a.t[t]) | reinterpret_cast<uintptr_t>(a.out[t]) | reinterpret_cast<uintptr_t>(a.out2[t])) & 15u) == 0;
+    // 32 rows per wavefront where that fills the GPU (1,024 SIMDs) with wavefronts of their own, 16 below, and a workgroup
+    // per tile where even those are few
+    const int64_t col_tiles = (a.n_out + 16 * V - 1) / (16 * V);
+    if (rows / 32 * col_tiles >= 1024) launch_layer_kernel<T, 2, false>(a, trans, whole, stream);
+    else if (rows / 16 * col_tiles >= 1024 || a.k < 8 * V) launch_layer_kernel<T, 1, false>(a, trans, whole, stream);
+    else launch_layer_kernel<T, 1, true>(a, trans, whole, stream);
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t launch_net_top(NetTop<T> a, hipStream_t stream)
+{
+    int total = 0;
+    for (int t = 0; t < 4; ++t) a.row_end[t] = total += a.n[t];
+    if (total == 0) return hipSuccess;
+    top_kernel<T><<<dim3((total + 15u) / 16u), dim3(256), 0, stream>>>(a, total);
+    return hipGetLastError();
+}
+
+// rows per workgroup, the workgroups' numbering, and the bytes of partial sums
+template <typename T>
+static int64_t plan_grads(NetGrads<T>& a)
+{
+    constexpr int kSide = 16 * MatrixOp<T>::kVec;
+    int64_t tiles = 0, rows = 0;
+    for (int l = 0; l < a.layers; ++l) tiles += static_cast<int64_t>((a.k[l] + kSide - 1) / kSide) * ((a.k[l + 1] + kSide - 1) / kSide);
+    for (int t = 0; t < 4; ++t) rows += a.n[t];
+    // about two workgroups per compute unit and wave: short shares where rows are few, and never fewer than 64 rows
+    int64_t per = 64;
+    while (per < 4096 && rows / per * tiles > 1024) per *= 2;
+    a.per = static_cast<int>(per);
+    int64_t end = 0;
+    for (int l = 0; l < a.layers; ++l) {
+        const int64_t lt = static_cast<int64_t>((a.k[l] + kSide - 1) / kSide) * ((a.k[l + 1] + kSide - 1) / kSide);
+        for (int t = 0; t < 4; ++t) {
+            end += (a.n[t] + per - 1) / per * lt;
+            a.job_end[l * 4 + t] = static_cast<int>(end);
+        }
+    }
+    return end * (kSide * kSide + kSide) * static_cast<int64_t>(sizeof(T));
+}
+
+template <typename T>
+size_t net_grads_workspace(NetGrads<T> a) { return static_cast<size_t>(plan_grads(a)) + 16; }
+
+template <typename T>
+hipError_t launch_net_grads(NetGrads<T> a, void* workspace, hipStream_t stream)
+{
+    plan_grads(a);
+    constexpr int V = MatrixOp<T>::kVec;
+    const int blocks = a.job_end[a.layers * 4 - 1];
+    int64_t elements = 0;
+    a.whole = 0;
+    for (int l = 0; l < a.layers; ++l) {
+        elements += 4 * (static_cast<int64_t>(a.k[l]) * a.k[l + 1] + a.k[l + 1]);
+        // (operands that a layer does not have are null, which is aligned)
+        const uintptr_t bits = reinterpret_cast<uintptr_t>(a.right[l]) | reinterpret_cast<uintptr_t>(a.right2[l]) |
+                               reinterpret_cast<uintptr_t>(a.left[l]) | reinterpret_cast<uintptr_t>(a.left2[l]);
+        const bool whole = a.k[l] % V == 0 && a.k[l + 1] % V == 0 && (bits & 15u) == 0 && (l > 0 || (aligned<T>(a.x, a.n) && aligned<T>(a.x2, a.n)));
+        if (whole) a.whole |= 1u << l;
+    }
+    if (blocks > 0) weight_grad_kernel<T><<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream>>>(a, static_cast<T*>(workspace));
+    grad_sum_kernel<T><<<dim3(static_cast<unsigned>((elements + 255) / 256)), dim3(256), 0, stream>>>(a, static_cast<const T*>(workspace), elements);
+    return hipGetLastError();
+}
+
+template hipError_t launch_net_layer<float>(NetLayer<float>, bool, hipStream_t);
+template hipError_t launch_net_layer<double>(NetLayer<double>, bool, hipStream_t);
+template hipError_t launch_net_top<float>(NetTop<float>, hipStream_t);
+template hipError_t launch_net_top<double>(NetTop<double>, hipStream_t);
+template size_t net_grads_workspace<float>(NetGrads<float>);
+template size_t net_grads_workspace<double>(NetGrads<double>);
+template hipError_t launch_net_grads<float>(NetGrads<float>, void*, hipStream_t);
+template hipError_t launch_net_grads<double>(NetGrads<double>, void*, hipStream_t);
+
+}  // namespace khan

@@ -1,0 +1,721 @@
+// torch.autograd functions of the path in native code: the AEV passes, the sums by molecule, the charge energy, and the
+// per-type networks with CELU (khan/training/trainer_multi_tower.py:23-120 for the gradient wiring, khan/model/nn.py:38-68
+// for the networks).  A training step on a thousand molecules spent most of its time between launches: Python functions on
+// either side of every node, a library product per layer and type, a transposed copy of every weight.
+#include <torch/csrc/autograd/custom_function.h>
+
+#include "torch_common.h"
+
+namespace khan_torch {
+
+namespace {
+
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+using torch::autograd::Variable;
+using torch::autograd::variable_list;
+using Saved = std::vector<int64_t>;
+
+// ---------------------------------------------------------------------------------------------- AEV passes
+void keep(AutogradContext* ctx, const AevArgs& a)
+{
+    ctx->saved_data["acs"] = Saved(a.acs.v, a.acs.v + 4);
+    if (a.classes) ctx->saved_data["classes"] = Saved(a.classes->v, a.classes->v + 4);
+}
+
+AevArgs kept(AutogradContext* ctx, const Variable& order)
+{
+    AevArgs a{};
+    const auto acs = ctx->saved_data["acs"].toIntVector();
+    for (int t = 0; t < 4; ++t) a.acs.v[t] = static_cast<int32_t>(acs[t]);
+    if (order.defined()) a.order = order;
+    if (ctx->saved_data.count("classes")) {
+        const auto c = ctx->saved_data["classes"].toIntVector();
+        a.classes = Counts{};
+        for (int t = 0; t < 4; ++t) a.classes->v[t] = static_cast<int32_t>(c[t]);
+    }
+    return a;
+}
+
+Atoms7 atoms_of(const variable_list& v) { return {v[0].detach(), v[1].detach(), v[2].detach(), v[3], v[4], v[5], v[6]}; }
+
+variable_list with_order(const Atoms7& in, const AevArgs& args)
+{
+    variable_list v(in.begin(), in.end());
+    v.push_back(args.order ? *args.order : Tensor());
+    return v;
+}
+
+struct FeaturizeGradFn : Function<FeaturizeGradFn> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos,
+                                 const Tensor& macs, const Tensor& sis, const Tensor& h, const Tensor& c, const Tensor& n, const Tensor& o,
+                                 const AevArgs& args)
+    {
+        const Atoms7 in = {xs, ys, zs, as, mos, macs, sis};
+        ctx->save_for_backward(with_order(in, args));
+        keep(ctx, args);
+        return run_featurize_grad(in, args, {h.contiguous(), c.contiguous(), n.contiguous(), o.contiguous()});
+    }
+    // d / d(upstream rows): the Jacobian applied to the incoming vectors; no second derivative by the coordinates, as in
+    // the reference (trainer_multi_tower.py:64-91)
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        const auto saved = ctx->get_saved_variables();
+        std::array<Tensor, 3> v;
+        for (int k = 0; k < 3; ++k) v[k] = g[k].defined() ? g[k].contiguous() : at::zeros_like(saved[0]);
+        const auto d = run_featurize_grad_inverse(atoms_of(saved), kept(ctx, saved[7]), v);
+        variable_list out(12);
+        for (int t = 0; t < 4; ++t) out[7 + t] = d[t];
+        return out;
+    }
+};
+
+struct FeaturizeFn : Function<FeaturizeFn> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos,
+                                 const Tensor& macs, const Tensor& sis, const AevArgs& args)
+    {
+        const Atoms7 in = {xs, ys, zs, as, mos, macs, sis};
+        ctx->save_for_backward(with_order(in, args));
+        keep(ctx, args);
+        return run_featurize(in, args);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const AevArgs args = kept(ctx, saved[7]);
+        for (int t = 0; t < 4; ++t)
+            if (!g[t].defined()) g[t] = at::zeros({args.acs.v[t] * kFeats}, saved[0].options());
+        const Atoms7 in = atoms_of(saved);
+        const auto d = FeaturizeGradFn::apply(in[0], in[1], in[2], in[3], in[4], in[5], in[6], g[0], g[1], g[2], g[3], args);
+        variable_list out(8);
+        for (int k = 0; k < 3; ++k) out[k] = d[k];
+        return out;
+    }
+};
+
+std::vector<Tensor> featurize_autograd(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos, const Tensor& macs,
+                                       const Tensor& sis, const py::object& acs, const c10::optional<Tensor>& order, const py::object& size_classes)
+{
+    const AevArgs args = aev_args(acs, order, size_classes);
+    return FeaturizeFn::apply(xs, ys, zs, as, mos, macs, sis, args);
+}
+
+struct AniChargeFn : Function<AniChargeFn> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& qs, const Tensor& mos,
+                          const Tensor& macs)
+    {
+        ctx->save_for_backward({xs, ys, zs, qs, mos, macs});
+        return ani_charge(xs, ys, zs, qs, mos, macs);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        const auto s = ctx->get_saved_variables();
+        const bool xyz = ctx->needs_input_grad(0) || ctx->needs_input_grad(1) || ctx->needs_input_grad(2);
+        const auto d = ani_charge_grads(s[0].detach(), s[1].detach(), s[2].detach(), s[3].detach(), s[4], s[5], g[0].contiguous(), xyz, false);
+        if (!xyz) return {Tensor(), Tensor(), Tensor(), d[0], Tensor(), Tensor()};
+        return {d[1], d[2], d[3], d[0], Tensor(), Tensor()};
+    }
+};
+
+Tensor ani_charge_autograd(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& qs, const Tensor& mos, const Tensor& macs)
+{
+    return AniChargeFn::apply(xs, ys, zs, qs, mos, macs);
+}
+
+// ---------------------------------------------------------------------------------------------- sums by molecule
+// Both maps are linear and each is the other's transpose: the pair is differentiable to any order.
+struct MolEnergyGradFn;
+struct MolEnergyFn : Function<MolEnergyFn> {
+    static Tensor forward(AutogradContext* ctx, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs, const Tensor& o0,
+                          const Tensor& o1, const Tensor& o2, const Tensor& o3)
+    {
+        ctx->save_for_backward({types, sis, mos, macs});
+        ctx->saved_data["counts"] = Saved{o0.numel(), o1.numel(), o2.numel(), o3.numel()};
+        std::vector<Saved> shapes;
+        for (const Tensor* o : {&o0, &o1, &o2, &o3}) shapes.push_back(o->sizes().vec());
+        ctx->saved_data["shapes"] = shapes;
+        return run_mol_energy({o0, o1, o2, o3}, types, sis, mos, macs);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g);
+};
+struct MolEnergyGradFn : Function<MolEnergyGradFn> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs, Saved counts,
+                                 const Tensor& ge)
+    {
+        ctx->save_for_backward({types, sis, mos, macs});
+        ctx->saved_data["counts"] = counts;
+        ctx->saved_data["double"] = ge.scalar_type() == at::kDouble;
+        Counts c{};
+        for (int t = 0; t < 4; ++t) c.v[t] = static_cast<int32_t>(counts[t]);
+        return run_mol_energy_grad(ge.contiguous(), types, sis, mos, macs, c);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        const auto s = ctx->get_saved_variables();
+        const auto counts = ctx->saved_data["counts"].toIntVector();
+        const auto dt = ctx->saved_data["double"].toBool() ? at::kDouble : at::kFloat;
+        for (int t = 0; t < 4; ++t)
+            g[t] = g[t].defined() ? g[t].contiguous() : at::zeros({counts[t]}, s[0].options().dtype(dt));
+        return {Tensor(), Tensor(), Tensor(), Tensor(), Tensor(), MolEnergyFn::apply(s[0], s[1], s[2], s[3], g[0], g[1], g[2], g[3])};
+    }
+};
+variable_list MolEnergyFn::backward(AutogradContext* ctx, variable_list g)
+{
+    const auto s = ctx->get_saved_variables();
+    auto d = MolEnergyGradFn::apply(s[0], s[1], s[2], s[3], ctx->saved_data["counts"].toIntVector(), g[0]);
+    variable_list out(8);
+    const auto shapes = ctx->saved_data["shapes"].toList();
+    for (int t = 0; t < 4; ++t) out[4 + t] = d[t].reshape(static_cast<c10::IValue>(shapes.get(t)).toIntVector());
+    return out;
+}
+
+Tensor mol_energy_autograd(const std::vector<Tensor>& o, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs)
+{
+    same_size(o.size() == 4, "type_outputs must hold the four per-type vectors");
+    return MolEnergyFn::apply(types, sis, mos, macs, o[0], o[1], o[2], o[3]);
+}
+
+// ---------------------------------------------------------------------------------------------- networks
+// A network of `widths` (feature width first, 1 last) for the four types with its parameters in one flat array: for every
+// layer the four types' weights [in, out], then for every layer the four types' biases.
+struct Net {
+    Saved widths;
+    double alpha;
+    int layers() const { return static_cast<int>(widths.size()) - 1; }        // products, the output layer included
+    int64_t weight_at(int l, int t) const
+    {
+        int64_t at = 0;
+        for (int k = 0; k < l; ++k) at += 4 * widths[k] * widths[k + 1];
+        return at + t * widths[l] * widths[l + 1];
+    }
+    int64_t bias_at(int l, int t) const
+    {
+        int64_t at = weight_at(layers(), 0);
+        for (int k = 0; k < l; ++k) at += 4 * widths[k + 1];
+        return at + t * widths[l + 1];
+    }
+    int64_t size() const { return bias_at(layers(), 0); }
+};
+
+struct Rows {
+    Four x;                // [n_t, widths[0]]
+    int64_t n[4], row0[4], total;
+};
+
+Rows rows_of(const Net& net, const Tensor& flat, const Tensor& h, const Tensor& c, const Tensor& n, const Tensor& o)
+{
+    if (net.widths.size() < 3 || net.layers() > KHAN_NET_MAX_LAYERS || net.widths.back() != 1)
+        throw py::value_error("a network of 2 to " + std::to_string(KHAN_NET_MAX_LAYERS) + " layers, the last of width 1");
+    const auto dt = float_dtype(flat, "parameters");
+    dev(flat, dt, "parameters");
+    same_size(flat.numel() == net.size(), "the parameters do not match the network's widths");
+    Rows r;
+    r.x = {h, c, n, o};
+    r.total = 0;
+    for (int t = 0; t < 4; ++t) {
+        r.x[t] = r.x[t].detach().reshape({-1});
+        dev(r.x[t], dt, "feature rows");
+        same_size(r.x[t].numel() % net.widths[0] == 0, "feature rows must be whole rows");
+        r.n[t] = r.x[t].numel() / net.widths[0];
+        r.row0[t] = r.total;
+        r.total += r.n[t];
+    }
+    same_size(r.total <= INT32_MAX, "too many rows");
+    return r;
+}
+
+// The passes over a network's layers (khan_net_*; the names are those of csrc/net_layers.hip).
+struct Pass {
+    const Net& net;
+    const Rows& rows;
+    const Tensor& flat;
+    khan_stream_t st = stream();
+    bool f64 = flat.scalar_type() == at::kDouble;
+    size_t w = f64 ? 8 : 4;
+    int L = net.layers() - 1;                 // hidden layers
+
+    Tensor make(int64_t width) const { return at::empty({rows.total, width}, flat.options()); }
+    char* param(int64_t at) const { return static_cast<char*>(flat.data_ptr()) + at * w; }
+    char* part(const Tensor& a, int64_t width, int t) const
+    {
+        return a.defined() && rows.n[t] > 0 ? static_cast<char*>(a.data_ptr()) + rows.row0[t] * width * w : nullptr;
+    }
+    khan_net_layer layer(int l, bool back, int kind) const
+    {
+        khan_net_layer a = {};
+        a.k = static_cast<int32_t>(net.widths[back ? l + 1 : l]);
+        a.n_out = static_cast<int32_t>(net.widths[back ? l : l + 1]);
+        a.transposed = back;
+        a.kind = kind;
+        a.alpha = net.alpha;
+        for (int t = 0; t < 4; ++t) {
+            a.n[t] = static_cast<int32_t>(rows.n[t]);
+            a.w[t] = param(net.weight_at(l, t));
+        }
+        return a;
+    }
+    void set(const void* (&p)[4], const Tensor& a, int64_t width) const
+    {
+        for (int t = 0; t < 4; ++t) p[t] = part(a, width, t);
+    }
+    void set(void* (&p)[4], const Tensor& a, int64_t width) const
+    {
+        for (int t = 0; t < 4; ++t) p[t] = part(a, width, t);
+    }
+    static void set(const void* (&p)[4], const Four& a)
+    {
+        for (int t = 0; t < 4; ++t) p[t] = ptr<char>(a[t]);
+    }
+    void run(const khan_net_layer& a) const { call(f64 ? api.khan_net_layer_f64 : api.khan_net_layer_f32, &a, st); }
+    void run(const khan_net_top& a) const { call(f64 ? api.khan_net_top_f64 : api.khan_net_top_f32, &a, st); }
+
+    // activations a_1 .. a_L
+    variable_list forward() const
+    {
+        variable_list acts;
+        for (int l = 0; l < L; ++l) {
+            khan_net_layer a = layer(l, false, KHAN_NET_CELU);
+            for (int t = 0; t < 4; ++t) a.bias[t] = param(net.bias_at(l, t));
+            if (l == 0) set(a.in, rows.x);
+            else set(a.in, acts[l - 1], net.widths[l]);
+            acts.push_back(make(net.widths[l + 1]));
+            set(a.out, acts[l], net.widths[l + 1]);
+            run(a);
+        }
+        return acts;
+    }
+    // the values (into `values`, where defined) and d_L (returned, where asked for)
+    Tensor top(const Tensor& last, const Four* values, bool want_d) const
+    {
+        khan_net_top a = {};
+        a.k = static_cast<int32_t>(net.widths[L]);
+        a.alpha = net.alpha;
+        const Tensor d = want_d ? make(net.widths[L]) : Tensor();
+        set(a.act, last, net.widths[L]);
+        set(a.out, d, net.widths[L]);
+        for (int t = 0; t < 4; ++t) {
+            a.n[t] = static_cast<int32_t>(rows.n[t]);
+            a.w[t] = param(net.weight_at(L, t));
+            a.bias[t] = param(net.bias_at(L, t));
+            a.value[t] = values ? ptr<char>((*values)[t]) : nullptr;
+        }
+        run(a);
+        return d;
+    }
+    // d_1 .. d_{L-1} from d_L (returned as d[0 .. L-1], d[l] of layer l + 1)
+    variable_list slopes(const variable_list& acts, const Tensor& d_last) const
+    {
+        variable_list d(L);
+        d[L - 1] = d_last;
+        for (int l = L - 1; l >= 1; --l) {
+            khan_net_layer a = layer(l, true, KHAN_NET_SLOPE);
+            d[l - 1] = make(net.widths[l]);
+            set(a.in, d[l], net.widths[l + 1]);
+            set(a.act, acts[l - 1], net.widths[l]);
+            set(a.out, d[l - 1], net.widths[l]);
+            run(a);
+        }
+        return d;
+    }
+    // first . W_1^T, times the rows' factors (scale may hold undefined tensors: ones), into `out` or added to it
+    void to_rows(const Tensor& first, const Four& scale, const Four& out, bool accumulate) const
+    {
+        khan_net_layer a = layer(0, true, KHAN_NET_ROWS);
+        a.accumulate = accumulate;
+        set(a.in, first, net.widths[1]);
+        set(a.scale, scale);
+        for (int t = 0; t < 4; ++t) a.out[t] = ptr<char>(out[t]);
+        run(a);
+    }
+    khan_net_grads grads(const Four& scale) const
+    {
+        khan_net_grads g = {};
+        g.layers = net.layers();
+        for (size_t k = 0; k < net.widths.size(); ++k) g.widths[k] = static_cast<int32_t>(net.widths[k]);
+        for (int t = 0; t < 4; ++t) {
+            g.n[t] = static_cast<int32_t>(rows.n[t]);
+            g.row0[t] = rows.row0[t];
+        }
+        set(g.x, rows.x);
+        set(g.scale, scale);
+        return g;
+    }
+    Tensor run(khan_net_grads& g) const
+    {
+        const int64_t bytes = (f64 ? api.khan_net_grads_workspace_bytes_f64 : api.khan_net_grads_workspace_bytes_f32)(&g);
+        const Tensor ws = at::empty({bytes}, flat.options().dtype(at::kByte)), out = at::empty_like(flat);
+        g.workspace = ws.data_ptr();
+        g.out = out.data_ptr();
+        call(f64 ? api.khan_net_grads_f64 : api.khan_net_grads_f32, &g, st);
+        return out;
+    }
+    // gradient of sum_r scale_r value_r by the parameters
+    Tensor first_order(const variable_list& acts, const variable_list& d, const Four& scale) const
+    {
+        khan_net_grads g = grads(scale);
+        g.first = (1u << net.layers()) - 1u;
+        g.scale_first = 1;
+        for (int l = 0; l <= L; ++l) {
+            if (l > 0) g.left[l] = ptr<char>(acts[l - 1]);
+            if (l < L) g.right[l] = ptr<char>(d[l]);         // the output layer: ones, times the factors
+        }
+        return run(g);
+    }
+};
+
+Four like_values(const Rows& rows, const Tensor& flat)
+{
+    return {at::empty({rows.n[0]}, flat.options()), at::empty({rows.n[1]}, flat.options()), at::empty({rows.n[2]}, flat.options()),
+            at::empty({rows.n[3]}, flat.options())};
+}
+
+Four like_rows(const Net& net, const Rows& rows, const Tensor& flat)
+{
+    const Tensor all = at::empty({rows.total * net.widths[0]}, flat.options());
+    Four out;
+    for (int t = 0; t < 4; ++t) out[t] = all.narrow(0, rows.row0[t] * net.widths[0], rows.n[t] * net.widths[0]);
+    return out;
+}
+
+// The values from library operations, for derivatives of an order the kernels have no form for.
+variable_list library_values(const Net& net, const Tensor& flat, const variable_list& x)
+{
+    variable_list out;
+    for (int t = 0; t < 4; ++t) {
+        Tensor a = x[t].reshape({-1, net.widths[0]});
+        for (int l = 0; l < net.layers(); ++l) {
+            const Tensor w = flat.narrow(0, net.weight_at(l, t), net.widths[l] * net.widths[l + 1]).view({net.widths[l], net.widths[l + 1]});
+            a = at::addmm(flat.narrow(0, net.bias_at(l, t), net.widths[l + 1]), a, w);
+            if (l + 1 < net.layers())
+                a = at::where(a >= 0, a, net.alpha * at::expm1(at::clamp_max(a, 0.0) / net.alpha));
+        }
+        out.push_back(a.reshape({-1}));
+    }
+    return out;
+}
+
+variable_list library_grad(const variable_list& outputs, const variable_list& inputs, const variable_list& grads)
+{
+    variable_list o, g;
+    for (size_t k = 0; k < outputs.size(); ++k)
+        if (grads[k].defined() && outputs[k].requires_grad()) {
+            o.push_back(outputs[k]);
+            g.push_back(grads[k].reshape(outputs[k].sizes()));
+        }
+    variable_list in;
+    for (const auto& v : inputs)
+        if (v.requires_grad()) in.push_back(v);
+    variable_list got = o.empty() || in.empty() ? variable_list(in.size()) : torch::autograd::grad(o, in, g, true, true, true), out;
+    size_t k = 0;
+    for (const auto& v : inputs) out.push_back(v.requires_grad() ? got[k++] : Tensor());
+    return out;
+}
+
+Net net_of(AutogradContext* ctx) { return Net{ctx->saved_data["widths"].toIntVector(), ctx->saved_data["alpha"].toDouble()}; }
+
+Four or_zeros(const Rows& rows, const Tensor& flat, const variable_list& g, int from, int64_t width)
+{
+    Four out;
+    for (int t = 0; t < 4; ++t) {
+        const Tensor& v = g[from + t];
+        out[t] = v.defined() ? v.detach().reshape({-1}).contiguous() : at::zeros({rows.n[t] * width}, flat.options());
+    }
+    return out;
+}
+
+// The rows' gradients s_r d value_r / d x_r as a function of the parameters, the rows and s: what a loss on forces
+// differentiates once more.
+struct NetRowsFn : Function<NetRowsFn> {
+    // inputs: flat, x[4], s[4]; saved behind them: the activations and d_1 .. d_L
+    static variable_list forward(AutogradContext* ctx, const Tensor& flat, const Tensor& x0, const Tensor& x1, const Tensor& x2, const Tensor& x3,
+                                 const Tensor& s0, const Tensor& s1, const Tensor& s2, const Tensor& s3, const variable_list& kept_acts, Saved widths,
+                                 double alpha)
+    {
+        const Net net{widths, alpha};
+        const Rows rows = rows_of(net, flat, x0, x1, x2, x3);
+        const Pass p{net, rows, flat};
+        const variable_list acts(kept_acts.begin(), kept_acts.begin() + p.L);
+        const variable_list d = p.slopes(acts, kept_acts[p.L]);
+        const Four s = {s0, s1, s2, s3};
+        const Four out = like_rows(net, rows, flat);
+        p.to_rows(d[0], s, out, false);
+        variable_list save = {flat, x0, x1, x2, x3, s0, s1, s2, s3};
+        save.insert(save.end(), acts.begin(), acts.end());
+        save.insert(save.end(), d.begin(), d.end());
+        ctx->save_for_backward(save);
+        ctx->saved_data["widths"] = widths;
+        ctx->saved_data["alpha"] = alpha;
+        const Four xs = {x0, x1, x2, x3};
+        variable_list res;
+        for (int t = 0; t < 4; ++t) res.push_back(out[t].reshape(xs[t].sizes()));
+        return res;
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list u)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const Net net = net_of(ctx);
+        const Tensor flat = saved[0];
+        const variable_list x(saved.begin() + 1, saved.begin() + 5), s(saved.begin() + 5, saved.begin() + 9);
+        variable_list out(12);
+        if (at::GradMode::is_enabled()) {
+            variable_list in = {flat};
+            in.insert(in.end(), x.begin(), x.end());
+            in.insert(in.end(), s.begin(), s.end());
+            // (rows that carry no graph of their own still have to be differentiated by)
+            variable_list xs = x;
+            for (auto& v : xs)
+                if (!v.requires_grad()) v = v.detach().requires_grad_(true);
+            const auto rows = library_grad(library_values(net, flat, xs), xs, s);
+            for (int t = 0; t < 4; ++t) in[1 + t] = xs[t];
+            const auto g = library_grad(rows, in, u);
+            for (int k = 0; k < 9; ++k)
+                if (k == 0 || k > 4 || x[k - 1].requires_grad()) out[k] = g[k];
+            return out;
+        }
+        const Rows rows = rows_of(net, flat, x[0], x[1], x[2], x[3]);
+        const Pass p{net, rows, flat};
+        const int L = p.L;
+        const variable_list acts(saved.begin() + 9, saved.begin() + 9 + L), d(saved.begin() + 9 + L, saved.begin() + 9 + 2 * L);
+        const Four v = or_zeros(rows, flat, u, 0, net.widths[0]);
+        const Four scale = {s[0].detach().contiguous(), s[1].detach().contiguous(), s[2].detach().contiguous(), s[3].detach().contiguous()};
+        // the tangents along u
+        variable_list dot, second;
+        for (int l = 0; l < L; ++l) {
+            khan_net_layer a = p.layer(l, false, KHAN_NET_TANGENT);
+            if (l == 0) Pass::set(a.in, v);
+            else p.set(a.in, dot[l - 1], net.widths[l]);
+            dot.push_back(p.make(net.widths[l + 1]));
+            second.push_back(p.make(net.widths[l + 1]));
+            p.set(a.act, acts[l], net.widths[l + 1]);
+            p.set(a.d, d[l], net.widths[l + 1]);
+            p.set(a.out, dot[l], net.widths[l + 1]);
+            p.set(a.out2, second[l], net.widths[l + 1]);
+            p.run(a);
+        }
+        const bool need_x = ctx->needs_input_grad(1) || ctx->needs_input_grad(2) || ctx->needs_input_grad(3) || ctx->needs_input_grad(4);
+        const bool need_s = ctx->needs_input_grad(5) || ctx->needs_input_grad(6) || ctx->needs_input_grad(7) || ctx->needs_input_grad(8);
+        if (need_s) {          // the values' tangents
+            khan_net_top a = {};
+            a.k = static_cast<int32_t>(net.widths[L]);
+            a.alpha = net.alpha;
+            const Four e = like_values(rows, flat);
+            p.set(a.act, dot[L - 1], net.widths[L]);
+            for (int t = 0; t < 4; ++t) {
+                a.n[t] = static_cast<int32_t>(rows.n[t]);
+                a.w[t] = p.param(net.weight_at(L, t));
+                a.value[t] = ptr<char>(e[t]);
+                out[5 + t] = e[t].reshape(s[t].sizes());
+            }
+            p.run(a);
+        }
+        if (!need_x && !ctx->needs_input_grad(0)) return out;
+        // q_L .. q_1
+        variable_list q(L);
+        {
+            khan_net_top a = {};
+            a.k = static_cast<int32_t>(net.widths[L]);
+            a.alpha = net.alpha;
+            a.second = 1;
+            q[L - 1] = p.make(net.widths[L]);
+            p.set(a.t, second[L - 1], net.widths[L]);
+            p.set(a.out, q[L - 1], net.widths[L]);
+            Pass::set(a.scale, scale);
+            for (int t = 0; t < 4; ++t) a.n[t] = static_cast<int32_t>(rows.n[t]);
+            p.run(a);
+        }
+        for (int l = L - 1; l >= 1; --l) {
+            khan_net_layer a = p.layer(l, true, KHAN_NET_SECOND);
+            q[l - 1] = p.make(net.widths[l]);
+            p.set(a.in, q[l], net.widths[l + 1]);
+            p.set(a.act, acts[l - 1], net.widths[l]);
+            p.set(a.t, second[l - 1], net.widths[l]);
+            Pass::set(a.scale, scale);
+            p.set(a.out, q[l - 1], net.widths[l]);
+            p.run(a);
+        }
+        if (need_x) {
+            const Four g = like_rows(net, rows, flat);
+            p.to_rows(q[0], Four{}, g, false);
+            for (int t = 0; t < 4; ++t) out[1 + t] = g[t].reshape(x[t].sizes());
+        }
+        if (ctx->needs_input_grad(0)) {
+            khan_net_grads g = p.grads(scale);
+            g.first = (1u << L) - 1u;                      // the hidden layers: a^T q ...
+            g.second = (1u << (L + 1)) - 1u;               // ... and all: a'^T (s d), d = 1 in the output layer
+            g.scale_second = 1;
+            Pass::set(g.x2, v);
+            for (int l = 0; l <= L; ++l) {
+                if (l > 0) {
+                    g.left[l] = l < L ? ptr<char>(acts[l - 1]) : nullptr;
+                    g.left2[l] = ptr<char>(dot[l - 1]);
+                }
+                if (l < L) {
+                    g.right[l] = ptr<char>(q[l]);
+                    g.right2[l] = ptr<char>(d[l]);
+                }
+            }
+            out[0] = p.run(g);
+        }
+        return out;
+    }
+};
+
+// The values of the four types' rows as a function of the parameters and the rows.
+struct NetFn : Function<NetFn> {
+    static variable_list forward(AutogradContext* ctx, const Tensor& flat, const Tensor& x0, const Tensor& x1, const Tensor& x2, const Tensor& x3,
+                                 Saved widths, double alpha, bool graph)
+    {
+        const Net net{widths, alpha};
+        const Rows rows = rows_of(net, flat, x0, x1, x2, x3);
+        const Pass p{net, rows, flat};
+        const Four values = like_values(rows, flat);
+        variable_list acts = p.forward();
+        const Tensor d = p.top(acts.back(), &values, graph);
+        if (graph) {
+            variable_list save = {flat, x0, x1, x2, x3};
+            save.insert(save.end(), acts.begin(), acts.end());
+            save.push_back(d);
+            ctx->save_for_backward(save);
+            ctx->saved_data["widths"] = widths;
+            ctx->saved_data["alpha"] = alpha;
+        }
+        return {values[0], values[1], values[2], values[3]};
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list gs)
+    {
+        const auto saved = ctx->get_saved_variables();
+        const Net net = net_of(ctx);
+        const Tensor flat = saved[0];
+        const variable_list x(saved.begin() + 1, saved.begin() + 5);
+        const bool need_x = ctx->needs_input_grad(1) || ctx->needs_input_grad(2) || ctx->needs_input_grad(3) || ctx->needs_input_grad(4);
+        const bool need_p = ctx->needs_input_grad(0);
+        variable_list out(8);
+        if (at::GradMode::is_enabled() && need_p) {
+            const auto g = library_grad(library_values(net, flat, x), {flat, x[0], x[1], x[2], x[3]}, gs);
+            for (int k = 0; k < 5; ++k) out[k] = g[k];
+            return out;
+        }
+        const Rows rows = rows_of(net, flat, x[0], x[1], x[2], x[3]);
+        if (at::GradMode::is_enabled()) {
+            variable_list s(4);
+            for (int t = 0; t < 4; ++t) s[t] = gs[t].defined() ? gs[t].contiguous() : at::zeros({rows.n[t]}, flat.options());
+            const variable_list kept_acts(saved.begin() + 5, saved.end());
+            const auto g = NetRowsFn::apply(flat, x[0], x[1], x[2], x[3], s[0], s[1], s[2], s[3], kept_acts, net.widths, net.alpha);
+            for (int t = 0; t < 4; ++t) out[1 + t] = g[t];
+            return out;
+        }
+        const Pass p{net, rows, flat};
+        const variable_list acts(saved.begin() + 5, saved.begin() + 5 + p.L);
+        const variable_list d = p.slopes(acts, saved[5 + p.L]);
+        const Four scale = or_zeros(rows, flat, gs, 0, 1);
+        if (need_x) {
+            const Four g = like_rows(net, rows, flat);
+            p.to_rows(d[0], scale, g, false);
+            for (int t = 0; t < 4; ++t) out[1 + t] = g[t].reshape(x[t].sizes());
+        }
+        if (need_p) out[0] = p.first_order(acts, d, scale);
+        return out;
+    }
+};
+
+std::vector<Tensor> network_autograd(const Tensor& flat, const std::vector<Tensor>& x, Saved widths, double alpha)
+{
+    same_size(x.size() == 4, "four feature buckets");
+    bool graph = flat.requires_grad();
+    for (const Tensor& v : x) graph |= v.requires_grad();
+    return NetFn::apply(flat, x[0], x[1], x[2], x[3], widths, alpha, graph && at::GradMode::is_enabled());
+}
+
+// The parameters of a network (tensors of any shape) end to end in one array.
+struct FlattenFn : Function<FlattenFn> {
+    static Tensor forward(AutogradContext* ctx, at::TensorList params)
+    {
+        std::vector<Saved> shapes;
+        std::vector<Tensor> flat;
+        for (const auto& p : params) {
+            shapes.push_back(p.sizes().vec());
+            flat.push_back(p.detach().reshape({-1}));
+        }
+        ctx->saved_data["shapes"] = shapes;
+        return at::cat(flat);
+    }
+    static variable_list backward(AutogradContext* ctx, variable_list g)
+    {
+        variable_list out;
+        const auto shapes = ctx->saved_data["shapes"].toList();
+        int64_t at = 0;
+        for (size_t k = 0; k < shapes.size(); ++k) {
+            const auto shape = static_cast<c10::IValue>(shapes.get(k)).toIntVector();
+            const int64_t n = c10::multiply_integers(shape);
+            out.push_back(g[0].defined() ? g[0].narrow(0, at, n).view(shape) : Tensor());
+            at += n;
+        }
+        return out;
+    }
+};
+
+Tensor flatten(const std::vector<Tensor>& params)
+{
+    return FlattenFn::apply(at::TensorList(params));
+}
+
+// The network without a graph: the values, and with `want_grad` what `network_rows` needs to form gradients
+// -> (values[4], activations..., d_L)
+std::vector<Tensor> network_forward(const Tensor& flat, const std::vector<Tensor>& x, Saved widths, double alpha, bool want_grad)
+{
+    same_size(x.size() == 4, "four feature buckets");
+    const Net net{widths, alpha};
+    const Rows rows = rows_of(net, flat, x[0], x[1], x[2], x[3]);
+    const Pass p{net, rows, flat};
+    const Four values = like_values(rows, flat);
+    variable_list acts = p.forward();
+    const Tensor d = p.top(acts.back(), &values, want_grad);
+    std::vector<Tensor> out(values.begin(), values.end());
+    if (want_grad) {
+        out.insert(out.end(), acts.begin(), acts.end());
+        out.push_back(d);
+    }
+    return out;
+}
+
+// scale_r d value_r / d x_r from what network_forward left behind the values (scale: four vectors, or none for ones), into
+// new arrays or added to `into` (four arrays of rows) -> the four arrays
+std::vector<Tensor> network_rows(const Tensor& flat, const std::vector<Tensor>& x, Saved widths, double alpha, const std::vector<Tensor>& state,
+                                 const c10::optional<std::vector<Tensor>>& scale, const c10::optional<std::vector<Tensor>>& into)
+{
+    same_size(x.size() == 4, "four feature buckets");
+    const Net net{widths, alpha};
+    const Rows rows = rows_of(net, flat, x[0], x[1], x[2], x[3]);
+    const Pass p{net, rows, flat};
+    same_size(static_cast<int>(state.size()) == p.L + 1 && (!scale || scale->size() == 4) && (!into || into->size() == 4),
+              "state as network_forward returned it behind the values, and four scales and four arrays of rows");
+    const variable_list acts(state.begin(), state.begin() + p.L);
+    const variable_list d = p.slopes(acts, state[p.L]);
+    Four s, out = into ? Four{(*into)[0], (*into)[1], (*into)[2], (*into)[3]} : like_rows(net, rows, flat);
+    for (int t = 0; t < 4; ++t) {
+        if (scale) {
+            s[t] = (*scale)[t].reshape({-1});
+            dev(s[t], flat.scalar_type(), "scale");
+            same_size(s[t].numel() == rows.n[t], "scale must have one element per row");
+        }
+        same_size(out[t].numel() == rows.n[t] * net.widths[0] && out[t].is_contiguous() && out[t].scalar_type() == flat.scalar_type(),
+                  "arrays of rows like the features");
+    }
+    p.to_rows(d[0], s, out, into.has_value());
+    return {out[0], out[1], out[2], out[3]};
+}
+
+}  // namespace
+
+void bind_autograd(py::module_& m)
+{
+    m.def("featurize_autograd", &featurize_autograd);
+    m.def("ani_charge_autograd", &ani_charge_autograd);
+    m.def("mol_energy_autograd", &mol_energy_autograd);
+    m.def("network_autograd", &network_autograd);
+    m.def("flatten", &flatten);
+    m.def("network_forward", &network_forward);
+    m.def("network_rows", &network_rows);
+}
+
+}  // namespace khan_torch

@@ -5,41 +5,14 @@
 // by path (init), so that a build named by KHAN_AEV_LIBRARY is used here too; nothing is linked against it.
 #include <dlfcn.h>
 
-#include <array>
-#include <string>
-#include <vector>
+#include "torch_common.h"
 
-#include <ATen/hip/CachingHostAllocator.h>
-#include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
-#include <c10/hip/HIPStream.h>
-#include <torch/extension.h>
+namespace khan_torch {
 
-#include "../../include/khan_aev.h"
-
-namespace py = pybind11;
-using at::Tensor;
-
-namespace {
-
-#define KHAN_API(X)                                                                                                    \
-    X(khan_status_string) X(khan_last_hip_error) X(khan_mol_offsets) X(khan_ani_sort) X(khan_size_order)               \
-    X(khan_prepare_batch_workspace_bytes) X(khan_prepare_batch)                                                        \
-    X(khan_featurize_f32) X(khan_featurize_f64) X(khan_featurize_ordered_f32) X(khan_featurize_ordered_f64)            \
-    X(khan_featurize_grad_f32) X(khan_featurize_grad_f64) X(khan_featurize_grad_ordered_f32)                           \
-    X(khan_featurize_grad_ordered_f64) X(khan_featurize_grad_inverse_f32) X(khan_featurize_grad_inverse_f64)           \
-    X(khan_featurize_grad_inverse_ordered_f32) X(khan_featurize_grad_inverse_ordered_f64)                              \
-    X(khan_ani_charges_f32) X(khan_ani_charges_f64) X(khan_mol_energy_f32) X(khan_mol_energy_f64) X(khan_mol_energy_grad_f32)               \
-    X(khan_mol_energy_grad_f64) X(khan_atomic_networks_packed_bytes) X(khan_atomic_networks_f32)
-
-struct Api {
-#define X(name) decltype(&::name) name = nullptr;
-    KHAN_API(X)
-#undef X
-} api;
-
+Api api;
 PyObject* khan_error = nullptr;
 
-void init(const std::string& path, py::object error_type)
+static void init(const std::string& path, py::object error_type)
 {
     void* lib = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
     if (!lib) throw std::runtime_error(dlerror());
@@ -50,61 +23,6 @@ void init(const std::string& path, py::object error_type)
 #undef X
     khan_error = error_type.release().ptr();
 }
-
-void check(int status)
-{
-    if (status == KHAN_OK) return;
-    const std::string detail = api.khan_last_hip_error();
-    const std::string msg = std::string("libkhan_aev: ") + api.khan_status_string(status) + (detail.empty() ? "" : " (" + detail + ")");
-    PyErr_SetString(khan_error, msg.c_str());
-    throw py::error_already_set();
-}
-
-// the launch, with the interpreter's lock given back as a foreign-function call gives it back
-template <typename Fn, typename... Args>
-void call(Fn fn, Args... args)
-{
-    int status;
-    {
-        py::gil_scoped_release release;
-        status = fn(args...);
-    }
-    check(status);
-}
-
-khan_stream_t stream() { return c10::hip::getCurrentHIPStream().stream(); }
-
-void dev(const Tensor& t, at::ScalarType dtype, const char* name)
-{
-    if (!t.is_cuda()) throw py::type_error(std::string(name) + " must be a CUDA tensor");
-    if (t.scalar_type() != dtype)
-        throw py::type_error(std::string(name) + " must have dtype " + c10::toString(dtype) + ", got " + c10::toString(t.scalar_type()));
-    if (t.dim() != 1) throw py::value_error(std::string(name) + " must be rank 1 (flat), got rank " + std::to_string(t.dim()));
-    if (!t.is_contiguous()) throw py::value_error(std::string(name) + " must be contiguous");
-}
-
-void same_size(bool ok, const char* what)
-{
-    if (!ok) throw py::value_error(what);
-}
-
-template <typename T>
-T* ptr(const Tensor& t)
-{
-    return t.numel() > 0 ? static_cast<T*>(t.data_ptr()) : nullptr;
-}
-
-at::ScalarType float_dtype(const Tensor& x, const char* what)
-{
-    const auto dt = x.scalar_type();
-    if (dt != at::kFloat && dt != at::kDouble) throw py::type_error(std::string(what) + " must be float32 or float64, got " + c10::toString(dt));
-    return dt;
-}
-
-struct Counts {
-    int32_t v[4];
-    int64_t sum() const { return static_cast<int64_t>(v[0]) + v[1] + v[2] + v[3]; }
-};
 
 // four ints from a tensor (a device tensor is copied) or a sequence
 Counts counts4(const py::object& o, const char* what)
@@ -125,12 +43,10 @@ Counts counts4(const py::object& o, const char* what)
     return c;
 }
 
-constexpr int64_t kFeats = 384;
-constexpr int64_t kOrderExtra = 520;
 
 // ---------------------------------------------------------------------------------------------- preparation
 // -> (macs, mos, scatter_idxs, gather_idxs, atom_counts, order), slices of one allocation
-std::vector<Tensor> prepare_batch(const Tensor& mol_idxs, const Tensor& types, int64_t n_mols, const c10::optional<Tensor>& counts_pinned)
+static std::vector<Tensor> prepare_batch(const Tensor& mol_idxs, const Tensor& types, int64_t n_mols, const c10::optional<Tensor>& counts_pinned)
 {
     dev(mol_idxs, at::kInt, "mol_idxs");
     dev(types, at::kInt, "atomic_numbers");
@@ -178,9 +94,16 @@ struct Atoms {
     const int32_t* classes_ptr() const { return classes_known ? classes.v : nullptr; }
 };
 
-Atoms check_atoms(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos, const Tensor& macs,
-                  const Tensor& sis, const py::object& acs, const c10::optional<Tensor>& order, const py::object& size_classes)
+AevArgs aev_args(const py::object& acs, const c10::optional<Tensor>& order, const py::object& size_classes)
 {
+    AevArgs a{counts4(acs, "acs must hold 4 atom counts"), order, c10::nullopt};
+    if (!size_classes.is_none()) a.classes = counts4(size_classes, "size_classes must hold 4 counts");
+    return a;
+}
+
+Atoms check_atoms(const Atoms7& in, const AevArgs& args)
+{
+    const Tensor &xs = in[0], &ys = in[1], &zs = in[2], &as = in[3], &mos = in[4], &macs = in[5], &sis = in[6];
     Atoms a;
     a.dt = float_dtype(xs, "coordinates");
     dev(xs, a.dt, "xs"); dev(ys, a.dt, "ys"); dev(zs, a.dt, "zs");
@@ -188,16 +111,16 @@ Atoms check_atoms(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Te
     a.n = xs.numel();
     same_size(ys.numel() == a.n && zs.numel() == a.n && as.numel() == a.n && sis.numel() == a.n, "xs, ys, zs, as, sis must have the same length");
     same_size(mos.numel() == macs.numel(), "mos and macs must have the same length");
-    a.acs = counts4(acs, "acs must hold 4 atom counts");
+    a.acs = args.acs;
     if (a.acs.sum() != a.n)
         throw py::value_error("sum(acs)=" + std::to_string(a.acs.sum()) + " does not match the number of atoms " + std::to_string(a.n));
-    if (order) {
-        dev(*order, at::kInt, "order");
-        same_size(order->numel() == macs.numel() + kOrderExtra, "order must come from size_order(macs) of this batch");
-        a.order = ptr<const int32_t>(*order);
+    if (args.order) {
+        dev(*args.order, at::kInt, "order");
+        same_size(args.order->numel() == macs.numel() + kOrderExtra, "order must come from size_order(macs) of this batch");
+        a.order = ptr<const int32_t>(*args.order);
         a.ordered = true;
-        if (!size_classes.is_none()) {
-            a.classes = counts4(size_classes, "size_classes must hold 4 counts");
+        if (args.classes) {
+            a.classes = *args.classes;
             a.classes_known = true;
         }
     }
@@ -205,7 +128,7 @@ Atoms check_atoms(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Te
 }
 
 // four consecutive slices of one array, acs[t] * 384 elements each
-std::vector<Tensor> buckets(const Tensor& packed, const Counts& acs, int64_t width = kFeats)
+std::vector<Tensor> buckets(const Tensor& packed, const Counts& acs, int64_t width)
 {
     std::vector<Tensor> out;
     int64_t at = 0;
@@ -230,14 +153,20 @@ void run_forward(Plain plain, Ordered ordered, const Atoms& a, const Tensor& xs,
              m, ptr<const int32_t>(sis), ptr<T>(o[0]), ptr<T>(o[1]), ptr<T>(o[2]), ptr<T>(o[3]), a.acs.v, st);
 }
 
-std::vector<Tensor> featurize(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos, const Tensor& macs,
-                              const Tensor& sis, const py::object& acs, const c10::optional<Tensor>& order, const py::object& size_classes)
+std::vector<Tensor> run_featurize(const Atoms7& in, const AevArgs& args)
 {
-    const Atoms a = check_atoms(xs, ys, zs, as, mos, macs, sis, acs, order, size_classes);
-    auto out = buckets(at::empty({a.n * kFeats}, xs.options()), a.acs);
+    const Atoms a = check_atoms(in, args);
+    auto out = buckets(at::empty({a.n * kFeats}, in[0].options()), a.acs, kFeats);
+    const auto& [xs, ys, zs, as, mos, macs, sis] = in;
     if (a.dt == at::kFloat) run_forward<float>(api.khan_featurize_f32, api.khan_featurize_ordered_f32, a, xs, ys, zs, as, mos, macs, sis, out);
     else run_forward<double>(api.khan_featurize_f64, api.khan_featurize_ordered_f64, a, xs, ys, zs, as, mos, macs, sis, out);
     return out;
+}
+
+static std::vector<Tensor> featurize(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos, const Tensor& macs,
+                                     const Tensor& sis, const py::object& acs, const c10::optional<Tensor>& order, const py::object& size_classes)
+{
+    return run_featurize({xs, ys, zs, as, mos, macs, sis}, aev_args(acs, order, size_classes));
 }
 
 template <typename T, typename Plain, typename Ordered>
@@ -256,25 +185,32 @@ void run_backward(Plain plain, Ordered ordered, const Atoms& a, const Tensor& xs
              ptr<T>(o[2]), a.acs.v, st);
 }
 
-std::vector<Tensor> featurize_grad(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos,
-                                   const Tensor& macs, const Tensor& sis, const py::object& acs, const Tensor& h, const Tensor& c,
-                                   const Tensor& nn, const Tensor& oo, const c10::optional<Tensor>& order, const py::object& size_classes)
+std::vector<Tensor> run_featurize_grad(const Atoms7& in, const AevArgs& args, const Four& upstream)
 {
-    const Atoms a = check_atoms(xs, ys, zs, as, mos, macs, sis, acs, order, size_classes);
+    const Atoms a = check_atoms(in, args);
     static const char* const names[4] = {"h_grads", "c_grads", "n_grads", "o_grads"};
-    std::array<Tensor, 4> g = {h.reshape({-1}), c.reshape({-1}), nn.reshape({-1}), oo.reshape({-1})};
+    Four g;
     for (int t = 0; t < 4; ++t) {
+        g[t] = upstream[t].reshape({-1});
         dev(g[t], a.dt, names[t]);
         if (g[t].numel() != a.acs.v[t] * kFeats)
             throw py::value_error(std::string(names[t]) + " has " + std::to_string(g[t].numel()) + " elements, expected " +
                                   std::to_string(a.acs.v[t] * kFeats));
     }
+    const auto& [xs, ys, zs, as, mos, macs, sis] = in;
     const std::vector<Tensor> out = {at::empty({a.n}, xs.options()), at::empty({a.n}, xs.options()), at::empty({a.n}, xs.options())};
     if (a.dt == at::kFloat)
         run_backward<float>(api.khan_featurize_grad_f32, api.khan_featurize_grad_ordered_f32, a, xs, ys, zs, as, mos, macs, sis, g, out);
     else
         run_backward<double>(api.khan_featurize_grad_f64, api.khan_featurize_grad_ordered_f64, a, xs, ys, zs, as, mos, macs, sis, g, out);
     return out;
+}
+
+static std::vector<Tensor> featurize_grad(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos,
+                                          const Tensor& macs, const Tensor& sis, const py::object& acs, const Tensor& h, const Tensor& c,
+                                          const Tensor& n, const Tensor& o, const c10::optional<Tensor>& order, const py::object& size_classes)
+{
+    return run_featurize_grad({xs, ys, zs, as, mos, macs, sis}, aev_args(acs, order, size_classes), {h, c, n, o});
 }
 
 template <typename T, typename Plain, typename Ordered>
@@ -294,21 +230,27 @@ void run_inverse(Plain plain, Ordered ordered, const Atoms& a, const Tensor& xs,
              a.acs.v, st);
 }
 
-std::vector<Tensor> featurize_grad_inverse(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos,
-                                           const Tensor& macs, const Tensor& sis, const py::object& acs, const Tensor& vx, const Tensor& vy,
-                                           const Tensor& vz, const c10::optional<Tensor>& order, const py::object& size_classes)
+std::vector<Tensor> run_featurize_grad_inverse(const Atoms7& in, const AevArgs& args, const std::array<Tensor, 3>& v)
 {
-    const Atoms a = check_atoms(xs, ys, zs, as, mos, macs, sis, acs, order, size_classes);
-    dev(vx, a.dt, "x_grads"); dev(vy, a.dt, "y_grads"); dev(vz, a.dt, "z_grads");
-    same_size(vx.numel() == a.n && vy.numel() == a.n && vz.numel() == a.n, "x_grads, y_grads, z_grads must have one element per atom");
-    auto out = buckets(at::empty({a.n * kFeats}, xs.options()), a.acs);
+    const Atoms a = check_atoms(in, args);
+    dev(v[0], a.dt, "x_grads"); dev(v[1], a.dt, "y_grads"); dev(v[2], a.dt, "z_grads");
+    same_size(v[0].numel() == a.n && v[1].numel() == a.n && v[2].numel() == a.n, "x_grads, y_grads, z_grads must have one element per atom");
+    auto out = buckets(at::empty({a.n * kFeats}, in[0].options()), a.acs, kFeats);
+    const auto& [xs, ys, zs, as, mos, macs, sis] = in;
     if (a.dt == at::kFloat)
-        run_inverse<float>(api.khan_featurize_grad_inverse_f32, api.khan_featurize_grad_inverse_ordered_f32, a, xs, ys, zs, as, mos, macs, sis, vx,
-                           vy, vz, out);
+        run_inverse<float>(api.khan_featurize_grad_inverse_f32, api.khan_featurize_grad_inverse_ordered_f32, a, xs, ys, zs, as, mos, macs, sis, v[0],
+                           v[1], v[2], out);
     else
-        run_inverse<double>(api.khan_featurize_grad_inverse_f64, api.khan_featurize_grad_inverse_ordered_f64, a, xs, ys, zs, as, mos, macs, sis, vx,
-                            vy, vz, out);
+        run_inverse<double>(api.khan_featurize_grad_inverse_f64, api.khan_featurize_grad_inverse_ordered_f64, a, xs, ys, zs, as, mos, macs, sis, v[0],
+                            v[1], v[2], out);
     return out;
+}
+
+static std::vector<Tensor> featurize_grad_inverse(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos,
+                                                  const Tensor& macs, const Tensor& sis, const py::object& acs, const Tensor& vx, const Tensor& vy,
+                                                  const Tensor& vz, const c10::optional<Tensor>& order, const py::object& size_classes)
+{
+    return run_featurize_grad_inverse({xs, ys, zs, as, mos, macs, sis}, aev_args(acs, order, size_classes), {vx, vy, vz});
 }
 
 // ---------------------------------------------------------------------------------------------- charges
@@ -375,17 +317,8 @@ std::vector<Tensor> ani_charge_grads(const Tensor& xs, const Tensor& ys, const T
 }
 
 // ---------------------------------------------------------------------------------------------- networks
-using Four = std::array<Tensor, 4>;
-
-Four four(const std::vector<Tensor>& v, const char* what)
+Tensor run_mol_energy(const Four& type_outputs, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs)
 {
-    same_size(v.size() == 4, what);
-    return {v[0], v[1], v[2], v[3]};
-}
-
-Tensor mol_energy(const std::vector<Tensor>& type_outputs, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs)
-{
-    same_size(type_outputs.size() == 4, "type_outputs must hold the four per-type vectors");
     const auto dt = float_dtype(type_outputs[0], "type_outputs");
     Four o;
     int64_t n = 0;
@@ -410,13 +343,18 @@ Tensor mol_energy(const std::vector<Tensor>& type_outputs, const Tensor& types, 
     return e;
 }
 
-std::vector<Tensor> mol_energy_grad(const Tensor& e_grads, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs,
-                                    const py::object& acs)
+static Tensor mol_energy(const std::vector<Tensor>& type_outputs, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs)
+{
+    same_size(type_outputs.size() == 4, "type_outputs must hold the four per-type vectors");
+    return run_mol_energy({type_outputs[0], type_outputs[1], type_outputs[2], type_outputs[3]}, types, sis, mos, macs);
+}
+
+std::vector<Tensor> run_mol_energy_grad(const Tensor& e_grads, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs,
+                                        const Counts& c)
 {
     const auto dt = float_dtype(e_grads, "e_grads");
     dev(e_grads, dt, "e_grads");
     dev(types, at::kInt, "atom_types"); dev(sis, at::kInt, "sis"); dev(mos, at::kInt, "mos"); dev(macs, at::kInt, "macs");
-    const Counts c = counts4(acs, "acs must hold 4 atom counts");
     same_size(c.sum() == types.numel() && sis.numel() == types.numel() && mos.numel() == macs.numel() && e_grads.numel() == macs.numel(),
               "acs must add up to the number of atoms, and e_grads / mos / macs hold one entry per molecule");
     // one cleared array cut into the four vectors (atoms outside every molecule keep 0)
@@ -433,10 +371,17 @@ std::vector<Tensor> mol_energy_grad(const Tensor& e_grads, const Tensor& types, 
     return out;
 }
 
-}  // namespace
+static std::vector<Tensor> mol_energy_grad(const Tensor& e_grads, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs,
+                                           const py::object& acs)
+{
+    return run_mol_energy_grad(e_grads, types, sis, mos, macs, counts4(acs, "acs must hold 4 atom counts"));
+}
+
+}  // namespace khan_torch
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
+    using namespace khan_torch;
     m.def("init", &init);
     m.def("prepare_batch", &prepare_batch);
     m.def("featurize", &featurize);
@@ -446,4 +391,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("ani_charge_grads", &ani_charge_grads);
     m.def("mol_energy", &mol_energy);
     m.def("mol_energy_grad", &mol_energy_grad);
+    bind_autograd(m);
 }

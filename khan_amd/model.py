@@ -6,10 +6,10 @@ save_numpy / load_numpy (451-499), predict (655-678), coordinate_gradients (580-
 features -> per-type networks -> gather -> segment_sum (+ ani_charge) of lines 306-385.
 
 The featurizer, its gradient and the charge energy are the HIP kernels of this package (through
-`khan_amd.autograd`).  In float32 the dense layers with CELU (all but the last of the reference's default network) run in
-this package's matrix-core kernel (`ops.dense`: bias and activation in the product's epilogue, the activation's
-derivative in the prologue of the data gradient), the first one right behind the featurizer; the last layer and every
-float64 layer are plain matrix products: PyTorch's (rocBLAS).  Parameter
+`khan_amd.autograd`).  On the GPU, networks with CELU run in this package's matrix-core kernels: the reference's default
+widths in float32 with constant weights in one launch (`ops.atomic_networks`), everything else layer by layer, forward,
+gradient, second order and weight gradients (csrc/net_layers.hip).  Other activations, and the CPU, take PyTorch's
+operations.  Parameter
 names are the reference's TensorFlow variable names, `<prefix>W_<type>_<in>x<out>_l<k>:0` and
 `<prefix>b_...` (nn.py:41-60), so a checkpoint written by the reference's `save_numpy` loads unchanged;
 whatever else such a file holds (optimizer slots, learning rate, moving averages) is ignored.
@@ -18,6 +18,8 @@ import os
 
 import numpy as np
 import torch
+
+from . import _native
 
 TYPE_MAP = ("H", "C", "N", "O")
 DEFAULT_LAYERS = (128, 128, 64, 1)                       # energy_server.py:121
@@ -121,10 +123,9 @@ class MoleculeNN:
         return cache[k][1]
 
     def kernel_layers(self):
-        """How many leading layers run in this package's matrix-core kernel (`ops.dense`): float32 on the GPU, CELU
-        with its default alpha, input width a multiple of 32 and output width a multiple of 64 -- for the reference's
-        default network 384-128-128-64-1 all but the last, which `atom_outputs` folds into the launch of the one
-        before it (`ops.dense_head`)."""
+        """How many leading layers have the widths of the split-operand matrix-core kernels (`ops.dense`,
+        `ops.atomic_networks`): float32 on the GPU, CELU with its default alpha, input width a multiple of 32 and output
+        width a multiple of 64 -- for the reference's default network 384-128-128-64-1 all but the last."""
         if not (self.first_layer_kernel and self.dtype == torch.float32 and self.device.type == "cuda"
                 and self.activation_fn is celu):
             return 0
@@ -164,32 +165,53 @@ class MoleculeNN:
         # indices first (a merge sort of n atoms in every backward pass)
         return torch.index_select(torch.cat(self.type_outputs(atom_type_features)), 0, gather_idxs.long())
 
+    def layer_launches(self):
+        """True if the layers run in this package's own launches for any widths, precision and order of derivative
+        (csrc/net_layers.hip): on the GPU with CELU, two to twelve layers."""
+        return (self.first_layer_kernel and self.device.type == "cuda" and self.activation_fn is celu
+                and self.dtype in (torch.float32, torch.float64) and 3 <= len(self.layer_sizes) <= 13)
+
+    def flat_parameters(self, live):
+        """The parameters end to end as those launches take them: for every layer the four types' weights, then for every
+        layer the four types' biases.  `live`: as part of the graph; otherwise kept until a parameter is written again."""
+        ps = [self.params[self.names[t][k][j]] for j in (0, 1) for k in range(len(self.layer_sizes) - 1) for t in TYPE_MAP]
+        native = _native.load()
+        if live:
+            return native.flatten(ps)
+        from . import ops
+        key = [ops._stream()] + [(p.data_ptr(), p._version) for p in ps]
+        if self.__dict__.get("_flat_key") != key:
+            with torch.no_grad():
+                self._flat, self._flat_key = native.flatten(ps), key
+        return self._flat
+
     def type_outputs(self, atom_type_features):
         """Per-type flat feature buckets -> the four per-type output vectors [acs[t]] (nn.py:165-175)."""
-        nk = self.kernel_layers()
-        if nk > 0:
-            from . import autograd
-            # inference: the weights are constants here (a custom autograd function cannot tell that only the
-            # coordinates' gradient was asked for, and would form the weights' gradient, a second product, every time)
-            par = (lambda k: self.params[k]) if self.weights_need_grad else (lambda k: self.params[k].detach())
-            a = atom_type_features
-            # the output layer rides in the last hidden layer's launch when that layer is a kernel layer of width 64
-            fuse_head = nk == len(self.layer_sizes) - 2 and self.layer_sizes[-2] == 64
-            for k in range(nk - 1 if fuse_head else nk):
-                rows = [self.names[t][k] for t in TYPE_MAP]
-                a = autograd.dense(a, [par(r[0]) for r in rows], [par(r[1]) for r in rows], alpha=0.1,
-                                   weights_t=self.layer_transposed(k))
-            if fuse_head:
-                rows = [self.names[t][nk - 1] for t in TYPE_MAP]
-                head = [self.names[t][nk] for t in TYPE_MAP]
-                outs = autograd.dense_head(a, [par(r[0]) for r in rows], [par(r[1]) for r in rows],
-                                           [par(r[0]) for r in head], [par(r[1]) for r in head], alpha=0.1,
-                                           weights_t=self.layer_transposed(nk - 1))
-            else:
-                outs = [self.atom_type_outputs(t, a[t], layers_done=nk) for t in range(4)]
-        else:
-            outs = [self.atom_type_outputs(t, f.reshape(-1, FEATURE_SIZE)) for t, f in enumerate(atom_type_features)]
-        return list(outs)
+        if not self.layer_launches():
+            return [self.atom_type_outputs(t, f.reshape(-1, FEATURE_SIZE)) for t, f in enumerate(atom_type_features)]
+        # in single precision inference is the default: the weights are constants
+        live = torch.is_grad_enabled() and (self.weights_need_grad or self.dtype == torch.float64 or self.kernel_layers() == 0)
+        return _native.load().network_autograd(self.flat_parameters(live), list(atom_type_features), self.layer_sizes, 0.1)
+
+
+    def values(self, feats, want_grad, scaled=False):
+        """The networks on the featurizer's buckets without a graph -> (the four vectors of values, rows), rows(scale, into)
+        the four buckets of scale * d value / d feature row (`scale`: four vectors, or None for ones), added to the buckets
+        `into` where given.  `scaled`: rows will be called with a scale, which is not known yet."""
+        from . import ops
+        feats = list(feats)
+        if self.one_launch():
+            packed, biases, head_w, head_b = self.one_launch_operands()
+            run = lambda scale, grad: ops.atomic_networks(feats, None, biases, head_w, head_b, scales=scale, want_grad=grad, packed=packed)
+            values, grads = run(None, want_grad and not scaled)
+
+            def rows(scale=None, into=None):
+                g = [r.reshape(-1) for r in (run(scale, True)[1] if scaled else grads)]
+                return g if into is None else torch._foreach_add(into, g)
+            return values, rows
+        native, flat = _native.load(), self.flat_parameters(False)
+        out = native.network_forward(flat, feats, self.layer_sizes, 0.1, want_grad)
+        return out[:4], lambda scale=None, into=None: native.network_rows(flat, feats, self.layer_sizes, 0.1, out[4:], scale, into)
 
 
 class AniModel:
@@ -239,22 +261,38 @@ class AniModel:
     # --------------------------------------------------------------------------------------- inference
     def batch_energies(self, b, need_grad=False):
         """DeviceBatch -> per-molecule energies [n_mols] (and d energy / d xyz when need_grad)."""
-        from . import autograd, ops
+        if not self.near.layer_launches():
+            return self._energies_through_autograd(b, need_grad)
+        from . import ops
         xs, ys, zs = b.xs, b.ys, b.zs
         acs, order, classes = b.host_counts()
-        if self.charge is None and self.near.one_launch():
-            # featurize -> the four networks in one launch (values, and the gradient of their sum with respect to the
-            # feature rows) -> sums by molecule; the coordinate gradient is featurize_grad of those rows' gradients
-            feats = ops.featurize(xs, ys, zs, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs, acs,
-                                  order=order, size_classes=classes)
-            packed, biases, head_w, head_b = self.near.one_launch_operands()
-            values, grads = ops.atomic_networks(feats, None, biases, head_w, head_b, want_grad=need_grad, packed=packed)
-            energies = ops.mol_energy(values, b.atom_types, b.scatter_idxs, b.mol_offsets, b.mol_atom_counts)
+        atoms = (xs, ys, zs, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs, acs)
+        feats = ops.featurize(*atoms, order=order, size_classes=classes)
+        # the networks' values and, with need_grad, the gradients by the feature rows; no graph: the order of the passes is
+        # known, and the gradient of the near network's sum needs nothing from behind it
+        values, rows = self.near.values(feats, need_grad)
+        energies = ops.mol_energy(values, b.atom_types, b.scatter_idxs, b.mol_offsets, b.mol_atom_counts)
+        if self.charge is None:
             if not need_grad:
                 return energies, None
-            gx, gy, gz = ops.featurize_grad(xs, ys, zs, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs, acs,
-                                            *[g.reshape(-1) for g in grads], order=order, size_classes=classes)
+            gx, gy, gz = ops.featurize_grad(*atoms, *rows(), order=order, size_classes=classes)
             return energies, torch.stack((gx, gy, gz), dim=1)
+        values, charge_rows = self.charge.values(feats, need_grad, scaled=True)
+        gather = b.gather_idxs.long()
+        qs = torch.cat(values).index_select(0, gather)
+        if not need_grad:
+            return energies + ops.ani_charge(xs, ys, zs, qs, b.mol_offsets, b.mol_atom_counts), None
+        charge_energies, by_q, qx, qy, qz = ops.ani_charge_all(xs, ys, zs, qs, b.mol_offsets, b.mol_atom_counts,
+                                                               torch.ones_like(energies))
+        by_value = torch.empty_like(by_q).index_copy_(0, gather, by_q).split(acs)
+        gx, gy, gz = ops.featurize_grad(*atoms, *charge_rows(by_value, rows()), order=order, size_classes=classes)
+        return energies + charge_energies, torch.stack((gx + qx, gy + qy, gz + qz), dim=1)
+
+    def _energies_through_autograd(self, b, need_grad):
+        """batch_energies for networks of library operations (other activations than CELU)."""
+        from . import autograd
+        xs, ys, zs = b.xs, b.ys, b.zs
+        acs, order, classes = b.host_counts()
         if need_grad:
             xs, ys, zs = (t.detach().clone().requires_grad_(True) for t in (xs, ys, zs))
         feats = autograd.featurize(xs, ys, zs, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs, acs,
