@@ -10,8 +10,8 @@ multi-threaded gather (csrc/host_batch.c) instead of one numpy operation per mol
 `DeviceFeeder` is what the reference does with a feed dict and a staging queue
 (khan/training/trainer_multi_tower.py:767-792, 291-303), done for one GPU with PyTorch as the memory
 and stream plumbing: it splits a batch into the flat arrays the ops take (xs, ys, zs, atom types,
-molecule indices), copies them through pinned host buffers with asynchronous host-to-device copies on a
-side stream, runs `mol_offsets` and `ani_sort` on the device, and keeps one batch in flight while the
+molecule indices) in one pinned host buffer (csrc/torch_feed.cpp), copies it asynchronously on a side stream,
+runs the batch's preparation (`mol_offsets`, `ani_sort`, `size_order`) on the device, and keeps one batch in flight while the
 caller works on the previous one.
 """
 import ctypes
@@ -19,6 +19,8 @@ import math
 import os
 
 import numpy as np
+
+from . import _native
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 HOST_LIB_PATH = os.path.join(_HERE, "csrc", "libkhan_host.so")
@@ -49,6 +51,15 @@ def _np_ptr(a):
     return ctypes.c_void_p(a.ctypes.data)
 
 
+def _selections(dataset, batch_size, shuffle, rng):
+    rng = np.random.default_rng() if rng is None else rng
+    perm = np.arange(dataset.num_mols(), dtype=np.int64)
+    if shuffle:
+        rng.shuffle(perm)
+    for batch_idx in range(dataset.num_batches(batch_size)):
+        yield perm[batch_idx * batch_size:min((batch_idx + 1) * batch_size, dataset.num_mols())]
+
+
 class RawDataset:
     """Ragged molecules [(n_i, 4) arrays of (type, x, y, z)], optional labels and per-atom gradients."""
 
@@ -74,22 +85,26 @@ class RawDataset:
         [-fuzz, fuzz] to the coordinates (dataset.py:166-169).  `rng` is a numpy Generator (the reference
         draws from numpy's global state)."""
         rng = np.random.default_rng() if rng is None else rng
-        perm = np.arange(self.num_mols())
-        if shuffle:
-            rng.shuffle(perm)
-        for batch_idx in range(self.num_batches(batch_size)):
-            sel = perm[batch_idx * batch_size:min((batch_idx + 1) * batch_size, self.num_mols())]
-            mols = [np.asarray(self.all_Xs[p]) for p in sel]
-            mol_ids = np.repeat(np.arange(len(sel), dtype=np.int32), [len(m) for m in mols])
-            mol_Xs = np.concatenate(mols, axis=0) if mols else np.zeros((0, 4))
-            if fuzz is not None:
-                mol_Xs = mol_Xs.copy()
-                mol_Xs[:, 1:4] += rng.uniform(-fuzz, fuzz, (mol_Xs.shape[0], 3))
-            mol_yts = None if self.all_ys is None else [self.all_ys[p] for p in sel]
-            mol_grads = None
-            if self.all_grads is not None:
-                mol_grads = np.concatenate([np.asarray(self.all_grads[p]) for p in sel], axis=0)
-            yield mol_Xs, mol_ids, mol_yts, mol_grads
+        for sel in self.selections(batch_size, shuffle, rng):
+            yield self.batch(sel, fuzz, rng)
+
+    def selections(self, batch_size, shuffle, rng=None):
+        """The molecule indices of every batch, in order (the last batch is not padded)."""
+        return _selections(self, batch_size, shuffle, rng)
+
+    def batch(self, sel, fuzz=None, rng=None):
+        """The tuple of `iterate` for the molecules `sel`."""
+        mols = [np.asarray(self.all_Xs[p]) for p in sel]
+        mol_ids = np.repeat(np.arange(len(sel), dtype=np.int32), [len(m) for m in mols])
+        mol_Xs = np.concatenate(mols, axis=0) if mols else np.zeros((0, 4))
+        if fuzz is not None:
+            mol_Xs = mol_Xs.copy()
+            mol_Xs[:, 1:4] += rng.uniform(-fuzz, fuzz, (mol_Xs.shape[0], 3))
+        mol_yts = None if self.all_ys is None else [self.all_ys[p] for p in sel]
+        mol_grads = None
+        if self.all_grads is not None:
+            mol_grads = np.concatenate([np.asarray(self.all_grads[p]) for p in sel], axis=0)
+        return mol_Xs, mol_ids, mol_yts, mol_grads
 
 
 class PackedDataset:
@@ -162,12 +177,7 @@ class PackedDataset:
 
     def selections(self, batch_size, shuffle, rng=None):
         """The molecule indices of every batch, in order (the last batch is not padded)."""
-        rng = np.random.default_rng() if rng is None else rng
-        perm = np.arange(self.num_mols(), dtype=np.int64)
-        if shuffle:
-            rng.shuffle(perm)
-        for batch_idx in range(self.num_batches(batch_size)):
-            yield perm[batch_idx * batch_size:min((batch_idx + 1) * batch_size, self.num_mols())]
+        return _selections(self, batch_size, shuffle, rng)
 
     def iterate(self, batch_size, shuffle, fuzz=None, rng=None):
         """Same tuples as RawDataset.iterate: (mol_Xs [N,4] float64, mol_ids, mol_yts or None, mol_grads or None)."""
@@ -196,14 +206,26 @@ class DeviceBatch:
     """One batch resident on the GPU, with everything `featurize` needs."""
 
     __slots__ = ("xs", "ys", "zs", "atom_types", "mol_idxs", "n_mols", "mol_atom_counts", "mol_offsets",
-                 "scatter_idxs", "gather_idxs", "atom_counts", "size_order", "counts_pinned", "labels", "grads", "ready")
+                 "scatter_idxs", "gather_idxs", "atom_counts", "size_order", "counts_pinned", "labels", "grads", "ready",
+                 "memory", "sizes", "totals")
+
+    def __init__(self):
+        self.labels = self.grads = self.counts_pinned = None
+        self.memory = self.sizes = self.totals = None    # of a batch from the host: its one buffer, molecule sizes, counts
 
     def host_counts(self):
         """-> (atoms per type [4], the size order on the device, molecules per size class [4] on the host): what the
-        host has to know before it can launch the passes.  The sort writes them to pinned memory; this waits for it."""
+        host has to know before it can launch the passes.  A batch from the host brings them along; otherwise the sort
+        writes them to pinned memory, and this waits for it."""
+        if self.totals is not None:
+            return list(self.totals[0]), self.size_order, list(self.totals[1])
         self.ready.synchronize()
         counts = self.counts_pinned.tolist()
         return counts[0:4], self.size_order, counts[4:8]
+
+    def host_sizes(self):
+        """The molecules' sizes, a list on the host."""
+        return self.mol_atom_counts.tolist() if self.sizes is None else self.sizes
 
     @classmethod
     def from_device_arrays(cls, xs, ys, zs, atom_types, mol_idxs, n_mols):
@@ -213,7 +235,6 @@ class DeviceBatch:
         from . import ops
         b = cls()
         b.xs, b.ys, b.zs, b.atom_types, b.mol_idxs, b.n_mols = xs, ys, zs, atom_types, mol_idxs, n_mols
-        b.labels = b.grads = None
         b.finish_on_current_stream()
         return b
 
@@ -232,40 +253,68 @@ class DeviceBatch:
         import torch
         cur = torch.cuda.current_stream()
         cur.wait_event(self.ready)
+        if self.memory is not None:        # the memory was allocated on the feeder's stream
+            self.memory.record_stream(cur)
+            if self.grads is not None:
+                self.grads.record_stream(cur)
+            return self
         for name in ("xs", "ys", "zs", "atom_types", "mol_idxs", "mol_atom_counts", "mol_offsets", "scatter_idxs",
                      "gather_idxs", "atom_counts", "size_order", "grads"):
             t = getattr(self, name)
             if t is not None:
-                t.record_stream(cur)       # the memory was allocated on the feeder's stream
+                t.record_stream(cur)
         return self
 
 
 class DeviceFeeder:
     """Iterates a RawDataset as DeviceBatch objects, one batch ahead of the consumer.
 
-    Pinned staging buffers are allocated once (for the largest batch seen so far, two sets), copies run on
-    a side stream of default priority, and `mol_offsets` + `ani_sort` are enqueued behind them on the same
-    stream.  The consumer calls `batch.wait()` before using the tensors on its own stream."""
+    Pinned staging buffers are allocated once (for the largest batch seen so far, two sets), a batch goes over in one
+    copy on a side stream of default priority (a single batch, which nothing can overlap with, on the current stream),
+    and its preparation is enqueued behind the copy.  The consumer calls `batch.wait()` before using the tensors on
+    its own stream."""
 
     def __init__(self, dataset, batch_size, shuffle=False, fuzz=None, dtype=np.float32, device="cuda:0", rng=None):
         import torch
         self.dataset, self.batch_size, self.shuffle, self.fuzz = dataset, batch_size, shuffle, fuzz
         self.dtype, self.device, self.rng = dtype, torch.device(device), rng
-        self.stream = torch.cuda.Stream(device=self.device)
+        self.f64 = np.dtype(dtype) == np.float64
+        alone = isinstance(dataset, (RawDataset, PackedDataset)) and dataset.num_batches(batch_size) <= 1
+        self.stream = torch.cuda.current_stream(self.device) if alone else torch.cuda.Stream(device=self.device)
         self._pinned = [None, None]
-        self._events = [None, None]       # consumer-side "done with this staging set" is implied by the H2D event
+        self._events = [None, None]       # the last copy out of a staging set
 
-    def _staging(self, slot, n_atoms):
+    def _staging(self, slot, n_bytes):
         import torch
-        cur = self._pinned[slot]
-        if cur is None or cur["cap"] < n_atoms:
-            cap = max(n_atoms, 1024)
-            tdt = torch.float32 if self.dtype == np.float32 else torch.float64
-            cur = {"cap": cap,
-                   "xyz": torch.empty((3, cap), dtype=tdt, pin_memory=True),
-                   "ints": torch.empty((2, cap), dtype=torch.int32, pin_memory=True)}
-            self._pinned[slot] = cur
-        return cur
+        if self._pinned[slot] is None or self._pinned[slot].numel() < n_bytes:
+            self._pinned[slot] = torch.empty(max(n_bytes, 1 << 16), dtype=torch.uint8, pin_memory=True)
+        return self._pinned[slot]
+
+    def _parts(self, slot, n):
+        """The staging set's arrays for n atoms: xs, ys, zs, types, molecule indices (host tensors)."""
+        native = _native.load()
+        return native.staging_parts(self._staging(slot, native.staging_bytes(n, self.f64)), n, self.f64)
+
+    def _fill_from_raw(self, slot, sel):
+        """Molecule selection of a RawDataset -> staging set, read natively from the molecules' arrays.  None if they are
+        not all contiguous float64 rows: numpy has to make those."""
+        ds, native = self.dataset, _native.load()
+        staged = native.stage_molecules(ds.all_Xs, sel, self._staging(slot, 0), self.f64)
+        if isinstance(staged, int):
+            staged = native.stage_molecules(ds.all_Xs, sel, self._staging(slot, staged), self.f64)
+        if staged is None:
+            return None
+        n, sizes, totals = staged
+        labels = grads = None
+        if ds.all_ys is not None:
+            labels = [ds.all_ys[p] for p in sel.tolist()]
+        else:
+            while sizes and sizes[-1] == 0:         # without labels the last molecule is the last that has atoms
+                sizes.pop()
+                totals = (totals[0], (totals[1][0] - 1,) + totals[1][1:])
+        if ds.all_grads is not None:
+            grads = np.concatenate([np.asarray(ds.all_grads[p]) for p in sel.tolist()], axis=0)
+        return n, len(sizes), labels, grads, sizes, totals
 
     def _fill_from_tuple(self, slot, item):
         """Reference-style tuple -> staging set; returns (n atoms, n molecules, labels, gradients)."""
@@ -277,54 +326,49 @@ class DeviceFeeder:
         n_mols = len(mol_yts) if mol_yts is not None else (int(mids[-1]) + 1 if n else 0)
         if n and int(mids[-1]) >= n_mols:
             raise ValueError("mol_ids names molecule %d but the batch has %d labels" % (int(mids[-1]), n_mols))
-        st = self._staging(slot, n)
-        if self._events[slot] is not None:
-            self._events[slot].synchronize()          # the previous copy out of this staging set has finished
-        st["xyz"][0, :n] = torch.from_numpy(xs)
-        st["xyz"][1, :n] = torch.from_numpy(ys)
-        st["xyz"][2, :n] = torch.from_numpy(zs)
-        st["ints"][0, :n] = torch.from_numpy(types)
-        st["ints"][1, :n] = torch.from_numpy(mids)
-        return n, n_mols, mol_yts, mol_grads
+        for part, values in zip(self._parts(slot, n), (xs, ys, zs, types, mids)):
+            part.copy_(torch.from_numpy(values))
+        return n, n_mols, mol_yts, mol_grads, None, None
 
     def _fill_from_packed(self, slot, sel):
         """Molecule selection of a PackedDataset -> staging set, gathered natively into the pinned buffers."""
         ds = self.dataset
         sel, out_off, n = ds.batch_atoms(sel)
-        st = self._staging(slot, n)
-        if self._events[slot] is not None:
-            self._events[slot].synchronize()
-        xyz, ints = st["xyz"].numpy(), st["ints"].numpy()
-        ds.gather_into(sel, out_off, xyz[0], xyz[1], xyz[2], ints[0], ints[1])
+        xs, ys, zs, types, mids = (part.numpy() for part in self._parts(slot, n))
+        ds.gather_into(sel, out_off, xs, ys, zs, types, mids)
         if self.fuzz is not None:
             rng = np.random.default_rng() if self.rng is None else self.rng
-            xyz[:, :n] += rng.uniform(-self.fuzz, self.fuzz, (3, n)).astype(xyz.dtype)
+            for part, noise in zip((xs, ys, zs), rng.uniform(-self.fuzz, self.fuzz, (3, n)).astype(xs.dtype)):
+                part += noise
         labels = None if ds.ys is None else ds.ys[sel]            # an array here (a list from a RawDataset)
         grads = None if ds.grads is None else ds.gather_grads(sel, out_off)
-        return n, sel.size, labels, grads
+        totals = _native.load().staged_totals(self._pinned[slot], n, out_off, self.f64)
+        return n, sel.size, labels, grads, np.diff(out_off).tolist(), totals
 
     def _enqueue(self, slot, item):
         import torch
-        from . import ops
+        if self._events[slot] is not None:
+            self._events[slot].synchronize()          # the previous copy out of this staging set has finished
         if isinstance(self.dataset, PackedDataset):
-            n, n_mols, mol_yts, mol_grads = self._fill_from_packed(slot, item)
+            filled = self._fill_from_packed(slot, item)
+        elif isinstance(item, np.ndarray):
+            filled = self._fill_from_raw(slot, item)
+            if filled is None:
+                filled = self._fill_from_tuple(slot, self.dataset.batch(item))
         else:
-            n, n_mols, mol_yts, mol_grads = self._fill_from_tuple(slot, item)
-        st = self._pinned[slot]
+            filled = self._fill_from_tuple(slot, item)
         b = DeviceBatch()
+        n, b.n_mols, b.labels, mol_grads, b.sizes, b.totals = filled
         with torch.cuda.stream(self.stream):
-            # each row of the staging arrays is contiguous pinned memory: five asynchronous copies
-            b.xs, b.ys, b.zs = (st["xyz"][k, :n].to(self.device, non_blocking=True) for k in range(3))
-            b.atom_types, b.mol_idxs = (st["ints"][k, :n].to(self.device, non_blocking=True) for k in range(2))
-            copied = torch.cuda.Event()
-            copied.record(self.stream)
-            self._events[slot] = copied
-            b.n_mols = n_mols
-            b.labels = mol_yts
-            b.grads = None
+            if b.totals is None:
+                b.counts_pinned = torch.empty(8, dtype=torch.int32, pin_memory=True)
+            (b.memory, b.xs, b.ys, b.zs, b.atom_types, b.mol_idxs, b.mol_atom_counts, b.mol_offsets, b.scatter_idxs, b.gather_idxs,
+             b.atom_counts, b.size_order) = _native.load().feed_batch(self._staging(slot, 0), n, b.n_mols, self.f64, self.device,
+                                                                      b.counts_pinned)
             if mol_grads is not None:
                 b.grads = torch.from_numpy(np.ascontiguousarray(mol_grads, dtype=self.dtype)).to(self.device)
-            b.finish_on_current_stream()          # the feeder's stream is current here
+            b.ready = self._events[slot] = torch.cuda.Event()
+            b.ready.record()
         return b
 
     def __iter__(self):
@@ -332,6 +376,8 @@ class DeviceFeeder:
             if self.dataset.dtype != np.dtype(self.dtype):
                 raise TypeError("the packed data set holds %s coordinates, the feeder was asked for %s"
                                 % (self.dataset.dtype, np.dtype(self.dtype)))
+            it = self.dataset.selections(self.batch_size, self.shuffle, self.rng)
+        elif type(self.dataset) is RawDataset and self.fuzz is None:
             it = self.dataset.selections(self.batch_size, self.shuffle, self.rng)
         else:
             it = self.dataset.iterate(self.batch_size, self.shuffle, self.fuzz, self.rng)

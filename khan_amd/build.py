@@ -298,7 +298,7 @@ def build_host():
     return out
 
 
-OPS_SOURCES = ("torch_ops.cpp", "torch_autograd.cpp", "torch_common.h", os.path.join(ROOT, "include", "khan_aev.h"))
+OPS_SOURCES = ("torch_ops.cpp", "torch_autograd.cpp", "torch_feed.cpp", "torch_common.h", os.path.join(ROOT, "include", "khan_aev.h"))
 OPS_LIBRARY = os.path.join(CSRC, "_khan_ops.so")
 
 

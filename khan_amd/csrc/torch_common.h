@@ -117,6 +117,10 @@ std::vector<Tensor> run_mol_energy_grad(const Tensor& e_grads, const Tensor& typ
 Counts counts4(const py::object& o, const char* what);
 AevArgs aev_args(const py::object& acs, const c10::optional<Tensor>& order, const py::object& size_classes);
 std::vector<Tensor> buckets(const Tensor& packed, const Counts& acs, int64_t width);
+int64_t prepare_batch_ints(int64_t n, int64_t n_mols);          // int32 elements prepare_batch_into takes for its results and workspace
+std::vector<Tensor> prepare_batch_into(const Tensor& mol_idxs, const Tensor& types, int64_t n_mols, const c10::optional<Tensor>& counts_pinned,
+                                       const Tensor& all);
 void bind_autograd(py::module_& m);
+void bind_feed(py::module_& m);
 
 }  // namespace khan_torch

@@ -46,22 +46,24 @@ Counts counts4(const py::object& o, const char* what)
 
 // ---------------------------------------------------------------------------------------------- preparation
 // -> (macs, mos, scatter_idxs, gather_idxs, atom_counts, order), slices of one allocation
-static std::vector<Tensor> prepare_batch(const Tensor& mol_idxs, const Tensor& types, int64_t n_mols, const c10::optional<Tensor>& counts_pinned)
+static int64_t up4(int64_t v) { return (v + 3) & ~int64_t(3); }
+
+static std::array<int64_t, 6> prepared_sizes(int64_t n, int64_t n_mols) { return {n_mols, n_mols, n, n, 4, n_mols + kOrderExtra}; }
+
+int64_t prepare_batch_ints(int64_t n, int64_t n_mols)
 {
-    dev(mol_idxs, at::kInt, "mol_idxs");
-    dev(types, at::kInt, "atomic_numbers");
+    int64_t total = up4(api.khan_prepare_batch_workspace_bytes(n) / 4);
+    for (const int64_t s : prepared_sizes(n, n_mols)) total += up4(s);
+    return total;
+}
+
+std::vector<Tensor> prepare_batch_into(const Tensor& mol_idxs, const Tensor& types, int64_t n_mols, const c10::optional<Tensor>& counts_pinned,
+                                       const Tensor& all)
+{
     const int64_t n = types.numel();
-    same_size(mol_idxs.numel() == n, "mol_idxs and atomic_numbers must have the same length");
-    same_size(n_mols >= 0, "n_mols must not be negative");
-    const auto up4 = [](int64_t v) { return (v + 3) & ~int64_t(3); };
-    const int64_t ws = up4(api.khan_prepare_batch_workspace_bytes(n) / 4);
-    const int64_t sizes[6] = {n_mols, n_mols, n, n, 4, n_mols + kOrderExtra};
-    int64_t total = ws;
-    for (const int64_t s : sizes) total += up4(s);
-    const Tensor all = at::empty({total}, types.options());
     std::vector<Tensor> out;
-    int64_t at = ws;
-    for (const int64_t s : sizes) {
+    int64_t at = up4(api.khan_prepare_batch_workspace_bytes(n) / 4);
+    for (const int64_t s : prepared_sizes(n, n_mols)) {
         out.push_back(all.narrow(0, at, s));
         at += up4(s);
     }
@@ -81,6 +83,15 @@ static std::vector<Tensor> prepare_batch(const Tensor& mol_idxs, const Tensor& t
          ptr<int32_t>(out[0]), ptr<int32_t>(out[1]), ptr<int32_t>(out[2]), ptr<int32_t>(out[3]), ptr<int32_t>(out[4]),
          ptr<int32_t>(out[5]), static_cast<void*>(all.data_ptr()), host, st);
     return out;
+}
+
+static std::vector<Tensor> prepare_batch(const Tensor& mol_idxs, const Tensor& types, int64_t n_mols, const c10::optional<Tensor>& counts_pinned)
+{
+    dev(mol_idxs, at::kInt, "mol_idxs");
+    dev(types, at::kInt, "atomic_numbers");
+    same_size(mol_idxs.numel() == types.numel(), "mol_idxs and atomic_numbers must have the same length");
+    same_size(n_mols >= 0, "n_mols must not be negative");
+    return prepare_batch_into(mol_idxs, types, n_mols, counts_pinned, at::empty({prepare_batch_ints(types.numel(), n_mols)}, types.options()));
 }
 
 // ---------------------------------------------------------------------------------------------- AEV passes
@@ -392,4 +403,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("mol_energy", &mol_energy);
     m.def("mol_energy_grad", &mol_energy_grad);
     bind_autograd(m);
+    bind_feed(m);
 }

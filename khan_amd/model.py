@@ -261,6 +261,11 @@ class AniModel:
     # --------------------------------------------------------------------------------------- inference
     def batch_energies(self, b, need_grad=False):
         """DeviceBatch -> per-molecule energies [n_mols] (and d energy / d xyz when need_grad)."""
+        energies, parts = self._energies(b, need_grad)
+        return energies, None if parts is None else torch.stack(parts, dim=1)
+
+    def _energies(self, b, need_grad):
+        """DeviceBatch -> (energies [n_mols], the energy's gradient by x, y and z, or None)."""
         if not self.near.layer_launches():
             return self._energies_through_autograd(b, need_grad)
         from . import ops
@@ -275,21 +280,19 @@ class AniModel:
         if self.charge is None:
             if not need_grad:
                 return energies, None
-            gx, gy, gz = ops.featurize_grad(*atoms, *rows(), order=order, size_classes=classes)
-            return energies, torch.stack((gx, gy, gz), dim=1)
+            return energies, ops.featurize_grad(*atoms, *rows(), order=order, size_classes=classes)
         values, charge_rows = self.charge.values(feats, need_grad, scaled=True)
         gather = b.gather_idxs.long()
         qs = torch.cat(values).index_select(0, gather)
         if not need_grad:
             return energies + ops.ani_charge(xs, ys, zs, qs, b.mol_offsets, b.mol_atom_counts), None
-        charge_energies, by_q, qx, qy, qz = ops.ani_charge_all(xs, ys, zs, qs, b.mol_offsets, b.mol_atom_counts,
-                                                               torch.ones_like(energies))
+        charge_energies, by_q, *by_xyz = ops.ani_charge_all(xs, ys, zs, qs, b.mol_offsets, b.mol_atom_counts, torch.ones_like(energies))
         by_value = torch.empty_like(by_q).index_copy_(0, gather, by_q).split(acs)
-        gx, gy, gz = ops.featurize_grad(*atoms, *charge_rows(by_value, rows()), order=order, size_classes=classes)
-        return energies + charge_energies, torch.stack((gx + qx, gy + qy, gz + qz), dim=1)
+        parts = ops.featurize_grad(*atoms, *charge_rows(by_value, rows()), order=order, size_classes=classes)
+        return energies + charge_energies, torch._foreach_add(parts, by_xyz)
 
     def _energies_through_autograd(self, b, need_grad):
-        """batch_energies for networks of library operations (other activations than CELU)."""
+        """_energies for networks of library operations (other activations than CELU)."""
         from . import autograd
         xs, ys, zs = b.xs, b.ys, b.zs
         acs, order, classes = b.host_counts()
@@ -305,30 +308,49 @@ class AniModel:
             energies = energies + autograd.ani_charge(xs, ys, zs, qs.contiguous(), b.mol_offsets, b.mol_atom_counts)
         if not need_grad:
             return energies.detach(), None
-        gx, gy, gz = torch.autograd.grad(energies, (xs, ys, zs), grad_outputs=torch.ones_like(energies))
-        return energies.detach(), torch.stack((gx, gy, gz), dim=1)
+        return energies.detach(), torch.autograd.grad(energies, (xs, ys, zs), grad_outputs=torch.ones_like(energies))
 
     def _feeder(self, dataset, batch_size):
         from .batching import DeviceFeeder
         np_dtype = np.float32 if self.dtype == torch.float32 else np.float64
         return DeviceFeeder(dataset, batch_size, shuffle=False, dtype=np_dtype, device=self.device)
 
+    def _results(self, dataset, batch_size, of_batch):
+        """For every batch of the data set (of_batch(batch) on the host, the batch), copied out asynchronously: the GPU
+        works on the next batch while the caller handles this one."""
+        ahead = None
+        for b in self._feeder(dataset, batch_size):
+            b.wait()
+            out = of_batch(b)
+            host = torch.empty(out.shape, dtype=out.dtype, pin_memory=True)
+            host.copy_(out, non_blocking=True)
+            done = torch.cuda.Event()
+            done.record()
+            if ahead is not None:
+                ahead[1].synchronize()
+                yield ahead[0].numpy(), ahead[2]
+            ahead = host, done, b
+        if ahead is not None:
+            ahead[1].synchronize()
+            yield ahead[0].numpy(), ahead[2]
+
     def predict(self, dataset, batch_size=2048):
         """-> [y0, y1, ...] in the order of the dataset's molecules (trainer_multi_tower.py:655-678)."""
         ys = []
-        for b in self._feeder(dataset, batch_size):
-            b.wait()
-            e, _ = self.batch_energies(b)
-            ys.extend(e.cpu().tolist())
+        for e, _ in self._results(dataset, batch_size, lambda b: self._energies(b, False)[0]):
+            ys.extend(e.tolist())
         return ys
 
     def coordinate_gradients(self, dataset, batch_size=1024):
         """Yields one [n_atoms, 3] array of d energy / d (x, y, z) per molecule (trainer_multi_tower.py:580-615)."""
-        for b in self._feeder(dataset, batch_size):
-            b.wait()
-            _, g = self.batch_energies(b, need_grad=True)
-            g = g.cpu().numpy()
-            mos = b.mol_offsets.cpu().numpy()
-            macs = b.mol_atom_counts.cpu().numpy()
-            for off, cnt in zip(mos, macs):
-                yield g[off:off + cnt]
+        for g, b in self._results(dataset, batch_size, lambda b: self.batch_energies(b, need_grad=True)[1]):
+            yield from _native.load().split_rows(g.copy(), b.host_sizes())       # (g is pinned memory: not to be kept)
+
+    def energies_and_gradients(self, dataset, batch_size=1024):
+        """Yields (energy, [n_atoms, 3] gradient) per molecule from one pass over the data set."""
+        def both(b):
+            energies, parts = self._energies(b, True)
+            return torch.cat((energies,) + tuple(parts))
+        for v, b in self._results(dataset, batch_size, both):
+            g = np.ascontiguousarray(v[b.n_mols:].reshape(3, -1).T)
+            yield from zip(v[:b.n_mols].tolist(), _native.load().split_rows(g, b.host_sizes()))

@@ -55,10 +55,8 @@ def format_response(energy, gradient):
 def handle_request(model, text):
     """One request through `model` (an AniModel): -> response text."""
     X_np = parse_request(text)
-    rd = RawDataset([X_np], [0.0])
-    energy = float(model.predict(rd)[0]) + self_interaction(X_np)
-    gradient = list(model.coordinate_gradients(rd))[0]
-    return format_response(energy, gradient)
+    (energy, gradient), = model.energies_and_gradients(RawDataset([X_np], [0.0]))
+    return format_response(energy + self_interaction(X_np), gradient)
 
 
 # ---------------------------------------------------------------------------- sockets (client_server.py:8-41)

@@ -1,0 +1,53 @@
+"""What the feeder puts on the GPU for molecules held in different forms, against the data set's own batches; and energies and
+gradients from one pass against those from two."""
+import numpy as np
+import pytest
+import torch
+
+from khan_amd import batching, model, ops
+
+pytestmark = pytest.mark.gpu
+
+FORMS = {"rows": lambda m: m, "columns": np.asfortranarray, "single": lambda m: m.astype(np.float32), "lists": lambda m: m.tolist()}
+
+
+def _molecules(sizes, seed=5):
+    rng = np.random.default_rng(seed)
+    return [np.concatenate([rng.integers(0, 4, (n, 1)).astype(np.float64), rng.uniform(0.0, 1.4 * max(n, 1) ** (1 / 3), (n, 3))], axis=1)
+            for n in sizes]
+
+
+@pytest.mark.parametrize("form", sorted(FORMS))
+@pytest.mark.parametrize("labelled", [True, False])
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+def test_feeder_takes_molecules_in_any_form(form, labelled, dtype):
+    sizes = [3, 1, 63, 64, 65, 257, 13, 32, 33, 5, 2]          # the size classes' edges, and the padding of the buffer
+    mols = [FORMS[form](m) for m in _molecules(sizes)]
+    raw = batching.RawDataset(mols, list(range(len(mols))) if labelled else None)
+    for batch_size in (4, 11):
+        feeder = batching.DeviceFeeder(raw, batch_size, dtype=dtype)
+        for b, (rows, ids, labels, _) in zip(feeder, raw.iterate(batch_size, False)):
+            b.wait()
+            want = batching.split_columns(rows, ids, dtype)
+            for got, ref in zip((b.xs, b.ys, b.zs, b.atom_types, b.mol_idxs), want):
+                assert got.cpu().numpy().dtype == ref.dtype and np.array_equal(got.cpu().numpy(), ref)
+            macs, mos = ops.mol_offsets(b.mol_idxs, b.n_mols)
+            assert torch.equal(macs, b.mol_atom_counts) and torch.equal(mos, b.mol_offsets)
+            assert b.labels == labels and b.host_sizes() == macs.tolist()
+            acs, _, classes = b.host_counts()
+            assert acs == np.bincount(want[3], minlength=4).tolist()
+            assert classes == np.histogram(macs.cpu().numpy(), [0, 33, 65, 257, 10 ** 9])[0].tolist()
+
+
+@pytest.mark.parametrize("fit_charges", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_energies_and_gradients_from_one_pass(fit_charges, dtype):
+    m = model.AniModel(dtype=dtype, fit_charges=fit_charges, seed=2)
+    raw = batching.RawDataset(_molecules([9, 1, 13, 40, 70, 3]))
+    energies, gradients = m.predict(raw), list(m.coordinate_gradients(raw, 4))
+    both = list(m.energies_and_gradients(raw, 4))
+    assert len(both) == len(energies) == len(gradients) == 6
+    tol = 1e-5 if dtype == torch.float32 else 1e-12
+    for (e, g), e_ref, g_ref in zip(both, energies, gradients):
+        assert isinstance(e, float) and abs(e - e_ref) <= tol * (1.0 + abs(e_ref))
+        assert g.shape == g_ref.shape and g.dtype == g_ref.dtype and np.abs(g - g_ref).max() <= tol * (1.0 + np.abs(g_ref).max())
