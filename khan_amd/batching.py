@@ -52,10 +52,9 @@ def _np_ptr(a):
 
 
 def _selections(dataset, batch_size, shuffle, rng):
-    rng = np.random.default_rng() if rng is None else rng
     perm = np.arange(dataset.num_mols(), dtype=np.int64)
     if shuffle:
-        rng.shuffle(perm)
+        (np.random.default_rng() if rng is None else rng).shuffle(perm)
     for batch_idx in range(dataset.num_batches(batch_size)):
         yield perm[batch_idx * batch_size:min((batch_idx + 1) * batch_size, dataset.num_mols())]
 
@@ -248,10 +247,10 @@ class DeviceBatch:
         self.ready = torch.cuda.Event()
         self.ready.record()
 
-    def wait(self):
-        """Makes the current stream wait for the copies and the sort of this batch."""
+    def wait(self, stream=None):
+        """Makes the current stream (`stream`, if the caller has it at hand) wait for the copies and the sort of this batch."""
         import torch
-        cur = torch.cuda.current_stream()
+        cur = torch.cuda.current_stream() if stream is None else stream
         cur.wait_event(self.ready)
         if self.memory is not None:        # the memory was allocated on the feeder's stream
             self.memory.record_stream(cur)
@@ -281,6 +280,7 @@ class DeviceFeeder:
         self.f64 = np.dtype(dtype) == np.float64
         alone = isinstance(dataset, (RawDataset, PackedDataset)) and dataset.num_batches(batch_size) <= 1
         self.stream = torch.cuda.current_stream(self.device) if alone else torch.cuda.Stream(device=self.device)
+        self._stream_id = (self.stream.stream_id, self.stream.device_index, self.stream.device_type)
         self._pinned = [None, None]
         self._events = [None, None]       # the last copy out of a staging set
 
@@ -359,16 +359,16 @@ class DeviceFeeder:
             filled = self._fill_from_tuple(slot, item)
         b = DeviceBatch()
         n, b.n_mols, b.labels, mol_grads, b.sizes, b.totals = filled
-        with torch.cuda.stream(self.stream):
-            if b.totals is None:
-                b.counts_pinned = torch.empty(8, dtype=torch.int32, pin_memory=True)
-            (b.memory, b.xs, b.ys, b.zs, b.atom_types, b.mol_idxs, b.mol_atom_counts, b.mol_offsets, b.scatter_idxs, b.gather_idxs,
-             b.atom_counts, b.size_order) = _native.load().feed_batch(self._staging(slot, 0), n, b.n_mols, self.f64, self.device,
-                                                                      b.counts_pinned)
-            if mol_grads is not None:
+        if b.totals is None:
+            b.counts_pinned = torch.empty(8, dtype=torch.int32, pin_memory=True)
+        (b.memory, b.xs, b.ys, b.zs, b.atom_types, b.mol_idxs, b.mol_atom_counts, b.mol_offsets, b.scatter_idxs, b.gather_idxs,
+         b.atom_counts, b.size_order) = _native.load().feed_batch(self._staging(slot, 0), n, b.n_mols, self.f64, self.device,
+                                                                  b.counts_pinned, self._stream_id)
+        if mol_grads is not None:
+            with torch.cuda.stream(self.stream):
                 b.grads = torch.from_numpy(np.ascontiguousarray(mol_grads, dtype=self.dtype)).to(self.device)
-            b.ready = self._events[slot] = torch.cuda.Event()
-            b.ready.record()
+        b.ready = self._events[slot] = torch.cuda.Event()
+        b.ready.record(self.stream)
         return b
 
     def __iter__(self):

@@ -363,6 +363,14 @@ struct Pass {
     }
 };
 
+// `all` cut into one part per type, `width` elements to a row
+Four by_type(const Rows& rows, const Tensor& all, int64_t width)
+{
+    Four out;
+    for (int t = 0; t < 4; ++t) out[t] = all.narrow(0, rows.row0[t] * width, rows.n[t] * width);
+    return out;
+}
+
 Four like_values(const Rows& rows, const Tensor& flat)
 {
     return {at::empty({rows.n[0]}, flat.options()), at::empty({rows.n[1]}, flat.options()), at::empty({rows.n[2]}, flat.options()),
@@ -371,10 +379,7 @@ Four like_values(const Rows& rows, const Tensor& flat)
 
 Four like_rows(const Net& net, const Rows& rows, const Tensor& flat)
 {
-    const Tensor all = at::empty({rows.total * net.widths[0]}, flat.options());
-    Four out;
-    for (int t = 0; t < 4; ++t) out[t] = all.narrow(0, rows.row0[t] * net.widths[0], rows.n[t] * net.widths[0]);
-    return out;
+    return by_type(rows, at::empty({rows.total * net.widths[0]}, flat.options()), net.widths[0]);
 }
 
 // The values from library operations, for derivatives of an order the kernels have no form for.
@@ -705,6 +710,146 @@ std::vector<Tensor> network_rows(const Tensor& flat, const std::vector<Tensor>& 
     return {out[0], out[1], out[2], out[3]};
 }
 
+// ---------------------------------------------------------------------------------------------- inference
+// One network of a model: its parameters (constants here) and, where its widths are those of the one-launch kernel, the
+// weights split and packed for it
+struct Weights {
+    Tensor flat, packed;
+    Net net;
+};
+
+// A network's pass over a batch: the values, then the rows' gradients.
+struct Inference {
+    const Weights& w;
+    const Rows rows;
+    const Pass pass;
+    Tensor values;                          // of all rows, type by type
+    variable_list state;                    // activations and d_L; in the one-launch form the rows' gradients
+
+    Inference(const Weights& w_, const Four& x)
+        : w(w_), rows(rows_of(w.net, w.flat, x[0], x[1], x[2], x[3])), pass{w.net, rows, w.flat}, values(at::empty({rows.total}, w.flat.options()))
+    {
+    }
+    bool one_launch() const { return w.packed.defined(); }
+
+    Tensor launch(const Four& scale, bool want_rows)
+    {
+        const Tensor grads = want_rows ? at::empty({rows.total * kFeats}, w.flat.options()) : Tensor();
+        const float *x[4], *bias[12], *head_w[4], *head_b[4], *sc[4];
+        float *value[4], *grad[4];
+        int32_t n[4];
+        for (int t = 0; t < 4; ++t) {
+            x[t] = ptr<float>(rows.x[t]);
+            n[t] = static_cast<int32_t>(rows.n[t]);
+            for (int l = 0; l < 3; ++l) bias[4 * l + t] = reinterpret_cast<const float*>(pass.param(w.net.bias_at(l, t)));
+            head_w[t] = reinterpret_cast<const float*>(pass.param(w.net.weight_at(3, t)));
+            head_b[t] = reinterpret_cast<const float*>(pass.param(w.net.bias_at(3, t)));
+            sc[t] = ptr<float>(scale[t]);
+            value[t] = ptr<float>(values) ? ptr<float>(values) + rows.row0[t] : nullptr;
+            grad[t] = want_rows && ptr<float>(grads) ? ptr<float>(grads) + rows.row0[t] * kFeats : nullptr;
+        }
+        call(api.khan_atomic_networks_f32, x, n, static_cast<const float* const*>(nullptr), static_cast<const float* const*>(nullptr),
+             static_cast<const void*>(w.packed.data_ptr()), bias, head_w, head_b, scale[0].defined() ? sc : static_cast<const float* const*>(nullptr),
+             static_cast<float>(w.net.alpha), value, want_rows ? grad : static_cast<float* const*>(nullptr), pass.st);
+        return grads;
+    }
+    // want_rows: row gradients will be asked for; scaled: with a scale, which is not known yet
+    Four forward(bool want_rows, bool scaled)
+    {
+        const Four v = by_type(rows, values, 1);
+        if (one_launch()) {
+            state = {launch({}, want_rows && !scaled)};
+        } else {
+            state = pass.forward();
+            state.push_back(pass.top(state.back(), &v, want_rows));
+        }
+        return v;
+    }
+    // the rows' gradients times scale (undefined: ones), added to `into` where defined -> [all rows, features]
+    Tensor gradients(const Four& scale, Tensor into)
+    {
+        if (one_launch()) {
+            const Tensor g = scale[0].defined() ? launch(scale, true) : state[0];
+            return into.defined() ? into.add_(g) : g;
+        }
+        const bool add = into.defined();
+        if (!add) into = at::empty({rows.total * w.net.widths[0]}, w.flat.options());
+        const variable_list d = pass.slopes(variable_list(state.begin(), state.end() - 1), state.back());
+        pass.to_rows(d[0], scale, by_type(rows, into, w.net.widths[0]), add);
+        return into;
+    }
+};
+
+Weights weights_of(const py::tuple& t, double alpha)
+{
+    Weights w;
+    w.flat = t[0].cast<Tensor>();
+    if (!t[1].is_none()) w.packed = t[1].cast<Tensor>();
+    w.net = {t[2].cast<Saved>(), alpha};
+    if (w.packed.defined())
+        same_size(w.flat.scalar_type() == at::kFloat && w.net.widths == Saved{kFeats, 128, 128, 64, 1} && w.packed.scalar_type() == at::kByte &&
+                      w.packed.is_cuda() && w.packed.numel() == api.khan_atomic_networks_packed_bytes(),
+                  "packed weights are those of the 384-128-128-64-1 networks in float32");
+    return w;
+}
+
+// A batch's energies and, with need_grad, their gradient by x, y and z: featurize, the networks' values and row gradients, the
+// sums by molecule, the charge energy, featurize_grad.  No graph: the order of the passes is known, and the gradient of
+// the near network's sum needs nothing from behind it.  near, charge: (flat parameters, packed or None, widths).
+// -> (energies,) or (energies, x, y, z); joined: all four are parts of one array, the last element of what is returned, which
+// holds the energies, padded to 64 elements, then the three gradients
+std::vector<Tensor> infer(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos, const Tensor& macs,
+                          const Tensor& sis, const Tensor& gather, const py::object& acs, const c10::optional<Tensor>& order,
+                          const py::object& size_classes, const py::tuple& near, const py::object& charge, double alpha, bool need_grad, bool joined)
+{
+    const at::NoGradGuard no_graph;
+    same_size(need_grad || !joined, "energies alone need no array to be joined in");
+    const Atoms7 in = {xs.detach(), ys.detach(), zs.detach(), as, mos, macs, sis};
+    const AevArgs args = aev_args(acs, order, size_classes);
+    const int64_t n = xs.numel(), m = mos.numel(), from = joined ? (m + 63) / 64 * 64 : 0;
+    const Tensor result = need_grad ? at::empty({from + 3 * n}, xs.options()) : Tensor();
+    std::vector<Tensor> out = {joined ? result.narrow(0, 0, m) : at::empty({m}, xs.options())};
+    if (need_grad)
+        for (int k = 0; k < 3; ++k) out.push_back(result.narrow(0, from + k * n, n));
+    if (joined) out.push_back(result);
+    const auto f = run_featurize(in, args);
+    const Four feats = {f[0], f[1], f[2], f[3]};
+    const Weights near_w = weights_of(near, alpha);
+    Inference near_net(near_w, feats);
+    run_mol_energy(near_net.forward(need_grad, false), as, sis, mos, macs, out[0]);
+    if (charge.is_none()) {
+        if (need_grad) run_featurize_grad(in, args, by_type(near_net.rows, near_net.gradients({}, Tensor()), kFeats), {out[1], out[2], out[3]});
+        return out;
+    }
+    const Weights charge_w = weights_of(charge.cast<py::tuple>(), alpha);
+    Inference charge_net(charge_w, feats);
+    charge_net.forward(need_grad, true);
+    const Tensor qs = charge_net.values.index_select(0, gather);
+    if (!need_grad) {
+        out[0].add_(ani_charge(in[0], in[1], in[2], qs, mos, macs));
+        return out;
+    }
+    const auto c = ani_charge_grads(in[0], in[1], in[2], qs, mos, macs, at::ones({m}, xs.options()), true, true);
+    const Tensor by_value = at::empty_like(qs).index_copy_(0, gather.to(at::kLong), c[1]);
+    const Tensor g = charge_net.gradients(by_type(charge_net.rows, by_value, 1), near_net.gradients({}, Tensor()));
+    run_featurize_grad(in, args, by_type(near_net.rows, g, kFeats), {out[1], out[2], out[3]});
+    out[0].add_(c[0]);
+    result.narrow(0, from, 3 * n).add_(c[2].as_strided({3 * n}, {1}));          // (x, y and z lie end to end)
+    return out;
+}
+
+// What the parameters are, for a caller that keeps something made from them: where each lies and how often it was written,
+// and the stream that what was kept has been made on
+py::bytes parameter_key(const std::vector<Tensor>& params)
+{
+    std::vector<uint64_t> key = {reinterpret_cast<uint64_t>(stream())};
+    for (const Tensor& p : params) {
+        key.push_back(reinterpret_cast<uint64_t>(p.data_ptr()));
+        key.push_back(p._version());
+    }
+    return py::bytes(reinterpret_cast<const char*>(key.data()), key.size() * sizeof(uint64_t));
+}
+
 }  // namespace
 
 void bind_autograd(py::module_& m)
@@ -716,6 +861,8 @@ void bind_autograd(py::module_& m)
     m.def("flatten", &flatten);
     m.def("network_forward", &network_forward);
     m.def("network_rows", &network_rows);
+    m.def("infer", &infer);
+    m.def("parameter_key", &parameter_key);
 }
 
 }  // namespace khan_torch

@@ -26,7 +26,8 @@ using Four = std::array<Tensor, 4>;
     X(khan_featurize_grad_inverse_ordered_f32) X(khan_featurize_grad_inverse_ordered_f64)                              \
     X(khan_ani_charges_f32) X(khan_ani_charges_f64) X(khan_mol_energy_f32) X(khan_mol_energy_f64) X(khan_mol_energy_grad_f32)               \
     X(khan_mol_energy_grad_f64) X(khan_net_layer_f32) X(khan_net_layer_f64) X(khan_net_top_f32) X(khan_net_top_f64)      \
-    X(khan_net_grads_workspace_bytes_f32) X(khan_net_grads_workspace_bytes_f64) X(khan_net_grads_f32) X(khan_net_grads_f64)
+    X(khan_net_grads_workspace_bytes_f32) X(khan_net_grads_workspace_bytes_f64) X(khan_net_grads_f32) X(khan_net_grads_f64) \
+    X(khan_atomic_networks_f32) X(khan_atomic_networks_packed_bytes)
 
 struct Api {
 #define X(name) decltype(&::name) name = nullptr;
@@ -106,12 +107,14 @@ struct AevArgs {
 using Atoms7 = std::array<Tensor, 7>;      // xs, ys, zs, as, mos, macs, sis
 
 std::vector<Tensor> run_featurize(const Atoms7& in, const AevArgs& args);
-std::vector<Tensor> run_featurize_grad(const Atoms7& in, const AevArgs& args, const Four& upstream);
+// (`out`: three vectors to write to, otherwise new ones)
+std::vector<Tensor> run_featurize_grad(const Atoms7& in, const AevArgs& args, const Four& upstream, std::vector<Tensor> out = {});
 std::vector<Tensor> run_featurize_grad_inverse(const Atoms7& in, const AevArgs& args, const std::array<Tensor, 3>& v);
 Tensor ani_charge(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& qs, const Tensor& mos, const Tensor& macs);
 std::vector<Tensor> ani_charge_grads(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& qs, const Tensor& mos, const Tensor& macs,
                                      const Tensor& grads, bool want_xyz, bool energies);
-Tensor run_mol_energy(const Four& type_outputs, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs);
+Tensor run_mol_energy(const Four& type_outputs, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs,
+                      Tensor out = Tensor());
 std::vector<Tensor> run_mol_energy_grad(const Tensor& e_grads, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs,
                                         const Counts& acs);
 Counts counts4(const py::object& o, const char* what);

@@ -5,6 +5,8 @@
 // the GPU's work on the batch.  Here a molecule costs one visit, and the counts are made on the way.
 #include <pybind11/numpy.h>
 
+#include <c10/core/StreamGuard.h>
+
 #include "torch_common.h"
 
 namespace khan_torch {
@@ -125,10 +127,13 @@ std::vector<Tensor> staging_parts(const Tensor& staging, int64_t n, bool f64)
     return {part(s.coord(0), s.w, dt), part(s.coord(1), s.w, dt), part(s.coord(2), s.w, dt), part(s.ints(0), 4, at::kInt), part(s.ints(1), 4, at::kInt)};
 }
 
-// Staging -> GPU in one copy on the current stream, and the batch's preparation behind it
+// Staging -> GPU in one copy on a stream (its id, device and device type), and the batch's preparation behind it
 // -> (the buffer, xs, ys, zs, types, molecule indices, and what prepare_batch returns), all of them parts of the buffer
-std::vector<Tensor> feed_batch(const Tensor& staging, int64_t n, int64_t n_mols, bool f64, const at::Device& device, const c10::optional<Tensor>& counts_pinned)
+std::vector<Tensor> feed_batch(const Tensor& staging, int64_t n, int64_t n_mols, bool f64, const at::Device& device, const c10::optional<Tensor>& counts_pinned,
+                               const std::tuple<int64_t, int64_t, int64_t>& on)
 {
+    const c10::StreamGuard guard(c10::Stream::unpack3(std::get<0>(on), static_cast<c10::DeviceIndex>(std::get<1>(on)),
+                                                      static_cast<c10::DeviceType>(std::get<2>(on))));
     check_staging(staging);
     const Staged s(n, f64);
     same_size(staging.numel() >= s.bytes(), "staging is too small");
@@ -146,21 +151,34 @@ std::vector<Tensor> feed_batch(const Tensor& staging, int64_t n, int64_t n_mols,
     return out;
 }
 
-// rows[0 : sizes[0]], rows[sizes[0] : ...], ...: the molecules' parts of an array, as views of it
-py::list split_rows(const py::array& rows, const py::list& sizes)
+// (x, y, z) [3, atoms] -> the molecules' [atoms, 3] arrays, views of one
+py::list molecule_rows(const py::array& planes, const py::list& sizes)
 {
     const auto& api = py::detail::npy_api::get();
-    const auto* a = py::detail::array_proxy(rows.ptr());
-    same_size(a->nd == 2, "an array of rows");
+    const auto* p = py::detail::array_proxy(planes.ptr());
+    same_size(p->nd == 2 && p->dimensions[0] == 3 && (p->flags & py::detail::npy_api::NPY_ARRAY_C_CONTIGUOUS_), "an array of three rows");
+    const py::ssize_t n = p->dimensions[1], w = planes.itemsize();
+    const py::array rows(planes.dtype(), std::vector<py::ssize_t>{n, 3});
+    const auto transpose = [&](auto zero) {
+        using T = decltype(zero);
+        const T* from = reinterpret_cast<const T*>(p->data);
+        T* to = static_cast<T*>(const_cast<void*>(rows.data()));
+        for (py::ssize_t i = 0; i < n; ++i)
+            for (int k = 0; k < 3; ++k) to[3 * i + k] = from[k * n + i];
+    };
+    same_size(w == 4 || w == 8, "single or double precision");
+    if (w == 4) transpose(float());
+    else transpose(double());
     py::list out(sizes.size());
-    Py_intptr_t shape[2] = {0, a->dimensions[1]}, strides[2] = {a->strides[0], a->strides[1]};
-    char* at = a->data;
-    int64_t left = a->dimensions[0];
+    auto* d = py::detail::array_proxy(rows.ptr());
+    Py_intptr_t shape[2] = {0, 3}, strides[2] = {3 * w, w};
+    char* at = d->data;
+    py::ssize_t left = n;
     for (size_t k = 0; k < sizes.size(); ++k) {
         shape[0] = PyLong_AsLongLong(PyList_GET_ITEM(sizes.ptr(), k));
         same_size(shape[0] >= 0 && shape[0] <= left, "the sizes do not fit the array");
-        Py_INCREF(a->descr);
-        PyObject* v = api.PyArray_NewFromDescr_(api.PyArray_Type_, a->descr, 2, shape, strides, at, py::detail::npy_api::NPY_ARRAY_WRITEABLE_, nullptr);
+        Py_INCREF(d->descr);
+        PyObject* v = api.PyArray_NewFromDescr_(api.PyArray_Type_, d->descr, 2, shape, strides, at, py::detail::npy_api::NPY_ARRAY_WRITEABLE_, nullptr);
         if (!v) throw py::error_already_set();
         PyList_SET_ITEM(out.ptr(), k, v);
         Py_INCREF(rows.ptr());
@@ -180,7 +198,7 @@ void bind_feed(py::module_& m)
     m.def("staging_bytes", &staging_bytes);
     m.def("staging_parts", &staging_parts);
     m.def("feed_batch", &feed_batch);
-    m.def("split_rows", &split_rows);
+    m.def("molecule_rows", &molecule_rows);
 }
 
 }  // namespace khan_torch

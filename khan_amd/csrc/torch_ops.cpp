@@ -196,7 +196,7 @@ void run_backward(Plain plain, Ordered ordered, const Atoms& a, const Tensor& xs
              ptr<T>(o[2]), a.acs.v, st);
 }
 
-std::vector<Tensor> run_featurize_grad(const Atoms7& in, const AevArgs& args, const Four& upstream)
+std::vector<Tensor> run_featurize_grad(const Atoms7& in, const AevArgs& args, const Four& upstream, std::vector<Tensor> out)
 {
     const Atoms a = check_atoms(in, args);
     static const char* const names[4] = {"h_grads", "c_grads", "n_grads", "o_grads"};
@@ -209,7 +209,7 @@ std::vector<Tensor> run_featurize_grad(const Atoms7& in, const AevArgs& args, co
                                   std::to_string(a.acs.v[t] * kFeats));
     }
     const auto& [xs, ys, zs, as, mos, macs, sis] = in;
-    const std::vector<Tensor> out = {at::empty({a.n}, xs.options()), at::empty({a.n}, xs.options()), at::empty({a.n}, xs.options())};
+    if (out.empty()) out = {at::empty({a.n}, xs.options()), at::empty({a.n}, xs.options()), at::empty({a.n}, xs.options())};
     if (a.dt == at::kFloat)
         run_backward<float>(api.khan_featurize_grad_f32, api.khan_featurize_grad_ordered_f32, a, xs, ys, zs, as, mos, macs, sis, g, out);
     else
@@ -328,7 +328,7 @@ std::vector<Tensor> ani_charge_grads(const Tensor& xs, const Tensor& ys, const T
 }
 
 // ---------------------------------------------------------------------------------------------- networks
-Tensor run_mol_energy(const Four& type_outputs, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs)
+Tensor run_mol_energy(const Four& type_outputs, const Tensor& types, const Tensor& sis, const Tensor& mos, const Tensor& macs, Tensor e)
 {
     const auto dt = float_dtype(type_outputs[0], "type_outputs");
     Four o;
@@ -341,7 +341,7 @@ Tensor run_mol_energy(const Four& type_outputs, const Tensor& types, const Tenso
     dev(types, at::kInt, "atom_types"); dev(sis, at::kInt, "sis"); dev(mos, at::kInt, "mos"); dev(macs, at::kInt, "macs");
     same_size(n == types.numel() && sis.numel() == n && mos.numel() == macs.numel(),
               "the four vectors must hold one value per atom, and mos / macs one entry per molecule");
-    const Tensor e = at::empty({macs.numel()}, o[0].options());
+    if (!e.defined()) e = at::empty({macs.numel()}, o[0].options());
     const int32_t m = static_cast<int32_t>(macs.numel());
     const khan_stream_t st = stream();
     auto run = [&](auto zero, auto fn) {

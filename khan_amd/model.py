@@ -171,19 +171,23 @@ class MoleculeNN:
         return (self.first_layer_kernel and self.device.type == "cuda" and self.activation_fn is celu
                 and self.dtype in (torch.float32, torch.float64) and 3 <= len(self.layer_sizes) <= 13)
 
-    def flat_parameters(self, live):
-        """The parameters end to end as those launches take them: for every layer the four types' weights, then for every
-        layer the four types' biases.  `live`: as part of the graph; otherwise kept until a parameter is written again."""
-        ps = [self.params[self.names[t][k][j]] for j in (0, 1) for k in range(len(self.layer_sizes) - 1) for t in TYPE_MAP]
-        native = _native.load()
-        if live:
-            return native.flatten(ps)
-        from . import ops
-        key = [ops._stream()] + [(p.data_ptr(), p._version) for p in ps]
-        if self.__dict__.get("_flat_key") != key:
+    def _in_flat_order(self):
+        """The parameters as the layer launches take them end to end: for every layer the four types' weights, then for every
+        layer the four types' biases."""
+        if "_flat_names" not in self.__dict__:
+            self._flat_names = [self.names[t][k][j] for j in (0, 1) for k in range(len(self.layer_sizes) - 1) for t in TYPE_MAP]
+        return [self.params[name] for name in self._flat_names]
+
+    def constants(self):
+        """-> (the parameters end to end, packed for the one-launch kernel or None, the widths): what inference takes, kept
+        until a parameter is written again (or asked for on another stream, which has not waited for the copies)."""
+        native, ps = _native.load(), self._in_flat_order()
+        key = (native.parameter_key(ps), self.one_launch())
+        kept = self.__dict__.get("_constants")
+        if kept is None or kept[0] != key:
             with torch.no_grad():
-                self._flat, self._flat_key = native.flatten(ps), key
-        return self._flat
+                kept = self._constants = (key, (native.flatten(ps), self.one_launch_operands()[0] if key[1] else None, list(self.layer_sizes)))
+        return kept[1]
 
     def type_outputs(self, atom_type_features):
         """Per-type flat feature buckets -> the four per-type output vectors [acs[t]] (nn.py:165-175)."""
@@ -191,27 +195,9 @@ class MoleculeNN:
             return [self.atom_type_outputs(t, f.reshape(-1, FEATURE_SIZE)) for t, f in enumerate(atom_type_features)]
         # in single precision inference is the default: the weights are constants
         live = torch.is_grad_enabled() and (self.weights_need_grad or self.dtype == torch.float64 or self.kernel_layers() == 0)
-        return _native.load().network_autograd(self.flat_parameters(live), list(atom_type_features), self.layer_sizes, 0.1)
-
-
-    def values(self, feats, want_grad, scaled=False):
-        """The networks on the featurizer's buckets without a graph -> (the four vectors of values, rows), rows(scale, into)
-        the four buckets of scale * d value / d feature row (`scale`: four vectors, or None for ones), added to the buckets
-        `into` where given.  `scaled`: rows will be called with a scale, which is not known yet."""
-        from . import ops
-        feats = list(feats)
-        if self.one_launch():
-            packed, biases, head_w, head_b = self.one_launch_operands()
-            run = lambda scale, grad: ops.atomic_networks(feats, None, biases, head_w, head_b, scales=scale, want_grad=grad, packed=packed)
-            values, grads = run(None, want_grad and not scaled)
-
-            def rows(scale=None, into=None):
-                g = [r.reshape(-1) for r in (run(scale, True)[1] if scaled else grads)]
-                return g if into is None else torch._foreach_add(into, g)
-            return values, rows
-        native, flat = _native.load(), self.flat_parameters(False)
-        out = native.network_forward(flat, feats, self.layer_sizes, 0.1, want_grad)
-        return out[:4], lambda scale=None, into=None: native.network_rows(flat, feats, self.layer_sizes, 0.1, out[4:], scale, into)
+        native = _native.load()
+        flat = native.flatten(self._in_flat_order()) if live else self.constants()[0]
+        return native.network_autograd(flat, list(atom_type_features), self.layer_sizes, 0.1)
 
 
 class AniModel:
@@ -261,35 +247,21 @@ class AniModel:
     # --------------------------------------------------------------------------------------- inference
     def batch_energies(self, b, need_grad=False):
         """DeviceBatch -> per-molecule energies [n_mols] (and d energy / d xyz when need_grad)."""
-        energies, parts = self._energies(b, need_grad)
-        return energies, None if parts is None else torch.stack(parts, dim=1)
+        energies, *parts = self._energies(b, need_grad)
+        return energies, torch.stack(parts, dim=1) if need_grad else None
 
-    def _energies(self, b, need_grad):
-        """DeviceBatch -> (energies [n_mols], the energy's gradient by x, y and z, or None)."""
+    def _energies(self, b, need_grad, joined=False):
+        """DeviceBatch -> [energies [n_mols]] and, with need_grad, the energy's gradient by x, y and z; with `joined` also the
+        one array all of them are parts of: the energies, padded to 64 elements, then the gradient's three parts."""
         if not self.near.layer_launches():
-            return self._energies_through_autograd(b, need_grad)
-        from . import ops
-        xs, ys, zs = b.xs, b.ys, b.zs
+            energies, *parts = self._energies_through_autograd(b, need_grad)
+            if joined:
+                parts.append(torch.cat([energies, energies.new_empty(-b.n_mols % 64)] + parts))
+            return [energies] + parts
         acs, order, classes = b.host_counts()
-        atoms = (xs, ys, zs, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs, acs)
-        feats = ops.featurize(*atoms, order=order, size_classes=classes)
-        # the networks' values and, with need_grad, the gradients by the feature rows; no graph: the order of the passes is
-        # known, and the gradient of the near network's sum needs nothing from behind it
-        values, rows = self.near.values(feats, need_grad)
-        energies = ops.mol_energy(values, b.atom_types, b.scatter_idxs, b.mol_offsets, b.mol_atom_counts)
-        if self.charge is None:
-            if not need_grad:
-                return energies, None
-            return energies, ops.featurize_grad(*atoms, *rows(), order=order, size_classes=classes)
-        values, charge_rows = self.charge.values(feats, need_grad, scaled=True)
-        gather = b.gather_idxs.long()
-        qs = torch.cat(values).index_select(0, gather)
-        if not need_grad:
-            return energies + ops.ani_charge(xs, ys, zs, qs, b.mol_offsets, b.mol_atom_counts), None
-        charge_energies, by_q, *by_xyz = ops.ani_charge_all(xs, ys, zs, qs, b.mol_offsets, b.mol_atom_counts, torch.ones_like(energies))
-        by_value = torch.empty_like(by_q).index_copy_(0, gather, by_q).split(acs)
-        parts = ops.featurize_grad(*atoms, *charge_rows(by_value, rows()), order=order, size_classes=classes)
-        return energies + charge_energies, torch._foreach_add(parts, by_xyz)
+        return _native.load().infer(
+            b.xs, b.ys, b.zs, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs, b.gather_idxs, acs, order, classes,
+            self.near.constants(), None if self.charge is None else self.charge.constants(), 0.1, need_grad, joined)
 
     def _energies_through_autograd(self, b, need_grad):
         """_energies for networks of library operations (other activations than CELU)."""
@@ -307,8 +279,8 @@ class AniModel:
             qs = self.charge.atom_outputs(feats, b.gather_idxs)
             energies = energies + autograd.ani_charge(xs, ys, zs, qs.contiguous(), b.mol_offsets, b.mol_atom_counts)
         if not need_grad:
-            return energies.detach(), None
-        return energies.detach(), torch.autograd.grad(energies, (xs, ys, zs), grad_outputs=torch.ones_like(energies))
+            return [energies.detach()]
+        return [energies.detach(), *torch.autograd.grad(energies, (xs, ys, zs), grad_outputs=torch.ones_like(energies))]
 
     def _feeder(self, dataset, batch_size):
         from .batching import DeviceFeeder
@@ -317,15 +289,16 @@ class AniModel:
 
     def _results(self, dataset, batch_size, of_batch):
         """For every batch of the data set (of_batch(batch) on the host, the batch), copied out asynchronously: the GPU
-        works on the next batch while the caller handles this one."""
+        works on the next batch while the caller handles this one.  The array is good until the next one is asked for."""
         ahead = None
         for b in self._feeder(dataset, batch_size):
-            b.wait()
+            stream = torch.cuda.current_stream(self.device)
+            b.wait(stream)
             out = of_batch(b)
             host = torch.empty(out.shape, dtype=out.dtype, pin_memory=True)
             host.copy_(out, non_blocking=True)
             done = torch.cuda.Event()
-            done.record()
+            done.record(stream)
             if ahead is not None:
                 ahead[1].synchronize()
                 yield ahead[0].numpy(), ahead[2]
@@ -343,14 +316,12 @@ class AniModel:
 
     def coordinate_gradients(self, dataset, batch_size=1024):
         """Yields one [n_atoms, 3] array of d energy / d (x, y, z) per molecule (trainer_multi_tower.py:580-615)."""
-        for g, b in self._results(dataset, batch_size, lambda b: self.batch_energies(b, need_grad=True)[1]):
-            yield from _native.load().split_rows(g.copy(), b.host_sizes())       # (g is pinned memory: not to be kept)
+        of_batch = lambda b: self._energies(b, True, joined=True)[-1][-3 * b.xs.numel():] if b.xs.numel() else b.xs
+        for g, b in self._results(dataset, batch_size, of_batch):
+            yield from _native.load().molecule_rows(g.reshape(3, -1), b.host_sizes())
 
     def energies_and_gradients(self, dataset, batch_size=1024):
         """Yields (energy, [n_atoms, 3] gradient) per molecule from one pass over the data set."""
-        def both(b):
-            energies, parts = self._energies(b, True)
-            return torch.cat((energies,) + tuple(parts))
-        for v, b in self._results(dataset, batch_size, both):
-            g = np.ascontiguousarray(v[b.n_mols:].reshape(3, -1).T)
-            yield from zip(v[:b.n_mols].tolist(), _native.load().split_rows(g, b.host_sizes()))
+        for v, b in self._results(dataset, batch_size, lambda b: self._energies(b, True, joined=True)[-1]):
+            gradient = v[v.size - 3 * b.xs.numel():].reshape(3, -1)
+            yield from zip(v[:b.n_mols].tolist(), _native.load().molecule_rows(gradient, b.host_sizes()))
