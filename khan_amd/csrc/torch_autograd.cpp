@@ -15,6 +15,11 @@ using torch::autograd::Function;
 using torch::autograd::Variable;
 using torch::autograd::variable_list;
 using Saved = std::vector<int64_t>;
+// Inside a node nothing is recorded: its few dozen views and allocations go past autograd's own dispatch, which costs as much
+// again as the work itself (a training step on 1,024 molecules is bound by the host).
+using Unrecorded = at::AutoDispatchBelowADInplaceOrView;
+
+Tensor flat1(const Tensor& t) { return t.dim() == 1 ? t : t.reshape({-1}); }
 
 // ---------------------------------------------------------------------------------------------- AEV passes
 void keep(AutogradContext* ctx, const AevArgs& a)
@@ -54,6 +59,7 @@ struct FeaturizeGradFn : Function<FeaturizeGradFn> {
         const Atoms7 in = {xs, ys, zs, as, mos, macs, sis};
         ctx->save_for_backward(with_order(in, args));
         keep(ctx, args);
+        const Unrecorded quiet;
         return run_featurize_grad(in, args, {h.contiguous(), c.contiguous(), n.contiguous(), o.contiguous()});
     }
     // d / d(upstream rows): the Jacobian applied to the incoming vectors; no second derivative by the coordinates, as in
@@ -74,6 +80,7 @@ struct FeaturizeFn : Function<FeaturizeFn> {
     static variable_list forward(AutogradContext* ctx, const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos,
                                  const Tensor& macs, const Tensor& sis, const AevArgs& args)
     {
+        const Unrecorded quiet;
         const Atoms7 in = {xs, ys, zs, as, mos, macs, sis};
         ctx->save_for_backward(with_order(in, args));
         keep(ctx, args);
@@ -134,6 +141,7 @@ struct MolEnergyFn : Function<MolEnergyFn> {
         std::vector<Saved> shapes;
         for (const Tensor* o : {&o0, &o1, &o2, &o3}) shapes.push_back(o->sizes().vec());
         ctx->saved_data["shapes"] = shapes;
+        const Unrecorded quiet;
         return run_mol_energy({o0, o1, o2, o3}, types, sis, mos, macs);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g);
@@ -147,6 +155,7 @@ struct MolEnergyGradFn : Function<MolEnergyGradFn> {
         ctx->saved_data["double"] = ge.scalar_type() == at::kDouble;
         Counts c{};
         for (int t = 0; t < 4; ++t) c.v[t] = static_cast<int32_t>(counts[t]);
+        const Unrecorded quiet;
         return run_mol_energy_grad(ge.contiguous(), types, sis, mos, macs, c);
     }
     static variable_list backward(AutogradContext* ctx, variable_list g)
@@ -165,7 +174,10 @@ variable_list MolEnergyFn::backward(AutogradContext* ctx, variable_list g)
     auto d = MolEnergyGradFn::apply(s[0], s[1], s[2], s[3], ctx->saved_data["counts"].toIntVector(), g[0]);
     variable_list out(8);
     const auto shapes = ctx->saved_data["shapes"].toList();
-    for (int t = 0; t < 4; ++t) out[4 + t] = d[t].reshape(static_cast<c10::IValue>(shapes.get(t)).toIntVector());
+    for (int t = 0; t < 4; ++t) {
+        const auto shape = static_cast<c10::IValue>(shapes.get(t)).toIntVector();
+        out[4 + t] = shape.size() == 1 ? d[t] : d[t].reshape(shape);
+    }
     return out;
 }
 
@@ -213,7 +225,7 @@ Rows rows_of(const Net& net, const Tensor& flat, const Tensor& h, const Tensor& 
     r.x = {h, c, n, o};
     r.total = 0;
     for (int t = 0; t < 4; ++t) {
-        r.x[t] = r.x[t].detach().reshape({-1});
+        r.x[t] = flat1(r.x[t]);
         dev(r.x[t], dt, "feature rows");
         same_size(r.x[t].numel() % net.widths[0] == 0, "feature rows must be whole rows");
         r.n[t] = r.x[t].numel() / net.widths[0];
@@ -423,7 +435,7 @@ Four or_zeros(const Rows& rows, const Tensor& flat, const variable_list& g, int 
     Four out;
     for (int t = 0; t < 4; ++t) {
         const Tensor& v = g[from + t];
-        out[t] = v.defined() ? v.detach().reshape({-1}).contiguous() : at::zeros({rows.n[t] * width}, flat.options());
+        out[t] = v.defined() ? flat1(v).contiguous() : at::zeros({rows.n[t] * width}, flat.options());
     }
     return out;
 }
@@ -436,6 +448,7 @@ struct NetRowsFn : Function<NetRowsFn> {
                                  const Tensor& s0, const Tensor& s1, const Tensor& s2, const Tensor& s3, const variable_list& kept_acts, Saved widths,
                                  double alpha)
     {
+        const Unrecorded quiet;
         const Net net{widths, alpha};
         const Rows rows = rows_of(net, flat, x0, x1, x2, x3);
         const Pass p{net, rows, flat};
@@ -477,12 +490,13 @@ struct NetRowsFn : Function<NetRowsFn> {
                 if (k == 0 || k > 4 || x[k - 1].requires_grad()) out[k] = g[k];
             return out;
         }
+        const Unrecorded quiet;
         const Rows rows = rows_of(net, flat, x[0], x[1], x[2], x[3]);
         const Pass p{net, rows, flat};
         const int L = p.L;
         const variable_list acts(saved.begin() + 9, saved.begin() + 9 + L), d(saved.begin() + 9 + L, saved.begin() + 9 + 2 * L);
         const Four v = or_zeros(rows, flat, u, 0, net.widths[0]);
-        const Four scale = {s[0].detach().contiguous(), s[1].detach().contiguous(), s[2].detach().contiguous(), s[3].detach().contiguous()};
+        const Four scale = {s[0].contiguous(), s[1].contiguous(), s[2].contiguous(), s[3].contiguous()};
         // the tangents along u
         variable_list dot, second;
         for (int l = 0; l < L; ++l) {
@@ -570,6 +584,7 @@ struct NetFn : Function<NetFn> {
     static variable_list forward(AutogradContext* ctx, const Tensor& flat, const Tensor& x0, const Tensor& x1, const Tensor& x2, const Tensor& x3,
                                  Saved widths, double alpha, bool graph)
     {
+        const Unrecorded quiet;
         const Net net{widths, alpha};
         const Rows rows = rows_of(net, flat, x0, x1, x2, x3);
         const Pass p{net, rows, flat};
@@ -609,6 +624,7 @@ struct NetFn : Function<NetFn> {
             for (int t = 0; t < 4; ++t) out[1 + t] = g[t];
             return out;
         }
+        const Unrecorded quiet;
         const Pass p{net, rows, flat};
         const variable_list acts(saved.begin() + 5, saved.begin() + 5 + p.L);
         const variable_list d = p.slopes(acts, saved[5 + p.L]);
@@ -635,11 +651,12 @@ std::vector<Tensor> network_autograd(const Tensor& flat, const std::vector<Tenso
 struct FlattenFn : Function<FlattenFn> {
     static Tensor forward(AutogradContext* ctx, at::TensorList params)
     {
+        const Unrecorded quiet;
         std::vector<Saved> shapes;
         std::vector<Tensor> flat;
         for (const auto& p : params) {
             shapes.push_back(p.sizes().vec());
-            flat.push_back(p.detach().reshape({-1}));
+            flat.push_back(flat1(p));
         }
         ctx->saved_data["shapes"] = shapes;
         return at::cat(flat);
@@ -649,11 +666,20 @@ struct FlattenFn : Function<FlattenFn> {
         variable_list out;
         const auto shapes = ctx->saved_data["shapes"].toList();
         int64_t at = 0;
-        for (size_t k = 0; k < shapes.size(); ++k) {
-            const auto shape = static_cast<c10::IValue>(shapes.get(k)).toIntVector();
-            const int64_t n = c10::multiply_integers(shape);
-            out.push_back(g[0].defined() ? g[0].narrow(0, at, n).view(shape) : Tensor());
-            at += n;
+        const auto parts = [&](bool strided) {
+            for (size_t k = 0; k < shapes.size(); ++k) {
+                const auto shape = static_cast<c10::IValue>(shapes.get(k)).toIntVector();
+                const int64_t n = c10::multiply_integers(shape);
+                if (strided) out.push_back(g[0].as_strided(shape, c10::contiguous_strides(shape), at));
+                else out.push_back(g[0].narrow(0, at, n).view(shape));
+                at += n;
+            }
+        };
+        if (at::GradMode::is_enabled() || !g[0].is_contiguous() || g[0].storage_offset() != 0) {
+            parts(false);
+        } else {
+            const Unrecorded quiet;
+            parts(true);
         }
         return out;
     }
