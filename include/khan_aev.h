@@ -82,10 +82,10 @@ int khan_ani_sort(const int32_t *atomic_numbers, int64_t n_atoms, int32_t *scatt
 
 /* khan_mol_offsets, khan_ani_sort and khan_size_order of one batch together (no counterpart; what a caller runs once per
  * batch before the passes): macs, mos, scatter_idxs, gather_idxs, atom_counts[4] and order[n_mols + 520] as those give
- * them, in three launches (one for a batch of up to 4,096 atoms and 2,048 molecules).  Allocates nothing: `workspace` is
+ * them, in three launches (one for a batch of up to 16,384 atoms and 2,048 molecules).  Allocates nothing: `workspace` is
  * khan_prepare_batch_workspace_bytes(n_atoms) bytes of device memory, 16-byte aligned.  counts_pinned (or null): eight
  * ints of host memory that the GPU can write (hipHostMalloc), which receive the four atom counts and the four size-class
- * totals (order[-4:]) when the work is done, in place of a copy.  n_mols = 0: nothing is written but atom_counts and the
+ * totals (order[-4:]) in place of a copy, each by one store, at the latest when the work is done.  n_mols = 0: nothing is written but atom_counts and the
  * indices. */
 int64_t khan_prepare_batch_workspace_bytes(int64_t n_atoms);
 int khan_prepare_batch(const int32_t *mol_idxs, const int32_t *atomic_numbers, int64_t n_atoms, int32_t n_mols,

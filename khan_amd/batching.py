@@ -218,8 +218,10 @@ class DeviceBatch:
         writes them to pinned memory, and this waits for it."""
         if self.totals is not None:
             return list(self.totals[0]), self.size_order, list(self.totals[1])
-        self.ready.synchronize()
-        counts = self.counts_pinned.tolist()
+        counts = _native.load().wait_for_counts(self.counts_pinned)
+        if counts is None:
+            self.ready.synchronize()
+            counts = self.counts_pinned.tolist()
         return counts[0:4], self.size_order, counts[4:8]
 
     def host_sizes(self):

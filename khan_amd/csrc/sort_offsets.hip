@@ -15,8 +15,8 @@
 //
 // A batch needs both and the size order at the bottom of this file before its first pass.  Each is a few microseconds of
 // work and was two or three launches (nine in all, 62 us of GPU time for 65,536 organic molecules, 50 us for 1,024, and two
-// copies to the host behind them); launch_prepare does the three together in three launches (24 and 18 us), and in one for
-// a small batch (5 us).
+// copies to the host behind them); launch_prepare does the three together in three launches (24 us for 65,536), and in one for
+// a batch of up to 16,384 atoms (9 us for 1,024 molecules, 5 us for a few hundred).
 #include "khan_internal.h"
 #include "khan_params.h"
 
@@ -363,8 +363,7 @@ __global__ __launch_bounds__(kOrderThreads) void size_hist_kernel(const int32_t*
     if (tid < kSizeBins && hist[tid] > 0) atomicAdd(&ghist[tid], hist[tid]);
 }
 
-// Exclusive prefix sums of total[0 .. kSizeBins) into start (shared arrays; every thread of the workgroup calls it).  The
-// first wavefront takes 64 bins at a time.
+// Exclusive prefix sums of total[0 .. kSizeBins) into start (shared arrays), by the first wavefront, 64 bins at a time
 __device__ __forceinline__ void bin_starts(const int* total, int* start)
 {
     if (threadIdx.x < 64) {
@@ -382,7 +381,6 @@ __device__ __forceinline__ void bin_starts(const int* total, int* start)
             carry += __shfl(x, 63, 64);
         }
     }
-    __syncthreads();
 }
 
 // Molecules of up to 32, of 33..64, of 65..256 and of more atoms (class c), from the starts of the bins (largest sizes
@@ -417,7 +415,8 @@ __global__ __launch_bounds__(kOrderThreads) void size_place_kernel(const int32_t
         bin = size_bin(MACs[m]);
         atomicAdd(&hist[bin], 1);
     }
-    bin_starts(total, start);           // (with a barrier at its end)
+    bin_starts(total, start);
+    __syncthreads();
     // the four totals that tell a host which kernels have work (behind the cursors)
     if (blockIdx.x == 0 && tid < kSizeClasses) {
         const int sum = class_total(tid, start, n_mols);
@@ -438,87 +437,119 @@ __global__ __launch_bounds__(kOrderThreads) void size_place_kernel(const int32_t
 }
 
 // The whole preparation of a small batch in one workgroup: what prep_count, prep_rank and size_place do, with barriers in
-// place of launches.  A thread ranks four consecutive atoms; the four types' counts ride in one 64-bit word, 16 bits each.
-constexpr int kSmallPrepAtoms = 4 * kOrderThreads, kSmallPrepMols = 2 * kOrderThreads;
+// place of launches.  A wavefront ranks 64 kPer consecutive atoms, 64 at a time; where it counts them, the four types'
+// counts ride in one 64-bit word, 16 bits each.  What bounds it is latency: its loads are all in flight at once, and the
+// rest is one compute unit's instruction rate.
+constexpr int kSmallPrepPer = 16;            // most atoms per thread
+constexpr int kSmallPrepAtoms = kSmallPrepPer * kOrderThreads, kSmallPrepMols = 2 * kOrderThreads;
+template <int kPer>
 __global__ __launch_bounds__(kOrderThreads) void prep_small_kernel(const int32_t* __restrict__ A, const int32_t* __restrict__ mol_idxs,
                                                                    int n, int32_t n_mols, int32_t* MACs, int32_t* MOs,
                                                                    int32_t* __restrict__ scatter, int32_t* __restrict__ gather,
                                                                    int32_t* __restrict__ counts4, int32_t* __restrict__ order,
                                                                    int32_t* __restrict__ host8)
 {
-    __shared__ int hist[kSizeBins], start[kSizeBins];
+    __shared__ int hist[kSizeBins], start[kSizeBins], mol_start[kSmallPrepMols + 1];
     __shared__ unsigned long long wave_total[kOrderThreads / 64];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     if (tid < kSizeBins) hist[tid] = 0;
-    int type[4];
-    unsigned long long mine = 0;
+    const int first = wave * 64 * kPer + lane;           // this lane's atoms: first, first + 64, ...
+    int type[kPer];
+    {
+        int id[kPer], prev[kPer];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int g = tid * 4 + k;
-        type[k] = g < n ? fold_type(A[g]) : -1;
-        if (type[k] >= 0) mine += 1ull << (16 * type[k]);
-    }
-    for (int g = tid; g <= n; g += kOrderThreads) mol_bounds(mol_idxs, g, n, n_mols, MOs);
-    unsigned long long incl = mine;
+        for (int k = 0; k < kPer; ++k) {
+            const int g = first + 64 * k;
+            type[k] = g < n ? A[g] : -1;
+            id[k] = g < n ? mol_idxs[g] : 0;
+            prev[k] = g < n && g > 0 ? mol_idxs[g - 1] : -1;
+        }
 #pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const unsigned long long y = __shfl_up(incl, d, 64);
-        if (lane >= d) incl += y;
-    }
-    if (lane == 63) wave_total[wave] = incl;
-    __threadfence_block();
-    __syncthreads();                    // MOs and the wavefronts' totals are complete
-    unsigned long long before = incl - mine, all = 0;
-#pragma unroll
-    for (int w = 0; w < kOrderThreads / 64; ++w) {
-        if (w < wave) before += wave_total[w];
-        all += wave_total[w];
-    }
-    int count[4], base[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-        count[t] = static_cast<int>((all >> (16 * t)) & 0xffffu);
-        base[t] = t == 0 ? 0 : base[t - 1] + count[t - 1];
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const int g = tid * 4 + k, t = type[k];
-        if (t >= 0) {
-            const int rank = static_cast<int>((before >> (16 * t)) & 0xffffu);
-            scatter[g] = rank;
-            gather[g] = (t == 0 ? base[0] : t == 1 ? base[1] : t == 2 ? base[2] : base[3]) + rank;
-            before += 1ull << (16 * t);
+        for (int k = 0; k < kPer; ++k) {
+            const int g = first + 64 * k;
+            if (g < n) {
+                type[k] = fold_type(type[k]);
+                if (id[k] != prev[k]) mol_starts(prev[k], id[k], g, n_mols, mol_start);
+            }
         }
     }
+    if (tid == 0) {
+        mol_bounds(mol_idxs, n, n, n_mols, mol_start);
+        mol_start[n_mols] = n;
+    }
+    unsigned long long mine = 0;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) mine += type[k] >= 0 ? 1ull << (16 * type[k]) : 0ull;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) mine += __shfl_xor(mine, d, 64);
+    if (lane == 0) wave_total[wave] = mine;
+    __syncthreads();                    // the molecules' starts and the wavefronts' totals are complete
     int bin[kSmallPrepMols / kOrderThreads];
 #pragma unroll
     for (int k = 0; k < kSmallPrepMols / kOrderThreads; ++k) {
         const int m = k * kOrderThreads + tid;
         if (m < n_mols) {
-            const int c = ((m + 1 < n_mols) ? MOs[m + 1] : n) - MOs[m];
+            const int at = mol_start[m], c = mol_start[m + 1] - at;
+            MOs[m] = at;
             MACs[m] = c;
             bin[k] = size_bin(c);
             atomicAdd(&hist[bin[k]], 1);
         }
     }
-    __syncthreads();
-    bin_starts(hist, start);
+    unsigned long long before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < kOrderThreads / 64; ++w) {
+        if (w < wave) before += wave_total[w];
+        all += wave_total[w];
+    }
+    int count[4], base[4], running[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        count[t] = static_cast<int>((all >> (16 * t)) & 0xffffu);
+        running[t] = __builtin_amdgcn_readfirstlane(static_cast<int>((before >> (16 * t)) & 0xffffu));
+        base[t] = t == 0 ? 0 : base[t - 1] + count[t - 1];
+    }
+    __syncthreads();                    // the molecules per size are complete
     int32_t* const scratch = order + n_mols;         // the counts, the cursors (as they end), the class totals
+    if (wave == 0) {
+        // what a host waits for comes first: it prepares its next launch while the ranks are still written
+        bin_starts(hist, start);
+        __threadfence_block();
+        if (lane < kSizeClasses) {
+            const int sum = class_total(lane, start, n_mols);
+            const int c = lane == 0 ? count[0] : lane == 1 ? count[1] : lane == 2 ? count[2] : count[3];
+            if (host8) {
+                host8[lane] = c;
+                host8[kSizeClasses + lane] = sum;
+            }
+            scratch[2 * kSizeBins + lane] = sum;
+            counts4[lane] = c;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+        const int g = first + 64 * k;
+        if (wave * 64 * kPer + 64 * k >= n) break;
+        int rank = 0, at = 0;
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const unsigned long long m = wave_ballot(type[k] == t);
+            const int r = running[t] + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(m >> 32),
+                                                                                  __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m), 0u)));
+            rank = type[k] == t ? r : rank;
+            at = type[k] == t ? base[t] + r : at;
+            running[t] += __popcll(m);
+        }
+        if (g < n && type[k] >= 0) {
+            scatter[g] = rank;
+            gather[g] = at;
+        }
+    }
+    __syncthreads();                    // the sizes' first positions are complete
     if (tid < kSizeBins) {
         scratch[tid] = hist[tid];
         scratch[kSizeBins + tid] = hist[tid];
     }
-    if (tid < kSizeClasses) {
-        const int sum = class_total(tid, start, n_mols);
-        const int c = tid == 0 ? count[0] : tid == 1 ? count[1] : tid == 2 ? count[2] : count[3];
-        scratch[2 * kSizeBins + tid] = sum;
-        counts4[tid] = c;
-        if (host8) {
-            host8[tid] = c;
-            host8[kSizeClasses + tid] = sum;
-        }
-    }
-    __syncthreads();
 #pragma unroll
     for (int k = 0; k < kSmallPrepMols / kOrderThreads; ++k) {
         const int m = k * kOrderThreads + tid;
@@ -548,10 +579,12 @@ hipError_t launch_prepare(const int32_t* mol_idxs, const int32_t* A, int64_t n_a
                           int32_t* scatter, int32_t* gather, int32_t* counts4, int32_t* order, int32_t* ws, int32_t* host8,
                           hipStream_t stream)
 {
-    // one workgroup up to 4,096 atoms (four per thread): 5 us, where the three launches take 18
+    // one workgroup up to 16,384 atoms (the reference trainer's batch of 1,024 organic molecules is
+    // 13,000: 9 us, where the three launches take 20 and the gaps between them), 5 us up to 4,096; above, one compute unit is slower
     if (n_atoms <= kSmallPrepAtoms && n_mols <= kSmallPrepMols) {
-        prep_small_kernel<<<dim3(1), dim3(kOrderThreads), 0, stream>>>(A, mol_idxs, static_cast<int>(n_atoms), n_mols, MACs, MOs, scatter,
-                                                                       gather, counts4, order, host8);
+        const auto kernel = n_atoms <= 4 * kOrderThreads ? prep_small_kernel<4> : prep_small_kernel<kSmallPrepPer>;
+        kernel<<<dim3(1), dim3(kOrderThreads), 0, stream>>>(A, mol_idxs, static_cast<int>(n_atoms), n_mols, MACs, MOs, scatter, gather,
+                                                            counts4, order, host8);
         return hipGetLastError();
     }
     const unsigned n_tiles = tiles_of(n_atoms);

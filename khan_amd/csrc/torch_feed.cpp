@@ -30,7 +30,7 @@ struct Staged {
 // four atom counts and the molecules of up to 32, 64, 256 and more atoms, as the preparation on the GPU counts them
 struct Totals {
     int32_t v[8] = {};
-    void atom(int32_t type) { if (type >= 0 && type < 4) ++v[type]; }
+    void atom(int32_t type) { ++v[static_cast<uint32_t>(type) > 3u ? 3 : type]; }
     void molecule(int64_t atoms) { ++v[4 + (atoms > 32) + (atoms > 64) + (atoms > 256)]; }
     py::tuple pair() const { return py::make_tuple(py::make_tuple(v[0], v[1], v[2], v[3]), py::make_tuple(v[4], v[5], v[6], v[7])); }
 };

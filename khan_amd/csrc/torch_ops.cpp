@@ -74,7 +74,7 @@ std::vector<Tensor> prepare_batch_into(const Tensor& mol_idxs, const Tensor& typ
         if (h.scalar_type() != at::kInt || h.numel() != 8 || !h.is_contiguous() || !h.is_pinned())
             throw py::value_error("counts_pinned must hold 8 int32 in pinned memory");
         host = h.data_ptr<int32_t>();
-        if (n_mols == 0) std::fill_n(host, 8, 0);
+        std::fill_n(host, 8, n_mols == 0 ? 0 : -1);               // -1: not written yet (wait_for_counts)
         // the GPU writes to it: not to be handed out again before this work is done, whoever drops the tensor
         at::getHostAllocator(at::kCUDA)->record_event(h.data_ptr(), h.storage().data_ptr().get_context(),
                                                       c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().unwrap());
@@ -82,6 +82,28 @@ std::vector<Tensor> prepare_batch_into(const Tensor& mol_idxs, const Tensor& typ
     call(api.khan_prepare_batch, ptr<const int32_t>(mol_idxs), ptr<const int32_t>(types), n, static_cast<int32_t>(n_mols),
          ptr<int32_t>(out[0]), ptr<int32_t>(out[1]), ptr<int32_t>(out[2]), ptr<int32_t>(out[3]), ptr<int32_t>(out[4]),
          ptr<int32_t>(out[5]), static_cast<void*>(all.data_ptr()), host, st);
+    return out;
+}
+
+// The counts that prepare_batch writes to pinned memory, or None if they have not arrived within about a millisecond.  They
+// are on the host while the kernel that wrote them still ranks atoms, some microseconds before an event behind it.
+static py::object wait_for_counts(const Tensor& counts_pinned)
+{
+    same_size(counts_pinned.scalar_type() == at::kInt && counts_pinned.numel() == 8 && counts_pinned.is_contiguous() && !counts_pinned.is_cuda(),
+              "counts_pinned must hold 8 int32 in host memory");
+    const volatile int32_t* c = counts_pinned.data_ptr<int32_t>();
+    const auto arrived = [&] {
+        for (int k = 0; k < 8; ++k)
+            if (c[k] < 0) return false;
+        return true;
+    };
+    {
+        py::gil_scoped_release release;
+        for (int spin = 0; spin < 20000 && !arrived(); ++spin) __builtin_ia32_pause();
+    }
+    if (!arrived()) return py::none();
+    py::list out(8);
+    for (int k = 0; k < 8; ++k) PyList_SET_ITEM(out.ptr(), k, PyLong_FromLong(c[k]));
     return out;
 }
 
@@ -395,6 +417,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     using namespace khan_torch;
     m.def("init", &init);
     m.def("prepare_batch", &prepare_batch);
+    m.def("wait_for_counts", &wait_for_counts);
     m.def("featurize", &featurize);
     m.def("featurize_grad", &featurize_grad);
     m.def("featurize_grad_inverse", &featurize_grad_inverse);

@@ -60,7 +60,7 @@ def test_molecules_shared_by_several_wavefronts(ops, kind, dtype, most, sizes):
         assert torch.equal(r, rows[:n]) and torch.equal(j, jvp[:n])
         assert float((g - grads[:n]).abs().max()) <= tol * float(grads[:n].abs().max())
 
-@pytest.mark.parametrize("n_atoms,n_mols", [(0, 0), (0, 3), (1, 1), (63, 5), (2047, 100), (2048, 2048), (4096, 2047), (4097, 300), (5000, 1),
+@pytest.mark.parametrize("n_atoms,n_mols", [(0, 0), (0, 3), (1, 1), (63, 5), (2047, 100), (2048, 2048), (4096, 2047), (4097, 300), (5000, 1), (16384, 2048), (16385, 1300),
                                             (100003, 9000), (3000, 2049)])
 def test_batch_preparation_in_one_call(ops, n_atoms, n_mols):
     """prepare_batch against mol_offsets, ani_sort and size_order, around the tile sizes and the line between its two forms."""
