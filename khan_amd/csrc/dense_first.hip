@@ -30,6 +30,7 @@
 #include <cstdlib>
 #include <cstring>
 #include "khan_internal.h"
+#include "split_bf16.h"
 #include "khan_params.h"
 
 namespace khan {
@@ -453,27 +454,11 @@ void dense_pipe_kernel(DenseArgs args, int total_tiles, float alpha, float inv_a
 // chunk's global loads are in flight during the products, and the workgroups that share a CU alternate.
 constexpr int kSplitStride = 40;       // bfloat16 elements between staged rows: 32 + 8
 
-typedef unsigned u2v __attribute__((ext_vector_type(2)));
-typedef unsigned u4v __attribute__((ext_vector_type(4)));
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f2v __attribute__((ext_vector_type(2)));
-
 template <int kTileCols, int kCT>
 struct __align__(16) SplitLds {
     unsigned short a[3][kTileRows][kSplitStride];
     unsigned short b[kCT][3][kTileCols][kSplitStride];
 };
-
-// two floats -> their three bfloat16 parts, each pair packed into one register (first value in the low half)
-__device__ __forceinline__ void split_pair(float x0, float x1, unsigned& p1, unsigned& p2, unsigned& p3)
-{
-    p1 = __builtin_bit_cast(unsigned, __builtin_convertvector(f2v{x0, x1}, bf16x2));
-    const float r0 = x0 - __uint_as_float(p1 << 16), r1 = x1 - __uint_as_float(p1 & 0xffff0000u);
-    p2 = __builtin_bit_cast(unsigned, __builtin_convertvector(f2v{r0, r1}, bf16x2));
-    const float s0 = r0 - __uint_as_float(p2 << 16), s1 = r1 - __uint_as_float(p2 & 0xffff0000u);
-    p3 = __builtin_bit_cast(unsigned, __builtin_convertvector(f2v{s0, s1}, bf16x2));
-}
 
 // kCT: column tiles that one workgroup multiplies at once (1, or all 3 of a 384-wide output: the rows are then staged
 // and split once for the three, a step holds three times the products between its barriers, and one workgroup of eight

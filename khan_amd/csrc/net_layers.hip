@@ -25,11 +25,14 @@
 // the lanes of group g = lane / 16 holding k = g kVec .. g kVec + kVec - 1, and the columns of a tile are
 // kVec (lane % 16) + j, so that weights as they are stored are read 16 bytes along their columns and outputs are stored 16
 // bytes at a time.  Per step a wavefront of the 32-row form loads six kilobytes for 32 matrix instructions (1,024
-// cycles): the matrix pipe binds, at the float32 rate (52,000 rows of the eleven-layer network: 74 TFLOP/s of 153).
+// cycles): the matrix pipe binds, at the float32 rate (52,000 rows of the eleven-layer network: 74 TFLOP/s of 153).  Float32
+// products with enough rows to fill the GPU run on the bfloat16 instructions instead (layer_split_kernel).
 #include <algorithm>
+#include <type_traits>
 
 #include "khan_internal.h"
 #include "net_layers.h"
+#include "split_bf16.h"
 
 namespace khan {
 
@@ -50,23 +53,105 @@ template <> struct MatrixOp<double> {
     static __device__ __forceinline__ int row(int lane, int v) { return (lane >> 4) + 4 * v; }
     static __device__ __forceinline__ double celu(double z, double alpha, double inv) { return z >= 0. ? z : alpha * expm1(z * inv); }
 };
-template <typename T> using Vec = T __attribute__((ext_vector_type(MatrixOp<T>::kVec)));
+template <typename T, int W = MatrixOp<T>::kVec> using Vec = T __attribute__((ext_vector_type(W)));
 
 template <typename T>
 __device__ __forceinline__ T slope(T a, T inv_alpha) { return a >= T(0) ? T(1) : fma(a, inv_alpha, T(1)); }
 
-// kVec values of a row from column c on; kWhole: 16-byte aligned and inside the row; otherwise one by one, zeros past `end`
-template <bool kWhole, typename T>
-__device__ __forceinline__ Vec<T> load(const T* __restrict__ row, int c, int end)
+// W values of a row from column c on; kWhole: aligned to their size and inside the row; otherwise one by one, zeros past `end`
+template <bool kWhole, typename T, int W = MatrixOp<T>::kVec>
+__device__ __forceinline__ Vec<T, W> load(const T* __restrict__ row, int c, int end)
 {
     if constexpr (kWhole) {
-        return *reinterpret_cast<const Vec<T>*>(row + c);
+        return *reinterpret_cast<const Vec<T, W>*>(row + c);
     } else {
-        Vec<T> v;
+        Vec<T, W> v;
 #pragma unroll
-        for (int e = 0; e < MatrixOp<T>::kVec; ++e) v[e] = c + e < end ? row[min(c + e, end - 1)] : T(0);
+        for (int e = 0; e < W; ++e) v[e] = c + e < end ? row[min(c + e, end - 1)] : T(0);
         return v;
     }
+}
+
+// W sums of each of R rows (r, may lie past the end: not stored) from column `cols` on -> the outputs of the product's kind
+// (NetKind); n: rows, N: width.  What the rows need from memory is loaded for all of them before the first is stored: a
+// load behind a store waits for that store, and row by row the sixteen round trips of a wavefront's tile were longer than its
+// products (gradient of 47,000 rows through 256 x 256: 48 -> 40 us).
+template <bool kWhole, int W, int R, typename T>
+__device__ __forceinline__ void finish(const NetLayer<T>& a, int t, const int (&r)[R], int n, int cols, int N, Vec<T, W> (&y)[R])
+{
+    size_t at[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) at[i] = static_cast<size_t>(min(r[i], n - 1)) * N;
+    auto put = [&](T* out, const Vec<T, W> (&v)[R]) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            if (r[i] >= n) continue;
+            if constexpr (kWhole) {
+                *reinterpret_cast<Vec<T, W>*>(out + at[i] + cols) = v[i];
+            } else {
+#pragma unroll
+                for (int e = 0; e < W; ++e)
+                    if (cols + e < N) out[at[i] + cols + e] = v[i][e];
+            }
+        }
+    };
+    auto get = [&](Vec<T, W> (&v)[R], const T* from) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) v[i] = load<kWhole, T, W>(from + at[i], cols, N);
+    };
+    T s[R];
+    if (a.kind >= kNetRows) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) s[i] = T(1);
+        if (a.scale[t]) {
+#pragma unroll
+            for (int i = 0; i < R; ++i) s[i] = a.scale[t][min(r[i], n - 1)];
+        }
+    }
+    if (a.kind == kNetCelu) {
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int j = 0; j < W; ++j) y[i][j] = MatrixOp<T>::celu(y[i][j], a.alpha, a.inv_alpha);
+    } else if (a.kind == kNetRows) {
+#pragma unroll
+        for (int i = 0; i < R; ++i) y[i] *= s[i];
+        if (a.accumulate) {
+            Vec<T, W> before[R];
+            get(before, a.out[t]);          // (a row past the end reads the last one, whose new value it does not use)
+#pragma unroll
+            for (int i = 0; i < R; ++i) y[i] += before[i];
+        }
+    } else {
+        Vec<T, W> h[R];
+        get(h, a.act[t]);
+        if (a.kind == kNetTangent) {
+            Vec<T, W> d[R];
+            get(d, a.d[t]);
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+#pragma unroll
+                for (int j = 0; j < W; ++j) {
+                    const T zd = y[i][j] * s[i];
+                    d[i][j] = h[i][j] >= T(0) ? T(0) : zd * d[i][j] * a.inv_alpha;
+                    y[i][j] = zd * slope(h[i][j], a.inv_alpha);
+                }
+            put(a.out2[t], d);
+        } else {
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+#pragma unroll
+                for (int j = 0; j < W; ++j) y[i][j] *= slope(h[i][j], a.inv_alpha);
+            if (a.kind == kNetSecond) {
+                get(h, a.t[t]);
+#pragma unroll
+                for (int i = 0; i < R; ++i)
+#pragma unroll
+                    for (int j = 0; j < W; ++j) y[i][j] = fma(s[i], h[i][j], y[i][j]);
+            }
+        }
+    }
+    put(a.out[t], y);
 }
 
 // One product for the four types, out = epilogue(in . W) with W [k, n_out] as stored, or (kTrans) in . W^T with W [n_out, k]
@@ -170,64 +255,140 @@ __global__ __launch_bounds__(256) void layer_kernel(const NetLayer<T> a, int tot
     if (cols >= N) return;
     Vec<T> bias = Vec<T>(T(0));
     if (a.bias[t]) bias = load<kWhole>(a.bias[t], cols, N);
-    auto put = [&](T* out, size_t at, Vec<T> y) {
-        if constexpr (kWhole) {
-            *reinterpret_cast<Vec<T>*>(out + at) = y;
-        } else {
-#pragma unroll
-            for (int e = 0; e < V; ++e)
-                if (cols + e < N) out[at + e] = y[e];
-        }
-    };
 #pragma unroll
     for (int i = 0; i < kMI; ++i) {
+        int r[4];
+        Vec<T> y[4];
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-            const int r = row0 + i * 16 + Op::row(lane, v);
-            if (r >= n) continue;
-            const size_t at = static_cast<size_t>(r) * N + cols, base = static_cast<size_t>(r) * N;
-            Vec<T> y;
+            r[v] = row0 + i * 16 + Op::row(lane, v);
 #pragma unroll
-            for (int j = 0; j < V; ++j) y[j] = acc[i][j][v] + bias[j];
-            switch (a.kind) {
-                case kNetCelu:
-#pragma unroll
-                    for (int j = 0; j < V; ++j) y[j] = Op::celu(y[j], a.alpha, a.inv_alpha);
-                    break;
-                case kNetRows: {
-                    const T s = a.scale[t] ? a.scale[t][r] : T(1);
-#pragma unroll
-                    for (int j = 0; j < V; ++j) y[j] *= s;
-                    if (a.accumulate) y += load<kWhole>(a.out[t] + base, cols, N);
-                    break;
-                }
-                case kNetTangent: {
-                    const T s = a.scale[t] ? a.scale[t][r] : T(1);
-                    const Vec<T> h = load<kWhole>(a.act[t] + base, cols, N), d = load<kWhole>(a.d[t] + base, cols, N);
-                    Vec<T> second;
-#pragma unroll
-                    for (int j = 0; j < V; ++j) {
-                        const T zd = y[j] * s;
-                        second[j] = h[j] >= T(0) ? T(0) : zd * d[j] * a.inv_alpha;
-                        y[j] = zd * slope(h[j], a.inv_alpha);
-                    }
-                    put(a.out2[t], at, second);
-                    break;
-                }
-                default: {          // kNetSlope, kNetSecond
-                    const Vec<T> h = load<kWhole>(a.act[t] + base, cols, N);
-#pragma unroll
-                    for (int j = 0; j < V; ++j) y[j] *= slope(h[j], a.inv_alpha);
-                    if (a.kind == kNetSecond) {
-                        const T s = a.scale[t] ? a.scale[t][r] : T(1);
-                        const Vec<T> second = load<kWhole>(a.t[t] + base, cols, N);
-#pragma unroll
-                        for (int j = 0; j < V; ++j) y[j] = fma(s, second[j], y[j]);
-                    }
-                }
-            }
-            put(a.out[t], at, y);
+            for (int j = 0; j < V; ++j) y[v][j] = acc[i][j][v] + bias[j];
         }
+        finish<kWhole, V, 4>(a, t, r, n, cols, N, y);
+    }
+}
+
+// The same product in float32 for many rows and wide layers, on the bfloat16 matrix instructions: every operand is split
+// into three bfloat16 values and the six largest of the nine partial products are accumulated in float32 (the split and
+// what it leaves out: dense_first.hip; infinite operands give NaN there as here).
+// A workgroup forms 128 rows x 32 kNB columns in chunks of 32 k.  A wavefront has 32 rows: its lanes load and split the
+// rows' values themselves, in registers, once per workgroup; the weights go through LDS, split by the workgroup for its
+// four wavefronts, a thread a block of 4 k x kNB columns.  LDS holds [plane][8 k][column] pieces of 16 bytes, column
+// kNB c + j of the tile at place 32 j + c: reads and writes run along consecutive places, or (writes of transposed weights)
+// over the four 8 k, two places apart in the banks: no bank conflicts; and a lane's kNB matrix blocks are neighbouring
+// columns, stored and loaded together.  The next chunk's loads are in flight during a chunk's products, its weights go into
+// the other of two buffers: one barrier per chunk.
+// Per chunk a wavefront issues 48 matrix instructions (1,536 cycles; kNB = 4) and 250 vector ones (1,000), most of them
+// splitting, and the two hide each other only in part: 172 TFLOP/s where the float32 instructions gave 70 (96,000 rows
+// 256 -> 256: 139 -> 73 us; 48,000 rows 73 -> 38; transposed 78 -> 40).
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f4v __attribute__((ext_vector_type(4)));
+constexpr int kWideRows = 128;
+
+template <int kNB, bool kTrans>
+__global__ __launch_bounds__(256, 3) void layer_split_kernel(const NetLayer<float> a, int row_tiles)
+{
+    typedef Vec<float, kNB> vec;
+    constexpr int kCols = 32 * kNB;
+    __shared__ u4v S[2][3][4][kCols + 2];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, half = lane >> 5;
+    // the column tiles of a row tile run side by side on one XCD (workgroup w is on XCD w % 8), whose L2 they share
+    const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
+    const int ct = q % a.col_tiles, tile = q / a.col_tiles * 8 + xcd;
+    if (tile >= row_tiles) return;
+    const int t = (tile >= a.tile_end[0]) + (tile >= a.tile_end[1]) + (tile >= a.tile_end[2]);
+    const int rt = tile - (t == 0 ? 0 : a.tile_end[t - 1]);
+    const int n = a.n[t], K = a.k, N = a.n_out;
+    const int row0 = rt * kWideRows + wave * 32;
+    const float* __restrict__ row = a.in[t] + static_cast<size_t>(min(row0 + l32, n - 1)) * K;
+    const float* __restrict__ w = a.w[t];
+    // this thread's weights: columns kNB wc .. of the tile (past the end: others again, never stored), k 4 wk .. + 3;
+    // neighbouring lanes along the weights' rows in memory
+    const int wc = kTrans ? threadIdx.x >> 3 : threadIdx.x & 31, wk = kTrans ? threadIdx.x & 7 : threadIdx.x >> 5;
+    const int wcol = min(ct * kCols + kNB * wc, N - kNB);
+    const float* __restrict__ wsrc = kTrans ? w + static_cast<size_t>(wcol) * K + 4 * wk : w + static_cast<size_t>(4 * wk) * N + wcol;
+    const size_t wnext = kTrans ? K : N, wstep = kTrans ? 32 : static_cast<size_t>(32) * N;
+
+    f4v av[4];
+    typename std::conditional<kTrans, f4v, vec>::type wv[kTrans ? kNB : 4];
+    auto fetch = [&](int c) {
+#pragma unroll
+        for (int i = 0; i < (kTrans ? kNB : 4); ++i) wv[i] = *reinterpret_cast<const decltype(wv[0] + wv[0])*>(wsrc + c * wstep + i * wnext);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) av[i] = *reinterpret_cast<const f4v*>(row + c * 32 + (i >> 1) * 16 + half * 8 + (i & 1) * 4);
+    };
+    auto stage = [&](int buffer) {
+#pragma unroll
+        for (int j = 0; j < kNB; ++j) {
+            unsigned lo[3], hi[3];
+            if constexpr (kTrans) {
+                split_pair(wv[j][0], wv[j][1], lo[0], lo[1], lo[2]);
+                split_pair(wv[j][2], wv[j][3], hi[0], hi[1], hi[2]);
+            } else {
+                split_pair(wv[0][j], wv[1][j], lo[0], lo[1], lo[2]);
+                split_pair(wv[2][j], wv[3][j], hi[0], hi[1], hi[2]);
+            }
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+                reinterpret_cast<u2v*>(&S[buffer][p][wk >> 1][32 * j + wc])[wk & 1] = u2v{lo[p], hi[p]};
+        }
+    };
+    f32x16 acc[kNB];
+#pragma unroll
+    for (int j = 0; j < kNB; ++j) acc[j] = f32x16(0.f);
+    const int chunks = K / 32;
+    fetch(0);
+    stage(0);
+    for (int c = 0; c < chunks; ++c) {
+        f4v x[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) x[i] = av[i];
+        __syncthreads();              // chunk c is in its buffer, and the reads of the other one are done
+        if (c + 1 < chunks) fetch(c + 1);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            u4v xs[3];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                unsigned p[3];
+                const f4v v = x[2 * s + (e >> 1)];
+                split_pair(v[2 * (e & 1)], v[2 * (e & 1) + 1], p[0], p[1], p[2]);
+                xs[0][e] = p[0], xs[1][e] = p[1], xs[2][e] = p[2];
+            }
+            auto mul = [&](int i, int p) {
+#pragma unroll
+                for (int j = 0; j < kNB; ++j)
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xs[i]),
+                                                                     __builtin_bit_cast(bf16x8, S[c & 1][p][2 * s + half][32 * j + l32]), acc[j], 0, 0, 0);
+            };
+            mul(0, 2);
+            mul(1, 1);
+            mul(0, 1);
+            mul(2, 0);
+            mul(1, 0);
+            mul(0, 0);
+        }
+        if (c + 1 < chunks) stage((c + 1) & 1);
+    }
+    // element v of a block: row 8 (v / 4) + 4 half + v % 4, column kNB l32 + (the block's number)
+    const int cols = ct * kCols + kNB * l32;
+    if (cols >= N) return;
+    vec bias = vec(0.f);
+    if (a.bias[t]) bias = load<true, float, kNB>(a.bias[t], cols, N);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        int r[4];
+        vec y[4];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            r[v] = row0 + 8 * i + 4 * half + v;
+            y[v] = bias;
+#pragma unroll
+            for (int j = 0; j < kNB; ++j) y[v][j] += acc[j][4 * i + v];
+        }
+        finish<true, kNB, 4>(a, t, r, n, cols, N, y);
     }
 }
 
@@ -446,6 +607,17 @@ void launch_layer_kernel(NetLayer<T>& a, bool trans, bool whole, hipStream_t str
     }
 }
 
+template <int kNB>
+void launch_split(NetLayer<float>& a, bool trans, hipStream_t stream)
+{
+    a.col_tiles = (a.n_out + 32 * kNB - 1) / (32 * kNB);
+    int total = 0;
+    for (int t = 0; t < 4; ++t) a.tile_end[t] = total += (a.n[t] + kWideRows - 1) / kWideRows;
+    const dim3 grid(static_cast<unsigned>((total + 7) / 8 * 8 * a.col_tiles));
+    if (trans) layer_split_kernel<kNB, true><<<grid, dim3(256), 0, stream>>>(a, total);
+    else layer_split_kernel<kNB, false><<<grid, dim3(256), 0, stream>>>(a, total);
+}
+
 }  // namespace
 
 template <typename T>
@@ -459,6 +631,18 @@ hipError_t launch_net_layer(NetLayer<T> a, bool trans, hipStream_t stream)
         if (a.n[t] > 0)
             whole = ((reinterpret_cast<uintptr_t>(a.bias[t]) | reinterpret_cast<uintptr_t>(a.act[t]) | reinterpret_cast<uintptr_t>(a.d[t]) |
                       reinterpret_cast<uintptr_t>(a.t[t]) | reinterpret_cast<uintptr_t>(a.out[t]) | reinterpret_cast<uintptr_t>(a.out2[t])) & 15u) == 0;
+    if constexpr (std::is_same<T, float>::value) {
+        // Split products from half a workgroup of 128 x 64 per compute unit on (us, float32 instructions -> split): 3,000 rows
+        // 256 -> 256 9.2 -> 12.1 (96 tiles), 128 -> 384 transposed 12.6 -> 9.0 (144); 12,000 rows 384 -> 128 22.9 -> 16.8
+        // (188), 128 -> 64 5.9 -> 8.5 (94).  128 columns instead of 64 from two such workgroups per compute unit on:
+        // 48,000 rows 256 -> 256 43.9 -> 38.4 (750 tiles), 384 -> 128 35.3 -> 34.4 (375), 12,000 rows 23.7 -> 23.4 (188).
+        const int64_t row_tiles = (rows + kWideRows - 1) / kWideRows;
+        if (whole && a.k % 32 == 0 && a.n_out >= 64 && row_tiles * ((a.n_out + 63) / 64) >= 128) {
+            if (row_tiles * ((a.n_out + 127) / 128) >= 512) launch_split<4>(a, trans, stream);
+            else launch_split<2>(a, trans, stream);
+            return hipGetLastError();
+        }
+    }
     // 32 rows per wavefront where that fills the GPU (1,024 SIMDs) with wavefronts of their own, 16 below, and a workgroup
     // per tile where even those are few
     const int64_t col_tiles = (a.n_out + 16 * V - 1) / (16 * V);

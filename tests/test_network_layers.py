@@ -1,5 +1,7 @@
 """The per-type networks of csrc/net_layers.hip (any widths, CELU) against library layers in float64 on the CPU: values,
 gradients by rows and parameters, and the parameters' gradient of a loss on the row gradients."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -83,3 +85,64 @@ def test_networks_of_any_widths(widths, rows, dtype):
     # which changes a few columns of the gradient
     close(by_flat2, want[3], "parameter gradients of a loss on the row gradients", but=0.02 if dtype == torch.float32 else 0.0)
     close(by_v, want[4], "factor gradients of a loss on the row gradients")
+
+
+
+class _Layer(ctypes.Structure):
+    _fields_ = ([(name, ctypes.c_void_p * 4) for name in ("x", "w", "bias", "act", "d", "t", "scale", "out", "out2")] +
+                [("n", ctypes.c_int32 * 4)] + [(name, ctypes.c_int32) for name in ("k", "n_out", "transposed", "kind", "accumulate")] +
+                [("alpha", ctypes.c_double)])
+
+
+# Float32 layers with split products: 64- and 128-column workgroups (from 128 and 512 tiles of 128 rows on), rows around the
+# 128 of a workgroup, output widths that are no multiple of a tile, one or more chunks of 32 k, every kind of epilogue.
+# What the split leaves out is below 2^-23 |x| |w|, the float32 sums of up to 96 products in 16s stay below 2e-6 of
+# sum |x| |w| (as for the dense layers), and the epilogue adds a few roundings of its own terms (1e-6 of them).
+@pytest.mark.parametrize("rows", [(16300, 127, 0, 1), (33000, 128, 129, 0)])
+@pytest.mark.parametrize("k,n_out", [(32, 64), (64, 132), (96, 384)])
+@pytest.mark.parametrize("transposed", [0, 1])
+def test_split_products(rows, k, n_out, transposed):
+    from khan_amd import _lib
+    lib = _lib.load()
+    print("case:", rows, k, n_out, transposed, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    make = lambda *shape: torch.randn(*shape, device="cuda", generator=gen)
+    x, w, bias = [make(n, k) for n in rows], [make(k, n_out) for _ in rows], [make(n_out) for _ in rows]
+    stored = [(a.t() if transposed else a).contiguous() for a in w]
+    act = [torch.nn.functional.celu(make(n, n_out), ALPHA) for n in rows]
+    d, t = ([make(n, n_out) for n in rows] for _ in range(2))
+    scale = [make(n) for n in rows]
+    for kind, name in enumerate(("celu", "slope", "rows", "tangent", "second")):
+        out, out2 = ([torch.ones(n, n_out, device="cuda") for n in rows] for _ in range(2))
+        a = _Layer(k=k, n_out=n_out, transposed=transposed, kind=kind, accumulate=1, alpha=ALPHA)
+        for i, n in enumerate(rows):
+            a.n[i] = n
+            for field, value in (("x", x), ("w", stored), ("act", act), ("d", d), ("t", t), ("scale", scale), ("out", out), ("out2", out2)):
+                getattr(a, field)[i] = value[i].data_ptr()
+            if name == "celu":
+                a.bias[i] = bias[i].data_ptr()
+        lib.khan_net_layer_f32.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+        assert lib.khan_net_layer_f32(ctypes.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+        for i in range(4):
+            y, size = x[i].double() @ w[i].double(), x[i].abs().double() @ w[i].abs().double()
+            h, s = act[i].double(), scale[i].double()[:, None]
+            slope = torch.where(h >= 0, 1.0, h / ALPHA + 1)
+            want2 = None
+            if name == "celu":
+                want = torch.nn.functional.celu(y + bias[i].double(), ALPHA)
+                bound = 2e-6 * size + 1e-6 * (bias[i].abs().double() + ALPHA)
+            elif name == "slope":
+                want, bound = y * slope, 2e-6 * size
+            elif name == "rows":
+                want, bound = y * s + 1, 2e-6 * size * s.abs() + 1e-6
+            elif name == "tangent":
+                want, bound = y * s * slope, 2e-6 * size * s.abs()
+                want2 = torch.where(h >= 0, 0.0, y * s * d[i].double() / ALPHA)
+                bound2 = 2e-6 * size * s.abs() * d[i].abs().double() / ALPHA
+            else:
+                want, bound = y * slope + s * t[i].double(), 2e-6 * size + 1e-6 * (s * t[i].double()).abs()
+            assert ((out[i].double() - want).abs() <= bound).all(), (name, i)
+            if want2 is not None:
+                assert ((out2[i].double() - want2).abs() <= bound2).all(), (name, i)
+            else:
+                assert (out2[i] == 1).all(), (name, i)
