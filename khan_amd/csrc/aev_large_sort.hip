@@ -1,6 +1,6 @@
 // Sorted copies of the molecules of more than 256 atoms, for the workgroup-per-molecule AEV kernels (aev_large.h).
 // One workgroup per molecule: a counting sort by (cell along a space-filling curve, atom type) that keeps the atoms'
-// order inside a bin, 256 atoms per step, and the box around every 64 consecutive sorted atoms.
+// order inside a bin, and the box around every 64 consecutive sorted atoms.
 #include "aev_large.h"
 #include "khan_params.h"
 
@@ -24,6 +24,8 @@ __device__ __forceinline__ float wave_maxf(float v)
     return v;
 }
 
+constexpr int kListedAtoms = 64;      // of a bin, at most, where atoms are ranked by their bins' lists
+
 template <typename T>
 __global__ __launch_bounds__(256) void large_sort_kernel(
     const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
@@ -39,7 +41,7 @@ __global__ __launch_bounds__(256) void large_sort_kernel(
     __shared__ int wshared[4];                 // how many of them each wavefront holds
     __shared__ __align__(16) int step_key[256];              // keys of the 256 atoms of the current step
     __shared__ float ext[4][6];                // each wavefront's share of the molecule's extent
-    __shared__ int wsum[4];
+    __shared__ int wsum[4], wtop[4];
     __shared__ unsigned long long want[4];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -50,14 +52,18 @@ __global__ __launch_bounds__(256) void large_sort_kernel(
 
         // ---- the molecule's extent, and the cell grid over it
         float lo[3] = {3.0e38f, 3.0e38f, 3.0e38f}, hi[3] = {-3.0e38f, -3.0e38f, -3.0e38f};
-        // (one workgroup walks the whole molecule: eight atoms' loads in flight per thread in this and the next loop)
-#pragma unroll 8
-        for (int j = tid; j < n; j += 256) {
-            const float p[3] = {static_cast<float>(X[off + j]), static_cast<float>(Y[off + j]), static_cast<float>(Z[off + j])};
+        // (one workgroup walks the whole molecule: eight atoms' loads in flight per thread in this and the next loops, past
+        // the end the last atom again, because a load under a condition is waited for on the spot)
+        for (int base = tid; base < n; base += 8 * 256) {
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                lo[k] = fminf(lo[k], p[k]);
-                hi[k] = fmaxf(hi[k], p[k]);
+            for (int u = 0; u < 8; ++u) {
+                const int j = off + min(base + 256 * u, n - 1);
+                const float p[3] = {static_cast<float>(X[j]), static_cast<float>(Y[j]), static_cast<float>(Z[j])};
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    lo[k] = fminf(lo[k], p[k]);
+                    hi[k] = fmaxf(hi[k], p[k]);
+                }
             }
         }
 #pragma unroll
@@ -84,13 +90,27 @@ __global__ __launch_bounds__(256) void large_sort_kernel(
             hi[k] = fmaxf(fmaxf(ext[0][3 + k], ext[1][3 + k]), fmaxf(ext[2][3 + k], ext[3][3 + k]));
             scale[k] = static_cast<float>(g) / fmaxf(hi[k] - lo[k], 1.0e-3f);
         }
-        // (cell, type) of atom j: the cell's index along the space-filling curve, then the type
-        auto key_of = [&](int j) -> int {
-            const float p[3] = {static_cast<float>(X[off + j]), static_cast<float>(Y[off + j]), static_cast<float>(Z[off + j])};
+        // (cell, type) of an atom: the cell's index along the space-filling curve, then the type
+        auto bin_of = [&](T x, T y, T z, int type) -> int {
+            const float p[3] = {static_cast<float>(x), static_cast<float>(y), static_cast<float>(z)};
             int c[3];
 #pragma unroll
             for (int k = 0; k < 3; ++k) c[k] = min(max(static_cast<int>((p[k] - lo[k]) * scale[k]), 0), g - 1);
-            return (spread4(c[0]) | (spread4(c[1]) << 1) | (spread4(c[2]) << 2)) * 4 + fold_type(A[off + j]);
+            return (spread4(c[0]) | (spread4(c[1]) << 1) | (spread4(c[2]) << 2)) * 4 + type;
+        };
+        // body(j, bin) for this thread's atoms j
+        auto for_each_bin = [&](auto&& body) {
+            for (int base = tid; base < n; base += 8 * 256) {
+                int key[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) {
+                    const int j = off + min(base + 256 * u, n - 1);
+                    key[u] = bin_of(X[j], Y[j], Z[j], fold_type(A[j]));
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (base + 256 * u < n) body(base + 256 * u, key[u]);
+            }
         };
 
         // ---- atoms per (cell, type)
@@ -99,13 +119,18 @@ __global__ __launch_bounds__(256) void large_sort_kernel(
             in_step[b] = 0;
         }
         __syncthreads();
-#pragma unroll 8
-        for (int j = tid; j < n; j += 256) atomicAdd(&hist[key_of(j)], 1);
+        for_each_bin([&](int, int key) { atomicAdd(&hist[key], 1); });
         __syncthreads();
         // ---- exclusive prefix sum over the bins: per_thread consecutive bins per thread
         {
-            int local = 0;
-            for (int q = 0; q < per_thread; ++q) local += hist[per_thread * tid + q];
+            int local = 0, top = 0;
+            for (int q = 0; q < per_thread; ++q) {
+                local += hist[per_thread * tid + q];
+                top = max(top, hist[per_thread * tid + q]);
+            }
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) top = max(top, __shfl_xor(top, d, 64));
+            if (lane == 0) wtop[wave] = top;
             int incl = local;
 #pragma unroll
             for (int d = 1; d < 64; d <<= 1) {
@@ -124,91 +149,110 @@ __global__ __launch_bounds__(256) void large_sort_kernel(
         }
         __syncthreads();
 
-        // ---- place the atoms, 256 per step, in index order inside a (cell, type): the result does not depend on timing.
-        // An atom's data are fetched one step ahead, so that the loads run under the previous step's ranking.
+        // ---- place the atoms in index order inside a (cell, type): the result does not depend on timing.
         struct Fetched {
             T x, y, z, vx, vy, vz;
             int type, si;
         };
-        auto fetch = [&](int j) -> Fetched {
+        auto fetch = [&](int j) -> Fetched {                      // (past the end: the last atom)
+            const int at = off + min(j, n - 1);
             Fetched f;
-            f.x = f.y = f.z = f.vx = f.vy = f.vz = T(0);
-            f.type = 0;
-            f.si = 0;
-            if (j < n) {
-                f.x = X[off + j];
-                f.y = Y[off + j];
-                f.z = Z[off + j];
-                f.type = fold_type(A[off + j]);
-                f.si = SIs[off + j];
-                if (sorted.vel) {
-                    f.vx = VX[off + j];
-                    f.vy = VY[off + j];
-                    f.vz = VZ[off + j];
-                }
+            f.x = X[at];
+            f.y = Y[at];
+            f.z = Z[at];
+            f.type = fold_type(A[at]);
+            f.si = SIs[at];
+            f.vx = f.vy = f.vz = T(0);
+            if (sorted.vel) {
+                f.vx = VX[at];
+                f.vy = VY[at];
+                f.vz = VZ[at];
             }
             return f;
         };
-        Fetched next = fetch(tid);
-        for (int base = 0; base < n; base += 256) {
-            const int j = base + tid;
-            const bool have = j < n;
-            const Fetched cur = next;
-            next = fetch(j + 256);
-            int key = -1 - tid;                                    // (no two threads without an atom match)
-            if (have) {
-                const float p[3] = {static_cast<float>(cur.x), static_cast<float>(cur.y), static_cast<float>(cur.z)};
-                int c[3];
+        auto place = [&](int j, int dest, const Fetched& f) {
+            sorted.atom[dest] = Fast<T>::make4(f.x, f.y, f.z, static_cast<T>(f.type));
+            sorted.aux[dest] = make_int2(j, f.si);
+            if (sorted.vel) sorted.vel[dest] = Fast<T>::make4(f.vx, f.vy, f.vz, T(0));
+            if (gX) {
+                gX[off + j] = T(0);
+                gY[off + j] = T(0);
+                gZ[off + j] = T(0);
+            }
+        };
+        if (n <= 4 * kSortCells && max(max(wtop[0], wtop[1]), max(wtop[2], wtop[3])) <= kListedAtoms) {
+            // The atoms' indices are listed by bin in whatever order they come (in LDS, one entry per atom), and an atom's
+            // rank is the number of smaller indices in its bin: three passes over the atoms without a barrier inside,
+            // where steps of 256 need five each.  The lists have room for 16,384 atoms, and a bin's are read by each of
+            // its atoms: for bins of up to 64 (a few in a molecule that fills its extent; 1,024-4,096 atoms: 106 -> 37 us with the boxes below).
+            int* list = in_step;
+            for_each_bin([&](int j, int key) { list[atomicAdd(&hist[key], 1)] = j; });
+            __syncthreads();                        // hist[b] is the end of bin b now
+            for (int base = tid; base < n; base += 4 * 256) {
+                Fetched f[4];
 #pragma unroll
-                for (int k = 0; k < 3; ++k) c[k] = min(max(static_cast<int>((p[k] - lo[k]) * scale[k]), 0), g - 1);
-                key = (spread4(c[0]) | (spread4(c[1]) << 1) | (spread4(c[2]) << 2)) * 4 + cur.type;
+                for (int u = 0; u < 4; ++u) f[u] = fetch(base + 256 * u);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int j = base + 256 * u;
+                    if (j >= n) break;
+                    const int key = bin_of(f[u].x, f[u].y, f[u].z, f[u].type);
+                    const int first = key == 0 ? 0 : hist[key - 1], end = hist[key];
+                    int rank = 0;
+                    for (int q = first; q < end; ++q) rank += list[q] < j;
+                    place(j, off + first + rank, f[u]);
+                }
             }
-            // Rank among the step's atoms of the same bin, by thread.  In a large molecule most atoms are alone in their
-            // bin within a step: the atoms that are not are listed (in thread order) and only they compare keys, with
-            // that list.  When the list is long (small molecules, few bins) every atom compares with the 255 others.
-            step_key[tid] = key;
-            if (have) atomicAdd(&in_step[key], 1);
-            __syncthreads();
-            const bool shares = have && in_step[key] > 1;
-            const unsigned long long smask = wave_ballot(shares);
-            if (lane == 0) wshared[wave] = popc64(smask);
-            __syncthreads();
-            int before = 0, n_shared = 0;
-            for (int w = 0; w < 4; ++w) {
-                before += w < wave ? wshared[w] : 0;
-                n_shared += wshared[w];
-            }
-            if (shares) shared_bin[before + popc64(smask & ((1ull << lane) - 1ull))] = make_int2(key, tid);
-            __syncthreads();
-            int rank = 0;
-            if (n_shared > 48) {
+        } else {
+            // 256 per step; an atom's data are fetched one step ahead, so that the loads run under the previous step's ranking
+            Fetched next = fetch(tid);
+            for (int base = 0; base < n; base += 256) {
+                const int j = base + tid;
+                const bool have = j < n;
+                const Fetched cur = next;
+                next = fetch(j + 256);
+                int key = -1 - tid;                                    // (no two threads without an atom match)
+                if (have) key = bin_of(cur.x, cur.y, cur.z, cur.type);
+                // Rank among the step's atoms of the same bin, by thread.  In a large molecule most atoms are alone in their
+                // bin within a step: the atoms that are not are listed (in thread order) and only they compare keys, with
+                // that list.  When the list is long (small molecules, few bins) every atom compares with the 255 others.
+                step_key[tid] = key;
+                if (have) atomicAdd(&in_step[key], 1);
+                __syncthreads();
+                const bool shares = have && in_step[key] > 1;
+                const unsigned long long smask = wave_ballot(shares);
+                if (lane == 0) wshared[wave] = popc64(smask);
+                __syncthreads();
+                int before = 0, n_shared = 0;
+                for (int w = 0; w < 4; ++w) {
+                    before += w < wave ? wshared[w] : 0;
+                    n_shared += wshared[w];
+                }
+                if (shares) shared_bin[before + popc64(smask & ((1ull << lane) - 1ull))] = make_int2(key, tid);
+                __syncthreads();
+                int rank = 0;
+                if (n_shared > 48) {
 #pragma unroll 8
-                for (int t = 0; t < 256; t += 4) {
-                    const int4 k4 = *reinterpret_cast<const int4*>(&step_key[t]);
-                    rank += (k4.x == key && t < tid) + (k4.y == key && t + 1 < tid) + (k4.z == key && t + 2 < tid) +
-                            (k4.w == key && t + 3 < tid);
+                    for (int t = 0; t < 256; t += 4) {
+                        const int4 k4 = *reinterpret_cast<const int4*>(&step_key[t]);
+                        rank += (k4.x == key && t < tid) + (k4.y == key && t + 1 < tid) + (k4.z == key && t + 2 < tid) +
+                                (k4.w == key && t + 3 < tid);
+                    }
+                } else if (shares) {
+                    for (int q = 0; q < n_shared; ++q) {
+                        const int2 e = shared_bin[q];
+                        rank += (e.x == key && e.y < tid);
+                    }
                 }
-            } else if (shares) {
-                for (int q = 0; q < n_shared; ++q) {
-                    const int2 e = shared_bin[q];
-                    rank += (e.x == key && e.y < tid);
+                const int dest = have ? off + hist[key] + rank : 0;
+                __syncthreads();                    // every thread has read its bin's position and the step's counts
+                if (have) in_step[key] = 0;
+                if (have) {
+                    atomicAdd(&hist[key], 1);
+                    place(j, dest, cur);
                 }
+                __syncthreads();                    // the bins are up to date, the keys may be overwritten
             }
-            const int dest = have ? off + hist[key] + rank : 0;
-            __syncthreads();                    // every thread has read its bin's position and the step's counts
-            if (have) in_step[key] = 0;
-            if (have) {
-                atomicAdd(&hist[key], 1);
-                sorted.atom[dest] = Fast<T>::make4(cur.x, cur.y, cur.z, static_cast<T>(cur.type));
-                sorted.aux[dest] = make_int2(j, cur.si);
-                if (sorted.vel) sorted.vel[dest] = Fast<T>::make4(cur.vx, cur.vy, cur.vz, T(0));
-                if (gX) {
-                    gX[off + j] = T(0);
-                    gY[off + j] = T(0);
-                    gZ[off + j] = T(0);
-                }
-            }
-            __syncthreads();                    // the bins are up to date, the keys may be overwritten
         }
 
         // ---- the box around every 64 consecutive sorted atoms
@@ -216,23 +260,30 @@ __global__ __launch_bounds__(256) void large_sort_kernel(
         __syncthreads();                        // the workgroup's stores to sorted.atom are visible to its loads
         const size_t cb = chunk_base(off, mol);
         const int n_chunks = (n + 63) >> 6;
-        for (int c = wave; c < n_chunks; c += 4) {
-            const int j = 64 * c + lane;
-            float p[3] = {0.0f, 0.0f, 0.0f};
-            const bool have = j < n;
-            if (have) {
-                const typename Fast<T>::vec4 a = sorted.atom[off + j];
-                p[0] = static_cast<float>(a.x);
-                p[1] = static_cast<float>(a.y);
-                p[2] = static_cast<float>(a.z);
-            }
-            float blo[3], bhi[3];
+        // four neighbouring lanes per chunk, sixteen atoms each, their loads in flight together (a wavefront per chunk spent
+        // most of the kernel in its 36 lane exchanges: 4,096 atoms are 64 chunks on four wavefronts, 20 us of 56)
+        for (int c0 = 0; c0 < n_chunks; c0 += 64) {
+            const int c = c0 + (tid >> 2), sub = tid & 3;
+            float blo[3] = {3.0e38f, 3.0e38f, 3.0e38f}, bhi[3] = {-3.0e38f, -3.0e38f, -3.0e38f};
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                blo[k] = wave_min(have ? p[k] : 3.0e38f);
-                bhi[k] = wave_maxf(have ? p[k] : -3.0e38f);
+            for (int i = 0; i < 16; ++i) {
+                // (past the end the last atom again, which is in the last chunk)
+                const typename Fast<T>::vec4 a = sorted.atom[off + min(64 * c + 4 * i + sub, n - 1)];
+                const float p[3] = {static_cast<float>(a.x), static_cast<float>(a.y), static_cast<float>(a.z)};
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    blo[k] = fminf(blo[k], p[k]);
+                    bhi[k] = fmaxf(bhi[k], p[k]);
+                }
             }
-            if (lane == 0) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k)
+#pragma unroll
+                for (int d = 1; d < 4; d <<= 1) {
+                    blo[k] = fminf(blo[k], __shfl_xor(blo[k], d, 64));
+                    bhi[k] = fmaxf(bhi[k], __shfl_xor(bhi[k], d, 64));
+                }
+            if (sub == 0 && c < n_chunks) {
                 sorted.box[2 * (cb + c)] = make_float4(blo[0], blo[1], blo[2], 0.0f);
                 sorted.box[2 * (cb + c) + 1] = make_float4(bhi[0], bhi[1], bhi[2], 0.0f);
             }

@@ -848,6 +848,20 @@ def test_large_molecules_in_every_regime_of_their_sort(ops):
     _check_charges(ops, c)
 
 
+@pytest.mark.parametrize("n,far", [(400, 1.0e3), (1300, 1.0e3), (4099, 0.0), (16385, 0.0)])
+def test_large_molecules_by_their_fullest_bin(ops, n, far):
+    # Atoms are ranked by their bins' lists up to 64 atoms a bin and 16,384 atoms, in steps of 256 beyond.  One atom far away
+    # puts all others into one cell (up to half of them of one type: 200 and 650 atoms in a bin); 4,099 and 16,385 atoms
+    # that fill their extent lie on the two sides of the second line.
+    say("case: one molecule of %d atoms, the last one moved by %g" % (n, far))
+    rng = np.random.default_rng(n)
+    xyz = _jittered_lattice(rng, n, 2.15, 0.5)
+    xyz[-1] += far
+    A = rng.choice(4, n, p=[0.5, 0.3, 0.1, 0.1]).astype(np.int32)
+    xyz = xyz.astype(np.float32).astype(np.float64)
+    check_forward_backward(ops, Case(xyz[:, 0], xyz[:, 1], xyz[:, 2], A, np.zeros(n, dtype=np.int32), 1))
+
+
 @pytest.mark.parametrize("seed", [1, 2, 3])
 def test_random_large_molecules(ops, seed):
     # batches of one to four molecules of up to 3,000 atoms, most of them above 256: cubes, slabs and rods at densities
