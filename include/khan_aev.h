@@ -371,7 +371,8 @@ int khan_atomic_networks_f32(const float *const *rows_host4, const int32_t *n_ho
 /* The per-type networks of any widths with CELU (khan/model/nn.py:38-68), layer by layer, in float32 and float64: forward,
  * gradient, second order (a loss on the gradient) and the weights' gradients; each call is a launch for the four types.
  * csrc/net_layers.hip describes the passes these are the steps of.  Arrays are row-major device memory of the precision
- * in the function's name; an unused pointer is NULL, an empty type's pointers may be NULL. */
+ * in the function's name; an unused pointer is NULL, an empty type's pointers may be NULL.  Float32 products of wide layers
+ * with many rows are formed from operands split into three bfloat16 values: infinite operands give NaN there. */
 #define KHAN_NET_CELU 0      /* out = celu(in . w + bias) */
 #define KHAN_NET_SLOPE 1     /* y celu'(act), celu' taken from the activations act */
 #define KHAN_NET_ROWS 2      /* scale[row] y (scale NULL: y), added to out where accumulate is set */
