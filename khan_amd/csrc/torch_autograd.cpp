@@ -214,13 +214,57 @@ struct Rows {
     int64_t n[4], row0[4], total;
 };
 
-Rows rows_of(const Net& net, const Tensor& flat, const Tensor& h, const Tensor& c, const Tensor& n, const Tensor& o)
+// Where a network's parameters lie: parts of one flat array, or the tensors themselves, read where they are, so that a pass
+// takes the values they have when it runs, whoever wrote them.
+struct Params {
+    std::vector<Tensor> held;             // what the addresses point into
+    std::vector<char*> at;                // for every layer the four types' weights, then for every layer their biases
+    at::TensorOptions options;
+    at::ScalarType dtype;
+
+    Params(const Net& net, const Tensor& flat) : held{flat}, options(flat.options()), dtype(float_dtype(flat, "parameters"))
+    {
+        check_net(net);
+        dev(flat, dtype, "parameters");
+        same_size(flat.numel() == net.size(), "the parameters do not match the network's widths");
+        char* base = static_cast<char*>(flat.data_ptr());
+        const int64_t w = static_cast<int64_t>(c10::elementSize(dtype));
+        for (int l = 0; l < net.layers(); ++l)
+            for (int t = 0; t < 4; ++t) at.push_back(base + net.weight_at(l, t) * w);
+        for (int l = 0; l < net.layers(); ++l)
+            for (int t = 0; t < 4; ++t) at.push_back(base + net.bias_at(l, t) * w);
+    }
+    Params(const Net& net, const std::vector<Tensor>& tensors)
+    {
+        check_net(net);
+        same_size(tensors.size() == 8 * static_cast<size_t>(net.layers()), "a weight and a bias for each layer and type");
+        options = at::TensorOptions().dtype(tensors[0].scalar_type()).device(tensors[0].device());
+        dtype = float_dtype(tensors[0], "parameters");
+        for (size_t k = 0; k < tensors.size(); ++k) {
+            const int l = static_cast<int>(k / 4) % net.layers();
+            const bool weight = k / 4 < static_cast<size_t>(net.layers());
+            const Tensor p = tensors[k].contiguous();
+            if (!p.is_cuda() || p.scalar_type() != dtype) throw py::type_error("the parameters must be CUDA tensors of one type");
+            same_size(p.numel() == (weight ? net.widths[l] * net.widths[l + 1] : net.widths[l + 1]),
+                      "the parameters do not match the network's widths");
+            held.push_back(p);
+            at.push_back(static_cast<char*>(p.data_ptr()));
+        }
+    }
+    char* weight(int l, int t) const { return at[4 * l + t]; }
+    char* bias(int l, int t) const { return at[at.size() / 2 + 4 * l + t]; }
+
+private:
+    static void check_net(const Net& net)
+    {
+        if (net.widths.size() < 3 || net.layers() > KHAN_NET_MAX_LAYERS || net.widths.back() != 1)
+            throw py::value_error("a network of 2 to " + std::to_string(KHAN_NET_MAX_LAYERS) + " layers, the last of width 1");
+    }
+};
+
+Rows rows_of(const Net& net, const Params& params, const Tensor& h, const Tensor& c, const Tensor& n, const Tensor& o)
 {
-    if (net.widths.size() < 3 || net.layers() > KHAN_NET_MAX_LAYERS || net.widths.back() != 1)
-        throw py::value_error("a network of 2 to " + std::to_string(KHAN_NET_MAX_LAYERS) + " layers, the last of width 1");
-    const auto dt = float_dtype(flat, "parameters");
-    dev(flat, dt, "parameters");
-    same_size(flat.numel() == net.size(), "the parameters do not match the network's widths");
+    const auto dt = params.dtype;
     Rows r;
     r.x = {h, c, n, o};
     r.total = 0;
@@ -240,14 +284,13 @@ Rows rows_of(const Net& net, const Tensor& flat, const Tensor& h, const Tensor& 
 struct Pass {
     const Net& net;
     const Rows& rows;
-    const Tensor& flat;
+    const Params& params;
     khan_stream_t st = stream();
-    bool f64 = flat.scalar_type() == at::kDouble;
+    bool f64 = params.dtype == at::kDouble;
     size_t w = f64 ? 8 : 4;
     int L = net.layers() - 1;                 // hidden layers
 
-    Tensor make(int64_t width) const { return at::empty({rows.total, width}, flat.options()); }
-    char* param(int64_t at) const { return static_cast<char*>(flat.data_ptr()) + at * w; }
+    Tensor make(int64_t width) const { return at::empty({rows.total, width}, params.options); }
     char* part(const Tensor& a, int64_t width, int t) const
     {
         return a.defined() && rows.n[t] > 0 ? static_cast<char*>(a.data_ptr()) + rows.row0[t] * width * w : nullptr;
@@ -262,7 +305,7 @@ struct Pass {
         a.alpha = net.alpha;
         for (int t = 0; t < 4; ++t) {
             a.n[t] = static_cast<int32_t>(rows.n[t]);
-            a.w[t] = param(net.weight_at(l, t));
+            a.w[t] = params.weight(l, t);
         }
         return a;
     }
@@ -287,7 +330,7 @@ struct Pass {
         variable_list acts;
         for (int l = 0; l < L; ++l) {
             khan_net_layer a = layer(l, false, KHAN_NET_CELU);
-            for (int t = 0; t < 4; ++t) a.bias[t] = param(net.bias_at(l, t));
+            for (int t = 0; t < 4; ++t) a.bias[t] = params.bias(l, t);
             if (l == 0) set(a.in, rows.x);
             else set(a.in, acts[l - 1], net.widths[l]);
             acts.push_back(make(net.widths[l + 1]));
@@ -307,8 +350,8 @@ struct Pass {
         set(a.out, d, net.widths[L]);
         for (int t = 0; t < 4; ++t) {
             a.n[t] = static_cast<int32_t>(rows.n[t]);
-            a.w[t] = param(net.weight_at(L, t));
-            a.bias[t] = param(net.bias_at(L, t));
+            a.w[t] = params.weight(L, t);
+            a.bias[t] = params.bias(L, t);
             a.value[t] = values ? ptr<char>((*values)[t]) : nullptr;
         }
         run(a);
@@ -355,7 +398,7 @@ struct Pass {
     Tensor run(khan_net_grads& g) const
     {
         const int64_t bytes = (f64 ? api.khan_net_grads_workspace_bytes_f64 : api.khan_net_grads_workspace_bytes_f32)(&g);
-        const Tensor ws = at::empty({bytes}, flat.options().dtype(at::kByte)), out = at::empty_like(flat);
+        const Tensor ws = at::empty({bytes}, params.options.dtype(at::kByte)), out = at::empty({net.size()}, params.options);
         g.workspace = ws.data_ptr();
         g.out = out.data_ptr();
         call(f64 ? api.khan_net_grads_f64 : api.khan_net_grads_f32, &g, st);
@@ -383,15 +426,15 @@ Four by_type(const Rows& rows, const Tensor& all, int64_t width)
     return out;
 }
 
-Four like_values(const Rows& rows, const Tensor& flat)
+Four like_values(const Rows& rows, const Params& params)
 {
-    return {at::empty({rows.n[0]}, flat.options()), at::empty({rows.n[1]}, flat.options()), at::empty({rows.n[2]}, flat.options()),
-            at::empty({rows.n[3]}, flat.options())};
+    return {at::empty({rows.n[0]}, params.options), at::empty({rows.n[1]}, params.options), at::empty({rows.n[2]}, params.options),
+            at::empty({rows.n[3]}, params.options)};
 }
 
-Four like_rows(const Net& net, const Rows& rows, const Tensor& flat)
+Four like_rows(const Net& net, const Rows& rows, const Params& params)
 {
-    return by_type(rows, at::empty({rows.total * net.widths[0]}, flat.options()), net.widths[0]);
+    return by_type(rows, at::empty({rows.total * net.widths[0]}, params.options), net.widths[0]);
 }
 
 // The values from library operations, for derivatives of an order the kernels have no form for.
@@ -450,12 +493,13 @@ struct NetRowsFn : Function<NetRowsFn> {
     {
         const Unrecorded quiet;
         const Net net{widths, alpha};
-        const Rows rows = rows_of(net, flat, x0, x1, x2, x3);
-        const Pass p{net, rows, flat};
+        const Params params(net, flat);
+        const Rows rows = rows_of(net, params, x0, x1, x2, x3);
+        const Pass p{net, rows, params};
         const variable_list acts(kept_acts.begin(), kept_acts.begin() + p.L);
         const variable_list d = p.slopes(acts, kept_acts[p.L]);
         const Four s = {s0, s1, s2, s3};
-        const Four out = like_rows(net, rows, flat);
+        const Four out = like_rows(net, rows, params);
         p.to_rows(d[0], s, out, false);
         variable_list save = {flat, x0, x1, x2, x3, s0, s1, s2, s3};
         save.insert(save.end(), acts.begin(), acts.end());
@@ -491,8 +535,9 @@ struct NetRowsFn : Function<NetRowsFn> {
             return out;
         }
         const Unrecorded quiet;
-        const Rows rows = rows_of(net, flat, x[0], x[1], x[2], x[3]);
-        const Pass p{net, rows, flat};
+        const Params params(net, flat);
+        const Rows rows = rows_of(net, params, x[0], x[1], x[2], x[3]);
+        const Pass p{net, rows, params};
         const int L = p.L;
         const variable_list acts(saved.begin() + 9, saved.begin() + 9 + L), d(saved.begin() + 9 + L, saved.begin() + 9 + 2 * L);
         const Four v = or_zeros(rows, flat, u, 0, net.widths[0]);
@@ -517,11 +562,11 @@ struct NetRowsFn : Function<NetRowsFn> {
             khan_net_top a = {};
             a.k = static_cast<int32_t>(net.widths[L]);
             a.alpha = net.alpha;
-            const Four e = like_values(rows, flat);
+            const Four e = like_values(rows, params);
             p.set(a.act, dot[L - 1], net.widths[L]);
             for (int t = 0; t < 4; ++t) {
                 a.n[t] = static_cast<int32_t>(rows.n[t]);
-                a.w[t] = p.param(net.weight_at(L, t));
+                a.w[t] = params.weight(L, t);
                 a.value[t] = ptr<char>(e[t]);
                 out[5 + t] = e[t].reshape(s[t].sizes());
             }
@@ -553,7 +598,7 @@ struct NetRowsFn : Function<NetRowsFn> {
             p.run(a);
         }
         if (need_x) {
-            const Four g = like_rows(net, rows, flat);
+            const Four g = like_rows(net, rows, params);
             p.to_rows(q[0], Four{}, g, false);
             for (int t = 0; t < 4; ++t) out[1 + t] = g[t].reshape(x[t].sizes());
         }
@@ -586,9 +631,10 @@ struct NetFn : Function<NetFn> {
     {
         const Unrecorded quiet;
         const Net net{widths, alpha};
-        const Rows rows = rows_of(net, flat, x0, x1, x2, x3);
-        const Pass p{net, rows, flat};
-        const Four values = like_values(rows, flat);
+        const Params params(net, flat);
+        const Rows rows = rows_of(net, params, x0, x1, x2, x3);
+        const Pass p{net, rows, params};
+        const Four values = like_values(rows, params);
         variable_list acts = p.forward();
         const Tensor d = p.top(acts.back(), &values, graph);
         if (graph) {
@@ -615,7 +661,8 @@ struct NetFn : Function<NetFn> {
             for (int k = 0; k < 5; ++k) out[k] = g[k];
             return out;
         }
-        const Rows rows = rows_of(net, flat, x[0], x[1], x[2], x[3]);
+        const Params params(net, flat);
+        const Rows rows = rows_of(net, params, x[0], x[1], x[2], x[3]);
         if (at::GradMode::is_enabled()) {
             variable_list s(4);
             for (int t = 0; t < 4; ++t) s[t] = gs[t].defined() ? gs[t].contiguous() : at::zeros({rows.n[t]}, flat.options());
@@ -625,12 +672,12 @@ struct NetFn : Function<NetFn> {
             return out;
         }
         const Unrecorded quiet;
-        const Pass p{net, rows, flat};
+        const Pass p{net, rows, params};
         const variable_list acts(saved.begin() + 5, saved.begin() + 5 + p.L);
         const variable_list d = p.slopes(acts, saved[5 + p.L]);
         const Four scale = or_zeros(rows, flat, gs, 0, 1);
         if (need_x) {
-            const Four g = like_rows(net, rows, flat);
+            const Four g = like_rows(net, rows, params);
             p.to_rows(d[0], scale, g, false);
             for (int t = 0; t < 4; ++t) out[1 + t] = g[t].reshape(x[t].sizes());
         }
@@ -690,58 +737,13 @@ Tensor flatten(const std::vector<Tensor>& params)
     return FlattenFn::apply(at::TensorList(params));
 }
 
-// The network without a graph: the values, and with `want_grad` what `network_rows` needs to form gradients
-// -> (values[4], activations..., d_L)
-std::vector<Tensor> network_forward(const Tensor& flat, const std::vector<Tensor>& x, Saved widths, double alpha, bool want_grad)
-{
-    same_size(x.size() == 4, "four feature buckets");
-    const Net net{widths, alpha};
-    const Rows rows = rows_of(net, flat, x[0], x[1], x[2], x[3]);
-    const Pass p{net, rows, flat};
-    const Four values = like_values(rows, flat);
-    variable_list acts = p.forward();
-    const Tensor d = p.top(acts.back(), &values, want_grad);
-    std::vector<Tensor> out(values.begin(), values.end());
-    if (want_grad) {
-        out.insert(out.end(), acts.begin(), acts.end());
-        out.push_back(d);
-    }
-    return out;
-}
-
-// scale_r d value_r / d x_r from what network_forward left behind the values (scale: four vectors, or none for ones), into
-// new arrays or added to `into` (four arrays of rows) -> the four arrays
-std::vector<Tensor> network_rows(const Tensor& flat, const std::vector<Tensor>& x, Saved widths, double alpha, const std::vector<Tensor>& state,
-                                 const c10::optional<std::vector<Tensor>>& scale, const c10::optional<std::vector<Tensor>>& into)
-{
-    same_size(x.size() == 4, "four feature buckets");
-    const Net net{widths, alpha};
-    const Rows rows = rows_of(net, flat, x[0], x[1], x[2], x[3]);
-    const Pass p{net, rows, flat};
-    same_size(static_cast<int>(state.size()) == p.L + 1 && (!scale || scale->size() == 4) && (!into || into->size() == 4),
-              "state as network_forward returned it behind the values, and four scales and four arrays of rows");
-    const variable_list acts(state.begin(), state.begin() + p.L);
-    const variable_list d = p.slopes(acts, state[p.L]);
-    Four s, out = into ? Four{(*into)[0], (*into)[1], (*into)[2], (*into)[3]} : like_rows(net, rows, flat);
-    for (int t = 0; t < 4; ++t) {
-        if (scale) {
-            s[t] = (*scale)[t].reshape({-1});
-            dev(s[t], flat.scalar_type(), "scale");
-            same_size(s[t].numel() == rows.n[t], "scale must have one element per row");
-        }
-        same_size(out[t].numel() == rows.n[t] * net.widths[0] && out[t].is_contiguous() && out[t].scalar_type() == flat.scalar_type(),
-                  "arrays of rows like the features");
-    }
-    p.to_rows(d[0], s, out, into.has_value());
-    return {out[0], out[1], out[2], out[3]};
-}
-
 // ---------------------------------------------------------------------------------------------- inference
-// One network of a model: its parameters (constants here) and, where its widths are those of the one-launch kernel, the
-// weights split and packed for it
+// One network of a model: its parameters and, where its widths are those of the one-launch kernel, the weights split and
+// packed for it
 struct Weights {
-    Tensor flat, packed;
     Net net;
+    Params params;
+    Tensor packed;
 };
 
 // A network's pass over a batch: the values, then the rows' gradients.
@@ -753,23 +755,24 @@ struct Inference {
     variable_list state;                    // activations and d_L; in the one-launch form the rows' gradients
 
     Inference(const Weights& w_, const Four& x)
-        : w(w_), rows(rows_of(w.net, w.flat, x[0], x[1], x[2], x[3])), pass{w.net, rows, w.flat}, values(at::empty({rows.total}, w.flat.options()))
+        : w(w_), rows(rows_of(w.net, w.params, x[0], x[1], x[2], x[3])), pass{w.net, rows, w.params},
+          values(at::empty({rows.total}, w.params.options))
     {
     }
     bool one_launch() const { return w.packed.defined(); }
 
     Tensor launch(const Four& scale, bool want_rows)
     {
-        const Tensor grads = want_rows ? at::empty({rows.total * kFeats}, w.flat.options()) : Tensor();
+        const Tensor grads = want_rows ? at::empty({rows.total * kFeats}, w.params.options) : Tensor();
         const float *x[4], *bias[12], *head_w[4], *head_b[4], *sc[4];
         float *value[4], *grad[4];
         int32_t n[4];
         for (int t = 0; t < 4; ++t) {
             x[t] = ptr<float>(rows.x[t]);
             n[t] = static_cast<int32_t>(rows.n[t]);
-            for (int l = 0; l < 3; ++l) bias[4 * l + t] = reinterpret_cast<const float*>(pass.param(w.net.bias_at(l, t)));
-            head_w[t] = reinterpret_cast<const float*>(pass.param(w.net.weight_at(3, t)));
-            head_b[t] = reinterpret_cast<const float*>(pass.param(w.net.bias_at(3, t)));
+            for (int l = 0; l < 3; ++l) bias[4 * l + t] = reinterpret_cast<const float*>(w.params.bias(l, t));
+            head_w[t] = reinterpret_cast<const float*>(w.params.weight(3, t));
+            head_b[t] = reinterpret_cast<const float*>(w.params.bias(3, t));
             sc[t] = ptr<float>(scale[t]);
             value[t] = ptr<float>(values) ? ptr<float>(values) + rows.row0[t] : nullptr;
             grad[t] = want_rows && ptr<float>(grads) ? ptr<float>(grads) + rows.row0[t] * kFeats : nullptr;
@@ -799,7 +802,7 @@ struct Inference {
             return into.defined() ? into.add_(g) : g;
         }
         const bool add = into.defined();
-        if (!add) into = at::empty({rows.total * w.net.widths[0]}, w.flat.options());
+        if (!add) into = at::empty({rows.total * w.net.widths[0]}, w.params.options);
         const variable_list d = pass.slopes(variable_list(state.begin(), state.end() - 1), state.back());
         pass.to_rows(d[0], scale, by_type(rows, into, w.net.widths[0]), add);
         return into;
@@ -808,20 +811,56 @@ struct Inference {
 
 Weights weights_of(const py::tuple& t, double alpha)
 {
-    Weights w;
-    w.flat = t[0].cast<Tensor>();
+    const Net net{t[2].cast<Saved>(), alpha};
+    Weights w{net, Params(net, t[0].cast<std::vector<Tensor>>()), Tensor()};
     if (!t[1].is_none()) w.packed = t[1].cast<Tensor>();
-    w.net = {t[2].cast<Saved>(), alpha};
     if (w.packed.defined())
-        same_size(w.flat.scalar_type() == at::kFloat && w.net.widths == Saved{kFeats, 128, 128, 64, 1} && w.packed.scalar_type() == at::kByte &&
+        same_size(w.params.dtype == at::kFloat && w.net.widths == Saved{kFeats, 128, 128, 64, 1} && w.packed.scalar_type() == at::kByte &&
                       w.packed.is_cuda() && w.packed.numel() == api.khan_atomic_networks_packed_bytes(),
                   "packed weights are those of the 384-128-128-64-1 networks in float32");
     return w;
 }
 
+// The networks' part of `infer` alone, for a caller that has the rows: the values of the four types' rows and, with want_grad,
+// what `network_rows` needs to form gradients -> (values[4], activations..., d_L)
+std::vector<Tensor> network_forward(const Tensor& flat, const std::vector<Tensor>& x, Saved widths, double alpha, bool want_grad)
+{
+    same_size(x.size() == 4, "four feature buckets");
+    const Net net{widths, alpha};
+    const Weights w{net, Params(net, flat), Tensor()};
+    Inference net_pass(w, {x[0], x[1], x[2], x[3]});
+    const Four values = net_pass.forward(want_grad, false);
+    std::vector<Tensor> out(values.begin(), values.end());
+    if (want_grad) out.insert(out.end(), net_pass.state.begin(), net_pass.state.end());
+    return out;
+}
+
+// scale_r d value_r / d x_r from what network_forward left behind the values (scale: four vectors, or none for ones), into
+// new arrays or added to `into` (four arrays of rows, end to end in one) -> the four arrays
+std::vector<Tensor> network_rows(const Tensor& flat, const std::vector<Tensor>& x, Saved widths, double alpha, const std::vector<Tensor>& state,
+                                 const c10::optional<std::vector<Tensor>>& scale, const c10::optional<std::vector<Tensor>>& into)
+{
+    same_size(x.size() == 4, "four feature buckets");
+    const Net net{widths, alpha};
+    const Weights w{net, Params(net, flat), Tensor()};
+    Inference net_pass(w, {x[0], x[1], x[2], x[3]});
+    net_pass.state = state;
+    same_size(static_cast<int>(state.size()) == net.layers() && (!scale || scale->size() == 4) && (!into || into->size() == 4),
+              "state as network_forward returned it behind the values, and four scales and four arrays of rows");
+    Four s;
+    for (int t = 0; t < 4 && scale; ++t) {
+        s[t] = (*scale)[t].reshape({-1});
+        dev(s[t], w.params.dtype, "scale");
+        same_size(s[t].numel() == net_pass.rows.n[t], "scale must have one element per row");
+    }
+    const Four out = by_type(net_pass.rows, net_pass.gradients(s, into ? at::cat(*into) : Tensor()), net.widths[0]);
+    return {out[0], out[1], out[2], out[3]};
+}
+
 // A batch's energies and, with need_grad, their gradient by x, y and z: featurize, the networks' values and row gradients, the
 // sums by molecule, the charge energy, featurize_grad.  No graph: the order of the passes is known, and the gradient of
-// the near network's sum needs nothing from behind it.  near, charge: (flat parameters, packed or None, widths).
+// the near network's sum needs nothing from behind it.  near, charge: (the parameters as Params takes them, packed or None,
+// widths).
 // -> (energies,) or (energies, x, y, z); joined: all four are parts of one array, the last element of what is returned, which
 // holds the energies, padded to 64 elements, then the three gradients
 std::vector<Tensor> infer(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos, const Tensor& macs,
@@ -864,18 +903,6 @@ std::vector<Tensor> infer(const Tensor& xs, const Tensor& ys, const Tensor& zs, 
     return out;
 }
 
-// What the parameters are, for a caller that keeps something made from them: where each lies and how often it was written,
-// and the stream that what was kept has been made on
-py::bytes parameter_key(const std::vector<Tensor>& params)
-{
-    std::vector<uint64_t> key = {reinterpret_cast<uint64_t>(stream())};
-    for (const Tensor& p : params) {
-        key.push_back(reinterpret_cast<uint64_t>(p.data_ptr()));
-        key.push_back(p._version());
-    }
-    return py::bytes(reinterpret_cast<const char*>(key.data()), key.size() * sizeof(uint64_t));
-}
-
 }  // namespace
 
 void bind_autograd(py::module_& m)
@@ -888,7 +915,6 @@ void bind_autograd(py::module_& m)
     m.def("network_forward", &network_forward);
     m.def("network_rows", &network_rows);
     m.def("infer", &infer);
-    m.def("parameter_key", &parameter_key);
 }
 
 }  // namespace khan_torch

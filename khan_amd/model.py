@@ -179,15 +179,9 @@ class MoleculeNN:
         return [self.params[name] for name in self._flat_names]
 
     def constants(self):
-        """-> (the parameters end to end, packed for the one-launch kernel or None, the widths): what inference takes, kept
-        until a parameter is written again (or asked for on another stream, which has not waited for the copies)."""
-        native, ps = _native.load(), self._in_flat_order()
-        key = (native.parameter_key(ps), self.one_launch())
-        kept = self.__dict__.get("_constants")
-        if kept is None or kept[0] != key:
-            with torch.no_grad():
-                kept = self._constants = (key, (native.flatten(ps), self.one_launch_operands()[0] if key[1] else None, list(self.layer_sizes)))
-        return kept[1]
+        """-> (the parameters in flat order, packed for the one-launch kernel or None, the widths): what inference takes.  The
+        passes read the parameters where they lie: nothing is copied that a write to them could leave behind."""
+        return self._in_flat_order(), self.one_launch_operands()[0] if self.one_launch() else None, list(self.layer_sizes)
 
     def type_outputs(self, atom_type_features):
         """Per-type flat feature buckets -> the four per-type output vectors [acs[t]] (nn.py:165-175)."""
@@ -196,7 +190,9 @@ class MoleculeNN:
         # in single precision inference is the default: the weights are constants
         live = torch.is_grad_enabled() and (self.weights_need_grad or self.dtype == torch.float64 or self.kernel_layers() == 0)
         native = _native.load()
-        flat = native.flatten(self._in_flat_order()) if live else self.constants()[0]
+        flat = native.flatten(self._in_flat_order())
+        if not live:
+            flat = flat.detach()
         return native.network_autograd(flat, list(atom_type_features), self.layer_sizes, 0.1)
 
 

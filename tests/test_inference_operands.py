@@ -1,0 +1,62 @@
+"""Inference takes the parameters as they are when it runs: written to past the version counter, replaced by other tensors, or held
+in another order of memory."""
+import numpy as np
+import pytest
+import torch
+
+from khan_amd import datagen, model
+from khan_amd.batching import DeviceBatch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _batch(n_mols, dtype, kind="organic", first=0):
+    b = datagen.make_batch(kind, n_mols, first_mol=first)
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
+    return DeviceBatch.from_device_arrays(*(d(v).to(dtype) for v in (b.X, b.Y, b.Z)), d(b.A), d(b.mol_idxs), b.n_mols)
+
+
+def _like(m, layers, dtype, charges):
+    """A model of its own with the parameters that m has now."""
+    other = model.AniModel(layers, model.celu, dtype, DEV, fit_charges=charges, seed=99)
+    with torch.no_grad():
+        for k, p in other.named_parameters().items():
+            p.copy_(m.named_parameters()[k])
+    return other
+
+
+# every way a network runs in inference: one launch, layer by layer in both precisions, with a charge network
+@pytest.mark.parametrize("layers,dtype,charges,only", [
+    (model.DEFAULT_LAYERS, torch.float32, False, "b_"), (model.DEFAULT_LAYERS, torch.float64, False, ""),
+    ((100, 1), torch.float32, False, ""), (model.DEFAULT_LAYERS, torch.float64, True, "")])
+def test_parameters_written_past_the_version_counter(layers, dtype, charges, only):
+    m = model.AniModel(layers, model.celu, dtype, DEV, fit_charges=charges, seed=1)
+    b = _batch(50, dtype)
+    before, _ = m.batch_energies(b, need_grad=True)
+    for k, p in m.named_parameters().items():
+        if only in k:
+            version = p._version
+            p.data.add_(0.01)
+            assert p._version == version
+    got, got_g = m.batch_energies(b, need_grad=True)
+    want, want_g = _like(m, layers, dtype, charges).batch_energies(b, need_grad=True)
+    assert torch.equal(got, want) and torch.equal(got_g, want_g) and not torch.equal(got, before)
+
+
+@pytest.mark.parametrize("layers,dtype", [(model.DEFAULT_LAYERS, torch.float64), ((100, 1), torch.float32)])
+def test_parameters_replaced_and_strided(layers, dtype):
+    """New tensors in `params`, weights in column order and biases with a stride; a parameter of another type is refused."""
+    m = model.AniModel(layers, model.celu, dtype, DEV, seed=1)
+    b = _batch(50, dtype)
+    m.batch_energies(b)
+    for k, p in list(m.near.params.items()):
+        v = p.detach() + 0.01
+        m.near.params[k] = (v.t().contiguous().t() if v.dim() == 2 else torch.stack([v, v], dim=1)[:, 0]).requires_grad_(True)
+    got, got_g = m.batch_energies(b, need_grad=True)
+    want, want_g = _like(m, layers, dtype, False).batch_energies(b, need_grad=True)
+    assert torch.equal(got, want) and torch.equal(got_g, want_g)
+    k = m.near.names["C"][0][0]
+    m.near.params[k] = m.near.params[k].detach().to(torch.float32 if dtype == torch.float64 else torch.float64)
+    with pytest.raises((TypeError, ValueError)):
+        m.batch_energies(b)
