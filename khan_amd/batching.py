@@ -206,16 +206,19 @@ class DeviceBatch:
 
     __slots__ = ("xs", "ys", "zs", "atom_types", "mol_idxs", "n_mols", "mol_atom_counts", "mol_offsets",
                  "scatter_idxs", "gather_idxs", "atom_counts", "size_order", "counts_pinned", "labels", "grads", "ready",
-                 "memory", "sizes", "totals")
+                 "memory", "sizes", "totals", "made_on")
 
     def __init__(self):
         self.labels = self.grads = self.counts_pinned = None
+        self.made_on = None       # the stream that `ready` was recorded on
         self.memory = self.sizes = self.totals = None    # of a batch from the host: its one buffer, molecule sizes, counts
 
     def host_counts(self):
         """-> (atoms per type [4], the size order on the device, molecules per size class [4] on the host): what the
         host has to know before it can launch the passes.  A batch from the host brings them along; otherwise the sort
-        writes them to pinned memory, and this waits for it."""
+        writes them to pinned memory, and this waits for it.  The numbers may be there before the batch's arrays are, so
+        the current stream is made to wait for those: what it is given from here on finds them."""
+        self._join()
         if self.totals is not None:
             return list(self.totals[0]), self.size_order, list(self.totals[1])
         counts = _native.load().wait_for_counts(self.counts_pinned)
@@ -226,6 +229,8 @@ class DeviceBatch:
 
     def host_sizes(self):
         """The molecules' sizes, a list on the host."""
+        if self.sizes is None:
+            self._join()
         return self.mol_atom_counts.tolist() if self.sizes is None else self.sizes
 
     @classmethod
@@ -246,8 +251,16 @@ class DeviceBatch:
         self.counts_pinned = torch.empty(8, dtype=torch.int32, pin_memory=True)     # from the pinned-memory cache; the sort writes it
         (self.mol_atom_counts, self.mol_offsets, self.scatter_idxs, self.gather_idxs, self.atom_counts,
          self.size_order) = ops.prepare_batch(self.mol_idxs, self.atom_types, self.n_mols, self.counts_pinned)
+        self.made_on = torch.cuda.current_stream()
         self.ready = torch.cuda.Event()
-        self.ready.record()
+        self.ready.record(self.made_on)
+
+    def _join(self):
+        """`wait()`, where the current stream is not the one the batch was made on."""
+        import torch
+        cur = torch.cuda.current_stream()
+        if cur != self.made_on:
+            self.wait(cur)
 
     def wait(self, stream=None):
         """Makes the current stream (`stream`, if the caller has it at hand) wait for the copies and the sort of this batch."""
@@ -370,7 +383,8 @@ class DeviceFeeder:
             with torch.cuda.stream(self.stream):
                 b.grads = torch.from_numpy(np.ascontiguousarray(mol_grads, dtype=self.dtype)).to(self.device)
         b.ready = self._events[slot] = torch.cuda.Event()
-        b.ready.record(self.stream)
+        b.made_on = self.stream
+        b.ready.record(b.made_on)
         return b
 
     def __iter__(self):
