@@ -362,6 +362,9 @@ int khan_dense_head_grad_f32(const float *const *scale_host4, const float *const
 int64_t khan_atomic_networks_packed_bytes(void);
 int khan_atomic_networks_pack_f32(const float *const *weights_t_host12, const float *const *weights_host12,
                                   void *packed, khan_stream_t stream);
+/* The same buffer from the matrices as stored alone, in one launch: what a caller whose weights may have changed does before
+ * every khan_atomic_networks_f32. */
+int khan_atomic_networks_pack_stored_f32(const float *const *weights_host12, void *packed, khan_stream_t stream);
 int khan_atomic_networks_f32(const float *const *rows_host4, const int32_t *n_host4,
                              const float *const *weights_t_host12, const float *const *weights_host12,
                              const void *packed, const float *const *biases_host12, const float *const *head_w_host4,

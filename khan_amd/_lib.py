@@ -80,6 +80,7 @@ _SIGNATURES = {
                                                 ctypes.POINTER(_ptr), ctypes.POINTER(_ptr), _ptr]),
     "khan_atomic_networks_packed_bytes": (ctypes.c_int64, []),
     "khan_atomic_networks_pack_f32": (ctypes.c_int, [ctypes.POINTER(_ptr), ctypes.POINTER(_ptr), _ptr, _ptr]),
+    "khan_atomic_networks_pack_stored_f32": (ctypes.c_int, [ctypes.POINTER(_ptr), _ptr, _ptr]),
     "khan_atomic_networks_f32": (ctypes.c_int, [ctypes.POINTER(_ptr), ctypes.POINTER(ctypes.c_int32), ctypes.POINTER(_ptr),
                                                 ctypes.POINTER(_ptr), _ptr] + [ctypes.POINTER(_ptr)] * 4
                                  + [ctypes.c_float, ctypes.POINTER(_ptr), ctypes.POINTER(_ptr), _ptr]),

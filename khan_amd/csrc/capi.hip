@@ -878,6 +878,16 @@ int khan_atomic_networks_pack_f32(const float* const* weights_t_host12, const fl
                                                  weights_host12 + 4, weights_host12 + 8, packed, as_stream(stream)));
 }
 
+int khan_atomic_networks_pack_stored_f32(const float* const* weights_host12, void* packed, khan_stream_t stream)
+{
+    if (!weights_host12 || !packed) return KHAN_ERR_INVALID_ARG;
+    for (int k = 0; k < 12; ++k)
+        if (!weights_host12[k]) return KHAN_ERR_INVALID_ARG;
+    if (reinterpret_cast<uintptr_t>(packed) & 15u) return KHAN_ERR_INVALID_ARG;
+    return hip_status(khan::launch_networks_pack(nullptr, nullptr, nullptr, weights_host12, weights_host12 + 4, weights_host12 + 8, packed,
+                                                 as_stream(stream)));
+}
+
 int khan_atomic_networks_f32(const float* const* rows_host4, const int32_t* n_host4, const float* const* weights_t_host12,
                              const float* const* weights_host12, const void* packed, const float* const* biases_host12,
                              const float* const* head_w_host4, const float* const* head_b_host4,

@@ -439,7 +439,10 @@ void networks_fused_kernel(FusedArgs args, float alpha, float inv_alpha)
     }
 }
 
-// one float32 weight -> its two half-precision parts in the packed buffer; a thread per weight of one type's six matrices
+// one float32 weight -> its two half-precision parts in the packed buffer; a thread per weight of one type's six matrices.
+// kStored: the transposed matrices are read from the stored ones, neighbouring threads along a stored row (a transposed copy
+// of twelve matrices is twelve launches; the strided two-byte writes stay in L2).
+template <bool kStored>
 __global__ __launch_bounds__(256) void pack_weights_kernel(FusedArgs args, unsigned short* __restrict__ packed)
 {
     const int t = blockIdx.y;
@@ -448,10 +451,12 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(FusedArgs args, unsig
     if (i >= 2 * (n1 + n2 + n3)) return;
     const float* src;
     int at, cols, k_len, j = i;      // the matrix: where it starts in the packed buffer, its columns and its summed length
-    if (j < n1) { src = args.w1t[t]; at = kPackF1; cols = kN1; k_len = kK1; }
-    else if ((j -= n1) < n2) { src = args.w2t[t]; at = kPackF2; cols = kN2; k_len = kN1; }
-    else if ((j -= n2) < n3) { src = args.w3t[t]; at = kPackF3; cols = kN3; k_len = kN2; }
+    bool across = kStored;           // src is [k][column]
+    if (j < n1) { src = kStored ? args.w1[t] : args.w1t[t]; at = kPackF1; cols = kN1; k_len = kK1; }
+    else if ((j -= n1) < n2) { src = kStored ? args.w2[t] : args.w2t[t]; at = kPackF2; cols = kN2; k_len = kN1; }
+    else if ((j -= n2) < n3) { src = kStored ? args.w3[t] : args.w3t[t]; at = kPackF3; cols = kN3; k_len = kN2; }
     else if ((j -= n3) < n1) {       // layer 1 as stored, [384][128]: three matrices of 128 columns
+        across = false;
         src = args.w1[t];
         const int ct = j / (128 * kN1);
         src += ct * 128 * kN1;
@@ -460,11 +465,12 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(FusedArgs args, unsig
         cols = 128;
         k_len = kN1;
     }
-    else if ((j -= n1) < n2) { src = args.w2[t]; at = kPackB2; cols = kN1; k_len = kN2; }
-    else { j -= n2; src = args.w3[t]; at = kPackB3; cols = kN2; k_len = kN3; }
+    else if ((j -= n1) < n2) { across = false; src = args.w2[t]; at = kPackB2; cols = kN1; k_len = kN2; }
+    else { j -= n2; across = false; src = args.w3[t]; at = kPackB3; cols = kN2; k_len = kN3; }
     unsigned p1, p2;
     split_pair(src[j], 0.f, p1, p2);
-    const int r = j / k_len, k = j - r * k_len;
+    const int line = across ? cols : k_len, major = j / line, minor = j - major * line;
+    const int r = across ? minor : major, k = across ? major : minor;
     unsigned short* dst = packed + static_cast<size_t>(t) * kPackPerType + at + ((k / kKC) * kParts * cols + r) * kKC + (k % kKC);
     dst[0] = static_cast<unsigned short>(p1 & 0xffffu);
     dst[cols * kKC] = static_cast<unsigned short>(p2 & 0xffffu);
@@ -474,18 +480,21 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(FusedArgs args, unsig
 
 size_t networks_packed_bytes() { return static_cast<size_t>(4) * kPackPerType * sizeof(unsigned short); }
 
-// the six weight matrices of each type (three transposed, three as stored) split into `packed` (networks_packed_bytes())
-hipError_t launch_networks_pack(const float* const w1t[4], const float* const w2t[4], const float* const w3t[4],
+// the six weight matrices of each type (three transposed, three as stored) split into `packed` (networks_packed_bytes());
+// w*t null: the transposed ones from the stored ones
+hipError_t launch_networks_pack(const float* const* w1t, const float* const* w2t, const float* const* w3t,
                                 const float* const w1[4], const float* const w2[4], const float* const w3[4],
                                 void* packed, hipStream_t stream)
 {
     FusedArgs a = {};
     for (int t = 0; t < 4; ++t) {
-        a.w1t[t] = w1t[t]; a.w2t[t] = w2t[t]; a.w3t[t] = w3t[t];
+        if (w1t) { a.w1t[t] = w1t[t]; a.w2t[t] = w2t[t]; a.w3t[t] = w3t[t]; }
         a.w1[t] = w1[t]; a.w2[t] = w2[t]; a.w3[t] = w3[t];
     }
     constexpr int per_type = 2 * (kN1 * kK1 + kN2 * kN1 + kN3 * kN2);
-    pack_weights_kernel<<<dim3((per_type + 255) / 256, 4), dim3(256), 0, stream>>>(a, static_cast<unsigned short*>(packed));
+    const dim3 grid((per_type + 255) / 256, 4);
+    if (w1t) pack_weights_kernel<false><<<grid, dim3(256), 0, stream>>>(a, static_cast<unsigned short*>(packed));
+    else pack_weights_kernel<true><<<grid, dim3(256), 0, stream>>>(a, static_cast<unsigned short*>(packed));
     return hipGetLastError();
 }
 

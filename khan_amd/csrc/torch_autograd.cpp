@@ -738,8 +738,7 @@ Tensor flatten(const std::vector<Tensor>& params)
 }
 
 // ---------------------------------------------------------------------------------------------- inference
-// One network of a model: its parameters and, where its widths are those of the one-launch kernel, the weights split and
-// packed for it
+// One network of a model: its parameters and, for the one-launch kernel, the weights split and packed
 struct Weights {
     Net net;
     Params params;
@@ -813,11 +812,16 @@ Weights weights_of(const py::tuple& t, double alpha)
 {
     const Net net{t[2].cast<Saved>(), alpha};
     Weights w{net, Params(net, t[0].cast<std::vector<Tensor>>()), Tensor()};
-    if (!t[1].is_none()) w.packed = t[1].cast<Tensor>();
-    if (w.packed.defined())
-        same_size(w.params.dtype == at::kFloat && w.net.widths == Saved{kFeats, 128, 128, 64, 1} && w.packed.scalar_type() == at::kByte &&
-                      w.packed.is_cuda() && w.packed.numel() == api.khan_atomic_networks_packed_bytes(),
-                  "packed weights are those of the 384-128-128-64-1 networks in float32");
+    if (t[1].cast<bool>()) {
+        same_size(w.params.dtype == at::kFloat && net.widths == Saved{kFeats, 128, 128, 64, 1},
+                  "the one-launch kernel takes 384-128-128-64-1 networks in float32");
+        // One launch of 6 us on the stream that reads it: what the parameters are now, without a word about who may write to
+        // them and when.
+        w.packed = at::empty({api.khan_atomic_networks_packed_bytes()}, w.params.options.dtype(at::kByte));
+        const float* stored[12];
+        for (int k = 0; k < 12; ++k) stored[k] = reinterpret_cast<const float*>(w.params.weight(k / 4, k % 4));
+        call(api.khan_atomic_networks_pack_stored_f32, static_cast<const float* const*>(stored), w.packed.data_ptr(), stream());
+    }
     return w;
 }
 
@@ -859,8 +863,8 @@ std::vector<Tensor> network_rows(const Tensor& flat, const std::vector<Tensor>& 
 
 // A batch's energies and, with need_grad, their gradient by x, y and z: featurize, the networks' values and row gradients, the
 // sums by molecule, the charge energy, featurize_grad.  No graph: the order of the passes is known, and the gradient of
-// the near network's sum needs nothing from behind it.  near, charge: (the parameters as Params takes them, packed or None,
-// widths).
+// the near network's sum needs nothing from behind it.  near, charge: (the parameters as Params takes them, whether in
+// one launch, widths).
 // -> (energies,) or (energies, x, y, z); joined: all four are parts of one array, the last element of what is returned, which
 // holds the energies, padded to 64 elements, then the three gradients
 std::vector<Tensor> infer(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& as, const Tensor& mos, const Tensor& macs,

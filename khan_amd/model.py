@@ -113,14 +113,8 @@ class MoleculeNN:
         return a.reshape(-1)
 
     def layer_transposed(self, k):
-        """The four weights of layer k transposed ([out, in], the summed index contiguous), as `ops.dense` takes them;
-        kept until a weight is written again."""
-        ws = [self.params[self.names[t][k][0]] for t in TYPE_MAP]
-        key = tuple((w.data_ptr(), w._version) for w in ws)
-        cache = self.__dict__.setdefault("_wt_cache", {})
-        if k not in cache or cache[k][0] != key:
-            cache[k] = (key, [w.detach().t().contiguous() for w in ws])
-        return cache[k][1]
+        """The four weights of layer k transposed ([out, in], the summed index contiguous), as `ops.dense` takes them."""
+        return [self.params[self.names[t][k][0]].detach().t().contiguous() for t in TYPE_MAP]
 
     def kernel_layers(self):
         """How many leading layers have the widths of the split-operand matrix-core kernels (`ops.dense`,
@@ -146,18 +140,10 @@ class MoleculeNN:
 
     def one_launch_operands(self):
         """-> (packed weights, biases, head_weights, head_biases) as `ops.atomic_networks` takes them; the weights are
-        split into their half-precision parts once and kept until a weight is written again."""
+        split into their half-precision parts by one launch on the current stream, as they are when it runs."""
         from . import ops
-        rows = [[self.names[t][k] for t in TYPE_MAP] for k in range(4)]
-        ws = [self.params[r[0]] for k in range(3) for r in rows[k]]
-        key = tuple((w.data_ptr(), w._version) for w in ws)
-        cache = self.__dict__.setdefault("_packed_cache", {})
-        if cache.get("key") != key:
-            weights_t = [self.layer_transposed(k) for k in range(3)]
-            weights = [[self.params[r[0]].detach() for r in rows[k]] for k in range(3)]
-            cache["key"], cache["packed"] = key, ops.pack_network_weights(weights_t, weights)
-        biases = [[self.params[r[1]].detach() for r in rows[k]] for k in range(3)]
-        return cache["packed"], biases, [self.params[r[0]].detach() for r in rows[3]], [self.params[r[1]].detach() for r in rows[3]]
+        rows = [[self.params[self.names[t][k][j]].detach() for t in TYPE_MAP] for j in (0, 1) for k in range(4)]
+        return ops.pack_stored_network_weights(rows[:3]), rows[4:7], rows[3], rows[7]
 
     def atom_outputs(self, atom_type_features, gather_idxs):
         """Per-type flat feature buckets -> one number per atom in the batch's atom order (nn.py:176-177)."""
@@ -179,9 +165,10 @@ class MoleculeNN:
         return [self.params[name] for name in self._flat_names]
 
     def constants(self):
-        """-> (the parameters in flat order, packed for the one-launch kernel or None, the widths): what inference takes.  The
-        passes read the parameters where they lie: nothing is copied that a write to them could leave behind."""
-        return self._in_flat_order(), self.one_launch_operands()[0] if self.one_launch() else None, list(self.layer_sizes)
+        """-> (the parameters in flat order, True if the one-launch kernel takes them, the widths): what inference takes.  The
+        passes read the parameters where they lie, and the one-launch kernel's packed form is made of them in every pass:
+        nothing is kept that a write to them could leave behind."""
+        return self._in_flat_order(), self.one_launch(), list(self.layer_sizes)
 
     def type_outputs(self, atom_type_features):
         """Per-type flat feature buckets -> the four per-type output vectors [acs[t]] (nn.py:165-175)."""

@@ -344,6 +344,19 @@ def pack_network_weights(weights_t, weights):
     return packed
 
 
+def pack_stored_network_weights(weights):
+    """`pack_network_weights` from the matrices as stored alone (weights[l][t], any strides), in one launch."""
+    lib = _lib.load()
+    ws = []
+    for l in range(3):
+        for t in range(4):
+            n_out, k = _NETWORK_SHAPES_T[l]
+            ws.append(_dense_weights(weights[l][t].contiguous(), k, n_out, "weights[%d][%d]" % (l, t)))
+    packed = torch.empty(int(lib.khan_atomic_networks_packed_bytes()), dtype=torch.uint8, device=ws[0].device)
+    _lib.check(lib.khan_atomic_networks_pack_stored_f32((ctypes.c_void_p * 12)(*[w.data_ptr() for w in ws]), _p(packed), _stream()))
+    return packed
+
+
 def atomic_networks(rows, weights_t, biases, head_weights, head_biases=None, weights=None, scales=None, want_grad=False,
                     alpha=0.1, packed=None):
     """The 384-128-128-64-1 CELU networks of the four atom types in one launch, float32: -> (values, grads).

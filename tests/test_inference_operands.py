@@ -28,7 +28,7 @@ def _like(m, layers, dtype, charges):
 
 # every way a network runs in inference: one launch, layer by layer in both precisions, with a charge network
 @pytest.mark.parametrize("layers,dtype,charges,only", [
-    (model.DEFAULT_LAYERS, torch.float32, False, "b_"), (model.DEFAULT_LAYERS, torch.float64, False, ""),
+    (model.DEFAULT_LAYERS, torch.float32, False, ""), (model.DEFAULT_LAYERS, torch.float64, False, ""),
     ((100, 1), torch.float32, False, ""), (model.DEFAULT_LAYERS, torch.float64, True, "")])
 def test_parameters_written_past_the_version_counter(layers, dtype, charges, only):
     m = model.AniModel(layers, model.celu, dtype, DEV, fit_charges=charges, seed=1)
@@ -44,7 +44,7 @@ def test_parameters_written_past_the_version_counter(layers, dtype, charges, onl
     assert torch.equal(got, want) and torch.equal(got_g, want_g) and not torch.equal(got, before)
 
 
-@pytest.mark.parametrize("layers,dtype", [(model.DEFAULT_LAYERS, torch.float64), ((100, 1), torch.float32)])
+@pytest.mark.parametrize("layers,dtype", [(model.DEFAULT_LAYERS, torch.float64), ((100, 1), torch.float32), (model.DEFAULT_LAYERS, torch.float32)])
 def test_parameters_replaced_and_strided(layers, dtype):
     """New tensors in `params`, weights in column order and biases with a stride; a parameter of another type is refused."""
     m = model.AniModel(layers, model.celu, dtype, DEV, seed=1)
@@ -60,3 +60,20 @@ def test_parameters_replaced_and_strided(layers, dtype):
     m.near.params[k] = m.near.params[k].detach().to(torch.float32 if dtype == torch.float64 else torch.float64)
     with pytest.raises((TypeError, ValueError)):
         m.batch_energies(b)
+
+
+def test_weights_packed_from_the_stored_matrices():
+    """The same bytes as from the transposed copies, and a stream's own: nothing is kept between calls that another stream would
+    have to wait for."""
+    from khan_amd import ops
+    net = model.AniModel(seed=4).near
+    stored = [[net.params[net.names[t][k][0]].detach() for t in model.TYPE_MAP] for k in range(3)]
+    want = ops.pack_network_weights([net.layer_transposed(k) for k in range(3)], stored)
+    assert torch.equal(ops.pack_stored_network_weights(stored), want)
+    assert torch.equal(ops.pack_stored_network_weights([[w.t().contiguous().t() for w in layer] for layer in stored]), want)
+    torch.cuda.synchronize()
+    first = net.one_launch_operands()[0]
+    with torch.cuda.stream(torch.cuda.Stream()):
+        second = net.one_launch_operands()[0]
+    torch.cuda.synchronize()
+    assert torch.equal(first, want) and torch.equal(second, want) and first.data_ptr() != second.data_ptr()
