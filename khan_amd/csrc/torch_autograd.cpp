@@ -760,10 +760,10 @@ struct Inference {
     }
     bool one_launch() const { return w.packed.defined(); }
 
-    Tensor launch(const Four& scale, bool want_rows)
+    Tensor launch(bool want_rows)
     {
         const Tensor grads = want_rows ? at::empty({rows.total * kFeats}, w.params.options) : Tensor();
-        const float *x[4], *bias[12], *head_w[4], *head_b[4], *sc[4];
+        const float *x[4], *bias[12], *head_w[4], *head_b[4];
         float *value[4], *grad[4];
         int32_t n[4];
         for (int t = 0; t < 4; ++t) {
@@ -772,34 +772,31 @@ struct Inference {
             for (int l = 0; l < 3; ++l) bias[4 * l + t] = reinterpret_cast<const float*>(w.params.bias(l, t));
             head_w[t] = reinterpret_cast<const float*>(w.params.weight(3, t));
             head_b[t] = reinterpret_cast<const float*>(w.params.bias(3, t));
-            sc[t] = ptr<float>(scale[t]);
             value[t] = ptr<float>(values) ? ptr<float>(values) + rows.row0[t] : nullptr;
             grad[t] = want_rows && ptr<float>(grads) ? ptr<float>(grads) + rows.row0[t] * kFeats : nullptr;
         }
         call(api.khan_atomic_networks_f32, x, n, static_cast<const float* const*>(nullptr), static_cast<const float* const*>(nullptr),
-             static_cast<const void*>(w.packed.data_ptr()), bias, head_w, head_b, scale[0].defined() ? sc : static_cast<const float* const*>(nullptr),
+             static_cast<const void*>(w.packed.data_ptr()), bias, head_w, head_b, static_cast<const float* const*>(nullptr),
              static_cast<float>(w.net.alpha), value, want_rows ? grad : static_cast<float* const*>(nullptr), pass.st);
         return grads;
     }
-    // want_rows: row gradients will be asked for; scaled: with a scale, which is not known yet
-    Four forward(bool want_rows, bool scaled)
+    // want_rows: row gradients will be asked for
+    Four forward(bool want_rows)
     {
         const Four v = by_type(rows, values, 1);
         if (one_launch()) {
-            state = {launch({}, want_rows && !scaled)};
+            state = {launch(want_rows)};
         } else {
             state = pass.forward();
             state.push_back(pass.top(state.back(), &v, want_rows));
         }
         return v;
     }
-    // the rows' gradients times scale (undefined: ones), added to `into` where defined -> [all rows, features]
+    // the rows' gradients times scale (undefined: ones), added to `into` where defined -> [all rows, features]; the one-launch
+    // form has them already, and neither scale nor anything to add to
     Tensor gradients(const Four& scale, Tensor into)
     {
-        if (one_launch()) {
-            const Tensor g = scale[0].defined() ? launch(scale, true) : state[0];
-            return into.defined() ? into.add_(g) : g;
-        }
+        if (one_launch()) return state[0];
         const bool add = into.defined();
         if (!add) into = at::empty({rows.total * w.net.widths[0]}, w.params.options);
         const variable_list d = pass.slopes(variable_list(state.begin(), state.end() - 1), state.back());
@@ -833,7 +830,7 @@ std::vector<Tensor> network_forward(const Tensor& flat, const std::vector<Tensor
     const Net net{widths, alpha};
     const Weights w{net, Params(net, flat), Tensor()};
     Inference net_pass(w, {x[0], x[1], x[2], x[3]});
-    const Four values = net_pass.forward(want_grad, false);
+    const Four values = net_pass.forward(want_grad);
     std::vector<Tensor> out(values.begin(), values.end());
     if (want_grad) out.insert(out.end(), net_pass.state.begin(), net_pass.state.end());
     return out;
@@ -884,15 +881,17 @@ std::vector<Tensor> infer(const Tensor& xs, const Tensor& ys, const Tensor& zs, 
     const auto f = run_featurize(in, args);
     const Four feats = {f[0], f[1], f[2], f[3]};
     const Weights near_w = weights_of(near, alpha);
+    same_size(charge.is_none() || !near_w.packed.defined(), "networks beside a charge network run layer by layer");
     Inference near_net(near_w, feats);
-    run_mol_energy(near_net.forward(need_grad, false), as, sis, mos, macs, out[0]);
+    run_mol_energy(near_net.forward(need_grad), as, sis, mos, macs, out[0]);
     if (charge.is_none()) {
         if (need_grad) run_featurize_grad(in, args, by_type(near_net.rows, near_net.gradients({}, Tensor()), kFeats), {out[1], out[2], out[3]});
         return out;
     }
     const Weights charge_w = weights_of(charge.cast<py::tuple>(), alpha);
+    same_size(!charge_w.packed.defined(), "a charge network runs layer by layer");
     Inference charge_net(charge_w, feats);
-    charge_net.forward(need_grad, true);
+    charge_net.forward(need_grad);
     const Tensor qs = charge_net.values.index_select(0, gather);
     if (!need_grad) {
         out[0].add_(ani_charge(in[0], in[1], in[2], qs, mos, macs));

@@ -164,11 +164,11 @@ class MoleculeNN:
             self._flat_names = [self.names[t][k][j] for j in (0, 1) for k in range(len(self.layer_sizes) - 1) for t in TYPE_MAP]
         return [self.params[name] for name in self._flat_names]
 
-    def constants(self):
-        """-> (the parameters in flat order, True if the one-launch kernel takes them, the widths): what inference takes.  The
-        passes read the parameters where they lie, and the one-launch kernel's packed form is made of them in every pass:
-        nothing is kept that a write to them could leave behind."""
-        return self._in_flat_order(), self.one_launch(), list(self.layer_sizes)
+    def constants(self, one_launch=True):
+        """-> (the parameters in flat order, True if the one-launch kernel takes them (never without `one_launch`), the
+        widths): what inference takes.  The passes read the parameters where they lie, and the one-launch kernel's packed
+        form is made of them in every pass: nothing is kept that a write to them could leave behind."""
+        return self._in_flat_order(), one_launch and self.one_launch(), list(self.layer_sizes)
 
     def type_outputs(self, atom_type_features):
         """Per-type flat feature buckets -> the four per-type output vectors [acs[t]] (nn.py:165-175)."""
@@ -242,9 +242,12 @@ class AniModel:
                 parts.append(torch.cat([energies, energies.new_empty(-b.n_mols % 64)] + parts))
             return [energies] + parts
         acs, order, classes = b.host_counts()
+        # Networks beside a charge network run layer by layer: products of all 24 bits over float32's range, where the
+        # one-launch kernel's operands keep 2^-24 of their size between 6e-5 and 65,504.
+        alone = self.charge is None
         return _native.load().infer(
             b.xs, b.ys, b.zs, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs, b.gather_idxs, acs, order, classes,
-            self.near.constants(), None if self.charge is None else self.charge.constants(), 0.1, need_grad, joined)
+            self.near.constants(alone), None if alone else self.charge.constants(False), 0.1, need_grad, joined)
 
     def _energies_through_autograd(self, b, need_grad):
         """_energies for networks of library operations (other activations than CELU)."""

@@ -77,3 +77,26 @@ def test_weights_packed_from_the_stored_matrices():
         second = net.one_launch_operands()[0]
     torch.cuda.synchronize()
     assert torch.equal(first, want) and torch.equal(second, want) and first.data_ptr() != second.data_ptr()
+
+
+@pytest.mark.parametrize("exponent", [0, 24, -30])
+def test_float32_networks_beside_a_charge_network(exponent):
+    """Default networks in float32 with a charge network: products of all 24 bits over float32's range.  Layer 1 (kept clear
+    of CELU's knee by its biases) scaled by 2^exponent and layer 2 by the inverse leave the result what it is, and carry
+    activations and weights past half precision's range (65,504; 6e-5).  Bound: the roundings of four layers' sums and the
+    way back, 2e-6 of sum |x| |w| each as for one layer, whose terms are some times the largest result here."""
+    models = [model.AniModel(model.DEFAULT_LAYERS, model.celu, dt, DEV, fit_charges=True, seed=6) for dt in (torch.float32, torch.float64)]
+    single, double = (m.named_parameters() for m in models)
+    with torch.no_grad():
+        for k, p in single.items():
+            if "_l1:" in k:
+                if "b_" in k:
+                    p.fill_(8.0)
+                p.mul_(2.0 ** exponent)
+            if "_l2:" in k and "W_" in k:
+                p.mul_(2.0 ** -exponent)
+            double[k].copy_(p)
+    got, want = (m.batch_energies(_batch(400, dt), need_grad=True) for m, dt in zip(models, (torch.float32, torch.float64)))
+    for g, w in zip(got, want):
+        assert torch.isfinite(g).all()
+        assert float((g.double() - w).abs().max()) <= 2e-5 * float(w.abs().max())
