@@ -300,6 +300,11 @@ __global__ __launch_bounds__(256) void layer_kernel(const NetLayer<T> a, int tot
 // Per chunk a wavefront issues 48 matrix instructions (1,536 cycles; kNB = 4) and 250 vector ones (1,000), most of them
 // splitting, and the two hide each other only in part: 172 TFLOP/s where the float32 instructions gave 70 (96,000 rows
 // 256 -> 256: 139 -> 73 us; 48,000 rows 73 -> 38; transposed 78 -> 40).
+// With 64 columns the five small partial products have accumulators of their own (kApart): the large sum is then rounded
+// once in 16 k instead of six times, a layer's distance from float64 falls to 0.4 of the float32 library product's, and it
+// costs nothing (12,000 rows 384 -> 128: 17.9 -> 17.8 us; 47,000 rows 128 -> 64: 13.0 -> 12.9).  With 128 columns there are no
+// registers for them at three workgroups per compute unit (two: deep networks on 47,000 rows 1,790 -> 1,950 us): the sums
+// there are rounded as often as those of dense_first.hip's kernel, and the form is kept to the widths that kernel takes.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 constexpr int kWideRows = 128;
@@ -309,6 +314,7 @@ __global__ __launch_bounds__(256, 3) void layer_split_kernel(const NetLayer<floa
 {
     typedef Vec<float, kNB> vec;
     constexpr int kCols = 32 * kNB;
+    constexpr bool kApart = kNB == 2;
     __shared__ u4v S[2][3][4][kCols + 2];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, half = lane >> 5;
@@ -353,9 +359,13 @@ __global__ __launch_bounds__(256, 3) void layer_split_kernel(const NetLayer<floa
                 reinterpret_cast<u2v*>(&S[buffer][p][wk >> 1][32 * j + wc])[wk & 1] = u2v{lo[p], hi[p]};
         }
     };
-    f32x16 acc[kNB];
+    f32x16 acc[kNB], apart[kApart ? kNB : 1];
+    auto& small = [&]() -> f32x16(&)[kNB] {
+        if constexpr (kApart) return apart;
+        else return acc;
+    }();
 #pragma unroll
-    for (int j = 0; j < kNB; ++j) acc[j] = f32x16(0.f);
+    for (int j = 0; j < kNB; ++j) acc[j] = small[j] = f32x16(0.f);
     const int chunks = K / 32;
     fetch(0);
     stage(0);
@@ -375,20 +385,24 @@ __global__ __launch_bounds__(256, 3) void layer_split_kernel(const NetLayer<floa
                 split_pair(v[2 * (e & 1)], v[2 * (e & 1) + 1], p[0], p[1], p[2]);
                 xs[0][e] = p[0], xs[1][e] = p[1], xs[2][e] = p[2];
             }
-            auto mul = [&](int i, int p) {
+            auto mul = [&](f32x16 (&to)[kNB], int i, int p) {
 #pragma unroll
                 for (int j = 0; j < kNB; ++j)
-                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xs[i]),
-                                                                     __builtin_bit_cast(bf16x8, S[c & 1][p][2 * s + half][32 * j + l32]), acc[j], 0, 0, 0);
+                    to[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xs[i]),
+                                                                    __builtin_bit_cast(bf16x8, S[c & 1][p][2 * s + half][32 * j + l32]), to[j], 0, 0, 0);
             };
-            mul(0, 2);
-            mul(1, 1);
-            mul(0, 1);
-            mul(2, 0);
-            mul(1, 0);
-            mul(0, 0);
+            mul(small, 0, 2);
+            mul(small, 1, 1);
+            mul(small, 0, 1);
+            mul(small, 2, 0);
+            mul(small, 1, 0);
+            mul(acc, 0, 0);
         }
         if (c + 1 < chunks) stage((c + 1) & 1);
+    }
+    if constexpr (kApart) {
+#pragma unroll
+        for (int j = 0; j < kNB; ++j) acc[j] += small[j];
     }
     // element v of a block: row 8 (v / 4) + 4 half + v % 4, column kNB l32 + (the block's number)
     const int cols = ct * kCols + kNB * l32;
@@ -655,10 +669,11 @@ hipError_t launch_net_layer(NetLayer<T> a, bool trans, hipStream_t stream)
         // Split products from half a workgroup of 128 x 64 per compute unit on (us, float32 instructions -> split): 3,000 rows
         // 256 -> 256 9.2 -> 12.1 (96 tiles), 128 -> 384 transposed 12.6 -> 9.0 (144); 12,000 rows 384 -> 128 22.9 -> 16.8
         // (188), 128 -> 64 5.9 -> 8.5 (94).  128 columns instead of 64 from two such workgroups per compute unit on:
-        // 48,000 rows 256 -> 256 43.9 -> 38.4 (750 tiles), 384 -> 128 35.3 -> 34.4 (375), 12,000 rows 23.7 -> 23.4 (188).
+        // 48,000 rows 256 -> 256 43.9 -> 38.4 (750 tiles), 384 -> 128 35.3 -> 34.4 (375), 12,000 rows 23.7 -> 23.4 (188); and
+        // only for output widths that are multiples of 64, whose sums may be rounded as often as that form's are.
         const int64_t row_tiles = (rows + kWideRows - 1) / kWideRows;
         if (whole && a.k % 32 == 0 && a.n_out >= 64 && row_tiles * ((a.n_out + 63) / 64) >= 128) {
-            if (row_tiles * ((a.n_out + 127) / 128) >= 512) launch_split<4>(a, trans, stream);
+            if (a.n_out % 64 == 0 && row_tiles * ((a.n_out + 127) / 128) >= 512) launch_split<4>(a, trans, stream);
             else launch_split<2>(a, trans, stream);
             return hipGetLastError();
         }
