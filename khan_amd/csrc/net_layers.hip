@@ -300,21 +300,20 @@ __global__ __launch_bounds__(256) void layer_kernel(const NetLayer<T> a, int tot
 // Per chunk a wavefront issues 48 matrix instructions (1,536 cycles; kNB = 4) and 250 vector ones (1,000), most of them
 // splitting, and the two hide each other only in part: 172 TFLOP/s where the float32 instructions gave 70 (96,000 rows
 // 256 -> 256: 139 -> 73 us; 48,000 rows 73 -> 38; transposed 78 -> 40).
-// With 64 columns the five small partial products have accumulators of their own (kApart): the large sum is then rounded
-// once in 16 k instead of six times, a layer's distance from float64 falls to 0.4 of the float32 library product's, and it
-// costs nothing (12,000 rows 384 -> 128: 17.9 -> 17.8 us; 47,000 rows 128 -> 64: 13.0 -> 12.9).  With 128 columns there are no
-// registers for them at three workgroups per compute unit (two: deep networks on 47,000 rows 1,790 -> 1,950 us): the sums
-// there are rounded as often as those of dense_first.hip's kernel, and the form is kept to the widths that kernel takes.
+// kApart (64 columns): the five small partial products have accumulators of their own.  The large sum is then rounded once in
+// 16 k instead of six times, and a layer's distance from float64 is 0.4 of the float32 library product's, where without it
+// it can lie above (values of 384-192-100-8-1 networks on 47,000 rows: library 2.17e-7, without 2.40e-7, with 2.12e-7).  It
+// costs nothing with 64 columns (12,000 rows 384 -> 128: 17.9 -> 17.8 us); with 128 there are no registers for it at three
+// workgroups per compute unit (two: deep networks on 47,000 rows 1,790 -> 1,950 us).
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 constexpr int kWideRows = 128;
 
-template <int kNB, bool kTrans>
+template <int kNB, bool kTrans, bool kApart>
 __global__ __launch_bounds__(256, 3) void layer_split_kernel(const NetLayer<float> a, int row_tiles)
 {
     typedef Vec<float, kNB> vec;
     constexpr int kCols = 32 * kNB;
-    constexpr bool kApart = kNB == 2;
     __shared__ u4v S[2][3][4][kCols + 2];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l32 = lane & 31, half = lane >> 5;
@@ -641,15 +640,15 @@ void launch_layer_kernel(NetLayer<T>& a, bool trans, bool whole, hipStream_t str
     }
 }
 
-template <int kNB>
+template <int kNB, bool kApart>
 void launch_split(NetLayer<float>& a, bool trans, hipStream_t stream)
 {
     a.col_tiles = (a.n_out + 32 * kNB - 1) / (32 * kNB);
     int total = 0;
     for (int t = 0; t < 4; ++t) a.tile_end[t] = total += (a.n[t] + kWideRows - 1) / kWideRows;
     const dim3 grid(static_cast<unsigned>((total + 7) / 8 * 8 * a.col_tiles));
-    if (trans) layer_split_kernel<kNB, true><<<grid, dim3(256), 0, stream>>>(a, total);
-    else layer_split_kernel<kNB, false><<<grid, dim3(256), 0, stream>>>(a, total);
+    if (trans) layer_split_kernel<kNB, true, kApart><<<grid, dim3(256), 0, stream>>>(a, total);
+    else layer_split_kernel<kNB, false, kApart><<<grid, dim3(256), 0, stream>>>(a, total);
 }
 
 }  // namespace
@@ -669,12 +668,14 @@ hipError_t launch_net_layer(NetLayer<T> a, bool trans, hipStream_t stream)
         // Split products from half a workgroup of 128 x 64 per compute unit on (us, float32 instructions -> split): 3,000 rows
         // 256 -> 256 9.2 -> 12.1 (96 tiles), 128 -> 384 transposed 12.6 -> 9.0 (144); 12,000 rows 384 -> 128 22.9 -> 16.8
         // (188), 128 -> 64 5.9 -> 8.5 (94).  128 columns instead of 64 from two such workgroups per compute unit on:
-        // 48,000 rows 256 -> 256 43.9 -> 38.4 (750 tiles), 384 -> 128 35.3 -> 34.4 (375), 12,000 rows 23.7 -> 23.4 (188); and
-        // only for output widths that are multiples of 64, whose sums may be rounded as often as that form's are.
+        // 48,000 rows 256 -> 256 43.9 -> 38.4 (750 tiles), 384 -> 128 35.3 -> 34.4 (375), 12,000 rows 23.7 -> 23.4 (188).
+        // Output widths that are multiples of 64 are those that dense_first.hip's split products take, with sums rounded as
+        // often as here; others are measured against float32 sums, which kApart stays below.
         const int64_t row_tiles = (rows + kWideRows - 1) / kWideRows;
         if (whole && a.k % 32 == 0 && a.n_out >= 64 && row_tiles * ((a.n_out + 63) / 64) >= 128) {
-            if (a.n_out % 64 == 0 && row_tiles * ((a.n_out + 127) / 128) >= 512) launch_split<4>(a, trans, stream);
-            else launch_split<2>(a, trans, stream);
+            if (a.n_out % 64) launch_split<2, true>(a, trans, stream);
+            else if (row_tiles * ((a.n_out + 127) / 128) >= 512) launch_split<4, false>(a, trans, stream);
+            else launch_split<2, false>(a, trans, stream);
             return hipGetLastError();
         }
     }
