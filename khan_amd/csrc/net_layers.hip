@@ -454,8 +454,22 @@ __global__ __launch_bounds__(256) void top_kernel(const NetTop<T> a, int total)
 // sixteen each; a lane's 16 bytes of a row are kVec of the tile's rows (left) or columns (right), the four groups of lanes
 // hold four rows: one load of each operand per kVec^2 matrix instructions.  The wavefronts' sums meet in LDS, the
 // workgroups' in memory, where grad_sum_kernel adds them up in a fixed order: no atomics, the same bits every time.
+// The column sums (the biases' gradients, factors of random sign that cancel) are formed by the first row of tiles alone and
+// carry their rounding errors along: added up plainly, 64 rows to a lane, they were 2e-7 off where a library sum is 4e-8 off
+// (124 -> 126 us a launch at 35,000 rows).
 // 62 TFLOP/s of the float32 instructions' 153 at 35,000 rows of 384-128-128-64-1 (82 us).  The compiler's overlap of the
 // unrolled loop's loads with the products beats four row groups loaded ahead by hand (104 us a launch there).
+// sum += x, its rounding error added to `lost` (Knuth's two-sum)
+template <typename V>
+__device__ __forceinline__ void add_exactly(V& sum, V& lost, V x)
+{
+    const V s = sum + x, b = s - sum;
+    lost += (sum - (s - b)) + (x - b);
+    sum = s;
+}
+template <typename T>
+__device__ __forceinline__ T with_lost(T sum, T lost) { return isfinite(sum) ? sum + lost : sum; }      // (lost is NaN beside an infinite sum)
+
 template <typename T>
 struct GradLds {
     static constexpr int kVec = MatrixOp<T>::kVec;
@@ -482,7 +496,7 @@ __device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __rest
     for (int i = 0; i < V; ++i)
 #pragma unroll
         for (int j = 0; j < V; ++j) acc[i][j] = acc_t(T(0));
-    Vec<T> bias = Vec<T>(T(0));
+    Vec<T> bias = Vec<T>(T(0)), bias_lost = Vec<T>(T(0));
     const int ci = i0 + V * l16, cj = j0 + V * l16;
     const int li = kWhole ? min(ci, K - V) : ci, lj = kWhole ? min(cj, N - V) : cj;
 #pragma unroll 1
@@ -507,7 +521,7 @@ __device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __rest
                 x[e] = live ? x[e] : T(0);
                 y[e] = live ? y[e] * s : T(0);
             }
-            if (pair == 0) bias += y;
+            if (pair == 0 && i0 == 0) add_exactly(bias, bias_lost, y);
 #pragma unroll
             for (int i = 0; i < V; ++i)
 #pragma unroll
@@ -533,7 +547,7 @@ __device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __rest
     };
 #pragma unroll
     for (int e = 0; e < V; ++e) {
-        T b = bias[e];
+        T b = with_lost(bias[e], bias_lost[e]);
         b += __shfl_xor(b, 16, 64);
         b += __shfl_xor(b, 32, 64);
         if (grp == 0) S.bias[wave][V * l16 + e] = b;
@@ -609,10 +623,10 @@ __global__ __launch_bounds__(256) void grad_sum_kernel(const NetGrads<T> a, cons
         within = (i % kSide) * kSide + j % kSide;
     }
     const T* p = partial + static_cast<size_t>((job == 0 ? 0 : a.job_end[job - 1]) + tile) * kStride + within;
-    T sum = T(0);
+    T sum = T(0), lost = T(0);
 #pragma unroll 4
-    for (int s = 0; s < splits; ++s) sum += p[static_cast<size_t>(s) * tiles * kStride];
-    a.out[e] = sum;
+    for (int s = 0; s < splits; ++s) add_exactly(sum, lost, p[static_cast<size_t>(s) * tiles * kStride]);
+    a.out[e] = with_lost(sum, lost);
 }
 
 template <typename T>

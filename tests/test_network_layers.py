@@ -174,3 +174,32 @@ def test_celu_of_small_and_large_arguments():
         assert ((got - want).abs() <= 2.0 ** -21 * want.abs())[known & ~torch.isinf(want)].all()
         assert (got < 0)[known & (arg < 0)].all() and torch.isnan(got[torch.isnan(arg)]).all()
         assert first == 0 or got[-1] == float("inf")
+
+
+@pytest.mark.parametrize("dtype,unit", [(torch.float32, 2.0 ** -24), (torch.float64, 2.0 ** -53)])
+def test_bias_gradients_of_many_rows(dtype, unit):
+    """Bias gradients are sums over all rows of factors of either sign: the output layer's of four types' 20,000 to 50,000 rows,
+    ten sets of factors, lie within two roundings of the sums (2-norm; 0.9 measured in both precisions, 3.0 in single precision
+    where the lanes' sums drop their rounding errors).  An infinite factor gives an infinity of its sign, not NaN."""
+    from khan_amd import _native
+    widths, rows = [8, 64, 1], (50000, 40000, 30000, 20000)
+    rng = np.random.default_rng(8)
+    flat = torch.from_numpy(rng.standard_normal(4 * sum((k + 1) * m for k, m in zip(widths, widths[1:])))).to(dtype).cuda().requires_grad_(True)
+    xs = [torch.from_numpy(rng.standard_normal(n * 8)).to(dtype).cuda() for n in rows]
+    values = _native.load().network_autograd(flat, xs, widths, ALPHA)
+    got, want = [], []
+
+    def of_outputs(factors):
+        g, = torch.autograd.grad(values, flat, [torch.from_numpy(f).cuda() for f in factors], retain_graph=True)
+        return g[-4:].cpu().numpy().astype(np.longdouble)
+
+    for _ in range(10):
+        factors = [torch.from_numpy(rng.standard_normal(n)).to(dtype).numpy() for n in rows]
+        got.append(of_outputs(factors))
+        want.append([f.astype(np.longdouble).sum() for f in factors])
+    got, want = np.array(got), np.array(want)
+    off = float(np.sqrt(((got - want) ** 2).sum() / (want ** 2).sum())) / unit
+    print("bias gradients:", dtype, "%.3g units" % off, flush=True)
+    assert off <= 2.0
+    factors[1][17] = float("inf")
+    assert np.isposinf(of_outputs(factors)[1])
