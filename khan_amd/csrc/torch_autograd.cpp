@@ -193,6 +193,8 @@ Tensor mol_energy_autograd(const std::vector<Tensor>& o, const Tensor& types, co
 struct Net {
     Saved widths;
     double alpha;
+    int64_t live_from = 0;      // the parameters of earlier layers are constants: no gradients are formed for them
+    uint32_t live() const { return ((1u << layers()) - 1u) & ~((1u << live_from) - 1u); }
     int layers() const { return static_cast<int>(widths.size()) - 1; }        // products, the output layer included
     int64_t weight_at(int l, int t) const
     {
@@ -408,7 +410,7 @@ struct Pass {
     Tensor first_order(const variable_list& acts, const variable_list& d, const Four& scale) const
     {
         khan_net_grads g = grads(scale);
-        g.first = (1u << net.layers()) - 1u;
+        g.first = net.live();
         g.scale_first = 1;
         for (int l = 0; l <= L; ++l) {
             if (l > 0) g.left[l] = ptr<char>(acts[l - 1]);
@@ -471,7 +473,16 @@ variable_list library_grad(const variable_list& outputs, const variable_list& in
     return out;
 }
 
-Net net_of(AutogradContext* ctx) { return Net{ctx->saved_data["widths"].toIntVector(), ctx->saved_data["alpha"].toDouble()}; }
+Net net_of(AutogradContext* ctx)
+{
+    return Net{ctx->saved_data["widths"].toIntVector(), ctx->saved_data["alpha"].toDouble(), ctx->saved_data["live_from"].toInt()};
+}
+void keep(AutogradContext* ctx, const Net& net)
+{
+    ctx->saved_data["widths"] = net.widths;
+    ctx->saved_data["alpha"] = net.alpha;
+    ctx->saved_data["live_from"] = net.live_from;
+}
 
 Four or_zeros(const Rows& rows, const Tensor& flat, const variable_list& g, int from, int64_t width)
 {
@@ -488,11 +499,9 @@ Four or_zeros(const Rows& rows, const Tensor& flat, const variable_list& g, int 
 struct NetRowsFn : Function<NetRowsFn> {
     // inputs: flat, x[4], s[4]; saved behind them: the activations and d_1 .. d_L
     static variable_list forward(AutogradContext* ctx, const Tensor& flat, const Tensor& x0, const Tensor& x1, const Tensor& x2, const Tensor& x3,
-                                 const Tensor& s0, const Tensor& s1, const Tensor& s2, const Tensor& s3, const variable_list& kept_acts, Saved widths,
-                                 double alpha)
+                                 const Tensor& s0, const Tensor& s1, const Tensor& s2, const Tensor& s3, const variable_list& kept_acts, const Net& net)
     {
         const Unrecorded quiet;
-        const Net net{widths, alpha};
         const Params params(net, flat);
         const Rows rows = rows_of(net, params, x0, x1, x2, x3);
         const Pass p{net, rows, params};
@@ -505,8 +514,7 @@ struct NetRowsFn : Function<NetRowsFn> {
         save.insert(save.end(), acts.begin(), acts.end());
         save.insert(save.end(), d.begin(), d.end());
         ctx->save_for_backward(save);
-        ctx->saved_data["widths"] = widths;
-        ctx->saved_data["alpha"] = alpha;
+        keep(ctx, net);
         const Four xs = {x0, x1, x2, x3};
         variable_list res;
         for (int t = 0; t < 4; ++t) res.push_back(out[t].reshape(xs[t].sizes()));
@@ -518,7 +526,7 @@ struct NetRowsFn : Function<NetRowsFn> {
         const Net net = net_of(ctx);
         const Tensor flat = saved[0];
         const variable_list x(saved.begin() + 1, saved.begin() + 5), s(saved.begin() + 5, saved.begin() + 9);
-        variable_list out(12);
+        variable_list out(11);
         if (at::GradMode::is_enabled()) {
             variable_list in = {flat};
             in.insert(in.end(), x.begin(), x.end());
@@ -604,8 +612,8 @@ struct NetRowsFn : Function<NetRowsFn> {
         }
         if (ctx->needs_input_grad(0)) {
             khan_net_grads g = p.grads(scale);
-            g.first = (1u << L) - 1u;                      // the hidden layers: a^T q ...
-            g.second = (1u << (L + 1)) - 1u;               // ... and all: a'^T (s d), d = 1 in the output layer
+            g.first = net.live() & ((1u << L) - 1u);       // the hidden layers: a^T q ...
+            g.second = net.live();                         // ... and all: a'^T (s d), d = 1 in the output layer
             g.scale_second = 1;
             Pass::set(g.x2, v);
             for (int l = 0; l <= L; ++l) {
@@ -627,10 +635,9 @@ struct NetRowsFn : Function<NetRowsFn> {
 // The values of the four types' rows as a function of the parameters and the rows.
 struct NetFn : Function<NetFn> {
     static variable_list forward(AutogradContext* ctx, const Tensor& flat, const Tensor& x0, const Tensor& x1, const Tensor& x2, const Tensor& x3,
-                                 Saved widths, double alpha, bool graph)
+                                 const Net& net, bool graph)
     {
         const Unrecorded quiet;
-        const Net net{widths, alpha};
         const Params params(net, flat);
         const Rows rows = rows_of(net, params, x0, x1, x2, x3);
         const Pass p{net, rows, params};
@@ -642,8 +649,7 @@ struct NetFn : Function<NetFn> {
             save.insert(save.end(), acts.begin(), acts.end());
             save.push_back(d);
             ctx->save_for_backward(save);
-            ctx->saved_data["widths"] = widths;
-            ctx->saved_data["alpha"] = alpha;
+            keep(ctx, net);
         }
         return {values[0], values[1], values[2], values[3]};
     }
@@ -655,7 +661,7 @@ struct NetFn : Function<NetFn> {
         const variable_list x(saved.begin() + 1, saved.begin() + 5);
         const bool need_x = ctx->needs_input_grad(1) || ctx->needs_input_grad(2) || ctx->needs_input_grad(3) || ctx->needs_input_grad(4);
         const bool need_p = ctx->needs_input_grad(0);
-        variable_list out(8);
+        variable_list out(7);
         if (at::GradMode::is_enabled() && need_p) {
             const auto g = library_grad(library_values(net, flat, x), {flat, x[0], x[1], x[2], x[3]}, gs);
             for (int k = 0; k < 5; ++k) out[k] = g[k];
@@ -667,7 +673,7 @@ struct NetFn : Function<NetFn> {
             variable_list s(4);
             for (int t = 0; t < 4; ++t) s[t] = gs[t].defined() ? gs[t].contiguous() : at::zeros({rows.n[t]}, flat.options());
             const variable_list kept_acts(saved.begin() + 5, saved.end());
-            const auto g = NetRowsFn::apply(flat, x[0], x[1], x[2], x[3], s[0], s[1], s[2], s[3], kept_acts, net.widths, net.alpha);
+            const auto g = NetRowsFn::apply(flat, x[0], x[1], x[2], x[3], s[0], s[1], s[2], s[3], kept_acts, net);
             for (int t = 0; t < 4; ++t) out[1 + t] = g[t];
             return out;
         }
@@ -686,12 +692,15 @@ struct NetFn : Function<NetFn> {
     }
 };
 
-std::vector<Tensor> network_autograd(const Tensor& flat, const std::vector<Tensor>& x, Saved widths, double alpha)
+// live_from: the parameters of earlier layers are constants
+std::vector<Tensor> network_autograd(const Tensor& flat, const std::vector<Tensor>& x, Saved widths, double alpha, int64_t live_from)
 {
     same_size(x.size() == 4, "four feature buckets");
+    const Net net{widths, alpha, live_from};
+    same_size(live_from >= 0 && live_from <= net.layers(), "live_from must be a layer's number, or the number of layers");
     bool graph = flat.requires_grad();
     for (const Tensor& v : x) graph |= v.requires_grad();
-    return NetFn::apply(flat, x[0], x[1], x[2], x[3], widths, alpha, graph && at::GradMode::is_enabled());
+    return NetFn::apply(flat, x[0], x[1], x[2], x[3], net, graph && at::GradMode::is_enabled());
 }
 
 // The parameters of a network (tensors of any shape) end to end in one array.
@@ -913,7 +922,7 @@ void bind_autograd(py::module_& m)
     m.def("featurize_autograd", &featurize_autograd);
     m.def("ani_charge_autograd", &ani_charge_autograd);
     m.def("mol_energy_autograd", &mol_energy_autograd);
-    m.def("network_autograd", &network_autograd);
+    m.def("network_autograd", &network_autograd, py::arg("flat"), py::arg("x"), py::arg("widths"), py::arg("alpha"), py::arg("live_from") = 0);
     m.def("flatten", &flatten);
     m.def("network_forward", &network_forward);
     m.def("network_rows", &network_rows);

@@ -174,13 +174,21 @@ class MoleculeNN:
         """Per-type flat feature buckets -> the four per-type output vectors [acs[t]] (nn.py:165-175)."""
         if not self.layer_launches():
             return [self.atom_type_outputs(t, f.reshape(-1, FEATURE_SIZE)) for t, f in enumerate(atom_type_features)]
-        # in single precision inference is the default: the weights are constants
-        live = torch.is_grad_enabled() and (self.weights_need_grad or self.dtype == torch.float64 or self.kernel_layers() == 0)
-        native = _native.load()
-        flat = native.flatten(self._in_flat_order())
-        if not live:
-            flat = flat.detach()
-        return native.network_autograd(flat, list(atom_type_features), self.layer_sizes, 0.1)
+        native, ps, layers = _native.load(), self._in_flat_order(), len(self.layer_sizes) - 1
+        live = self._live_from()
+        ps = [p if k // 4 % layers >= live else p.detach() for k, p in enumerate(ps)]
+        return native.network_autograd(native.flatten(ps), list(atom_type_features), self.layer_sizes, 0.1, live)
+
+    def _live_from(self):
+        """The first layer whose parameters are differentiated by.  In single precision inference is the default: unless
+        `weights_need_grad` the leading `kernel_layers` are constants, and with them an output layer right behind the last
+        of them where that has width 64 (it rides in that layer's launch in `ops.dense_head`)."""
+        layers, constant = len(self.layer_sizes) - 1, self.kernel_layers()
+        if not torch.is_grad_enabled():
+            return layers
+        if self.weights_need_grad:
+            return 0
+        return layers if constant == layers - 1 and self.layer_sizes[-2] == 64 else constant
 
 
 class AniModel:

@@ -203,3 +203,30 @@ def test_bias_gradients_of_many_rows(dtype, unit):
     assert off <= 2.0
     factors[1][17] = float("inf")
     assert np.isposinf(of_outputs(factors)[1])
+
+
+@pytest.mark.parametrize("layers,live", [((256, 64, 8, 1), 2), ((128, 128, 1), 2), ((128, 64, 1), 3), ((100, 1), 0)])
+def test_parameters_behind_the_constant_layers_have_gradients(layers, live):
+    """Without `weights_need_grad` the leading layers of a float32 network are constants and those behind them are not: their
+    gradients, and those of a loss on the row gradients, are what `weights_need_grad` gives, and no other parameter has one."""
+    from khan_amd import model
+    net = model.MoleculeNN(layers, model.celu, torch.float32, "cuda:0", seed=2)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    feats = [torch.rand(n * 384, device="cuda", generator=gen).requires_grad_(True) for n in (300, 0, 17, 64)]
+    params = net.parameters()
+    results = []
+    for need in (False, True):
+        net.weights_need_grad = need
+        energy = sum(v.sum() for v in net.type_outputs(feats))
+        first = torch.autograd.grad(energy, params, allow_unused=True, retain_graph=True) if energy.requires_grad else [None] * len(params)
+        rows = torch.autograd.grad(energy, feats, create_graph=True)
+        loss = sum((r ** 2).sum() for r in rows)
+        second = torch.autograd.grad(loss, params, allow_unused=True) if loss.requires_grad else [None] * len(params)
+        results.append((first, second))
+    layer_of = [k for t in model.TYPE_MAP for k, _ in enumerate(net.names[t]) for _ in (0, 1)]
+    for (some, every) in zip(*results):
+        for k, (a, b) in enumerate(zip(some, every)):
+            if layer_of[k] < live:
+                assert a is None
+            else:
+                assert a is not None and torch.equal(a, b)
