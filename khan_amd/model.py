@@ -18,6 +18,7 @@ import os
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from . import _native
 
@@ -70,6 +71,16 @@ def parameter_names(prefix, layer_sizes):
             rows.append((prefix + "W" + name + ":0", prefix + "b" + name + ":0", x, y))
         out[t] = rows
     return out
+
+
+def _transformed(tensors):
+    """True where the tensors stand for something else than their elements: under a tracer or compiler, torch.func's
+    transforms, forward-mode differentiation, a dispatch mode, or as a subclass.  Launches would see none of that;
+    library operations do."""
+    return (torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()
+            or torch._C._functorch.peek_interpreter_stack() is not None or forward_ad._current_level >= 0
+            or torch._C._len_torch_dispatch_stack() > 0
+            or any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in tensors))
 
 
 class MoleculeNN:
@@ -172,7 +183,7 @@ class MoleculeNN:
 
     def type_outputs(self, atom_type_features):
         """Per-type flat feature buckets -> the four per-type output vectors [acs[t]] (nn.py:165-175)."""
-        if not self.layer_launches():
+        if not self.layer_launches() or _transformed(atom_type_features):
             return [self.atom_type_outputs(t, f.reshape(-1, FEATURE_SIZE)) for t, f in enumerate(atom_type_features)]
         native, ps, layers = _native.load(), self._in_flat_order(), len(self.layer_sizes) - 1
         live = self._live_from()

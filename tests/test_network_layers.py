@@ -230,3 +230,36 @@ def test_parameters_behind_the_constant_layers_have_gradients(layers, live):
                 assert a is None
             else:
                 assert a is not None and torch.equal(a, b)
+
+
+def test_networks_under_tracing_and_transforms():
+    """Forward mode, vmap, torch.func's gradients and tracers go through type_outputs as library operations did: a launch's values
+    with the tangents, batches and graphs of those operations.  Float64: 1e-12 for sums of a few hundred products."""
+    from khan_amd import model
+    net = model.MoleculeNN((32, 16, 1), model.celu, torch.float64, "cuda:0", seed=2)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    rand = lambda *shape: torch.rand(*shape, device="cuda", generator=gen, dtype=torch.float64)
+    rows = (5, 0, 3, 2)
+    feats, tangents = [rand(n * 384) for n in rows], [rand(n * 384) for n in rows]
+    energy = lambda *f: sum(v.sum() for v in net.type_outputs(f))
+    plain = lambda *f: sum(net.atom_type_outputs(t, x.reshape(-1, 384)).sum() for t, x in enumerate(f))
+    close = lambda a, b: bool(((a - b).detach().abs().max() <= 1e-12 * (1 + b.detach().abs().max())).item())
+    grads = torch.func.grad(plain, argnums=(0, 2))(*feats)
+    leaves = [f.clone().requires_grad_(True) for f in feats]
+    directional = sum((g * v).sum() for g, v in zip(torch.autograd.grad(plain(*leaves), leaves), tangents))
+    # forward mode, both forms
+    value, tangent = torch.func.jvp(energy, tuple(feats), tuple(tangents))
+    assert close(value, plain(*feats)) and close(tangent, directional)
+    with torch.autograd.forward_ad.dual_level():
+        duals = [torch.autograd.forward_ad.make_dual(f, v) for f, v in zip(feats, tangents)]
+        assert close(torch.autograd.forward_ad.unpack_dual(energy(*duals)).tangent, directional)
+    assert all(close(a, b) for a, b in zip(torch.func.grad(energy, argnums=(0, 2))(*feats), grads))
+    batch = [torch.stack([f, v]) for f, v in zip(feats, tangents)]
+    assert all(close(a, b) for a, b in zip(torch.vmap(energy)(*batch), (plain(*feats), plain(*tangents))))
+    # tracers record operations, not the values of one call (torch.jit takes no constants that require gradients)
+    for p in net.parameters():
+        p.requires_grad_(False)
+    assert close(torch.jit.trace(energy, tuple(feats), check_trace=False)(*tangents), plain(*tangents))
+    from torch.fx.experimental.proxy_tensor import make_fx
+    assert close(make_fx(energy)(*feats)(*tangents), plain(*tangents))
+    assert close(energy(*feats), plain(*feats))
