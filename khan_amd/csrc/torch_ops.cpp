@@ -24,25 +24,25 @@ static void init(const std::string& path, py::object error_type)
     khan_error = error_type.release().ptr();
 }
 
-// four ints from a tensor (a device tensor is copied) or a sequence
+// four ints from a tensor (a device tensor is copied) or a sequence, whatever int() takes; fractions are cut off
 Counts counts4(const py::object& o, const char* what)
 {
     Counts c{};
     if (THPVariable_Check(o.ptr())) {
-        const Tensor t = THPVariable_Unpack(o.ptr()).detach().cpu().to(at::kInt).contiguous();
+        Tensor t = THPVariable_Unpack(o.ptr());
+        if (t.is_cuda() || t.scalar_type() != at::kInt || !t.is_contiguous()) t = t.detach().cpu().to(at::kInt).contiguous();
         same_size(t.numel() == 4, what);
         std::copy_n(t.data_ptr<int32_t>(), 4, c.v);
     } else {
         int k = 0;
         for (const auto& item : o) {
             same_size(k < 4, what);
-            c.v[k++] = item.cast<int32_t>();
+            c.v[k++] = PyLong_CheckExact(item.ptr()) ? item.cast<int32_t>() : py::int_(py::reinterpret_borrow<py::object>(item)).cast<int32_t>();
         }
         same_size(k == 4, what);
     }
     return c;
 }
-
 
 // ---------------------------------------------------------------------------------------------- preparation
 // -> (macs, mos, scatter_idxs, gather_idxs, atom_counts, order), slices of one allocation

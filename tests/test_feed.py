@@ -51,3 +51,21 @@ def test_energies_and_gradients_from_one_pass(fit_charges, dtype):
     for (e, g), e_ref, g_ref in zip(both, energies, gradients):
         assert isinstance(e, float) and abs(e - e_ref) <= tol * (1.0 + abs(e_ref))
         assert g.shape == g_ref.shape and g.dtype == g_ref.dtype and np.abs(g - g_ref).max() <= tol * (1.0 + np.abs(g_ref).max())
+
+
+@pytest.mark.parametrize("of", [float, np.float32, np.int64, lambda v: torch.tensor(v), lambda v: torch.tensor(float(v))])
+def test_counts_of_any_kind_of_number(of):
+    """Atom counts and class totals as int() takes them: Python and numpy floats, zero-dimensional tensors, and whole tensors of
+    another type."""
+    m = _molecules([9, 40, 70])
+    b = next(iter(batching.DeviceFeeder(batching.RawDataset(m, [0.0] * 3), 3))).wait()
+    acs, order, classes = b.host_counts()
+    args = (b.xs, b.ys, b.zs, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs)
+    want = ops.featurize(*args, list(acs), order=order, size_classes=list(classes))
+    for counts, totals in (([of(v) for v in acs], [of(v) for v in classes]), (torch.tensor(acs, dtype=torch.float64), np.array(classes, dtype=np.float32))):
+        got = ops.featurize(*args, counts, order=order, size_classes=totals)
+        assert all(torch.equal(a, b) for a, b in zip(got, want))
+    with pytest.raises(ValueError):
+        ops.featurize(*args, [float(v) for v in acs] + [0.0], order=order)
+    with pytest.raises(Exception):
+        ops.featurize(*args, [float("nan")] * 4, order=order)
