@@ -214,20 +214,28 @@ class DeviceBatch:
         self.memory = self.sizes = self.totals = None    # of a batch from the host: its one buffer, molecule sizes, counts
 
     def host_counts(self):
-        """-> (atoms per type [4], the size order on the device, molecules per size class [4] on the host): what the
-        host has to know before it can launch the passes.  A batch from the host brings them along; otherwise the sort
+        """-> (atoms per type, a list of 4; the size order on the device; molecules per size class, int32[4] on the host): what
+        the host has to know before it can launch the passes.  A batch from the host brings them along; otherwise the sort
         writes them to pinned memory, and this waits for it.  The numbers may be there before the batch's arrays are, so
         the current stream is made to wait for those: what it is given from here on finds them (work for a further stream:
         `wait()` there).  Waiting for them on the host instead costs 8 us: 74 -> 83 us for the featurizer's step on 1,024
         organic molecules."""
+        acs, order, classes = self._counts()
+        if isinstance(classes, tuple):
+            import torch
+            classes = torch.tensor(classes, dtype=torch.int32)
+        return acs, order, classes
+
+    def _counts(self):
+        """`host_counts()`, with the class totals of a batch from the host as they are held (a tuple; a tensor costs 10 us)."""
         self._join()
         if self.totals is not None:
-            return list(self.totals[0]), self.size_order, list(self.totals[1])
+            return list(self.totals[0]), self.size_order, self.totals[1]
         counts = _native.load().wait_for_counts(self.counts_pinned)
         if counts is None:
             self.ready.synchronize()
-            counts = self.counts_pinned.tolist()
-        return counts[0:4], self.size_order, counts[4:8]
+            counts = self.counts_pinned[0:4].tolist(), self.counts_pinned[4:8].clone()
+        return counts[0], self.size_order, counts[1]
 
     def host_sizes(self):
         """The molecules' sizes, a list on the host."""

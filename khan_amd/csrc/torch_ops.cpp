@@ -85,8 +85,9 @@ std::vector<Tensor> prepare_batch_into(const Tensor& mol_idxs, const Tensor& typ
     return out;
 }
 
-// The counts that prepare_batch writes to pinned memory, or None if they have not arrived within about a millisecond.  They
-// are on the host while the kernel that wrote them still ranks atoms, some microseconds before an event behind it.
+// The counts that prepare_batch writes to pinned memory (a list of the atom counts, a tensor of the class totals), or None if
+// they have not arrived within about a millisecond.  They are on the host while the kernel that wrote them still ranks atoms,
+// some microseconds before an event behind it.
 static py::object wait_for_counts(const Tensor& counts_pinned)
 {
     same_size(counts_pinned.scalar_type() == at::kInt && counts_pinned.numel() == 8 && counts_pinned.is_contiguous() && !counts_pinned.is_cuda(),
@@ -102,9 +103,13 @@ static py::object wait_for_counts(const Tensor& counts_pinned)
         for (int spin = 0; spin < 20000 && !arrived(); ++spin) __builtin_ia32_pause();
     }
     if (!arrived()) return py::none();
-    py::list out(8);
-    for (int k = 0; k < 8; ++k) PyList_SET_ITEM(out.ptr(), k, PyLong_FromLong(c[k]));
-    return out;
+    py::list acs(4);
+    const Tensor classes = at::empty({4}, at::kInt);
+    for (int k = 0; k < 4; ++k) {
+        PyList_SET_ITEM(acs.ptr(), k, PyLong_FromLong(c[k]));
+        classes.data_ptr<int32_t>()[k] = c[4 + k];
+    }
+    return py::make_tuple(acs, classes);
 }
 
 static std::vector<Tensor> prepare_batch(const Tensor& mol_idxs, const Tensor& types, int64_t n_mols, const c10::optional<Tensor>& counts_pinned)

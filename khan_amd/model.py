@@ -185,20 +185,22 @@ class MoleculeNN:
         """Per-type flat feature buckets -> the four per-type output vectors [acs[t]] (nn.py:165-175)."""
         if not self.layer_launches() or _transformed(atom_type_features):
             return [self.atom_type_outputs(t, f.reshape(-1, FEATURE_SIZE)) for t, f in enumerate(atom_type_features)]
-        native, ps, layers = _native.load(), self._in_flat_order(), len(self.layer_sizes) - 1
-        live = self._live_from()
-        ps = [p if k // 4 % layers >= live else p.detach() for k, p in enumerate(ps)]
+        native, ps, live = _native.load(), self._in_flat_order(), self._live_from()
+        if live > 0:
+            layers = len(self.layer_sizes) - 1
+            ps = [p if k // 4 % layers >= live else p.detach() for k, p in enumerate(ps)]
         return native.network_autograd(native.flatten(ps), list(atom_type_features), self.layer_sizes, 0.1, live)
 
     def _live_from(self):
         """The first layer whose parameters are differentiated by.  In single precision inference is the default: unless
         `weights_need_grad` the leading `kernel_layers` are constants, and with them an output layer right behind the last
         of them where that has width 64 (it rides in that layer's launch in `ops.dense_head`)."""
-        layers, constant = len(self.layer_sizes) - 1, self.kernel_layers()
+        layers = len(self.layer_sizes) - 1
         if not torch.is_grad_enabled():
             return layers
         if self.weights_need_grad:
             return 0
+        constant = self.kernel_layers()
         return layers if constant == layers - 1 and self.layer_sizes[-2] == 64 else constant
 
 
@@ -260,7 +262,7 @@ class AniModel:
             if joined:
                 parts.append(torch.cat([energies, energies.new_empty(-b.n_mols % 64)] + parts))
             return [energies] + parts
-        acs, order, classes = b.host_counts()
+        acs, order, classes = b._counts()
         # Networks beside a charge network run layer by layer: products of all 24 bits over float32's range, where the
         # one-launch kernel's operands keep 2^-24 of their size between 6e-5 and 65,504.
         alone = self.charge is None
@@ -272,7 +274,7 @@ class AniModel:
         """_energies for networks of library operations (other activations than CELU)."""
         from . import autograd
         xs, ys, zs = b.xs, b.ys, b.zs
-        acs, order, classes = b.host_counts()
+        acs, order, classes = b._counts()
         if need_grad:
             xs, ys, zs = (t.detach().clone().requires_grad_(True) for t in (xs, ys, zs))
         feats = autograd.featurize(xs, ys, zs, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs, acs,

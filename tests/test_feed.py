@@ -36,7 +36,8 @@ def test_feeder_takes_molecules_in_any_form(form, labelled, dtype):
             assert b.labels == labels and b.host_sizes() == macs.tolist()
             acs, _, classes = b.host_counts()
             assert acs == np.bincount(want[3], minlength=4).tolist()
-            assert classes == np.histogram(macs.cpu().numpy(), [0, 33, 65, 257, 10 ** 9])[0].tolist()
+            assert isinstance(classes, torch.Tensor) and classes.dtype == torch.int32
+            assert classes.tolist() == np.histogram(macs.cpu().numpy(), [0, 33, 65, 257, 10 ** 9])[0].tolist()
 
 
 @pytest.mark.parametrize("fit_charges", [False, True])
@@ -61,8 +62,8 @@ def test_counts_of_any_kind_of_number(of):
     b = next(iter(batching.DeviceFeeder(batching.RawDataset(m, [0.0] * 3), 3))).wait()
     acs, order, classes = b.host_counts()
     args = (b.xs, b.ys, b.zs, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs)
-    want = ops.featurize(*args, list(acs), order=order, size_classes=list(classes))
-    for counts, totals in (([of(v) for v in acs], [of(v) for v in classes]), (torch.tensor(acs, dtype=torch.float64), np.array(classes, dtype=np.float32))):
+    want = ops.featurize(*args, list(acs), order=order, size_classes=classes)
+    for counts, totals in (([of(v) for v in acs], [of(v) for v in classes.tolist()]), (torch.tensor(acs, dtype=torch.float64), np.array(classes, dtype=np.float32))):
         got = ops.featurize(*args, counts, order=order, size_classes=totals)
         assert all(torch.equal(a, b) for a, b in zip(got, want))
     with pytest.raises(ValueError):
