@@ -246,7 +246,7 @@ struct Params {
             const int l = static_cast<int>(k / 4) % net.layers();
             const bool weight = k / 4 < static_cast<size_t>(net.layers());
             const Tensor p = tensors[k].contiguous();
-            if (!p.is_cuda() || p.scalar_type() != dtype) throw py::type_error("the parameters must be CUDA tensors of one type");
+            if (!p.is_cuda() || p.scalar_type() != dtype) raise(PyExc_TypeError, "the parameters must be CUDA tensors of one type");
             same_size(p.numel() == (weight ? net.widths[l] * net.widths[l + 1] : net.widths[l + 1]),
                       "the parameters do not match the network's widths");
             held.push_back(p);
@@ -260,7 +260,7 @@ private:
     static void check_net(const Net& net)
     {
         if (net.widths.size() < 3 || net.layers() > KHAN_NET_MAX_LAYERS || net.widths.back() != 1)
-            throw py::value_error("a network of 2 to " + std::to_string(KHAN_NET_MAX_LAYERS) + " layers, the last of width 1");
+            raise(PyExc_ValueError, "a network of 2 to " + std::to_string(KHAN_NET_MAX_LAYERS) + " layers, the last of width 1");
     }
 };
 

@@ -37,14 +37,15 @@ struct Api {
 extern Api api;
 extern PyObject* khan_error;
 
+// A Python exception of that type; in a thread of the autograd engine (which does not hold the interpreter's lock) in the form
+// that the engine carries over to the thread that asked for the gradients.
+[[noreturn]] void raise(PyObject* type, const std::string& message);
+
 inline void check(int status)
 {
     if (status == KHAN_OK) return;
     const std::string detail = api.khan_last_hip_error();
-    const std::string msg = std::string("libkhan_aev: ") + api.khan_status_string(status) + (detail.empty() ? "" : " (" + detail + ")");
-    if (!PyGILState_Check()) throw std::runtime_error(msg);       // a thread of the autograd engine
-    PyErr_SetString(khan_error, msg.c_str());
-    throw py::error_already_set();
+    raise(khan_error, std::string("libkhan_aev: ") + api.khan_status_string(status) + (detail.empty() ? "" : " (" + detail + ")"));
 }
 
 // the launch, with the interpreter's lock (where this thread holds it) given back as a foreign-function call gives it back
@@ -65,16 +66,16 @@ inline khan_stream_t stream() { return c10::hip::getCurrentHIPStream().stream();
 
 inline void dev(const Tensor& t, at::ScalarType dtype, const char* name)
 {
-    if (!t.is_cuda()) throw py::type_error(std::string(name) + " must be a CUDA tensor");
+    if (!t.is_cuda()) raise(PyExc_TypeError, std::string(name) + " must be a CUDA tensor");
     if (t.scalar_type() != dtype)
-        throw py::type_error(std::string(name) + " must have dtype " + c10::toString(dtype) + ", got " + c10::toString(t.scalar_type()));
-    if (t.dim() != 1) throw py::value_error(std::string(name) + " must be rank 1 (flat), got rank " + std::to_string(t.dim()));
-    if (!t.is_contiguous()) throw py::value_error(std::string(name) + " must be contiguous");
+        raise(PyExc_TypeError, std::string(name) + " must have dtype " + c10::toString(dtype) + ", got " + c10::toString(t.scalar_type()));
+    if (t.dim() != 1) raise(PyExc_ValueError, std::string(name) + " must be rank 1 (flat), got rank " + std::to_string(t.dim()));
+    if (!t.is_contiguous()) raise(PyExc_ValueError, std::string(name) + " must be contiguous");
 }
 
 inline void same_size(bool ok, const char* what)
 {
-    if (!ok) throw py::value_error(what);
+    if (!ok) raise(PyExc_ValueError, what);
 }
 
 template <typename T>
@@ -86,7 +87,7 @@ T* ptr(const Tensor& t)
 inline at::ScalarType float_dtype(const Tensor& x, const char* what)
 {
     const auto dt = x.scalar_type();
-    if (dt != at::kFloat && dt != at::kDouble) throw py::type_error(std::string(what) + " must be float32 or float64, got " + c10::toString(dt));
+    if (dt != at::kFloat && dt != at::kDouble) raise(PyExc_TypeError, std::string(what) + " must be float32 or float64, got " + c10::toString(dt));
     return dt;
 }
 

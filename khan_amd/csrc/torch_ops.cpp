@@ -5,12 +5,29 @@
 // by path (init), so that a build named by KHAN_AEV_LIBRARY is used here too; nothing is linked against it.
 #include <dlfcn.h>
 
+#include <torch/csrc/Exceptions.h>
+
 #include "torch_common.h"
 
 namespace khan_torch {
 
 Api api;
 PyObject* khan_error = nullptr;
+
+void raise(PyObject* type, const std::string& message)
+{
+    if (PyGILState_Check()) {
+        PyErr_SetString(type, message.c_str());
+        throw py::error_already_set();
+    }
+    python_error e;
+    {
+        const py::gil_scoped_acquire lock;
+        PyErr_SetString(type, message.c_str());
+        e.persist();
+    }
+    throw python_error(std::move(e));
+}
 
 static void init(const std::string& path, py::object error_type)
 {
@@ -72,7 +89,7 @@ std::vector<Tensor> prepare_batch_into(const Tensor& mol_idxs, const Tensor& typ
     if (counts_pinned) {
         const Tensor& h = *counts_pinned;
         if (h.scalar_type() != at::kInt || h.numel() != 8 || !h.is_contiguous() || !h.is_pinned())
-            throw py::value_error("counts_pinned must hold 8 int32 in pinned memory");
+            raise(PyExc_ValueError, "counts_pinned must hold 8 int32 in pinned memory");
         host = h.data_ptr<int32_t>();
         std::fill_n(host, 8, n_mols == 0 ? 0 : -1);               // -1: not written yet (wait_for_counts)
         // the GPU writes to it: not to be handed out again before this work is done, whoever drops the tensor
@@ -151,7 +168,7 @@ Atoms check_atoms(const Atoms7& in, const AevArgs& args)
     same_size(mos.numel() == macs.numel(), "mos and macs must have the same length");
     a.acs = args.acs;
     if (a.acs.sum() != a.n)
-        throw py::value_error("sum(acs)=" + std::to_string(a.acs.sum()) + " does not match the number of atoms " + std::to_string(a.n));
+        raise(PyExc_ValueError, "sum(acs)=" + std::to_string(a.acs.sum()) + " does not match the number of atoms " + std::to_string(a.n));
     if (args.order) {
         dev(*args.order, at::kInt, "order");
         same_size(args.order->numel() == macs.numel() + kOrderExtra, "order must come from size_order(macs) of this batch");
@@ -232,7 +249,7 @@ std::vector<Tensor> run_featurize_grad(const Atoms7& in, const AevArgs& args, co
         g[t] = upstream[t].reshape({-1});
         dev(g[t], a.dt, names[t]);
         if (g[t].numel() != a.acs.v[t] * kFeats)
-            throw py::value_error(std::string(names[t]) + " has " + std::to_string(g[t].numel()) + " elements, expected " +
+            raise(PyExc_ValueError, std::string(names[t]) + " has " + std::to_string(g[t].numel()) + " elements, expected " +
                                   std::to_string(a.acs.v[t] * kFeats));
     }
     const auto& [xs, ys, zs, as, mos, macs, sis] = in;

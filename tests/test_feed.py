@@ -63,10 +63,27 @@ def test_counts_of_any_kind_of_number(of):
     acs, order, classes = b.host_counts()
     args = (b.xs, b.ys, b.zs, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs)
     want = ops.featurize(*args, list(acs), order=order, size_classes=classes)
-    for counts, totals in (([of(v) for v in acs], [of(v) for v in classes.tolist()]), (torch.tensor(acs, dtype=torch.float64), np.array(classes, dtype=np.float32))):
+    for counts, totals in (([of(v) for v in acs], [of(v) for v in classes.tolist()]), (torch.tensor(acs, dtype=torch.float64), np.array(classes.tolist(), dtype=np.float32))):
         got = ops.featurize(*args, counts, order=order, size_classes=totals)
         assert all(torch.equal(a, b) for a, b in zip(got, want))
     with pytest.raises(ValueError):
         ops.featurize(*args, [float(v) for v in acs] + [0.0], order=order)
     with pytest.raises(Exception):
         ops.featurize(*args, [float("nan")] * 4, order=order)
+
+
+def test_errors_of_the_backward_pass_keep_their_type():
+    """What an autograd node refuses in the engine's own thread arrives as the exception it is; here coordinates swapped for
+    fewer between the passes (past the version counter: the node sees them)."""
+    from khan_amd import autograd
+    m = _molecules([9, 12])
+    b = next(iter(batching.DeviceFeeder(batching.RawDataset(m, [0.0] * 2), 2))).wait()
+    acs, order, classes = b.host_counts()
+    xyz = [v.detach().clone().requires_grad_(True) for v in (b.xs, b.ys, b.zs)]
+    rows = autograd.featurize(*xyz, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs, acs, order=order, size_classes=classes)
+    loss = sum(r.sum() for r in rows)
+    kept, xyz[1].data = xyz[1].data, xyz[1].data[:5].clone()
+    with pytest.raises(ValueError, match="same length"):
+        torch.autograd.grad(loss, xyz[0], retain_graph=True)
+    xyz[1].data = kept
+    assert torch.isfinite(torch.autograd.grad(loss, xyz[0])[0]).all()
