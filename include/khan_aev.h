@@ -17,7 +17,9 @@
  * with hardware floating-point atomics, which fine-grained or host-coherent memory does not support
  * (the adds would be lost), and whose order varies: those gradients differ from run to run in the
  * last bits.  Everything else is bit-reproducible, and after khan_set_reproducible_gradients(1) so are the
- * gradients of every molecule of up to 256 atoms.
+ * gradients of every molecule of up to 256 atoms: the same call gives the same bits every time.  A molecule's gradients in
+ * ANOTHER batch can differ in the last bits with or without that setting: in batches too small to fill the GPU 2, 4 or 8
+ * wavefronts share a molecule of up to 32 atoms (64 in float64), and its forces are the sums of as many partial ones.
  *
  * Return value: KHAN_OK, or a KHAN_ERR_* code; khan_status_string() describes it.  Nothing here
  * calls exit().  An empty batch (0 atoms, 0 molecules) is a successful no-op: the reference trainer
@@ -55,7 +57,8 @@ const char *khan_last_hip_error(void);
  * the reference's gradient runs on the CPU in a fixed order, kernel_cpu.cpp:217-366).  With 1, khan_featurize_grad_*
  * sums the forces of molecules of 33..256 atoms (float32; 65..256 in float64) in on-chip memory in a fixed order and
  * stores every gradient once: the same bits on every run, no atomics, and no requirement on the kind of memory the
- * gradient arrays live in.  Costs 11 % of that kernel's speed in float32 (it runs three workgroups per CU instead
+ * gradient arrays live in.  (The same call: how many partial sums make up a small molecule's forces depends on how many
+ * molecules the batch holds, see above.)  Costs 11 % of that kernel's speed in float32 (it runs three workgroups per CU instead
  * of four) and more in float64 (one instead of two).  Not covered: molecules of more than 256 atoms, centres with more than 64
  * partners inside the angular cutoff, and upstream buckets that are not 16-byte aligned (the general kernels, atomics). */
 int khan_set_reproducible_gradients(int on);

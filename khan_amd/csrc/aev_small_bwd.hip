@@ -351,6 +351,7 @@ void aev_bwd_small_kernel(
     }
 
     // ------------------------------------------------------------ every lane stores its own atom
+    // (kW partial sums in a fixed order: the same bits on every run, but other last bits in a batch of another kW)
     if constexpr (kW > 1) __syncthreads();
     else wave_lds_fence();
     if (have && wave == 0) {

@@ -87,7 +87,9 @@ SIZE_ORDER_EXTRA = 520
 
 def set_reproducible_gradients(on):
     """Process-wide: with True, `featurize_grad` sums the forces of molecules of up to 256 atoms in a fixed order (the
-    same bits on every run, no atomics) at some cost in speed; returns the previous setting."""
+    same bits on every run, no atomics) at some cost in speed; returns the previous setting.  On every run of the same
+    batch: in another one a small molecule's forces may be the sums of 1, 2, 4 or 8 partial ones (as many as wavefronts
+    share it where a batch is too small to fill the GPU), which differ in the last bits."""
     return bool(_lib.load().khan_set_reproducible_gradients(1 if on else 0))
 
 
