@@ -210,7 +210,7 @@ class DeviceBatch:
 
     def __init__(self):
         self.labels = self.grads = self.counts_pinned = None
-        self.made_on = None       # the stream that `ready` was recorded on
+        self.made_on = None       # the stream that `ready` was recorded on (its address, on the arrays' device)
         self.memory = self.sizes = self.totals = None    # of a batch from the host: its one buffer, molecule sizes, counts
 
     def host_counts(self):
@@ -226,9 +226,11 @@ class DeviceBatch:
             classes = torch.tensor(classes, dtype=torch.int32)
         return acs, order, classes
 
-    def _counts(self):
-        """`host_counts()`, with the class totals of a batch from the host as they are held (a tuple; a tensor costs 10 us)."""
-        self._join()
+    def _counts(self, waited=False):
+        """`host_counts()`, with the class totals of a batch from the host as they are held (a tuple; a tensor costs 10 us).
+        `waited`: the current stream has done so already."""
+        if not waited:
+            self._join()
         if self.totals is not None:
             return list(self.totals[0]), self.size_order, self.totals[1]
         counts = _native.load().wait_for_counts(self.counts_pinned)
@@ -261,16 +263,18 @@ class DeviceBatch:
         self.counts_pinned = torch.empty(8, dtype=torch.int32, pin_memory=True)     # from the pinned-memory cache; the sort writes it
         (self.mol_atom_counts, self.mol_offsets, self.scatter_idxs, self.gather_idxs, self.atom_counts,
          self.size_order) = ops.prepare_batch(self.mol_idxs, self.atom_types, self.n_mols, self.counts_pinned)
-        self.made_on = torch.cuda.current_stream()
         self.ready = torch.cuda.Event()
-        self.ready.record(self.made_on)
+        self.ready.record()
+        self.made_on = self._current()
+
+    def _current(self):
+        import torch
+        return torch._C._cuda_getCurrentRawStream(self.xs.device.index)
 
     def _join(self):
         """`wait()`, where the current stream is not the one the batch was made on."""
-        import torch
-        cur = torch.cuda.current_stream()
-        if cur != self.made_on:
-            self.wait(cur)
+        if self._current() != self.made_on:
+            self.wait()
 
     def wait(self, stream=None):
         """Makes the current stream (`stream`, if the caller has it at hand) wait for the copies and the sort of this batch."""
@@ -393,8 +397,8 @@ class DeviceFeeder:
             with torch.cuda.stream(self.stream):
                 b.grads = torch.from_numpy(np.ascontiguousarray(mol_grads, dtype=self.dtype)).to(self.device)
         b.ready = self._events[slot] = torch.cuda.Event()
-        b.made_on = self.stream
-        b.ready.record(b.made_on)
+        b.made_on = self.stream.cuda_stream
+        b.ready.record(self.stream)
         return b
 
     def __iter__(self):

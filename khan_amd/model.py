@@ -254,15 +254,16 @@ class AniModel:
         energies, *parts = self._energies(b, need_grad)
         return energies, torch.stack(parts, dim=1) if need_grad else None
 
-    def _energies(self, b, need_grad, joined=False):
+    def _energies(self, b, need_grad, joined=False, waited=False):
         """DeviceBatch -> [energies [n_mols]] and, with need_grad, the energy's gradient by x, y and z; with `joined` also the
-        one array all of them are parts of: the energies, padded to 64 elements, then the gradient's three parts."""
+        one array all of them are parts of: the energies, padded to 64 elements, then the gradient's three parts.  `waited`:
+        the caller has had the current stream wait for the batch."""
         if not self.near.layer_launches():
             energies, *parts = self._energies_through_autograd(b, need_grad)
             if joined:
                 parts.append(torch.cat([energies, energies.new_empty(-b.n_mols % 64)] + parts))
             return [energies] + parts
-        acs, order, classes = b._counts()
+        acs, order, classes = b._counts(waited)
         # Networks beside a charge network run layer by layer: products of all 24 bits over float32's range, where the
         # one-launch kernel's operands keep 2^-24 of their size between 6e-5 and 65,504.
         alone = self.charge is None
@@ -317,18 +318,18 @@ class AniModel:
     def predict(self, dataset, batch_size=2048):
         """-> [y0, y1, ...] in the order of the dataset's molecules (trainer_multi_tower.py:655-678)."""
         ys = []
-        for e, _ in self._results(dataset, batch_size, lambda b: self._energies(b, False)[0]):
+        for e, _ in self._results(dataset, batch_size, lambda b: self._energies(b, False, waited=True)[0]):
             ys.extend(e.tolist())
         return ys
 
     def coordinate_gradients(self, dataset, batch_size=1024):
         """Yields one [n_atoms, 3] array of d energy / d (x, y, z) per molecule (trainer_multi_tower.py:580-615)."""
-        of_batch = lambda b: self._energies(b, True, joined=True)[-1][-3 * b.xs.numel():] if b.xs.numel() else b.xs
+        of_batch = lambda b: self._energies(b, True, joined=True, waited=True)[-1][-3 * b.xs.numel():] if b.xs.numel() else b.xs
         for g, b in self._results(dataset, batch_size, of_batch):
             yield from _native.load().molecule_rows(g.reshape(3, -1), b.host_sizes())
 
     def energies_and_gradients(self, dataset, batch_size=1024):
         """Yields (energy, [n_atoms, 3] gradient) per molecule from one pass over the data set."""
-        for v, b in self._results(dataset, batch_size, lambda b: self._energies(b, True, joined=True)[-1]):
+        for v, b in self._results(dataset, batch_size, lambda b: self._energies(b, True, joined=True, waited=True)[-1]):
             gradient = v[v.size - 3 * b.xs.numel():].reshape(3, -1)
             yield from zip(v[:b.n_mols].tolist(), _native.load().molecule_rows(gradient, b.host_sizes()))

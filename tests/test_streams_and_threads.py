@@ -30,9 +30,10 @@ def test_the_counts_bring_the_batch_with_them(monkeypatch):
     batch and tells the allocator, on another stream than the batch's own."""
     own, other = _Stream(), _Stream()
     b = batching.DeviceBatch()
-    b.ready, b.made_on, b.memory, b.size_order, b.totals = object(), own, _Tensor(), None, ((1, 2, 3, 4), (1, 0, 0, 0))
+    b.xs, b.ready, b.made_on, b.memory, b.size_order, b.totals = torch.zeros(1), object(), id(own), _Tensor(), None, ((1, 2, 3, 4), (1, 0, 0, 0))
     for current, waited in ((own, []), (other, [b.ready])):
         monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: current)
+        monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda *a: id(current), raising=False)
         assert b.host_counts()[0] == [1, 2, 3, 4]
         assert current.waited == waited
     assert b.memory.used_on == [other]
