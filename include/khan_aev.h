@@ -384,6 +384,7 @@ int khan_atomic_networks_f32(const float *const *rows_host4, const int32_t *n_ho
 #define KHAN_NET_ROWS 2      /* scale[row] y (scale NULL: y), added to out where accumulate is set */
 #define KHAN_NET_TANGENT 3   /* y' = scale[row] y: out = y' celu'(act), out2 = y' d / alpha where act < 0, else 0 */
 #define KHAN_NET_SECOND 4    /* y celu'(act) + scale[row] t */
+#define KHAN_NET_CELU_ABSOLUTE 5    /* celu to 2^-23 alpha, in float32 the faster: activations far below alpha in size lose digits */
 typedef struct khan_net_layer {
     const void *in[4], *w[4], *bias[4];                  /* [n, k]; [k, n_out], or [n_out, k] with transposed; [n_out] */
     const void *act[4], *d[4], *t[4], *scale[4];         /* [n, n_out] and [n] */

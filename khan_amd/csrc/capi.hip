@@ -437,7 +437,7 @@ static int ani_charges(const T* xs, const T* ys, const T* zs, const T* qs, const
 template <typename T>
 static int net_layer_impl(const khan_net_layer* l, khan_stream_t stream)
 {
-    if (!l || l->k <= 0 || l->n_out <= 0 || !(l->alpha > 0.0) || l->kind < KHAN_NET_CELU || l->kind > KHAN_NET_SECOND) return KHAN_ERR_INVALID_ARG;
+    if (!l || l->k <= 0 || l->n_out <= 0 || !(l->alpha > 0.0) || l->kind < KHAN_NET_CELU || l->kind > KHAN_NET_CELU_ABSOLUTE) return KHAN_ERR_INVALID_ARG;
     khan::NetLayer<T> a = {};
     int64_t rows = 0;
     for (int t = 0; t < 4; ++t) {
@@ -455,7 +455,9 @@ static int net_layer_impl(const khan_net_layer* l, khan_stream_t stream)
         rows += l->n[t];
     }
     if (rows > INT32_MAX) return KHAN_ERR_TOO_LARGE;
-    a.k = l->k; a.n_out = l->n_out; a.kind = l->kind; a.accumulate = l->accumulate;
+    a.k = l->k; a.n_out = l->n_out; a.accumulate = l->accumulate;
+    a.absolute = l->kind == KHAN_NET_CELU_ABSOLUTE;
+    a.kind = a.absolute ? KHAN_NET_CELU : l->kind;
     a.alpha = static_cast<T>(l->alpha); a.inv_alpha = static_cast<T>(1.0 / l->alpha);
     return hip_status(khan::launch_net_layer<T>(a, l->transposed != 0, as_stream(stream)));
 }

@@ -25,6 +25,7 @@ struct NetLayer {
     int n[4];                       // rows per type
     int k, n_out;
     int kind, accumulate;
+    bool absolute;                  // kNetCelu: an error of 2^-24 alpha is small enough, that of small activations may be larger
     T alpha, inv_alpha;
     int tile_end[4], col_tiles;     // filled by the launcher
 };

@@ -13,10 +13,13 @@
 // these is formed in its epilogue, so that every operand of the next one is read as it lies in memory.
 //
 // These replace library products (rocBLAS, one per type, with elementwise passes between them) in training, in force
-// training, for networks the one-launch kernel (dense_fused.hip) is not made for, and in float64: a step on 1,024 organic
-// molecules was 95 launches, one with a loss on forces 430, an energy request 330.  Measured with what goes with it (no graph
-// in inference, csrc/torch_autograd.cpp): training on 1,024 organic molecules 1.62 -> 0.57 ms, with a loss on the forces of
-// 3,001 6.95 -> 1.04 ms, a request for an energy and a gradient in float64 3.75 -> 0.65 ms.
+// training, for networks the one-launch kernel (dense_fused.hip) is not made for or may not take (float64, charge networks): a
+// step on 1,024 organic molecules was 95 launches, one with a loss on forces 430, an energy request 330.  Measured with what
+// goes with it (no graph in inference, csrc/torch_autograd.cpp), us a pass, library products -> here: a request for an energy
+// and a gradient in float64 4,000 -> 210; training, float32 default networks, 1,024 / 16,384 / 65,536 organic molecules
+// 1,840 -> 480, 4,870 -> 1,120, 16,200 -> 3,630, deep networks on 1,024 / 16,384 6,450 -> 910, 12,700 -> 5,410; in float64
+// 1,024 / 16,384 3,550 -> 490, 39,300 -> 2,540; with a loss on forces, float32 1,024 / 16,384 6,470 -> 830, 17,500 -> 3,280,
+// float64 7,520 -> 970, 80,000 -> 7,760.  No size was found where library products are faster, so there is no line to draw.
 //
 // The products run on the matrix instructions of the operands' own precision, v_mfma_f32_16x16x4_f32 and
 // v_mfma_f64_16x16x4_f64, with nothing staged through LDS: a lane's piece of either operand is 16 contiguous bytes of a
@@ -42,7 +45,7 @@ namespace {
 // counts as its positive side, and 0.6 % off at -1e-5): x = k ln 2 + f with |f| <= ln 2 / 2 (k from the bits of x log2 e +
 // 1.5 2^23, ln 2 in two parts), exp(f) - 1 = f + f^2 r(f) with r interpolated at Chebyshev points, and 2^k (exp(f) - 1) +
 // (2^k - 1).  Below -88 it is -1, in float32 too; x is not NaN.  Twelve vector instructions more than the other form per
-// activation.
+// activation, 9 % of a layer's time (47,000 rows 256 -> 256: 39.7 -> 43.2 us).
 __device__ __forceinline__ float expm1_down(float x)
 {
     x = fmaxf(x, -88.0f);
@@ -63,6 +66,7 @@ template <> struct MatrixOp<float> {
     static __device__ __forceinline__ acc mul(float a, float b, acc c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
     static __device__ __forceinline__ int row(int lane, int v) { return 4 * (lane >> 4) + v; }      // of result element v
     static __device__ __forceinline__ float celu(float z, float alpha, float inv) { return z < 0.f ? alpha * expm1_down(z * inv) : z; }
+    static __device__ __forceinline__ float celu_abs(float z, float alpha, float inv) { return z >= 0.f ? z : alpha * (__expf(z * inv) - 1.0f); }
 };
 template <> struct MatrixOp<double> {
     typedef double acc __attribute__((ext_vector_type(4)));
@@ -70,6 +74,7 @@ template <> struct MatrixOp<double> {
     static __device__ __forceinline__ acc mul(double a, double b, acc c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
     static __device__ __forceinline__ int row(int lane, int v) { return (lane >> 4) + 4 * v; }
     static __device__ __forceinline__ double celu(double z, double alpha, double inv) { return z >= 0. ? z : alpha * expm1(z * inv); }
+    static __device__ __forceinline__ double celu_abs(double z, double alpha, double inv) { return celu(z, alpha, inv); }
 };
 template <typename T, int W = MatrixOp<T>::kVec> using Vec = T __attribute__((ext_vector_type(W)));
 
@@ -127,10 +132,17 @@ __device__ __forceinline__ void finish(const NetLayer<T>& a, int t, const int (&
         }
     }
     if (a.kind == kNetCelu) {
+        if (a.absolute) {
 #pragma unroll
-        for (int i = 0; i < R; ++i)
+            for (int i = 0; i < R; ++i)
 #pragma unroll
-            for (int j = 0; j < W; ++j) y[i][j] = MatrixOp<T>::celu(y[i][j], a.alpha, a.inv_alpha);
+                for (int j = 0; j < W; ++j) y[i][j] = MatrixOp<T>::celu_abs(y[i][j], a.alpha, a.inv_alpha);
+        } else {
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+#pragma unroll
+                for (int j = 0; j < W; ++j) y[i][j] = MatrixOp<T>::celu(y[i][j], a.alpha, a.inv_alpha);
+        }
     } else if (a.kind == kNetRows) {
 #pragma unroll
         for (int i = 0; i < R; ++i) y[i] *= s[i];

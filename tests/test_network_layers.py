@@ -152,11 +152,12 @@ def test_split_products(rows, k, n_out, transposed):
                 assert (out2[i] == 1).all(), (name, i)
 
 
-def test_celu_of_small_and_large_arguments():
-    """The layers' float32 CELU over the binades of negative arguments from -1e-30 (the split operands' smallest parts reach float32's
-    subnormal numbers below) on: within 2^-21 of alpha expm1(z / alpha) (five roundings
-    of 2^-24: alpha, its inverse, the argument, the function, the last product; the function has 1.5), never zero below
-    zero, NaN kept.  One input column and a weight of one make the layer's sum its argument."""
+@pytest.mark.parametrize("absolute", [False, True])
+def test_celu_of_small_and_large_arguments(absolute):
+    """The layers' float32 CELU over the binades of negative arguments from -1e-30 on (below, the split operands' smallest parts
+    are subnormal): within 2^-21 of alpha expm1(z / alpha) (five roundings of 2^-24: alpha, its inverse, the argument, the
+    function, the last product; the function has 1.5), never zero below zero, NaN kept; in its absolute form within
+    2^-23 alpha more.  One input column and a weight of one make the layer's sum its argument."""
     from khan_amd import _lib
     lib = _lib.load()
     lib.khan_net_layer_f32.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
@@ -167,7 +168,7 @@ def test_celu_of_small_and_large_arguments():
     for first in (0, z.numel() - 64):                     # split products, which make NaN of infinities; the float32 instructions
         rows, arg = x[first:].contiguous(), z[first:].double()
         out = torch.empty(rows.shape[0], 64, device="cuda")
-        a = _Layer(k=32, n_out=64, kind=0, alpha=ALPHA)
+        a = _Layer(k=32, n_out=64, kind=5 if absolute else 0, alpha=ALPHA)
         a.n[1] = rows.shape[0]
         for field, value in (("x", rows), ("w", w), ("out", out)):
             getattr(a, field)[1] = value.data_ptr()
@@ -175,8 +176,9 @@ def test_celu_of_small_and_large_arguments():
         got = out[:, 0].double()
         want = torch.where(arg < 0, ALPHA * torch.expm1(arg / ALPHA), arg)
         known = torch.isfinite(arg) if first == 0 else ~torch.isnan(arg)
-        assert ((got - want).abs() <= 2.0 ** -21 * want.abs())[known & ~torch.isinf(want)].all()
-        assert (got < 0)[known & (arg < 0)].all() and torch.isnan(got[torch.isnan(arg)]).all()
+        bound = torch.where(arg < 0, 2.0 ** -23 * ALPHA, 0.0) if absolute else 0.0
+        assert ((got - want).abs() <= 2.0 ** -21 * want.abs() + bound)[known & ~torch.isinf(want)].all()
+        assert ((got < 0) | absolute)[known & (arg < 0)].all() and torch.isnan(got[torch.isnan(arg)]).all()
         assert first == 0 or got[-1] == float("inf")
 
 
