@@ -37,21 +37,22 @@ if ROOT not in sys.path:
 RECORD = os.path.join(ROOT, "profiles", "hbm_traffic.json")
 COPY_BYTES = 64 * 1024 * 1024
 
-# the kernel that dominates each pass of each bench workload (substring of the name rocprofv3 prints)
+# the kernel that dominates each pass of each bench workload (start of the name rocprofv3 prints, up to the template
+# arguments that the size of the batch decides)
 DOMINANT = {
-    ("organic65536", "fwd"): "aev_fwd_small_kernel<float, false, false>",
-    ("organic65536", "bwd"): "aev_bwd_small_kernel<float>",
-    ("organic16384", "fwd"): "aev_fwd_small_kernel<float, false, false>",
-    ("organic16384", "bwd"): "aev_bwd_small_kernel<float>",
-    ("organic1024", "fwd"): "aev_fwd_small_kernel<float, false, false>",
-    ("organic1024", "bwd"): "aev_bwd_small_kernel<float>",
-    ("organic16384_f64", "fwd"): "aev_fwd_small_kernel<double, false, false>",
-    ("organic16384_f64", "bwd"): "aev_bwd_small_kernel<double>",
-    ("boxes4096", "fwd"): "aev_fwd_medium_kernel<float, false, false>",
-    ("boxes4096", "bwd"): "aev_bwd_medium_kernel<float, false, false>",
+    ("organic65536", "fwd"): "aev_fwd_small_kernel<float, false,",
+    ("organic65536", "bwd"): "aev_bwd_small_kernel<float,",
+    ("organic16384", "fwd"): "aev_fwd_small_kernel<float, false,",
+    ("organic16384", "bwd"): "aev_bwd_small_kernel<float,",
+    ("organic1024", "fwd"): "aev_fwd_small_kernel<float, false,",
+    ("organic1024", "bwd"): "aev_bwd_small_kernel<float,",
+    ("organic16384_f64", "fwd"): "aev_fwd_small_kernel<double, false,",
+    ("organic16384_f64", "bwd"): "aev_bwd_small_kernel<double,",
+    ("boxes4096", "fwd"): "aev_fwd_medium_kernel<float, false, false,",
+    ("boxes4096", "bwd"): "aev_bwd_medium_kernel<float, false, false,",
     ("organic65536", "networks"): "networks_fused_kernel<true, true>",
-    ("organic65536", "jvp"): "aev_fwd_small_kernel<float, true, false>",
-    ("charges_boxes4096_f64", "charges"): "charge_tile_kernel<double",
+    ("organic65536", "jvp"): "aev_fwd_small_kernel<float, true,",
+    ("charges_boxes4096_f64", "charges"): "charge_kernel<double, true, true>",
 }
 # the sources an entry's digest covers, by pass
 _DIGEST_SOURCES = {"networks": ("dense_fused.hip", "khan_internal.h"), "charges": ("charges.hip", "khan_internal.h")}
