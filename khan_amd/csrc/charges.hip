@@ -48,7 +48,7 @@ template <bool kDamped> struct PairTerms<float, kDamped> {
 // double: no library call, no square root and no angle.  1/r from v_rsq_f64 (5e-8) and one third-order step.  1 - f_C =
 // sin^2(pi r / 2 R_c) = d2 q(d2) and 2 d(1 - f_C)/d(d2) = (d/dr) / r are entire functions of d2: polynomials of degree
 // nine in d2 (Chebyshev interpolation on [0, R_c^2]), exact to 4e-16 of q and 1e-16.  (Before: a square root, a folded half
-// angle, its sine and cosine: 106 vector instructions per pair of the tile kernel, 78 now, with everything around it.)
+// angle, its sine and cosine: 106 vector instructions per pair over the whole kernel, 92 now.)
 template <bool kDamped> struct PairTerms<double, kDamped> {
     static __device__ __forceinline__ double poly(const double (&c)[10], double x)
     {

@@ -100,3 +100,25 @@ def test_float32_networks_beside_a_charge_network(exponent):
     for g, w in zip(got, want):
         assert torch.isfinite(g).all()
         assert float((g.double() - w).abs().max()) <= 2e-5 * float(w.abs().max())
+
+
+@pytest.mark.parametrize("layers,dtype", [(model.DEFAULT_LAYERS, torch.float32), (model.DEFAULT_LAYERS, torch.float64), ((100, 1), torch.float32)])
+def test_captured_inference_reads_the_parameters_when_it_is_replayed(layers, dtype):
+    """batch_energies of a batch made on another stream, recorded into a graph: every replay, with eager work and parameter
+    writes in between, gives what an eager pass gives then."""
+    m = model.AniModel(layers, model.celu, dtype, DEV, seed=1)
+    b = _batch(300, dtype)
+    m.batch_energies(b, need_grad=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = m.batch_energies(b, need_grad=True)
+    for k in range(3):
+        for o in out:
+            o.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        want = m.batch_energies(b, need_grad=True)
+        assert all(torch.equal(a, w) for a, w in zip(out, want)), k
+        for p in m.near.parameters():
+            p.data.add_(0.01)
+        torch.cuda.synchronize()
