@@ -469,8 +469,9 @@ __global__ __launch_bounds__(256) void top_kernel(const NetTop<T> a, int total)
 // The column sums (the biases' gradients, factors of random sign that cancel) are formed by the first row of tiles alone and
 // carry their rounding errors along: added up plainly, 64 rows to a lane, they were 2e-7 off where a library sum is 4e-8 off
 // (124 -> 126 us a launch at 35,000 rows).
-// 62 TFLOP/s of the float32 instructions' 153 at 35,000 rows of 384-128-128-64-1 (82 us).  The compiler's overlap of the
-// unrolled loop's loads with the products beats four row groups loaded ahead by hand (104 us a launch there).
+// In float32 this form is left for layers narrower than 64, for few rows and for operands that are not aligned
+// (weight_grad_split_tile takes the others): 62 TFLOP/s of the instructions' 153 at 35,000 rows of 384-128-128-64-1 (82 us).
+// The compiler's overlap of the unrolled loop's loads with the products beats four row groups loaded ahead by hand (104 us).
 // sum += x, its rounding error added to `lost` (Knuth's two-sum)
 template <typename V>
 __device__ __forceinline__ void add_exactly(V& sum, V& lost, V x)
@@ -489,7 +490,7 @@ struct GradLds {
     T bias[4][16 * kVec];
 };
 template <typename T, bool kWhole>
-__device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __restrict__ partial, GradLds<T>& S, int job)
+__device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __restrict__ partial, GradLds<T>& S, int job, int rel)
 {
     typedef MatrixOp<T> Op;
     typedef typename Op::acc acc_t;
@@ -497,7 +498,6 @@ __device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __rest
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, grp = lane >> 4;
     const int layer = job >> 2, t = job & 3;
-    const int rel = static_cast<int>(blockIdx.x) - (job == 0 ? 0 : a.job_end[job - 1]);
     const int K = a.k[layer], N = a.k[layer + 1], n = a.n[t];
     const int tiles_n = (N + kSide - 1) / kSide, tiles = (K + kSide - 1) / kSide * tiles_n;
     const int split = rel / tiles, tile = rel - split * tiles;
@@ -573,7 +573,7 @@ __device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __rest
     if (wave != 0) return;
     take(0);
     // tile element (i, j): row kVec row(v) + i of the tile, column kVec l16 + j
-    T* __restrict__ out = partial + static_cast<size_t>(blockIdx.x) * (kSide * kSide + kSide);
+    T* __restrict__ out = partial + a.job_base[job] + static_cast<size_t>(rel) * (kSide * kSide + kSide);
 #pragma unroll
     for (int i = 0; i < V; ++i)
 #pragma unroll
@@ -586,59 +586,300 @@ __device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __rest
     if (lane < kSide) out[kSide * kSide + lane] = (S.bias[0][lane] + S.bias[1][lane]) + (S.bias[2][lane] + S.bias[3][lane]);
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void weight_grad_kernel(const NetGrads<T> a, T* __restrict__ partial)
+// The same in float32 on the bfloat16 matrix instructions (the split of layer_split_kernel), for layers of at least 64 x 64.
+// A workgroup forms 128 of the left operand's columns x 128 (kWide) or 64 of the right's over `per_split` rows, 32 rows at a
+// time.  The rows are what is summed over, so that a matrix instruction's operand is eight rows of one column, which lie a row
+// apart in memory: a thread loads two neighbouring columns of eight rows (a wavefront 512 contiguous bytes of each row), splits
+// them and writes them to LDS as [part][eight rows][column] pieces of 16 bytes, column 2 c + j at place 64 j + c, so that
+// writes and reads run along consecutive places.  A wavefront multiplies 64 x 64 (32 x 64) from there.  The five small partial
+// products have accumulators of their own, so that the large sum is rounded once in 32 rows: the distance from float64 is half
+// of the float32 instructions' (35,000 rows: 2.85e-7 -> 1.39e-7; with one set of accumulators 3.06e-7).  The next rows'
+// loads are in flight during the products; two workgroups share a compute unit and fill each other's barriers.
+// Gradients of 384-128-128-64-1 on 35,000 rows, one pair of operands 86 -> 51 us, both 157 -> 85 (101 TFLOP/s); 12,132 rows
+// 42 -> 28.  What is left is products (14 us), splitting and the loads of 144 MB (30 us) one after the other.  No faster: two
+// chunks in flight instead of one (with the small products added to the large ones chunk by chunk, for its registers),
+// splitting by v_dot2_f32_bf16 (seven instructions instead of eleven).
+// An element that is not finite (infinite, NaN or overflowing operands: the split makes NaN of infinities) has the workgroup
+// form its tile again by float32 multiply-adds, so that infinities and NaN come out as they do there.
+constexpr int kGradLeft = 128, kGradChunk = 32;
+struct SplitGradLds {
+    u4v left[3][4][kGradLeft], right[3][4][128];
+};
+__device__ __forceinline__ int grad_place(int column) { return 64 * (column & 1) + (column >> 1); }
+__device__ __forceinline__ int grad_column(int place) { return 2 * (place & 63) + (place >> 6); }
+
+template <bool kWide>
+__device__ __forceinline__ void weight_grad_split_tile(const NetGrads<float>& a, float* __restrict__ partial, SplitGradLds& S, int job, int rel)
 {
-    __shared__ GradLds<T> S;
-    int job = 0;
-    while (static_cast<int>(blockIdx.x) >= a.job_end[job]) ++job;                 // (layer, type)
-    if ((a.whole >> (job >> 2)) & 1u) weight_grad_tile<T, true>(a, partial, S, job);
-    else weight_grad_tile<T, false>(a, partial, S, job);
+    constexpr int kCols = kWide ? 128 : 64, kRC = kCols / 64;       // right columns of the tile, and per thread
+    constexpr int kLB = kWide ? 4 : 2, kRB = 4;                     // a wavefront's blocks of 16 left and right columns
+    typedef Vec<float, kRC> rvec;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, grp = lane >> 4;
+    const int lb0 = kWide ? 4 * (wave >> 1) : 2 * wave, rb0 = kWide ? 4 * (wave & 1) : 0;
+    const int layer = job >> 2, t = job & 3;
+    const int K = a.k[layer], N = a.k[layer + 1], n = a.n[t];
+    const int tiles_n = (N + kCols - 1) / kCols, tiles = (K + kGradLeft - 1) / kGradLeft * tiles_n;
+    const int share = rel / tiles, tile = rel - share * tiles;
+    const int i0 = tile / tiles_n * kGradLeft, j0 = tile % tiles_n * kCols;
+    const int r0 = share * a.per_split, r1 = min(n, r0 + a.per_split);
+    const int chunks = (r1 - r0 + kGradChunk - 1) / kGradChunk;
+    // this thread's columns (past the end: the last ones again, whose sums are never read)
+    const int li = min(i0 + 2 * lane, K - 2), lj = min(j0 + kRC * lane, N - kRC);
+
+    struct Operands {
+        const float *left, *right, *scale;
+    };
+    auto operands = [&](int pair) -> Operands {
+        const float* left = pair == 0 ? a.left[layer] : a.left2[layer];
+        const float* right = pair == 0 ? a.right[layer] : a.right2[layer];
+        left = layer == 0 ? (pair == 0 ? a.x[t] : a.x2[t]) : left + static_cast<size_t>(a.row0[t]) * K;
+        return {left, right + static_cast<size_t>(a.row0[t]) * N, (pair == 0 ? a.scale_first : a.scale_second) ? a.scale[t] : nullptr};
+    };
+    auto live_pair = [&](int pair) { return (((pair == 0 ? a.first : a.second) >> layer) & 1u) != 0; };
+    f4v acc[kRB][kLB], small[kRB][kLB];
+#pragma unroll
+    for (int i = 0; i < kRB; ++i)
+#pragma unroll
+        for (int j = 0; j < kLB; ++j) acc[i][j] = small[i][j] = f4v(0.f);
+    rvec bias = rvec(0.f), bias_lost = rvec(0.f);
+    f2v x[8];
+    rvec y[8];
+#pragma unroll 1
+    for (int pair = 0; pair < 2; ++pair) {
+        if (!live_pair(pair)) continue;
+        const Operands op = operands(pair);
+        auto fetch = [&](int c) {
+            const int r = r0 + c * kGradChunk + 8 * wave;
+            if (r + 8 <= r1) {
+                const float* left = op.left + static_cast<size_t>(r) * K;
+                const float* right = op.right + static_cast<size_t>(r) * N;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    x[i] = *reinterpret_cast<const f2v*>(left + li);
+                    y[i] = *reinterpret_cast<const rvec*>(right + lj);
+                    left += K;
+                    right += N;
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const size_t at = static_cast<size_t>(min(r + i, r1 - 1));
+                    x[i] = *reinterpret_cast<const f2v*>(op.left + at * K + li);
+                    y[i] = *reinterpret_cast<const rvec*>(op.right + at * N + lj);
+                }
+            }
+        };
+        fetch(0);
+#pragma unroll 1
+        for (int c = 0; c < chunks; ++c) {
+            const int r = r0 + c * kGradChunk + 8 * wave;
+            if (r + 8 <= r1) {
+                if (op.scale) {
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) y[i] *= op.scale[r + i];
+                }
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float s = op.scale ? op.scale[min(r + i, r1 - 1)] : 1.0f;
+                    y[i] = r + i < r1 ? y[i] * s : rvec(0.f);
+                    if (r + i >= r1) x[i] = f2v(0.f);
+                }
+            }
+            if (pair == 0 && i0 == 0) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) add_exactly(bias, bias_lost, y[i]);
+            }
+            __syncthreads();                   // the planes' previous contents have been read
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                u4v p[3];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    unsigned q[3];
+                    split_pair(x[2 * e][j], x[2 * e + 1][j], q[0], q[1], q[2]);
+                    p[0][e] = q[0], p[1][e] = q[1], p[2][e] = q[2];
+                }
+#pragma unroll
+                for (int q = 0; q < 3; ++q) S.left[q][wave][64 * j + lane] = p[q];
+            }
+#pragma unroll
+            for (int j = 0; j < kRC; ++j) {
+                u4v p[3];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    unsigned q[3];
+                    split_pair(y[2 * e][j], y[2 * e + 1][j], q[0], q[1], q[2]);
+                    p[0][e] = q[0], p[1][e] = q[1], p[2][e] = q[2];
+                }
+#pragma unroll
+                for (int q = 0; q < 3; ++q) S.right[q][wave][64 * j + lane] = p[q];
+            }
+            __syncthreads();
+            if (c + 1 < chunks) fetch(c + 1);  // in flight while this chunk is multiplied
+            bf16x8 lv[3][kLB];
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+#pragma unroll
+                for (int j = 0; j < kLB; ++j) lv[q][j] = __builtin_bit_cast(bf16x8, S.left[q][grp][16 * (lb0 + j) + l16]);
+#pragma unroll
+            for (int q = 2; q >= 0; --q) {
+                bf16x8 rv[kRB];
+#pragma unroll
+                for (int i = 0; i < kRB; ++i) rv[i] = __builtin_bit_cast(bf16x8, S.right[q][grp][16 * (rb0 + i) + l16]);
+#pragma unroll
+                for (int p = 2 - q; p >= 0; --p)
+#pragma unroll
+                    for (int i = 0; i < kRB; ++i)
+#pragma unroll
+                        for (int j = 0; j < kLB; ++j) {
+                            f4v& to = p + q == 0 ? acc[i][j] : small[i][j];
+                            to = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rv[i], lv[p][j], to, 0, 0, 0);
+                        }
+            }
+        }
+    }
+    // element v of a block: right place 16 (rb0 + i) + 4 grp + v, left place 16 (lb0 + j) + l16
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < kRB; ++i)
+#pragma unroll
+        for (int j = 0; j < kLB; ++j) {
+            acc[i][j] += small[i][j];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) bad = bad || !isfinite(acc[i][j][v]);
+        }
+    if (__syncthreads_or(bad)) {
+#pragma unroll
+        for (int i = 0; i < kRB; ++i)
+#pragma unroll
+            for (int j = 0; j < kLB; ++j) acc[i][j] = f4v(0.f);
+#pragma unroll 1
+        for (int pair = 0; pair < 2; ++pair) {
+            if (!live_pair(pair)) continue;
+            const Operands op = operands(pair);
+#pragma unroll 1
+            for (int r = r0; r < r1; ++r) {
+                const float s = op.scale ? op.scale[r] : 1.0f;
+                float lv[kLB];
+#pragma unroll
+                for (int j = 0; j < kLB; ++j)
+                    lv[j] = op.left[static_cast<size_t>(r) * K + min(i0 + grad_column(16 * (lb0 + j) + l16), K - 1)];
+#pragma unroll
+                for (int i = 0; i < kRB; ++i)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int place = 16 * (rb0 + i) + 4 * grp + v, column = j0 + (kWide ? grad_column(place) : place);
+                        const float rv = op.right[static_cast<size_t>(r) * N + min(column, N - 1)] * s;
+#pragma unroll
+                        for (int j = 0; j < kLB; ++j) acc[i][j][v] = fmaf(lv[j], rv, acc[i][j][v]);
+                    }
+            }
+        }
+    }
+    // partial sums: [left place][right place], then the right columns' own sums by place
+    float* __restrict__ out = partial + a.job_base[job] + static_cast<size_t>(rel) * (kGradLeft * kCols + kCols);
+#pragma unroll
+    for (int j = 0; j < kLB; ++j)
+#pragma unroll
+        for (int i = 0; i < kRB; ++i)
+            *reinterpret_cast<f4v*>(out + (16 * (lb0 + j) + l16) * kCols + 16 * (rb0 + i) + 4 * grp) = acc[i][j];
+    if (i0 != 0) return;
+    float* const sums = reinterpret_cast<float*>(S.left);       // (the last reads of the planes lie before the barrier above)
+#pragma unroll
+    for (int j = 0; j < kRC; ++j) sums[wave * 128 + 64 * j + lane] = with_lost(bias[j], bias_lost[j]);
+    __syncthreads();
+    if (threadIdx.x < kCols) {
+        const float* b = sums + threadIdx.x;
+        out[kGradLeft * kCols + threadIdx.x] = (b[0] + b[128]) + (b[256] + b[384]);
+    }
 }
 
-// the workgroups' partial tiles and bias sums -> the gradients, a thread per element
 template <typename T>
-__global__ __launch_bounds__(256) void grad_sum_kernel(const NetGrads<T> a, const T* __restrict__ partial, int64_t elements)
+__global__ __launch_bounds__(256, 2) void weight_grad_kernel(const NetGrads<T> a, T* __restrict__ partial)
 {
-    constexpr int V = MatrixOp<T>::kVec, kSide = 16 * V, kStride = kSide * kSide + kSide;
-    const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-    if (e >= elements) return;
-    // all weights first (type by type inside a layer), then all biases
-    int64_t at = e;
-    int layer = 0, t = 0;
-    bool is_bias = false;
-    for (;; ++layer) {
-        if (layer == a.layers) {
-            if (is_bias) return;
-            is_bias = true;
-            layer = 0;
+    int job = 0;
+    while (static_cast<int>(blockIdx.x) >= a.job_end[job]) ++job;                 // (layer, type)
+    const int rel = static_cast<int>(blockIdx.x) - (job == 0 ? 0 : a.job_end[job - 1]);
+    if constexpr (std::is_same<T, float>::value) {
+        __shared__ union {
+            GradLds<float> plain;
+            SplitGradLds split;
+        } S;
+        if ((a.split >> (job >> 2)) & 1u) {
+            if (a.k[(job >> 2) + 1] > 64) weight_grad_split_tile<true>(a, partial, S.split, job, rel);
+            else weight_grad_split_tile<false>(a, partial, S.split, job, rel);
+        } else if ((a.whole >> (job >> 2)) & 1u) {
+            weight_grad_tile<T, true>(a, partial, S.plain, job, rel);
+        } else {
+            weight_grad_tile<T, false>(a, partial, S.plain, job, rel);
         }
-        const int64_t size = is_bias ? a.k[layer + 1] : static_cast<int64_t>(a.k[layer]) * a.k[layer + 1];
-        if (at < 4 * size) {
-            t = static_cast<int>(at / size);
-            at -= t * size;
-            break;
-        }
-        at -= 4 * size;
-    }
-    const int K = a.k[layer], N = a.k[layer + 1];
-    const int tiles_n = (N + kSide - 1) / kSide, tiles = (K + kSide - 1) / kSide * tiles_n;
-    const int splits = (a.n[t] + a.per - 1) / a.per, job = layer * 4 + t;
-    int tile;
-    int64_t within;
-    if (is_bias) {
-        tile = static_cast<int>(at) / kSide;                    // the first row of tiles holds the bias sums
-        within = kSide * kSide + at % kSide;
     } else {
-        const int i = static_cast<int>(at / N), j = static_cast<int>(at % N);
-        tile = i / kSide * tiles_n + j / kSide;
-        within = (i % kSide) * kSide + j % kSide;
+        __shared__ GradLds<T> S;
+        if ((a.whole >> (job >> 2)) & 1u) weight_grad_tile<T, true>(a, partial, S, job, rel);
+        else weight_grad_tile<T, false>(a, partial, S, job, rel);
     }
-    const T* p = partial + static_cast<size_t>((job == 0 ? 0 : a.job_end[job - 1]) + tile) * kStride + within;
-    T sum = T(0), lost = T(0);
-#pragma unroll 4
-    for (int s = 0; s < splits; ++s) add_exactly(sum, lost, p[static_cast<size_t>(s) * tiles * kStride]);
-    a.out[e] = with_lost(sum, lost);
+}
+
+// The workgroups' partial tiles and bias sums -> the gradients.  A workgroup takes 64 runs of 16 bytes of one tile, its
+// wavefronts a quarter of the shares each, one after the other; the quarters are added in order.  (A thread per element of
+// the result waits for as many loads of its own as there are shares: 45 us for 100 of them, 39 MB.)
+template <typename T>
+__global__ __launch_bounds__(256) void grad_sum_kernel(const NetGrads<T> a, const T* __restrict__ partial)
+{
+    constexpr int V = MatrixOp<T>::kVec, kSide = 16 * V, kRun = 64 * V;
+    __shared__ Vec<T> quarter[4][2][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int64_t out = 0;                       // where the layer's weights begin
+    int block = static_cast<int>(blockIdx.x), layer = 0, rows, cols, tiles_n, tiles, runs;
+    bool split;
+    for (;; ++layer) {
+        split = (a.split >> layer) & 1u;
+        rows = split ? kGradLeft : kSide;
+        cols = split ? (a.k[layer + 1] > 64 ? 128 : 64) : kSide;
+        tiles_n = (a.k[layer + 1] + cols - 1) / cols;
+        tiles = (a.k[layer] + rows - 1) / rows * tiles_n;
+        runs = (rows * cols + cols + kRun - 1) / kRun;
+        if (block < 4 * tiles * runs) break;
+        block -= 4 * tiles * runs;
+        out += 4 * static_cast<int64_t>(a.k[layer]) * a.k[layer + 1];
+    }
+    const int t = block / (tiles * runs), tile = block / runs - t * tiles, at = (block % runs * 64 + lane) * V;
+    const int K = a.k[layer], N = a.k[layer + 1], size = rows * cols + cols;
+    const int per = split ? a.per_split : a.per, shares = (a.n[t] + per - 1) / per;
+    const T* p = partial + a.job_base[layer * 4 + t] + static_cast<size_t>(tile) * size + min(at, size - V);
+    const size_t stride = static_cast<size_t>(tiles) * size;
+    Vec<T> sum = Vec<T>(T(0)), lost = Vec<T>(T(0));
+    const int first = wave * shares >> 2, last = (wave + 1) * shares >> 2;
+#pragma unroll 8
+    for (int s = first; s < last; ++s) add_exactly(sum, lost, *reinterpret_cast<const Vec<T>*>(p + s * stride));
+    quarter[wave][0][lane] = sum;
+    quarter[wave][1][lane] = lost;
+    __syncthreads();
+    if (wave > 0 || at >= size) return;
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+        add_exactly(sum, lost, quarter[w][0][lane]);
+        lost += quarter[w][1][lane];
+    }
+    const bool is_bias = at >= rows * cols;
+    if (is_bias && tile >= tiles_n) return;                    // the first row of tiles holds the bias sums
+    int row = tile / tiles_n * rows;
+    if (!is_bias) row += split ? grad_column(at / cols) : at / cols;
+    if (is_bias) {
+        // behind all weights, layer by layer
+        for (int l = layer; l < a.layers; ++l) out += 4 * static_cast<int64_t>(a.k[l]) * a.k[l + 1];
+        for (int l = 0; l < layer; ++l) out += 4 * a.k[l + 1];
+    }
+#pragma unroll
+    for (int e = 0; e < V; ++e) {
+        const int place = at % cols + e, column = tile % tiles_n * cols + (split && cols == 128 ? grad_column(place) : place);
+        if (column >= N || row >= K) continue;
+        const T value = with_lost(sum[e], lost[e]);
+        if (is_bias) a.out[out + t * N + column] = value;
+        else a.out[out + (static_cast<int64_t>(t) * K + row) * N + column] = value;
+    }
 }
 
 template <typename T>
@@ -724,50 +965,93 @@ hipError_t launch_net_top(NetTop<T> a, hipStream_t stream)
     return hipGetLastError();
 }
 
-// rows per workgroup, the workgroups' numbering, and the bytes of partial sums
+// rows per workgroup, the workgroups' numbering, and the bytes of partial sums; `split`: layers of at least 64 x 64 on split
+// products
 template <typename T>
-static int64_t plan_grads(NetGrads<T>& a)
+static int64_t plan_grads(NetGrads<T>& a, bool split)
 {
     constexpr int kSide = 16 * MatrixOp<T>::kVec;
-    int64_t tiles = 0, rows = 0;
-    for (int l = 0; l < a.layers; ++l) tiles += static_cast<int64_t>((a.k[l] + kSide - 1) / kSide) * ((a.k[l + 1] + kSide - 1) / kSide);
+    a.split = 0;
+    int64_t tiles = 0, split_tiles = 0, rows = 0;
     for (int t = 0; t < 4; ++t) rows += a.n[t];
-    // about two workgroups per compute unit and wave: short shares where rows are few, and never fewer than 64 rows
-    int64_t per = 64;
-    while (per < 4096 && rows / per * tiles > 1024) per *= 2;
-    a.per = static_cast<int>(per);
-    int64_t end = 0;
+    auto tiles_of = [&](int l) -> int64_t {
+        const int height = (a.split >> l) & 1u ? kGradLeft : kSide, width = (a.split >> l) & 1u ? (a.k[l + 1] > 64 ? 128 : 64) : kSide;
+        return static_cast<int64_t>((a.k[l] + height - 1) / height) * ((a.k[l + 1] + width - 1) / width);
+    };
     for (int l = 0; l < a.layers; ++l) {
-        const int64_t lt = static_cast<int64_t>((a.k[l] + kSide - 1) / kSide) * ((a.k[l + 1] + kSide - 1) / kSide);
+        if (split && a.k[l] >= 64 && a.k[l + 1] >= 64) a.split |= 1u << l;
+        ((a.split >> l) & 1u ? split_tiles : tiles) += tiles_of(l);
+    }
+    // Few rows are faster on the float32 instructions, whose tiles are smaller (us with the summation, float32 -> split):
+    // 384-128-128-64-1, 5 tiles: 2,000 rows 21 -> 25, 6,000 33 -> 27, 12,132 48 -> 35, 35,000 93 -> 59, with both pairs of
+    // operands 185 -> 107; eleven layers, 33 tiles: 300 rows 39 -> 49, 2,000 64 -> 63, 12,132 250 -> 150, 47,000 845 -> 420.
+    if (a.split && rows * split_tiles < 20000) return plan_grads(a, false);
+    auto blocks_of = [&](int64_t per, int64_t per_row) {
+        int64_t shares = 0;
+        for (int t = 0; t < 4; ++t) shares += (a.n[t] + per - 1) / per;
+        return shares * per_row;
+    };
+    // about two workgroups per compute unit and wave: short shares where rows are few, and never fewer than 64 rows; beside
+    // split products a sixth of that
+    int64_t per = 64;
+    while (per < 4096 && (split_tiles ? blocks_of(per, tiles) > 96 : rows / per * tiles > 1024)) per *= 2;
+    a.per = static_cast<int>(per);
+    // split products: all workgroups at once, two per compute unit, or as few such rounds as shares of up to 2,048 rows make
+    // (520 workgroups on 512 places took 56 us where 505 take 50)
+    const int64_t plain = split_tiles ? std::min<int64_t>(blocks_of(per, tiles), 128) : 0;
+    int64_t share = 4 * kGradChunk;
+    for (int64_t rounds = 1; split_tiles && blocks_of(share, split_tiles) > 512 * rounds - plain;) {
+        share += kGradChunk;
+        if (share > 64 * kGradChunk) share = 4 * kGradChunk, ++rounds;
+    }
+    a.per_split = static_cast<int>(share);
+    int64_t end = 0, base = 0;
+    for (int l = 0; l < a.layers; ++l) {
+        const bool is_split = (a.split >> l) & 1u;
+        const int64_t size = is_split ? (kGradLeft + 1) * (a.k[l + 1] > 64 ? 128 : 64) : kSide * kSide + kSide;
+        const int64_t rows_each = is_split ? a.per_split : per;
         for (int t = 0; t < 4; ++t) {
-            end += (a.n[t] + per - 1) / per * lt;
-            a.job_end[l * 4 + t] = static_cast<int>(end);
+            const int64_t blocks = (a.n[t] + rows_each - 1) / rows_each * tiles_of(l);
+            a.job_base[l * 4 + t] = base;
+            base += blocks * size;
+            a.job_end[l * 4 + t] = static_cast<int>(end += blocks);
         }
     }
-    return end * (kSide * kSide + kSide) * static_cast<int64_t>(sizeof(T));
+    return base * static_cast<int64_t>(sizeof(T));
 }
 
+// (which of the two plans a launch takes depends on its operands' alignment too, which may not be known yet)
 template <typename T>
-size_t net_grads_workspace(NetGrads<T> a) { return static_cast<size_t>(plan_grads(a)) + 16; }
+size_t net_grads_workspace(NetGrads<T> a)
+{
+    const int64_t plain = plan_grads(a, false), split = std::is_same<T, float>::value ? plan_grads(a, true) : 0;
+    return static_cast<size_t>(std::max(plain, split)) + 16;
+}
 
 template <typename T>
 hipError_t launch_net_grads(NetGrads<T> a, void* workspace, hipStream_t stream)
 {
-    plan_grads(a);
     constexpr int V = MatrixOp<T>::kVec;
-    const int blocks = a.job_end[a.layers * 4 - 1];
-    int64_t elements = 0;
     a.whole = 0;
+    bool split = std::is_same<T, float>::value;
     for (int l = 0; l < a.layers; ++l) {
-        elements += 4 * (static_cast<int64_t>(a.k[l]) * a.k[l + 1] + a.k[l + 1]);
         // (operands that a layer does not have are null, which is aligned)
         const uintptr_t bits = reinterpret_cast<uintptr_t>(a.right[l]) | reinterpret_cast<uintptr_t>(a.right2[l]) |
                                reinterpret_cast<uintptr_t>(a.left[l]) | reinterpret_cast<uintptr_t>(a.left2[l]);
         const bool whole = a.k[l] % V == 0 && a.k[l + 1] % V == 0 && (bits & 15u) == 0 && (l > 0 || (aligned<T>(a.x, a.n) && aligned<T>(a.x2, a.n)));
         if (whole) a.whole |= 1u << l;
+        const bool ones = ((a.first >> l & 1u) && !a.right[l]) || ((a.second >> l & 1u) && !a.right2[l]);
+        if (a.k[l] >= 64 && a.k[l + 1] >= 64 && (!whole || ones)) split = false;
     }
+    plan_grads(a, split);
+    const int blocks = a.job_end[a.layers * 4 - 1];
     if (blocks > 0) weight_grad_kernel<T><<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream>>>(a, static_cast<T*>(workspace));
-    grad_sum_kernel<T><<<dim3(static_cast<unsigned>((elements + 255) / 256)), dim3(256), 0, stream>>>(a, static_cast<const T*>(workspace), elements);
+    unsigned sums = 0;
+    for (int l = 0; l < a.layers; ++l) {
+        const int rows = a.split >> l & 1u ? kGradLeft : 16 * V, cols = a.split >> l & 1u ? (a.k[l + 1] > 64 ? 128 : 64) : 16 * V;
+        sums += 4u * ((a.k[l] + rows - 1) / rows) * ((a.k[l + 1] + cols - 1) / cols) * ((rows * cols + cols + 64 * V - 1) / (64 * V));
+    }
+    grad_sum_kernel<T><<<dim3(sums), dim3(256), 0, stream>>>(a, static_cast<const T*>(workspace));
     return hipGetLastError();
 }
 

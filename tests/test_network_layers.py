@@ -152,6 +152,77 @@ def test_split_products(rows, k, n_out, transposed):
                 assert (out2[i] == 1).all(), (name, i)
 
 
+class _Grads(ctypes.Structure):
+    _fields_ = ([(name, ctypes.c_void_p * 4) for name in ("x", "x2", "scale")] +
+                [(name, ctypes.c_void_p * 12) for name in ("left", "right", "left2", "right2")] +
+                [("row0", ctypes.c_int64 * 4), ("n", ctypes.c_int32 * 4), ("layers", ctypes.c_int32), ("widths", ctypes.c_int32 * 13)] +
+                [(name, ctypes.c_uint32) for name in ("first", "second")] + [(name, ctypes.c_int32) for name in ("scale_first", "scale_second")] +
+                [(name, ctypes.c_void_p) for name in ("out", "workspace")])
+
+
+# Weight gradients on split products (from 20,000 rows times tiles on): tiles of 128 x 128 and 128 x 64, widths that are no
+# multiple of them, narrow layers beside them; rows around the 32 of a chunk and the 128 of a share; both pairs of operands or
+# the first alone.  The float32 sums and the split stay below 2e-6 of sum |left| |right|.  Infinite and undefined operands
+# give what they give in float64, element by element; odd row numbers and a pointer off its alignment take the other form.
+@pytest.mark.parametrize("widths", [(384, 64, 128, 1), (64, 68, 132, 8, 1), (196, 192, 64, 1)])
+@pytest.mark.parametrize("rows", [(9001, 33, 0, 1023), (127, 12800, 1, 31)])
+@pytest.mark.parametrize("both", [False, True])
+def test_weight_gradients_on_split_products(widths, rows, both):
+    from khan_amd import _lib
+    lib = _lib.load()
+    print("case:", widths, rows, both, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    layers, total, row0 = len(widths) - 1, sum(rows), [sum(rows[:t]) for t in range(4)]
+    # (the first column of the padding keeps arrays apart, so that `shift` may move them off their alignment)
+    make = lambda w: torch.randn(total * w + 4, device="cuda", generator=gen)
+    left, left2 = ([make(k) for k in widths[:-1]] for _ in range(2))
+    right, right2 = ([make(k) for k in widths[1:]] for _ in range(2))
+    scale = [torch.randn(n + 1, device="cuda", generator=gen) for n in rows]
+
+    def gradients(shift=0):
+        a = _Grads(layers=layers, first=(1 << layers) - 1, second=(1 << layers) - 1 if both else 0, scale_first=1, scale_second=0)
+        for i, w in enumerate(widths):
+            a.widths[i] = w
+        for t in range(4):
+            a.n[t], a.row0[t], a.scale[t] = rows[t], row0[t], scale[t].data_ptr()
+            a.x[t], a.x2[t] = (v[0].data_ptr() + 4 * row0[t] * widths[0] for v in (left, left2))
+        for l in range(layers):
+            a.left[l], a.left2[l], a.right2[l] = left[l].data_ptr(), left2[l].data_ptr(), right2[l].data_ptr()
+            a.right[l] = right[l].data_ptr() + 4 * (shift if l == 0 else 0) if l < layers - 1 else None
+        out = torch.full((4 * sum((k + 1) * n for k, n in zip(widths, widths[1:])),), 7.0, device="cuda")
+        work = torch.empty(lib.khan_net_grads_workspace_bytes_f32(ctypes.byref(a)), dtype=torch.uint8, device="cuda")
+        a.out, a.workspace = out.data_ptr(), work.data_ptr()
+        assert lib.khan_net_grads_f32(ctypes.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+        return out.cpu().double()
+
+    def reference(shift=0):
+        weights, sizes, sums, sum_sizes = [], [], [], []
+        rows_of = lambda v, w, t, s=0: v[s:s + total * w].view(total, w)[row0[t]:row0[t] + rows[t]].cpu().double()
+        for l, (k, n) in enumerate(zip(widths, widths[1:])):
+            for t in range(4):
+                s = scale[t][:rows[t]].cpu().double()[:, None]
+                r = (rows_of(right[l], n, t, shift if l == 0 else 0) if l < layers - 1 else torch.ones(rows[t], 1, dtype=torch.float64)) * s
+                pairs = [(rows_of(left[l], k, t), r)] + ([(rows_of(left2[l], k, t), rows_of(right2[l], n, t))] if both else [])
+                weights.append(sum(p.t() @ q for p, q in pairs).reshape(-1))
+                sizes.append(sum(p.abs().t() @ q.abs() for p, q in pairs).reshape(-1))
+                sums.append(r.sum(0))
+                sum_sizes.append(r.abs().sum(0))
+        return torch.cat(weights + sums), torch.cat(sizes + sum_sizes)
+
+    for shift in (0, 1):
+        got, (want, size) = gradients(shift), reference(shift)
+        assert ((got - want).abs() <= 2e-6 * size).all(), (shift, ((got - want).abs() / size).max().item())
+    for what in (float("inf"), float("nan")):
+        big = rows.index(max(rows))
+        left[0][(row0[big] + 40) * widths[0] + 3] = what
+        right[1][(row0[big] + 7) * widths[2] + 1] = -what
+        got, (want, size) = gradients(), reference()
+        assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+        known = torch.isfinite(want)
+        assert torch.equal(got[torch.isinf(want)], want[torch.isinf(want)])
+        assert ((got - want).abs() <= 2e-6 * size)[known].all()
+
+
 @pytest.mark.parametrize("absolute", [False, True])
 def test_celu_of_small_and_large_arguments(absolute):
     """The layers' float32 CELU over the binades of negative arguments from -1e-30 on (below, the split operands' smallest parts
