@@ -454,6 +454,18 @@ int khan_ani_charges_f64(const double *xs, const double *ys, const double *zs, c
                          double *q_grads, double *x_grads, double *y_grads, double *z_grads, int32_t outputs_zeroed,
                          khan_stream_t stream);
 
+/* The same with gradients, for outputs that hold nothing yet: outputs[0 .. n_outputs), in which e and the gradients lie, is set
+ * to zero first (atoms outside every molecule keep the zeros).  order: n_mols ints of scratch, in which the same launch
+ * may leave the molecules by decreasing size for the pass to walk; NULL: batch order.  The results are the same. */
+int khan_ani_charges_begun_f32(const float *xs, const float *ys, const float *zs, const float *qs, const int32_t *mos,
+                               const int32_t *macs, int32_t n_mols, int64_t n_atoms, const float *grads, float *e,
+                               float *q_grads, float *x_grads, float *y_grads, float *z_grads, float *outputs,
+                               int64_t n_outputs, int32_t *order, khan_stream_t stream);
+int khan_ani_charges_begun_f64(const double *xs, const double *ys, const double *zs, const double *qs, const int32_t *mos,
+                               const int32_t *macs, int32_t n_mols, int64_t n_atoms, const double *grads, double *e,
+                               double *q_grads, double *x_grads, double *y_grads, double *z_grads, double *outputs,
+                               int64_t n_outputs, int32_t *order, khan_stream_t stream);
+
 /* Plain Coulomb sums, E_m = k sum_{i<j in m} q_i q_j / r_ij, and their gradients: the charge kernels with
  * the damping (1 - f_C) switched off and the constant chosen by the caller (k = 1 for charges in e and
  * distances in the unit the energy is wanted in).  No reference counterpart: khan's own op is the damped,

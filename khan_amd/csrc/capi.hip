@@ -386,14 +386,15 @@ int charge_impl(const T* xs, const T* ys, const T* zs, const T* qs, const int32_
 template <typename T>
 int charge_grad_impl(const T* xs, const T* ys, const T* zs, const T* qs, const int32_t* mos,
                      const int32_t* macs, int32_t n_mols, const T* grads, bool damped, T k, T* qg, T* gx, T* gy, T* gz,
-                     bool want_xyz, khan_stream_t stream, T* energies = nullptr, int64_t n_atoms = INT64_MAX, bool zeroed = false)
+                     bool want_xyz, khan_stream_t stream, T* energies = nullptr, int64_t n_atoms = INT64_MAX, bool zeroed = false,
+                     const int32_t* order = nullptr)
 {
     if (n_mols < 0) return KHAN_ERR_INVALID_ARG;
     if (n_mols == 0) return KHAN_OK;
     if (!xs || !ys || !zs || !qs || !mos || !macs || !grads) return KHAN_ERR_INVALID_ARG;
     if (want_xyz ? (!gx || !gy || !gz) : !qg) return KHAN_ERR_INVALID_ARG;
     return hip_status(khan::launch_charge_grad<T>(xs, ys, zs, qs, mos, macs, n_mols, n_atoms, grads, damped, k, qg,
-                                                  want_xyz ? gx : nullptr, gy, gz, energies, zeroed, as_stream(stream)));
+                                                  want_xyz ? gx : nullptr, gy, gz, energies, zeroed, order, as_stream(stream)));
 }
 
 }  // namespace
@@ -431,6 +432,17 @@ static int ani_charges(const T* xs, const T* ys, const T* zs, const T* qs, const
     if (!grads) return charge_impl<T>(xs, ys, zs, qs, mos, macs, n_mols, true, k, e, stream, n_atoms);
     return charge_grad_impl<T>(xs, ys, zs, qs, mos, macs, n_mols, grads, true, k, q_grads, gx, gy, gz, gx != nullptr, stream, e, n_atoms,
                                outputs_zeroed != 0);
+}
+
+template <typename T>
+static int ani_charges_begun(const T* xs, const T* ys, const T* zs, const T* qs, const int32_t* mos, const int32_t* macs, int32_t n_mols,
+                             int64_t n_atoms, const T* grads, T k, T* e, T* q_grads, T* gx, T* gy, T* gz, T* outputs, int64_t n_outputs,
+                             int32_t* order, khan_stream_t stream)
+{
+    if (n_mols < 0 || n_atoms < 0 || n_outputs < 0 || (n_outputs > 0 && !outputs) || (n_mols > 0 && !macs)) return KHAN_ERR_INVALID_ARG;
+    const int st = hip_status(khan::launch_charge_begin<T>(macs, n_mols, n_atoms, order, outputs, n_outputs, as_stream(stream)));
+    if (st != KHAN_OK) return st;
+    return charge_grad_impl<T>(xs, ys, zs, qs, mos, macs, n_mols, grads, true, k, q_grads, gx, gy, gz, gx != nullptr, stream, e, n_atoms, true, order);
 }
 
 // The per-type networks layer by layer (khan_net_*): the caller's structures, typed.
@@ -767,6 +779,21 @@ int khan_ani_charges_f64(const double* xs, const double* ys, const double* zs, c
 {
     return ani_charges<double>(xs, ys, zs, qs, mos, macs, n_mols, n_atoms, grads, static_cast<double>(khan::kChargeK_f), e, q_grads, gx, gy, gz,
                                outputs_zeroed, stream);
+}
+
+int khan_ani_charges_begun_f32(const float* xs, const float* ys, const float* zs, const float* qs, const int32_t* mos, const int32_t* macs,
+                               int32_t n_mols, int64_t n_atoms, const float* grads, float* e, float* q_grads, float* gx, float* gy, float* gz,
+                               float* outputs, int64_t n_outputs, int32_t* order, khan_stream_t stream)
+{
+    return ani_charges_begun<float>(xs, ys, zs, qs, mos, macs, n_mols, n_atoms, grads, khan::kChargeK_f, e, q_grads, gx, gy, gz, outputs, n_outputs,
+                                    order, stream);
+}
+int khan_ani_charges_begun_f64(const double* xs, const double* ys, const double* zs, const double* qs, const int32_t* mos, const int32_t* macs,
+                               int32_t n_mols, int64_t n_atoms, const double* grads, double* e, double* q_grads, double* gx, double* gy, double* gz,
+                               double* outputs, int64_t n_outputs, int32_t* order, khan_stream_t stream)
+{
+    return ani_charges_begun<double>(xs, ys, zs, qs, mos, macs, n_mols, n_atoms, grads, static_cast<double>(khan::kChargeK_f), e, q_grads, gx, gy,
+                                     gz, outputs, n_outputs, order, stream);
 }
 
 int khan_dense_first_f32(const float* const* rows_host4, const int32_t* acs_host, const float* const* wt_host4,

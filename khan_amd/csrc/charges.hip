@@ -27,10 +27,12 @@ namespace {
 // What a pair at squared distance d2 contributes: u = (1 - f_C) / r and du = d/dr[(1 - f_C) / r] / r, both zero for
 // coincident atoms.  kDamped = false drops the cutoff function: plain Coulomb pairs (the reference's op is the damped form).
 // f_C is evaluated in every lane and selected: a branch would be taken by nearly every wavefront anyway.
+// `Constants` are made once per kernel.
 template <typename T, bool kDamped> struct PairTerms;
 // float: the hardware reciprocal square root with one Newton step and the minimax cutoff polynomials of the AEV kernels
 template <bool kDamped> struct PairTerms<float, kDamped> {
-    static __device__ __forceinline__ void of(float d2, float& u, float& du)
+    struct Constants {};
+    static __device__ __forceinline__ void of(const Constants&, float d2, float& u, float& du)
     {
         const float r = Fast<float>::sqrt_rn(d2);
         const float inv = d2 > 0.0f ? Fast<float>::rcp(r) : 0.0f;
@@ -48,23 +50,39 @@ template <bool kDamped> struct PairTerms<float, kDamped> {
 // double: no library call, no square root and no angle.  1/r from v_rsq_f64 (5e-8) and one third-order step.  1 - f_C =
 // sin^2(pi r / 2 R_c) = d2 q(d2) and 2 d(1 - f_C)/d(d2) = (d/dr) / r are entire functions of d2: polynomials of degree
 // nine in d2 (Chebyshev interpolation on [0, R_c^2]), exact to 4e-16 of q and 1e-16.  (Before: a square root, a folded half
-// angle, its sine and cosine: 106 vector instructions per pair over the whole kernel, 92 now.)
+// angle, its sine and cosine: 106 vector instructions per pair over the whole kernel, 92 with the polynomials' coefficients in
+// vector registers, where every step of Horner's scheme copies one first, 74 with them in scalar registers.)
 template <bool kDamped> struct PairTerms<double, kDamped> {
+    struct Constants {
+        double q[10], t[10];
+        __device__ __forceinline__ Constants()
+        {
+            constexpr double kQ[10] = {0.11660686212575191, -0.004532386764938009, 7.046765314658188e-05, -5.869294224571146e-07,
+                                       3.0417776911092683e-09, -1.0748245519813352e-11, 2.7545314816657834e-14,
+                                       -5.3522125411118236e-17, 8.115026416218573e-20, -8.999642674693997e-23};
+            constexpr double kT[10] = {0.23321372425150377, -0.018129547059751505, 0.0004228059188787524, -4.695435379265704e-06,
+                                       3.0417776808067906e-08, -1.2897893108818512e-10, 3.856331055586389e-13,
+                                       -8.562890949169944e-16, 1.4589662776261427e-18, -1.7805957172843363e-21};
+            if constexpr (kDamped) {
+#pragma unroll
+                for (int k = 0; k < 10; ++k) {
+                    q[k] = kQ[k];
+                    t[k] = kT[k];
+                    asm("" : "+s"(q[k]));          // (a value of its own in scalar registers)
+                    asm("" : "+s"(t[k]));
+                }
+            }
+        }
+    };
     static __device__ __forceinline__ double poly(const double (&c)[10], double x)
     {
-        double v = c[9];
+        double v = fma(c[9], x, c[8]);
 #pragma unroll
-        for (int k = 8; k >= 0; --k) v = fma(v, x, c[k]);
+        for (int k = 7; k >= 0; --k) v = fma(v, x, c[k]);
         return v;
     }
-    static __device__ __forceinline__ void of(double d2, double& u, double& du)
+    static __device__ __forceinline__ void of(const Constants& k, double d2, double& u, double& du)
     {
-        constexpr double kQ[10] = {0.11660686212575191, -0.004532386764938009, 7.046765314658188e-05, -5.869294224571146e-07,
-                                   3.0417776911092683e-09, -1.0748245519813352e-11, 2.7545314816657834e-14,
-                                   -5.3522125411118236e-17, 8.115026416218573e-20, -8.999642674693997e-23};
-        constexpr double kT[10] = {0.23321372425150377, -0.018129547059751505, 0.0004228059188787524, -4.695435379265704e-06,
-                                   3.0417776808067906e-08, -1.2897893108818512e-10, 3.856331055586389e-13,
-                                   -8.562890949169944e-16, 1.4589662776261427e-18, -1.7805957172843363e-21};
         const double y = __builtin_amdgcn_rsq(d2);
         const double e = fma(-d2 * y, y, 1.0);
         double inv = fma(y * e, fma(e, 0.375, 0.5), y);
@@ -73,7 +91,7 @@ template <bool kDamped> struct PairTerms<double, kDamped> {
         if constexpr (kDamped) {
             constexpr double kRc2 = static_cast<double>(kR_Rc_f) * static_cast<double>(kR_Rc_f);
             const bool in = d2 <= kRc2;
-            const double sq = d2 * poly(kQ, d2), tq = poly(kT, d2);       // (without meaning outside)
+            const double sq = d2 * poly(k.q, d2), tq = poly(k.t, d2);       // (without meaning outside)
             s = in ? sq : 1.0;
             t = in ? tq : 0.0;
         }
@@ -90,11 +108,12 @@ struct ChargeArgs {
     const T* grads;          // gradients only
     T K;
     T *E, *q_grads, *gX, *gY, *gZ;      // with gradients each of E, q_grads and (gX, gY, gZ) may be null
+    const int32_t* order;               // the molecules of 65 to 256 atoms by decreasing size in front (charge_begin_kernel), or null
 };
 
 // A molecule of up to 64 atoms in one wavefront.
 template <typename T, bool kDamped, bool kGrad>
-__device__ __forceinline__ void charge_small(const ChargeArgs<T>& a, int mol, int n)
+__device__ __forceinline__ void charge_small(const ChargeArgs<T>& a, const typename PairTerms<T, kDamped>::Constants& constants, int mol, int n)
 {
     const int lane = threadIdx.x & 63;
     const int off = a.MOs[mol];
@@ -113,7 +132,7 @@ __device__ __forceinline__ void charge_small(const ChargeArgs<T>& a, int mol, in
         const bool valid = (i < n) && jok && (kGrad ? jl != i : jl > i);
         const T dx = xi - xj, dy = yi - yj, dz = zi - zj;
         T u, du;
-        PairTerms<T, kDamped>::of(dx * dx + dy * dy + dz * dz, u, du);
+        PairTerms<T, kDamped>::of(constants, dx * dx + dy * dy + dz * dz, u, du);
         if constexpr (!kGrad) {
             acc += valid ? qi * qj * u : T(0);
         } else {
@@ -164,7 +183,7 @@ template <typename T> struct __align__(16) ChargeTile<T, true> {
 };
 
 template <typename T, bool kDamped, bool kGrad>
-__device__ __forceinline__ void charge_tile(const ChargeArgs<T>& a, ChargeTile<T, kGrad>& S, int mol, int n)
+__device__ __forceinline__ void charge_tile(const ChargeArgs<T>& a, const typename PairTerms<T, kDamped>::Constants& constants, ChargeTile<T, kGrad>& S, int mol, int n)
 {
     typedef typename Fast<T>::vec2 vec2;
     static_assert(kMediumMaxAtoms == 256, "one atom per thread of a 256-thread workgroup");
@@ -199,35 +218,53 @@ __device__ __forceinline__ void charge_tile(const ChargeArgs<T>& a, ChargeTile<T
         j -= j >= n ? n : 0;
         j -= j >= n ? n : 0;
         T fx = T(0), fy = T(0), fz = T(0), dq = T(0);
-        auto pair = [&](T q_i, bool act) {
+        // what a pair adds to either side, and where its partner's slot is
+        struct Terms {
+            int j;
+            T q, u, wx, wy, wz;
+        };
+        auto terms = [&](T q_i, bool act) -> Terms {
             j = j + 1 == n ? 0 : j + 1;
             const vec2 xy = S.in[0][j], zq = S.in[1][j];
             const T dx = own_xy.x - xy.x, dy = own_xy.y - xy.y, dz = own_zq.x - zq.x;
             T u, du;
-            PairTerms<T, kDamped>::of(dx * dx + dy * dy + dz * dz, u, du);
+            PairTerms<T, kDamped>::of(constants, dx * dx + dy * dy + dz * dz, u, du);
             const T qq = q_i * zq.y;
             if constexpr (!kGrad) {
                 e_acc = fma(qq, u, e_acc);
+                return {};
             } else {
                 dq = fma(act ? zq.y : T(0), u, dq);
                 const T wq = qq * du;                    // q_i q_j d/dr[(1-f_C)/r] / r
-                const T wx = wq * dx, wy = wq * dy, wz = wq * dz;
-                fx += wx;
-                fy += wy;
-                fz += wz;
-                vec2 pa = S.acc[wave][0][j], pb = S.acc[wave][1][j];     // distinct j across the lanes of this wavefront
-                pa.x -= wx;
-                pa.y -= wy;
-                pb.x -= wz;
-                pb.y = fma(q_i, u, pb.y);
-                S.acc[wave][0][j] = pa;
-                S.acc[wave][1][j] = pb;
+                const Terms p = {j, q_i, u, wq * dx, wq * dy, wq * dz};
+                fx += p.wx;
+                fy += p.wy;
+                fz += p.wz;
+                return p;
+            }
+        };
+        auto give = [&](const Terms& p) {
+            if constexpr (kGrad) {
+                vec2 pa = S.acc[wave][0][p.j], pb = S.acc[wave][1][p.j];     // distinct j across the lanes of this wavefront
+                pa.x -= p.wx;
+                pa.y -= p.wy;
+                pb.x -= p.wz;
+                pb.y = fma(p.q, p.u, pb.y);
+                S.acc[wave][0][p.j] = pa;
+                S.acc[wave][1][p.j] = pb;
                 wave_lds_fence();                        // the next round may touch slots written here
             }
         };
+        // two rounds' terms side by side (their chains of dependent multiply-adds fill each other's waits), then their sums
         const int full = min(d1, half);
-        for (int d = d0; d < full; ++d) pair(q_own, true);
-        if (d1 > half) pair(i < (n >> 1) ? q_own : T(0), i < (n >> 1));      // the half round of an even n: the lower half only
+        int d = d0;
+        for (; d + 1 < full; d += 2) {
+            const Terms p0 = terms(q_own, true), p1 = terms(q_own, true);
+            give(p0);
+            give(p1);
+        }
+        if (d < full) give(terms(q_own, true));
+        if (d1 > half) give(terms(i < (n >> 1) ? q_own : T(0), i < (n >> 1)));      // the half round of an even n: the lower half only
         if constexpr (kGrad) {
             if (i < n) {                                 // the atoms' own side joins this wavefront's copy
                 vec2 pa = S.acc[wave][0][i], pb = S.acc[wave][1][i];
@@ -286,7 +323,7 @@ __device__ __forceinline__ void charge_tile(const ChargeArgs<T>& a, ChargeTile<T
 // blocks.  The energy is half the sum over atoms of q_i times the atom's sum, added to E[mol] (zeroed before the launch)
 // by one floating-point atomic per workgroup and block: its last bits depend on the order of those additions.
 template <typename T, bool kDamped, bool kGrad>
-__device__ __forceinline__ void charge_large(const ChargeArgs<T>& a, typename Fast<T>::vec4* tile, T* wpart, int column, int columns, int part, int parts)
+__device__ __forceinline__ void charge_large(const ChargeArgs<T>& a, const typename PairTerms<T, kDamped>::Constants& constants, typename Fast<T>::vec4* tile, T* wpart, int column, int columns, int part, int parts)
 {
     typedef typename Fast<T>::vec4 vec4;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -326,7 +363,7 @@ __device__ __forceinline__ void charge_large(const ChargeArgs<T>& a, typename Fa
                         const vec4 aj = tile[t];                   // the same address in every lane
                         const T dx = xi - aj.x, dy = yi - aj.y, dz = zi - aj.z;
                         T u, du;
-                        PairTerms<T, kDamped>::of(dx * dx + dy * dy + dz * dz, u, du);      // zero for the atom itself (r = 0)
+                        PairTerms<T, kDamped>::of(constants, dx * dx + dy * dy + dz * dz, u, du);      // zero for the atom itself (r = 0)
                         su = fma(aj.w, u, su);
                         if constexpr (kGrad) {
                             const T w = aj.w * du;
@@ -358,13 +395,18 @@ __device__ __forceinline__ void charge_large(const ChargeArgs<T>& a, typename Fa
 }
 
 // One launch for every size.  Workgroups 0 .. large - 1 (columns x parts of them) share the molecules of more than 256 atoms.
-// The workgroups behind them take `per` molecules each: the wavefronts those of up to 64 atoms (with per = 1 every fourth
-// workgroup the next four), the workgroup those of 65 to 256 one after the other.  (Three launches, one per size, cost
-// 10 us where two of them found nothing to do.)  Four workgroups per compute unit: 128 registers in double.
+// Behind them come, with per = 1, a workgroup for every four molecules, whose wavefronts take those of up to 64 atoms, and one
+// for every molecule, which takes those of 65 to 256 (in the first ones' places a wavefront with 64 atoms had the compute unit
+// that came upon it last work for 35 us after all others).  With per = 4 a workgroup does both for its four molecules.
+// (Three launches, one per size, cost 10 us where two of them found nothing to do.)  Four workgroups per compute unit, which
+// LDS allows.  4,096 boxes of 64 to 256 atoms in double, energy and both gradients with the launch before: 224 -> 156 us
+// (coefficients in scalar registers, size order, first places for the small molecules, two rounds side by side); vector
+// issue binds, 60 instructions a pair, with LDS (six 16-byte accesses a pair) at two thirds of its rate.
 template <typename T, bool kDamped, bool kGrad>
 __global__ __launch_bounds__(256, 4) void charge_kernel(ChargeArgs<T> a, int columns, int parts, int per)
 {
     __shared__ ChargeTile<T, kGrad> S;
+    const typename PairTerms<T, kDamped>::Constants constants;
     const int large = columns * parts;
     const int b = static_cast<int>(blockIdx.x) - large;
     if (b < 0) {
@@ -372,26 +414,77 @@ __global__ __launch_bounds__(256, 4) void charge_kernel(ChargeArgs<T> a, int col
         T* wpart;
         if constexpr (kGrad) wpart = reinterpret_cast<T*>(S.acc[0]);
         else wpart = S.wpart;
-        charge_large<T, kDamped, kGrad>(a, reinterpret_cast<typename Fast<T>::vec4*>(&S.in[0][0]), wpart, g % columns, columns, g / columns, parts);
+        charge_large<T, kDamped, kGrad>(a, constants, reinterpret_cast<typename Fast<T>::vec4*>(&S.in[0][0]), wpart, g % columns, columns, g / columns, parts);
         return;
     }
     const int wave = uniform(threadIdx.x >> 6);
-    const int64_t first = static_cast<int64_t>(b) * per;
-    if (per == 4 || (b & 3) == 0) {
-        const int64_t mol = first + wave;
+    const int fours = (a.n_mols - 1) / 4 + 1;
+    if (b < fours) {
+        const int64_t mol = 4 * static_cast<int64_t>(b) + wave;
         if (mol < a.n_mols) {
             const int n = uniform(a.MACs[mol]);
-            if (n <= kSmallMaxAtoms) charge_small<T, kDamped, kGrad>(a, static_cast<int>(mol), n);
+            if (n <= kSmallMaxAtoms) charge_small<T, kDamped, kGrad>(a, constants, static_cast<int>(mol), n);
         }
+        if (per == 1) return;
     }
-    for (int64_t mol = first; mol < min(first + per, static_cast<int64_t>(a.n_mols)); ++mol) {
+    const int64_t first = per == 1 ? b - fours : 4 * static_cast<int64_t>(b);
+    for (int64_t at = first; at < min(first + per, static_cast<int64_t>(a.n_mols)); ++at) {
+        const int mol = a.order ? a.order[at] : static_cast<int>(at);
         const int n = uniform(a.MACs[mol]);
         if (n > kSmallMaxAtoms && n <= kMediumMaxAtoms) {
-            charge_tile<T, kDamped, kGrad>(a, S, static_cast<int>(mol), n);
+            charge_tile<T, kDamped, kGrad>(a, constants, S, mol, n);
             __syncthreads();         // the next molecule reuses the tile
         }
     }
 }
+
+// Before the launch: zeros in the outputs (atoms outside every molecule keep them, and the energies of molecules of more than
+// 256 atoms are added up), and by the first workgroup, where `order` is asked for, the molecules of 65 to 256 atoms by
+// decreasing size, the others behind them: a counting sort, in no particular order inside a size (every molecule's results
+// are its own).  A launch lasts only a few molecules' time and in batch order ended with a third of the wavefronts' places empty.
+constexpr int kOrderMost = 16384;
+template <typename T>
+__global__ __launch_bounds__(1024) void charge_begin_kernel(const int32_t* __restrict__ MACs, int n_mols, int32_t* __restrict__ order,
+                                                            T* __restrict__ outputs, int64_t n_outputs)
+{
+    const int tid = threadIdx.x;
+    const int sorting = order ? 1 : 0;
+    if (static_cast<int>(blockIdx.x) >= sorting) {
+        const int64_t step = static_cast<int64_t>(gridDim.x - sorting) * 1024;
+        for (int64_t i = static_cast<int64_t>(blockIdx.x - sorting) * 1024 + tid; i < n_outputs; i += step) outputs[i] = T(0);
+        return;
+    }
+    constexpr int kBins = kMediumMaxAtoms + 1, kEach = kOrderMost / 1024;
+    __shared__ int bin[2][512];
+    if (tid < 512) bin[0][tid] = 0;
+    __syncthreads();
+    int key[kEach];
+#pragma unroll
+    for (int k = 0; k < kEach; ++k) {
+        const int mol = k * 1024 + tid;
+        const int n = mol < n_mols ? MACs[mol] : 0;
+        key[k] = mol >= n_mols ? -1 : n > kSmallMaxAtoms && n <= kMediumMaxAtoms ? kMediumMaxAtoms - n : kBins - 1;
+    }
+#pragma unroll
+    for (int k = 0; k < kEach; ++k)
+        if (key[k] >= 0) atomicAdd(&bin[0][key[k]], 1);
+    __syncthreads();
+    int from = 0;
+    for (int d = 1; d < kBins; d <<= 1) {                 // inclusive sums
+        if (tid < 512) bin[from ^ 1][tid] = bin[from][tid] + (tid >= d ? bin[from][tid - d] : 0);
+        from ^= 1;
+        __syncthreads();
+    }
+    if (tid < 512) bin[from ^ 1][tid] = tid > 0 ? bin[from][tid - 1] : 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kEach; ++k)
+        if (key[k] >= 0) order[atomicAdd(&bin[from ^ 1][key[k]], 1)] = k * 1024 + tid;
+}
+
+// a workgroup per four molecules where they are small, per molecule where a workgroup has to work on each: 4,096 boxes on a
+// quarter of the workgroups end when the compute unit with the largest boxes does
+int charge_mols_per_workgroup(int32_t n_mols, int64_t n_atoms) { return n_atoms > 32 * static_cast<int64_t>(n_mols) ? 1 : 4; }
 
 template <typename T, bool kGrad>
 hipError_t launch_charges(const ChargeArgs<T>& a, int64_t n_atoms, bool damped, bool zeroed, hipStream_t stream)
@@ -406,10 +499,8 @@ hipError_t launch_charges(const ChargeArgs<T>& a, int64_t n_atoms, bool damped, 
             if (e != hipSuccess) return e;
         }
     }
-    // a workgroup per four molecules where they are small, per molecule where a workgroup has to work on each: 4,096
-    // boxes on a quarter of the workgroups end when the compute unit with the largest boxes does
-    const int per = n_atoms > 32 * static_cast<int64_t>(a.n_mols) ? 1 : 4;
-    const int64_t blocks = (static_cast<int64_t>(a.n_mols) + per - 1) / per + static_cast<int64_t>(columns) * parts;
+    const int per = charge_mols_per_workgroup(a.n_mols, n_atoms);
+    const int64_t blocks = (static_cast<int64_t>(a.n_mols) + 3) / 4 + (per == 1 ? a.n_mols : 0) + static_cast<int64_t>(columns) * parts;
     const auto kernel = damped ? charge_kernel<T, true, kGrad> : charge_kernel<T, false, kGrad>;
     kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream>>>(a, std::max(columns, 1), columns ? parts : 0, per);
     return hipGetLastError();
@@ -421,21 +512,34 @@ template <typename T>
 hipError_t launch_charge_energy(const T* X, const T* Y, const T* Z, const T* Q, const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
                                 int64_t n_atoms, bool damped, T K, T* E, hipStream_t stream)
 {
-    return launch_charges<T, false>(ChargeArgs<T>{X, Y, Z, Q, MOs, MACs, n_mols, nullptr, K, E, nullptr, nullptr, nullptr, nullptr}, n_atoms, damped,
+    return launch_charges<T, false>(ChargeArgs<T>{X, Y, Z, Q, MOs, MACs, n_mols, nullptr, K, E, nullptr, nullptr, nullptr, nullptr, nullptr}, n_atoms, damped,
                                     false, stream);
 }
 
 template <typename T>
 hipError_t launch_charge_grad(const T* X, const T* Y, const T* Z, const T* Q, const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
                               int64_t n_atoms, const T* grads, bool damped, T K, T* q_grads, T* gX, T* gY, T* gZ, T* E, bool zeroed,
-                              hipStream_t stream)
+                              const int32_t* order, hipStream_t stream)
 {
-    return launch_charges<T, true>(ChargeArgs<T>{X, Y, Z, Q, MOs, MACs, n_mols, grads, K, E, q_grads, gX, gY, gZ}, n_atoms, damped, zeroed, stream);
+    return launch_charges<T, true>(ChargeArgs<T>{X, Y, Z, Q, MOs, MACs, n_mols, grads, K, E, q_grads, gX, gY, gZ, order}, n_atoms, damped, zeroed, stream);
 }
+
+// Zeros in `outputs`; `order` (n_mols ints): set to null where the size order does not pay.
+template <typename T>
+hipError_t launch_charge_begin(const int32_t* MACs, int32_t n_mols, int64_t n_atoms, int32_t*& order, T* outputs, int64_t n_outputs, hipStream_t stream)
+{
+    if (n_mols <= 256 || n_mols > kOrderMost || charge_mols_per_workgroup(n_mols, n_atoms) != 1) order = nullptr;
+    const int64_t zeroing = std::min<int64_t>((n_outputs + 8191) / 8192, 512);
+    if (zeroing == 0 && !order) return hipSuccess;
+    charge_begin_kernel<T><<<dim3(static_cast<unsigned>(zeroing + (order ? 1 : 0))), dim3(1024), 0, stream>>>(MACs, n_mols, order, outputs, n_outputs);
+    return hipGetLastError();
+}
+template hipError_t launch_charge_begin<float>(const int32_t*, int32_t, int64_t, int32_t*&, float*, int64_t, hipStream_t);
+template hipError_t launch_charge_begin<double>(const int32_t*, int32_t, int64_t, int32_t*&, double*, int64_t, hipStream_t);
 
 template hipError_t launch_charge_energy<float>(const float*, const float*, const float*, const float*, const int32_t*, const int32_t*, int32_t, int64_t, bool, float, float*, hipStream_t);
 template hipError_t launch_charge_energy<double>(const double*, const double*, const double*, const double*, const int32_t*, const int32_t*, int32_t, int64_t, bool, double, double*, hipStream_t);
-template hipError_t launch_charge_grad<float>(const float*, const float*, const float*, const float*, const int32_t*, const int32_t*, int32_t, int64_t, const float*, bool, float, float*, float*, float*, float*, float*, bool, hipStream_t);
-template hipError_t launch_charge_grad<double>(const double*, const double*, const double*, const double*, const int32_t*, const int32_t*, int32_t, int64_t, const double*, bool, double, double*, double*, double*, double*, double*, bool, hipStream_t);
+template hipError_t launch_charge_grad<float>(const float*, const float*, const float*, const float*, const int32_t*, const int32_t*, int32_t, int64_t, const float*, bool, float, float*, float*, float*, float*, float*, bool, const int32_t*, hipStream_t);
+template hipError_t launch_charge_grad<double>(const double*, const double*, const double*, const double*, const int32_t*, const int32_t*, int32_t, int64_t, const double*, bool, double, double*, double*, double*, double*, double*, bool, const int32_t*, hipStream_t);
 
 }  // namespace khan

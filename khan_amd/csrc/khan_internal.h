@@ -177,11 +177,14 @@ hipError_t launch_dense_first(const float* const rows[4], const int32_t n[4], co
 template <typename T>
 hipError_t launch_charge_energy(const T* X, const T* Y, const T* Z, const T* Q, const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
                                 int64_t n_atoms, bool damped, T K, T* E, hipStream_t stream);
-// E (may be null): the energies as well; zeroed: E holds zeros already
+// E (may be null): the energies as well; zeroed: E holds zeros already; order (may be null): of launch_charge_begin
 template <typename T>
 hipError_t launch_charge_grad(const T* X, const T* Y, const T* Z, const T* Q, const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
                               int64_t n_atoms, const T* grads, bool damped, T K, T* q_grads, T* gX, T* gY, T* gZ, T* E, bool zeroed,
-                              hipStream_t stream);
+                              const int32_t* order, hipStream_t stream);
+template <typename T>
+hipError_t launch_charge_begin(const int32_t* MACs, int32_t n_mols, int64_t n_atoms, int32_t*& order, T* outputs, int64_t n_outputs,
+                               hipStream_t stream);
 
 // ---- wavefront helpers (64 lanes) ----
 __device__ __forceinline__ unsigned long long wave_ballot(bool p) { return __ballot(p); }

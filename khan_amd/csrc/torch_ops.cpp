@@ -320,29 +320,24 @@ at::ScalarType check_charge(const Tensor& xs, const Tensor& ys, const Tensor& zs
     return dt;
 }
 
-template <typename Fn>
-void with_charges(at::ScalarType dt, Fn run)
-{
-    if (dt == at::kFloat) run(0.0f, api.khan_ani_charges_f32);
-    else run(0.0, api.khan_ani_charges_f64);
-}
-
 Tensor ani_charge(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& qs, const Tensor& mos, const Tensor& macs)
 {
     const auto dt = check_charge(xs, ys, zs, qs, mos, macs);
     const Tensor e = at::empty({mos.numel()}, xs.options());
     const khan_stream_t st = stream();
-    with_charges(dt, [&](auto zero, auto fn) {
+    auto run = [&](auto zero, auto fn) {
         using T = decltype(zero);
         call(fn, ptr<const T>(xs), ptr<const T>(ys), ptr<const T>(zs), ptr<const T>(qs), ptr<const int32_t>(mos), ptr<const int32_t>(macs),
              static_cast<int32_t>(mos.numel()), xs.numel(), static_cast<const T*>(nullptr), ptr<T>(e), static_cast<T*>(nullptr),
              static_cast<T*>(nullptr), static_cast<T*>(nullptr), static_cast<T*>(nullptr), 0, st);
-    });
+    };
+    if (dt == at::kFloat) run(0.0f, api.khan_ani_charges_f32);
+    else run(0.0, api.khan_ani_charges_f64);
     return e;
 }
 
-// Gradients (and with `energies` the energies) of the damped charge energy.  One zeroed allocation cut into the outputs:
-// atoms outside every molecule keep zeros.
+// Gradients (and with `energies` the energies) of the damped charge energy.  One allocation cut into the outputs, zeroed by the
+// launch that orders the molecules: atoms outside every molecule keep zeros.
 std::vector<Tensor> ani_charge_grads(const Tensor& xs, const Tensor& ys, const Tensor& zs, const Tensor& qs, const Tensor& mos, const Tensor& macs,
                                      const Tensor& grads, bool want_xyz, bool energies)
 {
@@ -350,7 +345,8 @@ std::vector<Tensor> ani_charge_grads(const Tensor& xs, const Tensor& ys, const T
     dev(grads, dt, "grads");
     same_size(grads.numel() == mos.numel(), "grads must have one element per molecule");
     const int64_t n = xs.numel(), m = mos.numel();
-    const Tensor all = at::zeros({n * (want_xyz ? 4 : 1) + (energies ? m : 0)}, xs.options());
+    const Tensor all = at::empty({n * (want_xyz ? 4 : 1) + (energies ? m : 0)}, xs.options());
+    const Tensor order = at::empty({m}, mos.options());
     std::vector<Tensor> out;
     int64_t at = 0;
     auto take = [&](int64_t size) {
@@ -360,14 +356,16 @@ std::vector<Tensor> ani_charge_grads(const Tensor& xs, const Tensor& ys, const T
     if (energies) take(m);
     for (int k = 0; k < (want_xyz ? 4 : 1); ++k) take(n);
     const khan_stream_t st = stream();
-    with_charges(dt, [&](auto zero, auto fn) {
+    auto run = [&](auto zero, auto fn) {
         using T = decltype(zero);
         const int q = energies ? 1 : 0;
         T* none = nullptr;
         call(fn, ptr<const T>(xs), ptr<const T>(ys), ptr<const T>(zs), ptr<const T>(qs), ptr<const int32_t>(mos), ptr<const int32_t>(macs),
              static_cast<int32_t>(m), n, ptr<const T>(grads), energies ? ptr<T>(out[0]) : none, ptr<T>(out[q]), want_xyz ? ptr<T>(out[q + 1]) : none,
-             want_xyz ? ptr<T>(out[q + 2]) : none, want_xyz ? ptr<T>(out[q + 3]) : none, 1, st);
-    });
+             want_xyz ? ptr<T>(out[q + 2]) : none, want_xyz ? ptr<T>(out[q + 3]) : none, ptr<T>(all), all.numel(), ptr<int32_t>(order), st);
+    };
+    if (dt == at::kFloat) run(0.0f, api.khan_ani_charges_begun_f32);
+    else run(0.0, api.khan_ani_charges_begun_f64);
     return out;
 }
 

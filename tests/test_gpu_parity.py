@@ -636,6 +636,36 @@ def test_plain_coulomb_sums(ops, kind, n_mols):
     assert not np.allclose(damped, helpers.CHARGE_K * _coulomb_brute(b.X, b.Y, b.Z, q, b.MOs, b.MACs, 1.0, g)[0], rtol=1e-3)
 
 
+@pytest.mark.parametrize("n_mols", [256, 257, 1025, 16384, 16385])
+@pytest.mark.parametrize("ndt", [np.float32, np.float64])
+def test_charges_in_size_order(ops, n_mols, ndt):
+    """Dense batches of 257 to 16,384 molecules are walked by decreasing size: every output has the bits that batch order
+    gives (khan_ani_charge_all), for sizes on either side of a wavefront and a workgroup and in a mixed order; atoms outside
+    every molecule keep zeros.  (The energy of a molecule of more than 256 atoms is added up in an order that varies: a few
+    roundings of the sum of its terms.)"""
+    say("case: charges in size order", n_mols, ndt.__name__)
+    rng = np.random.default_rng(n_mols)
+    sizes = rng.integers(34, 80, n_mols).astype(np.int32)
+    sizes[rng.integers(0, n_mols, 12)] = [0, 1, 63, 64, 65, 127, 128, 129, 192, 255, 256, 257]
+    n = int(sizes.sum()) + 3
+    mos, macs = dev((np.cumsum(sizes) - sizes).astype(np.int32)), dev(sizes)
+    x, y, z = (dev(rng.uniform(0, 9, n), ndt) for _ in range(3))
+    q, g = dev(rng.standard_normal(n), ndt), dev(rng.standard_normal(n_mols), ndt)
+    from khan_amd import _lib
+    got = ops.ani_charge_all(x, y, z, q, mos, macs, g)
+    lib = _lib.load()
+    plain = [torch.zeros_like(t) for t in got]
+    fn = lib.khan_ani_charge_all_f32 if ndt is np.float32 else lib.khan_ani_charge_all_f64
+    assert fn(*(t.data_ptr() for t in (x, y, z, q, mos, macs)), n_mols, g.data_ptr(), *(t.data_ptr() for t in plain),
+              torch.cuda.current_stream().cuda_stream) == 0
+    large = macs > 256
+    assert torch.equal(got[0][~large], plain[0][~large])
+    scale = ops.ani_charge(x, y, z, q.abs(), mos, macs)[large]
+    assert ((got[0] - plain[0])[large].abs() <= 8 * np.finfo(ndt).eps * scale).all()
+    for a, b in zip(got[1:], plain[1:]):
+        assert torch.equal(a, b) and (a[-3:] == 0).all()
+
+
 def test_charge_reference_fixture_gradient_consistency(ops):
     # the reference's only check of charges: dE/dq from the op agrees with a numeric derivative of the
     # energy op (gpu_featurizer/test_kernel.py:403-459, delta 1e-3, tol 1e-11 in float64)
