@@ -24,8 +24,11 @@ struct __align__(16) FwdWaveLds {
     static constexpr int kSegments = kNB * kNumPairBlocks;      // a segment per (centre, type pair) at most
     typename Fast<T>::vec4 nbr[kNB][kCap];     // unit vector (centre minus partner)/r, and r
     T nbr_fc[kNB][kCap];                       // f_C(r, A_Rc)
-    typename Fast<T>::vec2 rad[kRadN];        // (r, f_C(r, R_Rc)) of the radial partners of a scan step's centres
-    T rec[64][12];                            // phase-1 records: A_0..7, G_0..3
+    // phase-1 records, A_0..7 and G_0..3; before them, in the same place, the radial partners (r, f_C(r, R_Rc)) of a scan
+    // step's centres, which are used up when the angular part begins
+    T rec[64][12];
+    static_assert(kRadN * 2 <= 64 * 12, "the radial list lies in the records' place");
+    __device__ __forceinline__ typename Fast<T>::vec2* rad() { return reinterpret_cast<typename Fast<T>::vec2*>(&rec[0][0]); }
     SegDesc seg[kSegments];                   // non-empty segments of the batch, in order
     unsigned long long segrow[kSegments];     // where each of them puts its 32 output values (then: the empty blocks' addresses)
     unsigned bits[bit_words(kNB)];            // bit per triple slot: a segment starts here

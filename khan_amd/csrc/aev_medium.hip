@@ -199,7 +199,7 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
 #pragma unroll
                             for (int u = 0; u < kMedRadTrip; ++u) {
                                 const int at = min(obase + q0 + u * 4 + rslot, kRadCap - 1);
-                                e[u] = S.rad[at];
+                                e[u] = S.rad()[at];
                                 if constexpr (kJvp) ab[u] = S.jvp.rad_ab[at];
                             }
 #pragma unroll
@@ -225,7 +225,7 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                     int tR = -1;
                     vec2 e = Fast<T>::make2(T(0), T(0)), ab = Fast<T>::make2(T(0), T(0));
                     if (lane < count) {
-                        e = S.rad[lane];
+                        e = S.rad()[lane];
                         if constexpr (kJvp) ab = S.jvp.rad_ab[lane];
                         if constexpr (kJvp && kLarge) tR = M.rtype[wave][lane];
                         else tR = static_cast<int>(e.y);
@@ -241,10 +241,10 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                     wave_lds_fence();               // every entry has been read
                     if (lane < count) {
                         if constexpr (kJvp) {
-                            S.rad[dest] = e;
+                            S.rad()[dest] = e;
                             S.jvp.rad_ab[dest] = ab;
                         } else {
-                            S.rad[dest] = Fast<T>::make2(e.x, Fast<T>::cutoff(e.x, static_cast<T>(kR_Rc_f)));
+                            S.rad()[dest] = Fast<T>::make2(e.x, Fast<T>::cutoff(e.x, static_cast<T>(kR_Rc_f)));
                         }
                     }
                     wave_lds_fence();
@@ -284,7 +284,7 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                             if (p < kRadCap) {
                                 T fc, dfc;
                                 Fast<T>::cutoff_grad(r, static_cast<T>(kR_Rc_f), fc, dfc);
-                                S.rad[p] = Fast<T>::make2(r, fc);
+                                S.rad()[p] = Fast<T>::make2(r, fc);
                                 S.jvp.rad_ab[p] = Fast<T>::make2(dfc * rd, T(-2) * static_cast<T>(kR_eta_f) * fc * rd);
                                 if constexpr (kLarge) M.rtype[wave][p] = static_cast<unsigned char>(tj);
                             }
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                         // (the place of the cutoff value carries the partner's type until then)
                         if (inR) {
                             const int p = posR + popc64(mR & lt_mask);
-                            if (p < kRadCap) S.rad[p] = Fast<T>::make2(r, aj.w);
+                            if (p < kRadCap) S.rad()[p] = Fast<T>::make2(r, aj.w);
                         }
                         if (inA) {
                             const int p = posA + popc64(mA & lt_mask);
@@ -397,9 +397,9 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                     const bool haveR = !kLarge && lane < min(posR, kRadCap), haveA = lane < min(posA, kCapA);
                     int tR = -1, tA = -1;           // type of this lane's list entry
                     if (haveR) {
-                        const vec2 e = S.rad[lane];
+                        const vec2 e = S.rad()[lane];
                         tR = static_cast<int>(e.y);
-                        S.rad[lane] = Fast<T>::make2(e.x, Fast<T>::cutoff(e.x, static_cast<T>(kR_Rc_f)));
+                        S.rad()[lane] = Fast<T>::make2(e.x, Fast<T>::cutoff(e.x, static_cast<T>(kR_Rc_f)));
                     }
                     if (haveA) {
                         const vec4 d = S.nbr[b][lane];
@@ -536,15 +536,16 @@ hipError_t launch_fwd_large(const T* X, const T* Y, const T* Z, const int32_t* A
     return hipGetLastError();
 }
 
+#ifndef KHAN_UNIT_LARGE
 template hipError_t launch_fwd_medium<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<float>, int, const int32_t*, hipStream_t);
-template hipError_t launch_fwd_medium<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<double>, int, const int32_t*, hipStream_t);
-
 template hipError_t launch_jvp_medium<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const float*, const float*, const float*, Buckets<float>, int, const int32_t*, hipStream_t);
+#else
+template hipError_t launch_fwd_medium<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<double>, int, const int32_t*, hipStream_t);
 template hipError_t launch_jvp_medium<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const double*, const double*, const double*, Buckets<double>, int, const int32_t*, hipStream_t);
-
 template size_t large_scratch_bytes<float>(int64_t, int32_t, bool);
 template size_t large_scratch_bytes<double>(int64_t, int32_t, bool);
 template hipError_t launch_fwd_large<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const float*, const float*, const float*, Buckets<float>, const int32_t*, void*, int64_t, hipStream_t);
 template hipError_t launch_fwd_large<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const double*, const double*, const double*, Buckets<double>, const int32_t*, void*, int64_t, hipStream_t);
+#endif
 
 }  // namespace khan

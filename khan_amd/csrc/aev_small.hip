@@ -44,10 +44,11 @@ constexpr int kRadSlots = 96;
 // With kJvp the kernel computes the Jacobian-vector product instead (featurize_grad_inverse): every term of
 // the forward sums is replaced by its derivative along the per-atom vectors (VX, VY, VZ).
 // float: 4 wavefronts per SIMD (LDS 9.8 KB, <= 128 VGPRs; the kernel loses a fifth of its speed at three);
-// float kJvp: 3 (<= 168 VGPRs; its LDS, 13.4 KB, lets twelve wavefronts share a CU); double: 2 (LDS 17 KB); double kJvp: 1.
+// float kJvp: 3 (<= 168 VGPRs; its LDS lets twelve wavefronts share a CU); double: 3 (149 VGPRs, LDS 12.5 KB with four
+// centres); double kJvp: 1.
 template <typename T, bool kJvp, bool kShare = false, bool kMatrixPhase2 = false>
 __global__ __launch_bounds__(64 * kWavesPerBlock)
-__attribute__((amdgpu_waves_per_eu((kJvp && sizeof(T) == 4) ? 3 : (sizeof(T) == 4 ? 4 : 2) / (kJvp ? 2 : 1), (kJvp && sizeof(T) == 4) ? 3 : (sizeof(T) == 4 ? 4 : 2) / (kJvp ? 2 : 1))))
+__attribute__((amdgpu_waves_per_eu(kJvp ? (sizeof(T) == 4 ? 3 : 1) : (sizeof(T) == 4 ? 4 : 3), kJvp ? (sizeof(T) == 4 ? 3 : 1) : (sizeof(T) == 4 ? 4 : 3))))
 void aev_fwd_small_kernel(
     const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
     const int32_t* __restrict__ A, const int32_t* __restrict__ MOs,
@@ -58,7 +59,7 @@ void aev_fwd_small_kernel(
     typedef typename Fast<T>::vec4 vec4;
     typedef typename Fast<T>::vec2 vec2;
     // centres per batch: six; four in the float Jacobian-vector kernel (with kCap below: twelve wavefronts per CU)
-    constexpr int kNB = (kJvp && sizeof(T) == 4) ? 4 : kFB;
+    constexpr int kNB = (kJvp == (sizeof(T) == 4)) ? 4 : kFB;
     // angular partners kept per centre: 32; 28 in the float Jacobian-vector kernel, whose working set then is 13.4 KB
     // and twelve wavefronts share a CU (a centre with more goes to the general routine, as above 32 elsewhere)
     constexpr int kCap = (kJvp && sizeof(T) == 4) ? 28 : kCapA;
@@ -200,7 +201,7 @@ void aev_fwd_small_kernel(
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 const int at = e == 0 ? lane : 64 + (lane & 31);
-                S.rad[at] = Fast<T>::make2(T(0), T(0));
+                S.rad()[at] = Fast<T>::make2(T(0), T(0));
                 if constexpr (kJvp) S.jvp.rad_ab[at] = Fast<T>::make2(T(0), T(0));
             }
             const T dx = lane_fetch(x, ci) - xj, dy = lane_fetch(y, ci) - yj, dz = lane_fetch(z, ci) - zj;
@@ -226,10 +227,10 @@ void aev_fwd_small_kernel(
                 if constexpr (kJvp) {
                     T fc, dfc;
                     Fast<T>::cutoff_grad(r, static_cast<T>(kR_Rc_f), fc, dfc);
-                    S.rad[pos] = Fast<T>::make2(r, fc);
+                    S.rad()[pos] = Fast<T>::make2(r, fc);
                     S.jvp.rad_ab[pos] = Fast<T>::make2(dfc * rd, T(-2) * static_cast<T>(kR_eta_f) * fc * rd);
                 } else {
-                    S.rad[pos] = Fast<T>::make2(r, Fast<T>::cutoff(r, static_cast<T>(kR_Rc_f)));
+                    S.rad()[pos] = Fast<T>::make2(r, Fast<T>::cutoff(r, static_cast<T>(kR_Rc_f)));
                 }
             }
             if (inA && fits) {
@@ -266,7 +267,7 @@ void aev_fwd_small_kernel(
 
             // ---- radial features of the G centres of this step
             {
-                const vec2* list = &S.rad[rg_g * rad_stride + rg_s];
+                const vec2* list = &S.rad()[rg_g * rad_stride + rg_s];
                 const int cb = b0 + rg_g;
                 const int ci = min(c0 + cb, 63);
                 const unsigned rlo = static_cast<unsigned>(__builtin_amdgcn_ds_bpermute(ci << 2, rp_lo));
@@ -330,14 +331,14 @@ void aev_fwd_small_kernel(
 
 }  // namespace
 
-// Wavefronts per molecule (as a power of two).  organic molecules, 16 / 8 / 12 / 4 wavefronts per CU resident (float,
+// Wavefronts per molecule (as a power of two).  organic molecules, 16 / 12 / 12 / 4 wavefronts per CU resident (float,
 // double, and their Jacobian-vector forms); forward float 100 -> 24 us at 1,024 molecules, 106 -> 47 at 4,096,
 // 112 -> 78 at 8,192 (two each), and slower from 16,384 on (137 -> 150 with two); the Jacobian-vector form
 // 131 -> 31 us at 1,024, double forward 162 -> 51 us.  The rows are the same bits for any number.
 template <typename T, bool kJvp>
 static int log_parts_of(int32_t n_mols)
 {
-    constexpr int kResident = kCUs * (sizeof(T) == 4 ? (kJvp ? 12 : 16) : (kJvp ? 4 : 8));
+    constexpr int kResident = kCUs * (sizeof(T) == 4 ? (kJvp ? 12 : 16) : (kJvp ? 4 : 12));
     return __builtin_ctz(molecule_parts(n_mols, 4 * kResident, 8));
 }
 
@@ -384,9 +385,12 @@ hipError_t launch_jvp_small(const T* X, const T* Y, const T* Z, const int32_t* A
     return hipGetLastError();
 }
 
+#ifndef KHAN_UNIT_F64
 template hipError_t launch_fwd_small<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<float>, int, const int32_t*, hipStream_t);
-template hipError_t launch_fwd_small<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<double>, int, const int32_t*, hipStream_t);
 template hipError_t launch_jvp_small<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const float*, const float*, const float*, Buckets<float>, const int32_t*, hipStream_t);
+#else
+template hipError_t launch_fwd_small<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<double>, int, const int32_t*, hipStream_t);
 template hipError_t launch_jvp_small<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const double*, const double*, const double*, Buckets<double>, const int32_t*, hipStream_t);
+#endif
 
 }  // namespace khan

@@ -393,7 +393,10 @@ hipError_t launch_bwd_small(const T* X, const T* Y, const T* Z, const int32_t* A
     return hipGetLastError();
 }
 
+#ifndef KHAN_UNIT_F64
 template hipError_t launch_bwd_small<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<const float>, float*, float*, float*, int, const int32_t*, hipStream_t);
+#else
 template hipError_t launch_bwd_small<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<const double>, double*, double*, double*, int, const int32_t*, hipStream_t);
+#endif
 
 }  // namespace khan
