@@ -439,7 +439,7 @@ __global__ __launch_bounds__(256, 4) void charge_kernel(ChargeArgs<T> a, int col
 }
 
 // Before the launch: zeros in the outputs (atoms outside every molecule keep them, and the energies of molecules of more than
-// 256 atoms are added up), and by the first workgroup, where `order` is asked for, the molecules of 65 to 256 atoms by
+// 256 atoms are added up), and by the first workgroup the molecules of 65 to 256 atoms by
 // decreasing size, the others behind them: a counting sort, in no particular order inside a size (every molecule's results
 // are its own).  A launch lasts only a few molecules' time and in batch order ended with a third of the wavefronts' places empty.
 constexpr int kOrderMost = 16384;
@@ -448,10 +448,9 @@ __global__ __launch_bounds__(1024) void charge_begin_kernel(const int32_t* __res
                                                             T* __restrict__ outputs, int64_t n_outputs)
 {
     const int tid = threadIdx.x;
-    const int sorting = order ? 1 : 0;
-    if (static_cast<int>(blockIdx.x) >= sorting) {
-        const int64_t step = static_cast<int64_t>(gridDim.x - sorting) * 1024;
-        for (int64_t i = static_cast<int64_t>(blockIdx.x - sorting) * 1024 + tid; i < n_outputs; i += step) outputs[i] = T(0);
+    if (blockIdx.x > 0) {
+        const int64_t step = static_cast<int64_t>(gridDim.x - 1) * 1024;
+        for (int64_t i = static_cast<int64_t>(blockIdx.x - 1) * 1024 + tid; i < n_outputs; i += step) outputs[i] = T(0);
         return;
     }
     constexpr int kBins = kMediumMaxAtoms + 1, kEach = kOrderMost / 1024;
@@ -529,9 +528,9 @@ template <typename T>
 hipError_t launch_charge_begin(const int32_t* MACs, int32_t n_mols, int64_t n_atoms, int32_t*& order, T* outputs, int64_t n_outputs, hipStream_t stream)
 {
     if (n_mols <= 256 || n_mols > kOrderMost || charge_mols_per_workgroup(n_mols, n_atoms) != 1) order = nullptr;
+    if (!order) return n_outputs > 0 ? launch_zero<T>(outputs, n_outputs, stream) : hipSuccess;
     const int64_t zeroing = std::min<int64_t>((n_outputs + 8191) / 8192, 512);
-    if (zeroing == 0 && !order) return hipSuccess;
-    charge_begin_kernel<T><<<dim3(static_cast<unsigned>(zeroing + (order ? 1 : 0))), dim3(1024), 0, stream>>>(MACs, n_mols, order, outputs, n_outputs);
+    charge_begin_kernel<T><<<dim3(static_cast<unsigned>(zeroing + 1)), dim3(1024), 0, stream>>>(MACs, n_mols, order, outputs, n_outputs);
     return hipGetLastError();
 }
 template hipError_t launch_charge_begin<float>(const int32_t*, int32_t, int64_t, int32_t*&, float*, int64_t, hipStream_t);

@@ -346,7 +346,7 @@ std::vector<Tensor> ani_charge_grads(const Tensor& xs, const Tensor& ys, const T
     same_size(grads.numel() == mos.numel(), "grads must have one element per molecule");
     const int64_t n = xs.numel(), m = mos.numel();
     const Tensor all = at::empty({n * (want_xyz ? 4 : 1) + (energies ? m : 0)}, xs.options());
-    const Tensor order = at::empty({m}, mos.options());
+    const Tensor order = m > 256 && n > 32 * m ? at::empty({m}, mos.options()) : Tensor();      // (elsewhere it would not be used)
     std::vector<Tensor> out;
     int64_t at = 0;
     auto take = [&](int64_t size) {
@@ -362,7 +362,7 @@ std::vector<Tensor> ani_charge_grads(const Tensor& xs, const Tensor& ys, const T
         T* none = nullptr;
         call(fn, ptr<const T>(xs), ptr<const T>(ys), ptr<const T>(zs), ptr<const T>(qs), ptr<const int32_t>(mos), ptr<const int32_t>(macs),
              static_cast<int32_t>(m), n, ptr<const T>(grads), energies ? ptr<T>(out[0]) : none, ptr<T>(out[q]), want_xyz ? ptr<T>(out[q + 1]) : none,
-             want_xyz ? ptr<T>(out[q + 2]) : none, want_xyz ? ptr<T>(out[q + 3]) : none, ptr<T>(all), all.numel(), ptr<int32_t>(order), st);
+             want_xyz ? ptr<T>(out[q + 2]) : none, want_xyz ? ptr<T>(out[q + 3]) : none, ptr<T>(all), all.numel(), order.defined() ? ptr<int32_t>(order) : nullptr, st);
     };
     if (dt == at::kFloat) run(0.0f, api.khan_ani_charges_begun_f32);
     else run(0.0, api.khan_ani_charges_begun_f64);
