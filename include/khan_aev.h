@@ -426,6 +426,20 @@ int64_t khan_net_grads_workspace_bytes_f64(const khan_net_grads *grads);
 int khan_net_grads_f32(const khan_net_grads *grads, khan_stream_t stream);
 int khan_net_grads_f64(const khan_net_grads *grads, khan_stream_t stream);
 
+/* Whole networks with CELU in float64 on few rows, values and on request row gradients in one launch (a workgroup per sixteen
+ * rows of a type): `layers` products of the widths `widths` (the last 1), w[l][t] [in, out] and b[l][t] of layer l and type t.
+ * khan_net_few_fits: 1 for widths it takes, which are 384, 128, 128, 64, 1.  x and w must be 16-byte aligned; grad[t] NULL
+ * for all types: values only. */
+#define KHAN_NET_FEW_LAYERS 4
+typedef struct khan_net_few {
+    const void *x[4], *w[KHAN_NET_FEW_LAYERS][4], *b[KHAN_NET_FEW_LAYERS][4];
+    void *value[4], *grad[4];
+    int32_t n[4], layers, widths[KHAN_NET_FEW_LAYERS + 1];
+    double alpha;
+} khan_net_few;
+int32_t khan_net_few_fits(const int32_t *widths, int32_t layers);
+int khan_net_few_f64(const khan_net_few *net, khan_stream_t stream);
+
 /* Per-molecule sums of the atomic networks' outputs: e[m] = sum over the atoms g of molecule m of
  * out_{as[g]}[sis[g]] -- the gather to the batch's atom order and the segment sum by molecule of the reference
  * (khan/model/nn.py:165-177; trainer_multi_tower.py:350) in one launch, without the gathered copy, each molecule's

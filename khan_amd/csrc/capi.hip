@@ -7,6 +7,7 @@
 #include "../../include/khan_aev.h"
 #include "khan_internal.h"
 #include "khan_params.h"
+#include "net_few.h"
 #include "net_layers.h"
 
 // Size order of khan_featurize_f32_noalloc: the molecule indices by decreasing atom count, then the class counts
@@ -964,6 +965,40 @@ int khan_net_top_f32(const khan_net_top* top, khan_stream_t stream) { return net
 int khan_net_top_f64(const khan_net_top* top, khan_stream_t stream) { return net_top_impl<double>(top, stream); }
 int64_t khan_net_grads_workspace_bytes_f32(const khan_net_grads* grads) { return net_grads_bytes<float>(grads); }
 int64_t khan_net_grads_workspace_bytes_f64(const khan_net_grads* grads) { return net_grads_bytes<double>(grads); }
+int32_t khan_net_few_fits(const int32_t* widths, int32_t layers)
+{
+    return widths && layers >= 1 && layers <= khan::kFewLayers && khan::net_few_fits(widths, layers) ? 1 : 0;
+}
+int khan_net_few_f64(const khan_net_few* net, khan_stream_t stream)
+{
+    static_assert(KHAN_NET_FEW_LAYERS == khan::kFewLayers, "one limit");
+    if (!net || !khan_net_few_fits(net->widths, net->layers) || !(net->alpha > 0.0)) return KHAN_ERR_INVALID_ARG;
+    khan::NetFew a = {};
+    a.alpha = net->alpha;
+    a.inv_alpha = 1.0 / net->alpha;
+    int64_t rows = 0;
+    int with_grad = 0, with_rows = 0;
+    for (int t = 0; t < 4; ++t) {
+        a.n[t] = net->n[t];
+        if (net->n[t] < 0) return KHAN_ERR_INVALID_ARG;
+        if (net->n[t] == 0) continue;
+        rows += net->n[t];
+        a.x[t] = static_cast<const double*>(net->x[t]);
+        a.value[t] = static_cast<double*>(net->value[t]);
+        a.grad[t] = static_cast<double*>(net->grad[t]);
+        if (!a.x[t] || !a.value[t] || (reinterpret_cast<uintptr_t>(a.x[t]) & 15u)) return KHAN_ERR_INVALID_ARG;
+        with_rows += 1;
+        with_grad += a.grad[t] ? 1 : 0;
+        for (int l = 0; l < net->layers; ++l) {
+            a.w[l][t] = static_cast<const double*>(net->w[l][t]);
+            a.b[l][t] = static_cast<const double*>(net->b[l][t]);
+            if (!a.w[l][t] || !a.b[l][t] || (reinterpret_cast<uintptr_t>(a.w[l][t]) & 15u)) return KHAN_ERR_INVALID_ARG;
+        }
+    }
+    if (with_grad != 0 && with_grad != with_rows) return KHAN_ERR_INVALID_ARG;
+    if (rows > INT32_MAX) return KHAN_ERR_TOO_LARGE;
+    return hip_status(khan::launch_net_few(a, as_stream(stream)));
+}
 int khan_net_grads_f32(const khan_net_grads* grads, khan_stream_t stream) { return net_grads_impl<float>(grads, stream); }
 int khan_net_grads_f64(const khan_net_grads* grads, khan_stream_t stream) { return net_grads_impl<double>(grads, stream); }
 

@@ -764,7 +764,8 @@ struct Inference {
     const Rows rows;
     const Pass pass;
     Tensor values;                          // of all rows, type by type
-    variable_list state;                    // activations and d_L; in the one-launch form the rows' gradients
+    variable_list state;                    // activations and d_L; in the one-launch forms the rows' gradients
+    bool few = false;                       // float64 in one launch (net_few.hip): see take_few
 
     Inference(const Weights& w_, const Four& x)
         : w(w_), rows(rows_of(w.net, w.params, x[0], x[1], x[2], x[3])), pass{w.net, rows, w.params},
@@ -772,6 +773,44 @@ struct Inference {
     {
     }
     bool one_launch() const { return w.packed.defined(); }
+
+    // Float64 networks of the widths net_few.hip takes, whose rows' gradients are not to be scaled: one launch up to 256 tiles
+    // of sixteen rows, one for every compute unit (us, values and gradients, layer by layer -> one launch: 1 molecule 80 -> 67, 16 molecules 112 -> 86, 256 (2,970 rows) 152 -> 115, 330 (3,863) 175 -> 132; values alone 41 -> 29, 54 -> 39, 67 -> 47).
+    void take_few()
+    {
+        if (w.params.dtype != at::kDouble || w.net.layers() > KHAN_NET_FEW_LAYERS) return;
+        int32_t widths[KHAN_NET_FEW_LAYERS + 1];
+        for (size_t k = 0; k < w.net.widths.size(); ++k) widths[k] = static_cast<int32_t>(w.net.widths[k]);
+        if (!api.khan_net_few_fits(widths, w.net.layers())) return;
+        int64_t tiles = 0;
+        uintptr_t bits = 0;
+        for (int t = 0; t < 4; ++t) {
+            tiles += (rows.n[t] + 15) / 16;
+            if (rows.n[t] > 0) bits |= reinterpret_cast<uintptr_t>(rows.x[t].data_ptr());
+            for (int l = 0; l < w.net.layers(); ++l) bits |= reinterpret_cast<uintptr_t>(w.params.weight(l, t));
+        }
+        few = tiles <= 256 && (bits & 15u) == 0;
+    }
+    Tensor launch_few(bool want_rows)
+    {
+        const Tensor grads = want_rows ? at::empty({rows.total * w.net.widths[0]}, w.params.options) : Tensor();
+        khan_net_few a = {};
+        a.layers = w.net.layers();
+        for (size_t k = 0; k < w.net.widths.size(); ++k) a.widths[k] = static_cast<int32_t>(w.net.widths[k]);
+        a.alpha = w.net.alpha;
+        for (int t = 0; t < 4; ++t) {
+            a.n[t] = static_cast<int32_t>(rows.n[t]);
+            a.x[t] = rows.n[t] > 0 ? rows.x[t].data_ptr() : nullptr;
+            a.value[t] = pass.part(values, 1, t);
+            a.grad[t] = pass.part(grads, w.net.widths[0], t);
+            for (int l = 0; l < a.layers; ++l) {
+                a.w[l][t] = w.params.weight(l, t);
+                a.b[l][t] = w.params.bias(l, t);
+            }
+        }
+        call(api.khan_net_few_f64, static_cast<const khan_net_few*>(&a), pass.st);
+        return grads;
+    }
 
     Tensor launch(bool want_rows)
     {
@@ -799,6 +838,8 @@ struct Inference {
         const Four v = by_type(rows, values, 1);
         if (one_launch()) {
             state = {launch(want_rows)};
+        } else if (few) {
+            state = {launch_few(want_rows)};
         } else {
             state = pass.forward(!exact);
             state.push_back(pass.top(state.back(), &v, want_rows));
@@ -809,7 +850,7 @@ struct Inference {
     // form has them already, and neither scale nor anything to add to
     Tensor gradients(const Four& scale, Tensor into)
     {
-        if (one_launch()) return state[0];
+        if (one_launch() || few) return state[0];
         const bool add = into.defined();
         if (!add) into = at::empty({rows.total * w.net.widths[0]}, w.params.options);
         const variable_list d = pass.slopes(variable_list(state.begin(), state.end() - 1), state.back());
@@ -896,6 +937,7 @@ std::vector<Tensor> infer(const Tensor& xs, const Tensor& ys, const Tensor& zs, 
     const Weights near_w = weights_of(near, alpha);
     same_size(charge.is_none() || !near_w.packed.defined(), "networks beside a charge network run layer by layer");
     Inference near_net(near_w, feats);
+    near_net.take_few();
     run_mol_energy(near_net.forward(need_grad), as, sis, mos, macs, out[0]);
     if (charge.is_none()) {
         if (need_grad) run_featurize_grad(in, args, by_type(near_net.rows, near_net.gradients({}, Tensor()), kFeats), {out[1], out[2], out[3]});
@@ -904,6 +946,7 @@ std::vector<Tensor> infer(const Tensor& xs, const Tensor& ys, const Tensor& zs, 
     const Weights charge_w = weights_of(charge.cast<py::tuple>(), alpha);
     same_size(!charge_w.packed.defined(), "a charge network runs layer by layer");
     Inference charge_net(charge_w, feats);
+    if (!need_grad) charge_net.take_few();
     charge_net.forward(need_grad);
     const Tensor qs = charge_net.values.index_select(0, gather);
     if (!need_grad) {

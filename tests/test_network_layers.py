@@ -282,6 +282,71 @@ def test_bias_gradients_of_many_rows(dtype, unit):
     assert np.isposinf(of_outputs(factors)[1])
 
 
+class _Few(ctypes.Structure):
+    _fields_ = ([("x", ctypes.c_void_p * 4), ("w", ctypes.c_void_p * 4 * 4), ("b", ctypes.c_void_p * 4 * 4), ("value", ctypes.c_void_p * 4),
+                 ("grad", ctypes.c_void_p * 4), ("n", ctypes.c_int32 * 4), ("layers", ctypes.c_int32), ("widths", ctypes.c_int32 * 5),
+                 ("alpha", ctypes.c_double)])
+
+
+# Float64 networks in one launch: rows around its tiles of sixteen, an empty type, gradients by one workgroup a tile (from 86
+# tiles on) and by three.  Float64 library layers on the CPU: 1e-12 for sums of a few hundred products, as for the layers.
+@pytest.mark.parametrize("rows", [(0, 1, 15, 16), (17, 31, 33, 0), (1, 0, 0, 0), (1300, 50, 3, 0), (1400, 0, 0, 17)])
+def test_float64_networks_in_one_launch(rows):
+    from khan_amd import _lib
+    lib = _lib.load()
+    print("case:", rows, flush=True)
+    gen = torch.Generator().manual_seed(6)
+    widths = (384, 128, 128, 64, 1)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, dtype=torch.float64)
+    x = [rand(n, 384) for n in rows]
+    w, b = [[rand(k, m) * 0.1 for _ in rows] for k, m in zip(widths, widths[1:])], [[rand(m) * 0.1 for _ in rows] for m in widths[1:]]
+
+    def run(x, with_grad, shift=0):
+        put = lambda t: t.cuda()
+        xs, ws, bs = [torch.cat([torch.zeros(shift, dtype=t.dtype), t.reshape(-1)]).cuda()[shift:] for t in x], [list(map(put, v)) for v in w], [list(map(put, v)) for v in b]
+        a = _Few(layers=4, alpha=ALPHA)
+        values, grads = [torch.full((n + 1,), 7.0, device="cuda", dtype=torch.float64) for n in rows], [torch.full((n + 1, 384), 7.0, device="cuda", dtype=torch.float64) for n in rows]
+        for i, k in enumerate(widths):
+            a.widths[i] = k
+        for t, n in enumerate(rows):
+            a.n[t], a.x[t], a.value[t], a.grad[t] = n, xs[t].data_ptr(), values[t].data_ptr(), grads[t].data_ptr() if with_grad else None
+            for l in range(4):
+                a.w[l][t], a.b[l][t] = ws[l][t].data_ptr(), bs[l][t].data_ptr()
+        status = lib.khan_net_few_f64(ctypes.byref(a), torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert all((v[-1] == 7).item() and (g[-1] == 7).all().item() for v, g in zip(values, grads))
+        return status, [v[:-1].cpu() for v in values], [g[:-1].cpu() for g in grads]
+
+    want, want_grad = [], []
+    for t in range(4):
+        leaf = x[t].clone().requires_grad_(True)
+        a = leaf
+        for l in range(4):
+            a = torch.addmm(b[l][t], a, w[l][t])
+            if l < 3:
+                a = torch.where(a >= 0, a, ALPHA * torch.expm1(torch.clamp(a, max=0.0) / ALPHA))
+        want.append(a.detach().reshape(-1))
+        want_grad.append(torch.autograd.grad(a.sum(), leaf)[0])
+    close = lambda got, ref: ref.numel() == 0 or ((got - ref).abs() <= 1e-12 * (ref.abs().max() + 1e-3)).all().item()
+    for with_grad in (True, False):
+        status, values, grads = run(x, with_grad)
+        assert status == 0 and all(map(close, values, want))
+        assert all(map(close, grads, want_grad)) if with_grad else all((g == 7).all() for g in grads)
+    # a row that is not a number stays alone
+    big = rows.index(max(rows))
+    spoilt = [t.clone() for t in x]
+    spoilt[big][rows[big] // 2, 11] = float("nan")
+    _, values, grads = run(x, True)
+    _, other_values, other_grads = run(spoilt, True)
+    others = torch.arange(rows[big]) != rows[big] // 2
+    assert torch.isnan(other_values[big][~others]).all() and torch.isnan(other_grads[big][~others]).all()
+    assert torch.equal(values[big][others], other_values[big][others]) and torch.equal(grads[big][others], other_grads[big][others])
+    # operands off their alignment are refused; `infer` then goes layer by layer
+    assert run(x, True, shift=1)[0] != 0
+    widths_c = (ctypes.c_int32 * 5)(384, 128, 128, 65, 1)
+    assert lib.khan_net_few_fits(widths_c, 4) == 0
+
+
 @pytest.mark.parametrize("layers,live", [((256, 64, 8, 1), 2), ((128, 128, 1), 2), ((128, 64, 1), 3), ((100, 1), 0)])
 def test_parameters_behind_the_constant_layers_have_gradients(layers, live):
     """Without `weights_need_grad` the leading layers of a float32 network are constants and those behind them are not: their
