@@ -9,8 +9,9 @@
 // rows (every activation written, read again by the next layer and once more on the way back); this one moves the rows
 // and their gradients, 2.4 GB, and the values.
 //
-// One workgroup of four wavefronts owns 64 rows; two workgroups share a compute unit and, having no barriers in common,
-// fill each other's waits.  The products run on the 16-bit matrix instructions
+// One workgroup of four wavefronts owns 64 rows at a time; two workgroups share a compute unit and, having no barriers in
+// common, fill each other's waits.  A workgroup goes on to another tile of rows when it is through with one, and has the next
+// tile's first rows and weights on their way before it stores the gradients of the last.  The products run on the 16-bit matrix instructions
 // (v_mfma_f32_32x32x16_f16, sixteen times the rate of the float32 ones) with every float32 operand split into two
 // half-precision parts:
 //     x = h + 2^-11 l,   h = half(x),   l = half(2^11 (x - h))
@@ -33,8 +34,14 @@
 // do not pass through LDS: every wavefront loads its operands of a chunk of 16 k straight into registers (layer_product)
 // -- from the chunks the caller has had split once beforehand (launch_networks_pack), or from the float32 weights, which
 // a lane then splits itself.  Layer 1's feature rows, float32 in memory, go through a double-buffered LDS stage in the
-// space the activation planes take later.  LDS: 35 KB per workgroup; 2 wavefronts per SIMD (the accumulators and the
-// saved activations take 200 registers).
+// space the activation planes take later.  LDS: 41 KB per workgroup; 2 wavefronts per SIMD (the accumulators, the
+// saved activations and the weights on their way take 240 registers).
+//
+// 767,292 rows with gradients, one after another: 970 us -> 830 us (one tile per workgroup, weights asked for one chunk ahead and
+// anew at each product, biases from memory, two vector instructions of address per load -> all that is said here).  Bound by power
+// as much as by anything: 640 us with neither rows nor gradients in memory, at a clock of 1.8 GHz with the matrix units 55 % busy; with
+// them the matrix units are 39 % busy at 1.9 to 2.0 GHz; the rows and gradients alone are 440 us of memory traffic.
+// Tried and slower: gradients stored one run per chunk of the product after (4 %), stores marked as written once (18 %).
 #include "khan_internal.h"
 #include "khan_params.h"
 
@@ -50,9 +57,8 @@ typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 typedef float f2v __attribute__((ext_vector_type(2)));
 
-constexpr int kDepthRows = 4;       // chunks of weights in flight in layer 1 (= two pairs of chunks of the feature rows)
-constexpr int kDepthWeights = 4;    // and in the other products (2 measured 6 % slower, 8 the same)
 constexpr int kRows = 64;           // rows per workgroup
+constexpr int kResident = 2 * kCUs; // workgroups that the chip holds
 constexpr int kThreads = 256;       // four wavefronts: 64 rows x 32 columns each of a 128-wide output
 constexpr int kK1 = 384, kN1 = 128, kN2 = 128, kN3 = 64;
 constexpr int kActStride = 136;     // 16-bit elements between rows of the activation planes: 128 + 8 (16-byte reads without bank conflicts)
@@ -94,12 +100,18 @@ constexpr int kPackB2 = kPackB1 + kParts * kK1 * kN1;        // layer 2 as store
 constexpr int kPackB3 = kPackB2 + kParts * kN1 * kN2;        // layer 3 as stored: 128 x 64
 constexpr int kPackPerType = kPackB3 + kParts * kN2 * kN3;   // 294,912 half-precision values
 
+// a type's biases and output layer, one after the other
+constexpr int kAtB1 = 0, kAtB2 = kAtB1 + kN1, kAtB3 = kAtB2 + kN2, kAtW4 = kAtB3 + kN3, kAtB4 = kAtW4 + kN3, kFixed = kAtB4 + 4;
+
 struct __align__(16) FusedLds {
     union {
         unsigned short act[kParts][kRows][kActStride];        // a layer's activations or gradients, split: [part][row][k]
         unsigned short astage[2][kParts][kRows][kStStride];   // layer 1: pairs of chunks of the feature rows
     };
-    float rowval[2][kRows];                              // the output layer's partial sums; then the rows' upstream factors
+    float rowval[2][kRows];                              // the output layer's partial sums
+    // every type's biases and output layer: read from memory between two products they would be waited for behind the weights
+    // already asked for (loads come back in order)
+    float fixed[4][kFixed];
 };
 
 // two floats -> their two half-precision parts (the value rounded, and 2^11 times what the rounding left), each pair
@@ -108,10 +120,12 @@ __device__ __forceinline__ void split_pair(float x0, float x1, unsigned& p1, uns
 {
     const h2v h = __builtin_convertvector(f2v{x0, x1}, h2v);
     p1 = __builtin_bit_cast(unsigned, h);
-    // 2^11 x - 2^11 h in one fused multiply-add that reads h as it is (both products are exact, and so is the difference)
-    const float r0 = fmaf(static_cast<float>(h[0]), -kResidualScale, x0 * kResidualScale);
-    const float r1 = fmaf(static_cast<float>(h[1]), -kResidualScale, x1 * kResidualScale);
-    p2 = __builtin_bit_cast(unsigned, __builtin_convertvector(f2v{r0, r1}, h2v));
+    // 2^11 x - 2^11 h in one fused multiply-add that reads h and writes half precision as they are (both products are exact,
+    // and so is the difference)
+    h2v l;
+    l[0] = static_cast<_Float16>(fmaf(static_cast<float>(h[0]), -kResidualScale, x0 * kResidualScale));
+    l[1] = static_cast<_Float16>(fmaf(static_cast<float>(h[1]), -kResidualScale, x1 * kResidualScale));
+    p2 = __builtin_bit_cast(unsigned, l);
 }
 
 // a chunk piece (four consecutive k of one row or column) split into the planes of a stage buffer
@@ -125,76 +139,139 @@ __device__ __forceinline__ void stage_piece(unsigned short (&dst)[kParts][kR][kS
     for (int q = 0; q < kParts; ++q) *reinterpret_cast<u2v*>(&dst[q][r][k4]) = u2v{lo[q], hi[q]};
 }
 
-__device__ __forceinline__ float celu_of(float v, float alpha, float inv_alpha)
+__device__ __forceinline__ float celu_of(float v, float alpha, float to_exp2)
 {
-    return v >= 0.f ? v : alpha * (__expf(v * inv_alpha) - 1.0f);
+    const float below = fmaf(alpha, __builtin_amdgcn_exp2f(v * to_exp2), -alpha);
+    return v >= 0.f ? v : below;
 }
 // CELU' from CELU's own value: 1 for h >= 0, exp(z / alpha) = h / alpha + 1 below
-__device__ __forceinline__ float celu_slope(float h, float inv_alpha) { return h >= 0.f ? 1.0f : fmaf(h, inv_alpha, 1.0f); }
+__device__ __forceinline__ float celu_slope(float h, float inv_alpha) { return __builtin_elementwise_minimum(1.0f, fmaf(h, inv_alpha, 1.0f)); }
 
-// sum over the 32 lanes of each half of the wavefront; lanes 16-31 and 48-63 hold the result
-__device__ __forceinline__ float half_sum_to_upper_row(float v)
-{
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, false));   // row_ror:8
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, false));   // row_ror:4
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, false));   // row_ror:2
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, false));   // row_ror:1
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x142, 0xa, 0xf, false));   // row_bcast:15
-    return v;
-}
-
-// Positions.  A 128-wide output (kWide): the wavefront owns the tile's 64 rows x 32 columns, columns wave*32 + l32, as
-// two 32 x 32 blocks one above the other -- block j, accumulator e is row j*32 + 8 (e / 4) + 4 half + e % 4.  The
-// 64-wide output of layer 3: one block per wavefront, rows wr*32 + ..., columns wc*32 + l32.
+// Positions.  The weights are the matrix instruction's first operand and the rows its second, so that a lane has one row of
+// a block and four times four neighbouring columns of it, and what follows a product works on runs of four: the activations go to
+// LDS eight bytes at a time (with a row's columns spread over the lanes it was two bytes at a time, 64 writes a layer, and
+// the output layer's sums sixteen reductions over 32 lanes), the gradients to memory sixteen.  A 128-wide output (kWide): the
+// wavefront owns the tile's 64 rows x 32 columns as two 32 x 32 blocks, block j with row j*32 + l32, accumulator e with column
+// wave*32 + 8 (e / 4) + 4 half + e % 4.  The 64-wide output of layer 3: one block per wavefront, rows wr*32 + l32, columns
+// wc*32 + ...
 struct Place {
     int tid, lane, wave, wr, wc, l32, half;
-    __device__ __forceinline__ int rib(int e) const { return 8 * (e >> 2) + 4 * half + (e & 3); }      // row in the block
-    template <bool kWide> __device__ __forceinline__ int row(int j, int e) const { return (kWide ? j * 32 : wr * 32) + rib(e); }
-    template <bool kWide> __device__ __forceinline__ int col() const { return (kWide ? wave * 32 : wc * 32) + l32; }
+    template <bool kWide> __device__ __forceinline__ int row(int j) const { return (kWide ? j * 32 : wr * 32) + l32; }
+    template <bool kWide> __device__ __forceinline__ int col(int q) const { return (kWide ? wave * 32 : wc * 32) + 8 * q + 4 * half; }      // of accumulators 4 q .. 4 q + 3
+    template <bool kWide> __device__ __forceinline__ int operand_col() const { return (kWide ? wave * 32 : wc * 32) + l32; }               // of the weights this lane loads
 };
 
-// One layer's product for this workgroup's 64 rows: acc = A . B^T, A = 64 x kK (rows), B = (kWide ? 128 : 64) x kK
-// (`wt`: one row per output column), chunk by chunk of 16 k.
+// The products of the pass in their order; each is acc = A . B^T for this workgroup's 64 rows, A = 64 x K (rows), B = columns x K
+// (one row per output column), chunk by chunk of 16 k.
+enum Pass { kF1, kF2, kF3, kG3, kG2, kGx };          // layers 1 to 3, their data gradients back to a2, a1, and (128 columns at a time) the rows
+template <int kP> struct ProductOf {
+    static constexpr int kK = kP == kF1 ? kK1 : kP == kF2 ? kN1 : kP == kF3 ? kN2 : kP == kG3 ? kN3 : kP == kG2 ? kN2 : kN1;
+    static constexpr bool kWide = kP != kF3;
+    static constexpr int kCols = kWide ? 128 : 64;
+    static constexpr int kChunks = kK / kKC;
+    // the chunks of all products end to end, one after the other through the ring of register sets
+    static constexpr int kRing0 = kP <= kG3 ? 0 : kN3 / kKC;
+    static_assert(kN3 / kKC == 4 && kK1 / kKC % 8 == 0 && kN1 / kKC % 8 == 0 && kN2 / kKC % 8 == 0, "where each product's chunks begin in the ring");
+};
+
 // B never passes through LDS: a matrix instruction's operand is, per lane, eight consecutive k of one column -- 16
 // bytes of a packed chunk, and the 64 lanes' pieces are one contiguous kilobyte -- so every wavefront loads its own
-// operands straight into registers, kDepth chunks ahead.  In a 128-wide product a wavefront takes ALL 64 rows of 32
+// operands straight into registers, kAhead chunks ahead, across the ends of the products: the wait for a product's first
+// weights (2 us from L2 under this load, before every one of nine products) had been a third of the kernel, and the next product's
+// weights are asked for before the gradients' stores, which a load behind them would wait for (loads and stores share one
+// counter, in order).  In a 128-wide product a wavefront takes ALL 64 rows of 32
 // columns: its weight operand serves two matrix instructions' worth of rows, no other wavefront loads the same
 // columns, and the row operand -- from LDS, which has the bandwidth to spare -- is read twice as often instead.  (With
 // 32 rows x 64 columns per wavefront the two wavefronts of a column half loaded the same weights: the weights' loads,
 // 1.2 MB per tile through the compute unit's 64-byte-per-cycle load path, were the largest single part of the kernel.)
 // With the weights staged in LDS (the first version) the kernel was bound by LDS traffic: nine kilobytes read and
-// written per wavefront and chunk for six matrix instructions, and a barrier per chunk.  A comes from the activation
-// planes, with no barrier inside the product; or (kAGlobal: layer 1) from `arows` in memory through a double-buffered
-// LDS stage (the rows are float32 and have to be split and regrouped), one barrier per chunk.  Begins and ends with a
-// barrier: the planes written before the call are complete, and afterwards nobody reads the planes or the stage any more.
-// kPacked: `wt` points at the matrix's packed chunks (half precision); otherwise at float32 weights, of which a lane
-// loads its eight values and splits them itself.
-template <int kK, bool kWide, bool kAGlobal, bool kPacked, int kDepth>
-__device__ __forceinline__ void layer_product(FusedLds& S, const Place& P, v16 (&acc)[2], const void* __restrict__ wt,
-                                              const float* __restrict__ arows, int row0, int n)
-{
-    constexpr int chunks = kK / kKC;
-    constexpr int kCols = kWide ? 128 : 64;              // output columns
-    constexpr int kNB = kWide ? 2 : 1;                   // blocks (accumulators) of this wavefront
-    static_assert(chunks % kDepth == 0 && kDepth >= 2, "the chunk loop is unrolled by the number of register sets");
-    const int col = P.col<kWide>();
-    // a chunk's weight operand for this wavefront's columns, as loaded: the two parts (packed), or eight float32 weights
-    struct BSet {
-        u4v raw[2];
-    };
-    BSet B[kDepth];
-    auto bfetch = [&](int c, BSet& x) {
+// written per wavefront and chunk for six matrix instructions, and a barrier per chunk.
+// kPacked: the matrices' packed chunks (half precision); otherwise float32 weights, of which a lane loads its eight values and
+// splits them itself.
+// A stretch of memory by descriptor: a load takes the lane's offset from one 32-bit register and the wavefront's from a
+// scalar one, with no vector arithmetic (by address the compiler spends two vector instructions and two registers on each), and
+// one past the end gives zeros, a store there is dropped.
+struct Stretch {
+    __amdgpu_buffer_rsrc_t r;
+    __device__ __forceinline__ void set(const void* p, unsigned bytes) { r = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000); }
+    __device__ __forceinline__ u4v get(unsigned lane, unsigned uniform) const { return __builtin_amdgcn_raw_buffer_load_b128(r, lane, uniform, 0); }
+    // of data read once: it does not take the place of the weights in L2 (767k rows: 866 -> 830 us)
+    __device__ __forceinline__ u4v get_once(unsigned lane, unsigned uniform) const { return __builtin_amdgcn_raw_buffer_load_b128(r, lane, uniform, 2); }
+    // The whole offset is in the lane's register: behind a 16-byte store with a scalar offset the compiler sees no need to wait before
+    // it writes the data registers anew, and such stores were seen to take the new value (lanes 12 to 15 of each sixteen, the first
+    // of the four floats).  Not marked as written once: the stores take 160 us longer so.
+    __device__ __forceinline__ void put(const v4 x, unsigned lane) const
+    {
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u4v, x), r, lane, 0, 0);
+    }
+};
+
+struct BSet {
+    u4v raw[2];      // a chunk's operand for this wavefront's columns, as loaded: the two parts (packed), or eight float32 weights
+};
+constexpr int kAhead = 8;
+constexpr int kNoTile = 4;       // a type past the last: beyond the packed matrices' end
+template <bool kPacked>
+struct Weights {
+    Stretch packed;                                      // every type's packed matrices
+    const void* w[6];                                    // float32: of F1, F2, F3, G3, G2, Gx
+    const void* w_next;                                  // of F1 for the workgroup's next tile
+    int t, t_next;                                       // the types of this tile and of the workgroup's next one (kNoTile: none, and its loads give zeros)
+    BSet set[kAhead];
+
+    template <int kP>
+    __device__ __forceinline__ void fetch(const Place& P, int c, BSet& x, int column_tile = 0) const
+    {
+        fetch_of<kP>(t, w[kP], P, c, x, column_tile);
+    }
+    template <int kP>
+    __device__ __forceinline__ void fetch_of(int type, const void* w, const Place& P, int c, BSet& x, int column_tile) const
+    {
+        typedef ProductOf<kP> Q;
+        const unsigned col = P.operand_col<Q::kWide>();
         if constexpr (kPacked) {
-            const unsigned short* w = static_cast<const unsigned short*>(wt) + (c * kParts * kCols + col) * kKC + P.half * 8;
+            constexpr int kAt[6] = {kPackF1, kPackF2, kPackF3, kPackB3, kPackB2, kPackB1};
+            const unsigned at = (type * kPackPerType + kAt[kP] + column_tile * kParts * 128 * Q::kK + c * kParts * Q::kCols * kKC) * 2;
+            const unsigned lane = (col * kKC + P.half * 8) * 2;
 #pragma unroll
-            for (int m = 0; m < kParts; ++m) x.raw[m] = *reinterpret_cast<const u4v*>(w + m * kCols * kKC);
+            for (int m = 0; m < kParts; ++m) x.raw[m] = packed.get(lane, at + m * Q::kCols * kKC * 2);
         } else {
-            const float* w = static_cast<const float*>(wt) + static_cast<size_t>(col) * kK + c * kKC + P.half * 8;
-            x.raw[0] = *reinterpret_cast<const u4v*>(w);
-            x.raw[1] = *reinterpret_cast<const u4v*>(w + 4);
+            Stretch matrix;
+            matrix.set(w, type == kNoTile ? 0 : (kP == kGx ? kK1 : Q::kCols) * Q::kK * 4);
+            const unsigned at = (column_tile * 128 * Q::kK + c * kKC) * 4, lane = (col * Q::kK + P.half * 8) * 4;
+            x.raw[0] = matrix.get(lane, at);
+            x.raw[1] = matrix.get(lane, at + 16);
         }
-    };
-    auto boperand = [&](const BSet& x, h8v (&bv)[kParts]) {
+    }
+    // the chunk kAhead behind chunk c of product kP (compile-time c apart from layer 1's and the last product's repetitions)
+    template <int kP, bool kGrad>
+    __device__ __forceinline__ void fetch_behind(const Place& P, int c, BSet& x, int column_tile)
+    {
+        typedef ProductOf<kP> Q;
+        const int d = c + kAhead - Q::kChunks;           // in the product after this one
+        if (d < 0) {
+            fetch<kP>(P, c + kAhead, x, column_tile);
+        } else if constexpr (kP == kF1) {
+            fetch<kF2>(P, d, x);
+        } else if constexpr (kP == kF2) {
+            fetch<kF3>(P, d, x);
+        } else if constexpr (!kGrad) {
+            return;
+        } else if constexpr (kP == kF3) {
+            if (d < ProductOf<kG3>::kChunks) fetch<kG3>(P, d, x);
+            else fetch<kG2>(P, d - ProductOf<kG3>::kChunks, x);
+        } else if constexpr (kP == kG3) {
+            fetch<kG2>(P, d, x);
+        } else if constexpr (kP == kG2) {
+            fetch<kGx>(P, d, x);
+        } else {
+            // (a tile's chunks are four more than a multiple of the sets: chunk d + 4 of the next tile's layer 1 belongs here)
+            if (column_tile + 1 < kK1 / 128) fetch<kGx>(P, d, x, column_tile + 1);
+            else fetch_of<kF1>(t_next, w_next, P, (d + ProductOf<kGx>::kRing0) % kAhead, x, 0);
+        }
+    }
+    static __device__ __forceinline__ void operand(const BSet& x, h8v (&bv)[kParts])
+    {
         if constexpr (kPacked) {
 #pragma unroll
             for (int m = 0; m < kParts; ++m) bv[m] = __builtin_bit_cast(h8v, x.raw[m]);
@@ -215,23 +292,51 @@ __device__ __forceinline__ void layer_product(FusedLds& S, const Place& P, v16 (
 #pragma unroll
             for (int m = 0; m < kParts; ++m) bv[m] = __builtin_bit_cast(h8v, part[m]);
         }
-    };
-    // Layer 1: the feature rows go through LDS a PAIR of chunks (32 k = one 128-byte line per row) at a time: eight lanes
-    // fetch a row's line together, a thread two rows' pieces (rows r8 and r8 + 32, k8..k8+3 of the pair), and a barrier
-    // closes a pair, not a chunk.  kPairsAhead pairs are in flight in registers.
-    constexpr int kPairsAhead = 2;
-    static_assert(!kAGlobal || (kDepth == 2 * kPairsAhead && kRows == 64 && kThreads == 256), "the unrolled loop body is two pairs long");
-    const int r8 = P.tid >> 3, k8 = (P.tid & 7) << 2;
-    const int arow0 = min(row0 + r8, n - 1), arow1 = min(row0 + r8 + 32, n - 1);      // rows past the end: the last row again, never stored
-    struct APair {
+    }
+};
+
+// Layer 1: the feature rows go through LDS a PAIR of chunks (32 k = one 128-byte line per row) at a time: eight lanes
+// fetch a row's line together, a thread two rows' pieces (rows r8 and r8 + 32, k8..k8+3 of the pair), and a barrier
+// closes a pair, not a chunk.  kPairsAhead pairs are in flight in registers (as many as chunks of weights: a weight's wait is
+// one for the rows asked for before it).
+constexpr int kPairsAhead = kAhead / 2;
+static_assert(kRows == 64 && kThreads == 256, "a thread two rows' pieces");
+struct Rows {
+    struct Pair {
         v4 x[2];
     };
-    APair A[kAGlobal ? kPairsAhead : 1];
-    auto afetch = [&](int q, APair& a) {
-        a.x[0] = *reinterpret_cast<const v4*>(arows + static_cast<size_t>(arow0) * kK + q * 2 * kKC + k8);
-        a.x[1] = *reinterpret_cast<const v4*>(arows + static_cast<size_t>(arow1) * kK + q * 2 * kKC + k8);
-    };
-    auto astage_pair = [&](int q, const APair& a) {
+    Stretch tile;
+    Pair pair[kPairsAhead];
+
+    __device__ __forceinline__ void fetch(const Place& P, int q, Pair& a) const
+    {
+        // (rows past the end come back as zeros, and nothing of theirs is stored)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) a.x[u] = __builtin_bit_cast(v4, tile.get_once(lane(P) + u * 32 * kK1 * 4, q * 2 * kKC * 4));
+    }
+    static __device__ __forceinline__ unsigned lane(const Place& P) { return ((P.tid >> 3) * kK1 + ((P.tid & 7) << 2)) * 4; }
+    // the first pairs of a tile's rows
+    __device__ __forceinline__ void start(const Place& P, const float* rows, int row0, int n)
+    {
+        tile.set(rows + static_cast<size_t>(row0) * kK1, min(n - row0, kRows) * kK1 * 4);
+#pragma unroll
+        for (int q = 0; q < kPairsAhead; ++q) fetch(P, q, pair[q]);
+    }
+};
+
+// A comes from the activation planes, with no barrier inside the product; or (layer 1) from `rows` in memory, started by the
+// caller, through a double-buffered LDS stage (the rows are float32 and have to be split and regrouped), one barrier per pair of chunks.  Begins
+// and ends with a barrier: the planes written before the call are complete, and afterwards nobody reads the planes or the stage
+// any more.  The product's first kAhead chunks of weights have been asked for before.
+template <int kP, bool kGrad, bool kPacked>
+__device__ __forceinline__ void layer_product(FusedLds& S, const Place& P, v16 (&acc)[2], Weights<kPacked>& W, Rows& R, int column_tile = 0)
+{
+    typedef ProductOf<kP> Q;
+    constexpr bool kAGlobal = kP == kF1, kWide = Q::kWide;
+    constexpr int chunks = Q::kChunks;
+    constexpr int kNB = kWide ? 2 : 1;                   // blocks (accumulators) of this wavefront
+    auto astage_pair = [&](int q, const Rows::Pair& a) {
+        const int r8 = P.tid >> 3, k8 = (P.tid & 7) << 2;
         stage_piece(S.astage[q & 1], r8, k8, a.x[0]);
         stage_piece(S.astage[q & 1], r8 + 32, k8, a.x[1]);
     };
@@ -244,18 +349,14 @@ __device__ __forceinline__ void layer_product(FusedLds& S, const Place& P, v16 (
             acc[j][e] = 0.f;
             lo[j][e] = 0.f;
         }
-#pragma unroll
-    for (int s = 0; s < kDepth; ++s) bfetch(s, B[s]);
     if constexpr (kAGlobal) {
-#pragma unroll
-        for (int q = 0; q < kPairsAhead; ++q) afetch(q, A[q]);
-        astage_pair(0, A[0]);
-        if (2 * kPairsAhead < chunks) afetch(kPairsAhead, A[0]);
+        astage_pair(0, R.pair[0]);
+        R.fetch(P, kPairsAhead, R.pair[0]);
     }
     __syncthreads();             // pair 0 of the rows is staged; the activation planes written before this call are complete
     // chunk c: (layer 1, first chunk of a pair: stage the rows' next pair into the other buffer, ask for the pair
-    // kPairsAhead further on,) multiply chunk c, ask for the weights of chunk c + kDepth
-    auto step = [&](int c, BSet& b, APair& a_next) {
+    // kPairsAhead further on,) multiply chunk c, ask for the weights kAhead chunks behind it
+    auto step = [&](int c, BSet& b, Rows::Pair& a_next) {
         h8v av[2][kParts];
 #pragma unroll
         for (int j = 0; j < kNB; ++j) {
@@ -273,32 +374,37 @@ __device__ __forceinline__ void layer_product(FusedLds& S, const Place& P, v16 (
             const int q = c >> 1;
             if ((c & 1) == 0 && 2 * (q + 1) < chunks) {
                 astage_pair(q + 1, a_next);              // the other buffer: last read before the previous barrier
-                if (2 * (q + 1 + kPairsAhead) < chunks) afetch(q + 1 + kPairsAhead, a_next);
+                if (2 * (q + 1 + kPairsAhead) < chunks) R.fetch(P, q + 1 + kPairsAhead, a_next);
             }
         }
         h8v bv[kParts];
-        boperand(b, bv);
+        Weights<kPacked>::operand(b, bv);
         // independent accumulators alternate, so that no matrix instruction waits for the one before it
 #pragma unroll
-        for (int j = 0; j < kNB; ++j) lo[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[j][1], bv[0], lo[j], 0, 0, 0);
+        for (int j = 0; j < kNB; ++j) lo[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bv[0], av[j][1], lo[j], 0, 0, 0);
 #pragma unroll
-        for (int j = 0; j < kNB; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[j][0], bv[0], acc[j], 0, 0, 0);
+        for (int j = 0; j < kNB; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bv[0], av[j][0], acc[j], 0, 0, 0);
 #pragma unroll
-        for (int j = 0; j < kNB; ++j) lo[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(av[j][0], bv[1], lo[j], 0, 0, 0);
-        if (c + kDepth < chunks) bfetch(c + kDepth, b);
+        for (int j = 0; j < kNB; ++j) lo[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(bv[1], av[j][0], lo[j], 0, 0, 0);
+        W.template fetch_behind<kP, kGrad>(P, c, b, column_tile);
+        // the loads stay here, behind the chunk's products (0x386: vector, scalar and LDS instructions may pass): the compiler would
+        // gather them all behind the last product, where the next one waits for them
+        __builtin_amdgcn_sched_barrier(0x386);
         if constexpr (kAGlobal) {
             if (c & 1) __syncthreads();                  // the pair has been read, the next one is staged
         }
     };
-    for (int c = 0; c < chunks; c += kDepth) {
-        // (layer 1: kDepth = 2 kPairsAhead chunks; chunk c + u belongs to pair c / 2 + u / 2, and the pair staged during
-        // it, one further on, sits in register set (u / 2 + 1) % kPairsAhead)
+    // (layer 1: chunk c + u belongs to pair c / 2 + u / 2, and the pair staged during it, one further on, sits in register
+    // set (u / 2 + 1) % kPairsAhead)
+    constexpr int kBody = chunks < kAhead ? chunks : kAhead;
+#pragma unroll 1
+    for (int c = 0; c < chunks; c += kBody) {
 #pragma unroll
-        for (int u = 0; u < kDepth; ++u) step(c + u, B[u], A[kAGlobal ? ((u >> 1) + 1) % kPairsAhead : 0]);
+        for (int u = 0; u < kBody; ++u) step(c + u, W.set[(Q::kRing0 + u) % kAhead], R.pair[kAGlobal ? ((u >> 1) + 1) % kPairsAhead : 0]);
     }
     if constexpr (!kAGlobal) __syncthreads();
 #pragma unroll
-    for (int j = 0; j < kNB; ++j)
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[j][e] = fmaf(lo[j][e], kResidualBack, acc[j][e]);
 }
@@ -307,26 +413,34 @@ __device__ __forceinline__ void layer_product(FusedLds& S, const Place& P, v16 (
 template <bool kWide>
 __device__ __forceinline__ void to_planes(FusedLds& S, const Place& P, const v16 (&v)[2])
 {
-    const int col = P.col<kWide>();
 #pragma unroll
     for (int j = 0; j < (kWide ? 2 : 1); ++j) {
 #pragma unroll
-        for (int e = 0; e < 16; e += 2) {
-            unsigned p[kParts];
-            split_pair(v[j][e], v[j][e + 1], p[0], p[1]);
-            const int r0 = P.row<kWide>(j, e), r1 = P.row<kWide>(j, e + 1);
+        for (int q = 0; q < 4; ++q) {
+            unsigned lo[kParts], hi[kParts];
+            split_pair(v[j][4 * q], v[j][4 * q + 1], lo[0], lo[1]);
+            split_pair(v[j][4 * q + 2], v[j][4 * q + 3], hi[0], hi[1]);
 #pragma unroll
-            for (int q = 0; q < kParts; ++q) {
-                S.act[q][r0][col] = static_cast<unsigned short>(p[q] & 0xffffu);
-                S.act[q][r1][col] = static_cast<unsigned short>(p[q] >> 16);
-            }
+            for (int m = 0; m < kParts; ++m) *reinterpret_cast<u2v*>(&S.act[m][P.row<kWide>(j)][P.col<kWide>(q)]) = u2v{lo[m], hi[m]};
         }
+    }
+}
+
+// the four runs of four columns of this lane from a vector over the layer's columns
+template <bool kWide>
+__device__ __forceinline__ void of_columns(const Place& P, const float* __restrict__ from, float (&to)[16])
+{
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        const v4 f = *reinterpret_cast<const v4*>(from + P.col<kWide>(q));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) to[4 * q + e] = f[e];
     }
 }
 
 template <bool kGrad, bool kPacked>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void networks_fused_kernel(FusedArgs args, float alpha, float inv_alpha)
+void networks_fused_kernel(FusedArgs args, float alpha, float inv_alpha, float to_exp2)
 {
     static_assert(kRows == 64 && kThreads == 256, "four wavefronts: 64 rows x 32 columns each of a 128-wide output");
     __shared__ FusedLds S;
@@ -338,104 +452,172 @@ void networks_fused_kernel(FusedArgs args, float alpha, float inv_alpha)
     P.wc = P.wave & 1;
     P.l32 = P.lane & 31;
     P.half = P.lane >> 5;
-    const int tile = blockIdx.x;
-    const int t = (tile >= args.tile_end[0]) + (tile >= args.tile_end[1]) + (tile >= args.tile_end[2]);
-    const int first = t == 0 ? 0 : args.tile_end[t - 1];
-    const int row0 = (tile - first) * kRows, n = args.n[t];
-
-    // a layer's weights: split beforehand, or float32 as the caller holds them
-    const unsigned short* const pk = kPacked ? args.packed + static_cast<size_t>(t) * kPackPerType : nullptr;
-    auto weights = [&](const float* plain, int packed_at) -> const void* {
-        if constexpr (kPacked) return pk + packed_at;
-        else return plain;
+    const auto type_of = [&](int tile) { return (tile >= args.tile_end[0]) + (tile >= args.tile_end[1]) + (tile >= args.tile_end[2]); };
+    const auto row_of = [&](int tile, int t) { return (tile - (t == 0 ? 0 : args.tile_end[t - 1])) * kRows; };
+    Weights<kPacked> W;
+    Rows R;
+    W.packed.set(args.packed, 4 * kPackPerType * 2);
+    int tile = blockIdx.x, t = type_of(tile), row0 = row_of(tile, t);
+    const auto start = [&](int t, int row0) {
+        R.start(P, args.rows[t], row0, args.n[t]);
+#pragma unroll
+        for (int c = 0; c < kAhead; ++c) W.template fetch_of<kF1>(t, args.w1t[t], P, c, W.set[c], 0);
     };
-    const int cw = P.col<true>();                        // this lane's column of a 128-wide layer
+    {
+        static_assert(kThreads == kN1 + kN2 && kAtB2 == kN1 && kAtW4 == kAtB3 + kN3, "two values per thread");
+        float v[4][2], b4[4];
+        const int i = P.tid;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (args.n[k] <= 0) continue;
+            v[k][0] = i < kN1 ? args.b1[k][i] : args.b2[k][i - kN1];
+            if (i < 2 * kN3) v[k][1] = i < kN3 ? args.b3[k][i] : args.w4[k][i - kN3];
+            b4[k] = args.b4[k] ? args.b4[k][0] : 0.f;
+        }
+        start(t, row0);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (args.n[k] <= 0) continue;
+            S.fixed[k][kAtB1 + i] = v[k][0];
+            if (i < 2 * kN3) S.fixed[k][kAtB3 + i] = v[k][1];
+            if (i == 0) S.fixed[k][kAtB4] = b4[k];
+        }
+    }
+    // Of two workgroups on a compute unit the older one's wavefronts are served first, and it would be through its tiles long
+    // before the other (29 against 45 us a tile): every other tile the later workgroups have the precedence.
+    bool high = blockIdx.x >= kCUs;
+#pragma unroll 1
+    for (;;) {
+        if (high) __builtin_amdgcn_s_setprio(1); else __builtin_amdgcn_s_setprio(0);
+        high = !high;
+        const int n = args.n[t];
+        const int tile_next = tile + gridDim.x;
+        const bool more = tile_next < args.tile_end[3];
+        const int t_next = more ? type_of(tile_next) : 0, row0_next = more ? row_of(tile_next, t_next) : 0;
+        const auto advance = [&]() { tile = tile_next; t = t_next; row0 = row0_next; };
+        W.t = t;
+        W.t_next = more ? t_next : kNoTile;
+        if constexpr (!kPacked) {
+            W.w[kF1] = args.w1t[t];
+            W.w[kF2] = args.w2t[t];
+            W.w[kF3] = args.w3t[t];
+            W.w[kG3] = args.w3[t];
+            W.w[kG2] = args.w2[t];
+            W.w[kGx] = args.w1[t];
+            W.w_next = args.w1t[t_next];
+        }
 
-    v16 acc[2], a1[2], a2[2], a3[2];
-    // ------------------------------------------------------------ layer 1: 384 -> 128
-    layer_product<kK1, true, true, kPacked, kDepthRows>(S, P, acc, weights(args.w1t[t], kPackF1), args.rows[t], row0, n);
-    {
-        const float b = args.b1[t][cw];
+        v16 acc[2], a1[2], a2[2], a3[2];
+        // ------------------------------------------------------------ layer 1: 384 -> 128
+        layer_product<kF1, kGrad>(S, P, acc, W, R);
+        {
+            float b[16];
+            of_columns<true>(P, S.fixed[t] + kAtB1, b);
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) a1[j][e] = celu_of(acc[j][e] + b, alpha, inv_alpha);
-    }
-    to_planes<true>(S, P, a1);
-    // ------------------------------------------------------------ layer 2: 128 -> 128
-    layer_product<kN1, true, false, kPacked, kDepthWeights>(S, P, acc, weights(args.w2t[t], kPackF2), nullptr, row0, n);
-    {
-        const float b = args.b2[t][cw];
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) a2[j][e] = celu_of(acc[j][e] + b, alpha, inv_alpha);
-    }
-    to_planes<true>(S, P, a2);
-    // ------------------------------------------------------------ layer 3: 128 -> 64, and the output layer 64 -> 1
-    layer_product<kN2, false, false, kPacked, kDepthWeights>(S, P, acc, weights(args.w3t[t], kPackF3), nullptr, row0, n);
-    const int c3 = P.col<false>();                       // this lane's column of the 64
-    const float w4 = args.w4[t][c3];
-    {
-        const float b = args.b3[t][c3];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            a3[0][e] = celu_of(acc[0][e] + b, alpha, inv_alpha);
-            const float tot = half_sum_to_upper_row(a3[0][e] * w4);      // over this wavefront's 32 of the 64 columns
-            if (P.l32 == 16 + e) S.rowval[P.wc][P.row<false>(0, e)] = tot;
+                for (int e = 0; e < 16; ++e) a1[j][e] = celu_of(acc[j][e] + b[e], alpha, to_exp2);
         }
-    }
-    __syncthreads();
-    if (P.tid < kRows) {
-        const int gr = row0 + P.tid;
-        const float value = S.rowval[0][P.tid] + S.rowval[1][P.tid] + (args.b4[t] ? args.b4[t][0] : 0.f);
-        if (gr < n) args.value[t][gr] = value;
-    }
-    if constexpr (!kGrad) return;
-    // ------------------------------------------------------------ the way back
-    __syncthreads();             // the partial sums have been read
-    if (P.tid < kRows) S.rowval[0][P.tid] = args.scale[t] ? args.scale[t][min(row0 + P.tid, n - 1)] : 1.0f;
-    __syncthreads();
-    {
-        v16 g3[2];
+        to_planes<true>(S, P, a1);
+        // ------------------------------------------------------------ layer 2: 128 -> 128
+        layer_product<kF2, kGrad>(S, P, acc, W, R);
+        {
+            float b[16];
+            of_columns<true>(P, S.fixed[t] + kAtB2, b);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) g3[0][e] = w4 * celu_slope(a3[0][e], inv_alpha);     // for a unit upstream factor
-        to_planes<false>(S, P, g3);
-    }
-    // g2 = (g3 W3^T) .* celu'(a2): 64 -> 128
-    layer_product<kN3, true, false, kPacked, kDepthWeights>(S, P, acc, weights(args.w3[t], kPackB3), nullptr, row0, n);
+            for (int j = 0; j < 2; ++j)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+                for (int e = 0; e < 16; ++e) a2[j][e] = celu_of(acc[j][e] + b[e], alpha, to_exp2);
+        }
+        to_planes<true>(S, P, a2);
+        // ------------------------------------------------------------ layer 3: 128 -> 64, and the output layer 64 -> 1
+        layer_product<kF3, kGrad>(S, P, acc, W, R);
+        if constexpr (!kGrad) {
+            if (more) start(t_next, row0_next);
+        }
+        float w4[16];
+        of_columns<false>(P, S.fixed[t] + kAtW4, w4);
+        {
+            float b[16], part[4];
+            of_columns<false>(P, S.fixed[t] + kAtB3, b);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[j][e] *= celu_slope(a2[j][e], inv_alpha);
-    to_planes<true>(S, P, acc);
-    // g1 = (g2 W2^T) .* celu'(a1): 128 -> 128
-    layer_product<kN2, true, false, kPacked, kDepthWeights>(S, P, acc, weights(args.w2[t], kPackB2), nullptr, row0, n);
+            for (int q = 0; q < 4; ++q) {
+                part[q] = 0.f;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) acc[j][e] *= celu_slope(a1[j][e], inv_alpha);
-    to_planes<true>(S, P, acc);
-    // dx = g1 W1^T: 128 -> 384, three column tiles of 128
-    float* __restrict__ out = args.grad[t];
-    float upstream[2][16];       // the upstream factors of this lane's rows
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int e = 0; e < 16; ++e) upstream[j][e] = S.rowval[0][P.row<true>(j, e)];
-    for (int ct = 0; ct < kK1 / 128; ++ct) {
-        const void* w;
-        if constexpr (kPacked) w = pk + kPackB1 + static_cast<size_t>(ct) * kParts * 128 * kN1;
-        else w = args.w1[t] + static_cast<size_t>(ct) * 128 * kN1;
-        layer_product<kN1, true, false, kPacked, kDepthWeights>(S, P, acc, w, nullptr, row0, n);
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int gr = row0 + P.row<true>(j, e);
-                if (gr < n) out[static_cast<size_t>(gr) * kK1 + ct * 128 + cw] = acc[j][e] * upstream[j][e];
+                for (int e = 4 * q; e < 4 * q + 4; ++e) {
+                    a3[0][e] = celu_of(acc[0][e] + b[e], alpha, to_exp2);
+                    part[q] = fmaf(a3[0][e], w4[e], part[q]);
+                }
             }
+            float sum = (part[0] + part[1]) + (part[2] + part[3]);
+            sum += __shfl_xor(sum, 32, 64);                  // over this wavefront's 32 of the 64 columns
+            if (P.half == 0) S.rowval[P.wc][P.row<false>(0)] = sum;
         }
+        __syncthreads();
+        if (P.tid < kRows) {
+            const int gr = row0 + P.tid;
+            const float value = S.rowval[0][P.tid] + S.rowval[1][P.tid] + S.fixed[t][kAtB4];
+            if (gr < n) args.value[t][gr] = value;
+        }
+        if constexpr (!kGrad) {
+            if (!more) return;
+            advance();
+            continue;
+        }
+        // ------------------------------------------------------------ the way back
+        const bool given = args.scale[t] != nullptr;
+        float upstream[2];                                   // the upstream factors of this lane's rows, used after the products
+        {
+            Stretch scale;
+            scale.set(args.scale[t] + (given ? row0 : 0), given ? min(n - row0, kRows) * 4 : 0);
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                upstream[j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(scale.r, P.row<true>(j) * 4, 0, 0));
+        }
+        {
+            v16 g3[2];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) g3[0][e] = w4[e] * celu_slope(a3[0][e], inv_alpha);     // for a unit upstream factor
+            to_planes<false>(S, P, g3);
+        }
+        // g2 = (g3 W3^T) .* celu'(a2): 64 -> 128
+        layer_product<kG3, kGrad>(S, P, acc, W, R);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[j][e] *= celu_slope(a2[j][e], inv_alpha);
+        to_planes<true>(S, P, acc);
+        // g1 = (g2 W2^T) .* celu'(a1): 128 -> 128
+        layer_product<kG2, kGrad>(S, P, acc, W, R);
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[j][e] *= celu_slope(a1[j][e], inv_alpha);
+        to_planes<true>(S, P, acc);
+        // dx = g1 W1^T: 128 -> 384, three column tiles of 128
+#pragma unroll
+        for (int j = 0; j < 2; ++j) upstream[j] = given ? upstream[j] : 1.f;
+        Stretch out;
+        out.set(args.grad[t] + static_cast<size_t>(row0) * kK1, min(n - row0, kRows) * kK1 * 4);    // rows past the end are not stored
+        const auto store = [&](int ct) {
+            const unsigned lane = (P.row<true>(0) * kK1 + ct * 128 + P.col<true>(0)) * 4;
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    out.put(v4{acc[j][4 * q] * upstream[j], acc[j][4 * q + 1] * upstream[j], acc[j][4 * q + 2] * upstream[j], acc[j][4 * q + 3] * upstream[j]},
+                            lane + j * 32 * kK1 * 4 + 32 * q);
+        };
+#pragma unroll 1
+        for (int ct = 0; ct < kK1 / 128 - 1; ++ct) {
+            layer_product<kGx, kGrad>(S, P, acc, W, R, ct);
+            store(ct);
+        }
+        R.start(P, args.rows[t_next], row0_next, more ? args.n[t_next] : row0_next);      // (without a next tile: zero rows, loads that go nowhere)
+        layer_product<kGx, kGrad>(S, P, acc, W, R, kK1 / 128 - 1);
+        store(kK1 / 128 - 1);
+        if (!more) return;
+        advance();
     }
 }
 
@@ -529,13 +711,14 @@ hipError_t launch_networks_fused(const float* const rows[4], const int32_t n[4],
         want_grad = want_grad || (grad && grad[t]);
     }
     if (tiles == 0) return hipSuccess;
-    const dim3 grid(static_cast<unsigned>(tiles)), block(kThreads);
+    const dim3 grid(static_cast<unsigned>(tiles < kResident ? tiles : kResident)), block(kThreads);
+    const float to_exp2 = static_cast<float>(1.4426950408889634 / alpha);      // log2(e) / alpha
     if (want_grad) {
-        if (packed) networks_fused_kernel<true, true><<<grid, block, 0, stream>>>(a, alpha, 1.0f / alpha);
-        else networks_fused_kernel<true, false><<<grid, block, 0, stream>>>(a, alpha, 1.0f / alpha);
+        if (packed) networks_fused_kernel<true, true><<<grid, block, 0, stream>>>(a, alpha, 1.0f / alpha, to_exp2);
+        else networks_fused_kernel<true, false><<<grid, block, 0, stream>>>(a, alpha, 1.0f / alpha, to_exp2);
     } else {
-        if (packed) networks_fused_kernel<false, true><<<grid, block, 0, stream>>>(a, alpha, 1.0f / alpha);
-        else networks_fused_kernel<false, false><<<grid, block, 0, stream>>>(a, alpha, 1.0f / alpha);
+        if (packed) networks_fused_kernel<false, true><<<grid, block, 0, stream>>>(a, alpha, 1.0f / alpha, to_exp2);
+        else networks_fused_kernel<false, false><<<grid, block, 0, stream>>>(a, alpha, 1.0f / alpha, to_exp2);
     }
     return hipGetLastError();
 }

@@ -621,6 +621,43 @@ def test_whole_network_in_one_launch_matches_float64(with_scale):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ns", [(64 * 512, 0, 1, 0), (64 * 700 + 5, 1, 0, 64 * 400 + 33), (1, 64 * 512 - 63, 64 * 513, 63)])
+def test_whole_network_over_several_tiles_per_workgroup(ns):
+    """More tiles of 64 rows than the launch has workgroups (512): a workgroup then goes on from one tile to another, of its
+    own type or the next, with the next tile's rows and weights on their way while the last one's gradients are stored.  A row's
+    results do not depend on the tile it lies in, so every launch equals, bit for bit, launches over at most 8,064 rows
+    of a type (one tile per workgroup) -- values and gradients, weights split beforehand or not, again and again."""
+    from khan_amd import ops
+    dev = "cuda:0"
+    g = torch.Generator(device=dev).manual_seed(3)
+    rnd = lambda *shape: torch.randn(*shape, device=dev, generator=g)
+    widths = (384, 128, 128, 64)
+    rows = [rnd(n, 384).abs() * 0.5 for n in ns]
+    weights = [[rnd(a, b) * (2.0 / (a + b)) ** 0.5 for _ in ns] for a, b in zip(widths, widths[1:])]
+    weights_t = [[w.t().contiguous() for w in layer] for layer in weights]
+    biases = [[rnd(b) * 0.1 for _ in ns] for b in widths[1:]]
+    w4, b4, scales = [rnd(64) * 0.2 for _ in ns], [rnd(1) for _ in ns], [rnd(n) for n in ns]
+    packed = ops.pack_network_weights(weights_t, weights)
+
+    def launch(rows, scales, whole, want_grad):
+        return ops.atomic_networks(rows, None if whole else weights_t, biases, w4, b4, weights=None if whole or not want_grad else weights,
+                                   packed=packed if whole else None, scales=scales if want_grad else None, want_grad=want_grad)
+
+    want_v, want_g = [[] for _ in ns], [[] for _ in ns]
+    for at in range(0, max(ns), 8064):
+        v, gr = launch([r[at:at + 8064] for r in rows], [f[at:at + 8064].contiguous() for f in scales], True, True)
+        for t in range(4):
+            want_v[t].append(v[t])
+            want_g[t].append(gr[t])
+    want_v, want_g = [torch.cat(v) for v in want_v], [torch.cat(gr) for gr in want_g]
+    for whole, want_grad in ((True, True), (True, True), (False, True), (True, False), (False, False)):
+        v, gr = launch(rows, scales, whole, want_grad)
+        for t in range(4):
+            assert torch.equal(v[t], want_v[t]), (t, whole, want_grad)
+            assert not want_grad or torch.equal(gr[t], want_g[t]), (t, whole)
+
+
+@pytest.mark.gpu
 def test_whole_network_operand_range():
     """khan_atomic_networks_f32 forms its products from two half-precision parts per float32 operand.  Pinned here: the
     accuracy does not depend on the size of the upstream factors (1e-8, 1e+6: the gradient is carried for a unit factor
