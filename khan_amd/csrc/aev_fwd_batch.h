@@ -62,7 +62,7 @@ __device__ __forceinline__ void fwd_lds_init(FwdWaveLds<T, kJvp, kNB, kRadN, kCa
 // segment's records of A_t G_s is the product of an 8 x K by a K x 4 matrix, and v_mfma_f32_16x16x4_f32 takes four
 // records (K = 4) per instruction, using an 8 x 4 corner of its 16 x 16 result.  The variant exists to be measured
 // against the vector form; the launcher selects it on request only.
-template <bool kMatrixPhase2, typename T, bool kJvp, int kNB, int kRadN, int kCap, typename RowOfCentre>
+template <bool kMatrixPhase2, bool kOnce, typename T, bool kJvp, int kNB, int kRadN, int kCap, typename RowOfCentre>
 __device__ __forceinline__ void fwd_angular_batch(FwdWaveLds<T, kJvp, kNB, kRadN, kCap>& S, const LaneConsts<T>& L, int lane, int nb,
                                                   RowOfCentre row_of_centre)
 {
@@ -129,7 +129,7 @@ __device__ __forceinline__ void fwd_angular_batch(FwdWaveLds<T, kJvp, kNB, kRadN
     auto flush = [&]() {
         const T tot = half_wave_sum(acc);
         T* dst = reinterpret_cast<T*>((static_cast<unsigned long long>(cur_hi) << 32) | cur_lo);
-        if (lane < 32) store_global(dst + lane, tot);
+        if (lane < 32) store_global<kOnce>(dst + lane, tot);
     };
     // matrix-core form: result element (theta_t, Rs_s) of the open segment is register t % 4 of lane 16 (t / 4) + s
     typedef float mfma_acc __attribute__((ext_vector_type(4)));
@@ -139,7 +139,7 @@ __device__ __forceinline__ void fwd_angular_batch(FwdWaveLds<T, kJvp, kNB, kRadN
         if (lane < 32 && (lane & 15) < 4) {
             T* p = dst + (lane >> 4) * 16 + (lane & 15);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) store_global(p + 4 * v, static_cast<T>(macc[v]));
+            for (int v = 0; v < 4; ++v) store_global<kOnce>(p + 4 * v, static_cast<T>(macc[v]));
         }
     };
 
@@ -411,13 +411,13 @@ __device__ __forceinline__ void fwd_angular_batch(FwdWaveLds<T, kJvp, kNB, kRadN
                     const int e = e0 + lane / kLanesPer;
                     if (e < n_empty) {
                         char* dst = reinterpret_cast<char*>(S.segrow[e]) + (lane % kLanesPer) * 16;
-                        store_global16(dst);
+                        store_global16<kOnce>(dst);
                     }
                 }
                 wave_lds_fence();
             } else if (is_empty) {
                 T* dst = reinterpret_cast<T*>((static_cast<unsigned long long>(seg_row_hi) << 32) | seg_row_lo);
-                for (int q = 0; q < kAngBlock; ++q) store_global(dst + q, T(0));
+                for (int q = 0; q < kAngBlock; ++q) store_global<kOnce>(dst + q, T(0));
             }
         }
     }

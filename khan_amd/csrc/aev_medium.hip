@@ -54,7 +54,8 @@ struct __align__(16) MedShared<T, kJvp, true> {
 // With kShare the workgroups of one grid column (blockIdx.y = 0 .. gridDim.y - 1) share a molecule's centres batch by
 // batch (a form of its own: the grid's sizes in scalar registers cost the plain kernel 6 %).
 // With kLarge the kernel takes the molecules of more than 256 atoms: the atoms come type-sorted from `sorted`.
-template <typename T, bool kJvp, bool kLarge = false, bool kShare = kLarge>
+// kOnce: the rows are marked as written once (store_global)
+template <typename T, bool kJvp, bool kLarge = false, bool kShare = kLarge, bool kOnce = !kJvp && !kShare>
 __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
     const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
     const int32_t* __restrict__ A, const int32_t* __restrict__ MOs,
@@ -431,14 +432,14 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                         T acc_r = acc[a];
                         acc_r += __shfl_xor(acc_r, 16, 64);
                         acc_r += __shfl_xor(acc_r, 32, 64);
-                        if (rslot == 0) store_global(row + a * kNumRRs + (lane & 15), acc_r);
+                        if (rslot == 0) store_global<kOnce>(row + a * kNumRRs + (lane & 15), acc_r);
                     }
                 }
                 wave_lds_fence();
             }
 
             // ------------------------------------------------ segment table, phases 1 and 2, zero fill
-            fwd_angular_batch<false>(S, L, lane, nb, [&](int b) -> unsigned long long { return row_bits_of(c0 + b); });
+            fwd_angular_batch<false, kOnce>(S, L, lane, nb, [&](int b) -> unsigned long long { return row_bits_of(c0 + b); });
 
             // ------------------------------------------------ centres whose lists overflowed
             if (overflow) {
@@ -530,9 +531,12 @@ hipError_t launch_fwd_large(const T* X, const T* Y, const T* Z, const int32_t* A
     if (jvp)
         aev_fwd_medium_kernel<T, true, true><<<grid, dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, VX, VY, VZ, out,
                                                                          kMediumMaxAtoms + 1, order, sorted);
-    else
-        aev_fwd_medium_kernel<T, false, true><<<grid, dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr,
-                                                                          nullptr, out, kMediumMaxAtoms + 1, order, sorted);
+    else {
+        // rows beyond the second-level caches (32 MB) by a factor of two
+        const bool once = n_atoms * static_cast<int64_t>(kFeats * sizeof(T)) >= (64 << 20);
+        const auto kernel = once ? aev_fwd_medium_kernel<T, false, true, true, true> : aev_fwd_medium_kernel<T, false, true>;
+        kernel<<<grid, dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, out, kMediumMaxAtoms + 1, order, sorted);
+    }
     return hipGetLastError();
 }
 

@@ -58,6 +58,7 @@ void aev_fwd_small_kernel(
 {
     typedef typename Fast<T>::vec4 vec4;
     typedef typename Fast<T>::vec2 vec2;
+    constexpr bool kOnce = !kJvp && !kShare;      // a wavefront per molecule: 16,384 molecules (12,288 in double) and more
     // centres per batch: six; four in the float Jacobian-vector kernel (with kCap below: twelve wavefronts per CU)
     constexpr int kNB = (kJvp == (sizeof(T) == 4)) ? 4 : kFB;
     // angular partners kept per centre: 32; 28 in the float Jacobian-vector kernel, whose working set then is 13.4 KB
@@ -296,14 +297,14 @@ void aev_fwd_small_kernel(
                     }
                     if (rg_ns >= 2) acc_r += __shfl_xor(acc_r, 16, 64);
                     if (rg_ns == 4) acc_r += __shfl_xor(acc_r, 32, 64);
-                    if (rg_s == 0 && cb < nb) store_global(row + a * kNumRRs + (lane & 15), acc_r);
+                    if (rg_s == 0 && cb < nb) store_global<kOnce>(row + a * kNumRRs + (lane & 15), acc_r);
                 }
             }
             wave_lds_fence();
         }
 
         // ------------------------------------------------ segment table, phases 1 and 2, zero fill
-        fwd_angular_batch<kMatrixPhase2>(S, L, lane, nb, [&](int b) -> unsigned long long {
+        fwd_angular_batch<kMatrixPhase2, kOnce>(S, L, lane, nb, [&](int b) -> unsigned long long {
             const int cl = min(c0 + b, 63);
             const unsigned lo = static_cast<unsigned>(__builtin_amdgcn_ds_bpermute(cl << 2, rp_lo));
             const unsigned hi = static_cast<unsigned>(__builtin_amdgcn_ds_bpermute(cl << 2, rp_hi));

@@ -919,6 +919,27 @@ def test_random_large_molecules(ops, seed):
         check_forward_backward(ops, Case(xyz[:, 0], xyz[:, 1], xyz[:, 2], A, mi, len(mols)))
 
 
+@pytest.mark.parametrize("dtype,atoms,copies", [(torch.float32, 3, 16384), (torch.float64, 5, 16384), (torch.float32, 70, 4096),
+                                                (torch.float64, 66, 1024), (torch.float32, 700, 63), (torch.float64, 300, 74)])
+def test_rows_beyond_the_caches(ops, dtype, atoms, copies):
+    # Feature rows that together exceed the caches are stored as written once: many copies of one molecule (the sizes at which
+    # each forward kernel changes over) have the very rows that the molecule has in a batch of three.
+    say("case: %d copies of a molecule of %d atoms, %s" % (copies, atoms, dtype))
+    rng = np.random.default_rng(atoms)
+    xyz = _sparse_box(rng, atoms, 0.08, 0.9).astype(np.float32).astype(np.float64)
+    A = rng.choice(4, atoms, p=[0.5, 0.25, 0.1, 0.15]).astype(np.int32)
+
+    def rows_of(m):
+        c = Case(*(np.tile(xyz[:, k], m) for k in range(3)), np.tile(A, m), np.repeat(np.arange(m), atoms).astype(np.int32), m)
+        macs, mos, sc, ga, ac = gpu_sort_offsets(ops, c)
+        X, Y, Z = (dev(v).to(dtype) for v in (c.X, c.Y, c.Z))
+        f = ops.featurize(X, Y, Z, dev(c.A), mos, macs, sc, ac.cpu())
+        return torch.cat(f).view(-1, 384)[ga.long()].view(m, atoms, 384)
+
+    few, many = rows_of(3), rows_of(copies)
+    assert bool((few == few[:1]).all()) and bool((many == few[:1]).all())
+
+
 def test_radial_lists_at_their_fullest(ops):
     # The one-wavefront forward kernel gives every partner type a place of its own in a centre's radial list, each
     # rounded up to a whole trip of the walk.  Fullest lists: molecules of exactly 16, 32 and 64 atoms (the three scan
