@@ -256,8 +256,9 @@ __global__ __launch_bounds__(256) void large_sort_kernel(
         }
 
         // ---- the box around every 64 consecutive sorted atoms
-        __threadfence();
-        __syncthreads();                        // the workgroup's stores to sorted.atom are visible to its loads
+        // The barrier orders the workgroup's stores to sorted.atom before its loads of them: one compute unit's, through one cache.
+        // (A fence for the whole device beside it had the second-level cache written back: 34.3 -> 29.7 us.)
+        __syncthreads();
         const size_t cb = chunk_base(off, mol);
         const int n_chunks = (n + 63) >> 6;
         // four neighbouring lanes per chunk, sixteen atoms each, their loads in flight together (a wavefront per chunk spent
