@@ -41,8 +41,9 @@ HIPCC_FLAGS = [
 # kernels, and then keeps what does not fit in lanes of vector registers, to be read back inside the loops (88 to 385 scalar
 # registers spilled; 239 to 256 vector registers, 126 to 203 without).  Measured with and without, us: organic molecules in
 # float64, 16,384, forward 375 -> 362, backward 456 -> 395; 64 boxes of 1,024-4,096 atoms in float32 456 -> 435 and
-# 676 -> 665; 4,096 boxes backward 740 -> 721.  The other float32 kernels have registers to spare and are up to 2 % slower
-# without (4,096 boxes forward 630 -> 644): they are compiled as before.
+# 676 -> 665; 4,096 boxes backward 740 -> 721, and forward 638 -> 599, where the registers let a fifth workgroup in (at four it is
+# 2 % slower so).  The other float32 kernels have registers to spare and are up to 3 % slower without (4,096 boxes,
+# Jacobian-vector product, 1,518 -> 1,558): they are compiled as before.
 _NO_HOISTING = ["-mllvm", "-disable-machine-licm"]
 SOURCE_FLAGS = {name: _NO_HOISTING for name in ("aev_small_f64.hip", "aev_small_bwd_f64.hip", "aev_medium_large.hip", "aev_medium_bwd.hip")}
 

@@ -27,22 +27,19 @@ constexpr int kMedRadTrip = 1;                // list entries a lane takes per t
 template <typename T, bool kJvp> struct MedVel {};
 template <typename T> struct __align__(16) MedVel<T, true> {
     typename Fast<T>::vec4 vel[kMediumMaxAtoms];   // the incoming vector of every atom (sorted order)
+    unsigned short orig[kMediumMaxAtoms];          // its index inside the molecule
+    unsigned row_lo[kMediumMaxAtoms], row_hi[kMediumMaxAtoms];     // and the address of its output row (forward: orig in atom's last word, the address by batch)
 };
 
 template <typename T, bool kJvp, bool kLarge = false>
 struct __align__(16) MedShared {
-    typename Fast<T>::vec4 atom[kMediumMaxAtoms];   // x, y, z, type (sorted order)
-    unsigned row_lo[kMediumMaxAtoms];      // address of the atom's output row
-    unsigned row_hi[kMediumMaxAtoms];
-    unsigned short orig[kMediumMaxAtoms];  // sorted position -> index inside the molecule
+    typename Fast<T>::vec4 atom[kMediumMaxAtoms];   // x, y, z, type (kJvp) or type + 4 (index inside the molecule) (sorted order)
     int wcount[4][4];                      // atoms of each type held by each wavefront before the sort
     MedVel<T, kJvp> v;
 };
-// above 256 atoms the sorted atoms are in device memory (aev_large.h); what stays here are the output rows of the
-// centres of each wavefront's batch
+// above 256 atoms the sorted atoms are in device memory (aev_large.h)
 template <typename T, bool kJvp>
 struct __align__(16) MedShared<T, kJvp, true> {
-    unsigned long long row[4][8];
     // partner types of the entries of each wavefront's radial list and of the angular list it is building (used by the
     // Jacobian-vector product, whose list entries have no room for the type)
     unsigned char rtype[4][kRadCap];
@@ -66,10 +63,13 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
     typedef typename Fast<T>::vec4 vec4;
     typedef typename Fast<T>::vec2 vec2;
     __shared__ MedShared<T, kJvp, kLarge> M;
-    // Batches of four centres in float32: the forward kernel's working set then lets four workgroups share a CU
-    // (LDS 39.9 KB each) instead of three, which measured 21 % faster on dense boxes, and the Jacobian-vector kernel's
-    // two (75 KB each) instead of one; the float64 forward kernel keeps batches of six, and the float64 Jacobian-vector
-    // kernel takes batches of four (134 KB, one workgroup per CU; six measured the same at 157 KB of the CU's 160).
+    // Batches of four centres in float32: with them five workgroups of the forward kernel share a CU, which wants 32,000 bytes of
+    // LDS each (25 of the 1,280 that it is given out in; 31,920) and 102 registers (86, without hoisting: khan_amd/build.py).
+    // Dense boxes of 64-256 atoms, 638 -> 599 us at 4,096 and 188 -> 168 at 1,024 against four workgroups; so it has an atom's place
+    // among the rows from memory, batch by batch, and its index in the molecule beside its type, where 2.5 KB of LDS held them for
+    // every atom.  (The Jacobian-vector kernel, two workgroups either way, is 1.5 % slower so and keeps them.)  The float64
+    // forward kernel keeps batches of six, and the float64 Jacobian-vector kernel takes batches of four (one workgroup per
+    // CU; six measured the same).
     constexpr int kNB = (sizeof(T) == 4 || kJvp) ? 4 : kFB;
     __shared__ FwdWaveLds<T, kJvp, kNB> lds_wave[4];
     const int tid = threadIdx.x;
@@ -98,8 +98,8 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
             y = Y[off + tid];
             z = Z[off + tid];
             type = fold_type(A[off + tid]);
-            rowbits = reinterpret_cast<unsigned long long>(out.p[type] + static_cast<size_t>(SIs[off + tid]) * kFeats);
             if constexpr (kJvp) {
+                rowbits = reinterpret_cast<unsigned long long>(out.p[type] + static_cast<size_t>(SIs[off + tid]) * kFeats);
                 vx = VX[off + tid];
                 vy = VY[off + tid];
                 vz = VZ[off + tid];
@@ -125,11 +125,13 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
             for (int w = 0; w < wave; ++w) before += M.wcount[w][type];
             const unsigned long long mine = type == 0 ? tmask[0] : type == 1 ? tmask[1] : type == 2 ? tmask[2] : tmask[3];
             const int dest = sel4(type, tbase[0], tbase[1], tbase[2], tbase[3]) + before + popc64(mine & lt_mask);
-            M.atom[dest] = Fast<T>::make4(x, y, z, static_cast<T>(type));
-            M.row_lo[dest] = static_cast<unsigned>(rowbits & 0xffffffffull);
-            M.row_hi[dest] = static_cast<unsigned>(rowbits >> 32);
-            M.orig[dest] = static_cast<unsigned short>(tid);
-            if constexpr (kJvp) M.v.vel[dest] = Fast<T>::make4(vx, vy, vz, T(0));
+            M.atom[dest] = Fast<T>::make4(x, y, z, static_cast<T>(kJvp ? type : type + 4 * tid));
+            if constexpr (kJvp) {
+                M.v.vel[dest] = Fast<T>::make4(vx, vy, vz, T(0));
+                M.v.orig[dest] = static_cast<unsigned short>(tid);
+                M.v.row_lo[dest] = static_cast<unsigned>(rowbits);
+                M.v.row_hi[dest] = static_cast<unsigned>(rowbits >> 32);
+            }
         }
         __syncthreads();
         }
@@ -147,21 +149,31 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
         };
         auto orig_of = [&](int sorted_idx) -> int {          // wave-uniform index
             if constexpr (kLarge) return uniform(sorted.aux[off + sorted_idx].x);
-            else return uniform(static_cast<int>(M.orig[sorted_idx]));
+            else if constexpr (kJvp) return uniform(static_cast<int>(M.v.orig[sorted_idx]));
+            else return uniform(static_cast<int>(M.atom[sorted_idx].w) >> 2);
         };
         int c0 = 0;                                          // first centre of the wavefront's batch
-        auto row_bits_of = [&](int sorted_idx) -> unsigned long long {     // per-lane index inside the batch's range
-            if constexpr (kLarge) {
-                return M.row[wave][min(max(sorted_idx - c0, 0), 7)];
-            } else {
+        unsigned row_lo = 0, row_hi = 0;                     // lane b: address of the output row of the batch's centre b
+        auto row_bits_of = [&](int sorted_idx) -> unsigned long long {     // per-lane index inside the batch's range (every lane takes part)
+            if constexpr (kJvp && !kLarge) {
                 const int idx = min(sorted_idx, kMediumMaxAtoms - 1);
-                return (static_cast<unsigned long long>(M.row_hi[idx]) << 32) | M.row_lo[idx];
+                return (static_cast<unsigned long long>(M.v.row_hi[idx]) << 32) | M.v.row_lo[idx];
             }
+            const int from = min(max(sorted_idx - c0, 0), kNB - 1) << 2;
+            const unsigned lo = static_cast<unsigned>(__builtin_amdgcn_ds_bpermute(from, static_cast<int>(row_lo)));
+            const unsigned hi = static_cast<unsigned>(__builtin_amdgcn_ds_bpermute(from, static_cast<int>(row_hi)));
+            return (static_cast<unsigned long long>(hi) << 32) | lo;
         };
         auto row_of = [&](int sorted_idx) -> T* {            // wave-uniform index
-            const unsigned long long bits = row_bits_of(sorted_idx);
-            const unsigned lo = static_cast<unsigned>(uniform(static_cast<int>(bits & 0xffffffffull)));
-            const unsigned hi = static_cast<unsigned>(uniform(static_cast<int>(bits >> 32)));
+            unsigned lo, hi;
+            if constexpr (kJvp && !kLarge) {
+                const unsigned long long bits = row_bits_of(sorted_idx);
+                lo = static_cast<unsigned>(uniform(static_cast<int>(bits & 0xffffffffull)));
+                hi = static_cast<unsigned>(uniform(static_cast<int>(bits >> 32)));
+            } else {
+                lo = static_cast<unsigned>(lane_read(static_cast<int>(row_lo), sorted_idx - c0));
+                hi = static_cast<unsigned>(lane_read(static_cast<int>(row_hi), sorted_idx - c0));
+            }
             return reinterpret_cast<T*>((static_cast<unsigned long long>(hi) << 32) | lo);
         };
 
@@ -174,13 +186,15 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
         for (c0 = first_c0; c0 < n; c0 += stride_c0) {
             const int nb = min(batch, n - c0);
             unsigned overflow = 0;
-            if constexpr (kLarge) {
-                if (lane < nb) {
-                    const int type = static_cast<int>(sorted.atom[off + c0 + lane].w);
-                    T* const bucket = type == 0 ? out.p[0] : type == 1 ? out.p[1] : type == 2 ? out.p[2] : out.p[3];
-                    M.row[wave][lane] = reinterpret_cast<unsigned long long>(bucket + static_cast<size_t>(sorted.aux[off + c0 + lane].y) * kFeats);
-                }
-                wave_lds_fence();
+            if ((kLarge || !kJvp) && lane < nb) {                     // (the load is under way while the first centre is scanned)
+                const int w = static_cast<int>(atom_at(c0 + lane).w), type = w & 3;
+                int place;
+                if constexpr (kLarge) place = sorted.aux[off + c0 + lane].y;
+                else place = SIs[off + (w >> 2)];
+                T* const bucket = type == 0 ? out.p[0] : type == 1 ? out.p[1] : type == 2 ? out.p[2] : out.p[3];
+                const unsigned long long row = reinterpret_cast<unsigned long long>(bucket + static_cast<size_t>(place) * kFeats);
+                row_lo = static_cast<unsigned>(row);
+                row_hi = static_cast<unsigned>(row >> 32);
             }
 
             for (int b = 0; b < nb; ++b) {
@@ -229,7 +243,7 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                         e = S.rad()[lane];
                         if constexpr (kJvp) ab = S.jvp.rad_ab[lane];
                         if constexpr (kJvp && kLarge) tR = M.rtype[wave][lane];
-                        else tR = static_cast<int>(e.y);
+                        else tR = static_cast<int>(e.y) & 3;
                     }
                     int cnt[4], dest = 0, before = 0;
 #pragma unroll
@@ -373,7 +387,7 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                             nd = S.jvp.nbr_dfc[b][lane];
                             tA = M.atype[wave][lane];
                         } else {
-                            tA = static_cast<int>(fc);
+                            tA = static_cast<int>(fc) & 3;
                         }
                     }
                     int dest = 0, before = 0;
@@ -399,12 +413,12 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                     int tR = -1, tA = -1;           // type of this lane's list entry
                     if (haveR) {
                         const vec2 e = S.rad()[lane];
-                        tR = static_cast<int>(e.y);
+                        tR = static_cast<int>(e.y) & 3;
                         S.rad()[lane] = Fast<T>::make2(e.x, Fast<T>::cutoff(e.x, static_cast<T>(kR_Rc_f)));
                     }
                     if (haveA) {
                         const vec4 d = S.nbr[b][lane];
-                        tA = static_cast<int>(S.nbr_fc[b][lane]);
+                        tA = static_cast<int>(S.nbr_fc[b][lane]) & 3;
                         const T inv = Fast<T>::rcp(d.w);
                         S.nbr[b][lane] = Fast<T>::make4(d.x * inv, d.y * inv, d.z * inv, d.w);
                         S.nbr_fc[b][lane] = Fast<T>::cutoff(d.w, static_cast<T>(kA_Rc_f));
@@ -541,9 +555,9 @@ hipError_t launch_fwd_large(const T* X, const T* Y, const T* Z, const int32_t* A
 }
 
 #ifndef KHAN_UNIT_LARGE
-template hipError_t launch_fwd_medium<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<float>, int, const int32_t*, hipStream_t);
 template hipError_t launch_jvp_medium<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const float*, const float*, const float*, Buckets<float>, int, const int32_t*, hipStream_t);
 #else
+template hipError_t launch_fwd_medium<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<float>, int, const int32_t*, hipStream_t);
 template hipError_t launch_fwd_medium<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<double>, int, const int32_t*, hipStream_t);
 template hipError_t launch_jvp_medium<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const double*, const double*, const double*, Buckets<double>, int, const int32_t*, hipStream_t);
 template size_t large_scratch_bytes<float>(int64_t, int32_t, bool);

@@ -228,7 +228,12 @@ __device__ __forceinline__ void for_each_molecule_in_range(const int32_t* __rest
     if (size_counts) {          // molecules per size class: is there anything in [lo, hi] at all?
         int any = 0;
         for (int b = size_bin(hi) + tid; b <= size_bin(lo); b += nthreads) any |= size_counts[b];
-        if (!__syncthreads_or(any)) return;
+        const unsigned long long mask = __ballot(any != 0);      // (the library's vote takes 256 bytes of LDS)
+        if ((tid & 63) == 0) want[tid >> 6] = mask;
+        __syncthreads();
+        unsigned long long some = 0;
+        for (int w = 0; w < nwaves; ++w) some |= want[w];
+        if (!some) return;
     }
     for (long long base = blockIdx.x; base < n_mols; base += static_cast<long long>(gridDim.x) * nthreads) {
         const long long m = base + static_cast<long long>(tid) * gridDim.x;
