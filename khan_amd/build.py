@@ -26,7 +26,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 ROOT = os.path.dirname(HERE)
 
-HIP_SOURCES = ["capi.hip", "aev_generic.hip", "aev_small.hip", "aev_small_f64.hip", "aev_small_bwd.hip", "aev_small_bwd_f64.hip", "aev_medium.hip",
+HIP_SOURCES = ["capi.hip", "aev_generic.hip", "aev_small.hip", "aev_small_whole.hip", "aev_small_f64.hip", "aev_small_bwd.hip", "aev_small_bwd_f64.hip", "aev_medium.hip",
                "aev_medium_large.hip", "aev_medium_bwd.hip", "aev_large_sort.hip", "sort_offsets.hip", "charges.hip", "dense_first.hip", "dense_fused.hip", "net_layers.hip", "net_few.hip", "mol_sum.hip"]
 HIP_HEADERS = ["khan_internal.h", "khan_params.h", "aev_generic_center.h", "aev_small_common.h", "aev_fwd_batch.h", "aev_bwd_batch.h", "aev_large.h", "net_layers.h", "net_few.h", "split_bf16.h", os.path.join(ROOT, "include", "khan_aev.h")]
 
@@ -41,11 +41,12 @@ HIPCC_FLAGS = [
 # kernels, and then keeps what does not fit in lanes of vector registers, to be read back inside the loops (88 to 385 scalar
 # registers spilled; 239 to 256 vector registers, 126 to 203 without).  Measured with and without, us: organic molecules in
 # float64, 16,384, forward 375 -> 362, backward 456 -> 395; 64 boxes of 1,024-4,096 atoms in float32 456 -> 435 and
-# 676 -> 665; 4,096 boxes backward 740 -> 721, and forward 638 -> 599, where the registers let a fifth workgroup in (at four it is
-# 2 % slower so).  The other float32 kernels have registers to spare and are up to 3 % slower without (4,096 boxes,
-# Jacobian-vector product, 1,518 -> 1,558): they are compiled as before.
+# 676 -> 665; 4,096 boxes backward 740 -> 721, and forward 638 -> 599, where the registers let a fifth workgroup in (at four
+# it is 2 % slower so); 65,536 organic molecules forward 497 -> 468 with five wavefronts per SIMD instead of four.  The
+# other float32 kernels have registers to spare and are up to 3 % slower without (4,096 boxes, Jacobian-vector product,
+# 1,518 -> 1,558): they are compiled as before.
 _NO_HOISTING = ["-mllvm", "-disable-machine-licm"]
-SOURCE_FLAGS = {name: _NO_HOISTING for name in ("aev_small_f64.hip", "aev_small_bwd_f64.hip", "aev_medium_large.hip", "aev_medium_bwd.hip")}
+SOURCE_FLAGS = {name: _NO_HOISTING for name in ("aev_small_whole.hip", "aev_small_f64.hip", "aev_small_bwd_f64.hip", "aev_medium_large.hip", "aev_medium_bwd.hip")}
 
 
 def _run(cmd, cwd=None):
@@ -183,7 +184,7 @@ def build_stage_variants():
             for k in STAGE_SKIPS]
 
 
-DPP_SOURCES = ["aev_small.hip", "aev_medium.hip", "aev_medium_large.hip"]     # translation units that use fma_quad (aev_small_common.h)
+DPP_SOURCES = ["aev_small.hip", "aev_small_whole.hip", "aev_medium.hip", "aev_medium_large.hip"]     # translation units that use fma_quad (aev_small_common.h)
 
 
 def check_dpp_operands(asm_text, name="<asm>"):

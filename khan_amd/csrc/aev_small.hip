@@ -43,12 +43,15 @@ constexpr int kRadSlots = 96;
 
 // With kJvp the kernel computes the Jacobian-vector product instead (featurize_grad_inverse): every term of
 // the forward sums is replaced by its derivative along the per-atom vectors (VX, VY, VZ).
-// float: 4 wavefronts per SIMD (LDS 9.8 KB, <= 128 VGPRs; the kernel loses a fifth of its speed at three);
+// float: 4 wavefronts per SIMD (LDS 9.8 KB, <= 128 VGPRs; the kernel loses a fifth of its speed at three), and 5 with a wavefront
+// per molecule (6.9 KB, 96 VGPRs, without hoisting: khan_amd/build.py; 65,536 organic molecules 497 -> 468 us);
 // float kJvp: 3 (<= 168 VGPRs; its LDS lets twelve wavefronts share a CU); double: 3 (149 VGPRs, LDS 12.5 KB with four
 // centres); double kJvp: 1.
+constexpr int fwd_small_waves(size_t element, bool jvp, bool share) { return element == 4 ? (jvp ? 3 : share ? 4 : 5) : (jvp ? 1 : 3); }
+
 template <typename T, bool kJvp, bool kShare = false, bool kMatrixPhase2 = false>
 __global__ __launch_bounds__(64 * kWavesPerBlock)
-__attribute__((amdgpu_waves_per_eu(kJvp ? (sizeof(T) == 4 ? 3 : 1) : (sizeof(T) == 4 ? 4 : 3), kJvp ? (sizeof(T) == 4 ? 3 : 1) : (sizeof(T) == 4 ? 4 : 3))))
+__attribute__((amdgpu_waves_per_eu(fwd_small_waves(sizeof(T), kJvp, kShare), fwd_small_waves(sizeof(T), kJvp, kShare))))
 void aev_fwd_small_kernel(
     const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
     const int32_t* __restrict__ A, const int32_t* __restrict__ MOs,
@@ -59,8 +62,9 @@ void aev_fwd_small_kernel(
     typedef typename Fast<T>::vec4 vec4;
     typedef typename Fast<T>::vec2 vec2;
     constexpr bool kOnce = !kJvp && !kShare;      // a wavefront per molecule: 16,384 molecules (12,288 in double) and more
-    // centres per batch: six; four in the float Jacobian-vector kernel (with kCap below: twelve wavefronts per CU)
-    constexpr int kNB = (kJvp == (sizeof(T) == 4)) ? 4 : kFB;
+    // centres per batch: six; four in the float Jacobian-vector kernel (with kCap below: twelve wavefronts per CU) and in
+    // float with a wavefront per molecule (6.9 KB: six of the 1,280 bytes LDS is given out in, twenty wavefronts per CU)
+    constexpr int kNB = (kJvp == (sizeof(T) == 4) || (sizeof(T) == 4 && !kShare)) ? 4 : kFB;
     // angular partners kept per centre: 32; 28 in the float Jacobian-vector kernel, whose working set then is 13.4 KB
     // and twelve wavefronts share a CU (a centre with more goes to the general routine, as above 32 elsewhere)
     constexpr int kCap = (kJvp && sizeof(T) == 4) ? 28 : kCapA;
@@ -343,6 +347,24 @@ static int log_parts_of(int32_t n_mols)
     return __builtin_ctz(molecule_parts(n_mols, 4 * kResident, 8));
 }
 
+// A wavefront per molecule (in float32 a translation unit of its own: aev_small_whole.hip)
+template <typename T>
+hipError_t launch_fwd_small_whole(const T* X, const T* Y, const T* Z, const int32_t* A, const int32_t* MOs,
+                                  const int32_t* MACs, int32_t n_mols, const int32_t* SIs, Buckets<T> out,
+                                  int max_atoms, const int32_t* order, hipStream_t stream);
+#if defined(KHAN_UNIT_F64) || defined(KHAN_UNIT_WHOLE)
+template <typename T>
+hipError_t launch_fwd_small_whole(const T* X, const T* Y, const T* Z, const int32_t* A, const int32_t* MOs,
+                                  const int32_t* MACs, int32_t n_mols, const int32_t* SIs, Buckets<T> out,
+                                  int max_atoms, const int32_t* order, hipStream_t stream)
+{
+    const unsigned blocks = (static_cast<unsigned>(n_mols) + kWavesPerBlock - 1u) / kWavesPerBlock;
+    aev_fwd_small_kernel<T, false><<<dim3(blocks), dim3(64 * kWavesPerBlock), 0, stream>>>(
+        X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, out, max_atoms < 64 ? max_atoms : 64, order, 0);
+    return hipGetLastError();
+}
+#endif
+
 template <typename T>
 hipError_t launch_fwd_small(const T* X, const T* Y, const T* Z, const int32_t* A, const int32_t* MOs,
                             const int32_t* MACs, int32_t n_mols, const int32_t* SIs, Buckets<T> out,
@@ -366,8 +388,8 @@ hipError_t launch_fwd_small(const T* X, const T* Y, const T* Z, const int32_t* A
         }
     }
 #endif
-    const auto kernel = log_parts ? aev_fwd_small_kernel<T, false, true> : aev_fwd_small_kernel<T, false>;
-    kernel<<<dim3(blocks << log_parts), dim3(64 * kWavesPerBlock), 0, stream>>>(
+    if (log_parts == 0) return launch_fwd_small_whole<T>(X, Y, Z, A, MOs, MACs, n_mols, SIs, out, max_atoms, order, stream);
+    aev_fwd_small_kernel<T, false, true><<<dim3(blocks << log_parts), dim3(64 * kWavesPerBlock), 0, stream>>>(
         X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, out, max_atoms < 64 ? max_atoms : 64, order, log_parts);
     return hipGetLastError();
 }
@@ -386,7 +408,9 @@ hipError_t launch_jvp_small(const T* X, const T* Y, const T* Z, const int32_t* A
     return hipGetLastError();
 }
 
-#ifndef KHAN_UNIT_F64
+#if defined(KHAN_UNIT_WHOLE)
+template hipError_t launch_fwd_small_whole<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<float>, int, const int32_t*, hipStream_t);
+#elif !defined(KHAN_UNIT_F64)
 template hipError_t launch_fwd_small<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<float>, int, const int32_t*, hipStream_t);
 template hipError_t launch_jvp_small<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const float*, const float*, const float*, Buckets<float>, const int32_t*, hipStream_t);
 #else
