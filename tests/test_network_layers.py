@@ -253,6 +253,60 @@ def test_celu_of_small_and_large_arguments(absolute):
         assert first == 0 or got[-1] == float("inf")
 
 
+class _Top(ctypes.Structure):
+    _fields_ = ([(name, ctypes.c_void_p * 4) for name in ("act", "w", "bias", "t", "scale", "value", "out")]
+                + [("n", ctypes.c_int32 * 4), ("k", ctypes.c_int32), ("second", ctypes.c_int32), ("alpha", ctypes.c_double)])
+
+
+@pytest.mark.parametrize("dtype,unit", [(torch.float32, 2.0 ** -24), (torch.float64, 2.0 ** -53)])
+@pytest.mark.parametrize("k", [1, 5, 8, 63, 64, 68, 130, 256, 300])
+def test_output_layer_of_any_width(k, dtype, unit):
+    """The output layer alone, values and a w celu'(a) of it, and its second form scale t: widths on and off its steps of 64
+    (32) values, rows that are 16-byte aligned and rows that are not, a type without rows.  A value is a sum over lanes of
+    k / 16 + 1 products each, four steps and a bias: (k / 16 + 6) roundings of the products' sizes; celu' is three."""
+    from khan_amd import _lib
+    lib = _lib.load()
+    run = getattr(lib, "khan_net_top_f32" if dtype == torch.float32 else "khan_net_top_f64")
+    run.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    for shift in (0, 1):
+        some = lambda *shape: torch.randn(int(np.prod(shape)) + shift, dtype=dtype, device="cuda", generator=gen)[shift:].view(*shape)
+        rows = (17, 0, 1, 40)
+        act, t = [[0.1 * some(n, k) if n else None for n in rows] for _ in range(2)]
+        act = [torch.cat([torch.zeros(shift, dtype=dtype, device="cuda"), a.reshape(-1)])[shift:].view(-1, k) if a is not None else None for a in act]
+        w, bias, scale = [some(k) for _ in rows], [some(1) for _ in rows], [some(max(n, 1)) for n in rows]
+        out, value = [some(max(n, 1), k) for n in rows], [some(max(n, 1)) for n in rows]
+
+        def launch(second, scaled):
+            a = _Top(k=k, second=second, alpha=ALPHA)
+            for i, n in enumerate(rows):
+                a.n[i] = n
+                if n == 0:
+                    continue
+                a.out[i] = out[i].data_ptr()
+                if second:
+                    a.t[i] = t[i].data_ptr()
+                    if scaled:
+                        a.scale[i] = scale[i].data_ptr()
+                else:
+                    a.act[i], a.w[i], a.bias[i], a.value[i] = (v[i].data_ptr() for v in (act, w, bias, value))
+            assert run(ctypes.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+
+        launch(0, False)
+        for i, n in enumerate(rows):
+            if n:
+                h, weight = act[i].double(), w[i].double()
+                size = h.abs() @ weight.abs() + bias[i].double().abs()
+                assert ((value[i].double() - (h @ weight + bias[i].double())).abs() <= (k / 16 + 6) * unit * 1.01 * size + 4e-16 * size).all()
+                want = weight * torch.where(h >= 0, 1.0, h / ALPHA + 1)
+                assert ((out[i].double() - want).abs() <= 3 * unit * 1.01 * weight.abs() * (1 + h.abs() / ALPHA) + 4e-16).all()
+        for scaled in (False, True):
+            launch(1, scaled)
+            for i, n in enumerate(rows):
+                if n:
+                    assert torch.equal(out[i], t[i] * scale[i][:, None] if scaled else t[i])
+
+
 @pytest.mark.parametrize("dtype,unit", [(torch.float32, 2.0 ** -24), (torch.float64, 2.0 ** -53)])
 def test_bias_gradients_of_many_rows(dtype, unit):
     """Bias gradients are sums over all rows of factors of either sign: the output layer's of four types' 20,000 to 50,000 rows,
