@@ -55,7 +55,7 @@ DOMINANT = {
     ("charges_boxes4096_f64", "charges"): "charge_kernel<double, true, true>",
 }
 # the sources an entry's digest covers, by pass
-_DIGEST_SOURCES = {"networks": ("dense_fused.hip", "khan_internal.h"), "charges": ("charges.hip", "khan_internal.h")}
+_DIGEST_SOURCES = {"networks": ("dense_fused.hip", "dense_fused_tiles.h", "khan_internal.h"), "charges": ("charges.hip", "khan_internal.h")}
 
 
 def kernel_sources_digest(which="fwd"):

@@ -42,6 +42,7 @@
 // as much as by anything: 640 us with neither rows nor gradients in memory, at a clock of 1.8 GHz with the matrix units 55 % busy; with
 // them the matrix units are 39 % busy at 1.9 to 2.0 GHz; the rows and gradients alone are 440 us of memory traffic.
 // Tried and slower: gradients stored one run per chunk of the product after (4 %), stores marked as written once (18 %).
+#include "dense_fused_tiles.h"
 #include "khan_internal.h"
 #include "khan_params.h"
 
@@ -57,14 +58,14 @@ typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 typedef float f2v __attribute__((ext_vector_type(2)));
 
-constexpr int kRows = 64;           // rows per workgroup
+constexpr int kRows = kFusedRows;   // rows per workgroup
 constexpr int kResident = 2 * kCUs; // workgroups that the chip holds
 constexpr int kThreads = 256;       // four wavefronts: 64 rows x 32 columns each of a 128-wide output
-constexpr int kK1 = 384, kN1 = 128, kN2 = 128, kN3 = 64;
+constexpr int kK1 = kFusedK1, kN1 = kFusedN1, kN2 = kFusedN2, kN3 = kFusedN3;
 constexpr int kActStride = 136;     // 16-bit elements between rows of the activation planes: 128 + 8 (16-byte reads without bank conflicts)
-constexpr int kKC = 16;             // k per staged chunk = one matrix instruction deep
+constexpr int kKC = kFusedKC;       // k per staged chunk
 constexpr int kStStride = 40;       // 16-bit elements between staged rows: a pair of chunks (32 k) + 8
-constexpr int kParts = 2;           // half-precision parts per float32 operand
+constexpr int kParts = kFusedParts;
 constexpr float kResidualScale = 2048.0f, kResidualBack = 1.0f / 2048.0f;      // 2^11
 
 struct FusedArgs {
@@ -87,18 +88,6 @@ struct FusedArgs {
     float* grad[4];                 // [n_t, 384], or null
     const unsigned short* packed;   // the six weight matrices of every type already split (pack_weights_kernel), or null
 };
-
-// Packed weights: per type the six matrices one after the other (layer 1 as stored as three matrices of 128 columns),
-// each chunk by chunk of 16 k as [chunk][part][column][16 k] of half precision -- what a workgroup would otherwise split again
-// for every tile of rows it takes, laid out so that a chunk's part is one contiguous run that the workgroup's
-// threads copy 8 bytes each.
-constexpr int kPackF1 = 0;                              // layer 1 transposed: 128 columns x 384
-constexpr int kPackF2 = kPackF1 + kParts * kN1 * kK1;        // layer 2 transposed: 128 x 128
-constexpr int kPackF3 = kPackF2 + kParts * kN2 * kN1;        // layer 3 transposed: 64 x 128
-constexpr int kPackB1 = kPackF3 + kParts * kN3 * kN2;        // layer 1 as stored: 384 columns x 128
-constexpr int kPackB2 = kPackB1 + kParts * kK1 * kN1;        // layer 2 as stored: 128 x 128
-constexpr int kPackB3 = kPackB2 + kParts * kN1 * kN2;        // layer 3 as stored: 128 x 64
-constexpr int kPackPerType = kPackB3 + kParts * kN2 * kN3;   // 294,912 half-precision values
 
 // a type's biases and output layer, one after the other
 constexpr int kAtB1 = 0, kAtB2 = kAtB1 + kN1, kAtB3 = kAtB2 + kN2, kAtW4 = kAtB3 + kN3, kAtB4 = kAtW4 + kN3, kFixed = kAtB4 + 4;
@@ -190,7 +179,8 @@ template <int kP> struct ProductOf {
 // splits them itself.
 // A stretch of memory by descriptor: a load takes the lane's offset from one 32-bit register and the wavefront's from a
 // scalar one, with no vector arithmetic (by address the compiler spends two vector instructions and two registers on each), and
-// one past the end gives zeros, a store there is dropped.
+// one whose lane's offset lies past the end gives zeros, a store there is dropped.  (Whether the scalar offset counts in that is not
+// relied on: it always lies inside.)
 struct Stretch {
     __amdgpu_buffer_rsrc_t r;
     __device__ __forceinline__ void set(const void* p, unsigned bytes) { r = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000); }
@@ -210,35 +200,35 @@ struct BSet {
     u4v raw[2];      // a chunk's operand for this wavefront's columns, as loaded: the two parts (packed), or eight float32 weights
 };
 constexpr int kAhead = 8;
-constexpr int kNoTile = 4;       // a type past the last: beyond the packed matrices' end
 template <bool kPacked>
 struct Weights {
     Stretch packed;                                      // every type's packed matrices
     const void* w[6];                                    // float32: of F1, F2, F3, G3, G2, Gx
     const void* w_next;                                  // of F1 for the workgroup's next tile
-    int t, t_next;                                       // the types of this tile and of the workgroup's next one (kNoTile: none, and its loads give zeros)
+    int t, t_next;                                       // the types of this tile and of the workgroup's next one (without one: of this,
+    unsigned skip_next;                                  // and what is asked for ahead for it lies this far past the end, where a load gives zeros)
     BSet set[kAhead];
 
     template <int kP>
     __device__ __forceinline__ void fetch(const Place& P, int c, BSet& x, int column_tile = 0) const
     {
-        fetch_of<kP>(t, w[kP], P, c, x, column_tile);
+        fetch_of<kP>(t, w[kP], 0, P, c, x, column_tile);
     }
     template <int kP>
-    __device__ __forceinline__ void fetch_of(int type, const void* w, const Place& P, int c, BSet& x, int column_tile) const
+    __device__ __forceinline__ void fetch_of(int type, const void* w, unsigned skip, const Place& P, int c, BSet& x, int column_tile) const
     {
         typedef ProductOf<kP> Q;
         const unsigned col = P.operand_col<Q::kWide>();
         if constexpr (kPacked) {
             constexpr int kAt[6] = {kPackF1, kPackF2, kPackF3, kPackB3, kPackB2, kPackB1};
-            const unsigned at = (type * kPackPerType + kAt[kP] + column_tile * kParts * 128 * Q::kK + c * kParts * Q::kCols * kKC) * 2;
-            const unsigned lane = (col * kKC + P.half * 8) * 2;
+            const unsigned at = packed_chunk_at(type, kAt[kP], Q::kCols, Q::kK, column_tile, c);
+            const unsigned lane = (col * kKC + P.half * 8) * 2 + skip;
 #pragma unroll
             for (int m = 0; m < kParts; ++m) x.raw[m] = packed.get(lane, at + m * Q::kCols * kKC * 2);
         } else {
             Stretch matrix;
-            matrix.set(w, type == kNoTile ? 0 : (kP == kGx ? kK1 : Q::kCols) * Q::kK * 4);
-            const unsigned at = (column_tile * 128 * Q::kK + c * kKC) * 4, lane = (col * Q::kK + P.half * 8) * 4;
+            matrix.set(w, (kP == kGx ? kK1 : Q::kCols) * Q::kK * 4);
+            const unsigned at = (column_tile * 128 * Q::kK + c * kKC) * 4, lane = (col * Q::kK + P.half * 8) * 4 + skip;
             x.raw[0] = matrix.get(lane, at);
             x.raw[1] = matrix.get(lane, at + 16);
         }
@@ -267,7 +257,7 @@ struct Weights {
         } else {
             // (a tile's chunks are four more than a multiple of the sets: chunk d + 4 of the next tile's layer 1 belongs here)
             if (column_tile + 1 < kK1 / 128) fetch<kGx>(P, d, x, column_tile + 1);
-            else fetch_of<kF1>(t_next, w_next, P, (d + ProductOf<kGx>::kRing0) % kAhead, x, 0);
+            else fetch_of<kF1>(t_next, w_next, skip_next, P, (d + ProductOf<kGx>::kRing0) % kAhead, x, 0);
         }
     }
     static __device__ __forceinline__ void operand(const BSet& x, h8v (&bv)[kParts])
@@ -308,19 +298,19 @@ struct Rows {
     Stretch tile;
     Pair pair[kPairsAhead];
 
-    __device__ __forceinline__ void fetch(const Place& P, int q, Pair& a) const
+    __device__ __forceinline__ void fetch(const Place& P, int q, Pair& a, unsigned skip = 0) const
     {
         // (rows past the end come back as zeros, and nothing of theirs is stored)
 #pragma unroll
-        for (int u = 0; u < 2; ++u) a.x[u] = __builtin_bit_cast(v4, tile.get_once(lane(P) + u * 32 * kK1 * 4, q * 2 * kKC * 4));
+        for (int u = 0; u < 2; ++u) a.x[u] = __builtin_bit_cast(v4, tile.get_once(lane(P) + u * 32 * kK1 * 4 + skip, q * 2 * kKC * 4));
     }
     static __device__ __forceinline__ unsigned lane(const Place& P) { return ((P.tid >> 3) * kK1 + ((P.tid & 7) << 2)) * 4; }
-    // the first pairs of a tile's rows
-    __device__ __forceinline__ void start(const Place& P, const float* rows, int row0, int n)
+    // the first pairs of a tile's rows (skip: kFusedSkip where there is no tile, and zeros come back)
+    __device__ __forceinline__ void start(const Place& P, const float* rows, int row0, int n, unsigned skip = 0)
     {
         tile.set(rows + static_cast<size_t>(row0) * kK1, min(n - row0, kRows) * kK1 * 4);
 #pragma unroll
-        for (int q = 0; q < kPairsAhead; ++q) fetch(P, q, pair[q]);
+        for (int q = 0; q < kPairsAhead; ++q) fetch(P, q, pair[q], skip);
     }
 };
 
@@ -452,16 +442,14 @@ void networks_fused_kernel(FusedArgs args, float alpha, float inv_alpha, float t
     P.wc = P.wave & 1;
     P.l32 = P.lane & 31;
     P.half = P.lane >> 5;
-    const auto type_of = [&](int tile) { return (tile >= args.tile_end[0]) + (tile >= args.tile_end[1]) + (tile >= args.tile_end[2]); };
-    const auto row_of = [&](int tile, int t) { return (tile - (t == 0 ? 0 : args.tile_end[t - 1])) * kRows; };
     Weights<kPacked> W;
     Rows R;
-    W.packed.set(args.packed, 4 * kPackPerType * 2);
-    int tile = blockIdx.x, t = type_of(tile), row0 = row_of(tile, t);
+    W.packed.set(args.packed, kPackBytes);
+    FusedTile at = fused_tile(args.tile_end, static_cast<int>(blockIdx.x));
     const auto start = [&](int t, int row0) {
         R.start(P, args.rows[t], row0, args.n[t]);
 #pragma unroll
-        for (int c = 0; c < kAhead; ++c) W.template fetch_of<kF1>(t, args.w1t[t], P, c, W.set[c], 0);
+        for (int c = 0; c < kAhead; ++c) W.template fetch_of<kF1>(t, args.w1t[t], 0, P, c, W.set[c], 0);
     };
     {
         static_assert(kThreads == kN1 + kN2 && kAtB2 == kN1 && kAtW4 == kAtB3 + kN3, "two values per thread");
@@ -474,7 +462,7 @@ void networks_fused_kernel(FusedArgs args, float alpha, float inv_alpha, float t
             if (i < 2 * kN3) v[k][1] = i < kN3 ? args.b3[k][i] : args.w4[k][i - kN3];
             b4[k] = args.b4[k] ? args.b4[k][0] : 0.f;
         }
-        start(t, row0);
+        start(at.type, at.row0);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             if (args.n[k] <= 0) continue;
@@ -490,13 +478,12 @@ void networks_fused_kernel(FusedArgs args, float alpha, float inv_alpha, float t
     for (;;) {
         if (high) __builtin_amdgcn_s_setprio(1); else __builtin_amdgcn_s_setprio(0);
         high = !high;
-        const int n = args.n[t];
-        const int tile_next = tile + gridDim.x;
-        const bool more = tile_next < args.tile_end[3];
-        const int t_next = more ? type_of(tile_next) : 0, row0_next = more ? row_of(tile_next, t_next) : 0;
-        const auto advance = [&]() { tile = tile_next; t = t_next; row0 = row0_next; };
+        const FusedTile next = fused_next(args.tile_end, at, static_cast<int>(gridDim.x));
+        const bool more = next.tile != at.tile;
+        const int t = at.type, row0 = at.row0, n = args.n[t];
         W.t = t;
-        W.t_next = more ? t_next : kNoTile;
+        W.t_next = next.type;
+        W.skip_next = more ? 0u : kFusedSkip;
         if constexpr (!kPacked) {
             W.w[kF1] = args.w1t[t];
             W.w[kF2] = args.w2t[t];
@@ -504,7 +491,7 @@ void networks_fused_kernel(FusedArgs args, float alpha, float inv_alpha, float t
             W.w[kG3] = args.w3[t];
             W.w[kG2] = args.w2[t];
             W.w[kGx] = args.w1[t];
-            W.w_next = args.w1t[t_next];
+            W.w_next = args.w1t[next.type];
         }
 
         v16 acc[2], a1[2], a2[2], a3[2];
@@ -533,7 +520,7 @@ void networks_fused_kernel(FusedArgs args, float alpha, float inv_alpha, float t
         // ------------------------------------------------------------ layer 3: 128 -> 64, and the output layer 64 -> 1
         layer_product<kF3, kGrad>(S, P, acc, W, R);
         if constexpr (!kGrad) {
-            if (more) start(t_next, row0_next);
+            if (more) start(next.type, next.row0);
         }
         float w4[16];
         of_columns<false>(P, S.fixed[t] + kAtW4, w4);
@@ -561,7 +548,7 @@ void networks_fused_kernel(FusedArgs args, float alpha, float inv_alpha, float t
         }
         if constexpr (!kGrad) {
             if (!more) return;
-            advance();
+            at = next;
             continue;
         }
         // ------------------------------------------------------------ the way back
@@ -613,11 +600,11 @@ void networks_fused_kernel(FusedArgs args, float alpha, float inv_alpha, float t
             layer_product<kGx, kGrad>(S, P, acc, W, R, ct);
             store(ct);
         }
-        R.start(P, args.rows[t_next], row0_next, more ? args.n[t_next] : row0_next);      // (without a next tile: zero rows, loads that go nowhere)
+        R.start(P, args.rows[next.type], next.row0, args.n[next.type], W.skip_next);
         layer_product<kGx, kGrad>(S, P, acc, W, R, kK1 / 128 - 1);
         store(kK1 / 128 - 1);
         if (!more) return;
-        advance();
+        at = next;
     }
 }
 
@@ -660,7 +647,7 @@ __global__ __launch_bounds__(256) void pack_weights_kernel(FusedArgs args, unsig
 
 }  // namespace
 
-size_t networks_packed_bytes() { return static_cast<size_t>(4) * kPackPerType * sizeof(unsigned short); }
+size_t networks_packed_bytes() { return kPackBytes; }
 
 // the six weight matrices of each type (three transposed, three as stored) split into `packed` (networks_packed_bytes());
 // w*t null: the transposed ones from the stored ones
