@@ -635,9 +635,14 @@ __device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __rest
 // 42 -> 28.  What is left is products (14 us), splitting and the loads of 144 MB (30 us) one after the other.  No faster: two
 // chunks in flight instead of one (with the small products added to the large ones chunk by chunk, for its registers),
 // splitting by v_dot2_f32_bf16 (seven instructions instead of eleven).
-// An element that is not finite (infinite, NaN or overflowing operands: the split makes NaN of infinities) has the workgroup
-// form its tile again by float32 multiply-adds, so that infinities and NaN come out as they do there.
+// Both operands are split 2^24 times their size (the bias sums are formed before): a value's third part has its exponent 24
+// below the value's, and of values below 2^-110 it would lose bits at the end of bfloat16's exponents (2^-115: gradients 1e-6
+// off, 2^-125: 1e-3), as they are when a loss is scaled down that far.  The sums are scaled back exactly.
+// An element that is not finite (infinite, NaN or overflowing operands: the split makes NaN of infinities; sums from 2^80 on)
+// has the workgroup form its tile again by float32 multiply-adds whose roundings are carried along (2,048 rows added up plainly
+// are further off than the matrix instructions' sums), so that infinities and NaN come out as they do there.
 constexpr int kGradLeft = 128, kGradChunk = 32;
+constexpr float kGradLift = 0x1p24f;
 struct SplitGradLds {
     u4v left[3][4][kGradLeft], right[3][4][128];
 };
@@ -727,6 +732,11 @@ __device__ __forceinline__ void weight_grad_split_tile(const NetGrads<float>& a,
 #pragma unroll
                 for (int i = 0; i < 8; ++i) add_exactly(bias, bias_lost, y[i]);
             }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                x[i] *= kGradLift;
+                y[i] *= kGradLift;
+            }
             __syncthreads();                   // the planes' previous contents have been read
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
@@ -786,11 +796,16 @@ __device__ __forceinline__ void weight_grad_split_tile(const NetGrads<float>& a,
 #pragma unroll
             for (int v = 0; v < 4; ++v) bad = bad || !isfinite(acc[i][j][v]);
         }
-    if (__syncthreads_or(bad)) {
+    const bool again = __syncthreads_or(bad);
+#pragma unroll
+    for (int i = 0; i < kRB; ++i)
+#pragma unroll
+        for (int j = 0; j < kLB; ++j) acc[i][j] *= 1.0f / (kGradLift * kGradLift);
+    if (again) {
 #pragma unroll
         for (int i = 0; i < kRB; ++i)
 #pragma unroll
-            for (int j = 0; j < kLB; ++j) acc[i][j] = f4v(0.f);
+            for (int j = 0; j < kLB; ++j) acc[i][j] = small[i][j] = f4v(0.f);        // (small: what the sums' roundings lost)
 #pragma unroll 1
         for (int pair = 0; pair < 2; ++pair) {
             if (!live_pair(pair)) continue;
@@ -809,10 +824,20 @@ __device__ __forceinline__ void weight_grad_split_tile(const NetGrads<float>& a,
                         const int place = 16 * (rb0 + i) + 4 * grp + v, column = j0 + (kWide ? grad_column(place) : place);
                         const float rv = op.right[static_cast<size_t>(r) * N + min(column, N - 1)] * s;
 #pragma unroll
-                        for (int j = 0; j < kLB; ++j) acc[i][j][v] = fmaf(lv[j], rv, acc[i][j][v]);
+                        for (int j = 0; j < kLB; ++j) {
+                            const float sum = acc[i][j][v], s1 = fmaf(lv[j], rv, sum), b = s1 - sum;
+                            small[i][j][v] += fmaf(lv[j], rv, -b) + (sum - (s1 - b));
+                            acc[i][j][v] = s1;
+                        }
                     }
             }
         }
+#pragma unroll
+        for (int i = 0; i < kRB; ++i)
+#pragma unroll
+            for (int j = 0; j < kLB; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) acc[i][j][v] = with_lost(acc[i][j][v], small[i][j][v]);
     }
     // partial sums: [left place][right place], then the right columns' own sums by place
     float* __restrict__ out = partial + a.job_base[job] + static_cast<size_t>(rel) * (kGradLeft * kCols + kCols);

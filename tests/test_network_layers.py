@@ -223,6 +223,39 @@ def test_weight_gradients_on_split_products(widths, rows, both):
         assert ((got - want).abs() <= 2e-6 * size)[known].all()
 
 
+def _one_layer_gradients(lib, left, right):
+    """The weight and bias gradients of one layer with rows of one type: left [n, k], right [n, n_out] -> float64 on the CPU."""
+    (n, k), n_out = left.shape, right.shape[1]
+    a = _Grads(layers=1, first=1, second=0, scale_first=0, scale_second=0)
+    a.widths[0], a.widths[1], a.n[0], a.x[0], a.right[0] = k, n_out, n, left.data_ptr(), right.data_ptr()
+    out = torch.full((4 * (k + 1) * n_out,), 7.0, device="cuda")
+    work = torch.empty(lib.khan_net_grads_workspace_bytes_f32(ctypes.byref(a)), dtype=torch.uint8, device="cuda")
+    a.out, a.workspace = out.data_ptr(), work.data_ptr()
+    assert lib.khan_net_grads_f32(ctypes.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+    return out[:k * n_out].view(k, n_out).cpu().double(), out[4 * k * n_out:][:n_out].cpu().double()
+
+
+# Operands at both ends of float32's exponents: near the bottom the third part of a bfloat16 split would run out of them, near
+# the top the sums leave the split form.  Sums of 12,800 products in float32: the 2e-6 of sum |left| |right| of the test above.
+# (sum |left| |right| stays below 2^127: beyond, which sums overflow depends on the order they are formed in.)
+@pytest.mark.parametrize("left_exponent,right_exponent", [(0, -112), (0, -118), (0, -125), (-118, 0), (-125, 0), (-118, 40), (-60, -60), (0, 100),
+                                                          (104, -104), (40, 30), (56, 56)])
+def test_weight_gradients_of_tiny_and_huge_operands(left_exponent, right_exponent):
+    from khan_amd import _lib
+    lib = _lib.load()
+    print("case:", left_exponent, right_exponent, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    make = lambda width, exponent: torch.ldexp(torch.randn(12800, width, device="cuda", generator=gen, dtype=torch.float64),
+                                               torch.tensor(exponent, device="cuda")).float()
+    left, right = make(384, left_exponent), make(128, right_exponent)
+    weights, bias = _one_layer_gradients(lib, left, right)
+    l, r = left.cpu().double(), right.cpu().double()
+    want, size = l.t() @ r, l.abs().t() @ r.abs()
+    assert size.max() < 2.0 ** 127
+    assert ((weights - want).abs() <= 2e-6 * size).all(), ((weights - want).abs() / size).max().item()
+    assert ((bias - r.sum(0)).abs() <= 2e-6 * r.abs().sum(0)).all()
+
+
 @pytest.mark.parametrize("absolute", [False, True])
 def test_celu_of_small_and_large_arguments(absolute):
     """The layers' float32 CELU over the binades of negative arguments from -1e-30 on (below, the split operands' smallest parts
