@@ -802,23 +802,23 @@ __device__ __forceinline__ void weight_grad_split_tile(const NetGrads<float>& a,
 #pragma unroll
         for (int j = 0; j < kLB; ++j) acc[i][j] *= 1.0f / (kGradLift * kGradLift);
     if (again) {
+        // (a block of 16 right columns at a time: the roundings of all of them do not fit in the registers)
 #pragma unroll
-        for (int i = 0; i < kRB; ++i)
+        for (int i = 0; i < kRB; ++i) {
+            f4v lost[kLB];
 #pragma unroll
-            for (int j = 0; j < kLB; ++j) acc[i][j] = small[i][j] = f4v(0.f);        // (small: what the sums' roundings lost)
+            for (int j = 0; j < kLB; ++j) acc[i][j] = lost[j] = f4v(0.f);
 #pragma unroll 1
-        for (int pair = 0; pair < 2; ++pair) {
-            if (!live_pair(pair)) continue;
-            const Operands op = operands(pair);
+            for (int pair = 0; pair < 2; ++pair) {
+                if (!live_pair(pair)) continue;
+                const Operands op = operands(pair);
 #pragma unroll 1
-            for (int r = r0; r < r1; ++r) {
-                const float s = op.scale ? op.scale[r] : 1.0f;
-                float lv[kLB];
+                for (int r = r0; r < r1; ++r) {
+                    const float s = op.scale ? op.scale[r] : 1.0f;
+                    float lv[kLB];
 #pragma unroll
-                for (int j = 0; j < kLB; ++j)
-                    lv[j] = op.left[static_cast<size_t>(r) * K + min(i0 + grad_column(16 * (lb0 + j) + l16), K - 1)];
-#pragma unroll
-                for (int i = 0; i < kRB; ++i)
+                    for (int j = 0; j < kLB; ++j)
+                        lv[j] = op.left[static_cast<size_t>(r) * K + min(i0 + grad_column(16 * (lb0 + j) + l16), K - 1)];
 #pragma unroll
                     for (int v = 0; v < 4; ++v) {
                         const int place = 16 * (rb0 + i) + 4 * grp + v, column = j0 + (kWide ? grad_column(place) : place);
@@ -826,18 +826,17 @@ __device__ __forceinline__ void weight_grad_split_tile(const NetGrads<float>& a,
 #pragma unroll
                         for (int j = 0; j < kLB; ++j) {
                             const float sum = acc[i][j][v], s1 = fmaf(lv[j], rv, sum), b = s1 - sum;
-                            small[i][j][v] += fmaf(lv[j], rv, -b) + (sum - (s1 - b));
+                            lost[j][v] += fmaf(lv[j], rv, -b) + (sum - (s1 - b));
                             acc[i][j][v] = s1;
                         }
                     }
+                }
             }
-        }
-#pragma unroll
-        for (int i = 0; i < kRB; ++i)
 #pragma unroll
             for (int j = 0; j < kLB; ++j)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) acc[i][j][v] = with_lost(acc[i][j][v], small[i][j][v]);
+                for (int v = 0; v < 4; ++v) acc[i][j][v] = with_lost(acc[i][j][v], lost[j][v]);
+        }
     }
     // partial sums: [left place][right place], then the right columns' own sums by place
     float* __restrict__ out = partial + a.job_base[job] + static_cast<size_t>(rel) * (kGradLeft * kCols + kCols);
