@@ -884,19 +884,19 @@ __global__ __launch_bounds__(256, kSplit ? 2 : 1) void weight_grad_kernel(const 
     }
 }
 
-// The workgroups' partial tiles and bias sums -> the gradients.  A workgroup takes 64 runs of 16 bytes of one tile, its
-// wavefronts a quarter of the shares each, one after the other; the quarters are added in order.  (A thread per element of
-// the result waits for as many loads of its own as there are shares: 45 us for 100 of them, 39 MB.)
-template <typename T>
+// The workgroups' partial tiles and bias sums -> the gradients: 64 runs of 16 bytes of one tile to a wavefront, or (kQuarters) to a
+// workgroup, whose wavefronts take a quarter of the shares each; the quarters are added in order.
+template <typename T, bool kQuarters>
 __global__ __launch_bounds__(256) void grad_sum_kernel(const NetGrads<T> a, const T* __restrict__ partial)
 {
     constexpr int V = MatrixOp<T>::kVec, kSide = 16 * V, kRun = 64 * V;
-    __shared__ Vec<T> quarter[4][2][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     int64_t out = 0;                       // where the layer's weights begin
     int block = static_cast<int>(blockIdx.x), layer = 0, rows, cols, tiles_n, tiles, runs;
+    if constexpr (!kQuarters) block = 4 * block + wave;
     bool split;
     for (;; ++layer) {
+        if (!kQuarters && layer == a.layers) return;
         split = (a.split >> layer) & 1u;
         rows = split ? kGradLeft : kSide;
         cols = split ? (a.k[layer + 1] > 64 ? 128 : 64) : kSide;
@@ -913,18 +913,37 @@ __global__ __launch_bounds__(256) void grad_sum_kernel(const NetGrads<T> a, cons
     const T* p = partial + a.job_base[layer * 4 + t] + static_cast<size_t>(tile) * size + min(at, size - V);
     const size_t stride = static_cast<size_t>(tiles) * size;
     Vec<T> sum = Vec<T>(T(0)), lost = Vec<T>(T(0));
-    const int first = wave * shares >> 2, last = (wave + 1) * shares >> 2;
-#pragma unroll 8
-    for (int s = first; s < last; ++s) add_exactly(sum, lost, *reinterpret_cast<const Vec<T>*>(p + s * stride));
-    quarter[wave][0][lane] = sum;
-    quarter[wave][1][lane] = lost;
-    __syncthreads();
-    if (wave > 0 || at >= size) return;
+    const int first = kQuarters ? wave * shares >> 2 : 0, last = kQuarters ? (wave + 1) * shares >> 2 : shares;
+    constexpr int U = kQuarters ? 8 : 4;       // loads in flight together
+    int s = first;
+    for (; s + U <= last; s += U) {
+        Vec<T> v[U];
 #pragma unroll
-    for (int w = 1; w < 4; ++w) {
-        add_exactly(sum, lost, quarter[w][0][lane]);
-        lost += quarter[w][1][lane];
+        for (int u = 0; u < U; ++u) v[u] = *reinterpret_cast<const Vec<T>*>(p + (s + u) * stride);
+#pragma unroll
+        for (int u = 0; u < U; ++u) add_exactly(sum, lost, v[u]);
     }
+    if (s < last) {
+        Vec<T> v[U - 1];
+#pragma unroll
+        for (int u = 0; u < U - 1; ++u) v[u] = *reinterpret_cast<const Vec<T>*>(p + min(s + u, last - 1) * stride);
+#pragma unroll
+        for (int u = 0; u < U - 1; ++u)
+            if (s + u < last) add_exactly(sum, lost, v[u]);
+    }
+    if constexpr (kQuarters) {
+        __shared__ Vec<T> quarter[4][2][64];
+        quarter[wave][0][lane] = sum;
+        quarter[wave][1][lane] = lost;
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int w = 1; w < 4; ++w) {
+            add_exactly(sum, lost, quarter[w][0][lane]);
+            lost += quarter[w][1][lane];
+        }
+    }
+    if (at >= size) return;
     const bool is_bias = at >= rows * cols;
     if (is_bias && tile >= tiles_n) return;                    // the first row of tiles holds the bias sums
     int row = tile / tiles_n * rows;
@@ -934,13 +953,21 @@ __global__ __launch_bounds__(256) void grad_sum_kernel(const NetGrads<T> a, cons
         for (int l = layer; l < a.layers; ++l) out += 4 * static_cast<int64_t>(a.k[l]) * a.k[l + 1];
         for (int l = 0; l < layer; ++l) out += 4 * a.k[l + 1];
     }
+    if (row >= K) return;
+    T* const to = a.out + out + (is_bias ? static_cast<int64_t>(t) : static_cast<int64_t>(t) * K + row) * N;
+    const int place = at % cols, column0 = tile % tiles_n * cols;
+    Vec<T> value;
+#pragma unroll
+    for (int e = 0; e < V; ++e) value[e] = with_lost(sum[e], lost[e]);
+    const bool apart = split && cols == 128;                   // (columns two apart)
+    if (!apart && column0 + place + V <= N && (reinterpret_cast<uintptr_t>(to + column0 + place) & 15u) == 0) {
+        *reinterpret_cast<Vec<T>*>(to + column0 + place) = value;
+        return;
+    }
 #pragma unroll
     for (int e = 0; e < V; ++e) {
-        const int place = at % cols + e, column = tile % tiles_n * cols + (split && cols == 128 ? grad_column(place) : place);
-        if (column >= N || row >= K) continue;
-        const T value = with_lost(sum[e], lost[e]);
-        if (is_bias) a.out[out + t * N + column] = value;
-        else a.out[out + (static_cast<int64_t>(t) * K + row) * N + column] = value;
+        const int column = column0 + (apart ? grad_column(place + e) : place + e);
+        if (column < N) to[column] = value[e];
     }
 }
 
@@ -1120,12 +1147,21 @@ hipError_t launch_net_grads(NetGrads<T> a, void* workspace, hipStream_t stream)
         }
         kernel<<<dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream>>>(a, static_cast<T*>(workspace));
     }
-    unsigned sums = 0;
+    int64_t sums = 0;
     for (int l = 0; l < a.layers; ++l) {
         const int rows = a.split >> l & 1u ? kGradLeft : 16 * V, cols = a.split >> l & 1u ? (a.k[l + 1] > 64 ? 128 : 64) : 16 * V;
-        sums += 4u * ((a.k[l] + rows - 1) / rows) * ((a.k[l + 1] + cols - 1) / cols) * ((rows * cols + cols + 64 * V - 1) / (64 * V));
+        sums += 4ll * ((a.k[l] + rows - 1) / rows) * ((a.k[l + 1] + cols - 1) / cols) * ((rows * cols + cols + 64 * V - 1) / (64 * V));
     }
-    grad_sum_kernel<T><<<dim3(sums), dim3(256), 0, stream>>>(a, static_cast<const T*>(workspace));
+    // A workgroup's four wavefronts to each run where there are few runs for the shares (us of gradients and sums, a wavefront to
+    // each run -> four): 384-128-128-64-1 (1,300 times 64 runs), 8 shares 15.4 -> 16.7, 17 shares 20.3 -> 20.4, 85 shares
+    // 69.7 -> 67.9; 384-64-1 (480), 10 shares 13.2 -> 12.8; eleven layers (9,600 to 11,600), 3 to 13 shares 31 -> 50, 61 -> 80, 372 -> 387.
+    const int per = a.split ? a.per_split : a.per;
+    int most = 0;
+    for (int t = 0; t < 4; ++t) most = std::max(most, a.n[t]);
+    if ((static_cast<int64_t>(most) + per - 1) / per * 50 > sums)
+        grad_sum_kernel<T, true><<<dim3(static_cast<unsigned>(sums)), dim3(256), 0, stream>>>(a, static_cast<const T*>(workspace));
+    else
+        grad_sum_kernel<T, false><<<dim3(static_cast<unsigned>((sums + 3) / 4)), dim3(256), 0, stream>>>(a, static_cast<const T*>(workspace));
     return hipGetLastError();
 }
 

@@ -235,6 +235,48 @@ def _one_layer_gradients(lib, left, right):
     return out[:k * n_out].view(k, n_out).cpu().double(), out[4 * k * n_out:][:n_out].cpu().double()
 
 
+# Every plan of the weight gradients: few rows of many tiles (a wavefront to each run of the sums) and many rows of few (a
+# workgroup), both sides of the lines between float32 and split products, several rounds of workgroups (36 tiles, 60,000 rows),
+# narrow layers beside wide ones, widths that are no multiple of anything.  A share's sum has at most 2,048 / 4 + 4 products one
+# after the other on a lane and 64 on the split form's, shares and quarters carry their roundings: float64 stays below 520 units of
+# 2^-53, float32 below the 2e-6 of the tests above (its sums over wavefronts and matrix steps are far from their worst case).
+@pytest.mark.parametrize("dtype,bound", [(torch.float32, 2e-6), (torch.float64, 520 * 2.0 ** -53)])
+@pytest.mark.parametrize("widths,rows", [((384, 512, 512, 256, 1), (5, 0, 1, 2)), ((384, 512, 512, 1), (31200, 20400, 3601, 4799)), ((384, 256, 1), (12000, 7000, 33, 1)),
+                                         ((384, 128, 128, 64, 1), (1000, 700, 200, 98)), ((384, 128, 128, 64, 1), (1300, 850, 150, 200)),
+                                         ((384, 128, 128, 64, 1), (2500, 1700, 300, 299)), ((384, 128, 128, 64, 1), (2500, 1700, 300, 301)),
+                                         ((384, 64, 1), (4000, 3000, 500, 499)), ((37, 66, 5, 1), (300, 0, 17, 1))])
+def test_weight_gradients_of_every_plan(widths, rows, dtype, bound):
+    from khan_amd import _lib
+    lib = _lib.load()
+    name = "f32" if dtype == torch.float32 else "f64"
+    print("case:", widths, rows, name, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(11)
+    layers, total, row0 = len(widths) - 1, sum(rows), [sum(rows[:t]) for t in range(4)]
+    left = [torch.randn(total, w, device="cuda", dtype=dtype, generator=gen) for w in widths[:-1]]
+    right = [torch.randn(total, w, device="cuda", dtype=dtype, generator=gen) for w in widths[1:]]
+    a = _Grads(layers=layers, first=(1 << layers) - 1, second=0, scale_first=0, scale_second=0)
+    for i, w in enumerate(widths):
+        a.widths[i] = w
+    for t in range(4):
+        a.n[t], a.row0[t], a.x[t] = rows[t], row0[t], left[0][row0[t]:].data_ptr() if rows[t] else None
+    for l in range(layers):
+        a.left[l], a.right[l] = left[l].data_ptr(), right[l].data_ptr()
+    out = torch.full((4 * sum((k + 1) * n for k, n in zip(widths, widths[1:])),), 7.0, device="cuda", dtype=dtype)
+    work = torch.empty(getattr(lib, "khan_net_grads_workspace_bytes_" + name)(ctypes.byref(a)), dtype=torch.uint8, device="cuda")
+    a.out, a.workspace = out.data_ptr(), work.data_ptr()
+    for _ in range(2):                  # (twice: the same bits, whatever the workspace holds)
+        previous = out.clone()
+        assert getattr(lib, "khan_net_grads_" + name)(ctypes.byref(a), torch.cuda.current_stream().cuda_stream) == 0
+    assert torch.equal(out, previous)
+    at, bias_at = 0, 4 * sum(k * n for k, n in zip(widths, widths[1:]))
+    for l, (k, n) in enumerate(zip(widths, widths[1:])):
+        for t in range(4):
+            x, y = (v[l][row0[t]:row0[t] + rows[t]].double() for v in (left, right))
+            for got, want, size in ((out[at:at + k * n].view(k, n), x.t() @ y, x.abs().t() @ y.abs()), (out[bias_at:bias_at + n], y.sum(0), y.abs().sum(0))):
+                assert ((got.double() - want).abs() <= bound * size).all(), (l, t, ((got.double() - want).abs() / size).max().item())
+            at, bias_at = at + k * n, bias_at + n
+
+
 # Operands at both ends of float32's exponents: near the bottom the third part of a bfloat16 split would run out of them, near
 # the top the sums leave the split form.  Sums of 12,800 products in float32: the 2e-6 of sum |left| |right| of the test above.
 # (sum |left| |right| stays below 2^127: beyond, which sums overflow depends on the order they are formed in.)
