@@ -623,7 +623,7 @@ __device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __rest
 }
 
 // The same in float32 on the bfloat16 matrix instructions (the split of layer_split_kernel), for layers of at least 64 x 64.
-// A workgroup forms 128 of the left operand's columns x 128 (kWide) or 64 of the right's over `per_split` rows, 32 rows at a
+// A workgroup forms 128 of the left operand's columns x 128 (kWide) or 64 of the right's over `per` rows, 32 rows at a
 // time.  The rows are what is summed over, so that a matrix instruction's operand is eight rows of one column, which lie a row
 // apart in memory: a thread loads two neighbouring columns of eight rows (a wavefront 512 contiguous bytes of each row), splits
 // them and writes them to LDS as [part][eight rows][column] pieces of 16 bytes, column 2 c + j at place 64 j + c, so that
@@ -663,7 +663,7 @@ __device__ __forceinline__ void weight_grad_split_tile(const NetGrads<float>& a,
     const int tiles_n = (N + kCols - 1) / kCols, tiles = (K + kGradLeft - 1) / kGradLeft * tiles_n;
     const int share = rel / tiles, tile = rel - share * tiles;
     const int i0 = tile / tiles_n * kGradLeft, j0 = tile % tiles_n * kCols;
-    const int r0 = share * a.per_split, r1 = min(n, r0 + a.per_split);
+    const int r0 = share * a.per, r1 = min(n, r0 + a.per);
     const int chunks = (r1 - r0 + kGradChunk - 1) / kGradChunk;
     // this thread's columns (past the end: the last ones again, whose sums are never read)
     const int li = min(i0 + 2 * lane, K - 2), lj = min(j0 + kRC * lane, N - kRC);
@@ -859,7 +859,7 @@ __device__ __forceinline__ void weight_grad_split_tile(const NetGrads<float>& a,
 // kSplit: some of the layers are on split products.  A form of its own: with them in one kernel the others' workgroups, 152
 // registers and 33.8 KB of LDS, had 255 and 49.4 KB and were two on a compute unit instead of three (3,500 rows 17.7 -> 22.2 us).
 template <typename T, bool kSplit>
-__global__ __launch_bounds__(256, kSplit ? 2 : 1) void weight_grad_kernel(const NetGrads<T> a, T* __restrict__ partial)
+__global__ __launch_bounds__(256, kSplit || sizeof(T) == 8 ? 2 : 1) void weight_grad_kernel(const NetGrads<T> a, T* __restrict__ partial)
 {
     int job = 0;
     while (static_cast<int>(blockIdx.x) >= a.job_end[job]) ++job;                 // (layer, type)
@@ -909,7 +909,7 @@ __global__ __launch_bounds__(256) void grad_sum_kernel(const NetGrads<T> a, cons
     }
     const int t = block / (tiles * runs), tile = block / runs - t * tiles, at = (block % runs * 64 + lane) * V;
     const int K = a.k[layer], N = a.k[layer + 1], size = rows * cols + cols;
-    const int per = split ? a.per_split : a.per, shares = (a.n[t] + per - 1) / per;
+    const int shares = (a.n[t] + a.per - 1) / a.per;
     const T* p = partial + a.job_base[layer * 4 + t] + static_cast<size_t>(tile) * size + min(at, size - V);
     const size_t stride = static_cast<size_t>(tiles) * size;
     Vec<T> sum = Vec<T>(T(0)), lost = Vec<T>(T(0));
@@ -1077,36 +1077,43 @@ static int64_t plan_grads(NetGrads<T>& a, bool split)
         if (split && a.k[l] >= 64 && a.k[l + 1] >= 64) a.split |= 1u << l;
         ((a.split >> l) & 1u ? split_tiles : tiles) += tiles_of(l);
     }
-    // Few rows are faster on the float32 instructions, whose tiles are smaller (us with the summation, float32 -> split):
-    // 384-128-128-64-1, 5 tiles: 2,000 rows 21 -> 25, 6,000 33 -> 27, 12,132 48 -> 35, 35,000 93 -> 59, with both pairs of
-    // operands 185 -> 107; eleven layers, 33 tiles: 300 rows 39 -> 49, 2,000 64 -> 63, 12,132 250 -> 150, 47,000 845 -> 420.
-    if (a.split && rows * split_tiles < 20000) return plan_grads(a, false);
+    // Few rows are faster on the float32 instructions, whose tiles are smaller, as long as their workgroups, three to a compute
+    // unit, are all resident (us with the summation, float32 -> split): 384-128-128-64-1, 5 tiles: 2,000 rows 21 -> 23, 2,500 (798
+    // workgroups) 26 -> 24, 4,000 (in larger shares 630) 23 -> 25, 5,000 31 -> 25, 24,000 75 -> 44, with both pairs of
+    // operands 125 -> 66; 384-256-1, 6 tiles: 3,000 rows 23 -> 24, 3,500 31 -> 25, 6,000 33 -> 28; 384-64-1, 3 tiles: 4,000
+    // rows 17 -> 17, 8,000 24 -> 19; eleven layers, 33 tiles: 300 rows 33 -> 31, 2,000 59 -> 40, 48,000 780 -> 378.
+    if (a.split && rows * split_tiles < 24000) {
+        NetGrads<T> plain = a;
+        const int64_t bytes = plan_grads(plain, false);
+        if (plain.job_end[4 * a.layers - 1] <= 3 * kCUs) {
+            a = plain;
+            return bytes;
+        }
+    }
     auto blocks_of = [&](int64_t per, int64_t per_row) {
         int64_t shares = 0;
         for (int t = 0; t < 4; ++t) shares += (a.n[t] + per - 1) / per;
         return shares * per_row;
     };
-    // about two workgroups per compute unit and wave: short shares where rows are few, and never fewer than 64 rows; beside
-    // split products a sixth of that
+    // about two workgroups per compute unit and wave: short shares where rows are few, and never fewer than 64 rows
     int64_t per = 64;
-    while (per < 4096 && (split_tiles ? blocks_of(per, tiles) > 96 : rows / per * tiles > 1024)) per *= 2;
-    a.per = static_cast<int>(per);
-    // split products: all workgroups at once, two per compute unit, or as few such rounds as shares of up to 2,048 rows make
-    // (520 workgroups on 512 places took 56 us where 505 take 50)
-    const int64_t plain = split_tiles ? std::min<int64_t>(blocks_of(per, tiles), 128) : 0;
-    int64_t share = 4 * kGradChunk;
-    for (int64_t rounds = 1; split_tiles && blocks_of(share, split_tiles) > 512 * rounds - plain;) {
-        share += kGradChunk;
-        if (share > 64 * kGradChunk) share = 4 * kGradChunk, ++rounds;
+    while (per < 4096 && rows / per * tiles > 1024) per *= 2;
+    // beside split products as many rows as theirs, whose workgroups take as long: all workgroups at once, two per compute unit, or
+    // as few such rounds as shares of up to 2,048 rows make (520 workgroups on 512 places took 56 us where 505 take 50)
+    if (split_tiles) {
+        per = 4 * kGradChunk;
+        for (int64_t rounds = 1; blocks_of(per, split_tiles + tiles) > 512 * rounds;) {
+            per += kGradChunk;
+            if (per > 64 * kGradChunk) per = 4 * kGradChunk, ++rounds;
+        }
     }
-    a.per_split = static_cast<int>(share);
+    a.per = static_cast<int>(per);
     int64_t end = 0, base = 0;
     for (int l = 0; l < a.layers; ++l) {
         const bool is_split = (a.split >> l) & 1u;
         const int64_t size = is_split ? (kGradLeft + 1) * (a.k[l + 1] > 64 ? 128 : 64) : kSide * kSide + kSide;
-        const int64_t rows_each = is_split ? a.per_split : per;
         for (int t = 0; t < 4; ++t) {
-            const int64_t blocks = (a.n[t] + rows_each - 1) / rows_each * tiles_of(l);
+            const int64_t blocks = (a.n[t] + per - 1) / per * tiles_of(l);
             a.job_base[l * 4 + t] = base;
             base += blocks * size;
             a.job_end[l * 4 + t] = static_cast<int>(end += blocks);
@@ -1155,10 +1162,9 @@ hipError_t launch_net_grads(NetGrads<T> a, void* workspace, hipStream_t stream)
     // A workgroup's four wavefronts to each run where there are few runs for the shares (us of gradients and sums, a wavefront to
     // each run -> four): 384-128-128-64-1 (1,300 times 64 runs), 8 shares 15.4 -> 16.7, 17 shares 20.3 -> 20.4, 85 shares
     // 69.7 -> 67.9; 384-64-1 (480), 10 shares 13.2 -> 12.8; eleven layers (9,600 to 11,600), 3 to 13 shares 31 -> 50, 61 -> 80, 372 -> 387.
-    const int per = a.split ? a.per_split : a.per;
     int most = 0;
     for (int t = 0; t < 4; ++t) most = std::max(most, a.n[t]);
-    if ((static_cast<int64_t>(most) + per - 1) / per * 50 > sums)
+    if ((static_cast<int64_t>(most) + a.per - 1) / a.per * 50 > sums)
         grad_sum_kernel<T, true><<<dim3(static_cast<unsigned>(sums)), dim3(256), 0, stream>>>(a, static_cast<const T*>(workspace));
     else
         grad_sum_kernel<T, false><<<dim3(static_cast<unsigned>((sums + 3) / 4)), dim3(256), 0, stream>>>(a, static_cast<const T*>(workspace));
