@@ -52,7 +52,7 @@ struct __align__(16) MedShared<T, kJvp, true> {
 // batch (a form of its own: the grid's sizes in scalar registers cost the plain kernel 6 %).
 // With kLarge the kernel takes the molecules of more than 256 atoms: the atoms come type-sorted from `sorted`.
 // kOnce: the rows are marked as written once (store_global)
-template <typename T, bool kJvp, bool kLarge = false, bool kShare = kLarge, bool kOnce = !kJvp && !kShare>
+template <typename T, bool kJvp, bool kLarge = false, bool kShare = kLarge, bool kOnce = false>
 __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
     const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
     const int32_t* __restrict__ A, const int32_t* __restrict__ MOs,
@@ -481,7 +481,7 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
 template <typename T>
 hipError_t launch_fwd_medium(const T* X, const T* Y, const T* Z, const int32_t* A,
                              const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
-                             const int32_t* SIs, Buckets<T> out, int min_atoms, const int32_t* order, hipStream_t stream)
+                             const int32_t* SIs, Buckets<T> out, int min_atoms, const int32_t* order, int64_t n_atoms, hipStream_t stream)
 {
     if (n_mols <= 0) return hipSuccess;
     // workgroups walk the molecules with the grid's stride and skip those of other sizes
@@ -496,6 +496,7 @@ hipError_t launch_fwd_medium(const T* X, const T* Y, const T* Z, const int32_t* 
                                                                                      out, min_atoms, order, SortedAtoms<T>{});
     };
     if (parts > 1) launch(aev_fwd_medium_kernel<T, false, false, true>);
+    else if (rows_beyond_caches<T>(n_atoms)) launch(aev_fwd_medium_kernel<T, false, false, false, true>);
     else launch(aev_fwd_medium_kernel<T, false>);
     return hipGetLastError();
 }
@@ -546,9 +547,11 @@ hipError_t launch_fwd_large(const T* X, const T* Y, const T* Z, const int32_t* A
         aev_fwd_medium_kernel<T, true, true><<<grid, dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, VX, VY, VZ, out,
                                                                          kMediumMaxAtoms + 1, order, sorted);
     else {
-        // rows beyond the second-level caches (32 MB) by a factor of two
-        const bool once = n_atoms * static_cast<int64_t>(kFeats * sizeof(T)) >= (64 << 20);
-        const auto kernel = once ? aev_fwd_medium_kernel<T, false, true, true, true> : aev_fwd_medium_kernel<T, false, true>;
+        // The rows are marked as written once from 64 MB on already: the backward pass, which reads its atoms and skeleton again
+        // many times, gains more than a reader of the rows loses (forward, reader and backward as at rows_beyond_caches: 24 boxes of
+        // 1,024-4,096 atoms, 94 MB, 472 -> 468 us, 32 635 -> 621, 48 1,116 -> 1,113, 64 the same; 16 in float64 739 -> 722; below
+        // 64 MB the same).
+        const auto kernel = rows_beyond_caches<T>(n_atoms, 64 << 20) ? aev_fwd_medium_kernel<T, false, true, true, true> : aev_fwd_medium_kernel<T, false, true>;
         kernel<<<grid, dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, out, kMediumMaxAtoms + 1, order, sorted);
     }
     return hipGetLastError();
@@ -557,8 +560,8 @@ hipError_t launch_fwd_large(const T* X, const T* Y, const T* Z, const int32_t* A
 #ifndef KHAN_UNIT_LARGE
 template hipError_t launch_jvp_medium<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const float*, const float*, const float*, Buckets<float>, int, const int32_t*, hipStream_t);
 #else
-template hipError_t launch_fwd_medium<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<float>, int, const int32_t*, hipStream_t);
-template hipError_t launch_fwd_medium<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<double>, int, const int32_t*, hipStream_t);
+template hipError_t launch_fwd_medium<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<float>, int, const int32_t*, int64_t, hipStream_t);
+template hipError_t launch_fwd_medium<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<double>, int, const int32_t*, int64_t, hipStream_t);
 template hipError_t launch_jvp_medium<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const double*, const double*, const double*, Buckets<double>, int, const int32_t*, hipStream_t);
 template size_t large_scratch_bytes<float>(int64_t, int32_t, bool);
 template size_t large_scratch_bytes<double>(int64_t, int32_t, bool);

@@ -43,15 +43,16 @@ constexpr int kRadSlots = 96;
 
 // With kJvp the kernel computes the Jacobian-vector product instead (featurize_grad_inverse): every term of
 // the forward sums is replaced by its derivative along the per-atom vectors (VX, VY, VZ).
-// float: 4 wavefronts per SIMD (LDS 9.8 KB, <= 128 VGPRs; the kernel loses a fifth of its speed at three), and 5 with a wavefront
-// per molecule (6.9 KB, 96 VGPRs, without hoisting: khan_amd/build.py; 65,536 organic molecules 497 -> 468 us);
+// float: 4 wavefronts per SIMD (LDS 9.8 KB, <= 128 VGPRs; the kernel loses a fifth of its speed at three), and 5 with kFive
+// (6.9 KB, 96 VGPRs, without hoisting: khan_amd/build.py; 65,536 organic molecules 497 -> 468 us);
 // float kJvp: 3 (<= 168 VGPRs; its LDS lets twelve wavefronts share a CU); double: 3 (149 VGPRs, LDS 12.5 KB with four
 // centres); double kJvp: 1.
-constexpr int fwd_small_waves(size_t element, bool jvp, bool share) { return element == 4 ? (jvp ? 3 : share ? 4 : 5) : (jvp ? 1 : 3); }
+constexpr int fwd_small_waves(size_t element, bool jvp, bool five) { return element == 4 ? (jvp ? 3 : five ? 5 : 4) : (jvp ? 1 : 3); }
 
-template <typename T, bool kJvp, bool kShare = false, bool kMatrixPhase2 = false>
+// kOnce: the rows are marked as written once (store_global)
+template <typename T, bool kJvp, bool kShare = false, bool kMatrixPhase2 = false, bool kOnce = false, bool kFive = false>
 __global__ __launch_bounds__(64 * kWavesPerBlock)
-__attribute__((amdgpu_waves_per_eu(fwd_small_waves(sizeof(T), kJvp, kShare), fwd_small_waves(sizeof(T), kJvp, kShare))))
+__attribute__((amdgpu_waves_per_eu(fwd_small_waves(sizeof(T), kJvp, kFive), fwd_small_waves(sizeof(T), kJvp, kFive))))
 void aev_fwd_small_kernel(
     const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
     const int32_t* __restrict__ A, const int32_t* __restrict__ MOs,
@@ -61,10 +62,9 @@ void aev_fwd_small_kernel(
 {
     typedef typename Fast<T>::vec4 vec4;
     typedef typename Fast<T>::vec2 vec2;
-    constexpr bool kOnce = !kJvp && !kShare;      // a wavefront per molecule: 16,384 molecules (12,288 in double) and more
-    // centres per batch: six; four in the float Jacobian-vector kernel (with kCap below: twelve wavefronts per CU) and in
-    // float with a wavefront per molecule (6.9 KB: six of the 1,280 bytes LDS is given out in, twenty wavefronts per CU)
-    constexpr int kNB = (kJvp == (sizeof(T) == 4) || (sizeof(T) == 4 && !kShare)) ? 4 : kFB;
+    // centres per batch: six; four in the float Jacobian-vector kernel (with kCap below: twelve wavefronts per CU), in double
+    // and with kFive (6.9 KB: six of the 1,280 bytes LDS is given out in, twenty wavefronts per CU)
+    constexpr int kNB = (kJvp == (sizeof(T) == 4) || kFive) ? 4 : kFB;
     // angular partners kept per centre: 32; 28 in the float Jacobian-vector kernel, whose working set then is 13.4 KB
     // and twelve wavefronts share a CU (a centre with more goes to the general routine, as above 32 elsewhere)
     constexpr int kCap = (kJvp && sizeof(T) == 4) ? 28 : kCapA;
@@ -339,7 +339,8 @@ void aev_fwd_small_kernel(
 // Wavefronts per molecule (as a power of two).  organic molecules, 16 / 12 / 12 / 4 wavefronts per CU resident (float,
 // double, and their Jacobian-vector forms); forward float 100 -> 24 us at 1,024 molecules, 106 -> 47 at 4,096,
 // 112 -> 78 at 8,192 (two each), and slower from 16,384 on (137 -> 150 with two); the Jacobian-vector form
-// 131 -> 31 us at 1,024, double forward 162 -> 51 us.  The rows are the same bits for any number.
+// 131 -> 31 us at 1,024, double forward 162 -> 51 us, 172 -> 98 at 4,097 and 177 -> 123 at 6,100 (two each).  The rows are
+// the same bits for any number.
 template <typename T, bool kJvp>
 static int log_parts_of(int32_t n_mols)
 {
@@ -347,28 +348,38 @@ static int log_parts_of(int32_t n_mols)
     return __builtin_ctz(molecule_parts(n_mols, 4 * kResident, 8));
 }
 
-// A wavefront per molecule (in float32 a translation unit of its own: aev_small_whole.hip)
-template <typename T>
-hipError_t launch_fwd_small_whole(const T* X, const T* Y, const T* Z, const int32_t* A, const int32_t* MOs,
-                                  const int32_t* MACs, int32_t n_mols, const int32_t* SIs, Buckets<T> out,
-                                  int max_atoms, const int32_t* order, hipStream_t stream);
-#if defined(KHAN_UNIT_F64) || defined(KHAN_UNIT_WHOLE)
-template <typename T>
-hipError_t launch_fwd_small_whole(const T* X, const T* Y, const T* Z, const int32_t* A, const int32_t* MOs,
-                                  const int32_t* MACs, int32_t n_mols, const int32_t* SIs, Buckets<T> out,
-                                  int max_atoms, const int32_t* order, hipStream_t stream)
+// A wavefront per molecule
+template <typename T, bool kFive>
+static hipError_t launch_whole(const T* X, const T* Y, const T* Z, const int32_t* A, const int32_t* MOs,
+                               const int32_t* MACs, int32_t n_mols, const int32_t* SIs, Buckets<T> out,
+                               int max_atoms, const int32_t* order, int64_t n_atoms, hipStream_t stream)
 {
     const unsigned blocks = (static_cast<unsigned>(n_mols) + kWavesPerBlock - 1u) / kWavesPerBlock;
-    aev_fwd_small_kernel<T, false><<<dim3(blocks), dim3(64 * kWavesPerBlock), 0, stream>>>(
+    const auto kernel = rows_beyond_caches<T>(n_atoms) ? aev_fwd_small_kernel<T, false, false, false, true, kFive>
+                                                       : aev_fwd_small_kernel<T, false, false, false, false, kFive>;
+    kernel<<<dim3(blocks), dim3(64 * kWavesPerBlock), 0, stream>>>(
         X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, out, max_atoms < 64 ? max_atoms : 64, order, 0);
     return hipGetLastError();
+}
+// (a translation unit of its own: aev_small_whole.hip)
+template <typename T>
+hipError_t launch_fwd_small_five(const T* X, const T* Y, const T* Z, const int32_t* A, const int32_t* MOs,
+                                 const int32_t* MACs, int32_t n_mols, const int32_t* SIs, Buckets<T> out,
+                                 int max_atoms, const int32_t* order, int64_t n_atoms, hipStream_t stream);
+#ifdef KHAN_UNIT_WHOLE
+template <typename T>
+hipError_t launch_fwd_small_five(const T* X, const T* Y, const T* Z, const int32_t* A, const int32_t* MOs,
+                                 const int32_t* MACs, int32_t n_mols, const int32_t* SIs, Buckets<T> out,
+                                 int max_atoms, const int32_t* order, int64_t n_atoms, hipStream_t stream)
+{
+    return launch_whole<T, true>(X, Y, Z, A, MOs, MACs, n_mols, SIs, out, max_atoms, order, n_atoms, stream);
 }
 #endif
 
 template <typename T>
 hipError_t launch_fwd_small(const T* X, const T* Y, const T* Z, const int32_t* A, const int32_t* MOs,
                             const int32_t* MACs, int32_t n_mols, const int32_t* SIs, Buckets<T> out,
-                            int max_atoms, const int32_t* order, hipStream_t stream)
+                            int max_atoms, const int32_t* order, int64_t n_atoms, hipStream_t stream)
 {
     if (n_mols <= 0) return hipSuccess;
     const unsigned blocks = (static_cast<unsigned>(n_mols) + kWavesPerBlock - 1u) / kWavesPerBlock;
@@ -388,7 +399,11 @@ hipError_t launch_fwd_small(const T* X, const T* Y, const T* Z, const int32_t* A
         }
     }
 #endif
-    if (log_parts == 0) return launch_fwd_small_whole<T>(X, Y, Z, A, MOs, MACs, n_mols, SIs, out, max_atoms, order, stream);
+    if (log_parts == 0) {
+        if constexpr (sizeof(T) == 4)
+            return launch_fwd_small_five<T>(X, Y, Z, A, MOs, MACs, n_mols, SIs, out, max_atoms, order, n_atoms, stream);
+        return launch_whole<T, false>(X, Y, Z, A, MOs, MACs, n_mols, SIs, out, max_atoms, order, n_atoms, stream);
+    }
     aev_fwd_small_kernel<T, false, true><<<dim3(blocks << log_parts), dim3(64 * kWavesPerBlock), 0, stream>>>(
         X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, out, max_atoms < 64 ? max_atoms : 64, order, log_parts);
     return hipGetLastError();
@@ -409,12 +424,12 @@ hipError_t launch_jvp_small(const T* X, const T* Y, const T* Z, const int32_t* A
 }
 
 #if defined(KHAN_UNIT_WHOLE)
-template hipError_t launch_fwd_small_whole<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<float>, int, const int32_t*, hipStream_t);
+template hipError_t launch_fwd_small_five<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<float>, int, const int32_t*, int64_t, hipStream_t);
 #elif !defined(KHAN_UNIT_F64)
-template hipError_t launch_fwd_small<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<float>, int, const int32_t*, hipStream_t);
+template hipError_t launch_fwd_small<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<float>, int, const int32_t*, int64_t, hipStream_t);
 template hipError_t launch_jvp_small<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const float*, const float*, const float*, Buckets<float>, const int32_t*, hipStream_t);
 #else
-template hipError_t launch_fwd_small<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<double>, int, const int32_t*, hipStream_t);
+template hipError_t launch_fwd_small<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<double>, int, const int32_t*, int64_t, hipStream_t);
 template hipError_t launch_jvp_small<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const double*, const double*, const double*, Buckets<double>, const int32_t*, hipStream_t);
 #endif
 

@@ -55,10 +55,7 @@ __device__ __forceinline__ double lane_push(int dest_lane, double v)
 // Row pointers are rebuilt from two 32-bit lane reads; storing through an explicit global-address-space
 // pointer keeps the stores on the global (not the flat) path.
 // kOnce: rows that together are more than the caches keep until somebody reads them; marked as written once, they leave
-// the caches to what is read meanwhile and afterwards.  Forward pass (and the backward pass behind it, whose upstream rows
-// then stay in the last cache): 65,536 organic molecules 515 (619) -> 500 (615) us, 64 boxes of 1,000 atoms
-// 437 (669) -> 435 (635); 16,384 in double the same.  Rows that do fit are better left there: with 1,024 molecules the forward
-// pass gains 1 us and the layer that reads its rows loses 2.
+// the caches to what is read meanwhile and afterwards (rows_beyond_caches).
 template <bool kOnce = false, typename T>
 __device__ __forceinline__ void store_global(T* p, T v)
 {
@@ -67,6 +64,14 @@ __device__ __forceinline__ void store_global(T* p, T v)
     else if constexpr (kOnce) __builtin_nontemporal_store(v, (global_t*)(p));
     else *((global_t*)(p)) = v;
 }
+// Whether a batch's feature rows are to be marked so: from 256 MB on, the size of the last cache.  Forward pass, a pass over its
+// rows and the backward pass one after the other, us without -> with the mark, organic molecules in float32: 12,000 (206 MB)
+// 284 -> 293, 14,000 (241 MB) 319 -> 327, 16,384 (282 MB) 362 -> 362, 18,000 (310 MB) 390 -> 387, 65,536 1,369 -> 1,310; in
+// float64: 6,145 (211 MB) 384 -> 387, 8,000 (275 MB) 431 -> 431, 12,000 588 -> 573, 16,384 804 -> 764; boxes of 64-256 atoms in
+// float64: 513 (241 MB) 915 -> 915, 700 (331 MB) 977 -> 968.  (What counts are all atoms of the batch.)
+constexpr int64_t kOnceBytes = int64_t{256} << 20;
+template <typename T>
+inline bool rows_beyond_caches(int64_t n_atoms, int64_t bytes = kOnceBytes) { return n_atoms * static_cast<int64_t>(kFeats * sizeof(T)) >= bytes; }
 // acc + a' * g, where a' is the value of `a` held by lane k of this lane's quad (k is a constant after unrolling).
 // The lane exchange is a modifier of the multiply-add, not an instruction of its own.  It reads `a` early: two
 // wait states have to lie between a vector instruction that writes `a` and this one, and the compiler does not

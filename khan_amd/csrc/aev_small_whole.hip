@@ -1,4 +1,4 @@
-// The instance of aev_small.hip for float32 with a wavefront per molecule,
+// The instances of aev_small.hip for float32 with five wavefronts per SIMD,
 // a translation unit of its own because it is compiled without the hoisting of constants out of loops (khan_amd/build.py,
 // SOURCE_FLAGS).
 #define KHAN_UNIT_WHOLE

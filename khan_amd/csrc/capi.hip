@@ -198,9 +198,9 @@ int forward_dispatch(const T* xs, const T* ys, const T* zs, const int32_t* as, c
     const SizeClasses cls(classes_host);
     int st = KHAN_OK;
     if (cls.any(0, small_max))
-        st = hip_status(khan::launch_fwd_small<T>(xs, ys, zs, as, mos, macs, n_mols, sis, out, small_max, order, stream));
+        st = hip_status(khan::launch_fwd_small<T>(xs, ys, zs, as, mos, macs, n_mols, sis, out, small_max, order, n_atoms, stream));
     if (st == KHAN_OK && cls.any(small_max + 1, khan::kMediumMaxAtoms))
-        st = hip_status(khan::launch_fwd_medium<T>(xs, ys, zs, as, mos, macs, n_mols, sis, out, small_max + 1, order, stream));
+        st = hip_status(khan::launch_fwd_medium<T>(xs, ys, zs, as, mos, macs, n_mols, sis, out, small_max + 1, order, n_atoms, stream));
     if (st == KHAN_OK && n_atoms > khan::kMediumMaxAtoms && cls.any(khan::kMediumMaxAtoms + 1, INT32_MAX)) {      // (n_atoms: of the whole batch)
         const LargeScratch scratch(may_allocate && n_atoms < kLargeAtomLimit ? khan::large_scratch_bytes<T>(n_atoms, n_mols, false) : 0, stream);
         if (scratch.get())

@@ -46,7 +46,7 @@ constexpr int kSmallPreferredMax = 32;
 template <typename T>
 hipError_t launch_fwd_small(const T* X, const T* Y, const T* Z, const int32_t* A, const int32_t* MOs,
                             const int32_t* MACs, int32_t n_mols, const int32_t* SIs, Buckets<T> out,
-                            int max_atoms, const int32_t* order, hipStream_t stream);
+                            int max_atoms, const int32_t* order, int64_t n_atoms, hipStream_t stream);
 
 template <typename T>
 hipError_t launch_jvp_small(const T* X, const T* Y, const T* Z, const int32_t* A, const int32_t* MOs,
@@ -58,7 +58,7 @@ constexpr int kMediumMaxAtoms = 256;
 template <typename T>
 hipError_t launch_fwd_medium(const T* X, const T* Y, const T* Z, const int32_t* A,
                              const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
-                             const int32_t* SIs, Buckets<T> out, int min_atoms, const int32_t* order, hipStream_t stream);
+                             const int32_t* SIs, Buckets<T> out, int min_atoms, const int32_t* order, int64_t n_atoms, hipStream_t stream);
 // the same kernel as Jacobian-vector product
 template <typename T>
 hipError_t launch_jvp_medium(const T* X, const T* Y, const T* Z, const int32_t* A,

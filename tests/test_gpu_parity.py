@@ -919,11 +919,20 @@ def test_random_large_molecules(ops, seed):
         check_forward_backward(ops, Case(xyz[:, 0], xyz[:, 1], xyz[:, 2], A, mi, len(mols)))
 
 
+# Both sides of each line between the forward kernels: 174,763 atoms in float32 (87,382 in float64) make 256 MB of rows, 43,691
+# (21,846) the 64 MB of molecules of more than 256 atoms; up to 8,192 molecules of 32 atoms in float32 (6,144 of 64 in float64)
+# and 2,048 (512) larger ones are shared, and from 16,385 on there are five wavefronts to a SIMD.
 @pytest.mark.parametrize("dtype,atoms,copies", [(torch.float32, 3, 16384), (torch.float64, 5, 16384), (torch.float32, 70, 4096),
-                                                (torch.float64, 66, 1024), (torch.float32, 700, 63), (torch.float64, 300, 74)])
+                                                (torch.float64, 66, 1024), (torch.float32, 700, 63), (torch.float64, 300, 74),
+                                                (torch.float32, 22, 8192), (torch.float32, 3, 8193), (torch.float32, 22, 8193),
+                                                (torch.float32, 11, 15887), (torch.float32, 11, 15888), (torch.float32, 3, 16385),
+                                                (torch.float32, 11, 16385), (torch.float64, 15, 6144), (torch.float64, 14, 6145),
+                                                (torch.float64, 15, 6145), (torch.float32, 86, 2048), (torch.float32, 85, 2049),
+                                                (torch.float32, 86, 2049), (torch.float64, 171, 512), (torch.float64, 170, 513),
+                                                (torch.float64, 171, 513), (torch.float32, 700, 62), (torch.float64, 300, 72)])
 def test_rows_beyond_the_caches(ops, dtype, atoms, copies):
-    # Feature rows that together exceed the caches are stored as written once: many copies of one molecule (the sizes at which
-    # each forward kernel changes over) have the very rows that the molecule has in a batch of three.
+    # Feature rows that together exceed the caches are stored as written once: many copies of one molecule have the very rows
+    # that the molecule has in a batch of three.
     say("case: %d copies of a molecule of %d atoms, %s" % (copies, atoms, dtype))
     rng = np.random.default_rng(atoms)
     xyz = _sparse_box(rng, atoms, 0.08, 0.9).astype(np.float32).astype(np.float64)
