@@ -376,6 +376,10 @@ hipError_t launch_fwd_small_five(const T* X, const T* Y, const T* Z, const int32
 }
 #endif
 
+// Molecules from which a fifth wavefront per SIMD pays: four rounds of those that four per SIMD hold.  Below, the fewer centres
+// per batch cost more (forward, four -> five wavefronts, rows not marked: 8,193 molecules 108 -> 114 us, 12,000 110 -> 117,
+// 16,384 125 -> 125, 18,000 137 -> 129, 32,768 243 -> 229).
+constexpr int32_t kFivePays = 16384;
 template <typename T>
 hipError_t launch_fwd_small(const T* X, const T* Y, const T* Z, const int32_t* A, const int32_t* MOs,
                             const int32_t* MACs, int32_t n_mols, const int32_t* SIs, Buckets<T> out,
@@ -401,7 +405,7 @@ hipError_t launch_fwd_small(const T* X, const T* Y, const T* Z, const int32_t* A
 #endif
     if (log_parts == 0) {
         if constexpr (sizeof(T) == 4)
-            return launch_fwd_small_five<T>(X, Y, Z, A, MOs, MACs, n_mols, SIs, out, max_atoms, order, n_atoms, stream);
+            if (n_mols > kFivePays) return launch_fwd_small_five<T>(X, Y, Z, A, MOs, MACs, n_mols, SIs, out, max_atoms, order, n_atoms, stream);
         return launch_whole<T, false>(X, Y, Z, A, MOs, MACs, n_mols, SIs, out, max_atoms, order, n_atoms, stream);
     }
     aev_fwd_small_kernel<T, false, true><<<dim3(blocks << log_parts), dim3(64 * kWavesPerBlock), 0, stream>>>(
