@@ -431,6 +431,8 @@ int khan_net_grads_f64(const khan_net_grads *grads, khan_stream_t stream);
  * khan_net_few_fits: 1 for widths it takes, which are 384, 128, 128, 64, 1.  x and w must be 16-byte aligned; grad[t] NULL
  * for all types: values only. */
 #define KHAN_NET_FEW_LAYERS 4
+#define KHAN_NET_FEW_ROWS 16        /* rows of a type that a workgroup takes */
+#define KHAN_NET_FEW_TILES 256      /* such tiles up to which it is the faster form: one for every compute unit */
 typedef struct khan_net_few {
     const void *x[4], *w[KHAN_NET_FEW_LAYERS][4], *b[KHAN_NET_FEW_LAYERS][4];
     void *value[4], *grad[4];

@@ -971,7 +971,7 @@ int32_t khan_net_few_fits(const int32_t* widths, int32_t layers)
 }
 int khan_net_few_f64(const khan_net_few* net, khan_stream_t stream)
 {
-    static_assert(KHAN_NET_FEW_LAYERS == khan::kFewLayers, "one limit");
+    static_assert(KHAN_NET_FEW_LAYERS == khan::kFewLayers && KHAN_NET_FEW_ROWS == khan::kFewRows && KHAN_NET_FEW_TILES == khan::kCUs, "one limit");
     if (!net || !khan_net_few_fits(net->widths, net->layers) || !(net->alpha > 0.0)) return KHAN_ERR_INVALID_ARG;
     khan::NetFew a = {};
     a.alpha = net->alpha;

@@ -774,8 +774,10 @@ struct Inference {
     }
     bool one_launch() const { return w.packed.defined(); }
 
-    // Float64 networks of the widths net_few.hip takes, whose rows' gradients are not to be scaled: one launch up to 256 tiles
-    // of sixteen rows, one for every compute unit (us, values and gradients, layer by layer -> one launch: 1 molecule 80 -> 67, 16 molecules 112 -> 86, 256 (2,970 rows) 152 -> 115, 330 (3,863) 175 -> 132; values alone 41 -> 29, 54 -> 39, 67 -> 47).
+    // Float64 networks of the widths net_few.hip takes, whose rows' gradients are not to be scaled: one launch up to
+    // KHAN_NET_FEW_TILES tiles of KHAN_NET_FEW_ROWS rows of a type, one for every compute unit (us, values and gradients, layer by
+    // layer -> one launch: 1 molecule 80 -> 67, 16 molecules 112 -> 86, 256 (2,970 rows) 152 -> 115, 330 (3,863) 175 -> 132; values
+    // alone 41 -> 29, 54 -> 39, 67 -> 47).
     void take_few()
     {
         if (w.params.dtype != at::kDouble || w.net.layers() > KHAN_NET_FEW_LAYERS) return;
@@ -785,11 +787,11 @@ struct Inference {
         int64_t tiles = 0;
         uintptr_t bits = 0;
         for (int t = 0; t < 4; ++t) {
-            tiles += (rows.n[t] + 15) / 16;
+            tiles += (rows.n[t] + KHAN_NET_FEW_ROWS - 1) / KHAN_NET_FEW_ROWS;
             if (rows.n[t] > 0) bits |= reinterpret_cast<uintptr_t>(rows.x[t].data_ptr());
             for (int l = 0; l < w.net.layers(); ++l) bits |= reinterpret_cast<uintptr_t>(w.params.weight(l, t));
         }
-        few = tiles <= 256 && (bits & 15u) == 0;
+        few = tiles <= KHAN_NET_FEW_TILES && (bits & 15u) == 0;
     }
     Tensor launch_few(bool want_rows)
     {
@@ -847,10 +849,14 @@ struct Inference {
         return v;
     }
     // the rows' gradients times scale (undefined: ones), added to `into` where defined -> [all rows, features]; the one-launch
-    // form has them already, and neither scale nor anything to add to
+    // forms have them already, and take neither scale nor anything to add to
     Tensor gradients(const Four& scale, Tensor into)
     {
-        if (one_launch() || few) return state[0];
+        if (one_launch() || few) {
+            for (const Tensor& s : scale) same_size(!s.defined(), "networks in one launch have no scaled gradients");
+            same_size(!into.defined(), "networks in one launch add their gradients to nothing");
+            return state[0];
+        }
         const bool add = into.defined();
         if (!add) into = at::empty({rows.total * w.net.widths[0]}, w.params.options);
         const variable_list d = pass.slopes(variable_list(state.begin(), state.end() - 1), state.back());

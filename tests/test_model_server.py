@@ -259,6 +259,34 @@ def test_charge_model_energy_and_gradient_match_the_oracle():
         assert abs(want_g[atom, axis] - fd) <= 1e-6 * max(1.0, abs(fd)), (atom, axis)
 
 
+# The default float64 networks in one launch and, from 257 tiles of sixteen rows of a type on, layer by layer; beside a charge
+# network, which goes layer by layer on top of the near network's row gradients, or goes the same way for energies alone.
+@pytest.mark.gpu
+@pytest.mark.parametrize("fit_charges", [False, True])
+@pytest.mark.parametrize("tiles", [None, 256, 257])
+def test_float64_inference_in_one_launch_and_layer_by_layer(fit_charges, tiles):
+    print("case:", fit_charges, tiles, flush=True)
+    b, mols = _molecules(n_mols=7 if tiles is None else 330, first=11)
+    if tiles is not None:                       # lone hydrogen atoms fill up the tiles
+        rows = np.bincount(b.A, minlength=4)
+        count = lambda: int(sum((n + 15) // 16 for n in rows))
+        assert count() < tiles
+        while count() < tiles or (tiles == 256 and rows[0] % 16):
+            mols.append(np.zeros((1, 4)))
+            rows[0] += 1
+        assert count() == tiles
+    m = model.AniModel(model.DEFAULT_LAYERS, model.celu, torch.float64, "cuda:0", fit_charges=fit_charges, seed=8)
+    atoms, sizes = np.concatenate(mols), np.array([len(x) for x in mols], dtype=np.int32)
+    mos = (np.cumsum(sizes) - sizes).astype(np.int32)
+    want_e, want_g = nn_ref.energies_and_gradients(atoms[:, 1], atoms[:, 2], atoms[:, 3], atoms[:, 0].astype(np.int32), mos, sizes, _np_params(m),
+                                                   model.DEFAULT_LAYERS, fit_charges=fit_charges)
+    ds = RawDataset(mols, [0.0] * len(mols))
+    got_e = np.array(m.predict(ds, batch_size=len(mols)))
+    assert np.max(np.abs(got_e - want_e)) <= 1e-10 * np.max(np.abs(want_e))
+    got_g = np.concatenate(list(m.coordinate_gradients(ds, batch_size=len(mols))), axis=0)
+    assert np.max(np.abs(got_g - want_g)) <= 1e-10 * max(1.0, np.max(np.abs(want_g)))
+
+
 @pytest.mark.gpu
 def test_gradient_is_the_derivative_of_the_energy():
     _, mols = _molecules(n_mols=1, first=40)
