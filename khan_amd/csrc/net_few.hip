@@ -2,15 +2,15 @@
 // khan/inference/energy_server.py:121), in float64 on few rows: values and row gradients in one launch.  Layer by layer
 // (net_layers.hip, whose names these are) a request for one molecule's energy and gradient is seven launches of 4 to 12 us, each of
 // which waits for a chain of loads and leaves the GPU empty: here a workgroup of sixteen wavefronts takes sixteen rows of one
-// type through the whole network and back, with every activation in LDS.
+// type through the whole network and back, its activations in LDS (the last layer's in registers).
 //
 // A product of the sixteen rows with 128 (or 64) columns: a wavefront has 32 columns and a quarter (an eighth) of the summed
 // index, on v_mfma_f64_16x16x4_f64 with operands as in layer_kernel: the rows' from LDS, the weights' 16 bytes at a time from
 // memory, four steps (eight loads) ahead, those of a product's first four steps before the sums of the product before it are
 // added up.  The shares' sums meet in LDS and are added up in order.  The widths are constants of the code: with widths read at
-// run time the index arithmetic between the products took as long as they did (54 us with gradients, 27 now, 28 of kernels and as many of gaps in seven launches before).
-// With gradients three workgroups form the same values and a third of the 384 gradient columns each, while that many find a
-// compute unit of their own (kFewSplit).
+// run time the index arithmetic between the products took as long as they did (with gradients 54 us, 27 now; seven launches
+// were 28 us of kernels and as many of gaps).  With gradients three workgroups form the same values and a third of the 384
+// gradient columns each, while that many find a compute unit of their own (launch_net_few).
 #include "khan_internal.h"
 #include "net_few.h"
 
@@ -28,7 +28,7 @@ constexpr int kIn = 384, kN1 = 128, kN2 = 128, kN3 = 64;
 struct __align__(16) FewLds {
     double x[kFewRows][kIn + kPad];           // the rows; then the gradients, layer by layer
     double part[8 * kFewRows * (64 + kPad)];  // [share][row][column] of a product (four shares of 128 columns need no more)
-    double a1[kFewRows][kN1 + kPad], a2[kFewRows][kN2 + kPad], a3[kFewRows][kN3 + kPad];
+    double a1[kFewRows][kN1 + kPad], a2[kFewRows][kN2 + kPad];
 };
 static_assert(4 * (128 + kPad) <= 8 * (64 + kPad), "the sums of four shares of 128 columns");
 static_assert(sizeof(FewLds) <= 160 * 1024, "one workgroup per compute unit");
