@@ -442,6 +442,11 @@ __global__ __launch_bounds__(256, 4) void charge_kernel(ChargeArgs<T> a, int col
 // 256 atoms are added up), and by the first workgroup the molecules of 65 to 256 atoms by
 // decreasing size, the others behind them: a counting sort, in no particular order inside a size (every molecule's results
 // are its own).  A launch lasts only a few molecules' time and in batch order ended with a third of the wavefronts' places empty.
+// From two workgroups a compute unit on in float32 and from one on in float64, though four find a place: those that share a unit
+// share its arithmetic, and in decreasing size the units' shares come out alike.  Boxes of 64 to 256 atoms, fill and pass in
+// batch order -> sorting launch and pass, us: float32 257 molecules 24.9 -> 27.4, 400 31.7 -> 34.1, 600 36.4 -> 34.7, 1,000
+// 46 -> 37, 4,096 103 -> 88; float64 257 35.5 -> 35.3, 400 45.7 -> 43.4, 600 56 -> 45, 1,000 67 -> 54, 4,096 170 -> 148.
+template <typename T> constexpr int kOrderFrom = (sizeof(T) == 4 ? 2 : 1) * kCUs;
 constexpr int kOrderMost = 16384;
 template <typename T>
 __global__ __launch_bounds__(1024) void charge_begin_kernel(const int32_t* __restrict__ MACs, int n_mols, int32_t* __restrict__ order,
@@ -527,7 +532,7 @@ hipError_t launch_charge_grad(const T* X, const T* Y, const T* Z, const T* Q, co
 template <typename T>
 hipError_t launch_charge_begin(const int32_t* MACs, int32_t n_mols, int64_t n_atoms, int32_t*& order, T* outputs, int64_t n_outputs, hipStream_t stream)
 {
-    if (n_mols <= 256 || n_mols > kOrderMost || charge_mols_per_workgroup(n_mols, n_atoms) != 1) order = nullptr;
+    if (n_mols <= kOrderFrom<T> || n_mols > kOrderMost || charge_mols_per_workgroup(n_mols, n_atoms) != 1) order = nullptr;
     if (!order) return n_outputs > 0 ? launch_zero<T>(outputs, n_outputs, stream) : hipSuccess;
     const int64_t zeroing = std::min<int64_t>((n_outputs + 8191) / 8192, 512);
     charge_begin_kernel<T><<<dim3(static_cast<unsigned>(zeroing + 1)), dim3(1024), 0, stream>>>(MACs, n_mols, order, outputs, n_outputs);

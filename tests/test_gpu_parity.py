@@ -636,10 +636,10 @@ def test_plain_coulomb_sums(ops, kind, n_mols):
     assert not np.allclose(damped, helpers.CHARGE_K * _coulomb_brute(b.X, b.Y, b.Z, q, b.MOs, b.MACs, 1.0, g)[0], rtol=1e-3)
 
 
-@pytest.mark.parametrize("n_mols", [256, 257, 1025, 16384, 16385])
+@pytest.mark.parametrize("n_mols", [256, 257, 512, 513, 1025, 16384, 16385])
 @pytest.mark.parametrize("ndt", [np.float32, np.float64])
 def test_charges_in_size_order(ops, n_mols, ndt):
-    """Dense batches of 257 to 16,384 molecules are walked by decreasing size: every output has the bits that batch order
+    """Dense batches of 257 (float32: 513) to 16,384 molecules are walked by decreasing size: every output has the bits that batch order
     gives (khan_ani_charge_all), for sizes on either side of a wavefront and a workgroup and in a mixed order; atoms outside
     every molecule keep zeros.  (The energy of a molecule of more than 256 atoms is added up in an order that varies: a few
     roundings of the sum of its terms.)"""
