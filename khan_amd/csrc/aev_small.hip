@@ -43,9 +43,10 @@ constexpr int kRadSlots = 96;
 
 // With kJvp the kernel computes the Jacobian-vector product instead (featurize_grad_inverse): every term of
 // the forward sums is replaced by its derivative along the per-atom vectors (VX, VY, VZ).
-// float: 4 wavefronts per SIMD (LDS 9.8 KB, <= 128 VGPRs; the kernel loses a fifth of its speed at three), and 5 with kFive
-// (6.9 KB, 96 VGPRs, without hoisting: khan_amd/build.py; 65,536 organic molecules 497 -> 468 us);
-// float kJvp: 3 (<= 168 VGPRs; its LDS lets twelve wavefronts share a CU); double: 3 (149 VGPRs, LDS 12.5 KB with four
+// float: 4 wavefronts per SIMD (LDS 8.8 KB, <= 128 VGPRs; the kernel loses a fifth of its speed at three), and 5 with kFive
+// (6.9 KB, 96 VGPRs and two more in scratch memory, without hoisting: khan_amd/build.py; 65,536 organic molecules
+// 497 -> 468 us);
+// float kJvp: 3 (<= 168 VGPRs; its LDS lets twelve wavefronts share a CU); double: 3 (148 VGPRs, LDS 12.6 KB with four
 // centres); double kJvp: 1.
 constexpr int fwd_small_waves(size_t element, bool jvp, bool five) { return element == 4 ? (jvp ? 3 : five ? 5 : 4) : (jvp ? 1 : 3); }
 
@@ -65,7 +66,7 @@ void aev_fwd_small_kernel(
     // centres per batch: six; four in the float Jacobian-vector kernel (with kCap below: twelve wavefronts per CU), in double
     // and with kFive (6.9 KB: six of the 1,280 bytes LDS is given out in, twenty wavefronts per CU)
     constexpr int kNB = (kJvp == (sizeof(T) == 4) || kFive) ? 4 : kFB;
-    // angular partners kept per centre: 32; 28 in the float Jacobian-vector kernel, whose working set then is 13.4 KB
+    // angular partners kept per centre: 32; 28 in the float Jacobian-vector kernel, whose working set then is 12.7 KB
     // and twelve wavefronts share a CU (a centre with more goes to the general routine, as above 32 elsewhere)
     constexpr int kCap = (kJvp && sizeof(T) == 4) ? 28 : kCapA;
     __shared__ FwdWaveLds<T, kJvp, kNB, kRadSlots, kCap> lds_all[kWavesPerBlock];

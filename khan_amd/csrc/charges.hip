@@ -50,8 +50,8 @@ template <bool kDamped> struct PairTerms<float, kDamped> {
 // double: no library call, no square root and no angle.  1/r from v_rsq_f64 (5e-8) and one third-order step.  1 - f_C =
 // sin^2(pi r / 2 R_c) = d2 q(d2) and 2 d(1 - f_C)/d(d2) = (d/dr) / r are entire functions of d2: polynomials of degree
 // nine in d2 (Chebyshev interpolation on [0, R_c^2]), exact to 4e-16 of q and 1e-16.  (Before: a square root, a folded half
-// angle, its sine and cosine: 106 vector instructions per pair over the whole kernel, 92 with the polynomials' coefficients in
-// vector registers, where every step of Horner's scheme copies one first, 74 with them in scalar registers.)
+// angle, its sine and cosine: 106 vector instructions per pair over the whole kernel by the counters, 92 with the polynomials'
+// coefficients in vector registers, where every step of Horner's scheme copies one first, 72 with them in scalar registers.)
 template <bool kDamped> struct PairTerms<double, kDamped> {
     struct Constants {
         double q[10], t[10];
@@ -183,7 +183,8 @@ template <typename T> struct __align__(16) ChargeTile<T, true> {
 };
 
 template <typename T, bool kDamped, bool kGrad>
-__device__ __forceinline__ void charge_tile(const ChargeArgs<T>& a, const typename PairTerms<T, kDamped>::Constants& constants, ChargeTile<T, kGrad>& S, int mol, int n)
+__device__ __forceinline__ void charge_tile(const ChargeArgs<T>& a, const typename PairTerms<T, kDamped>::Constants& constants,
+                                            ChargeTile<T, kGrad>& S, int mol, int n)
 {
     typedef typename Fast<T>::vec2 vec2;
     static_assert(kMediumMaxAtoms == 256, "one atom per thread of a 256-thread workgroup");
@@ -323,7 +324,8 @@ __device__ __forceinline__ void charge_tile(const ChargeArgs<T>& a, const typena
 // blocks.  The energy is half the sum over atoms of q_i times the atom's sum, added to E[mol] (zeroed before the launch)
 // by one floating-point atomic per workgroup and block: its last bits depend on the order of those additions.
 template <typename T, bool kDamped, bool kGrad>
-__device__ __forceinline__ void charge_large(const ChargeArgs<T>& a, const typename PairTerms<T, kDamped>::Constants& constants, typename Fast<T>::vec4* tile, T* wpart, int column, int columns, int part, int parts)
+__device__ __forceinline__ void charge_large(const ChargeArgs<T>& a, const typename PairTerms<T, kDamped>::Constants& constants,
+                                             typename Fast<T>::vec4* tile, T* wpart, int column, int columns, int part, int parts)
 {
     typedef typename Fast<T>::vec4 vec4;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -399,9 +401,10 @@ __device__ __forceinline__ void charge_large(const ChargeArgs<T>& a, const typen
 // for every molecule, which takes those of 65 to 256 (in the first ones' places a wavefront with 64 atoms had the compute unit
 // that came upon it last work for 35 us after all others).  With per = 4 a workgroup does both for its four molecules.
 // (Three launches, one per size, cost 10 us where two of them found nothing to do.)  Four workgroups per compute unit, which
-// LDS allows.  4,096 boxes of 64 to 256 atoms in double, energy and both gradients with the launch before: 224 -> 156 us
-// (coefficients in scalar registers, size order, first places for the small molecules, two rounds side by side); vector
-// issue binds, 60 instructions a pair, with LDS (six 16-byte accesses a pair) at two thirds of its rate.
+// LDS allows.  4,096 boxes of 64 to 256 atoms in double, energy and both gradients with the launch before: 217 -> 148 us
+// (coefficients in scalar registers, size order, first places for the small molecules, two rounds side by side; 170 in batch
+// order).  Vector issue binds: by the counters 72 instructions a pair keep it 76 % busy, with an LDS instruction executing on
+// a compute unit 82 % of the time (7.7 a pair).
 template <typename T, bool kDamped, bool kGrad>
 __global__ __launch_bounds__(256, 4) void charge_kernel(ChargeArgs<T> a, int columns, int parts, int per)
 {

@@ -506,7 +506,7 @@ __global__ __launch_bounds__(256) void top_kernel(const NetTop<T> a, int total)
 // carry their rounding errors along: added up plainly, 64 rows to a lane, they were 2e-7 off where a library sum is 4e-8 off
 // (124 -> 126 us a launch at 35,000 rows).
 // In float32 this form is left for layers narrower than 64, for few rows and for operands that are not aligned
-// (weight_grad_split_tile takes the others): 62 TFLOP/s of the instructions' 153 at 35,000 rows of 384-128-128-64-1 (82 us).
+// (weight_grad_split_tile takes the others): 61 TFLOP/s of the instructions' 153 at 35,000 rows of 384-128-128-64-1 (85 us).
 // The compiler's overlap of the unrolled loop's loads with the products beats four row groups loaded ahead by hand (104 us).
 // sum += x, its rounding error added to `lost` (Knuth's two-sum)
 template <typename V>
@@ -631,8 +631,8 @@ __device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __rest
 // products have accumulators of their own, so that the large sum is rounded once in 32 rows: the distance from float64 is half
 // of the float32 instructions' (35,000 rows: 2.85e-7 -> 1.39e-7; with one set of accumulators 3.06e-7).  The next rows'
 // loads are in flight during the products; two workgroups share a compute unit and fill each other's barriers.
-// Gradients of 384-128-128-64-1 on 35,000 rows, one pair of operands 86 -> 51 us, both 157 -> 85 (101 TFLOP/s); 12,132 rows
-// 42 -> 28.  What is left is products (14 us), splitting and the loads of 144 MB (30 us) one after the other.  No faster: two
+// Gradients of 384-128-128-64-1 on 35,000 rows, this launch alone: one pair of operands 85 -> 50 us (103 TFLOP/s), both 160 ->
+// 82 (126); 12,132 rows 41 -> 27.  With grad_sum_kernel 92 -> 60, 167 -> 92 and 49 -> 35.  What is left of one pair is products (14 us), splitting and the loads of 144 MB (30 us) one after the other.  No faster: two
 // chunks in flight instead of one (with the small products added to the large ones chunk by chunk, for its registers),
 // splitting by v_dot2_f32_bf16 (seven instructions instead of eleven).
 // Both operands are split 2^24 times their size (the bias sums are formed before): a value's third part has its exponent 24
