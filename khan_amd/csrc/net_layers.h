@@ -59,8 +59,9 @@ struct NetGrads {
     int k[kNetMaxLayers + 1];       // widths: layer l is [k[l], k[l + 1]]
     T* out;
     // filled by the launcher: rows per workgroup, the workgroups' numbering by layer and type and where their partial sums
-    // begin; the layers whose operands may be read 16 bytes at a time, and those on split products
-    int per, job_end[4 * kNetMaxLayers];
+    // begin; the layers whose operands may be read 16 bytes at a time, and those on split products (with their own rows per
+    // workgroup)
+    int per, per_split, job_end[4 * kNetMaxLayers];
     int64_t job_base[4 * kNetMaxLayers];
     unsigned whole, split;
 };

@@ -623,7 +623,7 @@ __device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __rest
 }
 
 // The same in float32 on the bfloat16 matrix instructions (the split of layer_split_kernel), for layers of at least 64 x 64.
-// A workgroup forms 128 of the left operand's columns x 128 (kWide) or 64 of the right's over `per` rows, 32 rows at a
+// A workgroup forms 128 of the left operand's columns x 128 (kWide) or 64 of the right's over `per_split` rows, 32 rows at a
 // time.  The rows are what is summed over, so that a matrix instruction's operand is eight rows of one column, which lie a row
 // apart in memory: a thread loads two neighbouring columns of eight rows (a wavefront 512 contiguous bytes of each row), splits
 // them and writes them to LDS as [part][eight rows][column] pieces of 16 bytes, column 2 c + j at place 64 j + c, so that
@@ -631,8 +631,8 @@ __device__ __forceinline__ void weight_grad_tile(const NetGrads<T>& a, T* __rest
 // products have accumulators of their own, so that the large sum is rounded once in 32 rows: the distance from float64 is half
 // of the float32 instructions' (35,000 rows: 2.85e-7 -> 1.39e-7; with one set of accumulators 3.06e-7).  The next rows'
 // loads are in flight during the products; two workgroups share a compute unit and fill each other's barriers.
-// Gradients of 384-128-128-64-1 on 35,000 rows, this launch alone: one pair of operands 85 -> 50 us (103 TFLOP/s), both 160 ->
-// 82 (126); 12,132 rows 41 -> 27.  With grad_sum_kernel 92 -> 60, 167 -> 92 and 49 -> 35.  What is left of one pair is products (14 us), splitting and the loads of 144 MB (30 us) one after the other.  No faster: two
+// Gradients of 384-128-128-64-1 on 35,000 rows, this launch alone: one pair of operands 85 -> 49 us (105 TFLOP/s), both 160 ->
+// 81 (128); 12,132 rows 41 -> 27.  With grad_sum_kernel 92 -> 58, 167 -> 90 and 49 -> 35.  What is left of one pair is products (14 us), splitting and the loads of 144 MB (30 us) one after the other.  No faster: two
 // chunks in flight instead of one (with the small products added to the large ones chunk by chunk, for its registers),
 // splitting by v_dot2_f32_bf16 (seven instructions instead of eleven).
 // Both operands are split 2^24 times their size (the bias sums are formed before): a value's third part has its exponent 24
@@ -663,7 +663,7 @@ __device__ __forceinline__ void weight_grad_split_tile(const NetGrads<float>& a,
     const int tiles_n = (N + kCols - 1) / kCols, tiles = (K + kGradLeft - 1) / kGradLeft * tiles_n;
     const int share = rel / tiles, tile = rel - share * tiles;
     const int i0 = tile / tiles_n * kGradLeft, j0 = tile % tiles_n * kCols;
-    const int r0 = share * a.per, r1 = min(n, r0 + a.per);
+    const int r0 = share * a.per_split, r1 = min(n, r0 + a.per_split);
     const int chunks = (r1 - r0 + kGradChunk - 1) / kGradChunk;
     // this thread's columns (past the end: the last ones again, whose sums are never read)
     const int li = min(i0 + 2 * lane, K - 2), lj = min(j0 + kRC * lane, N - kRC);
@@ -909,7 +909,7 @@ __global__ __launch_bounds__(256) void grad_sum_kernel(const NetGrads<T> a, cons
     }
     const int t = block / (tiles * runs), tile = block / runs - t * tiles, at = (block % runs * 64 + lane) * V;
     const int K = a.k[layer], N = a.k[layer + 1], size = rows * cols + cols;
-    const int shares = (a.n[t] + a.per - 1) / a.per;
+    const int per = split ? a.per_split : a.per, shares = (a.n[t] + per - 1) / per;
     const T* p = partial + a.job_base[layer * 4 + t] + static_cast<size_t>(tile) * size + min(at, size - V);
     const size_t stride = static_cast<size_t>(tiles) * size;
     Vec<T> sum = Vec<T>(T(0)), lost = Vec<T>(T(0));
@@ -1099,21 +1099,27 @@ static int64_t plan_grads(NetGrads<T>& a, bool split)
     int64_t per = 64;
     while (per < 4096 && rows / per * tiles > 1024) per *= 2;
     // beside split products as many rows as theirs, whose workgroups take as long: all workgroups at once, two per compute unit, or
-    // as few such rounds as shares of up to 2,048 rows make (520 workgroups on 512 places took 56 us where 505 take 50)
+    // as few such rounds as shares of up to 2,048 rows make (520 workgroups on 512 places took 56 us where 505 take 50).  Where the
+    // next larger shares would fit for the narrow layers' sake alone, those alone take them (35,000 rows of 384-128-128-64-1, 516
+    // workgroups of 416 rows, 510 with the narrow ones of 448: one pair 50.6 -> 49 us, both 83 -> 81).
+    int64_t share = per;
     if (split_tiles) {
-        per = 4 * kGradChunk;
-        for (int64_t rounds = 1; blocks_of(per, split_tiles + tiles) > 512 * rounds;) {
-            per += kGradChunk;
-            if (per > 64 * kGradChunk) per = 4 * kGradChunk, ++rounds;
+        per = share = 4 * kGradChunk;
+        for (int64_t rounds = 1; blocks_of(share, split_tiles) + blocks_of(per, tiles) > 512 * rounds;) {
+            if (per == share && share < 64 * kGradChunk) per += kGradChunk;
+            else if (share < 64 * kGradChunk) share = per;
+            else per = share = 4 * kGradChunk, ++rounds;
         }
     }
     a.per = static_cast<int>(per);
+    a.per_split = static_cast<int>(share);
     int64_t end = 0, base = 0;
     for (int l = 0; l < a.layers; ++l) {
         const bool is_split = (a.split >> l) & 1u;
         const int64_t size = is_split ? (kGradLeft + 1) * (a.k[l + 1] > 64 ? 128 : 64) : kSide * kSide + kSide;
+        const int64_t rows_each = is_split ? share : per;
         for (int t = 0; t < 4; ++t) {
-            const int64_t blocks = (a.n[t] + per - 1) / per * tiles_of(l);
+            const int64_t blocks = (a.n[t] + rows_each - 1) / rows_each * tiles_of(l);
             a.job_base[l * 4 + t] = base;
             base += blocks * size;
             a.job_end[l * 4 + t] = static_cast<int>(end += blocks);
@@ -1164,7 +1170,7 @@ hipError_t launch_net_grads(NetGrads<T> a, void* workspace, hipStream_t stream)
     // 69.7 -> 67.9; 384-64-1 (480), 10 shares 13.2 -> 12.8; eleven layers (9,600 to 11,600), 3 to 13 shares 31 -> 50, 61 -> 80, 372 -> 387.
     int most = 0;
     for (int t = 0; t < 4; ++t) most = std::max(most, a.n[t]);
-    if ((static_cast<int64_t>(most) + a.per - 1) / a.per * 50 > sums)
+    if ((static_cast<int64_t>(most) + a.per_split - 1) / a.per_split * 50 > sums)
         grad_sum_kernel<T, true><<<dim3(static_cast<unsigned>(sums)), dim3(256), 0, stream>>>(a, static_cast<const T*>(workspace));
     else
         grad_sum_kernel<T, false><<<dim3(static_cast<unsigned>((sums + 3) / 4)), dim3(256), 0, stream>>>(a, static_cast<const T*>(workspace));

@@ -237,13 +237,15 @@ def _one_layer_gradients(lib, left, right):
 
 # Every plan of the weight gradients: few rows of many tiles (a wavefront to each run of the sums) and many rows of few (a
 # workgroup), both sides of the lines between float32 and split products, several rounds of workgroups (36 tiles, 60,000 rows),
-# narrow layers beside wide ones, widths that are no multiple of anything.  A share's sum has at most 2,048 / 4 + 4 products one
-# after the other on a lane and 64 on the split form's, shares and quarters carry their roundings: float64 stays below 520 units of
-# 2^-53, float32 below the 2e-6 of the tests above (its sums over wavefronts and matrix steps are far from their worst case).
+# narrow layers beside wide ones, with the same shares and (35,000 rows) larger ones, widths that are no multiple of anything.  A
+# share's sum has at most 2,048 / 4 + 4 products one after the other on a lane and 64 on the split form's, shares and quarters
+# carry their roundings: float64 stays below 520 units of 2^-53, float32 below the 2e-6 of the tests above (its sums over
+# wavefronts and matrix steps are far from their worst case).
 @pytest.mark.parametrize("dtype,bound", [(torch.float32, 2e-6), (torch.float64, 520 * 2.0 ** -53)])
 @pytest.mark.parametrize("widths,rows", [((384, 512, 512, 256, 1), (5, 0, 1, 2)), ((384, 512, 512, 1), (31200, 20400, 3601, 4799)), ((384, 256, 1), (12000, 7000, 33, 1)),
                                          ((384, 128, 128, 64, 1), (1000, 700, 200, 98)), ((384, 128, 128, 64, 1), (1300, 850, 150, 200)),
                                          ((384, 128, 128, 64, 1), (2500, 1700, 300, 299)), ((384, 128, 128, 64, 1), (2500, 1700, 300, 301)),
+                                         ((384, 128, 128, 64, 1), (18200, 11900, 2100, 2800)),
                                          ((384, 64, 1), (4000, 3000, 500, 499)), ((37, 66, 5, 1), (300, 0, 17, 1))])
 def test_weight_gradients_of_every_plan(widths, rows, dtype, bound):
     from khan_amd import _lib
