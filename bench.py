@@ -101,7 +101,7 @@ def cpu_baseline(batch, sample_mols_fwd, sample_mols_bwd, w=4):
     # the same kernels sharded by molecule over the host cores (one slice of molecules per thread; the
     # reference runs one CPU tower per core this way, gdb8.py:73-76)
     import concurrent.futures
-    # a one-GPU box gives a job 16 host cores whatever os.cpu_count() shows there: at most that many threads
+    # a machine shared by GPU gives a job 16 host cores whatever os.cpu_count() shows there: at most that many threads
     host_cores = os.cpu_count() or 1
     threads = max(1, min(16, host_cores))
 

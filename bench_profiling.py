@@ -4,7 +4,7 @@
 a digest of the kernel sources it was measured on, and an entry whose digest differs from the sources in the tree
 is reported as stale (traffic null) instead of being passed on.
 
-Refreshing an entry (on a GPU box; four counter passes, one counter each, each a run of its own):
+Refreshing an entry (on a machine with the GPU; four counter passes, one counter each, each a run of its own):
 
     cd /tmp && export TMPDIR=/tmp
     rocprofv3 --pmc FETCH_SIZE --kernel-trace --output-format csv -d OUT/fwd_fetch -o p -- python3 bench.py --workload W --traffic-probe fwd

@@ -2,7 +2,7 @@
 /root/reference/gpu_featurizer/kernel_cpu.cpp built in place by `make -C oracle _ref`).
 
 Run once in the build container:   python tests/golden/make_golden.py
-The GPU box has no reference tree; tests there read only the committed .npz.
+A machine with a GPU need not have the reference tree; tests read only the committed .npz.
 
 Cases
   fx11   the reference's 11-atom / 2-molecule test fixture (gpu_featurizer/test_kernel.py:269-287)
