@@ -29,6 +29,13 @@ struct __align__(16) FwdWaveLds {
     T rec[64][12];
     static_assert(kRadN * 2 <= 64 * 12, "the radial list lies in the records' place");
     __device__ __forceinline__ typename Fast<T>::vec2* rad() { return reinterpret_cast<typename Fast<T>::vec2*>(&rec[0][0]); }
+    // behind the radial list, while the centres of a batch are scanned: `n` atoms (large molecules)
+    template <int n> __device__ __forceinline__ typename Fast<T>::vec4* atoms()
+    {
+        static_assert(sizeof(rec) + sizeof(seg) + sizeof(segrow) >= kRadN * sizeof(typename Fast<T>::vec2) + n * sizeof(typename Fast<T>::vec4),
+                      "the atoms lie in the place of the records and the segment table");
+        return reinterpret_cast<typename Fast<T>::vec4*>(&rec[0][0] + 2 * kRadN);
+    }
     SegDesc seg[kSegments];                   // non-empty segments of the batch, in order
     unsigned long long segrow[kSegments];     // where each of them puts its 32 output values (then: the empty blocks' addresses)
     unsigned bits[bit_words(kNB)];            // bit per triple slot: a segment starts here

@@ -171,10 +171,13 @@ __global__ __launch_bounds__(256) void large_sort_kernel(
             return f;
         };
         auto place = [&](int j, int dest, const Fetched& f) {
-            sorted.atom[dest] = Fast<T>::make4(f.x, f.y, f.z, static_cast<T>(f.type));
-            sorted.aux[dest] = make_int2(j, f.si);
+            T word;
+            set_atom_word(word, (f.type << kTypeShift) | f.si);
+            sorted.atom[dest] = Fast<T>::make4(f.x, f.y, f.z, word);
+            sorted.index[dest] = off + j;
             if (sorted.vel) sorted.vel[dest] = Fast<T>::make4(f.vx, f.vy, f.vz, T(0));
             if (gX) {
+                if (sorted.force) sorted.force[dest] = Fast<T>::make4(T(0), T(0), T(0), T(0));
                 gX[off + j] = T(0);
                 gY[off + j] = T(0);
                 gZ[off + j] = T(0);

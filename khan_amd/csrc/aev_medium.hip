@@ -40,10 +40,11 @@ struct __align__(16) MedShared {
 // above 256 atoms the sorted atoms are in device memory (aev_large.h)
 template <typename T, bool kJvp>
 struct __align__(16) MedShared<T, kJvp, true> {
-    // partner types of the entries of each wavefront's radial list and of the angular list it is building (used by the
+    // partner types of the entries of the radial list and of the angular list that is being built (used by the
     // Jacobian-vector product, whose list entries have no room for the type)
-    unsigned char rtype[4][kRadCap];
-    unsigned char atype[4][kCapA];
+    unsigned char rtype[kJvp ? kRadCap : 1];
+    unsigned char atype[kJvp ? kCapA : 1];
+    int candidates[kMaxCandidates];        // the atoms in reach of the run of centres
 };
 
 // With kJvp the kernel computes the Jacobian-vector product instead (featurize_grad_inverse), as the
@@ -53,7 +54,7 @@ struct __align__(16) MedShared<T, kJvp, true> {
 // With kLarge the kernel takes the molecules of more than 256 atoms: the atoms come type-sorted from `sorted`.
 // kOnce: the rows are marked as written once (store_global)
 template <typename T, bool kJvp, bool kLarge = false, bool kShare = kLarge, bool kOnce = false>
-__global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
+__global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 4 ? 5 : 1) void aev_fwd_medium_kernel(
     const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
     const int32_t* __restrict__ A, const int32_t* __restrict__ MOs,
     const int32_t* __restrict__ MACs, int32_t n_mols, const int32_t* __restrict__ SIs,
@@ -71,18 +72,18 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
     // forward kernel keeps batches of six, and the float64 Jacobian-vector kernel takes batches of four (one workgroup per
     // CU; six measured the same).
     constexpr int kNB = (sizeof(T) == 4 || kJvp) ? 4 : kFB;
-    __shared__ FwdWaveLds<T, kJvp, kNB> lds_wave[4];
+    __shared__ FwdWaveLds<T, kJvp, kNB> lds_wave[kLarge ? 1 : 4];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = uniform(tid >> 6);
+    const int wave = kLarge ? 0 : uniform(tid >> 6);
     FwdWaveLds<T, kJvp, kNB>& S = lds_wave[wave];
     const LaneConsts<T> L = lane_consts<T>(lane);
     const unsigned long long lt_mask = (1ull << lane) - 1ull;
     const int rslot = lane >> 4;                                 // radial walk: entry slot of this 16-lane group
 
     fwd_lds_init(S, lane);
-    __shared__ unsigned long long want[4];
-    for_each_molecule_in_range(MACs, n_mols, min_atoms, kLarge ? INT32_MAX : kMediumMaxAtoms, want, order, order ? order + n_mols : nullptr, [&](int mol) {
+    // (kLarge: of a run of the molecule's sorted atoms, from run_first on)
+    const auto run_molecule = [&](int mol, int run_first) {
         const int n = uniform(MACs[mol]);
         const int off = uniform(MOs[mol]);
 
@@ -142,13 +143,17 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
             if constexpr (kLarge) return sorted.atom[off + sorted_idx];
             else return M.atom[sorted_idx];
         };
+        auto type_at = [](T w) -> int {                      // from the atom's fourth component
+            if constexpr (kLarge) return atom_word(w) >> kTypeShift;
+            else return static_cast<int>(w) & 3;
+        };
         auto vel_at = [&](int sorted_idx) -> vec4 {
             if constexpr (!kJvp) return Fast<T>::make4(T(0), T(0), T(0), T(0));
             else if constexpr (kLarge) return sorted.vel[off + sorted_idx];
             else return M.v.vel[sorted_idx];
         };
         auto orig_of = [&](int sorted_idx) -> int {          // wave-uniform index
-            if constexpr (kLarge) return uniform(sorted.aux[off + sorted_idx].x);
+            if constexpr (kLarge) return uniform(sorted.index[off + sorted_idx]) - off;
             else if constexpr (kJvp) return uniform(static_cast<int>(M.v.orig[sorted_idx]));
             else return uniform(static_cast<int>(M.atom[sorted_idx].w) >> 2);
         };
@@ -178,19 +183,22 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
         };
 
         // ------------------------------------------------------------ batches of kNB centres per wavefront
-        // (few centres for many wavefronts: shorter batches, so that every wavefront gets some)
-        const int waves_y = kShare ? static_cast<int>(gridDim.y) * 4 : 4;
-        const int batch = kShare ? max(1, min(kNB, (n + waves_y - 1) / waves_y)) : kNB;
-        const int first_c0 = (kShare ? static_cast<int>(blockIdx.y) * 4 + wave : wave) * batch;
-        const int stride_c0 = waves_y * batch;
-        for (c0 = first_c0; c0 < n; c0 += stride_c0) {
-            const int nb = min(batch, n - c0);
+        vec4* candidate_vels = nullptr;                       // (in the place of the second records)
+        if constexpr (kLarge && kJvp) {
+            static_assert(sizeof(S.jvp.rec2) >= kMaxCandidates * sizeof(vec4), "");
+            candidate_vels = reinterpret_cast<vec4*>(&S.jvp.rec2[0][0]);
+        }
+        // the centres from first_c0 to end_c0, kNB or `batch` at a time
+        auto run_centres = [&](int first_c0, int end_c0, int batch, int stride_c0, int n_candidates) {
+        for (c0 = first_c0; c0 < end_c0; c0 += stride_c0) {
+            const int nb = min(batch, end_c0 - c0);
             unsigned overflow = 0;
             if ((kLarge || !kJvp) && lane < nb) {                     // (the load is under way while the first centre is scanned)
-                const int w = static_cast<int>(atom_at(c0 + lane).w), type = w & 3;
+                const T w = atom_at(c0 + lane).w;
+                const int type = type_at(w);
                 int place;
-                if constexpr (kLarge) place = sorted.aux[off + c0 + lane].y;
-                else place = SIs[off + (w >> 2)];
+                if constexpr (kLarge) place = atom_word(w) & kPlaceMask;
+                else place = SIs[off + (static_cast<int>(w) >> 2)];
                 T* const bucket = type == 0 ? out.p[0] : type == 1 ? out.p[1] : type == 2 ? out.p[2] : out.p[3];
                 const unsigned long long row = reinterpret_cast<unsigned long long>(bucket + static_cast<size_t>(place) * kFeats);
                 row_lo = static_cast<unsigned>(row);
@@ -242,8 +250,8 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                     if (lane < count) {
                         e = S.rad()[lane];
                         if constexpr (kJvp) ab = S.jvp.rad_ab[lane];
-                        if constexpr (kJvp && kLarge) tR = M.rtype[wave][lane];
-                        else tR = static_cast<int>(e.y) & 3;
+                        if constexpr (kJvp && kLarge) tR = M.rtype[lane];
+                        else tR = type_at(e.y);
                     }
                     int cnt[4], dest = 0, before = 0;
 #pragma unroll
@@ -266,12 +274,11 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                     radial_sums(racc, cnt);
                     wave_lds_fence();               // the list may be overwritten
                 };
-                // one chunk of 64 partners: aj (and with kJvp vjv) of the atom at sorted position jc + lane
-                auto scan_chunk = [&](int jc, const vec4 aj, const vec4 vjv) {
-                    const int j = jc + lane;
+                // 64 partners: aj (and with kJvp vjv) of the atom at sorted position j, where this lane has one
+                auto scan = [&](int j, bool have, const vec4 aj, const vec4 vjv) {
                     const T dx = ai.x - aj.x, dy = ai.y - aj.y, dz = ai.z - aj.z;
                     const T r = Fast<T>::sqrt_rn(dx * dx + dy * dy + dz * dz);
-                    const bool valid = (j < n) && (j != i);
+                    const bool valid = have && (j != i);
                     // r = 0, a coincident atom: no part in derivatives; in the features as the reference has it
                     const bool inR = valid && (r < kR_Rc_f) && (!kJvp || r > T(0));
                     const bool inA = valid && (r < kA_Rc_f) && (!kJvp || r > T(0));
@@ -283,7 +290,7 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                         }
                     }
                     if constexpr (kJvp) {
-                        const int tj = static_cast<int>(aj.w);
+                        const int tj = type_at(aj.w);
 #pragma unroll
                         for (int a = 0; a < 4; ++a) {
                             const unsigned long long ta = wave_ballot(tj == a);
@@ -301,7 +308,7 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                                 Fast<T>::cutoff_grad(r, static_cast<T>(kR_Rc_f), fc, dfc);
                                 S.rad()[p] = Fast<T>::make2(r, fc);
                                 S.jvp.rad_ab[p] = Fast<T>::make2(dfc * rd, T(-2) * static_cast<T>(kR_eta_f) * fc * rd);
-                                if constexpr (kLarge) M.rtype[wave][p] = static_cast<unsigned char>(tj);
+                                if constexpr (kLarge) M.rtype[p] = static_cast<unsigned char>(tj);
                             }
                         }
                         if (inA) {
@@ -313,7 +320,7 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                                 S.nbr_fc[b][p] = fc;
                                 S.jvp.nbr_p[b][p] = Fast<T>::make4(wx * inv, wy * inv, wz * inv, rd * inv);
                                 S.jvp.nbr_dfc[b][p] = dfc * rd;
-                                if constexpr (kLarge) M.atype[wave][p] = static_cast<unsigned char>(tj);
+                                if constexpr (kLarge) M.atype[p] = static_cast<unsigned char>(tj);
                             }
                         }
                     } else {
@@ -337,38 +344,11 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                     posA += popc64(mA);
                 };
                 if constexpr (kLarge) {
-                    // From device memory.  The atoms are sorted by type and, inside a type, along a space-filling
-                    // curve: 64 chunks' boxes are tested against the centre at a time (one per lane), and only the
-                    // chunks that reach into the radial cutoff are scanned, four chunks' loads in flight at a time.
-                    const float cx = static_cast<float>(ai.x), cy = static_cast<float>(ai.y), cz = static_cast<float>(ai.z);
-                    for (int ch0 = 0; ch0 < n_chunks; ch0 += 64) {
-                        unsigned long long near = wave_ballot(chunk_in_reach(sorted.box + 2 * chunk0, ch0 + lane, n_chunks, cx, cy, cz));
-                        while (near) {
-                            int ch[4];
-#pragma unroll
-                            for (int u = 0; u < 4; ++u) {
-                                ch[u] = -1;
-                                if (near) {
-                                    ch[u] = ch0 + lowest_bit(near);
-                                    near &= near - 1;
-                                }
-                            }
-                            vec4 at[4], vt[4];
-#pragma unroll
-                            for (int u = 0; u < 4; ++u) {
-                                const int jj = min(max(ch[u], 0) * 64 + lane, last_atom);
-                                at[u] = atom_at(jj);
-                                vt[u] = vel_at(jj);
-                            }
-#pragma unroll
-                            for (int u = 0; u < 4; ++u)
-                                if (ch[u] >= 0) scan_chunk(ch[u] * 64, at[u], vt[u]);
-                        }
-                    }
+                    scan_partners<T, kJvp, true>(sorted, off, n, chunk0, M.candidates, S.template atoms<kMaxCandidates>(), candidate_vels, n_candidates, ai, lane, scan);
                 } else {
                     for (int jc = 0; jc < n; jc += 64) {
                         const int jj = min(jc + lane, last_atom);
-                        scan_chunk(jc, atom_at(jj), vel_at(jj));
+                        scan(jc + lane, jc + lane < n, atom_at(jj), vel_at(jj));
                     }
                 }
                 if constexpr (kLarge) {
@@ -385,9 +365,9 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                         if constexpr (kJvp) {
                             np = S.jvp.nbr_p[b][lane];
                             nd = S.jvp.nbr_dfc[b][lane];
-                            tA = M.atype[wave][lane];
+                            tA = M.atype[lane];
                         } else {
-                            tA = static_cast<int>(fc) & 3;
+                            tA = type_at(fc);
                         }
                     }
                     int dest = 0, before = 0;
@@ -413,12 +393,12 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                     int tR = -1, tA = -1;           // type of this lane's list entry
                     if (haveR) {
                         const vec2 e = S.rad()[lane];
-                        tR = static_cast<int>(e.y) & 3;
+                        tR = type_at(e.y);
                         S.rad()[lane] = Fast<T>::make2(e.x, Fast<T>::cutoff(e.x, static_cast<T>(kR_Rc_f)));
                     }
                     if (haveA) {
                         const vec4 d = S.nbr[b][lane];
-                        tA = static_cast<int>(S.nbr_fc[b][lane]) & 3;
+                        tA = type_at(S.nbr_fc[b][lane]);
                         const T inv = Fast<T>::rcp(d.w);
                         S.nbr[b][lane] = Fast<T>::make4(d.x * inv, d.y * inv, d.z * inv, d.w);
                         S.nbr_fc[b][lane] = Fast<T>::cutoff(d.w, static_cast<T>(kA_Rc_f));
@@ -472,8 +452,37 @@ __global__ __launch_bounds__(256) void aev_fwd_medium_kernel(
                 wave_lds_fence();
             }
         }
-        __syncthreads();      // the next molecule reuses the sorted arrays
-    });
+        };
+        if constexpr (kLarge) {
+            // the run with its candidates, or, where the atoms are too close together for a list, shorter ones
+            static_assert(!kLarge || kRunCentres <= kNB, "a run is a batch: its candidates lie where the records go");
+            const int run_end = min(n, run_first + (1 << sorted.runs.log_run));
+            for (int from = run_first, length = run_end - run_first; from < run_end;) {
+                const int to = min(from + length, run_end);
+                const int n_candidates = list_candidates<T, kJvp>(sorted, off, n, chunk0, from, to, M.candidates, S.template atoms<kMaxCandidates>(),
+                                                                  candidate_vels, lane);
+                if (n_candidates < 0 && length > 1) {
+                    length = (length + 1) >> 1;
+                    continue;
+                }
+                run_centres(from, to, kNB, kNB, n_candidates);
+                from = to;
+            }
+        } else {
+            // (few centres for many wavefronts: shorter batches, so that every wavefront gets some)
+            const int waves_y = kShare ? static_cast<int>(gridDim.y) * 4 : 4;
+            const int batch = kShare ? max(1, min(kNB, (n + waves_y - 1) / waves_y)) : kNB;
+            run_centres((kShare ? static_cast<int>(blockIdx.y) * 4 + wave : wave) * batch, n, batch, waves_y * batch, 0);
+            __syncthreads();  // the next molecule reuses the sorted arrays
+        }
+    };
+    if constexpr (kLarge) {
+        for_each_run(MOs, MACs, n_mols, sorted.runs, order ? order + n_mols : nullptr, run_molecule);
+    } else {
+        __shared__ unsigned long long want[4];
+        for_each_molecule_in_range(MACs, n_mols, min_atoms, kMediumMaxAtoms, want, order, order ? order + n_mols : nullptr,
+                                   [&](int mol) { run_molecule(mol, 0); });
+    }
 }
 
 }  // namespace
@@ -529,22 +538,22 @@ size_t large_scratch_bytes(int64_t n_atoms, int32_t n_mols, bool with_vectors)
 }
 
 // Molecules of more than 256 atoms: the sort into `scratch` (large_scratch_bytes), then the kernel above with the
-// centres of a molecule spread over the workgroups of a grid column.
+// centres of a molecule spread over workgroups run by run.
 template <typename T>
 hipError_t launch_fwd_large(const T* X, const T* Y, const T* Z, const int32_t* A,
                             const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
                             const int32_t* SIs, const T* VX, const T* VY, const T* VZ, Buckets<T> out,
-                            const int32_t* order, void* scratch, int64_t n_atoms, hipStream_t stream)
+                            const int32_t* order, void* scratch, int64_t n_atoms, bool sure, hipStream_t stream)
 {
     if (n_mols <= 0) return hipSuccess;
     const bool jvp = VX != nullptr;
-    const SortedAtoms<T> sorted = carve_sorted_atoms<T>(scratch, n_atoms, n_mols, jvp);
+    const SortedAtoms<T> sorted = carve_sorted_atoms<T>(scratch, n_atoms, n_mols, sure, jvp, false);
     const hipError_t e = launch_large_sort<T>(X, Y, Z, A, MOs, MACs, n_mols, SIs, VX, VY, VZ, nullptr, nullptr, nullptr, order,
                                               sorted, stream);
     if (e != hipSuccess) return e;
-    const dim3 grid = large_grid(n_mols);
+    const dim3 grid(sorted.runs.blocks);
     if (jvp)
-        aev_fwd_medium_kernel<T, true, true><<<grid, dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, VX, VY, VZ, out,
+        aev_fwd_medium_kernel<T, true, true><<<grid, dim3(64), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, VX, VY, VZ, out,
                                                                          kMediumMaxAtoms + 1, order, sorted);
     else {
         // The rows are marked as written once from 64 MB on already: the backward pass, which reads its atoms and skeleton again
@@ -552,7 +561,7 @@ hipError_t launch_fwd_large(const T* X, const T* Y, const T* Z, const int32_t* A
         // 1,024-4,096 atoms, 94 MB, 472 -> 468 us, 32 635 -> 621, 48 1,116 -> 1,113, 64 the same; 16 in float64 739 -> 722; below
         // 64 MB the same).
         const auto kernel = rows_beyond_caches<T>(n_atoms, 64 << 20) ? aev_fwd_medium_kernel<T, false, true, true, true> : aev_fwd_medium_kernel<T, false, true>;
-        kernel<<<grid, dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, out, kMediumMaxAtoms + 1, order, sorted);
+        kernel<<<grid, dim3(64), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, out, kMediumMaxAtoms + 1, order, sorted);
     }
     return hipGetLastError();
 }
@@ -565,8 +574,8 @@ template hipError_t launch_fwd_medium<double>(const double*, const double*, cons
 template hipError_t launch_jvp_medium<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const double*, const double*, const double*, Buckets<double>, int, const int32_t*, hipStream_t);
 template size_t large_scratch_bytes<float>(int64_t, int32_t, bool);
 template size_t large_scratch_bytes<double>(int64_t, int32_t, bool);
-template hipError_t launch_fwd_large<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const float*, const float*, const float*, Buckets<float>, const int32_t*, void*, int64_t, hipStream_t);
-template hipError_t launch_fwd_large<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const double*, const double*, const double*, Buckets<double>, const int32_t*, void*, int64_t, hipStream_t);
+template hipError_t launch_fwd_large<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const float*, const float*, const float*, Buckets<float>, const int32_t*, void*, int64_t, bool, hipStream_t);
+template hipError_t launch_fwd_large<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, const double*, const double*, const double*, Buckets<double>, const int32_t*, void*, int64_t, bool, hipStream_t);
 #endif
 
 }  // namespace khan

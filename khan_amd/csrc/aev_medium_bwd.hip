@@ -28,7 +28,6 @@ namespace khan {
 namespace {
 
 constexpr int kChunks = kMediumMaxAtoms / 64;
-constexpr int kTypeShift = 28;     // large molecules: a radial queue entry is a sorted position with the atom's type above it
 // centres per batch: four, so that the pools of the four wavefronts leave room for four workgroups on a CU in float
 // (LDS 39.6 KB; 128 registers) and two in double (76 KB; 256 registers) -- the shorter batches fill fewer lanes, the
 // additional wavefronts per SIMD hide more (dense boxes: float 4 % faster than six-centre batches at three workgroups,
@@ -65,11 +64,14 @@ struct __align__(16) MedBwdShared {
     int next;                              // next centre (sorted position) to hand out
 };
 // above 256 atoms the sorted atoms are in device memory (aev_large.h); the list entries' sorted positions no
-// longer fit a byte and are kept here, one array per wavefront (the pool's byte array then holds the types)
+// longer fit a byte and are kept here (the pool's byte array then holds the types).  A radial queue entry is the partner's word
+// (atom_word) and the centre's place in the run.
 template <typename T>
 struct __align__(16) MedBwdShared<T, true, false> {
-    int pos[4][64];
-    int next;                              // centres handed out so far by this workgroup
+    int pos[64];
+    int centre_word[kRunCentres];          // the run's centres: word ...
+    T centre_force[kRunCentres][4];        // ... and the sum of their forces so far
+    int candidates[kMaxCandidates];        // the atoms in reach of the run of centres
 };
 
 // With kShare the workgroups of one grid column (blockIdx.y = 0 .. gridDim.y - 1) share a molecule's centres, and its
@@ -77,7 +79,7 @@ struct __align__(16) MedBwdShared<T, true, false> {
 // plain kernel 6 %).
 // With kLarge the kernel takes the molecules of more than 256 atoms: the atoms come type-sorted from `sorted`.
 template <typename T, bool kLarge = false, bool kLocal = false, bool kShare = kLarge>
-__global__ __launch_bounds__(256)
+__global__ __launch_bounds__(kLarge ? 64 : 256)
 __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (kLocal ? 3 : 4) : (kLocal ? 1 : 2), sizeof(T) == 4 ? (kLocal ? 3 : 4) : (kLocal ? 1 : 2))))
 void aev_bwd_medium_kernel(
     const T* __restrict__ X, const T* __restrict__ Y, const T* __restrict__ Z,
@@ -87,24 +89,49 @@ void aev_bwd_medium_kernel(
     const int32_t* __restrict__ order, bool walk_in_order, const SortedAtoms<T> sorted)
 {
     typedef typename Fast<T>::vec4 vec4;
-    typedef typename std::conditional<kLarge, int, unsigned short>::type idx_t;     // a sorted position in the radial queue
+    typedef typename std::conditional<kLarge, int, unsigned short>::type idx_t;     // a partner in the radial queue
+    typedef typename std::conditional<kLarge, unsigned char, unsigned short>::type centre_t;        // and its centre
     static_assert(!(kLarge && kLocal), "forces in LDS: molecules of up to 256 atoms only");
     __shared__ MedBwdShared<T, kLarge, kLocal> M;
     constexpr int kMB = kMedBwdCentres<T>;
     // the double kernel for 65-256 atoms runs at 256 registers (two workgroups per compute unit): with the cutoff's
     // polynomial constants resident it spills 21 of them and is 8 % slower than with the library's cos and sin
     constexpr bool kLibraryCutoff = sizeof(T) == 8 && !kLarge && !kLocal;
-    __shared__ BwdPool<T, kMB> pools[4];
+    __shared__ BwdPool<T, kMB> pools[kLarge ? 1 : 4];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = uniform(tid >> 6);
+    const int wave = kLarge ? 0 : uniform(tid >> 6);
     BwdPool<T, kMB>& P = pools[wave];
     const LaneConsts<T> L = lane_consts<T>(lane);
     const unsigned long long lt_mask = (1ull << lane) - 1ull;
 
-    __shared__ unsigned long long want[4];
-    for_each_molecule_in_range(MACs, n_mols, min_atoms, kLarge ? INT32_MAX : kMediumMaxAtoms, want, walk_in_order ? order : nullptr,
-                               order ? order + n_mols : nullptr, [&](int mol) {
+    // Large molecules: the forces are added up in sorted order, 16 (32) bytes an atom (sorted.force), so that the three additions to
+    // an atom, and those to its neighbours in an instruction, are one request beyond the L2, and are brought to the outputs by a
+    // kernel of their own (one by one to the three outputs, the additions were what the kernel waited for: 64 boxes of 1,024-4,096 atoms
+    // 434 us, 331 without any of them, 348 so; that is the form without sorted.force).  values: `count` atoms of the wavefront's LDS, four elements each; place_of(e): the
+    // e-th one's place.
+    const auto add_forces = [&](const T* values, int count, auto place_of) {
+        if constexpr (kLarge) {
+            if (!sorted.force) {
+                if (lane < count) {
+                    const int g = sorted.index[place_of(lane)];
+                    atomicAdd(&gX[g], values[4 * lane]);
+                    atomicAdd(&gY[g], values[4 * lane + 1]);
+                    atomicAdd(&gZ[g], values[4 * lane + 2]);
+                }
+                return;
+            }
+            const int k = lane & 3;
+            for (int e0 = 0; e0 < count; e0 += 16) {
+                const int e = min(e0 + (lane >> 2), count - 1);
+                const int place = place_of(e);
+                const T value = values[4 * e + k];
+                if (k < 3 && e0 + (lane >> 2) < count) atomicAdd(reinterpret_cast<T*>(sorted.force + place) + k, value);
+            }
+        }
+    };
+    // (kLarge: of a run of the molecule's sorted atoms, from run_first on)
+    const auto run_molecule = [&](int mol, int run_first) {
         const int n = uniform(MACs[mol]);
         const int off = uniform(MOs[mol]);
         int tb1, tb2, tb3;                     // sorted position of the first C, N, O atom
@@ -112,8 +139,6 @@ void aev_bwd_medium_kernel(
         // ------------------------------------------------------------ load, sort by type into LDS, zero outputs
         if constexpr (kLarge) {
             tb1 = tb2 = tb3 = 0;               // (the sorted atoms are not in order of type: types come with the atoms)
-            if (tid == 0) M.next = 0;
-            __syncthreads();
         } else {
         const bool have = tid < n;
         T x = T(0), y = T(0), z = T(0);
@@ -175,22 +200,27 @@ void aev_bwd_medium_kernel(
         };
         auto row_bits_of = [&](int sorted_idx, int type) -> unsigned long long {     // per-lane index, and that atom's type
             if constexpr (kLarge) {
+                // (sorted_idx: the row inside the type's bucket)
                 const T* const bucket = type == 0 ? gin.p[0] : type == 1 ? gin.p[1] : type == 2 ? gin.p[2] : gin.p[3];
-                return reinterpret_cast<unsigned long long>(bucket + static_cast<size_t>(sorted.aux[off + sorted_idx].y) * kFeats);
+                return reinterpret_cast<unsigned long long>(bucket + static_cast<size_t>(sorted_idx) * kFeats);
             } else {
                 return (static_cast<unsigned long long>(M.row_hi[sorted_idx]) << 32) | M.row_lo[sorted_idx];
             }
         };
-        auto row_of = [&](int sorted_idx) -> const T* {            // wave-uniform index
-            int type = 0;
-            if constexpr (kLarge) type = static_cast<int>(sorted.atom[off + sorted_idx].w);
-            const unsigned long long bits = row_bits_of(sorted_idx, type);
+        auto row_of = [&](int sorted_idx) -> const T* {            // wave-uniform index, of a centre
+            unsigned long long bits;
+            if constexpr (kLarge) {
+                const int word = M.centre_word[sorted_idx - run_first];
+                bits = row_bits_of(word & kPlaceMask, word >> kTypeShift);
+            } else {
+                bits = row_bits_of(sorted_idx, 0);
+            }
             const unsigned lo = static_cast<unsigned>(uniform(static_cast<int>(bits & 0xffffffffull)));
             const unsigned hi = static_cast<unsigned>(uniform(static_cast<int>(bits >> 32)));
             return reinterpret_cast<const T*>((static_cast<unsigned long long>(hi) << 32) | lo);
         };
         auto orig_of = [&](int sorted_idx) -> int {                // per-lane index
-            if constexpr (kLarge) return sorted.aux[off + sorted_idx].x;
+            if constexpr (kLarge) return sorted.index[off + sorted_idx] - off;
             else return M.orig[sorted_idx];
         };
         // per-lane target; with forces in LDS the caller sees to it that the lanes of one call hit distinct atoms
@@ -207,13 +237,23 @@ void aev_bwd_medium_kernel(
             }
         };
 
+        auto add_to_centre = [&](int place, T fx, T fy, T fz) {      // (large molecules; the lanes of a call have distinct places)
+            if constexpr (kLarge) {
+                M.centre_force[place][0] += fx;
+                M.centre_force[place][1] += fy;
+                M.centre_force[place][2] += fz;
+            }
+        };
         // Radial pairs are queued and worked off 64 at a time: only about an eighth of the (centre, partner)
         // pairs of a large molecule lie inside the radial cutoff, so evaluating them where they are found
         // would leave most lanes idle.  The queue lives in the pool's staging area, which is free while a
         // batch is being collected; it is emptied before the batch's upstream rows are staged.
         vec4* const q_d = reinterpret_cast<vec4*>(P.gst);                          // 128 x (dx, dy, dz, r)
-        idx_t* const q_j = reinterpret_cast<idx_t*>(q_d + 128);                    // partner (sorted position)
-        idx_t* const q_c = q_j + 128;                                              // centre (sorted position)
+        idx_t* const q_j = reinterpret_cast<idx_t*>(q_d + 128);                    // partner (sorted position; large molecules: word)
+        centre_t* const q_c = reinterpret_cast<centre_t*>(q_j + 128);              // centre (sorted position; large molecules: place in the run)
+        // behind it the atoms of a large molecule's candidates
+        vec4* const candidate_atoms = reinterpret_cast<vec4*>(q_c + 128);
+        static_assert(!kLarge || sizeof(P.gst) >= 128 * (sizeof(vec4) + sizeof(idx_t) + sizeof(centre_t)) + kMaxCandidates * sizeof(vec4), "");
         int qn = 0;
         auto radial_work_off = [&](int count) {      // entries 0..count-1, count <= 64
             T fx = T(0), fy = T(0), fz = T(0);
@@ -223,17 +263,21 @@ void aev_bwd_medium_kernel(
                 j = q_j[lane];
                 c = q_c[lane];
                 int tj, tc;
-                if constexpr (kLarge) {            // the queue carries the types in the four high bits
+                unsigned long long row_c, row_j;
+                if constexpr (kLarge) {
+                    const int wc = M.centre_word[c];
                     tj = j >> kTypeShift;
-                    tc = c >> kTypeShift;
-                    j &= (1 << kTypeShift) - 1;
-                    c &= (1 << kTypeShift) - 1;
+                    tc = wc >> kTypeShift;
+                    row_j = row_bits_of(j & kPlaceMask, tj);
+                    row_c = row_bits_of(wc & kPlaceMask, tc);
                 } else {
                     tj = type_of(j);
                     tc = type_of(c);
+                    row_c = row_bits_of(c, tc);
+                    row_j = row_bits_of(j, tj);
                 }
-                const T* grow_c = reinterpret_cast<const T*>(row_bits_of(c, tc));
-                const T* grow_j = reinterpret_cast<const T*>(row_bits_of(j, tj));
+                const T* grow_c = reinterpret_cast<const T*>(row_c);
+                const T* grow_j = reinterpret_cast<const T*>(row_j);
                 const T inv = Fast<T>::rcp(e.w);
                 // the pair's pull on the centre from both rows.  With forces in LDS the pair is queued once (by its
                 // centre of lower sorted position) and the partner gets minus this below; otherwise the partner gets
@@ -259,7 +303,9 @@ void aev_bwd_medium_kernel(
             const T qx = lane_fetch(px, at), qy = lane_fetch(py, at), qz = lane_fetch(pz, at);
             if (run_end) {
                 const bool whole = first == 0;
-                add_force(c, whole ? px : px - qx, whole ? py : py - qy, whole ? pz : pz - qz);
+                const T sx = whole ? px : px - qx, sy = whole ? py : py - qy, sz = whole ? pz : pz - qz;
+                if constexpr (kLarge) add_to_centre(c, sx, sy, sz);
+                else add_force(c, sx, sy, sz);
             }
             if constexpr (kLocal) {
                 // the partners: run after run, because the partners of one centre are distinct atoms and those of two
@@ -281,7 +327,8 @@ void aev_bwd_medium_kernel(
                 radial_work_off(take);
                 const int rest = qn - take;
                 vec4 e = Fast<T>::make4(T(0), T(0), T(0), T(1));
-                idx_t ej = 0, ec = 0;
+                idx_t ej = 0;
+                centre_t ec = 0;
                 if (lane < rest) {
                     e = q_d[64 + lane];
                     ej = q_j[64 + lane];
@@ -303,7 +350,8 @@ void aev_bwd_medium_kernel(
             radial_work_off(64);
             const int rest = qn - 64;
             vec4 e = Fast<T>::make4(T(0), T(0), T(0), T(1));
-            idx_t ej = 0, ec = 0;
+            idx_t ej = 0;
+            centre_t ec = 0;
             if (lane < rest) {
                 e = q_d[64 + lane];
                 ej = q_j[64 + lane];
@@ -321,7 +369,17 @@ void aev_bwd_medium_kernel(
 
         // (few centres for many wavefronts: shorter batches, so that every one of them gets some)
         const int most = kShare && !kLarge ? max(1, min(kMB, (n + static_cast<int>(gridDim.y) * 4 - 1) / (static_cast<int>(gridDim.y) * 4))) : kMB;
-        int dealt = 0;             // (forces in LDS) centres this wavefront has taken: it takes every fourth, by position
+        // the wavefront's centres: those it draws, every fourth by position (forces in LDS), or those from `from` to end_c (large
+        // molecules, with that many candidates)
+        auto run_centres = [&](int from, int end_c, int n_candidates) {
+        int dealt = from;
+        auto hold_candidates = [&]() {         // (large molecules) the run's candidates, again
+            if constexpr (kLarge) {
+                wave_lds_fence();
+                for (int q = lane; q < n_candidates; q += 64) candidate_atoms[q] = sorted.atom[off + M.candidates[q]];
+                wave_lds_fence();
+            }
+        };
         int pending = -1;          // a centre that was drawn but did not fit the previous batch
         int scanned = -1;          // (large molecules) the centre whose radial pairs were queued last
         for (;;) {
@@ -329,12 +387,18 @@ void aev_bwd_medium_kernel(
             int nb = 0, used = 0;
             int pfv = 0, cv = 0;   // lane k: first pool slot and sorted position of centre k of the batch
             P.facc[lane] = Fast<T>::make4(T(0), T(0), T(0), T(0));
+            if (kLarge && dealt > from) {
+                if (pending < 0 && dealt >= end_c) break;
+                hold_candidates();             // (the last batch's upstream rows lie where they were)
+            }
             while (nb < most) {
                 int c = pending;
                 pending = -1;
                 if (c < 0) {
                     if constexpr (kLocal) {
                         c = wave + 4 * dealt++;
+                    } else if constexpr (kLarge) {
+                        c = dealt++;
                     } else {
                         int drawn = 0;
                         if (lane == 0) drawn = atomicAdd(&M.next, 1);
@@ -342,7 +406,7 @@ void aev_bwd_medium_kernel(
                         if constexpr (kShare) c = static_cast<int>(blockIdx.y) + static_cast<int>(gridDim.y) * c;
                     }
                 }
-                if (c >= n) break;
+                if (c >= end_c) break;
                 const vec4 ai = atom_at(c);
                 int m_c = 0;
                 bool too_many;
@@ -352,19 +416,18 @@ void aev_bwd_medium_kernel(
                     // batch, where it is scanned again; its radial pairs are queued the first time only).
                     const bool again = c == scanned;
                     int pos = used;
-                    auto scan_chunk = [&](int jc, const vec4 aj) {
-                        const int j = jc + lane;
+                    auto scan = [&](int j, bool have, const vec4 aj, const vec4&) {
                         const T ddx = ai.x - aj.x, ddy = ai.y - aj.y, ddz = ai.z - aj.z;
                         const T rr = Fast<T>::sqrt_rn(ddx * ddx + ddy * ddy + ddz * ddz);
-                        const bool valid = (j < n) && (j != c);
+                        const bool valid = have && (j != c);
                         const unsigned long long mRb = wave_ballot(!kSkipRadial && !again && valid && (rr < kR_Rc_f) && (rr > T(0)));
                         const unsigned long long mAb = wave_ballot(valid && (rr < kA_Rc_f) && (rr > T(0)));
                         if ((mAb >> lane) & 1ull) {
                             const int p = pos + popc64(mAb & lt_mask);
                             if (p < 64) {
                                 P.nbr[p] = Fast<T>::make4(ddx, ddy, ddz, rr);
-                                P.nbr_idx[p] = static_cast<unsigned char>(static_cast<int>(aj.w));      // the partner's type
-                                M.pos[wave][p] = j;
+                                P.nbr_idx[p] = static_cast<unsigned char>(atom_word(aj.w) >> kTypeShift);      // the partner's type
+                                M.pos[p] = j;
                             }
                         }
                         pos += popc64(mAb);
@@ -372,37 +435,13 @@ void aev_bwd_medium_kernel(
                         if ((mRb >> lane) & 1ull) {
                             const int p = qn + popc64(mRb & lt_mask);
                             q_d[p] = Fast<T>::make4(ddx, ddy, ddz, rr);
-                            q_j[p] = static_cast<idx_t>(j | (static_cast<int>(aj.w) << kTypeShift));
-                            q_c[p] = static_cast<idx_t>(c | (static_cast<int>(ai.w) << kTypeShift));
+                            q_j[p] = static_cast<idx_t>(atom_word(aj.w));
+                            q_c[p] = static_cast<centre_t>(c - run_first);
                         }
                         qn += popc64(mRb);
                         if (qn >= 64) radial_work_off_full();
                     };
-                    // 64 chunks' boxes are tested against the centre at a time (one per lane); the chunks that reach into
-                    // the radial cutoff are scanned, four chunks' loads in flight at a time
-                    const float cx = static_cast<float>(ai.x), cy = static_cast<float>(ai.y), cz = static_cast<float>(ai.z);
-                    const int n_chunks = (n + 63) >> 6;
-                    const float4* const boxes = sorted.box + 2 * chunk_base(off, mol);
-                    for (int ch0 = 0; ch0 < n_chunks; ch0 += 64) {
-                        unsigned long long near = wave_ballot(chunk_in_reach(boxes, ch0 + lane, n_chunks, cx, cy, cz));
-                        while (near) {
-                            int ch[4];
-#pragma unroll
-                            for (int u = 0; u < 4; ++u) {
-                                ch[u] = -1;
-                                if (near) {
-                                    ch[u] = ch0 + lowest_bit(near);
-                                    near &= near - 1;
-                                }
-                            }
-                            vec4 at[4];
-#pragma unroll
-                            for (int u = 0; u < 4; ++u) at[u] = atom_at(min(max(ch[u], 0) * 64 + lane, n - 1));
-#pragma unroll
-                            for (int u = 0; u < 4; ++u)
-                                if (ch[u] >= 0) scan_chunk(ch[u] * 64, at[u]);
-                        }
-                    }
+                    scan_partners<T, false, false>(sorted, off, n, chunk_base(off, mol), M.candidates, candidate_atoms, nullptr, n_candidates, ai, lane, scan);
                     scanned = c;
                     too_many = m_c > 64;
                     if (!too_many && nb > 0 && used + m_c > 64) {       // full: this centre opens the next batch
@@ -496,6 +535,7 @@ void aev_bwd_medium_kernel(
                                               },
                                               false);
                     wave_lds_fence();
+                    if constexpr (kLarge) hold_candidates();
                     continue;
                 }
                 if (lane == nb) {
@@ -541,9 +581,13 @@ void aev_bwd_medium_kernel(
                     if (live && bs == bb) add_force(target, f.x, f.y, f.z);
                     wave_lds_fence();
                 }
+            } else if constexpr (kLarge) {
+                wave_lds_fence();              // (every lane has read its forces)
+                P.facc[lane] = f;
+                wave_lds_fence();
+                add_forces(reinterpret_cast<const T*>(P.facc), total, [&](int e) { return off + M.pos[e]; });
             } else if (live) {
-                if constexpr (kLarge) add_force(M.pos[wave][lane], f.x, f.y, f.z);
-                else add_force(P.nbr_idx[lane], f.x, f.y, f.z);
+                add_force(P.nbr_idx[lane], f.x, f.y, f.z);
             }
             {
                 // a centre's list is a run of lanes: its sum is the difference of two values of an add-scan,
@@ -561,9 +605,33 @@ void aev_bwd_medium_kernel(
                     sy -= qy;
                     sz -= qz;
                 }
-                if (lane < nb && hi > lo) add_force(cv, -sx, -sy, -sz);      // cv of lane b = centre b
+                if (lane < nb && hi > lo) {                                  // cv of lane b = centre b
+                    if constexpr (kLarge) add_to_centre(cv - run_first, -sx, -sy, -sz);
+                    else add_force(cv, -sx, -sy, -sz);
+                }
             }
             wave_lds_fence();
+        }
+        };
+        if constexpr (kLarge) {
+            // the run with its candidates, or, where the atoms are too close together for a list, shorter ones
+            const int run_end = min(n, run_first + (1 << sorted.runs.log_run));
+            if (lane < run_end - run_first) M.centre_word[lane] = atom_word(sorted.atom[off + run_first + lane].w);
+            if (lane < 4 * kRunCentres) M.centre_force[lane >> 2][lane & 3] = T(0);
+            wave_lds_fence();
+            for (int from = run_first, length = run_end - run_first; from < run_end;) {
+                const int to = min(from + length, run_end);
+                const int n_candidates = list_candidates<T, false>(sorted, off, n, chunk_base(off, mol), from, to, M.candidates, candidate_atoms, nullptr, lane);
+                if (n_candidates < 0 && length > 1) {
+                    length = (length + 1) >> 1;
+                    continue;
+                }
+                run_centres(from, to, n_candidates);
+                from = to;
+            }
+            add_forces(&M.centre_force[0][0], run_end - run_first, [&](int e) { return off + run_first + e; });
+        } else {
+            run_centres(0, n, 0);
         }
         if constexpr (kLocal) {
             __syncthreads();  // every wavefront's forces are complete
@@ -574,7 +642,32 @@ void aev_bwd_medium_kernel(
                 gZ[g] = (M.force.f[0][2][tid] + M.force.f[1][2][tid]) + (M.force.f[2][2][tid] + M.force.f[3][2][tid]);
             }
         }
-        __syncthreads();      // the next molecule reuses the sorted arrays
+        if constexpr (!kLarge) __syncthreads();      // the next molecule reuses the sorted arrays
+    };
+    if constexpr (kLarge) {
+        for_each_run(MOs, MACs, n_mols, sorted.runs, order ? order + n_mols : nullptr, run_molecule);
+    } else {
+        __shared__ unsigned long long want[4];
+        for_each_molecule_in_range(MACs, n_mols, min_atoms, kMediumMaxAtoms, want, walk_in_order ? order : nullptr,
+                                   order ? order + n_mols : nullptr, [&](int mol) { run_molecule(mol, 0); });
+    }
+}
+
+// The forces on the sorted atoms of large molecules, 64 to a workgroup, added to the gradients (which hold what the general per-centre
+// routine has added).
+template <typename T>
+__global__ __launch_bounds__(64) void large_force_kernel(const int32_t* __restrict__ MOs, const int32_t* __restrict__ MACs, int32_t n_mols,
+                                                         T* __restrict__ gX, T* __restrict__ gY, T* __restrict__ gZ,
+                                                         const int32_t* __restrict__ order, const SortedAtoms<T> sorted)
+{
+    for_each_run(MOs, MACs, n_mols, sorted.runs, order ? order + n_mols : nullptr, [&](int mol, int first) {
+        const int j = first + static_cast<int>(threadIdx.x);
+        if (j >= uniform(MACs[mol])) return;
+        const int at = uniform(MOs[mol]) + j, g = sorted.index[at];
+        const typename Fast<T>::vec4 f = sorted.force[at];
+        gX[g] += f.x;
+        gY[g] += f.y;
+        gZ[g] += f.z;
     });
 }
 
@@ -627,28 +720,32 @@ hipError_t launch_bwd_medium(const T* X, const T* Y, const T* Z, const int32_t* 
 }
 
 // Molecules of more than 256 atoms: the sort into `scratch` (large_scratch_bytes), which also zeroes their gradients,
-// then the kernel above with the centres of a molecule spread over the workgroups of a grid column.
+// then the kernel above with the centres of a molecule spread over workgroups run by run.
 template <typename T>
 hipError_t launch_bwd_large(const T* X, const T* Y, const T* Z, const int32_t* A,
                             const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
                             const int32_t* SIs, Buckets<const T> g, T* gX, T* gY, T* gZ,
-                            const int32_t* order, void* scratch, int64_t n_atoms, hipStream_t stream)
+                            const int32_t* order, void* scratch, int64_t n_atoms, bool sure, hipStream_t stream)
 {
     if (n_mols <= 0) return hipSuccess;
-    const SortedAtoms<T> sorted = carve_sorted_atoms<T>(scratch, n_atoms, n_mols, false);
+    // (a batch that may hold no such molecule goes without the kernel behind this one)
+    SortedAtoms<T> sorted = carve_sorted_atoms<T>(scratch, n_atoms, n_mols, sure, false, sure);
     const hipError_t e = launch_large_sort<T>(X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, gX, gY, gZ, order,
                                               sorted, stream);
     if (e != hipSuccess) return e;
-    const dim3 grid = large_grid(n_mols);
-    aev_bwd_medium_kernel<T, true><<<grid, dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, g, gX, gY, gZ,
+    const dim3 grid(sorted.runs.blocks);
+    aev_bwd_medium_kernel<T, true><<<grid, dim3(64), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, g, gX, gY, gZ,
                                                                   kMediumMaxAtoms + 1, order, false, sorted);
+    if (!sure) return hipGetLastError();
+    sorted.runs = runs_of(n_atoms, n_mols, true, 6);
+    large_force_kernel<T><<<dim3(sorted.runs.blocks), dim3(64), 0, stream>>>(MOs, MACs, n_mols, gX, gY, gZ, order, sorted);
     return hipGetLastError();
 }
 
 template hipError_t launch_bwd_medium<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<const float>, float*, float*, float*, int, const int32_t*, bool, bool, hipStream_t);
 template hipError_t launch_bwd_medium<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<const double>, double*, double*, double*, int, const int32_t*, bool, bool, hipStream_t);
 
-template hipError_t launch_bwd_large<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<const float>, float*, float*, float*, const int32_t*, void*, int64_t, hipStream_t);
-template hipError_t launch_bwd_large<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<const double>, double*, double*, double*, const int32_t*, void*, int64_t, hipStream_t);
+template hipError_t launch_bwd_large<float>(const float*, const float*, const float*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<const float>, float*, float*, float*, const int32_t*, void*, int64_t, bool, hipStream_t);
+template hipError_t launch_bwd_large<double>(const double*, const double*, const double*, const int32_t*, const int32_t*, const int32_t*, int32_t, const int32_t*, Buckets<const double>, double*, double*, double*, const int32_t*, void*, int64_t, bool, hipStream_t);
 
 }  // namespace khan

@@ -205,7 +205,7 @@ int forward_dispatch(const T* xs, const T* ys, const T* zs, const int32_t* as, c
         const LargeScratch scratch(may_allocate && n_atoms < kLargeAtomLimit ? khan::large_scratch_bytes<T>(n_atoms, n_mols, false) : 0, stream);
         if (scratch.get())
             st = hip_status(khan::launch_fwd_large<T>(xs, ys, zs, as, mos, macs, n_mols, sis, nullptr, nullptr, nullptr, out,
-                                                      order, scratch.get(), n_atoms, stream));
+                                                      order, scratch.get(), n_atoms, cls.known, stream));
         else
             st = hip_status(khan::launch_fwd_generic<T>(xs, ys, zs, as, mos, macs, n_mols, sis, out,
                                                         khan::kMediumMaxAtoms + 1, order, stream));
@@ -229,10 +229,10 @@ int backward_dispatch(const T* xs, const T* ys, const T* zs, const int32_t* as, 
     const SizeClasses cls(classes_host);
     int st = KHAN_OK;
     if (n_atoms > khan::kMediumMaxAtoms && cls.any(khan::kMediumMaxAtoms + 1, INT32_MAX)) {
-        const LargeScratch scratch(n_atoms < kLargeAtomLimit ? khan::large_scratch_bytes<T>(n_atoms, n_mols, false) : 0, stream);
+        const LargeScratch scratch(n_atoms < kLargeAtomLimit ? khan::large_scratch_bytes<T>(n_atoms, n_mols, cls.known) : 0, stream);
         if (scratch.get())
             st = hip_status(khan::launch_bwd_large<T>(xs, ys, zs, as, mos, macs, n_mols, sis, g, gx, gy, gz, order,
-                                                      scratch.get(), n_atoms, stream));
+                                                      scratch.get(), n_atoms, cls.known, stream));
         else
             st = hip_status(khan::launch_bwd_generic<T>(xs, ys, zs, as, mos, macs, n_mols, sis, g, gx, gy, gz,
                                                         n_atoms, khan::kMediumMaxAtoms + 1, order, stream));
@@ -366,7 +366,7 @@ int featurize_grad_inverse_impl(const T* xs, const T* ys, const T* zs, const int
                                    as_stream(stream));
         if (scratch.get())
             st = hip_status(khan::launch_fwd_large<T>(xs, ys, zs, as, mos, macs, n_mols, sis, vx, vy, vz, out, order,
-                                                      scratch.get(), n_atoms, as_stream(stream)));
+                                                      scratch.get(), n_atoms, cls.known, as_stream(stream)));
         else if (n_atoms > khan::kMediumMaxAtoms)
             st = hip_status(khan::launch_jvp_generic<T>(xs, ys, zs, as, mos, macs, n_mols, sis, vx, vy, vz, out,
                                                         khan::kMediumMaxAtoms + 1, order, as_stream(stream)));

@@ -75,14 +75,14 @@ template <typename T>
 hipError_t launch_fwd_large(const T* X, const T* Y, const T* Z, const int32_t* A,
                             const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
                             const int32_t* SIs, const T* VX, const T* VY, const T* VZ, Buckets<T> out,
-                            const int32_t* order, void* scratch, int64_t n_atoms, hipStream_t stream);
+                            const int32_t* order, void* scratch, int64_t n_atoms, bool sure, hipStream_t stream);
 
 // backward (the molecules' gradients need no zeroing beforehand)
 template <typename T>
 hipError_t launch_bwd_large(const T* X, const T* Y, const T* Z, const int32_t* A,
                             const int32_t* MOs, const int32_t* MACs, int32_t n_mols,
                             const int32_t* SIs, Buckets<const T> g, T* gX, T* gY, T* gZ,
-                            const int32_t* order, void* scratch, int64_t n_atoms, hipStream_t stream);
+                            const int32_t* order, void* scratch, int64_t n_atoms, bool sure, hipStream_t stream);
 
 template <typename T>
 hipError_t launch_bwd_medium(const T* X, const T* Y, const T* Z, const int32_t* A,

@@ -919,6 +919,56 @@ def test_random_large_molecules(ops, seed):
         check_forward_backward(ops, Case(xyz[:, 0], xyz[:, 1], xyz[:, 2], A, mi, len(mols)))
 
 
+# Large molecules are worked on in runs of one, two or four neighbouring atoms by the size of the batch (lines at 9,000 and 40,000
+# atoms), with the forces summed beside the outputs where the host knows that there are such molecules.  The dense box's runs have more
+# atoms in reach than a list holds and are halved; some centres of the crowded ball go to the general routine.
+@pytest.mark.parametrize("copies", [1, 4, 16])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_runs_of_large_molecules(ops, dtype, copies):
+    say("case: runs of large molecules, %s, %d copies" % (dtype, copies))
+    rng = np.random.default_rng(83)
+    types = lambda n: rng.choice(4, n, p=[0.5, 0.3, 0.1, 0.1])
+    mols = [(types(1025), _jittered_lattice(rng, 1025, 2.15, 0.5)), (types(257), _jittered_lattice(rng, 257, 2.15, 0.5)),
+            (types(3), _jittered_lattice(rng, 3, 1.5, 0.2)), (types(729), _jittered_lattice(rng, 729, 1.55, 0.15)),
+            (types(70), _jittered_lattice(rng, 70, 2.15, 0.5)), (rng.integers(0, 4, 420), _packed_ball(rng, 420, 5.0, 0.85)),
+            (types(320), _jittered_lattice(rng, 320, 2.15, 0.5))]
+    near = mols[3][1][np.argsort(np.linalg.norm(mols[3][1] - mols[3][1].mean(axis=0), axis=1))[:4]]
+    away = np.maximum(np.maximum(near.min(axis=0) - mols[3][1], mols[3][1] - near.max(axis=0)), 0.0)
+    assert (np.linalg.norm(away, axis=1) < 4.6).sum() > 176      # more than a list holds
+    rtol, atol = (F32_RTOL, F32_ATOL) if dtype == torch.float32 else (F64_RTOL, F64_ATOL)
+    one = Case(*np.concatenate([m[1] for m in mols]).T, np.concatenate([m[0] for m in mols]),
+               np.repeat(np.arange(len(mols)), [len(m[0]) for m in mols]), len(mols))
+    up = rng.standard_normal((one.N, 384)).astype(np.float32).astype(np.float64)
+    vectors = rng.standard_normal((3, one.N))
+    order_of = rng.permutation(copies * len(mols))              # the copies' molecules in an order of their own
+    at = np.concatenate([np.arange(one.MOs[m % len(mols)], one.MOs[m % len(mols)] + one.MACs[m % len(mols)]) for m in order_of])
+    many = Case(one.X[at], one.Y[at], one.Z[at], one.A[at], np.repeat(np.arange(len(order_of)), one.MACs[order_of % len(mols)]), len(order_of))
+    X, Y, Z = (dev(v).to(dtype) for v in (many.X, many.Y, many.Z))
+    mos, macs, sc, A = dev(many.MOs), dev(many.MACs), dev(many.sc), dev(many.A)
+    order = ops.size_order(macs)
+    classes = order[-4:].cpu()
+    assert int(classes[3]) == 5 * copies
+    acs = torch.from_numpy(np.asarray(many.ac, dtype=np.int32))
+    ups = [dev(u).to(dtype) for u in ob.scatter_rows(up[at], many.A, many.sc, many.ac)]
+    rows64 = ob.gather_rows(one.oracle_feat(np.float64), one.ga)[at]
+    grad64 = one.oracle_grad(ob.scatter_rows(up, one.A, one.sc, one.ac))[at]
+    scale = mol_scale(grad64, many.MOs, many.MACs)
+    for known in (True, False):
+        kw = dict(order=order, size_classes=classes) if known else {}
+        args = (X, Y, Z, A, mos, macs, sc, acs)
+        rows = ob.gather_rows([host(f).astype(np.float64) for f in ops.featurize(*args, **kw)], many.ga)
+        assert_close("rows, classes %s" % known, rows, rows64, rtol, atol)
+        g = host(torch.stack(ops.featurize_grad(*args, *ups, **kw), dim=1))
+        assert_close("gradients, classes %s" % known, g, grad64, rtol, atol, scale)
+        v = [dev(w[at]).to(dtype) for w in vectors]
+        jv = ops.featurize_grad_inverse(*args, *v, **kw)
+        # <up, J v> = <J^T up, v>, molecule by molecule: both sides are sums of terms of both signs
+        dot = sum((a.double() * b.double()).view(-1, 384).sum(1).sum() for a, b in zip(jv, ups))
+        back = sum((dev(g[:, k]).double() * v[k].double()).sum() for k in range(3))
+        bound = sum((a.double() * b.double()).abs().sum() for a, b in zip(jv, ups))
+        assert abs(float(dot - back)) <= rtol * float(bound), (float(dot), float(back), float(bound))
+
+
 # Both sides of each line between the forward kernels: 174,763 atoms in float32 (87,382 in float64) make 256 MB of rows, 43,691
 # (21,846) the 64 MB of molecules of more than 256 atoms; up to 8,192 molecules of 32 atoms in float32 (6,144 of 64 in float64)
 # and 2,048 (512) larger ones are shared, and from 16,385 on there are five wavefronts to a SIMD.
