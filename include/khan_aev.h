@@ -442,6 +442,27 @@ typedef struct khan_net_few {
 int32_t khan_net_few_fits(const int32_t *widths, int32_t layers);
 int khan_net_few_f64(const khan_net_few *net, khan_stream_t stream);
 
+/* Whole networks with CELU in float32 for inference, all layers in one launch each way (a workgroup per 32 or 64 rows of a type).
+ * `layers` products of the widths `widths` (the last 1), w[l][t] [in, out] and b[l][t] of layer l and type t (b NULL: zeros).
+ * khan_net_chain_fits: 1 for widths it takes: the first a multiple of 128, the hidden ones up to 256.  x and grad must be 16-byte
+ * aligned.  Operands are split into three bfloat16 values: infinite ones give NaN.  A bit l of `absolute`: the CELU of hidden layer
+ * l is formed as alpha (exp(z / alpha) - 1), with an absolute error of 2^-24 alpha (KHAN_NET_CELU_ABSOLUTE).
+ * khan_net_chain_values_f32 packs the weights into `workspace` (khan_net_chain_workspace_bytes(), 16-byte aligned) and forms value;
+ * with want_rows the workspace then holds what khan_net_chain_rows_f32 needs: grad[t][r, :] = scale[t][r] d value[t][r] / d x[t][r, :]
+ * (scale[t] NULL: ones), added to what grad holds with `accumulate`.  The structure is the same for both, apart from value, scale and
+ * grad. */
+typedef struct khan_net_chain {
+    const void *x[4], *w[KHAN_NET_MAX_LAYERS][4], *b[KHAN_NET_MAX_LAYERS][4], *scale[4];
+    void *value[4], *grad[4], *workspace;
+    int32_t n[4], layers, widths[KHAN_NET_MAX_LAYERS + 1], want_rows, accumulate;
+    uint32_t absolute;
+    double alpha;
+} khan_net_chain;
+int32_t khan_net_chain_fits(const int32_t *widths, int32_t layers);
+int64_t khan_net_chain_workspace_bytes(const khan_net_chain *net);
+int khan_net_chain_values_f32(const khan_net_chain *net, khan_stream_t stream);
+int khan_net_chain_rows_f32(const khan_net_chain *net, khan_stream_t stream);
+
 /* Per-molecule sums of the atomic networks' outputs: e[m] = sum over the atoms g of molecule m of
  * out_{as[g]}[sis[g]] -- the gather to the batch's atom order and the segment sum by molecule of the reference
  * (khan/model/nn.py:165-177; trainer_multi_tower.py:350) in one launch, without the gathered copy, each molecule's

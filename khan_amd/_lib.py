@@ -94,6 +94,10 @@ _SIGNATURES = {
     "khan_net_grads_workspace_bytes_f64": (ctypes.c_int64, [_ptr]),
     "khan_net_few_fits": (ctypes.c_int32, [ctypes.POINTER(ctypes.c_int32), ctypes.c_int32]),
     "khan_net_few_f64": (ctypes.c_int, [_ptr, _ptr]),
+    "khan_net_chain_fits": (ctypes.c_int32, [ctypes.POINTER(ctypes.c_int32), ctypes.c_int32]),
+    "khan_net_chain_workspace_bytes": (ctypes.c_int64, [_ptr]),
+    "khan_net_chain_values_f32": (ctypes.c_int, [_ptr, _ptr]),
+    "khan_net_chain_rows_f32": (ctypes.c_int, [_ptr, _ptr]),
     "khan_net_grads_f32": (ctypes.c_int, [_ptr, _ptr]),
     "khan_net_grads_f64": (ctypes.c_int, [_ptr, _ptr]),
     "khan_mol_energy_f32": (ctypes.c_int, [ctypes.POINTER(_ptr)] + [_ptr] * 4 + [ctypes.c_int32, _ptr, _ptr]),

@@ -7,6 +7,7 @@
 #include "../../include/khan_aev.h"
 #include "khan_internal.h"
 #include "khan_params.h"
+#include "net_chain.h"
 #include "net_few.h"
 #include "net_layers.h"
 
@@ -447,6 +448,33 @@ static int ani_charges_begun(const T* xs, const T* ys, const T* zs, const T* qs,
 }
 
 // The per-type networks layer by layer (khan_net_*): the caller's structures, typed.
+static int net_chain_of(const khan_net_chain* net, khan::NetChain& a)
+{
+    static_assert(KHAN_NET_MAX_LAYERS == khan::kNetMaxLayers, "one limit");
+    if (!net || !khan_net_chain_fits(net->widths, net->layers) || !(net->alpha > 0.0)) return KHAN_ERR_INVALID_ARG;
+    a = {};
+    a.hidden = net->layers - 1;
+    a.alpha = static_cast<float>(net->alpha);
+    a.absolute = net->absolute;
+    a.want_rows = net->want_rows != 0;
+    for (int l = 0; l <= net->layers; ++l) a.widths[l] = net->widths[l];
+    int64_t rows = 0;
+    for (int t = 0; t < 4; ++t) {
+        if (net->n[t] < 0) return KHAN_ERR_INVALID_ARG;
+        a.n[t] = net->n[t];
+        rows += net->n[t];
+        if (net->n[t] == 0) continue;
+        a.x[t] = static_cast<const float*>(net->x[t]);
+        if (!a.x[t] || (reinterpret_cast<uintptr_t>(a.x[t]) & 15u)) return KHAN_ERR_INVALID_ARG;
+        for (int l = 0; l < net->layers; ++l) {
+            a.w[l][t] = static_cast<const float*>(net->w[l][t]);
+            a.b[l][t] = static_cast<const float*>(net->b[l][t]);
+            if (!a.w[l][t]) return KHAN_ERR_INVALID_ARG;
+        }
+    }
+    return rows > INT32_MAX ? KHAN_ERR_TOO_LARGE : KHAN_OK;
+}
+
 template <typename T>
 static int net_layer_impl(const khan_net_layer* l, khan_stream_t stream)
 {
@@ -998,6 +1026,43 @@ int khan_net_few_f64(const khan_net_few* net, khan_stream_t stream)
     if (with_grad != 0 && with_grad != with_rows) return KHAN_ERR_INVALID_ARG;
     if (rows > INT32_MAX) return KHAN_ERR_TOO_LARGE;
     return hip_status(khan::launch_net_few(a, as_stream(stream)));
+}
+int32_t khan_net_chain_fits(const int32_t* widths, int32_t layers)
+{
+    return widths && layers >= 2 && layers <= KHAN_NET_MAX_LAYERS && widths[layers] == 1 && khan::net_chain_fits(widths, layers - 1) ? 1 : 0;
+}
+int64_t khan_net_chain_workspace_bytes(const khan_net_chain* net)
+{
+    khan::NetChain a;
+    return net_chain_of(net, a) == KHAN_OK ? static_cast<int64_t>(khan::net_chain_workspace(a)) : 0;
+}
+int khan_net_chain_values_f32(const khan_net_chain* net, khan_stream_t stream)
+{
+    khan::NetChain a;
+    const int st = net_chain_of(net, a);
+    if (st != KHAN_OK) return st;
+    if (!net->workspace || (reinterpret_cast<uintptr_t>(net->workspace) & 15u)) return KHAN_ERR_INVALID_ARG;
+    float* value[4];
+    for (int t = 0; t < 4; ++t) {
+        value[t] = static_cast<float*>(net->value[t]);
+        if (a.n[t] > 0 && !value[t]) return KHAN_ERR_INVALID_ARG;
+    }
+    return hip_status(khan::launch_net_chain_values(a, net->workspace, value, as_stream(stream)));
+}
+int khan_net_chain_rows_f32(const khan_net_chain* net, khan_stream_t stream)
+{
+    khan::NetChain a;
+    const int st = net_chain_of(net, a);
+    if (st != KHAN_OK) return st;
+    if (!net->workspace || !net->want_rows || (reinterpret_cast<uintptr_t>(net->workspace) & 15u)) return KHAN_ERR_INVALID_ARG;
+    const float* scale[4];
+    float* grad[4];
+    for (int t = 0; t < 4; ++t) {
+        scale[t] = static_cast<const float*>(net->scale[t]);
+        grad[t] = static_cast<float*>(net->grad[t]);
+        if (a.n[t] > 0 && (!grad[t] || (reinterpret_cast<uintptr_t>(grad[t]) & 15u))) return KHAN_ERR_INVALID_ARG;
+    }
+    return hip_status(khan::launch_net_chain_rows(a, net->workspace, scale, grad, net->accumulate != 0, as_stream(stream)));
 }
 int khan_net_grads_f32(const khan_net_grads* grads, khan_stream_t stream) { return net_grads_impl<float>(grads, stream); }
 int khan_net_grads_f64(const khan_net_grads* grads, khan_stream_t stream) { return net_grads_impl<double>(grads, stream); }

@@ -766,6 +766,7 @@ struct Inference {
     Tensor values;                          // of all rows, type by type
     variable_list state;                    // activations and d_L; in the one-launch forms the rows' gradients
     bool few = false;                       // float64 in one launch (net_few.hip): see take_few
+    bool chain = false;                     // float32, a launch each way (net_chain.hip): see take_chain; state: its workspace
 
     Inference(const Weights& w_, const Four& x)
         : w(w_), rows(rows_of(w.net, w.params, x[0], x[1], x[2], x[3])), pass{w.net, rows, w.params},
@@ -814,6 +815,47 @@ struct Inference {
         return grads;
     }
 
+    // Float32 networks layer by layer otherwise: of hidden widths up to 256.
+    void take_chain()
+    {
+        if (w.params.dtype != at::kFloat || one_launch()) return;
+        const khan_net_chain a = chain_net(false);
+        uintptr_t bits = 0;
+        for (int t = 0; t < 4; ++t) bits |= reinterpret_cast<uintptr_t>(a.x[t]);
+        chain = rows.total > 0 && (bits & 15u) == 0 && api.khan_net_chain_fits(a.widths, a.layers);
+    }
+    khan_net_chain chain_net(bool want_rows) const
+    {
+        khan_net_chain a = {};
+        a.layers = w.net.layers();
+        a.alpha = w.net.alpha;
+        a.want_rows = want_rows;
+        for (size_t k = 0; k < w.net.widths.size(); ++k) a.widths[k] = static_cast<int32_t>(w.net.widths[k]);
+        bool leading = true;                // (the CELU of Pass::forward)
+        for (int l = 0; l < a.layers; ++l) {
+            leading = leading && l + 1 < a.layers && a.widths[l] % 32 == 0 && a.widths[l + 1] % 64 == 0;
+            if (leading) a.absolute |= 1u << l;
+            for (int t = 0; t < 4; ++t) {
+                a.w[l][t] = w.params.weight(l, t);
+                a.b[l][t] = w.params.bias(l, t);
+            }
+        }
+        for (int t = 0; t < 4; ++t) {
+            a.n[t] = static_cast<int32_t>(rows.n[t]);
+            a.x[t] = rows.n[t] > 0 ? rows.x[t].data_ptr() : nullptr;
+            a.value[t] = pass.part(values, 1, t);
+        }
+        return a;
+    }
+    Tensor launch_chain(bool want_rows)
+    {
+        khan_net_chain a = chain_net(want_rows);
+        const Tensor workspace = at::empty({api.khan_net_chain_workspace_bytes(&a)}, w.params.options.dtype(at::kByte));
+        a.workspace = workspace.data_ptr();
+        call(api.khan_net_chain_values_f32, static_cast<const khan_net_chain*>(&a), pass.st);
+        return workspace;
+    }
+
     Tensor launch(bool want_rows)
     {
         const Tensor grads = want_rows ? at::empty({rows.total * kFeats}, w.params.options) : Tensor();
@@ -842,6 +884,8 @@ struct Inference {
             state = {launch(want_rows)};
         } else if (few) {
             state = {launch_few(want_rows)};
+        } else if (chain) {
+            state = {launch_chain(want_rows)};
         } else {
             state = pass.forward(!exact);
             state.push_back(pass.top(state.back(), &v, want_rows));
@@ -859,6 +903,18 @@ struct Inference {
         }
         const bool add = into.defined();
         if (!add) into = at::empty({rows.total * w.net.widths[0]}, w.params.options);
+        if (chain) {
+            khan_net_chain a = chain_net(true);
+            a.workspace = state[0].data_ptr();
+            a.accumulate = add;
+            const Four out = by_type(rows, into, w.net.widths[0]);
+            for (int t = 0; t < 4; ++t) {
+                a.scale[t] = scale[t].defined() && rows.n[t] > 0 ? scale[t].data_ptr() : nullptr;
+                a.grad[t] = rows.n[t] > 0 ? out[t].data_ptr() : nullptr;
+            }
+            call(api.khan_net_chain_rows_f32, static_cast<const khan_net_chain*>(&a), pass.st);
+            return into;
+        }
         const variable_list d = pass.slopes(variable_list(state.begin(), state.end() - 1), state.back());
         pass.to_rows(d[0], scale, by_type(rows, into, w.net.widths[0]), add);
         return into;
@@ -944,6 +1000,7 @@ std::vector<Tensor> infer(const Tensor& xs, const Tensor& ys, const Tensor& zs, 
     same_size(charge.is_none() || !near_w.packed.defined(), "networks beside a charge network run layer by layer");
     Inference near_net(near_w, feats);
     near_net.take_few();
+    near_net.take_chain();
     run_mol_energy(near_net.forward(need_grad), as, sis, mos, macs, out[0]);
     if (charge.is_none()) {
         if (need_grad) run_featurize_grad(in, args, by_type(near_net.rows, near_net.gradients({}, Tensor()), kFeats), {out[1], out[2], out[3]});
@@ -953,6 +1010,7 @@ std::vector<Tensor> infer(const Tensor& xs, const Tensor& ys, const Tensor& zs, 
     same_size(!charge_w.packed.defined(), "a charge network runs layer by layer");
     Inference charge_net(charge_w, feats);
     if (!need_grad) charge_net.take_few();
+    charge_net.take_chain();
     charge_net.forward(need_grad);
     const Tensor qs = charge_net.values.index_select(0, gather);
     if (!need_grad) {

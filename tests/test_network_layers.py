@@ -478,6 +478,92 @@ def test_float64_networks_in_one_launch(rows):
     assert lib.khan_net_few_fits(widths_c, 4) == 0
 
 
+class _Chain(ctypes.Structure):
+    _fields_ = ([("x", ctypes.c_void_p * 4), ("w", ctypes.c_void_p * 4 * 12), ("b", ctypes.c_void_p * 4 * 12)] +
+                [(name, ctypes.c_void_p * 4) for name in ("scale", "value", "grad")] + [("workspace", ctypes.c_void_p), ("n", ctypes.c_int32 * 4), ("layers", ctypes.c_int32),
+                 ("widths", ctypes.c_int32 * 13), ("want_rows", ctypes.c_int32), ("accumulate", ctypes.c_int32), ("absolute", ctypes.c_uint32), ("alpha", ctypes.c_double)])
+
+
+# Float32 networks in a launch each way: rows around the 32 and the 64 of a workgroup, either form (64 rows: with four wavefronts
+# 262 tiles of them, with eight 144), an empty type; four wavefronts and eight, widths on and off the padding to 64, layers so narrow
+# that two wavefronts share their columns, one hidden layer and eleven, row gradients of one and of more passes over a workgroup's
+# columns.  A layer's sums are within 2e-6 of their products' sizes (as for single layers), and the weights are drawn to keep the
+# sizes, so that a value is within 2e-6 of the largest a layer; a slope takes its activation's error over alpha, and
+# the way back adds that of as many layers again.
+@pytest.mark.parametrize("rows", [(0, 1, 31, 33), (32, 63, 64, 65), (16500, 33, 0, 129), (9001, 65, 0, 31)])
+@pytest.mark.parametrize("widths", [(384, 128, 128, 64, 1), (128, 5, 1), (384, 256, 256, 200, 8, 1), (256, 129, 64, 1), (384,) + (64,) * 10 + (70, 1)])
+def test_float32_networks_in_one_launch_each_way(widths, rows):
+    from khan_amd import _lib
+    lib = _lib.load()
+    print("case:", widths, rows, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device="cuda")
+    layers, alpha, st = len(widths) - 1, 0.5, torch.cuda.current_stream().cuda_stream
+    x, scale, start = [rand(n, widths[0]) for n in rows], [rand(n) for n in rows], [rand(n + 1, widths[0]) for n in rows]
+    w, b = [[rand(k, m) * k ** -0.5 for _ in rows] for k, m in zip(widths, widths[1:])], [[rand(m) * 0.1 for _ in rows] for m in widths[1:]]
+
+    def run(x, want_rows, plain=False):
+        a = _Chain(layers=layers, want_rows=want_rows, accumulate=not plain, alpha=alpha, absolute=1)
+        values, grads = [torch.full((n + 1,), 7.0, device="cuda") for n in rows], [g.clone() for g in start]
+        for i, k in enumerate(widths):
+            a.widths[i] = k
+        for t, n in enumerate(rows):
+            a.n[t], a.x[t], a.value[t], a.grad[t] = n, x[t].data_ptr(), values[t].data_ptr(), grads[t].data_ptr()
+            a.scale[t] = None if plain else scale[t].data_ptr()
+            for l in range(layers):
+                a.w[l][t] = w[l][t].data_ptr()
+                a.b[l][t] = None if l == 0 and t == 1 else b[l][t].data_ptr()
+        size = lib.khan_net_chain_workspace_bytes(ctypes.byref(a))
+        workspace = torch.full((size + 64,), 255, dtype=torch.uint8, device="cuda")      # NaN wherever it is read before it is written
+        a.workspace = workspace.data_ptr()
+        assert lib.khan_net_chain_values_f32(ctypes.byref(a), st) == 0
+        if want_rows:
+            assert lib.khan_net_chain_rows_f32(ctypes.byref(a), st) == 0
+        else:
+            assert lib.khan_net_chain_rows_f32(ctypes.byref(a), st) != 0
+        assert all((v[-1] == 7).item() and torch.equal(g[-1], s[-1]) for v, g, s in zip(values, grads, start)) and (workspace[size:] == 255).all()
+        return [v[:-1] for v in values], [g[:-1] for g in grads]
+
+    want, want_grad = [], []
+    for t in range(4):
+        leaf = x[t].double().requires_grad_(True)
+        h = leaf
+        for l in range(layers):
+            h = h @ w[l][t].double() + (0.0 if l == 0 and t == 1 else b[l][t].double())
+            if l + 1 < layers:
+                h = torch.nn.functional.celu(h, alpha)
+        want.append(h.detach().reshape(-1))
+        want_grad.append(torch.autograd.grad(h.sum(), leaf)[0])
+    tol = 2e-6 * layers
+
+    def close(got, ref, tol):
+        off = max(((g.double() - r).abs().max().item() if r.numel() else 0.0) for g, r in zip(got, ref))
+        size = max(r.abs().max().item() for r in ref if r.numel())
+        assert off <= tol * size, (off, size)
+    values, grads = run(x, True)
+    close(values, want, tol)
+    close([g - s[:-1] for g, s in zip(grads, start)], [g * c.double()[:, None] for g, c in zip(want_grad, scale)], tol * (1 + 1 / alpha) + 1e-6)
+    close(run(x, True, plain=True)[1], want_grad, tol * (1 + 1 / alpha))
+    assert all(map(torch.equal, run(x, False)[0], values))
+    # a row that is not a number stays alone
+    big = rows.index(max(rows))
+    spoilt = [t.clone() for t in x]
+    spoilt[big][rows[big] // 2, 11] = float("nan")
+    other_values, other_grads = run(spoilt, True)
+    others = torch.arange(rows[big], device="cuda") != rows[big] // 2
+    assert torch.isnan(other_values[big][~others]).all() and torch.isnan(other_grads[big][~others]).all()
+    assert torch.equal(values[big][others], other_values[big][others]) and torch.equal(grads[big][others], other_grads[big][others])
+
+
+def test_networks_that_one_launch_does_not_take():
+    """Feature widths off 128, hidden layers wider than 256, more than eleven of them or none, an output that is no single value."""
+    from khan_amd import _lib
+    lib = _lib.load()
+    fits = lambda *widths: lib.khan_net_chain_fits((ctypes.c_int32 * 16)(*widths), len(widths) - 1)
+    assert fits(384, 256, 1) and fits(128, *[8] * 11, 1)
+    assert not any((fits(96, 64, 1), fits(0, 64, 1), fits(384, 257, 1), fits(384, 0, 1), fits(128, *[8] * 12, 1), fits(384, 1), fits(384, 64, 2)))
+
+
 @pytest.mark.parametrize("layers,live", [((256, 64, 8, 1), 2), ((128, 128, 1), 2), ((128, 64, 1), 3), ((100, 1), 0)])
 def test_parameters_behind_the_constant_layers_have_gradients(layers, live):
     """Without `weights_need_grad` the leading layers of a float32 network are constants and those behind them are not: their
