@@ -3,28 +3,32 @@
 // With the names of net_layers.hip, a_l = celu(a_{l-1} W_l + b_l), value = a_L w + b; d_L = w celu'(a_L), d_{l-1} = (d_l W_l^T)
 // celu'(a_{l-1}), row gradient = s d_1 W_1^T.
 //
-// The products are those of layer_split_kernel (net_layers.hip): every operand the exact sum of three bfloat16 values, the six
-// largest of the nine partial products accumulated in float32, the five small ones in accumulators of their own.  What differs is
-// where the operands come from.  Layer by layer, the tiles of a launch run side by side, first all waiting for their rows, then
-// all multiplying, then all storing: 43-49 us for 47,000 rows 256 -> 256, of which the products need 19.  Here a workgroup takes 64 (or
-// 32) rows through all layers: the rows of the next product are split once, by the lanes that have just formed them, into three planes
-// in LDS (98 KB for 64 rows of 256), and the weights, split and packed beforehand by a launch of their own, go from memory straight to
+// The products are made of half-precision ones (split_half.h, dense_fused.hip): every operand as the sum of two half-precision values,
+// three of the four partial products accumulated in float32, the two small ones in an accumulator of their own.  Half precision has
+// no room for float32's exponents, so a row's operand is scaled by the power of two that brings its largest value to 2^14, and so is each
+// column of the weights: what is within 2^-28 of its row's (column's) largest value keeps all its bits, what is smaller an error of
+// 2^-52 of that value.  The three-way bfloat16 split needs six products: deep networks with charges on 4,001 organic molecules
+// 1,527 us so and 1,266 like this, deep ones alone on 100 molecules 182 and 164, default ones with charges on 16,384 1,264 and 1,226.
+// Relative errors against float64 of energies and gradients of the first of these, layer by layer on the bfloat16 split
+// 4.5e-7 and 1.28e-6, in one launch on it 2.8e-7 and 8.2e-7, like this 2.9e-7 and 9.2e-7 (of default networks with charges on 3,000:
+// 4.0e-7 and 8.3e-7, 3.3e-7 and 6.9e-7, 3.3e-7 and 7.4e-7; boxes with deep ones 9.9e-7 and 10.5e-7, 7.2e-7 and 7.4e-7, 5.3e-7 and 8.2e-7).
+//
+// Layer by layer, the tiles of a launch run side by side, first all waiting for their rows, then
+// all multiplying, then all storing.  Here a workgroup takes 64 (or
+// 32) rows through all layers: the rows of the next product are split once, by the lanes that have just formed them, into two planes
+// in LDS (66 KB for 64 rows of 256), and the weights, split and packed beforehand by a launch of their own, go from memory straight to
 // registers, four chunks of 16 k ahead, across the ends of the layers.  A wavefront takes 32 columns of all 64 rows (of 32 where the layer
 // is so narrow that its columns would leave wavefronts idle), so that no two of a workgroup load the same weights.
 // The weights are the matrix instruction's first operand and the rows its second: a lane has one row and, with the columns packed in a
 // suitable order, twice eight neighbouring columns of it, which go to the planes 16 bytes at a time.  The activations that the
 // way back needs go to memory in the order in which the lanes hold them, a kilobyte at a time, and come back the same way.
 // Widths are padded to multiples of 64 with weights and biases of zero.
-// Measured, inference with gradients against layer by layer: deep networks (seven layers of 256, 128, 64 and 8 on 384) and a charge network
-// on 4,001 organic molecules (47,000 atoms) 1,734 -> 1,564 us, the networks alone 100 molecules 184 -> 155; default networks
-// (128 128 64) with charges on 16,384 molecules 1,367 -> 1,213, on 256 167 -> 148.  The matrix instructions take two fifths of the time of the
-// compute units in use (504 of 755 us for the 47,000 rows with the barriers, the activations' way through memory 125, splitting and CELU the rest).
 #include <algorithm>
 
 #include "khan_internal.h"
 #include "net_chain.h"
 #include "net_celu.h"
-#include "split_bf16.h"
+#include "split_half.h"
 
 namespace khan {
 
@@ -33,19 +37,22 @@ namespace {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f4v __attribute__((ext_vector_type(4)));
 
-constexpr int kChunkBytes = 3 * 1024;        // packed weights of 16 k x 32 columns: [part][lane][8 k]
+constexpr int kParts = 2;                    // half-precision values that an operand is split into
+constexpr int kChunkBytes = kParts * 1024;   // packed weights of 16 k x 32 columns: [part][lane][8 k]
 constexpr int kRing = 4;                     // chunks of weights on their way
 constexpr int kWaitLoads = 0x0f70;           // s_waitcnt vmcnt(0)
 
 struct ChainProduct {
     int64_t at;                  // packed weights of type 0: [type][32 columns][16 k]
     int blocks, chunks;          // 32 columns, 16 k; multiples of 2 and 4
+    int back_at;                 // 2^(15 - shift) of the columns of type 0: [type][column]
 };
 struct ChainArgs {
     const float* x[4];
     int n[4], tile_end[4];
     const char* packed;
     const float* fixed;          // per type: the hidden layers' biases one after the other, the output layer's weights, its bias
+    const float* backs;
     ChainProduct p[kNetMaxLayers];       // the pass's products in its order
     float* act[kNetMaxLayers];           // activations of the hidden layers, or null: [tile][32 columns][32 rows][half a column block][lane][8]
     int act_blocks[kNetMaxLayers];       // their padded widths / 32
@@ -67,10 +74,22 @@ __device__ __forceinline__ int column_of(int matrix_row)
     return 16 * (q >> 1) + 8 * half + 4 * (q & 1) + (matrix_row & 3);
 }
 
+// The power of two that brings a row's or a column's largest value (its bits: never negative) to between 2^14 and 2^15, as it
+// is multiplied by: rows, at most 2^111; columns, at least 2^-112 (from 2^128 (1 - 2^-11) on a weight becomes infinite, and NaN)
+__device__ __forceinline__ float row_scale(unsigned largest) { return __uint_as_float((268u - max(largest >> 23, 30u)) << 23); }
+__device__ __forceinline__ float column_scale(unsigned largest) { return __uint_as_float((268u - min(max(largest >> 23, 15u), 253u)) << 23); }
+// what brings a sum of their products back is the product of the two inverses, a factor of 2^15 moved from the row's to the column's
+// so that neither the factors nor the sum between them leave float32's range before row and product do
+__device__ __forceinline__ float row_back(unsigned largest) { return __uint_as_float((max(largest >> 23, 30u) - 29u) << 23); }
+__device__ __forceinline__ float column_back(unsigned largest) { return __uint_as_float((min(max(largest >> 23, 15u), 253u) + 1u) << 23); }
+
 template <int kWaves, int kRB>
 struct ChainLds {
     static constexpr int kRows = 32 * kRB;
-    u4v planes[3][4 * kWaves][kRows + 1];        // [part][8 columns][row]
+    u4v planes[kParts][4 * kWaves][kRows + 1];   // [part][8 columns][row]
+    // the rows' largest values, as they come from products 0, 1, 2, 0, ...: of the operand in the planes, of the one that is being made,
+    // and zeros for the one after
+    unsigned largest[3][kRows];
     float sums[kWaves][kRows];
     float fixed[kNetMaxLayers * 32 * kWaves + 4];        // the type's biases and output layer
 };
@@ -79,11 +98,11 @@ struct Lane {
     int lane, wave, l32, half;
 };
 struct Ring {
-    u4v part[kRing][3];
+    u4v part[kRing][kParts];
     __device__ __forceinline__ void load(int u, const char* chunk, unsigned lane16)
     {
 #pragma unroll
-        for (int m = 0; m < 3; ++m) part[u][m] = *reinterpret_cast<const u4v*>(chunk + m * 1024 + lane16);
+        for (int m = 0; m < kParts; ++m) part[u][m] = *reinterpret_cast<const u4v*>(chunk + m * 1024 + lane16);
     }
     __device__ __forceinline__ void start(const char* weights, unsigned lane16)
     {
@@ -110,34 +129,31 @@ __device__ __forceinline__ Share share_of(int wave, int blocks)
     return {min(wave, blocks - 1), 0, wave < blocks};
 }
 
-// acc, small += the planes' columns from 8 first8 on (16 `chunks` of them) times the weights from `weights` on, whose first kRing chunks
+// acc + 2^-11 low += the planes' columns from 8 first8 on (16 `chunks` of them) times the weights from `weights` on, whose first kRing chunks
 // are in the ring; `next`: the weights that come after these
 template <int kWaves, int kRB, int RB>
 __device__ __forceinline__ void multiply(const ChainLds<kWaves, kRB>& S, const Lane& P, int first8, int rb0, int chunks, const char* weights, const char* next,
-                                         Ring& ring, f32x16 (&acc)[RB], f32x16 (&small)[RB])
+                                         Ring& ring, f32x16 (&acc)[RB], f32x16 (&low)[RB])
 {
     const unsigned lane16 = P.lane * 16;
     const auto group = [&](int c) {
         const char* const ahead = c + kRing < chunks ? weights + (c + kRing) * kChunkBytes : next;
 #pragma unroll
         for (int u = 0; u < kRing; ++u) {
-            bf16x8 x[RB][3], w[3];
+            h8v x[RB][kParts], w[kParts];
 #pragma unroll
             for (int j = 0; j < RB; ++j)
 #pragma unroll
-                for (int m = 0; m < 3; ++m) x[j][m] = __builtin_bit_cast(bf16x8, S.planes[m][first8 + 2 * (c + u) + P.half][32 * (rb0 + j) + P.l32]);
+                for (int m = 0; m < kParts; ++m) x[j][m] = __builtin_bit_cast(h8v, S.planes[m][first8 + 2 * (c + u) + P.half][32 * (rb0 + j) + P.l32]);
 #pragma unroll
-            for (int m = 0; m < 3; ++m) w[m] = __builtin_bit_cast(bf16x8, ring.part[u][m]);
+            for (int m = 0; m < kParts; ++m) w[m] = __builtin_bit_cast(h8v, ring.part[u][m]);
             const auto mul = [&](f32x16 (&to)[RB], int xi, int wi) {
 #pragma unroll
-                for (int j = 0; j < RB; ++j) to[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w[wi], x[j][xi], to[j], 0, 0, 0);
+                for (int j = 0; j < RB; ++j) to[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(w[wi], x[j][xi], to[j], 0, 0, 0);
             };
-            mul(small, 0, 2);
+            mul(low, 1, 0);
             mul(acc, 0, 0);
-            mul(small, 1, 1);
-            mul(small, 2, 0);
-            mul(small, 0, 1);
-            mul(small, 1, 0);
+            mul(low, 0, 1);
             ring.load(u, ahead + u * kChunkBytes, lane16);
             // the loads stay behind the chunk's products (vector, scalar and LDS instructions may pass): the compiler would gather
             // them behind the last one
@@ -150,24 +166,38 @@ __device__ __forceinline__ void multiply(const ChainLds<kWaves, kRB>& S, const L
     for (int c = kRing; c < chunks; c += kRing) group(c);
 }
 
-// a lane's values of a layer -> the planes, split
+// the largest of a lane's values of a layer, to those of their rows
 template <int kWaves, int kRB, int RB>
-__device__ __forceinline__ void to_planes(ChainLds<kWaves, kRB>& S, const Lane& P, int cb, int rb0, const f32x16 (&y)[RB])
+__device__ __forceinline__ void note_largest(ChainLds<kWaves, kRB>& S, const Lane& P, int product, int rb0, const f32x16 (&y)[RB])
 {
 #pragma unroll
-    for (int j = 0; j < RB; ++j)
+    for (int j = 0; j < RB; ++j) {
+        float m[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int v = 0; v < 16; ++v) m[v & 3] = fmaxf(m[v & 3], fabsf(y[j][v]));
+        atomicMax(&S.largest[product % 3][32 * (rb0 + j) + P.l32], __float_as_uint(fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3]))));
+    }
+}
+// a lane's values of a layer -> the planes, scaled and split
+template <int kWaves, int kRB, int RB>
+__device__ __forceinline__ void to_planes(ChainLds<kWaves, kRB>& S, const Lane& P, int product, int cb, int rb0, const f32x16 (&y)[RB])
+{
+#pragma unroll
+    for (int j = 0; j < RB; ++j) {
+        const float scale = row_scale(S.largest[product % 3][32 * (rb0 + j) + P.l32]);
 #pragma unroll
         for (int g = 0; g < 2; ++g) {
-            u4v p[3];
+            u4v p[kParts];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                unsigned q[3];
-                split_pair(y[j][8 * g + 2 * e], y[j][8 * g + 2 * e + 1], q[0], q[1], q[2]);
-                p[0][e] = q[0], p[1][e] = q[1], p[2][e] = q[2];
+                unsigned q[kParts];
+                split_pair(y[j][8 * g + 2 * e] * scale, y[j][8 * g + 2 * e + 1] * scale, q[0], q[1]);
+                p[0][e] = q[0], p[1][e] = q[1];
             }
 #pragma unroll
-            for (int m = 0; m < 3; ++m) S.planes[m][4 * cb + 2 * g + P.half][32 * (rb0 + j) + P.l32] = p[m];
+            for (int m = 0; m < kParts; ++m) S.planes[m][4 * cb + 2 * g + P.half][32 * (rb0 + j) + P.l32] = p[m];
         }
+    }
 }
 
 template <int RB>
@@ -190,7 +220,7 @@ __device__ __forceinline__ void store_block(float* block, const Lane& P, const f
     for (int q = 0; q < 4; ++q)
         *reinterpret_cast<f4v*>(block + (q >> 1) * 512 + P.lane * 8 + (q & 1) * 4) = f4v{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
 }
-// a lane's sixteen columns of a vector over the layer's columns (LDS)
+// a lane's sixteen columns of a vector over the layer's columns
 __device__ __forceinline__ f32x16 of_columns(const float* from, const Lane& P, int cb)
 {
     f32x16 v;
@@ -204,8 +234,8 @@ __device__ __forceinline__ f32x16 of_columns(const float* from, const Lane& P, i
 }
 __device__ __forceinline__ float slope_of(float a, float inv_alpha) { return a >= 0.f ? 1.f : fmaf(a, inv_alpha, 1.f); }
 
-// wavefronts per SIMD: one workgroup of eight wavefronts with 64 rows of 256 (114 KB) on a compute unit or two of four with 64 of 128
-// (57 KB; three would have 168 registers, 100 too few), and with 32 rows two and four
+// wavefronts per SIMD: one workgroup of eight wavefronts with 64 rows of 256 on a compute unit or two of four with 64 of 128
+// (three would have 168 registers, 40 too few), and with 32 rows two and four
 constexpr int chain_waves(int, int rb) { return rb == 2 ? 2 : 4; }
 
 template <int kWaves, int kRB, bool kBack>
@@ -230,9 +260,11 @@ void chain_kernel(const ChainArgs a)
     };
     Ring ring;
     ring.start(weights_of(a.p[0], share_of<kWaves, kRB>(P.wave, min(a.p[0].blocks, kWaves)).cb), lane16);
+    for (int i = tid; i < 3 * kRows; i += kThreads) S.largest[0][i] = 0u;
     for (int i = tid; i < a.fixed_size; i += kThreads) fixed[i] = a.fixed[static_cast<size_t>(t) * a.fixed_size + i];
 
-    // product l, column blocks from `cb0` on, in one of the two shares; `before(multiply)` may call it more than once
+    // product l, column blocks from `cb0` on, in one of the two shares; `operands(multiply)` may call it more than once.  `finish` has the
+    // sums but for the columns' factors.
     const auto run = [&](auto rb_count, int l, int cb0, auto&& before, auto&& operands, auto&& finish) {
         constexpr int RB = decltype(rb_count)::value;
         const ChainProduct& p = a.p[l];
@@ -242,26 +274,35 @@ void chain_kernel(const ChainArgs a)
         const char* next = weights;
         if (cb0 + kWaves < p.blocks) next = weights_of(p, cb0 + kWaves + share_of<kWaves, kRB>(P.wave, min(p.blocks - cb0 - kWaves, kWaves)).cb);
         else if (l + 1 < H) next = weights_of(a.p[l + 1], share_of<kWaves, kRB>(P.wave, min(a.p[l + 1].blocks, kWaves)).cb);
-        f32x16 acc[RB], small[RB];
+        f32x16 acc[RB], low[RB];
 #pragma unroll
-        for (int j = 0; j < RB; ++j) acc[j] = small[j] = f32x16(0.f);
+        for (int j = 0; j < RB; ++j) acc[j] = low[j] = f32x16(0.f);
+        const f32x16 back = of_columns(a.backs + p.back_at + 32 * (t * p.blocks + cb0), P, s.cb);
         auto met = before(rb_count, s);
         operands(p, s, [&](int first8, int first, int chunks) {
             if (s.active) {
                 const char* const from = weights + first * kChunkBytes;
-                multiply<kWaves, kRB, RB>(S, P, first8, s.rb0, chunks, from, first + chunks < p.chunks ? from + chunks * kChunkBytes : next, ring, acc, small);
+                multiply<kWaves, kRB, RB>(S, P, first8, s.rb0, chunks, from, first + chunks < p.chunks ? from + chunks * kChunkBytes : next, ring, acc, low);
             }
         });
         if (!s.active) ring.start(next, lane16);
 #pragma unroll
-        for (int j = 0; j < RB; ++j) acc[j] += small[j];
-        finish(rb_count, s, cb0, acc, met);
+        for (int j = 0; j < RB; ++j) {
+            const float rows_back = row_back(S.largest[l % 3][32 * (s.rb0 + j) + P.l32]);
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[j][v] = fmaf(low[j][v], kResidualBack, acc[j][v]) * rows_back;
+        }
+        finish(rb_count, s, cb0, acc, back, met);
     };
     const auto run_any = [&](int l, int cb0, auto&& before, auto&& operands, auto&& finish) {
         if constexpr (kRB == 2) {
             if (by_rows<kWaves, kRB>(min(a.p[l].blocks - cb0, kWaves))) return run(std::integral_constant<int, 1>(), l, cb0, before, operands, finish);
         }
         run(std::integral_constant<int, kRB>(), l, cb0, before, operands, finish);
+    };
+    // (product's place was last read as that of the operand of product - 3, which every wavefront is through with)
+    const auto clear_largest = [&](int product) {
+        if (tid < kRows) S.largest[product % 3][tid] = 0u;
     };
     const auto nothing = [](auto, const Share&) { return 0; };
     const auto from_planes = [&](const ChainProduct& p, const Share&, auto&& mul) { mul(0, 0, p.chunks); };
@@ -288,16 +329,33 @@ void chain_kernel(const ChainArgs a)
         const auto stage = [&](int i, int first8, const f4v (&x)[2]) {
             int row, k8;
             place(i, row, k8);
-            u4v p[3];
+            const float scale = row_scale(S.largest[0][row]);
+            u4v p[kParts];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                unsigned q[3];
-                split_pair(x[e >> 1][2 * (e & 1)], x[e >> 1][2 * (e & 1) + 1], q[0], q[1], q[2]);
-                p[0][e] = q[0], p[1][e] = q[1], p[2][e] = q[2];
+                unsigned q[kParts];
+                split_pair(x[e >> 1][2 * (e & 1)] * scale, x[e >> 1][2 * (e & 1) + 1] * scale, q[0], q[1]);
+                p[0][e] = q[0], p[1][e] = q[1];
             }
 #pragma unroll
-            for (int m = 0; m < 3; ++m) S.planes[m][first8 + k8][row] = p[m];
+            for (int m = 0; m < kParts; ++m) S.planes[m][first8 + k8][row] = p[m];
         };
+        // the rows' largest values before anything of them is split: a reading more, of which the second finds the lines in the L2
+        __syncthreads();
+#pragma unroll 3
+        for (int piece = 0; piece < (a.k0 + kPiece - 1) / kPiece; ++piece)
+#pragma unroll
+            for (int i = 0; i < kUnits; ++i) {
+                f4v x[2];
+                int row, k8;
+                place(i, row, k8);
+                fetch(i, piece, x);
+                float m = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(x[e >> 2][e & 3]));
+                atomicMax(&S.largest[0][row], __float_as_uint(m));
+            }
+        __syncthreads();
         const auto through_pieces = [&](const ChainProduct&, const Share&, auto&& mul) {
             if constexpr (kHeld) {
                 const int pieces = a.k0 / kPiece;
@@ -332,7 +390,7 @@ void chain_kernel(const ChainArgs a)
             }
         };
         const auto layer = [&](int l, auto&& operands) {
-            run_any(l, 0, nothing, operands, [&](auto rb_count, const Share& s, int, auto& y, int) {
+            run_any(l, 0, nothing, operands, [&](auto rb_count, const Share& s, int, auto& y, const f32x16& back, int) {
                 constexpr int RB = decltype(rb_count)::value;
                 if (s.active) {
                     const f32x16 bias = of_columns(fixed + a.fixed_at[l], P, s.cb);
@@ -341,17 +399,19 @@ void chain_kernel(const ChainArgs a)
                     for (int j = 0; j < RB; ++j) {
                         if (absolute) {
 #pragma unroll
-                            for (int v = 0; v < 16; ++v) y[j][v] = celu_absolute(y[j][v] + bias[v], a.alpha, a.inv_alpha);
+                            for (int v = 0; v < 16; ++v) y[j][v] = celu_absolute(fmaf(y[j][v], back[v], bias[v]), a.alpha, a.inv_alpha);
                         } else {
 #pragma unroll
-                            for (int v = 0; v < 16; ++v) y[j][v] = celu_exact(y[j][v] + bias[v], a.alpha, a.inv_alpha);
+                            for (int v = 0; v < 16; ++v) y[j][v] = celu_exact(fmaf(y[j][v], back[v], bias[v]), a.alpha, a.inv_alpha);
                         }
                     }
+                    if (l + 1 < H) note_largest<kWaves, kRB, RB>(S, P, l + 1, s.rb0, y);
                 }
-                __syncthreads();           // the planes have been read
+                clear_largest(l + 2);
+                __syncthreads();           // the planes have been read, the rows' largest values are there
                 if (s.active) {
                     if (l + 1 < H) {
-                        to_planes<kWaves, kRB, RB>(S, P, s.cb, s.rb0, y);
+                        to_planes<kWaves, kRB, RB>(S, P, l + 1, s.cb, s.rb0, y);
                     } else {
                         const f32x16 w = of_columns(fixed + a.fixed_at[H], P, s.cb);
 #pragma unroll
@@ -386,14 +446,23 @@ void chain_kernel(const ChainArgs a)
     } else {
         // ---- d_L = w celu'(a_L)
         __syncthreads();
-        for (int u = P.wave; u < a.act_blocks[H - 1] * kRB; u += kWaves) {
-            const int cb = u / kRB, rb = u - cb * kRB;
-            f32x16 y[1];
-            load_block(act_at(H - 1, cb, rb), P, y[0]);
+        f32x16 d[kRB][1];
+#pragma unroll
+        for (int i = 0; i < kRB; ++i) {
+            const int u = P.wave + i * kWaves, cb = u / kRB, rb = u - cb * kRB;
+            if (cb >= a.act_blocks[H - 1]) break;
+            load_block(act_at(H - 1, cb, rb), P, d[i][0]);
             const f32x16 w = of_columns(fixed + a.fixed_at[H], P, cb);
 #pragma unroll
-            for (int v = 0; v < 16; ++v) y[0][v] = w[v] * slope_of(y[0][v], a.inv_alpha);
-            to_planes<kWaves, kRB, 1>(S, P, cb, rb, y);
+            for (int v = 0; v < 16; ++v) d[i][0][v] = w[v] * slope_of(d[i][0][v], a.inv_alpha);
+            note_largest<kWaves, kRB, 1>(S, P, 0, rb, d[i]);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kRB; ++i) {
+            const int u = P.wave + i * kWaves, cb = u / kRB, rb = u - cb * kRB;
+            if (cb >= a.act_blocks[H - 1]) break;
+            to_planes<kWaves, kRB, 1>(S, P, 0, cb, rb, d[i]);
         }
         __syncthreads();
         // ---- d_{L-1} .. d_1
@@ -407,21 +476,23 @@ void chain_kernel(const ChainArgs a)
                 for (int j = 0; j < RB; ++j) load_block(act_at(h, s.cb, s.rb0 + j), P, act.v[j]);
                 return act;
             };
-            run_any(l, 0, activations, from_planes, [&](auto rb_count, const Share& s, int, auto& y, auto& act) {
+            run_any(l, 0, activations, from_planes, [&](auto rb_count, const Share& s, int, auto& y, const f32x16& back, auto& act) {
                 constexpr int RB = decltype(rb_count)::value;
 #pragma unroll
                 for (int j = 0; j < RB; ++j)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) y[j][v] *= slope_of(act.v[j][v], a.inv_alpha);
-                __syncthreads();           // the planes have been read
-                if (s.active) to_planes<kWaves, kRB, RB>(S, P, s.cb, s.rb0, y);
+                    for (int v = 0; v < 16; ++v) y[j][v] = y[j][v] * back[v] * slope_of(act.v[j][v], a.inv_alpha);
+                if (s.active) note_largest<kWaves, kRB, RB>(S, P, l + 1, s.rb0, y);
+                clear_largest(l + 2);
+                __syncthreads();           // the planes have been read, the rows' largest values are there
+                if (s.active) to_planes<kWaves, kRB, RB>(S, P, l + 1, s.cb, s.rb0, y);
                 __syncthreads();
             });
         }
         // ---- the rows
 #pragma unroll 1
         for (int cb0 = 0; cb0 < a.p[H - 1].blocks; cb0 += kWaves) {
-            run_any(H - 1, cb0, nothing, from_planes, [&](auto rb_count, const Share& s, int cb0, auto& y, int) {
+            run_any(H - 1, cb0, nothing, from_planes, [&](auto rb_count, const Share& s, int cb0, auto& y, const f32x16& back, int) {
                 constexpr int RB = decltype(rb_count)::value;
                 if (!s.active) return;
 #pragma unroll
@@ -433,7 +504,7 @@ void chain_kernel(const ChainArgs a)
 #pragma unroll
                     for (int q = 0; q < 4; ++q)
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) v[q][e] = y[j][4 * q + e] * scale;
+                        for (int e = 0; e < 4; ++e) v[q][e] = y[j][4 * q + e] * back[4 * q + e] * scale;
                     if (a.accumulate) {
 #pragma unroll
                         for (int q = 0; q < 4; ++q) v[q] += *reinterpret_cast<const f4v*>(out + 16 * (q >> 1) + 4 * (q & 1));
@@ -448,27 +519,32 @@ void chain_kernel(const ChainArgs a)
     }
 }
 
-// The weights of all products, split and in the order in which the lanes take them, and the padded biases; a wavefront per chunk.
+// The weights of all products, scaled by columns, split and in the order in which the lanes take them, and the padded biases; a workgroup
+// per 32 columns, which it holds between their largest values and the split where a column has no more than 512 (all loads are then on
+// their way at once).
+constexpr int kPackWaves = 8, kPackHeld = 4;         // chunks of a wavefront
 struct PackProduct {
     const float* w[4];           // [k, n_out] as stored, or [n_out, k] (back)
-    int k, n_out, blocks, chunks, end;       // end: running number of chunks of all types
+    int k, n_out, blocks, chunks, end;       // end: running number of column blocks of all types
     bool back;
     int64_t at;
+    int back_at;
 };
 struct PackArgs {
     PackProduct p[2 * kNetMaxLayers];
     const float *bias[kNetMaxLayers][4];
     int products, layers, widths[kNetMaxLayers + 1], fixed_at[kNetMaxLayers + 2], fixed_size;
     char* packed;
-    float* fixed;
+    float *fixed, *backs;
     const float* top[4];
 };
-__global__ __launch_bounds__(256) void chain_pack_kernel(const PackArgs a)
+__global__ __launch_bounds__(64 * kPackWaves) void chain_pack_kernel(const PackArgs a)
 {
-    const int lane = threadIdx.x & 63, number = static_cast<int>(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr int kThreads = 64 * kPackWaves;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), number = static_cast<int>(blockIdx.x);
     if (number >= a.p[a.products - 1].end) {
-        // behind the weights: the biases, 64 values to a wavefront
-        const int i = (number - a.p[a.products - 1].end) * 64 + lane, t = i / a.fixed_size, at = i - t * a.fixed_size;
+        // behind the weights: the biases, a value to a thread
+        const int i = (number - a.p[a.products - 1].end) * kThreads + static_cast<int>(threadIdx.x), t = i / a.fixed_size, at = i - t * a.fixed_size;
         if (t >= 4) return;
         float v = 0.f;
         const int H = a.layers - 1;
@@ -484,30 +560,74 @@ __global__ __launch_bounds__(256) void chain_pack_kernel(const PackArgs a)
         a.fixed[i] = v;
         return;
     }
+    __shared__ unsigned largest[32];
+    if (threadIdx.x < 32) largest[threadIdx.x] = 0u;
+    __syncthreads();
     int m = 0;
     while (number >= a.p[m].end) ++m;
     const PackProduct& p = a.p[m];
-    const int rel = number - (m == 0 ? 0 : a.p[m - 1].end), t = rel / (p.blocks * p.chunks), block = rel - t * p.blocks * p.chunks;
-    const int cb = block / p.chunks, chunk = block - cb * p.chunks;
-    const int col = 32 * cb + column_of(lane & 31), k0 = 16 * chunk + 8 * (lane >> 5);
+    const int rel = number - (m == 0 ? 0 : a.p[m - 1].end), t = rel / p.blocks, cb = rel - t * p.blocks;
+    const int col = 32 * cb + column_of(lane & 31);
     const float* const w = p.w[t];
-    float v[8];
+    const bool wide = p.back && p.k % 8 == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0;      // sixteen bytes at a time
+    float v[kPackHeld][8];
+    const auto fetch = [&](int first) {
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const bool inside = w && col < p.n_out && k0 + e < p.k;
-        const size_t at = p.back ? static_cast<size_t>(col) * p.k + k0 + e : static_cast<size_t>(k0 + e) * p.n_out + col;
-        v[e] = inside ? w[inside ? at : 0] : 0.f;
+        for (int i = 0; i < kPackHeld; ++i) {
+            const int k0 = 16 * (first + i * kPackWaves + wave) + 8 * (lane >> 5);
+            if (wide) {
+                const bool inside = w && col < p.n_out && k0 < p.k;          // (a type without rows has no weights)
+                const f4v* const from = reinterpret_cast<const f4v*>(w + static_cast<size_t>(col) * p.k + k0);
+#pragma unroll
+                for (int q = 0; q < 2; ++q) {
+                    const f4v x = inside ? from[q] : f4v(0.f);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[i][4 * q + e] = x[e];
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const bool inside = w && col < p.n_out && k0 + e < p.k;
+                    const size_t at = p.back ? static_cast<size_t>(col) * p.k + k0 + e : static_cast<size_t>(k0 + e) * p.n_out + col;
+                    v[i][e] = inside ? w[at] : 0.f;
+                }
+            }
+        }
+    };
+    constexpr int kGroup = kPackWaves * kPackHeld;
+    float most = 0.f;
+#pragma unroll 1
+    for (int first = 0; first < p.chunks; first += kGroup) {
+        fetch(first);
+#pragma unroll
+        for (int i = 0; i < kPackHeld; ++i)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) most = fmaxf(most, fabsf(v[i][e]));
     }
-    u4v part[3];
+    atomicMax(&largest[lane & 31], __float_as_uint(most));
+    __syncthreads();
+    const unsigned of_column = largest[lane & 31];
+    const float scale = column_scale(of_column);
+    if (wave == 0 && lane < 32) a.backs[p.back_at + 32 * rel + column_of(lane)] = column_back(of_column);
+#pragma unroll 1
+    for (int first = 0; first < p.chunks; first += kGroup) {
+        if (p.chunks > kGroup) fetch(first);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        unsigned q[3];
-        split_pair(v[2 * e], v[2 * e + 1], q[0], q[1], q[2]);
-        part[0][e] = q[0], part[1][e] = q[1], part[2][e] = q[2];
+        for (int i = 0; i < kPackHeld; ++i) {
+            const int c = first + i * kPackWaves + wave;
+            if (c >= p.chunks) break;
+            u4v part[kParts];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                unsigned q[kParts];
+                split_pair(v[i][2 * e] * scale, v[i][2 * e + 1] * scale, q[0], q[1]);
+                part[0][e] = q[0], part[1][e] = q[1];
+            }
+            char* const to = a.packed + p.at + (static_cast<int64_t>(rel) * p.chunks + c) * kChunkBytes + lane * 16;
+#pragma unroll
+            for (int q = 0; q < kParts; ++q) *reinterpret_cast<u4v*>(to + q * 1024) = part[q];
+        }
     }
-    char* const to = a.packed + p.at + static_cast<int64_t>(rel) * kChunkBytes + lane * 16;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) *reinterpret_cast<u4v*>(to + q * 1024) = part[q];
 }
 
 // ---- host
@@ -516,7 +636,7 @@ int padded(int width) { return (width + 63) / 64 * 64; }
 struct Layout {
     int waves, rb, hidden, tiles;
     ChainProduct f[kNetMaxLayers], r[kNetMaxLayers];
-    int64_t fixed_bytes_at, act_at[kNetMaxLayers], bytes;
+    int64_t fixed_bytes_at, backs_bytes_at, act_at[kNetMaxLayers], bytes;
     int fixed_at[kNetMaxLayers + 2], fixed_size, act_blocks[kNetMaxLayers], tile_end[4];
 
     explicit Layout(const NetChain& net) : hidden(net.hidden)
@@ -526,9 +646,11 @@ struct Layout {
         waves = widest <= 128 ? 4 : 8;
         // (the last chunks' places are loaded from ahead of need)
         int64_t at = 0;
+        int backs = 0;
         const auto product = [&](int k, int n_out) {
-            const ChainProduct p = {at, padded(n_out) / 32, padded(k) / 16};
+            const ChainProduct p = {at, padded(n_out) / 32, padded(k) / 16, backs};
             at += 4ll * p.blocks * p.chunks * kChunkBytes;
+            backs += 4 * p.blocks * 32;
             return p;
         };
         for (int l = 0; l < hidden; ++l) f[l] = product(net.widths[l], net.widths[l + 1]);
@@ -543,6 +665,8 @@ struct Layout {
         fixed_size += 4;
         fixed_bytes_at = at;
         at += (4ll * fixed_size * 4 + 255) / 256 * 256;
+        backs_bytes_at = at;
+        at += 4ll * backs;
         int64_t tiles64 = 0;
         for (int t = 0; t < 4; ++t) tiles64 += (net.n[t] + 63) / 64;
         // 32 or 64 rows to a workgroup.  64 halve the weights' way from the L2 and are the faster form of a full chip (organic molecules;
@@ -587,6 +711,7 @@ ChainArgs args_of(const NetChain& net, const Layout& L, const void* workspace)
     }
     a.packed = ws;
     a.fixed = reinterpret_cast<const float*>(ws + L.fixed_bytes_at);
+    a.backs = reinterpret_cast<const float*>(ws + L.backs_bytes_at);
     for (int l = 0; l < L.hidden; ++l) {
         a.act[l] = net.want_rows ? reinterpret_cast<float*>(ws + L.act_at[l]) : nullptr;
         a.act_blocks[l] = L.act_blocks[l];
@@ -631,7 +756,8 @@ hipError_t launch_net_chain_values(const NetChain& net, void* workspace, float* 
             q.chunks = c.chunks;
             q.back = back != 0;
             q.at = c.at;
-            q.end = end += 4 * c.blocks * c.chunks;
+            q.back_at = c.back_at;
+            q.end = end += 4 * c.blocks;
         }
     for (int l = 0; l <= L.hidden; ++l)
         for (int t = 0; t < 4; ++t) p.bias[l][t] = net.n[t] > 0 ? net.b[l][t] : nullptr;
@@ -642,8 +768,8 @@ hipError_t launch_net_chain_values(const NetChain& net, void* workspace, float* 
     p.fixed_size = L.fixed_size;
     p.packed = static_cast<char*>(workspace);
     p.fixed = reinterpret_cast<float*>(p.packed + L.fixed_bytes_at);
-    const int waves = end + (4 * L.fixed_size + 63) / 64;
-    chain_pack_kernel<<<dim3(static_cast<unsigned>((waves + 3) / 4)), dim3(256), 0, stream>>>(p);
+    p.backs = reinterpret_cast<float*>(p.packed + L.backs_bytes_at);
+    chain_pack_kernel<<<dim3(static_cast<unsigned>(end + (4 * L.fixed_size + 64 * kPackWaves - 1) / (64 * kPackWaves))), dim3(64 * kPackWaves), 0, stream>>>(p);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     ChainArgs a = args_of(net, L, workspace);

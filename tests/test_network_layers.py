@@ -555,6 +555,56 @@ def test_float32_networks_in_one_launch_each_way(widths, rows):
     assert torch.equal(values[big][others], other_values[big][others]) and torch.equal(grads[big][others], other_grads[big][others])
 
 
+# Rows of very different sizes, and columns of a layer whose sizes the next layer's weights undo: every row has the accuracy of its own
+# size.  Without biases and with the exact CELU a small row's network is its linear part, a large one's no larger than that; the sizes
+# within a row and a column stay within the 2^28 over which a scaled operand keeps all its bits.  Bound: as above, per row.
+@pytest.mark.parametrize("rows", [(3, 70, 0, 33), (16500, 33, 0, 129)])
+@pytest.mark.parametrize("widths", [(128, 128, 64, 1), (384, 256, 64, 256, 1)])
+def test_float32_networks_in_one_launch_over_float32s_range(widths, rows):
+    from khan_amd import _lib
+    lib = _lib.load()
+    print("case:", widths, rows, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device="cuda")
+    layers, alpha, st = len(widths) - 1, 0.5, torch.cuda.current_stream().cuda_stream
+    powers = lambda n, most: torch.exp2(torch.randint(-most, most + 1, (n,), generator=gen, device="cuda").float())
+    size = [powers(n, 80) for n in rows]
+    x = [rand(n, widths[0]) * s[:, None] for n, s in zip(rows, size)]
+    w = [[rand(k, m) * k ** -0.5 for _ in rows] for k, m in zip(widths, widths[1:])]
+    for l in range(layers - 1):
+        for t in range(4):
+            by = powers(widths[l + 1], 12)
+            w[l][t] *= by
+            w[l + 1][t] /= by[:, None]
+    a = _Chain(layers=layers, want_rows=1, alpha=alpha)
+    values, grads = [torch.empty(n, device="cuda") for n in rows], [torch.empty(n, widths[0], device="cuda") for n in rows]
+    for i, k in enumerate(widths):
+        a.widths[i] = k
+    for t, n in enumerate(rows):
+        a.n[t], a.x[t], a.value[t], a.grad[t] = n, x[t].data_ptr(), values[t].data_ptr(), grads[t].data_ptr()
+        for l in range(layers):
+            a.w[l][t] = w[l][t].data_ptr()
+    workspace = torch.full((lib.khan_net_chain_workspace_bytes(ctypes.byref(a)),), 255, dtype=torch.uint8, device="cuda")
+    a.workspace = workspace.data_ptr()
+    assert lib.khan_net_chain_values_f32(ctypes.byref(a), st) == 0
+    assert lib.khan_net_chain_rows_f32(ctypes.byref(a), st) == 0
+    for t, n in enumerate(rows):
+        if n == 0:
+            continue
+        leaf = x[t].double().requires_grad_(True)
+        h, sizes = leaf, leaf.detach().abs()
+        for l in range(layers):
+            h = h @ w[l][t].double()
+            sizes = sizes @ w[l][t].double().abs() * widths[l] ** -0.5
+            if l + 1 < layers:
+                h = torch.where(h > 0, h, alpha * torch.expm1(h.clamp(max=0.0) / alpha))
+        grad, = torch.autograd.grad(h.sum(), leaf)
+        assert ((values[t] - h.detach()[:, 0]).abs() <= 2e-6 * layers * 4 * sizes.amax(1)).all()
+        # (a slope is known where its activation's error is small beside alpha)
+        off = (grads[t] - grad).abs().amax(1)
+        assert torch.isfinite(grads[t]).all() and (off[size[t] < 2.0 ** -20] <= 2e-6 * layers * 4 * grad.abs().max()).all()
+
+
 def test_networks_that_one_launch_does_not_take():
     """Feature widths off 128, hidden layers wider than 256, more than eleven of them or none, an output that is no single value."""
     from khan_amd import _lib
