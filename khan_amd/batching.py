@@ -336,7 +336,7 @@ class DeviceFeeder:
         n, sizes, totals = staged
         labels = grads = None
         if ds.all_ys is not None:
-            labels = [ds.all_ys[p] for p in sel.tolist()]
+            labels = native.picked(ds.all_ys, sel) if type(ds.all_ys) is list else [ds.all_ys[p] for p in sel.tolist()]
         else:
             while sizes and sizes[-1] == 0:         # without labels the last molecule is the last that has atoms
                 sizes.pop()

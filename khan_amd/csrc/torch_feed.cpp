@@ -116,6 +116,21 @@ py::tuple staged_totals(const Tensor& staging, int64_t n, const py::array_t<int6
     return totals.pair();
 }
 
+// [values[k] for k in sel] of a list (the interpreter takes 30 ns an entry, a sixth of what a data set's pass takes)
+py::list picked(const py::list& values, const py::array_t<int64_t>& sel)
+{
+    const int64_t count = sel.size();
+    py::list out(static_cast<size_t>(count));
+    for (int64_t k = 0; k < count; ++k) {
+        const int64_t id = sel.data()[k];
+        if (id < 0 || id >= PyList_GET_SIZE(values.ptr())) throw py::index_error("molecule index out of range");
+        PyObject* o = PyList_GET_ITEM(values.ptr(), id);
+        Py_INCREF(o);
+        PyList_SET_ITEM(out.ptr(), k, o);
+    }
+    return out;
+}
+
 int64_t staging_bytes(int64_t n, bool f64) { return Staged(n, f64).bytes(); }
 
 // The staging area's parts as host tensors: xs, ys, zs, types, molecule indices
@@ -194,6 +209,7 @@ py::list molecule_rows(const py::array& planes, const py::list& sizes)
 void bind_feed(py::module_& m)
 {
     m.def("stage_molecules", &stage_molecules);
+    m.def("picked", &picked);
     m.def("staged_totals", &staged_totals);
     m.def("staging_bytes", &staging_bytes);
     m.def("staging_parts", &staging_parts);
