@@ -77,8 +77,6 @@ __device__ __forceinline__ void fwd_angular_batch(FwdWaveLds<T, kJvp, kNB, kRadN
     static_assert(!kMatrixPhase2 || (sizeof(T) == 4 && !kJvp), "the matrix-core phase 2 is float, forward only");
     typedef typename Fast<T>::vec4 vec4;
     typedef typename Fast<T>::vec2 vec2;
-    const unsigned long long lane_bit = 1ull << lane;
-    const unsigned long long lt_mask = lane_bit - 1ull;
     // segment-table lanes: lane = centre-in-batch * 10 + type-pair index (HH HC HN HO CC CN CO NN NO OO)
     const int seg_b = lane / kNumPairBlocks, seg_pt = lane - seg_b * kNumPairBlocks;
     const int seg_a = seg_pt < 4 ? 0 : seg_pt < 7 ? 1 : seg_pt < 9 ? 2 : 3;
@@ -121,7 +119,7 @@ __device__ __forceinline__ void fwd_angular_batch(FwdWaveLds<T, kJvp, kNB, kRadN
     wave_lds_fence();
     if (cnt > 0) {
         mine.start_cnt = static_cast<unsigned>(start) | (static_cast<unsigned>(cnt) << 16);
-        const int at = popc64(nonempty & lt_mask);
+        const int at = rank_in(nonempty);
         S.seg[at] = mine;
         S.segrow[at] = (static_cast<unsigned long long>(seg_row_hi) << 32) | seg_row_lo;
         atomicOr(&S.bits[start >> 5], 1u << (start & 31));
@@ -154,7 +152,7 @@ __device__ __forceinline__ void fwd_angular_batch(FwdWaveLds<T, kJvp, kNB, kRadN
         const unsigned w0 = static_cast<unsigned>(uniform(static_cast<int>(S.bits[base >> 5])));
         const unsigned w1 = static_cast<unsigned>(uniform(static_cast<int>(S.bits[(base >> 5) + 1])));
         const unsigned long long starts = (static_cast<unsigned long long>(w1) << 32) | w0;
-        const int ord = carry + popc64(starts & (lt_mask | lane_bit)) - 1;
+        const int ord = rank_in(starts >> 1, carry + static_cast<int>(w0 & 1u) - 1);         // (starts up to the lane itself)
         carry += popc64(starts);
         const int seg_at = max(ord, 0);
         const SegDesc d = S.seg[seg_at];
@@ -412,7 +410,7 @@ __device__ __forceinline__ void fwd_angular_batch(FwdWaveLds<T, kJvp, kNB, kRadN
                 constexpr int kLanesPer = kAngBlock * static_cast<int>(sizeof(T)) / 16;      // lanes per segment: 8 or 16
                 constexpr int kPerStep = 64 / kLanesPer;
                 const int n_empty = popc64(empties);
-                if (is_empty) S.segrow[popc64(empties & lt_mask)] = (static_cast<unsigned long long>(seg_row_hi) << 32) | seg_row_lo;
+                if (is_empty) S.segrow[rank_in(empties)] = (static_cast<unsigned long long>(seg_row_hi) << 32) | seg_row_lo;
                 wave_lds_fence();
                 for (int e0 = 0; e0 < n_empty; e0 += kPerStep) {
                     const int e = e0 + lane / kLanesPer;

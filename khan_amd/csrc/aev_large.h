@@ -184,7 +184,6 @@ __device__ __forceinline__ int list_candidates(const SortedAtoms<T>& sorted, int
             }
         }
     }
-    const unsigned long long lt_mask = (1ull << lane) - 1ull;
     const float4* const boxes = sorted.box + 2 * first_chunk;
     const int n_chunks = (n + 63) >> 6;
     int count = 0;
@@ -211,7 +210,7 @@ __device__ __forceinline__ int list_candidates(const SortedAtoms<T>& sorted, int
                 const int j = ch[u] * 64 + lane;
                 const float4 p = make_float4(static_cast<float>(at[u].x), static_cast<float>(at[u].y), static_cast<float>(at[u].z), 0.0f);
                 const unsigned long long take = wave_ballot(j < n && in_reach(lo, hi, p, p));
-                const int to = count + popc64(take & lt_mask);
+                const int to = rank_in(take, count);
                 if (((take >> lane) & 1ull) && to < kMaxCandidates) {
                     positions[to] = j;
                     atoms[to] = at[u];

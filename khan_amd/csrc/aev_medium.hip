@@ -78,7 +78,6 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
     const int wave = kLarge ? 0 : uniform(tid >> 6);
     FwdWaveLds<T, kJvp, kNB>& S = lds_wave[wave];
     const LaneConsts<T> L = lane_consts<T>(lane);
-    const unsigned long long lt_mask = (1ull << lane) - 1ull;
     const int rslot = lane >> 4;                                 // radial walk: entry slot of this 16-lane group
 
     fwd_lds_init(S, lane);
@@ -125,7 +124,7 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
             int before = 0;                     // atoms of my type held by earlier wavefronts
             for (int w = 0; w < wave; ++w) before += M.wcount[w][type];
             const unsigned long long mine = type == 0 ? tmask[0] : type == 1 ? tmask[1] : type == 2 ? tmask[2] : tmask[3];
-            const int dest = sel4(type, tbase[0], tbase[1], tbase[2], tbase[3]) + before + popc64(mine & lt_mask);
+            const int dest = sel4(type, tbase[0], tbase[1], tbase[2], tbase[3]) + rank_in(mine, before);
             M.atom[dest] = Fast<T>::make4(x, y, z, static_cast<T>(kJvp ? type : type + 4 * tid));
             if constexpr (kJvp) {
                 M.v.vel[dest] = Fast<T>::make4(vx, vy, vz, T(0));
@@ -258,7 +257,7 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
                     for (int a = 0; a < 4; ++a) {
                         const unsigned long long ma = wave_ballot(tR == a);
                         cnt[a] = popc64(ma);
-                        if (tR == a) dest = before + popc64(ma & lt_mask);
+                        if (tR == a) dest = rank_in(ma, before);
                         before += cnt[a];
                     }
                     wave_lds_fence();               // every entry has been read
@@ -302,7 +301,7 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
                         const T wx = vi.x - vjv.x, wy = vi.y - vjv.y, wz = vi.z - vjv.z;     // v_centre - v_partner
                         const T rd = (dx * wx + dy * wy + dz * wz) * inv;                    // d r along it
                         if (inR) {
-                            const int p = posR + popc64(mR & lt_mask);
+                            const int p = rank_in(mR, posR);
                             if (p < kRadCap) {
                                 T fc, dfc;
                                 Fast<T>::cutoff_grad(r, static_cast<T>(kR_Rc_f), fc, dfc);
@@ -312,7 +311,7 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
                             }
                         }
                         if (inA) {
-                            const int p = posA + popc64(mA & lt_mask);
+                            const int p = rank_in(mA, posA);
                             if (p < kCapA) {
                                 T fc, dfc;
                                 Fast<T>::cutoff_grad(r, static_cast<T>(kA_Rc_f), fc, dfc);
@@ -329,11 +328,11 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
                         // worked out once per centre on the compacted lists below, not once per chunk on every lane.
                         // (the place of the cutoff value carries the partner's type until then)
                         if (inR) {
-                            const int p = posR + popc64(mR & lt_mask);
+                            const int p = rank_in(mR, posR);
                             if (p < kRadCap) S.rad()[p] = Fast<T>::make2(r, aj.w);
                         }
                         if (inA) {
-                            const int p = posA + popc64(mA & lt_mask);
+                            const int p = rank_in(mA, posA);
                             if (p < kCapA) {
                                 S.nbr[b][p] = Fast<T>::make4(dx, dy, dz, r);
                                 S.nbr_fc[b][p] = aj.w;
@@ -374,7 +373,7 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
 #pragma unroll
                     for (int a = 0; a < 4; ++a) {
                         const unsigned long long ma = wave_ballot(tA == a);
-                        if (tA == a) dest = before + popc64(ma & lt_mask);
+                        if (tA == a) dest = rank_in(ma, before);
                         before += popc64(ma);
                     }
                     wave_lds_fence();               // every entry has been read

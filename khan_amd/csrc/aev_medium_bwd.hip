@@ -103,7 +103,6 @@ void aev_bwd_medium_kernel(
     const int wave = kLarge ? 0 : uniform(tid >> 6);
     BwdPool<T, kMB>& P = pools[wave];
     const LaneConsts<T> L = lane_consts<T>(lane);
-    const unsigned long long lt_mask = (1ull << lane) - 1ull;
 
     // Large molecules: the forces are added up in sorted order, 16 (32) bytes an atom (sorted.force), so that the three additions to
     // an atom, and those to its neighbours in an instruction, are one request beyond the L2, and are brought to the outputs by a
@@ -181,7 +180,7 @@ void aev_bwd_medium_kernel(
             int before = 0;                     // atoms of my type held by earlier wavefronts
             for (int w = 0; w < wave; ++w) before += M.wcount[w][type];
             const unsigned long long mine = type == 0 ? tmask[0] : type == 1 ? tmask[1] : type == 2 ? tmask[2] : tmask[3];
-            const int dest = sel4(type, tbase[0], tbase[1], tbase[2], tbase[3]) + before + popc64(mine & lt_mask);
+            const int dest = sel4(type, tbase[0], tbase[1], tbase[2], tbase[3]) + rank_in(mine, before);
             M.atom[dest] = Fast<T>::make4(x, y, z, static_cast<T>(type));
             M.row_lo[dest] = static_cast<unsigned>(rowbits & 0xffffffffull);
             M.row_hi[dest] = static_cast<unsigned>(rowbits >> 32);
@@ -423,7 +422,7 @@ void aev_bwd_medium_kernel(
                         const unsigned long long mRb = wave_ballot(!kSkipRadial && !again && valid && (rr < kR_Rc_f) && (rr > T(0)));
                         const unsigned long long mAb = wave_ballot(valid && (rr < kA_Rc_f) && (rr > T(0)));
                         if ((mAb >> lane) & 1ull) {
-                            const int p = pos + popc64(mAb & lt_mask);
+                            const int p = rank_in(mAb, pos);
                             if (p < 64) {
                                 P.nbr[p] = Fast<T>::make4(ddx, ddy, ddz, rr);
                                 P.nbr_idx[p] = static_cast<unsigned char>(atom_word(aj.w) >> kTypeShift);      // the partner's type
@@ -433,7 +432,7 @@ void aev_bwd_medium_kernel(
                         pos += popc64(mAb);
                         m_c += popc64(mAb);
                         if ((mRb >> lane) & 1ull) {
-                            const int p = qn + popc64(mRb & lt_mask);
+                            const int p = rank_in(mRb, qn);
                             q_d[p] = Fast<T>::make4(ddx, ddy, ddz, rr);
                             q_j[p] = static_cast<idx_t>(atom_word(aj.w));
                             q_c[p] = static_cast<centre_t>(c - run_first);
@@ -486,13 +485,13 @@ void aev_bwd_medium_kernel(
                         if (!too_many && ((mA[ch] >> lane) & 1ull)) {
                             // the entry as found; unit vector and cutoff are worked out once per centre below, on
                             // the compacted list, not once per chunk on every lane
-                            const int p = pos + popc64(mA[ch] & lt_mask);
+                            const int p = rank_in(mA[ch], pos);
                             P.nbr[p] = Fast<T>::make4(dx[ch], dy[ch], dz[ch], r[ch]);
                             P.nbr_idx[p] = static_cast<unsigned char>(j);
                         }
                         pos += popc64(mA[ch]);
                         if ((mR[ch] >> lane) & 1ull) {
-                            const int p = qn + popc64(mR[ch] & lt_mask);
+                            const int p = rank_in(mR[ch], qn);
                             q_d[p] = Fast<T>::make4(dx[ch], dy[ch], dz[ch], r[ch]);
                             q_j[p] = static_cast<unsigned short>(j);
                             q_c[p] = static_cast<unsigned short>(c);

@@ -102,7 +102,7 @@ void aev_bwd_small_kernel(
         tbase[3] = tbase[2] + tcount[2];
         if (have) {
             const unsigned long long mine = type == 0 ? tmask[0] : type == 1 ? tmask[1] : type == 2 ? tmask[2] : tmask[3];
-            dest = sel4(type, tbase[0], tbase[1], tbase[2], tbase[3]) + popc64(mine & lt_mask);
+            dest = sel4(type, tbase[0], tbase[1], tbase[2], tbase[3]) + rank_in(mine);
         }
     }
     x = lane_push(dest, x);

@@ -230,6 +230,13 @@ __device__ __forceinline__ int sel4(int a, int v0, int v1, int v2, int v3)
     return a == 0 ? v0 : a == 1 ? v1 : a == 2 ? v2 : v3;
 }
 __device__ __forceinline__ int popc64(unsigned long long m) { return __popcll(m); }
+// base + the number of the mask's bits below this lane (two instructions, and no mask of the lanes below held for it: popc64 of
+// the masked bits takes four)
+__device__ __forceinline__ int rank_in(unsigned long long m, int base = 0)
+{
+    return static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<unsigned>(m >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo(static_cast<unsigned>(m), static_cast<unsigned>(base))));
+}
 __device__ __forceinline__ unsigned long long low_bits(int w)   // w ones, 1 <= w <= 64
 {
     return w >= 64 ? ~0ull : ((1ull << w) - 1ull);
