@@ -276,7 +276,9 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
                 // 64 partners: aj (and with kJvp vjv) of the atom at sorted position j, where this lane has one
                 auto scan = [&](int j, bool have, const vec4 aj, const vec4 vjv) {
                     const T dx = ai.x - aj.x, dy = ai.y - aj.y, dz = ai.z - aj.z;
-                    const T r = Fast<T>::sqrt_rn(dx * dx + dy * dy + dz * dz);
+                    // (the multiply-adds as they stand here: this is in the code several times, and the compiler fused one product in one
+                    // copy and another in the next, so that a row's last bits depended on where in a list its partners came)
+                    const T r = Fast<T>::sqrt_rn(fma(dz, dz, fma(dx, dx, dy * dy)));
                     const bool valid = have && (j != i);
                     // r = 0, a coincident atom: no part in derivatives; in the features as the reference has it
                     const bool inR = valid && (r < kR_Rc_f) && (!kJvp || r > T(0));
