@@ -481,6 +481,19 @@ int khan_mol_energy_grad_f32(const float *e_grads, const int32_t *as, const int3
 int khan_mol_energy_grad_f64(const double *e_grads, const int32_t *as, const int32_t *sis, const int32_t *mos,
                              const int32_t *macs, int32_t n_mols, double *const *grad_host4, khan_stream_t stream);
 
+/* What a charge network's passes hand to one another (khan/model/nn.py:122-201 gathers and scatters by tf.gather): values of rows to
+ * the batch's atoms, out[i] = rows[row_of[i]] for n atoms, and n_ones ones (the molecules' energy gradients) in the same launch; values
+ * of atoms to rows; and the two sums with the charges' part, a += a_add of n_a and b += b_add of n_b elements.  Entries of row_of outside
+ * 0 .. n_rows - 1 give NaN, or are not written. */
+int khan_take_rows_f32(const float *rows, const int32_t *row_of, int64_t n, int64_t n_rows, float *out, float *ones, int64_t n_ones,
+                       khan_stream_t stream);
+int khan_put_rows_f32(const float *values, const int32_t *row_of, int64_t n, int64_t n_rows, float *rows, khan_stream_t stream);
+int khan_add_two_f32(float *a, const float *a_add, int64_t n_a, float *b, const float *b_add, int64_t n_b, khan_stream_t stream);
+int khan_take_rows_f64(const double *rows, const int32_t *row_of, int64_t n, int64_t n_rows, double *out, double *ones, int64_t n_ones,
+                       khan_stream_t stream);
+int khan_put_rows_f64(const double *values, const int32_t *row_of, int64_t n, int64_t n_rows, double *rows, khan_stream_t stream);
+int khan_add_two_f64(double *a, const double *a_add, int64_t n_a, double *b, const double *b_add, int64_t n_b, khan_stream_t stream);
+
 /* The charge entry points above with the number of atoms known (which spares the work of looking for molecules of sizes
  * that so many atoms cannot hold).  grads NULL: the energies only; otherwise the gradients, and the energies too unless e is
  * NULL; x/y/z_grads all NULL: no coordinate gradients (q_grads must then be given).  outputs_zeroed: e holds zeros already. */

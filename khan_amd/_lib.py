@@ -104,6 +104,12 @@ _SIGNATURES = {
     "khan_mol_energy_f64": (ctypes.c_int, [ctypes.POINTER(_ptr)] + [_ptr] * 4 + [ctypes.c_int32, _ptr, _ptr]),
     "khan_mol_energy_grad_f32": (ctypes.c_int, [_ptr] * 5 + [ctypes.c_int32, ctypes.POINTER(_ptr), _ptr]),
     "khan_mol_energy_grad_f64": (ctypes.c_int, [_ptr] * 5 + [ctypes.c_int32, ctypes.POINTER(_ptr), _ptr]),
+    "khan_take_rows_f32": (ctypes.c_int, [_ptr, _ptr, ctypes.c_int64, ctypes.c_int64, _ptr, _ptr, ctypes.c_int64, _ptr]),
+    "khan_put_rows_f32": (ctypes.c_int, [_ptr, _ptr, ctypes.c_int64, ctypes.c_int64, _ptr, _ptr]),
+    "khan_add_two_f32": (ctypes.c_int, [_ptr, _ptr, ctypes.c_int64, _ptr, _ptr, ctypes.c_int64, _ptr]),
+    "khan_take_rows_f64": (ctypes.c_int, [_ptr, _ptr, ctypes.c_int64, ctypes.c_int64, _ptr, _ptr, ctypes.c_int64, _ptr]),
+    "khan_put_rows_f64": (ctypes.c_int, [_ptr, _ptr, ctypes.c_int64, ctypes.c_int64, _ptr, _ptr]),
+    "khan_add_two_f64": (ctypes.c_int, [_ptr, _ptr, ctypes.c_int64, _ptr, _ptr, ctypes.c_int64, _ptr]),
     "khan_coulomb_f32": (ctypes.c_int, [_ptr] * 6 + [ctypes.c_int32, ctypes.c_float, _ptr, _ptr]),
     "khan_coulomb_f64": (ctypes.c_int, [_ptr] * 6 + [ctypes.c_int32, ctypes.c_double, _ptr, _ptr]),
     "khan_coulomb_grad_f32": (ctypes.c_int, [_ptr] * 6 + [ctypes.c_int32, _ptr, ctypes.c_float] + [_ptr] * 5),

@@ -426,6 +426,31 @@ static int mol_energy_grad_impl(const T* e_grads, const int32_t* as, const int32
     return hip_status(khan::launch_mol_sum_grad<T>(e_grads, as, sis, mos, macs, n_mols, out, as_stream(stream)));
 }
 
+// counts that a launch takes: a thread to an element, workgroups of 256
+static bool countable(int64_t n) { return n >= 0 && n <= INT64_C(256) * INT32_MAX; }
+
+template <typename T>
+static int take_rows_impl(const T* rows, const int32_t* row_of, int64_t n, int64_t n_rows, T* out, T* ones, int64_t n_ones, khan_stream_t stream)
+{
+    if (!countable(n) || !countable(n_ones) || n_rows < 0 || (n > 0 && (!row_of || !out)) || (n_rows > 0 && !rows) || (n_ones > 0 && !ones))
+        return KHAN_ERR_INVALID_ARG;
+    return hip_status(khan::launch_take_rows<T>(rows, row_of, n, n_rows, out, ones, n_ones, as_stream(stream)));
+}
+
+template <typename T>
+static int put_rows_impl(const T* values, const int32_t* row_of, int64_t n, int64_t n_rows, T* rows, khan_stream_t stream)
+{
+    if (!countable(n) || n_rows < 0 || (n > 0 && (!row_of || !values)) || (n_rows > 0 && !rows)) return KHAN_ERR_INVALID_ARG;
+    return hip_status(khan::launch_put_rows<T>(values, row_of, n, n_rows, rows, as_stream(stream)));
+}
+
+template <typename T>
+static int add_two_impl(T* a, const T* a_add, int64_t n_a, T* b, const T* b_add, int64_t n_b, khan_stream_t stream)
+{
+    if (!countable(n_a) || !countable(n_b) || (n_a > 0 && (!a || !a_add)) || (n_b > 0 && (!b || !b_add))) return KHAN_ERR_INVALID_ARG;
+    return hip_status(khan::launch_add_two<T>(a, a_add, n_a, b, b_add, n_b, as_stream(stream)));
+}
+
 template <typename T>
 static int ani_charges(const T* xs, const T* ys, const T* zs, const T* qs, const int32_t* mos, const int32_t* macs, int32_t n_mols, int64_t n_atoms,
                        const T* grads, T k, T* e, T* q_grads, T* gx, T* gy, T* gz, int outputs_zeroed, khan_stream_t stream)
@@ -1087,6 +1112,30 @@ int khan_mol_energy_grad_f64(const double* e_grads, const int32_t* as, const int
                              const int32_t* macs, int32_t n_mols, double* const* grad_host4, khan_stream_t stream)
 {
     return mol_energy_grad_impl<double>(e_grads, as, sis, mos, macs, n_mols, grad_host4, stream);
+}
+int khan_take_rows_f32(const float* rows, const int32_t* row_of, int64_t n, int64_t n_rows, float* out, float* ones, int64_t n_ones, khan_stream_t stream)
+{
+    return take_rows_impl<float>(rows, row_of, n, n_rows, out, ones, n_ones, stream);
+}
+int khan_put_rows_f32(const float* values, const int32_t* row_of, int64_t n, int64_t n_rows, float* rows, khan_stream_t stream)
+{
+    return put_rows_impl<float>(values, row_of, n, n_rows, rows, stream);
+}
+int khan_add_two_f32(float* a, const float* a_add, int64_t n_a, float* b, const float* b_add, int64_t n_b, khan_stream_t stream)
+{
+    return add_two_impl<float>(a, a_add, n_a, b, b_add, n_b, stream);
+}
+int khan_take_rows_f64(const double* rows, const int32_t* row_of, int64_t n, int64_t n_rows, double* out, double* ones, int64_t n_ones, khan_stream_t stream)
+{
+    return take_rows_impl<double>(rows, row_of, n, n_rows, out, ones, n_ones, stream);
+}
+int khan_put_rows_f64(const double* values, const int32_t* row_of, int64_t n, int64_t n_rows, double* rows, khan_stream_t stream)
+{
+    return put_rows_impl<double>(values, row_of, n, n_rows, rows, stream);
+}
+int khan_add_two_f64(double* a, const double* a_add, int64_t n_a, double* b, const double* b_add, int64_t n_b, khan_stream_t stream)
+{
+    return add_two_impl<double>(a, a_add, n_a, b, b_add, n_b, stream);
 }
 
 // Plain Coulomb sums: the charge kernels with the cutoff function switched off and the constant given by the caller.

@@ -141,6 +141,13 @@ hipError_t launch_mol_sum(Buckets<const T> in, const int32_t* A, const int32_t* 
 template <typename T>
 hipError_t launch_mol_sum_grad(const T* e_grad, const int32_t* A, const int32_t* SIs, const int32_t* MOs, const int32_t* MACs,
                                int32_t n_mols, Buckets<T> out, hipStream_t stream);
+// out[i] = rows[row_of[i]] (NaN where that is outside 0 .. n_rows - 1), and n_ones ones; rows[row_of[i]] = values[i]; a += a_add, b += b_add
+template <typename T>
+hipError_t launch_take_rows(const T* rows, const int32_t* row_of, int64_t n, int64_t n_rows, T* out, T* ones, int64_t n_ones, hipStream_t stream);
+template <typename T>
+hipError_t launch_put_rows(const T* values, const int32_t* row_of, int64_t n, int64_t n_rows, T* rows, hipStream_t stream);
+template <typename T>
+hipError_t launch_add_two(T* a, const T* a_add, int64_t n_a, T* b, const T* b_add, int64_t n_b, hipStream_t stream);
 
 // ---- first dense layer behind the featurizer: out_t = act(rows_t . W_t + b_t) for the four types, float32 ----
 // rows[t]: [n[t], 384]; wt[t]: [128, 384] (the weights transposed); bias[t]: [128]; out[t]: [n[t], 128]

@@ -1012,17 +1012,41 @@ std::vector<Tensor> infer(const Tensor& xs, const Tensor& ys, const Tensor& zs, 
     if (!need_grad) charge_net.take_few();
     charge_net.take_chain();
     charge_net.forward(need_grad);
-    const Tensor qs = charge_net.values.index_select(0, gather);
+    const Tensor row_of = gather.to(at::kInt).contiguous(), qs = at::empty({n}, xs.options());
+    dev(row_of, at::kInt, "gather_idxs");
+    same_size(row_of.numel() == n, "gather_idxs must have one element per atom");
+    const Tensor ones = need_grad ? at::empty({m}, xs.options()) : Tensor();
+    const int64_t n_rows = charge_net.rows.total;
+    const auto in_type = [&](auto f32, auto f64) { return xs.scalar_type() == at::kFloat ? f32(0.0f) : f64(0.0); };
+    const auto take = [&](auto fn) {
+        return [&, fn](auto zero) {
+            using T = decltype(zero);
+            call(fn, ptr<const T>(charge_net.values), ptr<const int32_t>(row_of), n, n_rows, ptr<T>(qs), ptr<T>(ones), need_grad ? m : 0, charge_net.pass.st);
+        };
+    };
+    in_type(take(api.khan_take_rows_f32), take(api.khan_take_rows_f64));
     if (!need_grad) {
         out[0].add_(ani_charge(in[0], in[1], in[2], qs, mos, macs));
         return out;
     }
-    const auto c = ani_charge_grads(in[0], in[1], in[2], qs, mos, macs, at::ones({m}, xs.options()), true, true);
-    const Tensor by_value = at::empty_like(qs).index_copy_(0, gather.to(at::kLong), c[1]);
+    const auto c = ani_charge_grads(in[0], in[1], in[2], qs, mos, macs, ones, true, true);
+    const Tensor by_value = at::empty({n_rows}, xs.options());
+    const auto put = [&](auto fn) {
+        return [&, fn](auto zero) {
+            using T = decltype(zero);
+            call(fn, ptr<const T>(c[1]), ptr<const int32_t>(row_of), n, n_rows, ptr<T>(by_value), charge_net.pass.st);
+        };
+    };
+    in_type(put(api.khan_put_rows_f32), put(api.khan_put_rows_f64));
     const Tensor g = charge_net.gradients(by_type(charge_net.rows, by_value, 1), near_net.gradients({}, Tensor()));
     run_featurize_grad(in, args, by_type(near_net.rows, g, kFeats), {out[1], out[2], out[3]});
-    out[0].add_(c[0]);
-    result.narrow(0, from, 3 * n).add_(c[2].as_strided({3 * n}, {1}));          // (x, y and z lie end to end)
+    const auto add = [&](auto fn) {                                              // (x, y and z lie end to end)
+        return [&, fn](auto zero) {
+            using T = decltype(zero);
+            call(fn, ptr<T>(out[0]), ptr<const T>(c[0]), m, ptr<T>(out[1]), ptr<const T>(c[2]), 3 * n, charge_net.pass.st);
+        };
+    };
+    in_type(add(api.khan_add_two_f32), add(api.khan_add_two_f64));
     return out;
 }
 

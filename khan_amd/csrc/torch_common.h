@@ -29,6 +29,7 @@ using Four = std::array<Tensor, 4>;
     X(khan_mol_energy_grad_f64) X(khan_net_layer_f32) X(khan_net_layer_f64) X(khan_net_top_f32) X(khan_net_top_f64)      \
     X(khan_net_grads_workspace_bytes_f32) X(khan_net_grads_workspace_bytes_f64) X(khan_net_grads_f32) X(khan_net_grads_f64) \
     X(khan_net_few_fits) X(khan_net_few_f64) X(khan_net_chain_fits) X(khan_net_chain_workspace_bytes)                  \
+    X(khan_take_rows_f32) X(khan_take_rows_f64) X(khan_put_rows_f32) X(khan_put_rows_f64) X(khan_add_two_f32) X(khan_add_two_f64)   \
     X(khan_net_chain_values_f32) X(khan_net_chain_rows_f32)                                                            \
     X(khan_atomic_networks_f32) X(khan_atomic_networks_packed_bytes) X(khan_atomic_networks_pack_stored_f32)
 

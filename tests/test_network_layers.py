@@ -738,3 +738,35 @@ def test_differentiable_layers_one_by_one():
         for got, want in zip(*results):
             assert got.shape == want.shape
             assert want.numel() == 0 or float((got - want).abs().max()) <= 2e-5 * (1 + float(want.abs().max())), (head, first)
+
+
+# What a charge network's passes hand to one another: rows to atoms and back, ones and sums, around the 256 elements of a workgroup; an
+# index outside the rows gives NaN and writes nothing.  Copies and single additions: exact.
+@pytest.mark.parametrize("n, other", [(1, 700), (255, 0), (256, 257), (1025, 3)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_rows_to_atoms_and_back(dtype, n, other):
+    from khan_amd import _lib
+    lib, suffix, st = _lib.load(), "f32" if dtype == torch.float32 else "f64", torch.cuda.current_stream().cuda_stream
+    print("case:", dtype, n, other, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(8)
+    rand = lambda k: torch.randn(k, generator=gen, device="cuda", dtype=dtype)
+    row_of, rows = torch.randperm(n, generator=gen, device="cuda").int(), rand(n)
+    bad = row_of.clone()
+    bad[n // 2] = n
+    bad[-1] = -1
+    inside = (bad >= 0) & (bad < n)
+    for index in (row_of, bad):
+        out, ones = torch.zeros(n + 1, device="cuda", dtype=dtype), torch.zeros(other + 1, device="cuda", dtype=dtype)
+        assert getattr(lib, "khan_take_rows_" + suffix)(rows.data_ptr(), index.data_ptr(), n, n, out.data_ptr(), ones.data_ptr(), other, st) == 0
+        back = torch.zeros(n + 1, device="cuda", dtype=dtype)
+        assert getattr(lib, "khan_put_rows_" + suffix)(out.data_ptr(), index.data_ptr(), n, n, back.data_ptr(), st) == 0
+        use = inside if index is bad else torch.ones_like(inside)
+        assert torch.equal(out[:-1][use], rows[index[use].long()]) and torch.isnan(out[:-1][~use]).all()
+        assert (ones[:-1] == 1).all() and ones[-1] == 0 and out[-1] == 0 and back[-1] == 0
+        want = torch.zeros(n, device="cuda", dtype=dtype)
+        want[index[use].long()] = rows[index[use].long()]
+        assert torch.equal(back[:-1], want)
+    a, b, c, d = rand(n + 1), rand(other + 1), rand(n + 1), rand(other + 1)
+    want = torch.cat([a[:-1] + c[:-1], a[-1:]]), torch.cat([b[:-1] + d[:-1], b[-1:]])
+    assert getattr(lib, "khan_add_two_" + suffix)(a.data_ptr(), c.data_ptr(), n, b.data_ptr(), d.data_ptr(), other, st) == 0
+    assert torch.equal(a, want[0]) and torch.equal(b, want[1])
