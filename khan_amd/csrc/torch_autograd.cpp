@@ -815,7 +815,10 @@ struct Inference {
         return grads;
     }
 
-    // Float32 networks layer by layer otherwise: of hidden widths up to 256.
+    // Float32 networks that would go layer by layer otherwise, of hidden widths up to 256 and rows of a multiple of 128 (us, layer by layer
+    // -> this; deep networks with gradients: 1 organic molecule 184 -> 151, 400 322 -> 185, 4,096 924 -> 670; values alone 1 93 -> 91,
+    // 256 130 -> 101; default ones beside charges, values alone: 16 97 -> 98, 256 108 -> 106, 4,096 240 -> 199; with gradients 65,536
+    // 5,060 -> 4,300).
     void take_chain()
     {
         if (w.params.dtype != at::kFloat || one_launch()) return;
@@ -997,7 +1000,7 @@ std::vector<Tensor> infer(const Tensor& xs, const Tensor& ys, const Tensor& zs, 
     const auto f = run_featurize(in, args);
     const Four feats = {f[0], f[1], f[2], f[3]};
     const Weights near_w = weights_of(near, alpha);
-    same_size(charge.is_none() || !near_w.packed.defined(), "networks beside a charge network run layer by layer");
+    same_size(charge.is_none() || !near_w.packed.defined(), "networks beside a charge network take no packed weights");
     Inference near_net(near_w, feats);
     near_net.take_few();
     near_net.take_chain();
@@ -1007,7 +1010,7 @@ std::vector<Tensor> infer(const Tensor& xs, const Tensor& ys, const Tensor& zs, 
         return out;
     }
     const Weights charge_w = weights_of(charge.cast<py::tuple>(), alpha);
-    same_size(!charge_w.packed.defined(), "a charge network runs layer by layer");
+    same_size(!charge_w.packed.defined(), "a charge network takes no packed weights");
     Inference charge_net(charge_w, feats);
     if (!need_grad) charge_net.take_few();
     charge_net.take_chain();

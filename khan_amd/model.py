@@ -7,8 +7,9 @@ features -> per-type networks -> gather -> segment_sum (+ ani_charge) of lines 3
 
 The featurizer, its gradient and the charge energy are the HIP kernels of this package (through
 `khan_amd.autograd`).  On the GPU, networks with CELU run in this package's matrix-core kernels: the reference's default
-widths in float32 with constant weights in one launch (`ops.atomic_networks`), everything else layer by layer, forward,
-gradient, second order and weight gradients (csrc/net_layers.hip).  Other activations, and the CPU, take PyTorch's
+widths in float32 with constant weights in one launch (`ops.atomic_networks`), inference of other widths and of models with
+charges in float32 in a launch each way (csrc/net_chain.hip), everything else layer by layer, forward, gradient, second order
+and weight gradients (csrc/net_layers.hip).  Other activations, and the CPU, take PyTorch's
 operations.  Parameter
 names are the reference's TensorFlow variable names, `<prefix>W_<type>_<in>x<out>_l<k>:0` and
 `<prefix>b_...` (nn.py:41-60), so a checkpoint written by the reference's `save_numpy` loads unchanged;
@@ -264,8 +265,8 @@ class AniModel:
                 parts.append(torch.cat([energies, energies.new_empty(-b.n_mols % 64)] + parts))
             return [energies] + parts
         acs, order, classes = b._counts(waited)
-        # Networks beside a charge network run layer by layer: products of all 24 bits over float32's range, where the
-        # one-launch kernel's operands keep 2^-24 of their size between 6e-5 and 65,504.
+        # Networks beside a charge network have products of all 24 bits over float32's range (net_chain.hip, or layer by
+        # layer), where the one-launch kernel's operands keep 2^-24 of their size between 6e-5 and 65,504.
         alone = self.charge is None
         return _native.load().infer(
             b.xs, b.ys, b.zs, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs, b.gather_idxs, acs, order, classes,
