@@ -28,7 +28,7 @@ ROOT = os.path.dirname(HERE)
 
 HIP_SOURCES = ["capi.hip", "aev_generic.hip", "aev_small.hip", "aev_small_whole.hip", "aev_small_f64.hip", "aev_small_bwd.hip", "aev_small_bwd_f64.hip", "aev_medium.hip",
                "aev_medium_large.hip", "aev_medium_bwd.hip", "aev_large_sort.hip", "sort_offsets.hip", "charges.hip", "dense_first.hip", "dense_fused.hip", "net_layers.hip", "net_few.hip", "net_chain.hip", "mol_sum.hip"]
-HIP_HEADERS = ["khan_internal.h", "khan_params.h", "aev_generic_center.h", "aev_small_common.h", "aev_fwd_batch.h", "aev_bwd_batch.h", "aev_large.h", "net_layers.h", "net_few.h", "net_chain.h", "net_celu.h", "dense_fused_tiles.h", "split_bf16.h", "split_half.h", os.path.join(ROOT, "include", "khan_aev.h")]
+HIP_HEADERS = ["khan_internal.h", "khan_params.h", "aev_generic_center.h", "aev_small_common.h", "aev_fwd_batch.h", "aev_bwd_batch.h", "aev_large.h", "net_layers.h", "net_few.h", "net_chain.h", "net_celu.h", "dense_fused_tiles.h", "split_bf16.h", os.path.join(ROOT, "include", "khan_aev.h")]
 
 # packed-FP32 instruction selection is switched off on purpose (target feature -packed-fp32-ops)
 HIPCC_FLAGS = [

@@ -45,7 +45,6 @@
 #include "dense_fused_tiles.h"
 #include "khan_internal.h"
 #include "khan_params.h"
-#include "split_half.h"
 
 namespace khan {
 
@@ -53,6 +52,11 @@ namespace {
 
 typedef float v4 __attribute__((ext_vector_type(4)));
 typedef float v16 __attribute__((ext_vector_type(16)));
+typedef unsigned u2v __attribute__((ext_vector_type(2)));
+typedef unsigned u4v __attribute__((ext_vector_type(4)));
+typedef _Float16 h2v __attribute__((ext_vector_type(2)));
+typedef _Float16 h8v __attribute__((ext_vector_type(8)));
+typedef float f2v __attribute__((ext_vector_type(2)));
 
 constexpr int kRows = kFusedRows;   // rows per workgroup
 constexpr int kResident = 2 * kCUs; // workgroups that the chip holds
@@ -62,6 +66,7 @@ constexpr int kActStride = 136;     // 16-bit elements between rows of the activ
 constexpr int kKC = kFusedKC;       // k per staged chunk
 constexpr int kStStride = 40;       // 16-bit elements between staged rows: a pair of chunks (32 k) + 8
 constexpr int kParts = kFusedParts;
+constexpr float kResidualScale = 2048.0f, kResidualBack = 1.0f / 2048.0f;      // 2^11
 
 struct FusedArgs {
     const float* rows[4];           // [n_t, 384] feature rows per type
@@ -97,6 +102,20 @@ struct __align__(16) FusedLds {
     // already asked for (loads come back in order)
     float fixed[4][kFixed];
 };
+
+// two floats -> their two half-precision parts (the value rounded, and 2^11 times what the rounding left), each pair
+// packed into one register (first value in the low half).  Both differences are exact in float32.
+__device__ __forceinline__ void split_pair(float x0, float x1, unsigned& p1, unsigned& p2)
+{
+    const h2v h = __builtin_convertvector(f2v{x0, x1}, h2v);
+    p1 = __builtin_bit_cast(unsigned, h);
+    // 2^11 x - 2^11 h in one fused multiply-add that reads h and writes half precision as they are (both products are exact,
+    // and so is the difference)
+    h2v l;
+    l[0] = static_cast<_Float16>(fmaf(static_cast<float>(h[0]), -kResidualScale, x0 * kResidualScale));
+    l[1] = static_cast<_Float16>(fmaf(static_cast<float>(h[1]), -kResidualScale, x1 * kResidualScale));
+    p2 = __builtin_bit_cast(unsigned, l);
+}
 
 // a chunk piece (four consecutive k of one row or column) split into the planes of a stage buffer
 template <int kR>

@@ -816,9 +816,9 @@ struct Inference {
     }
 
     // Float32 networks that would go layer by layer otherwise, of hidden widths up to 256 and rows of a multiple of 128 (us, layer by layer
-    // -> this; deep networks with gradients: 1 organic molecule 184 -> 151, 400 322 -> 185, 4,096 924 -> 670; values alone 1 93 -> 91,
-    // 256 130 -> 101; default ones beside charges, values alone: 16 97 -> 98, 256 108 -> 106, 4,096 240 -> 199; with gradients 65,536
-    // 5,060 -> 4,300).
+    // -> this; deep networks with gradients: 1 organic molecule 191 -> 168, 400 321 -> 202, 4,096 904 -> 814; values alone 1 104 -> 99,
+    // 256 136 -> 107; default ones beside charges, values alone: 16 97 -> 91, 256 108 -> 98, 4,096 239 -> 201; with gradients 65,536
+    // 5,013 -> 4,665).
     void take_chain()
     {
         if (w.params.dtype != at::kFloat || one_launch()) return;

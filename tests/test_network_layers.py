@@ -484,8 +484,8 @@ class _Chain(ctypes.Structure):
                  ("widths", ctypes.c_int32 * 13), ("want_rows", ctypes.c_int32), ("accumulate", ctypes.c_int32), ("absolute", ctypes.c_uint32), ("alpha", ctypes.c_double)])
 
 
-# Float32 networks in a launch each way: rows around the 32 and the 64 of a workgroup, either form (64 rows for full rounds of 512
-# workgroups and more than three quarters of one, here 409) and both, divided inside a type and at its end, an empty type; widths on and off the padding to 64, layers so narrow
+# Float32 networks in a launch each way: rows around the 32 and the 64 of a workgroup, either form (64 rows: with four wavefronts
+# 262, 409 and 549 tiles of them, with eight 144, 262 and 409), an empty type; four wavefronts and eight, widths on and off the padding to 64, layers so narrow
 # that two wavefronts share their columns, one hidden layer and eleven, row gradients of one and of more passes over a workgroup's
 # columns.  A layer's sums are within 2e-6 of their products' sizes (as for single layers), and the weights are drawn to keep the
 # sizes, so that a value is within 2e-6 of the largest a layer; a slope takes its activation's error over alpha, and
@@ -555,18 +555,84 @@ def test_float32_networks_in_one_launch_each_way(widths, rows):
     assert torch.equal(values[big][others], other_values[big][others]) and torch.equal(grads[big][others], other_grads[big][others])
 
 
+def _run_chain(widths, x, w, alpha):
+    """The four types' values and row gradients, without biases."""
+    from khan_amd import _lib
+    lib, st, layers = _lib.load(), torch.cuda.current_stream().cuda_stream, len(widths) - 1
+    a = _Chain(layers=layers, want_rows=1, alpha=alpha)
+    values, grads = [torch.empty(r.shape[0], device="cuda") for r in x], [torch.empty_like(r) for r in x]
+    for i, k in enumerate(widths):
+        a.widths[i] = k
+    for t, r in enumerate(x):
+        a.n[t], a.x[t], a.value[t], a.grad[t] = r.shape[0], r.data_ptr(), values[t].data_ptr(), grads[t].data_ptr()
+        for l in range(layers):
+            a.w[l][t] = w[l][t].data_ptr()
+    workspace = torch.full((lib.khan_net_chain_workspace_bytes(ctypes.byref(a)),), 255, dtype=torch.uint8, device="cuda")
+    a.workspace = workspace.data_ptr()
+    assert lib.khan_net_chain_values_f32(ctypes.byref(a), st) == 0
+    assert lib.khan_net_chain_rows_f32(ctypes.byref(a), st) == 0
+    return values, grads
+
+
+# No operand loses a bit, whatever stands beside it: a column of zeros but for one weight, and positive sums, pass a value through
+# every layer as it is, and the weight comes back as the row's gradient; beside them are values 2^40 and weights 2^10 times as large
+# that do not reach the result.  Exact: a value times one is the sum of its three parts.
+@pytest.mark.parametrize("rows", [(3, 70, 0, 33), (26000, 33, 0, 129)])
+@pytest.mark.parametrize("widths", [(128, 5, 1), (128, 128, 64, 1), (384, 256, 64, 256, 1)])
+def test_float32_networks_in_one_launch_keep_every_bit(widths, rows):
+    print("case:", widths, rows, flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    values_of = lambda n: (torch.rand(n, generator=gen, device="cuda") + 1.0) * torch.exp2(torch.randint(-60, 40, (n,), generator=gen, device="cuda").float())
+    rand = lambda *shape: torch.randn(*shape, generator=gen, device="cuda")
+    x, w = [], [[torch.zeros(k, m, device="cuda") for _ in rows] for k, m in zip(widths, widths[1:])]
+    for t, n in enumerate(rows):
+        x.append(rand(n, widths[0]) * 2.0 ** 80)
+        x[t][:, 7] = values_of(n)
+        if n > 2:
+            x[t][:3, 7] = torch.tensor([1.0 + 2049.0 * 2.0 ** -23, 1.0 - 2.0 ** -24, 2.0 ** 24 - 1.0], device="cuda")
+        at = 7
+        for l in range(len(widths) - 1):
+            to = (5 * l + 3) % widths[l + 1]
+            if l + 1 < len(widths) - 1:
+                w[l][t][:8, 0 if to else 1] = rand(8) * 2.0 ** 10           # (a column that nothing takes)
+            w[l][t][:, to] = 0.0
+            w[l][t][at, to] = 1.0
+            at = to
+    values, grads = _run_chain(widths, x, w, 0.5)
+    for t, n in enumerate(rows):
+        assert torch.equal(values[t], x[t][:, 7])
+        assert (grads[t][:, 7] == 1).all() and grads[t].count_nonzero() == n
+    # the weights' bits, in every layer; and the slopes', which take theirs from the layer above
+    for l in range(len(widths) - 1):
+        for v in values_of(3).tolist() + [1.0 + 2049.0 * 2.0 ** -23]:
+            ones = [torch.where(torch.arange(widths[0], device="cuda") == 7, 1.0, r * 2.0 ** -70) for r in x]
+            with_v = [[m * v if k == l else m for m in layer] for k, layer in enumerate(w)]
+            values, grads = _run_chain(widths, ones, with_v, 0.5)
+            want = torch.tensor(v, device="cuda")
+            assert all((g == want).all() for g in values) and all((g[:, 7] == want).all() and g.count_nonzero() == g.shape[0] for g in grads)
+
+
+# A sum of 256 terms whose result float32 holds is finite, whatever the sizes of its factors.
+def test_float32_networks_in_one_launch_reach_as_far_as_float32():
+    widths = (256, 64, 1)
+    for up, down in ((121, -20), (-20, 110), (100, 10), (-60, -40)):
+        x = [torch.full((n, 256), 2.0 ** up, device="cuda") for n in (33, 0, 2, 65)]
+        w = [[torch.full((256, 64), 2.0 ** down, device="cuda") for _ in x], [torch.full((64, 1), 0.5, device="cuda") for _ in x]]
+        values, grads = _run_chain(widths, x, w, 0.5)
+        assert all((v == 2.0 ** (up + down + 8 + 5)).all() for v in values) and all((g == 2.0 ** (down + 5)).all() for g in grads)
+
+
 # Rows of very different sizes, and columns of a layer whose sizes the next layer's weights undo: every row has the accuracy of its own
-# size.  Without biases and with the exact CELU a small row's network is its linear part, a large one's no larger than that; the sizes
-# within a row and a column stay within the 2^28 over which a scaled operand keeps all its bits.  Bound: as above, per row.
+# size, in its value and in its gradient.  Bound: a layer's sums are within 2e-6 of their products' sizes (root mean squares, four times
+# for the largest of many); an activation's error is handed on by the next weights, a slope lies between those at both ends of
+# its activation's error, and the way back hands on the slopes' errors and adds as much of its own.
 @pytest.mark.parametrize("rows", [(3, 70, 0, 33), (26000, 33, 0, 129)])
 @pytest.mark.parametrize("widths", [(128, 128, 64, 1), (384, 256, 64, 256, 1)])
 def test_float32_networks_in_one_launch_over_float32s_range(widths, rows):
-    from khan_amd import _lib
-    lib = _lib.load()
     print("case:", widths, rows, flush=True)
     gen = torch.Generator(device="cuda").manual_seed(7)
     rand = lambda *shape: torch.randn(*shape, generator=gen, device="cuda")
-    layers, alpha, st = len(widths) - 1, 0.5, torch.cuda.current_stream().cuda_stream
+    layers, alpha = len(widths) - 1, 0.5
     powers = lambda n, most: torch.exp2(torch.randint(-most, most + 1, (n,), generator=gen, device="cuda").float())
     size = [powers(n, 80) for n in rows]
     x = [rand(n, widths[0]) * s[:, None] for n, s in zip(rows, size)]
@@ -576,33 +642,32 @@ def test_float32_networks_in_one_launch_over_float32s_range(widths, rows):
             by = powers(widths[l + 1], 12)
             w[l][t] *= by
             w[l + 1][t] /= by[:, None]
-    a = _Chain(layers=layers, want_rows=1, alpha=alpha)
-    values, grads = [torch.empty(n, device="cuda") for n in rows], [torch.empty(n, widths[0], device="cuda") for n in rows]
-    for i, k in enumerate(widths):
-        a.widths[i] = k
-    for t, n in enumerate(rows):
-        a.n[t], a.x[t], a.value[t], a.grad[t] = n, x[t].data_ptr(), values[t].data_ptr(), grads[t].data_ptr()
-        for l in range(layers):
-            a.w[l][t] = w[l][t].data_ptr()
-    workspace = torch.full((lib.khan_net_chain_workspace_bytes(ctypes.byref(a)),), 255, dtype=torch.uint8, device="cuda")
-    a.workspace = workspace.data_ptr()
-    assert lib.khan_net_chain_values_f32(ctypes.byref(a), st) == 0
-    assert lib.khan_net_chain_rows_f32(ctypes.byref(a), st) == 0
+    values, grads = _run_chain(widths, x, w, alpha)
+    each = 2e-6 * 4
+    slope = lambda z: torch.exp(z.clamp(max=0.0) / alpha)
     for t, n in enumerate(rows):
         if n == 0:
             continue
-        leaf = x[t].double().requires_grad_(True)
-        h, sizes = leaf, leaf.detach().abs()
+        h, err, zs, errs = x[t].double(), torch.zeros_like(x[t], dtype=torch.float64), [], []
         for l in range(layers):
-            h = h @ w[l][t].double()
-            sizes = sizes @ w[l][t].double().abs() * widths[l] ** -0.5
+            m = w[l][t].double()
+            err = (err.square() @ m.square()).sqrt() + each * (h.square() @ m.square()).sqrt()
+            h = h @ m
             if l + 1 < layers:
+                zs.append(h)
+                errs.append(err)
                 h = torch.where(h > 0, h, alpha * torch.expm1(h.clamp(max=0.0) / alpha))
-        grad, = torch.autograd.grad(h.sum(), leaf)
-        assert ((values[t] - h.detach()[:, 0]).abs() <= 2e-6 * layers * 4 * sizes.amax(1)).all()
-        # (a slope is known where its activation's error is small beside alpha)
-        off = (grads[t] - grad).abs().amax(1)
-        assert torch.isfinite(grads[t]).all() and (off[size[t] < 2.0 ** -20] <= 2e-6 * layers * 4 * grad.abs().max()).all()
+        assert ((values[t] - h[:, 0]).abs() <= err[:, 0]).all()
+        d, off = torch.ones(n, 1, dtype=torch.float64, device="cuda"), torch.zeros(n, 1, dtype=torch.float64, device="cuda")
+        for l in reversed(range(layers)):
+            m = w[l][t].double().t()
+            off = (off.square() @ m.square()).sqrt() + each * (d.square() @ m.square()).sqrt()
+            d = d @ m
+            if l > 0:
+                z, e = zs[l - 1], errs[l - 1]
+                off = off * slope(z + e) + d.abs() * (slope(z + e) - slope(z - e) + 1e-6)         # (1 + a / alpha, of a rounded a)
+                d = d * slope(z)
+        assert ((grads[t] - d).abs() <= off + each * d.abs()).all()
 
 
 def test_networks_that_one_launch_does_not_take():
