@@ -238,8 +238,9 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
                         obase += cnt_a;
                     }
                 };
-                // Large molecules: a centre's radial list is worked off whenever the next chunk's entries would not fit
-                // (no limit on the number of radial partners); racc collects the sums.
+                // Large molecules: a centre's radial list is worked off whenever it is full (no limit on the number of radial
+                // partners); racc collects the sums.  Always full: the cuts are then at the same partners however many atoms a step of
+                // the scan tests, and the sums have the same bits in runs of any length.
                 T racc[4] = {T(0), T(0), T(0), T(0)};
                 auto radial_flush = [&](int count) {
                     wave_lds_fence();
@@ -284,12 +285,19 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
                     const bool inR = valid && (r < kR_Rc_f) && (!kJvp || r > T(0));
                     const bool inA = valid && (r < kA_Rc_f) && (!kJvp || r > T(0));
                     const unsigned long long mR = wave_ballot(inR), mA = wave_ballot(inA);
-                    if constexpr (kLarge) {
-                        if (posR + popc64(mR) > kRadCap) {
-                            radial_flush(posR);
-                            posR = 0;
+                    // stores this lane's radial partner by put(place); of a large molecule's, those that do not fit once the list is empty
+                    auto put_radial = [&](auto put) {
+                        const int p = rank_in(mR, posR);
+                        if (inR && p < kRadCap) put(p);
+                        posR += popc64(mR);
+                        if constexpr (kLarge) {
+                            if (posR > kRadCap) {
+                                radial_flush(kRadCap);
+                                posR -= kRadCap;
+                                if (inR && p >= kRadCap) put(p - kRadCap);
+                            }
                         }
-                    }
+                    };
                     if constexpr (kJvp) {
                         const int tj = type_at(aj.w);
 #pragma unroll
@@ -301,17 +309,14 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
                         const T inv = Fast<T>::rcp(r);
                         const vec4 vi = vel_at(i);
                         const T wx = vi.x - vjv.x, wy = vi.y - vjv.y, wz = vi.z - vjv.z;     // v_centre - v_partner
-                        const T rd = (dx * wx + dy * wy + dz * wz) * inv;                    // d r along it
-                        if (inR) {
-                            const int p = rank_in(mR, posR);
-                            if (p < kRadCap) {
-                                T fc, dfc;
-                                Fast<T>::cutoff_grad(r, static_cast<T>(kR_Rc_f), fc, dfc);
-                                S.rad()[p] = Fast<T>::make2(r, fc);
-                                S.jvp.rad_ab[p] = Fast<T>::make2(dfc * rd, T(-2) * static_cast<T>(kR_eta_f) * fc * rd);
-                                if constexpr (kLarge) M.rtype[p] = static_cast<unsigned char>(tj);
-                            }
-                        }
+                        const T rd = fma(dz, wz, fma(dx, wx, dy * wy)) * inv;                // d r along it (as with r)
+                        put_radial([&](int p) {
+                            T fc, dfc;
+                            Fast<T>::cutoff_grad(r, static_cast<T>(kR_Rc_f), fc, dfc);
+                            S.rad()[p] = Fast<T>::make2(r, fc);
+                            S.jvp.rad_ab[p] = Fast<T>::make2(dfc * rd, T(-2) * static_cast<T>(kR_eta_f) * fc * rd);
+                            if constexpr (kLarge) M.rtype[p] = static_cast<unsigned char>(tj);
+                        });
                         if (inA) {
                             const int p = rank_in(mA, posA);
                             if (p < kCapA) {
@@ -329,10 +334,7 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
                         // as it is (distance; difference vector), and the cutoff functions and unit vectors are
                         // worked out once per centre on the compacted lists below, not once per chunk on every lane.
                         // (the place of the cutoff value carries the partner's type until then)
-                        if (inR) {
-                            const int p = rank_in(mR, posR);
-                            if (p < kRadCap) S.rad()[p] = Fast<T>::make2(r, aj.w);
-                        }
+                        put_radial([&](int p) { S.rad()[p] = Fast<T>::make2(r, aj.w); });
                         if (inA) {
                             const int p = rank_in(mA, posA);
                             if (p < kCapA) {
@@ -341,7 +343,6 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
                             }
                         }
                     }
-                    posR += popc64(mR);
                     posA += popc64(mA);
                 };
                 if constexpr (kLarge) {

@@ -969,6 +969,39 @@ def test_runs_of_large_molecules(ops, dtype, copies):
         assert abs(float(dot - back)) <= rtol * float(bound), (float(dot), float(back), float(bound))
 
 
+# A row and a Jacobian-vector product of a large molecule are the same bits whatever else is in the batch: in runs of one, two and four
+# centres (batches of up to 9,000, 40,000 and more atoms), beside small molecules, and with the classes unknown to the host.  Radial
+# lists hold 64 partners: the lattice's centres have about 41, 85 and 120.
+@pytest.mark.parametrize("spacing", [2.15, 1.7, 1.5])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_rows_of_large_molecules_are_the_same_bits_in_any_batch(ops, dtype, spacing):
+    say("case: one molecule of 700 atoms, spacing %g, in batches of 1 to 58 copies, %s" % (spacing, dtype))
+    rng = np.random.default_rng(41)
+    n = 700
+    xyz = _jittered_lattice(rng, n, spacing, 0.2)
+    A = rng.choice(4, n, p=[0.5, 0.25, 0.1, 0.15])
+    vectors = rng.standard_normal((3, n))
+    apart = np.linalg.norm(xyz[:, None] - xyz[None], axis=2)
+    assert ((apart < 4.6).sum(axis=1) - 1).max() > (30 if spacing > 2 else 64)
+
+    def rows_of(copies, smalls, known):
+        mols = [(A, xyz, vectors)] * copies + [(A[:7], xyz[:7] * 1.1, vectors[:, :7])] * smalls
+        sizes = [len(m[0]) for m in mols]
+        c = Case(*np.concatenate([m[1] for m in mols]).T, np.concatenate([m[0] for m in mols]), np.repeat(np.arange(len(mols)), sizes), len(mols))
+        macs, mos, sc, ga, ac = gpu_sort_offsets(ops, c)
+        args = (*(dev(v).to(dtype) for v in (c.X, c.Y, c.Z)), dev(c.A), mos, macs, sc, ac.cpu())
+        order = ops.size_order(macs)
+        kw = dict(order=order, size_classes=order[-4:].cpu()) if known else {}
+        v = [dev(np.concatenate([m[2][k] for m in mols])).to(dtype) for k in range(3)]
+        return [torch.cat(f).view(-1, 384)[ga.long()][:copies * n].view(copies, n, 384)
+                for f in (ops.featurize(*args, **kw), ops.featurize_grad_inverse(*args, *v, **kw))]
+
+    first = rows_of(1, 0, True)
+    for copies, smalls, known in ((1, 0, False), (3, 40, True), (13, 0, True), (13, 2000, True), (58, 0, True), (58, 0, False), (2, 6000, True), (1, 6000, False)):
+        for got, want in zip(rows_of(copies, smalls, known), first):
+            assert bool((got == want).all()), (copies, smalls, known, int((got != want).sum()))
+
+
 # Both sides of each line between the forward kernels: 174,763 atoms in float32 (87,382 in float64) make 256 MB of rows, 43,691
 # (21,846) the 64 MB of molecules of more than 256 atoms; up to 8,192 molecules of 32 atoms in float32 (6,144 of 64 in float64)
 # and 2,048 (512) larger ones are shared, and from 16,385 on there are five wavefronts to a SIMD.
