@@ -57,9 +57,9 @@ __global__ __launch_bounds__(256) void mol_sum_grad_kernel(const T* __restrict__
 }
 
 // What the passes of a model with a charge network hand to one another, a thread per element; index entries outside 0 .. n_rows - 1 give
-// NaN, or are not written.  Bound by the launch (a megabyte or two for 47,000 atoms): three of them stand where six library
-// kernels stood.  Energies and gradients with charges, organic molecules: default networks on one 157 -> 143 us, on 256 187 -> 172, on
-// 4,001 399 -> 382, deep ones on 4,001 1,183 -> 1,168.
+// NaN, or are not written.  Bound by the launch (a megabyte or two for 47,000 atoms): a pass with gradients has the library's gather, which
+// refuses such entries, and one of each of these where six library kernels stood (default networks with charges, one organic molecule
+// 149-154 us with those six and the networks layer by layer, 123-125 with neither).
 template <typename T>
 __global__ __launch_bounds__(256) void take_rows_kernel(const T* __restrict__ rows, const int32_t* __restrict__ row_of, int64_t n, int64_t n_rows,
                                                         T* __restrict__ out, T* __restrict__ ones, int64_t n_ones)

@@ -1015,25 +1015,28 @@ std::vector<Tensor> infer(const Tensor& xs, const Tensor& ys, const Tensor& zs, 
     if (!need_grad) charge_net.take_few();
     charge_net.take_chain();
     charge_net.forward(need_grad);
-    const Tensor row_of = gather.to(at::kInt).contiguous(), qs = at::empty({n}, xs.options());
-    dev(row_of, at::kInt, "gather_idxs");
-    same_size(row_of.numel() == n, "gather_idxs must have one element per atom");
-    const Tensor ones = need_grad ? at::empty({m}, xs.options()) : Tensor();
-    const int64_t n_rows = charge_net.rows.total;
-    const auto in_type = [&](auto f32, auto f64) { return xs.scalar_type() == at::kFloat ? f32(0.0f) : f64(0.0); };
-    const auto take = [&](auto fn) {
-        return [&, fn](auto zero) {
-            using T = decltype(zero);
-            call(fn, ptr<const T>(charge_net.values), ptr<const int32_t>(row_of), n, n_rows, ptr<T>(qs), ptr<T>(ones), need_grad ? m : 0, charge_net.pass.st);
-        };
-    };
-    in_type(take(api.khan_take_rows_f32), take(api.khan_take_rows_f64));
+    // (the library's gather, which refuses an index that is no integer or lies outside the rows)
+    const Tensor qs = charge_net.values.index_select(0, gather);
+    same_size(qs.numel() == n, "gather_idxs must have one element per atom");
     if (!need_grad) {
         out[0].add_(ani_charge(in[0], in[1], in[2], qs, mos, macs));
         return out;
     }
-    const auto c = ani_charge_grads(in[0], in[1], in[2], qs, mos, macs, ones, true, true);
+    const Tensor row_of = gather.to(at::kInt).contiguous(), ones = at::empty({m}, xs.options());
+    const int64_t n_rows = charge_net.rows.total;
+    same_size(n_rows <= n, "no more feature rows than atoms");
+    const auto in_type = [&](auto f32, auto f64) { return xs.scalar_type() == at::kFloat ? f32(0.0f) : f64(0.0); };
+    // the ones that the energies' gradients are and, of no rows at all, NaN for every row's derivative: what a row that no atom's index
+    // names then has
     const Tensor by_value = at::empty({n_rows}, xs.options());
+    const auto begin = [&](auto fn) {
+        return [&, fn](auto zero) {
+            using T = decltype(zero);
+            call(fn, static_cast<const T*>(nullptr), ptr<const int32_t>(row_of), n_rows, int64_t{0}, ptr<T>(by_value), ptr<T>(ones), m, charge_net.pass.st);
+        };
+    };
+    in_type(begin(api.khan_take_rows_f32), begin(api.khan_take_rows_f64));
+    const auto c = ani_charge_grads(in[0], in[1], in[2], qs, mos, macs, ones, true, true);
     const auto put = [&](auto fn) {
         return [&, fn](auto zero) {
             using T = decltype(zero);

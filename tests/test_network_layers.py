@@ -805,7 +805,7 @@ def test_differentiable_layers_one_by_one():
             assert want.numel() == 0 or float((got - want).abs().max()) <= 2e-5 * (1 + float(want.abs().max())), (head, first)
 
 
-# What a charge network's passes hand to one another: rows to atoms and back, ones and sums, around the 256 elements of a workgroup; an
+# The kernels between a charge network's passes: rows to atoms and back, ones and sums, around the 256 elements of a workgroup; an
 # index outside the rows gives NaN and writes nothing.  Copies and single additions: exact.
 @pytest.mark.parametrize("n, other", [(1, 700), (255, 0), (256, 257), (1025, 3)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
@@ -835,3 +835,40 @@ def test_rows_to_atoms_and_back(dtype, n, other):
     want = torch.cat([a[:-1] + c[:-1], a[-1:]]), torch.cat([b[:-1] + d[:-1], b[-1:]])
     assert getattr(lib, "khan_add_two_" + suffix)(a.data_ptr(), c.data_ptr(), n, b.data_ptr(), d.data_ptr(), other, st) == 0
     assert torch.equal(a, want[0]) and torch.equal(b, want[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_charges_refuse_what_is_no_index_of_a_row(dtype):
+    """A model with charges: indices from atoms to rows are integers, one to an atom; 64 bits and strides change nothing.  A row that no
+    index names has an undefined gradient, in its molecule and no other (an index outside the rows is the library gather's device
+    assertion, and no test's)."""
+    from khan_amd import datagen, model
+    from khan_amd.batching import DeviceBatch
+    m = model.AniModel((128, 64, 1), model.celu, dtype, "cuda:0", fit_charges=True, seed=2)
+    c = datagen.make_batch("organic", 40)
+    xyz = [torch.from_numpy(v).to("cuda", dtype) for v in (c.X, c.Y, c.Z)]
+    types, mols = torch.from_numpy(c.A).cuda(), torch.from_numpy(np.repeat(np.arange(40, dtype=np.int32), c.MACs)).cuda()
+
+    def passes(index=None, need_grad=True):
+        b = DeviceBatch.from_device_arrays(*xyz, types, mols, 40)
+        if index is not None:
+            b.gather_idxs = index(b.gather_idxs)
+        return m.batch_energies(b, need_grad=need_grad)
+
+    want, want_g = passes()
+    assert torch.isfinite(want).all() and torch.isfinite(want_g).all()
+    for index in (lambda g: g.long(), lambda g: torch.stack([g, g], dim=1)[:, 0]):
+        e, g = passes(index)
+        assert torch.equal(e, want) and torch.allclose(g, want_g, rtol=1e-4, atol=1e-6)
+    for index in (lambda g: g.float(), lambda g: g.double(), lambda g: g.short(), lambda g: g[:-1], lambda g: g[:, None], lambda g: torch.cat([g, g[:1]])):
+        for need_grad in (True, False):
+            with pytest.raises((RuntimeError, IndexError, ValueError, TypeError)):
+                passes(index, need_grad)
+
+    def twice(g):
+        g = g.clone()
+        g[-1] = g[0]
+        return g
+    g = passes(twice)[1]
+    last = mols == 39
+    assert torch.isnan(g[last]).any() and not torch.isnan(g[~last]).any()
