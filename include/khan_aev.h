@@ -102,7 +102,7 @@ int khan_prepare_batch(const int32_t *mol_idxs, const int32_t *atomic_numbers, i
  * out: h_feat[acs[0]*384], c_feat[acs[1]*384], n_feat[acs[2]*384], o_feat[acs[3]*384], row-major;
  *      the row of atom g is bucket[as[g]] + sis[g]*384.
  * Scratch, from the stream-ordered allocator on every call: the molecule indices in order of decreasing size, and,
- * for molecules of more than 256 atoms, a sorted copy of the atoms (about 21 bytes per atom and 32 per molecule of the batch in float32, 37 per atom in
+ * for molecules of more than 256 atoms, a sorted copy of the atoms (about 23 bytes per atom and 32 per molecule of the batch in float32, 39 per atom in
  * float64; in the backward pass 16 and 32 more per atom, the forces on it, where the host knows the size classes).  While the stream is being captured into a graph neither is taken: molecules then run in the order given,
  * and those of more than 256 atoms in slower kernels that need no scratch.
  * Precondition for batches with molecules of more than 256 atoms: mos increases with the molecule index and the

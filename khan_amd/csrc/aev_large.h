@@ -14,37 +14,18 @@
 namespace khan {
 
 // The work of the kernels for large molecules: a workgroup is one wavefront and takes runs of 2^log_run (up to kRunCentres)
-// consecutive sorted atoms of a molecule, which lie close together.  Runs are numbered by the chunks' boxes (chunk_base), so that a
-// run's molecule is found by bisection of the offsets; numbers between the molecules' ranges, and those of molecules of up to 256
-// atoms, belong to no run.
+// consecutive sorted atoms of a molecule, which lie close together.
 // (A molecule to a column of 64 workgroups and 32 columns side by side kept 62 % of the wavefront slots busy on 64 boxes of
 // 1,024-4,096 atoms: a column's molecules add up as they come.)
-constexpr int kRunCentres = 4;
+constexpr int kLogRunCentres = 2, kRunCentres = 1 << kLogRunCentres;
 constexpr int kMaxCandidates = 176;        // atoms in reach of a run's centres (list_candidates)
 
-struct Runs {
-    int log_run;
-    int64_t count;                         // the numbers of runs, those that belong to none among them
-    unsigned blocks;                       // workgroups
-    bool sure;                             // the batch holds large molecules
-};
-
-// Runs of 2^log_run atoms (less than 0: by the batch).  Long ones share a list of candidates, short ones spread a small batch over
-// the GPU, where a centre takes 8-10 us whatever goes on beside it (forward / backward with the sort, us, runs of 4, 2 and 1; boxes of
+// Long runs share a list of candidates, short ones spread a small batch over the GPU, where a centre takes 8-10 us whatever goes on
+// beside it.  By the atoms of the large molecules (forward / backward with the sort, us, runs of 4, 2 and 1; boxes of
 // 1,024-4,096 atoms in float32: 171,000 atoms 277 / 348, 302 / 394, 377 / 503; 64,000 143 / 171, 145 / 180, 173 / 219; 21,000
 // 103 / 111, 88 / 100, 91 / 111; 8,000 81 / 86, 63 / 71, 60 / 70; 2,700 78 / 83, 58 / 64, 48 / 53; in float64 43,000 211 / 241,
-// 210 / 247, 245 / 303).  Where the host does not know that the batch holds such molecules (`sure`) the workgroups are fewer: they
-// mostly find nothing to do.
-__host__ inline Runs runs_of(int64_t n_atoms, int32_t n_mols, bool sure, int log_run = -1)
-{
-    Runs r;
-    r.log_run = log_run >= 0 ? log_run : n_atoms >= 40000 ? 2 : n_atoms >= 9000 ? 1 : 0;
-    r.count = ((n_atoms >> 6) + n_mols + 1) << (6 - r.log_run);
-    r.sure = sure;
-    const int64_t most = sure ? 16384 : 4096;
-    r.blocks = static_cast<unsigned>(r.count < most ? (r.count + 7) / 8 * 8 : most);
-    return r;
-}
+// 210 / 247, 245 / 303), and not by those of the batch.
+__device__ __forceinline__ int log_run_for(int64_t atoms) { return atoms >= 40000 ? 2 : atoms >= 9000 ? 1 : 0; }
 
 // An atom's type and its scatter index (the row inside its type's bucket) in one word, which travels with the coordinates: a
 // partner's row and block are known where it is found.  (Rows fit 28 bits: 2^28 of them are 400 GB.)
@@ -62,7 +43,11 @@ struct SortedAtoms {
     typename Fast<T>::vec4* force;  // the sum of the forces on it (backward pass, see there), else null
     int* index;                     // its index in the batch
     float4* box;                    // per chunk of 64 sorted atoms: lowest x, y, z and highest x, y, z (two entries)
-    Runs runs;                      // the split of the work
+    // The large molecules cut into units of kRunCentres sorted atoms (the last one of a molecule may be shorter), one after the other: molecule,
+    // and 4 x first sorted atom + atoms - 1.  A run is a unit or an even part of one.
+    int2* unit;
+    int* n_units;
+    int most_units;                 // that there is room for
 };
 
 // The atoms are ordered along a space-filling curve (up to 16 x 16 x 16 cells over the molecule's extent, Morton order;
@@ -76,17 +61,21 @@ constexpr int kSortCells = kSortCellsPerDim * kSortCellsPerDim * kSortCellsPerDi
 
 __host__ __device__ __forceinline__ size_t round_up_256(size_t v) { return (v + 255u) & ~static_cast<size_t>(255u); }
 
+// a unit per four atoms, and one more per molecule of more than 256
+__host__ inline int64_t most_units(int64_t n_atoms) { return n_atoms / kRunCentres + n_atoms / (kMediumMaxAtoms + 1); }
+
 template <typename T>
 __host__ inline size_t sorted_atoms_bytes(int64_t n_atoms, int32_t n_mols, bool with_vectors)
 {
     const size_t vec = round_up_256(sizeof(typename Fast<T>::vec4) * static_cast<size_t>(n_atoms));
     return vec * (with_vectors ? 2 : 1) + round_up_256(sizeof(int) * static_cast<size_t>(n_atoms)) +
-           round_up_256(2 * sizeof(float4) * (static_cast<size_t>(n_atoms) / 64 + static_cast<size_t>(n_mols) + 1));
+           round_up_256(2 * sizeof(float4) * (static_cast<size_t>(n_atoms) / 64 + static_cast<size_t>(n_mols) + 1)) +
+           256 + sizeof(int2) * static_cast<size_t>(most_units(n_atoms));
 }
 
 // the arrays inside one allocation of sorted_atoms_bytes (256-byte aligned)
 template <typename T>
-__host__ inline SortedAtoms<T> carve_sorted_atoms(void* scratch, int64_t n_atoms, int32_t n_mols, bool sure, bool with_vel, bool with_force)
+__host__ inline SortedAtoms<T> carve_sorted_atoms(void* scratch, int64_t n_atoms, int32_t n_mols, bool with_vel, bool with_force)
 {
     typedef typename Fast<T>::vec4 vec4;
     char* p = static_cast<char*>(scratch);
@@ -100,7 +89,10 @@ __host__ inline SortedAtoms<T> carve_sorted_atoms(void* scratch, int64_t n_atoms
     s.index = reinterpret_cast<int*>(p);
     p += round_up_256(sizeof(int) * static_cast<size_t>(n_atoms));
     s.box = reinterpret_cast<float4*>(p);
-    s.runs = runs_of(n_atoms, n_mols, sure);
+    p += round_up_256(2 * sizeof(float4) * (static_cast<size_t>(n_atoms) / 64 + static_cast<size_t>(n_mols) + 1));
+    s.n_units = reinterpret_cast<int*>(p);
+    s.unit = reinterpret_cast<int2*>(p + 256);
+    s.most_units = static_cast<int>(most_units(n_atoms));
     return s;
 }
 
@@ -115,46 +107,42 @@ __device__ __forceinline__ bool in_reach(const float (&lo)[3], const float (&hi)
     return dx * dx + dy * dy + dz * dz < reach * reach;
 }
 
-// Calls body(molecule, first sorted atom of the run) for the workgroup's runs.
-template <typename Body>
-__device__ __forceinline__ void for_each_run(const int32_t* __restrict__ MOs, const int32_t* __restrict__ MACs, int32_t n_mols,
-                                             const Runs& runs, const int32_t* __restrict__ size_counts, Body body)
+// Workgroups for the runs of a batch of n_atoms.  Where the host does not know that it holds large molecules (`sure`) they are fewer: they
+// mostly find nothing to do.
+__host__ inline dim3 run_grid(int64_t n_atoms, bool sure)
+{
+    const int64_t most = sure ? 16384 : 4096;
+    return dim3(static_cast<unsigned>(n_atoms < most ? (n_atoms + 7) / 8 * 8 : most));
+}
+
+// Calls body(molecule, first sorted atom of the run, log2 of a run's atoms) for the workgroup's runs.
+// (The units are listed beside the sort, by a workgroup of its own.  Numbers for all atoms of the batch, a run's molecule found by
+// bisection of the offsets, have most of the numbers of a mixed batch belong to no run, and the others may lie in one of the eight parts
+// below: 100 molecules of 300 atoms behind 3,400 small ones, forward / backward with theirs, 308 / 387 us, so 103 / 134; one of
+// 2,700 122 / 159 and 85 / 105; 64 boxes of 1,024-4,096 atoms alone 252 and 245, 312 and 305 the kernels by themselves.)
+template <typename T, typename Body>
+__device__ __forceinline__ void for_each_run(const SortedAtoms<T>& sorted, Body body)
 {
     const int lane = threadIdx.x & 63;
-    // is there a large molecule at all?
-    if (size_counts) {
-        if (size_counts[size_bin(kMediumMaxAtoms + 1)] == 0) return;
-    } else if (!runs.sure) {
-        int most = 0;
-#pragma unroll 4
-        for (int m = lane; m < n_mols; m += 64) most = max(most, MACs[m]);
-        if (wave_ballot(most > kMediumMaxAtoms) == 0ull) return;
-    }
+    const int units = uniform(*sorted.n_units);
+    const int log_run = log_run_for(static_cast<int64_t>(units) << kLogRunCentres), log_parts = kLogRunCentres - log_run;
     // Workgroup w is on XCD w % 8: an XCD's workgroups take consecutive runs, whose atoms and rows its L2 then holds (64 boxes of
     // 1,024-4,096 atoms, backward 371 -> 358 us).
-    const int64_t each = (runs.count + 7) >> 3;
-    for (int64_t base = blockIdx.x; base < 8 * each; base += static_cast<int64_t>(gridDim.x) * 64) {
-        const int64_t number = base + static_cast<int64_t>(lane) * gridDim.x;
-        const int64_t at = (number & 7) * each + (number >> 3);
+    const int count = units << log_parts, each = (count + 7) >> 3;
+    for (int base = blockIdx.x; base < 8 * each; base += static_cast<int>(gridDim.x) * 64) {
+        const int number = base + lane * static_cast<int>(gridDim.x), at = (number & 7) * each + (number >> 3);
         int mol = 0, first = 0;
-        bool mine = false;
-        if (number < 8 * each && at < runs.count) {
-            // the last molecule whose chunks begin at or before this run's
-            const int64_t chunk = at >> (6 - runs.log_run);
-            int hi = n_mols;                           // its number is in [mol, hi)
-            while (hi - mol > 1) {
-                const int mid = mol + ((hi - mol) >> 1);
-                if (static_cast<int64_t>(chunk_base(MOs[mid], mid)) <= chunk) mol = mid;
-                else hi = mid;
-            }
-            const int n = MACs[mol];
-            const int64_t from = (at << runs.log_run) - 64 * static_cast<int64_t>(chunk_base(MOs[mol], mol));
-            mine = n > kMediumMaxAtoms && from >= 0 && from < n;
-            first = mine ? static_cast<int>(from) : 0;
+        bool mine = number < 8 * each && at < count;
+        if (mine) {
+            const int2 u = sorted.unit[at >> log_parts];
+            const int part = (at & ((1 << log_parts) - 1)) << log_run;
+            mol = u.x;
+            first = (u.y >> kLogRunCentres) + part;
+            mine = part <= (u.y & (kRunCentres - 1));
         }
         for (unsigned long long left = wave_ballot(mine); left; left &= left - 1) {
             const int b = lowest_bit(left);
-            body(lane_read(mol, b), lane_read(first, b));
+            body(lane_read(mol, b), lane_read(first, b), log_run);
         }
     }
 }

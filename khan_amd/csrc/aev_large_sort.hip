@@ -1,6 +1,8 @@
 // Sorted copies of the molecules of more than 256 atoms, for the workgroup-per-molecule AEV kernels (aev_large.h).
 // One workgroup per molecule: a counting sort by (cell along a space-filling curve, atom type) that keeps the atoms'
-// order inside a bin, and the box around every 64 consecutive sorted atoms.
+// order inside a bin, and the box around every 64 consecutive sorted atoms; and the list of what those kernels share out among them.
+#include <algorithm>
+
 #include "aev_large.h"
 #include "khan_params.h"
 
@@ -22,6 +24,44 @@ __device__ __forceinline__ float wave_maxf(float v)
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) v = fmaxf(v, __shfl_xor(v, d, 64));
     return v;
+}
+
+// Lists the units of the large molecules (SortedAtoms): kListers workgroups, each of which goes through all molecules, 256 at a time, and
+// writes its share of every one's units (one workgroup alone takes 44 us for the 43,000 units of 64 boxes of 1,024-4,096 atoms).
+constexpr int kListers = 16;
+template <typename T>
+__device__ __forceinline__ void list_units(const int32_t* __restrict__ MACs, int32_t n_mols, const int32_t* __restrict__ order, const SortedAtoms<T>& sorted,
+                                           int (&wave_units)[4])
+{
+    const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
+    const int count = order ? order[n_mols + size_bin(kMediumMaxAtoms + 1)] : n_mols;      // (they are the first of the order)
+    int total = 0;
+    for (int m0 = 0; m0 < count; m0 += 256) {
+        const int m = m0 + tid;
+        const int mol = m < count ? (order ? order[m] : m) : 0, n = m < count ? MACs[mol] : 0;
+        const int units = n > kMediumMaxAtoms ? (n + kRunCentres - 1) >> kLogRunCentres : 0;
+        int end = units;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int before = __shfl_up(end, d, 64);
+            end += lane >= d ? before : 0;
+        }
+        if (lane == 63) wave_units[wave] = end;
+        __syncthreads();
+        const int all[4] = {wave_units[0], wave_units[1], wave_units[2], wave_units[3]};
+        const int begin = total + (wave > 0 ? all[0] : 0) + (wave > 1 ? all[1] : 0) + (wave > 2 ? all[2] : 0) + end - units;
+        for (unsigned long long left = wave_ballot(units > 0); left; left &= left - 1) {
+            const int b = lowest_bit(left), of = lane_read(mol, b), atoms = lane_read(n, b), at = lane_read(begin, b), most = lane_read(units, b);
+            for (int u = 64 * static_cast<int>(blockIdx.x) + lane; u < most; u += 64 * kListers) {
+                const int first = u << kLogRunCentres;
+                // (more than there is room for: the molecules overlap)
+                if (at + u < sorted.most_units) sorted.unit[at + u] = make_int2(of, (first << kLogRunCentres) + min(atoms - first, kRunCentres) - 1);
+            }
+        }
+        total += (all[0] + all[1]) + (all[2] + all[3]);
+        __syncthreads();                        // the next 256 molecules' counts go to the same places
+    }
+    if (blockIdx.x == 0 && tid == 0) *sorted.n_units = min(total, sorted.most_units);
 }
 
 constexpr int kListedAtoms = 64;      // of a bin, at most, where atoms are ranked by their bins' lists
@@ -46,6 +86,10 @@ __global__ __launch_bounds__(256) void large_sort_kernel(
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = uniform(tid >> 6);
+    if (blockIdx.y == 0) {                     // (the first to start)
+        if (blockIdx.x < kListers) list_units(MACs, n_mols, order, sorted, wsum);
+        return;
+    }
     for_each_molecule_in_range(MACs, n_mols, kMediumMaxAtoms + 1, INT32_MAX, want, order, order ? order + n_mols : nullptr, [&](int mol) {
         const int n = uniform(MACs[mol]);
         const int off = uniform(MOs[mol]);
@@ -306,7 +350,7 @@ hipError_t launch_large_sort(const T* X, const T* Y, const T* Z, const int32_t* 
 {
     if (n_mols <= 0) return hipSuccess;
     const unsigned blocks = static_cast<unsigned>(n_mols < 1024 ? n_mols : 1024);
-    large_sort_kernel<T><<<dim3(blocks), dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, VX, VY, VZ, gX, gY, gZ,
+    large_sort_kernel<T><<<dim3(std::max(blocks, static_cast<unsigned>(kListers)), 2), dim3(256), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, VX, VY, VZ, gX, gY, gZ,
                                                              order, sorted);
     return hipGetLastError();
 }

@@ -82,7 +82,7 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
 
     fwd_lds_init(S, lane);
     // (kLarge: of a run of the molecule's sorted atoms, from run_first on)
-    const auto run_molecule = [&](int mol, int run_first) {
+    const auto run_molecule = [&](int mol, int run_first, int log_run) {
         const int n = uniform(MACs[mol]);
         const int off = uniform(MOs[mol]);
 
@@ -458,7 +458,7 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
         if constexpr (kLarge) {
             // the run with its candidates, or, where the atoms are too close together for a list, shorter ones
             static_assert(!kLarge || kRunCentres <= kNB, "a run is a batch: its candidates lie where the records go");
-            const int run_end = min(n, run_first + (1 << sorted.runs.log_run));
+            const int run_end = min(n, run_first + (1 << log_run));
             for (int from = run_first, length = run_end - run_first; from < run_end;) {
                 const int to = min(from + length, run_end);
                 const int n_candidates = list_candidates<T, kJvp>(sorted, off, n, chunk0, from, to, M.candidates, S.template atoms<kMaxCandidates>(),
@@ -479,11 +479,11 @@ __global__ __launch_bounds__(kLarge ? 64 : 256, kLarge && !kJvp && sizeof(T) == 
         }
     };
     if constexpr (kLarge) {
-        for_each_run(MOs, MACs, n_mols, sorted.runs, order ? order + n_mols : nullptr, run_molecule);
+        for_each_run(sorted, run_molecule);
     } else {
         __shared__ unsigned long long want[4];
         for_each_molecule_in_range(MACs, n_mols, min_atoms, kMediumMaxAtoms, want, order, order ? order + n_mols : nullptr,
-                                   [&](int mol) { run_molecule(mol, 0); });
+                                   [&](int mol) { run_molecule(mol, 0, 0); });
     }
 }
 
@@ -549,11 +549,11 @@ hipError_t launch_fwd_large(const T* X, const T* Y, const T* Z, const int32_t* A
 {
     if (n_mols <= 0) return hipSuccess;
     const bool jvp = VX != nullptr;
-    const SortedAtoms<T> sorted = carve_sorted_atoms<T>(scratch, n_atoms, n_mols, sure, jvp, false);
+    const SortedAtoms<T> sorted = carve_sorted_atoms<T>(scratch, n_atoms, n_mols, jvp, false);
     const hipError_t e = launch_large_sort<T>(X, Y, Z, A, MOs, MACs, n_mols, SIs, VX, VY, VZ, nullptr, nullptr, nullptr, order,
                                               sorted, stream);
     if (e != hipSuccess) return e;
-    const dim3 grid(sorted.runs.blocks);
+    const dim3 grid = run_grid(n_atoms, sure);
     if (jvp)
         aev_fwd_medium_kernel<T, true, true><<<grid, dim3(64), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, VX, VY, VZ, out,
                                                                          kMediumMaxAtoms + 1, order, sorted);

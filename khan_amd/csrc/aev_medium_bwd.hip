@@ -130,7 +130,7 @@ void aev_bwd_medium_kernel(
         }
     };
     // (kLarge: of a run of the molecule's sorted atoms, from run_first on)
-    const auto run_molecule = [&](int mol, int run_first) {
+    const auto run_molecule = [&](int mol, int run_first, int log_run) {
         const int n = uniform(MACs[mol]);
         const int off = uniform(MOs[mol]);
         int tb1, tb2, tb3;                     // sorted position of the first C, N, O atom
@@ -614,7 +614,7 @@ void aev_bwd_medium_kernel(
         };
         if constexpr (kLarge) {
             // the run with its candidates, or, where the atoms are too close together for a list, shorter ones
-            const int run_end = min(n, run_first + (1 << sorted.runs.log_run));
+            const int run_end = min(n, run_first + (1 << log_run));
             if (lane < run_end - run_first) M.centre_word[lane] = atom_word(sorted.atom[off + run_first + lane].w);
             if (lane < 4 * kRunCentres) M.centre_force[lane >> 2][lane & 3] = T(0);
             wave_lds_fence();
@@ -644,30 +644,35 @@ void aev_bwd_medium_kernel(
         if constexpr (!kLarge) __syncthreads();      // the next molecule reuses the sorted arrays
     };
     if constexpr (kLarge) {
-        for_each_run(MOs, MACs, n_mols, sorted.runs, order ? order + n_mols : nullptr, run_molecule);
+        for_each_run(sorted, run_molecule);
     } else {
         __shared__ unsigned long long want[4];
         for_each_molecule_in_range(MACs, n_mols, min_atoms, kMediumMaxAtoms, want, walk_in_order ? order : nullptr,
-                                   order ? order + n_mols : nullptr, [&](int mol) { run_molecule(mol, 0); });
+                                   order ? order + n_mols : nullptr, [&](int mol) { run_molecule(mol, 0, 0); });
     }
 }
 
-// The forces on the sorted atoms of large molecules, 64 to a workgroup, added to the gradients (which hold what the general per-centre
+// The forces on the sorted atoms of large molecules, an atom to a thread, added to the gradients (which hold what the general per-centre
 // routine has added).
 template <typename T>
-__global__ __launch_bounds__(64) void large_force_kernel(const int32_t* __restrict__ MOs, const int32_t* __restrict__ MACs, int32_t n_mols,
-                                                         T* __restrict__ gX, T* __restrict__ gY, T* __restrict__ gZ,
-                                                         const int32_t* __restrict__ order, const SortedAtoms<T> sorted)
+__global__ __launch_bounds__(256) void large_force_kernel(const int32_t* __restrict__ MOs, T* __restrict__ gX, T* __restrict__ gY, T* __restrict__ gZ,
+                                                          const SortedAtoms<T> sorted)
 {
-    for_each_run(MOs, MACs, n_mols, sorted.runs, order ? order + n_mols : nullptr, [&](int mol, int first) {
-        const int j = first + static_cast<int>(threadIdx.x);
-        if (j >= uniform(MACs[mol])) return;
-        const int at = uniform(MOs[mol]) + j, g = sorted.index[at];
+    // (an eighth of the atoms to each XCD, as in for_each_run: a molecule's gradients are lines of one L2; 10.6 -> 6.1 us for 64
+    // boxes of 1,024-4,096 atoms)
+    const int units = *sorted.n_units, each = (units + 8 * 64 - 1) / (8 * 64);
+    for (int b = blockIdx.x; b < 8 * each; b += static_cast<int>(gridDim.x)) {
+        const int i = ((b & 7) * each + (b >> 3)) * 64 + static_cast<int>(threadIdx.x >> kLogRunCentres);
+        if (i >= units) continue;
+        const int2 u = sorted.unit[i];
+        const int part = threadIdx.x & (kRunCentres - 1);
+        if (part > (u.y & (kRunCentres - 1))) continue;
+        const int at = MOs[u.x] + (u.y >> kLogRunCentres) + part, g = sorted.index[at];
         const typename Fast<T>::vec4 f = sorted.force[at];
         gX[g] += f.x;
         gY[g] += f.y;
         gZ[g] += f.z;
-    });
+    }
 }
 
 // Zeroes the gradients of the molecules of min_atoms to 256 atoms, for launches whose workgroups share molecules.
@@ -728,16 +733,16 @@ hipError_t launch_bwd_large(const T* X, const T* Y, const T* Z, const int32_t* A
 {
     if (n_mols <= 0) return hipSuccess;
     // (a batch that may hold no such molecule goes without the kernel behind this one)
-    SortedAtoms<T> sorted = carve_sorted_atoms<T>(scratch, n_atoms, n_mols, sure, false, sure);
+    const SortedAtoms<T> sorted = carve_sorted_atoms<T>(scratch, n_atoms, n_mols, false, sure);
     const hipError_t e = launch_large_sort<T>(X, Y, Z, A, MOs, MACs, n_mols, SIs, nullptr, nullptr, nullptr, gX, gY, gZ, order,
                                               sorted, stream);
     if (e != hipSuccess) return e;
-    const dim3 grid(sorted.runs.blocks);
+    const dim3 grid = run_grid(n_atoms, sure);
     aev_bwd_medium_kernel<T, true><<<grid, dim3(64), 0, stream>>>(X, Y, Z, A, MOs, MACs, n_mols, SIs, g, gX, gY, gZ,
                                                                   kMediumMaxAtoms + 1, order, false, sorted);
     if (!sure) return hipGetLastError();
-    sorted.runs = runs_of(n_atoms, n_mols, true, 6);
-    large_force_kernel<T><<<dim3(sorted.runs.blocks), dim3(64), 0, stream>>>(MOs, MACs, n_mols, gX, gY, gZ, order, sorted);
+    const int64_t blocks = (most_units(n_atoms) + 8 * 64 - 1) / (8 * 64) * 8;
+    large_force_kernel<T><<<dim3(static_cast<unsigned>(blocks < 4096 ? blocks : 4096)), dim3(256), 0, stream>>>(MOs, gX, gY, gZ, sorted);
     return hipGetLastError();
 }
 

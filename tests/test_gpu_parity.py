@@ -970,12 +970,12 @@ def test_runs_of_large_molecules(ops, dtype, copies):
 
 
 # A row and a Jacobian-vector product of a large molecule are the same bits whatever else is in the batch: in runs of one, two and four
-# centres (batches of up to 9,000, 40,000 and more atoms), beside small molecules, and with the classes unknown to the host.  Radial
-# lists hold 64 partners: the lattice's centres have about 41, 85 and 120.
+# centres (up to 9,000, 40,000 and more atoms of large molecules), beside small molecules, with the classes unknown to the host, and on both
+# sides of the 256 molecules whose runs are listed at a time.  Radial lists hold 64 partners: the lattice's centres have about 41, 85 and 120.
 @pytest.mark.parametrize("spacing", [2.15, 1.7, 1.5])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
 def test_rows_of_large_molecules_are_the_same_bits_in_any_batch(ops, dtype, spacing):
-    say("case: one molecule of 700 atoms, spacing %g, in batches of 1 to 58 copies, %s" % (spacing, dtype))
+    say("case: one molecule of 700 atoms, spacing %g, in batches of 1 to 300 copies, %s" % (spacing, dtype))
     rng = np.random.default_rng(41)
     n = 700
     xyz = _jittered_lattice(rng, n, spacing, 0.2)
@@ -997,9 +997,47 @@ def test_rows_of_large_molecules_are_the_same_bits_in_any_batch(ops, dtype, spac
                 for f in (ops.featurize(*args, **kw), ops.featurize_grad_inverse(*args, *v, **kw))]
 
     first = rows_of(1, 0, True)
-    for copies, smalls, known in ((1, 0, False), (3, 40, True), (13, 0, True), (13, 2000, True), (58, 0, True), (58, 0, False), (2, 6000, True), (1, 6000, False)):
+    for copies, smalls, known in ((1, 0, False), (3, 40, True), (13, 0, True), (13, 2000, True), (58, 0, True), (58, 0, False), (2, 6000, True), (1, 6000, False),
+                                   (70, 3000, True), (70, 3000, False), (256, 9, True), (300, 300, True)):
         for got, want in zip(rows_of(copies, smalls, known), first):
             assert bool((got == want).all()), (copies, smalls, known, int((got != want).sum()))
+
+
+def test_large_molecules_among_small_ones_take_no_longer_than_apart(ops):
+    # 100 molecules of 300 atoms behind 3,400 small ones: forward, backward and Jacobian-vector passes against those of the two batches
+    # by themselves, one after the other (the quickest of ten).  Sharing out the large ones by the whole batch's atoms had them in one
+    # eighth of the GPU, 2.6 times as long; together they take less than apart.
+    say("case: 100 molecules of 300 atoms behind 3,400 small ones, timed against both alone")
+    rng = np.random.default_rng(19)
+    small = datagen.make_batch("organic", 3400)
+    large = [(rng.choice(4, 300, p=[0.5, 0.3, 0.1, 0.1]), _jittered_lattice(rng, 300, 2.15, 0.5)) for _ in range(100)]
+
+    def passes_of(parts):
+        A, xyz, sizes = np.concatenate([p[0] for p in parts]), np.concatenate([p[1] for p in parts]), np.concatenate([p[2] for p in parts])
+        c = Case(*xyz.T, A, np.repeat(np.arange(len(sizes)), sizes), len(sizes))
+        macs, mos, sc, ga, ac = gpu_sort_offsets(ops, c)
+        order = ops.size_order(macs)
+        args, kw = (*(dev(v).float() for v in (c.X, c.Y, c.Z)), dev(c.A), mos, macs, sc, ac.cpu()), dict(order=order, size_classes=order[-4:].cpu())
+        up, v = ops.featurize(*args, **kw), [dev(rng.standard_normal(c.N)).float() for _ in range(3)]
+        return [lambda: ops.featurize(*args, **kw), lambda: ops.featurize_grad(*args, *up, **kw), lambda: ops.featurize_grad_inverse(*args, *v, **kw)]
+
+    def quickest(f):
+        times = []
+        for _ in range(10):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(5):
+                f()
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end) / 5)
+        return min(times)
+
+    parts = [(small.A, np.stack([small.X, small.Y, small.Z], axis=1), small.MACs),
+             (np.concatenate([m[0] for m in large]), np.concatenate([m[1] for m in large]), np.full(100, 300))]
+    for apart, together in zip(zip(passes_of(parts[:1]), passes_of(parts[1:])), passes_of(parts)):
+        limit = 1.5 * sum(quickest(f) for f in apart)
+        assert quickest(together) <= limit
 
 
 # Both sides of each line between the forward kernels: 174,763 atoms in float32 (87,382 in float64) make 256 MB of rows, 43,691
