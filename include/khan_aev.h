@@ -340,9 +340,9 @@ int khan_dense_head_grad_f32(const float *const *scale_host4, const float *const
  * (layer by layer, khan_dense_f32 and khan_dense_head_f32 write every activation and read it twice).  It is the pass of
  * energy-and-force inference (energy_server.py:141-187): the values summed by molecule are the energies, and grad with
  * scale = 1 is what khan_featurize_grad_f32 takes as its upstream rows.
- * The products are float32 products to float32 accuracy, formed on the half-precision matrix instructions: every float32
- * operand x is split into h = half(x) and l = half(2^11 (x - h)) (x - h - 2^-11 l is at most 2^-24 |x|), and three of
- * the four partial products are accumulated in float32 (the fourth is below 2^-24 of the product).  OPERAND RANGE: a
+ * The products are float32 products to within 2^-21 of each, formed on the half-precision matrix instructions: every float32
+ * operand x is split into h = half(x) and l = half(2^11 (x - h)) (x - h - 2^-11 l is at most 2^-23 |x|), and three of
+ * the four partial products are accumulated in float32 (the fourth is at most 2^-22 of the product).  OPERAND RANGE: a
  * feature, activation or weight of 65,504 or more in size (half precision's largest number) makes that row's value and
  * gradient NaN -- never a wrong finite number, and no other row's; an operand below 6e-5 in size keeps an absolute
  * accuracy of 2^-36 instead of a relative one (it then no longer counts beside the row's other terms).  The gradient

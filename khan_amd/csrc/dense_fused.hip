@@ -15,14 +15,14 @@
 // (v_mfma_f32_32x32x16_f16, sixteen times the rate of the float32 ones) with every float32 operand split into two
 // half-precision parts:
 //     x = h + 2^-11 l,   h = half(x),   l = half(2^11 (x - h))
-// h carries 11 significant bits, x - h is exact in float32 and at most 2^-12 |x|, and l carries its 11 leading bits:
-// |x - h - 2^-11 l| <= 2^-24 |x|, the rounding of float32 itself.  The residual is scaled by 2^11 so that it has
+// h carries 11 significant bits, x - h is exact in float32 and at most 2^-11 |x|, and l carries its 11 leading bits:
+// |x - h - 2^-11 l| <= 2^-23 |x|, and 0 for three values of four (where x - h needs a twelfth bit, the last one goes).  The residual is scaled by 2^11 so that it has
 // x's exponent and not one twelve binary orders below it, where half precision would run out of exponent for every
 // |x| < 0.25.  Of the four partial products of x w three are kept, each an exact 22-bit product accumulated in
 // float32, in two accumulators:
-//     hi += h_x h_w,   lo += h_x l_w + l_x h_w,   x w ~ hi + 2^-11 lo      (left out: l_x l_w 2^-22 <= 2^-24 |x w|)
-// which is a float32 product to float32 accuracy (three terms of 2^-24 |x w| each) from three matrix instructions;
-// the three-way bfloat16 split of dense_first.hip needs six.  What it costs is range: half precision ends at 65,504,
+//     hi += h_x h_w,   lo += h_x l_w + l_x h_w,   x w ~ hi + 2^-11 lo      (left out: l_x l_w 2^-22 <= 2^-22 |x w|)
+// which is a float32 product to within 2^-21 |x w| (a term of 2^-22 and two of 2^-23) from three matrix instructions;
+// the three-way bfloat16 split of dense_first.hip, which keeps every bit of the operands, needs six.  What it costs is range: half precision ends at 65,504,
 // so an operand (feature, activation, weight) of that size or more gives NaN -- never a wrong finite number -- and an
 // |x| below 6e-5 keeps an absolute accuracy of 2^-36 instead of a relative one.  On the way back the gradient is
 // carried for a unit upstream factor and multiplied by the row's factor only when it is stored (the pass is linear

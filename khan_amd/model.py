@@ -266,7 +266,7 @@ class AniModel:
             return [energies] + parts
         acs, order, classes = b._counts(waited)
         # Networks beside a charge network have products of all 24 bits over float32's range (net_chain.hip, or layer by
-        # layer), where the one-launch kernel's operands keep 2^-24 of their size between 6e-5 and 65,504.
+        # layer), where the one-launch kernel's operands are off by up to 2^-23 of their size between 6e-5 and 65,504.
         alone = self.charge is None
         return _native.load().infer(
             b.xs, b.ys, b.zs, b.atom_types, b.mol_offsets, b.mol_atom_counts, b.scatter_idxs, b.gather_idxs, acs, order, classes,
