@@ -445,7 +445,7 @@ int khan_net_few_f64(const khan_net_few *net, khan_stream_t stream);
 /* Whole networks with CELU in float32 for inference, all layers in one launch each way (a workgroup per 32 or 64 rows of a type).
  * `layers` products of the widths `widths` (the last 1), w[l][t] [in, out] and b[l][t] of layer l and type t (b NULL: zeros).
  * khan_net_chain_fits: 1 for widths it takes: the first a multiple of 128, the hidden ones up to 256.  x and grad must be 16-byte
- * aligned.  Operands are the exact sums of three bfloat16 values (what the third would need below 2^-133 is lost); those from 2^128 (1 - 2^-9)
+ * aligned.  Operands are the exact sums of three bfloat16 values (parts below 2^-126 may be lost); those from 2^128 (1 - 2^-9)
  * on, and infinite ones, give NaN.  A bit l of `absolute`: the CELU of hidden layer
  * l is formed as alpha (exp(z / alpha) - 1), with an absolute error of 2^-24 alpha (KHAN_NET_CELU_ABSOLUTE).
  * khan_net_chain_values_f32 packs the weights into `workspace` (khan_net_chain_workspace_bytes(), 16-byte aligned) and forms value;

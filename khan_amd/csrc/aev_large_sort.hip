@@ -26,20 +26,29 @@ __device__ __forceinline__ float wave_maxf(float v)
     return v;
 }
 
-// Lists the units of the large molecules (SortedAtoms): kListers workgroups, each of which goes through all molecules, 256 at a time, and
+// Lists the units of the large molecules (SortedAtoms): kListers workgroups, each of which goes through all molecules, 2,048 at a time, and
 // writes its share of every one's units (one workgroup alone takes 44 us for the 43,000 units of 64 boxes of 1,024-4,096 atoms).
 constexpr int kListers = 16;
 template <typename T>
 __device__ __forceinline__ void list_units(const int32_t* __restrict__ MACs, int32_t n_mols, const int32_t* __restrict__ order, const SortedAtoms<T>& sorted,
                                            int (&wave_units)[4])
 {
+    constexpr int kEach = 8;                    // molecules of a thread, their loads in flight together (without an order all have to be looked at)
     const int tid = threadIdx.x, lane = tid & 63, wave = uniform(tid >> 6);
     const int count = order ? order[n_mols + size_bin(kMediumMaxAtoms + 1)] : n_mols;      // (they are the first of the order)
     int total = 0;
-    for (int m0 = 0; m0 < count; m0 += 256) {
-        const int m = m0 + tid;
-        const int mol = m < count ? (order ? order[m] : m) : 0, n = m < count ? MACs[mol] : 0;
-        const int units = n > kMediumMaxAtoms ? (n + kRunCentres - 1) >> kLogRunCentres : 0;
+    for (int64_t m0 = 0; m0 < count; m0 += kEach * 256) {
+        int mol[kEach], n[kEach], units = 0;
+#pragma unroll
+        for (int k = 0; k < kEach; ++k) {
+            const int64_t m = m0 + k * 256 + tid;
+            mol[k] = m < count ? (order ? order[m] : static_cast<int>(m)) : -1;
+        }
+#pragma unroll
+        for (int k = 0; k < kEach; ++k) n[k] = mol[k] >= 0 ? MACs[mol[k]] : 0;
+        const auto units_of = [](int atoms) { return atoms > kMediumMaxAtoms ? (atoms + kRunCentres - 1) >> kLogRunCentres : 0; };
+#pragma unroll
+        for (int k = 0; k < kEach; ++k) units += units_of(n[k]);
         int end = units;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
@@ -49,17 +58,21 @@ __device__ __forceinline__ void list_units(const int32_t* __restrict__ MACs, int
         if (lane == 63) wave_units[wave] = end;
         __syncthreads();
         const int all[4] = {wave_units[0], wave_units[1], wave_units[2], wave_units[3]};
-        const int begin = total + (wave > 0 ? all[0] : 0) + (wave > 1 ? all[1] : 0) + (wave > 2 ? all[2] : 0) + end - units;
-        for (unsigned long long left = wave_ballot(units > 0); left; left &= left - 1) {
-            const int b = lowest_bit(left), of = lane_read(mol, b), atoms = lane_read(n, b), at = lane_read(begin, b), most = lane_read(units, b);
-            for (int u = 64 * static_cast<int>(blockIdx.x) + lane; u < most; u += 64 * kListers) {
-                const int first = u << kLogRunCentres;
-                // (more than there is room for: the molecules overlap)
-                if (at + u < sorted.most_units) sorted.unit[at + u] = make_int2(of, (first << kLogRunCentres) + min(atoms - first, kRunCentres) - 1);
+        int begin = total + (wave > 0 ? all[0] : 0) + (wave > 1 ? all[1] : 0) + (wave > 2 ? all[2] : 0) + end - units;
+#pragma unroll
+        for (int k = 0; k < kEach; ++k) {
+            for (unsigned long long left = wave_ballot(n[k] > kMediumMaxAtoms); left; left &= left - 1) {
+                const int b = lowest_bit(left), of = lane_read(mol[k], b), atoms = lane_read(n[k], b), at = lane_read(begin, b), most = units_of(atoms);
+                for (int u = 64 * static_cast<int>(blockIdx.x) + lane; u < most; u += 64 * kListers) {
+                    const int first = u << kLogRunCentres;
+                    // (more than there is room for: the molecules overlap)
+                    if (at + u < sorted.most_units) sorted.unit[at + u] = make_int2(of, (first << kLogRunCentres) + min(atoms - first, kRunCentres) - 1);
+                }
             }
+            begin += units_of(n[k]);
         }
         total += (all[0] + all[1]) + (all[2] + all[3]);
-        __syncthreads();                        // the next 256 molecules' counts go to the same places
+        __syncthreads();                        // the next molecules' counts go to the same places
     }
     if (blockIdx.x == 0 && tid == 0) *sorted.n_units = min(total, sorted.most_units);
 }
