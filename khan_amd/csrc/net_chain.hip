@@ -22,7 +22,7 @@
 // Two half-precision values for an operand, scaled by rows and columns, need three products and 1,180 us, but hold 23 bits of it, and
 // nothing of what is 2^-50 of its row's largest value or less.  Full rounds of 64-row tiles and the rest of 32 rows in two launches
 // measured as one form (1,490; 1,500 molecules 440 for 427), 64 columns of 32 rows to each of four wavefronts 1,614.
-// 340 us each way for those 47,000 rows (741 tiles of 64, three rounds of 256, at 2 GHz): matrix pipe busy 44 % forward and 42 % back, other vector
+// 340-347 us each way for those 47,000 rows (741 tiles of 64, three rounds of 256, at 2 GHz): matrix pipe busy 43 % forward and 42 % back, other vector
 // instructions 21 and 15 %, wavefronts waiting half of their time (profiles/networks_chain_deep4001_counters.md).
 #include <algorithm>
 
